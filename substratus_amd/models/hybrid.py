@@ -24,7 +24,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
-from ..ops import hybrid as ops, linear
+from ..ops import hybrid as ops, linear, linear_gated
 from ..parallel.comm import state
 from ..parallel.tp import Linear
 from ..serve.batch import StepBatch
@@ -456,7 +456,10 @@ class HybridLayer(nn.Module):
     def feed_forward(self, y: torch.Tensor):
         if self.spec.moe:
             return self.experts(y)
-        return self.w_down(ops.silu_mul(self.w_gateup(y)))
+        h = linear_gated(y, self.w_gateup.weight)
+        if h is None:
+            h = ops.silu_mul(self.w_gateup(y))
+        return self.w_down(h)
 
 
 class ParallelLayer(nn.Module):

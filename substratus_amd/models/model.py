@@ -126,7 +126,7 @@ class Block(nn.Module):
 
     def _mlp(self, y: torch.Tensor) -> torch.Tensor:
         if self.cfg.activation == "silu":
-            return self.w_down(ops.silu_mul(self.w_gateup(y)))
+            return self.w_down(self.w_gateup.gated(y))
         return self.w_down(ops.gelu(self.w_up(y)))
 
     # -- decode -------------------------------------------------------------
@@ -156,9 +156,9 @@ class Block(nn.Module):
         if self.parallel_attn:
             mlp_in = self.norm2(h, self.eps) if self.parallel_norms else y
             if self.cfg.activation == "silu":
-                gu = self.w_gateup(mlp_in)
+                a = self.w_gateup.gated(mlp_in)
                 yield
-                out = attn_out + self.w_down(ops.silu_mul(gu))
+                out = attn_out + self.w_down(a)
             else:
                 u = self.w_up(mlp_in)
                 yield
@@ -166,9 +166,9 @@ class Block(nn.Module):
             return out, h
         y2, h = fused_norm_residual(attn_out, h, self.norm2, self.eps)
         if self.cfg.activation == "silu":
-            gu = self.w_gateup(y2)
+            a = self.w_gateup.gated(y2)
             yield
-            out = self.w_down(ops.silu_mul(gu))
+            out = self.w_down(a)
         else:
             u = self.w_up(y2)
             yield

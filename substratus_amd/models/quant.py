@@ -20,6 +20,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import ops
 from .gguf import (QK, QK_K, Q4_K_BLOCK_BYTES, Q6_K_BLOCK_BYTES,
                    QUANT_CODECS, _pack_scale_min_k4, _unpack_scale_min_k4,
                    dequantize_q4_0, dequantize_q8_0, quantize_q4_0,
@@ -173,6 +174,10 @@ class QuantLinear(nn.Module):
         if self.bias is not None:
             y = y + self.bias
         return y.reshape(*shape[:-1], self.out_features)
+
+    def gated(self, x: torch.Tensor) -> torch.Tensor:
+        """silu(first half of the outputs) * second half."""
+        return ops.silu_mul(self(x))
 
 
 def quantize_model(model: nn.Module, quant: str) -> nn.Module:

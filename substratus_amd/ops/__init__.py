@@ -209,17 +209,71 @@ def flash_attn_train_available(d: int) -> bool:
 _GEMM_WS: dict = {}
 
 
+def inference_only(*tensors: torch.Tensor) -> bool:
+    """Nothing but values is asked of an op on these: no gradients in either
+    direction, no transform, trace, autocast or dispatch mode that expects
+    torch's own ops, no tensor subclass."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    if any(type(t) not in (torch.Tensor, torch.nn.Parameter)
+           for t in tensors):
+        return False
+    return not (torch.is_autocast_enabled("cuda")
+                or torch.compiler.is_compiling()
+                or torch._C._are_functorch_transforms_active()
+                or torch._C._len_torch_dispatch_stack()
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _few_rows(x: torch.Tensor, weight: torch.Tensor,
+              bias: Optional[torch.Tensor], gated: bool):
+    """(x as rows, extension) where the product goes to rows_gemm.hip, or
+    None. From 17 rows on the library is as fast or faster (28 x 4096 x 4096:
+    13.3 us there, 12.9 here; 28 x 22016 x 4096: 43.6, 47.6)."""
+    if not (x.is_cuda and weight.is_cuda and x.device == weight.device
+            and x.dtype == weight.dtype == torch.bfloat16 and x.dim() >= 1
+            and weight.dim() == 2 and x.shape[-1] == weight.shape[1]
+            and 0 < x.numel() <= 16 * x.shape[-1]):
+        return None
+    if bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_cuda
+                                 and bias.is_contiguous()
+                                 and bias.shape == weight.shape[:1]):
+        return None
+    given = (x, weight) if bias is None else (x, weight, bias)
+    ext = _load_ext()
+    if ext is None or not inference_only(*given):
+        return None
+    n, k = weight.shape
+    if x.dim() != 2:
+        x = x.reshape(-1, k)
+    if not (ext.rows_gemm_ok(x.shape[0], n, k, gated)
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and x.stride(1) == 1 and x.data_ptr() % 16 == 0
+            and (x.stride(0) % 8 == 0 and x.stride(0) >= k
+                 or x.shape[0] == 1)):
+        return None
+    return x, ext
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """F.linear, with an opt-in route (SUB_MGEMM=1) to the first-party
-    256x256 glds GEMM (mfma_gemm.hip) on decode-shaped inference cases.
+    """F.linear. Up to 16 rows of bf16 without gradients take the kernel that
+    streams weights at the memory's rate (rows_gemm.hip). SUB_MGEMM=1 routes
+    decode shapes of 256 rows and more to the 256x256 glds GEMM
+    (mfma_gemm.hip).
 
-    NOT on by default: the round-3 measurement (profiles/mgemm_r02.md)
-    shows hipBLASLt's MT192/MT256 solutions at 1.3-4.1 TB/s of weight
-    stream on the llama2-7b decode shapes vs our kernel's 1.0-2.25 — the
-    library's measured rates reach the ceiling measured for a deep-pipelined
-    schedule on this chip (~1.33-1.47 PF). The kernel stays for measurement and as the
-    base for a future counted-vmcnt schedule."""
+    The latter is NOT on by default: the round-3 measurement
+    (profiles/mgemm_r02.md) shows hipBLASLt's MT192/MT256 solutions at 1.3-4.1
+    TB/s of weight stream on the llama2-7b decode shapes vs our kernel's
+    1.0-2.25 — the library's measured rates reach the ceiling measured for a
+    deep-pipelined schedule on this chip (~1.33-1.47 PF). The kernel stays for
+    measurement and as the base for a future counted-vmcnt schedule."""
+    few = _few_rows(x, weight, bias, False)
+    if few is not None:
+        rows, ext = few
+        y = rows.new_empty(rows.shape[0], weight.shape[0])
+        ext.rows_gemm(y, rows, weight, bias, False)
+        return y if x.dim() == 2 else y.view(*x.shape[:-1], weight.shape[0])
     if (os.environ.get("SUB_MGEMM") != "1" or x.dtype != torch.bfloat16
             or torch.is_grad_enabled() and (
                 x.requires_grad or weight.requires_grad)):
@@ -246,6 +300,21 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
             _GEMM_WS[key] = part
     ext.mfma_gemm(y.view(m, n), x2.contiguous(), weight, bias, part, splitk)
     return y
+
+
+def linear_gated(x: torch.Tensor, weight: torch.Tensor,
+                 bias: Optional[torch.Tensor] = None
+                 ) -> Optional[torch.Tensor]:
+    """silu(first half) * second half of F.linear's columns, in one kernel, or
+    None where it is not made for that."""
+    few = _few_rows(x, weight, bias, True)
+    if few is None:
+        return None
+    rows, ext = few
+    n = weight.shape[0] // 2
+    y = rows.new_empty(rows.shape[0], n)
+    ext.rows_gemm(y, rows, weight, bias, True)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], n)
 
 
 def silu_mul(x: torch.Tensor) -> torch.Tensor:

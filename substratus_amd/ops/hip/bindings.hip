@@ -36,6 +36,8 @@ void launch_cross_entropy(float*, bf16_t*, const bf16_t*, const long*, long, int
 void launch_adamw(bf16_t*, const bf16_t*, float*, float*, long, float, float, float, float, float, int, float, hipStream_t);
 void launch_adamw_f32(float*, const float*, float*, float*, long, float, float, float, float, float, int, float, hipStream_t);
 void launch_quant_gemv(bf16_t*, const bf16_t*, const void*, const unsigned char*, int, int, int, bool, hipStream_t);
+bool rows_gemm_takes(int, int, int, bool);
+void launch_rows_gemm(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, int, int, int, long, long, bool, hipStream_t);
 void launch_dequant(bf16_t*, const void*, const unsigned char*, long, int, bool, hipStream_t);
 void launch_quant_gemv_k(bf16_t*, const bf16_t*, const void*, const unsigned char*, int, int, int, bool, hipStream_t);
 void launch_dequant_k(bf16_t*, const void*, const unsigned char*, int, int, bool, hipStream_t);
@@ -77,6 +79,10 @@ void check_bf16(const torch::Tensor& t, const char* name) {
   TORCH_CHECK(t.is_cuda(), name, " must be on GPU");
   TORCH_CHECK(t.scalar_type() == torch::kBFloat16, name, " must be bf16");
   TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
+}
+
+bool aligned16(const torch::Tensor& t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
 void post_launch_check(const char* op) {
@@ -374,6 +380,36 @@ long mfma_gemm_pick_splitk(long m, long n, long k) {
   return mfma_gemm_splitk((int)m, (int)n, (int)k);
 }
 
+// y = x w^T + bias, at most 16 rows of x; gated: y has half the columns,
+// silu(first half) * second half
+bool rows_gemm_ok(long m, long n, long k, bool gated) {
+  return rows_gemm_takes((int)m, (int)n, (int)k, gated);
+}
+
+void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias, bool gated) {
+  check_bf16(y, "y"); check_bf16(w, "w");
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
+              x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0,
+              "x must be bf16 rows that begin on 16-byte pieces");
+  const int m = x.size(0), k = x.size(1), n = w.size(0);
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == k && y.dim() == 2 &&
+              y.size(0) == m && y.size(1) == (gated ? n / 2 : n),
+              "rows_gemm: shape mismatch");
+  TORCH_CHECK(rows_gemm_takes(m, n, k, gated), "rows_gemm: unsupported shape ",
+              m, "x", n, "x", k);
+  TORCH_CHECK(aligned16(x) && aligned16(w), "rows_gemm: misaligned operand");
+  const bf16_t* bp = nullptr;
+  if (bias.has_value()) {
+    check_bf16(*bias, "bias");
+    TORCH_CHECK(bias->numel() == n, "bias size");
+    bp = bfc(*bias);
+  }
+  launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0),
+                   y.stride(0), gated, stream());
+  post_launch_check("rows_gemm");
+}
+
 void quant_gemv_k(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
                   torch::Tensor qs, bool q6) {
   check_bf16(y, "y"); check_bf16(x, "x");
@@ -557,6 +593,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_gemm_ok", &decode_gemm_ok);
   m.def("wstream_gemm", &wstream_gemm);
   m.def("wstream_ok", &wstream_ok);
+  m.def("rows_gemm", &rows_gemm);
+  m.def("rows_gemm_ok", &rows_gemm_ok);
   m.def("quant_gemv", &quant_gemv);
   m.def("dequant", &dequant);
   m.def("rms_norm", &rms_norm);

@@ -1,0 +1,149 @@
+// y = x w^T + bias of at most 16 rows with a bf16 weight matrix [n, k], as
+// single tokens of a small batch need it; or, of a matrix whose first half
+// gates its second, silu(gate) * up.
+//
+// Bound by reading the weights once. A workgroup takes 16 weight rows; its
+// four waves share k. A wave's loads go straight to LDS, 16 rows x 64
+// contiguous bytes each with consecutive lanes on consecutive 16-byte pieces:
+// loaded in the order of the matrix operands, where consecutive lanes have
+// different rows, every lane is a cache lookup of its own, and that, not
+// memory, sets the pace (4.5 TB/s). x takes the same way, since by registers
+// its rows would cost the lookups that the weights no longer do. A stage is 64
+// columns; four are in flight per wave and waited for one by one (64 KB, two
+// workgroups per CU). Pieces are permuted by the row, so that operand reads
+// meet no bank conflicts.
+//
+// us on a MI355X, from the library's product to this one:
+//   1 x 6144 x 2048    12.3 -> 7.1     8 x 12288 x 4096   28.2 -> 19.8
+//   1 x 2048 x 2048    10.8 -> 4.2     8 x 4096 x 4096    15.4 -> 8.0
+//   1 x 11264 x 2048   16.1 -> 10.2    8 x 22016 x 4096   52.8 -> 35.9
+//   1 x 2048 x 5632    11.2 -> 7.4     8 x 4096 x 11008   37.7 -> 19.5
+// (5.0 to 5.4 TB/s where the matrix is large). 8 and 16 waves, or 32 rows of
+// weights, are slower: fewer workgroups per CU. With 28 rows of x and more,
+// two operand tiles of x per wave, the library is the faster one.
+#include "rows_gemm.h"
+
+namespace {
+
+constexpr int KW = 4;             // waves, which share k
+constexpr int P = 4;              // stages in flight
+constexpr int U = 2;              // 32-column chunks of a stage
+constexpr int TILE = 64;          // 16-byte pieces of 16 rows x 32 columns
+constexpr int STAGE = U * 2 * TILE;
+constexpr int LOADS = U * 2;      // of a stage
+constexpr int PAD = 4;
+
+template <bool GATED>
+__global__ __launch_bounds__(KW * WAVE, 2)
+void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
+                      const bf16_t* __restrict__ w,
+                      const bf16_t* __restrict__ bias, int m, int n, int k,
+                      long x_ld, long y_ld) {
+  __shared__ alignas(16) uint4 s_all[KW * P * STAGE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE;
+  const int lo = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * (GATED ? 8 : 16);
+  const int chunks = k / 32;
+  const int c0 = chunks * wave / KW, c1 = chunks * (wave + 1) / KW;
+  const int steps = (c1 - c0 + U - 1) / U;
+  uint4* ring = s_all + wave * P * STAGE;
+
+  // a lane loads 16 bytes of row lane / 4 of a tile
+  const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
+  const char* wp = reinterpret_cast<const char*>(
+      w + (long)weight_row<GATED>(n0, row, n) * k) + piece * 16;
+  const char* xp = reinterpret_cast<const char*>(
+      x + min(row, m - 1) * x_ld) + piece * 16;
+  auto load = [&](int s, int i) {
+    #pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // a stage may be half of one: then its last chunk comes twice
+      const unsigned at = (unsigned)min(c0 + i * U + u, c1 - 1) * 64;
+      load_to_lds<16>(wp + at, ring + s * STAGE + u * 2 * TILE);
+      load_to_lds<16>(xp + at, ring + s * STAGE + (u * 2 + 1) * TILE);
+    }
+  };
+  const int at = lo * 4 + (g ^ ((lo >> 2) & 3));
+  float4v acc = {0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int s, int i, bool more) {
+    short8 wf[U], xf[U];
+    #pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint4* t = ring + s * STAGE + u * 2 * TILE + at;
+      wf[u] = *reinterpret_cast<const short8*>(t);
+      xf[u] = *reinterpret_cast<const short8*>(t + TILE);
+    }
+    if (more) {
+      wait_lds_reads();
+      load(s, i + P);
+    }
+    #pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (c0 + i * U + u < c1)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0,
+                                                      0);
+  };
+  #pragma unroll
+  for (int s = 0; s < P; ++s)
+    if (s < steps) load(s, s);
+  int i = 0;
+  for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
+    #pragma unroll
+    for (int s = 0; s < P; ++s) {
+      wait_loads<(P - 1) * LOADS>();
+      step(s, i + s, true);
+    }
+  }
+  for (; i < steps; i += P) {               // the ring runs dry
+    #pragma unroll
+    for (int s = 0; s < P; ++s)
+      if (i + s < steps) {
+        if (i + s + P <= steps) wait_loads<(P - 1) * LOADS>();
+        else wait_loads<0>();
+        step(s, i + s, i + s + P < steps);
+      }
+  }
+  __syncthreads();
+
+  // the waves' shares are added up; a lane has four columns of one row
+  float* red = reinterpret_cast<float*>(s_all);
+  *reinterpret_cast<float4v*>(&red[(wave * 16 + lo) * (16 + PAD) + g * 4]) =
+      acc;
+  __syncthreads();
+  const int r = threadIdx.x / 16, c = threadIdx.x % 16;
+  if (r >= m) return;
+  auto sum = [&](int c) {
+    float v = 0.f;
+    #pragma unroll
+    for (int q = 0; q < KW; ++q) v += red[(q * 16 + r) * (16 + PAD) + c];
+    if (bias != nullptr) v += bf2f(bias[weight_row<GATED>(n0, c, n)]);
+    return v;
+  };
+  if constexpr (GATED) {
+    if (c < 8) y[r * y_ld + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
+  } else {
+    if (n0 + c < n) y[r * y_ld + n0 + c] = f2bf(sum(c));
+  }
+}
+
+}  // namespace
+
+// Rows begin on 16-byte pieces; offsets within a row fit 32 bits.
+bool rows_gemm_takes(int m, int n, int k, bool gated) {
+  return m >= 1 && m <= 16 && n >= 1 && k >= 32 && k % 32 == 0 &&
+         (!gated || n % 16 == 0);
+}
+
+void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
+                      const bf16_t* bias, int m, int n, int k, long x_ld,
+                      long y_ld, bool gated, hipStream_t stream) {
+  if (gated) {
+    rows_gemm_kernel<true><<<dim3(n / 16), dim3(KW * WAVE), 0, stream>>>(
+        y, x, w, bias, m, n, k, x_ld, y_ld);
+  } else {
+    rows_gemm_kernel<false>
+        <<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
+            y, x, w, bias, m, n, k, x_ld, y_ld);
+  }
+}

@@ -49,6 +49,11 @@ class Linear(nn.Module):
         # else to hipBLASLt
         return ops.linear(x, self.weight, self.bias)
 
+    def gated(self, x: torch.Tensor) -> torch.Tensor:
+        """silu(first half of the outputs) * second half."""
+        y = ops.linear_gated(x, self.weight, self.bias)
+        return ops.silu_mul(self(x)) if y is None else y
+
 
 class ColumnParallelLinear(Linear):
     """Output features sharded across TP ranks; output stays sharded."""

@@ -125,6 +125,7 @@ class GraphDecodeRunner:
             self.tokens[sl], self.positions[sl], self.eng.kv.layers,
             self.slots[sl], self.block_table[sl], self.seq_lens[sl], *state)
 
+    @torch.no_grad()    # kernels without a backward may be taken
     def _step_body(self, b: int) -> None:
         # Op-skewed dual-stream decode: split the batch in half and
         # interleave the two forwards op-group by op-group on two HIP

@@ -1,0 +1,122 @@
+"""Products of a few rows (rows_gemm.hip) against 64 bits, at
+the sizes where their tiles, stages and shares of the inner dimension end."""
+
+import pytest
+import torch
+
+from substratus_amd import ops
+from substratus_amd.parallel.tp import Linear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def close(got, x, w, bias=None, extra=0.0):
+    """Within what rounding allows: half a bf16 step of the result (2^-9), and
+    32-bit sums whose order is free: 2^-24 per addend, of which a wave's share
+    has at most some hundreds and their errors partly cancel (2^-18 of the sum
+    of magnitudes)."""
+    want = x.double() @ w.double().T
+    room = 2.0 ** -18 * (x.double().abs() @ w.double().abs().T)
+    if bias is not None:
+        want = want + bias.double()
+    assert got.dtype == torch.bfloat16 and got.shape == want.shape
+    off = (got.double() - want).abs()
+    assert bool((off <= (2.0 ** -8 + extra) * want.abs() + room + 1e-30).all())
+
+
+def gated(y):
+    g, u = y.chunk(2, -1)
+    return torch.nn.functional.silu(g) * u
+
+
+# chunks of 32 columns for four waves, two to a stage, four stages in flight:
+# fewer chunks than waves, half stages, a full ring, more than one round
+@pytest.mark.parametrize("m", [1, 3, 16])
+@pytest.mark.parametrize("k", [32, 96, 160, 1024, 1056, 4544])
+@pytest.mark.parametrize("n", [16, 40, 55, 768])
+@torch.no_grad()
+def test_rows_gemm(m, n, k):
+    torch.manual_seed(m * 10000 + n + k)
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    b = torch.randn(n, device=DEV).bfloat16()
+    close(ops.linear(x, w), x, w)
+    close(ops.linear(x, w, b), x, w, b)
+    # rows of a wider buffer
+    wide = torch.randn(m, k + 64, device=DEV).bfloat16()
+    close(ops.linear(wide[:, 32:32 + k], w), wide[:, 32:32 + k], w)
+    y = ops.linear_gated(x, w)
+    assert (y is None) == (n % 16 != 0)
+    if y is not None:
+        want = gated(x.double() @ w.double().T)
+        room = (x.double().abs() @ w.double().abs().T).chunk(2, -1)
+        # a gate's error reaches the product by silu's slope, at most 1.1
+        full = (x.double() @ w.double().T).abs().chunk(2, -1)
+        assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs()
+                     + 2.0 ** -18 * 1.1 * (room[0] * full[1]
+                                           + room[1] * full[0]) + 1e-6).all())
+
+
+@torch.no_grad()
+def test_linear_forms_that_stay_with_the_library():
+    """The same results whichever way a product goes: other shapes of x, rows
+    that do not begin on 16 bytes, more rows, other types."""
+    torch.manual_seed(1)
+    w = torch.randn(64, 128, device=DEV).bfloat16()
+    for x in (torch.randn(128, device=DEV).bfloat16(),
+              torch.randn(2, 3, 128, device=DEV).bfloat16(),
+              torch.randn(128, 5, device=DEV).bfloat16().t(),
+              torch.randn(4, 132, device=DEV).bfloat16()[:, 4:],
+              torch.randn(4, 131, device=DEV).bfloat16()[:, 3:],
+              torch.randn(1, 128, device=DEV).bfloat16().expand(3, 128),
+              torch.randn(17, 128, device=DEV).bfloat16()):
+        got = ops.linear(x, w)
+        assert got.shape == (*x.shape[:-1], 64)
+        close(got.reshape(-1, 64), x.reshape(-1, 128), w)
+    x = torch.randn(3, 128, device=DEV)
+    assert torch.equal(ops.linear(x, w.float()),
+                       torch.nn.functional.linear(x, w.float()))
+    assert ops.linear(x[:0].bfloat16(), w).shape == (0, 64)
+
+
+def test_linear_keeps_gradients():
+    w = torch.nn.Parameter(torch.randn(64, 128, device=DEV).bfloat16())
+    x = torch.randn(3, 128, device=DEV).bfloat16()
+    ops.linear(x, w).float().sum().backward()
+    assert w.grad is not None
+    lin = Linear(128, 64, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(w)
+    lin.gated  # noqa: B018  (there beside the plain product)
+    xx = x.clone().requires_grad_()
+    (got,) = torch.func.vmap(lambda r: (ops.linear(r, w.detach()),))(x)
+    close(got, x, w.detach())
+    ops.linear(xx, w.detach()).float().sum().backward()
+    assert xx.grad is not None
+
+
+@torch.no_grad()
+def test_products_of_few_rows_in_a_graph():
+    """Replays with other inputs, eager work between."""
+    torch.manual_seed(3)
+    lin = Linear(512, 96, device=DEV, dtype=torch.bfloat16)
+    lin.weight.normal_()
+    x = torch.randn(3, 512, device=DEV).bfloat16()
+
+    def step():
+        return lin(x), lin.gated(x)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for seed in range(4):
+        x.copy_(torch.randn(3, 512, device=DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, step()):
+            assert torch.equal(a, b)
