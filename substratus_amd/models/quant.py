@@ -4,10 +4,10 @@ serving path rebuilt first-party).
 QuantLinear keeps weights resident as repacked GGUF blocks — fp16 scales
 [N, K/32] plus packed q4_0 nibbles [N, K/2] or q8_0 int8 [N, K] — and
 dispatches:
-  * GPU, M <= 8 (single-stream decode): fused block-dequant GEMV HIP kernel
-    (~4.25 bits/weight of HBM traffic instead of 16 — the decode-latency win
-    quantization exists for).
-  * GPU, M > 8 (prefill): dequant kernel to a transient bf16 buffer +
+  * GPU, up to 64 rows (decode): blocks are unpacked into matrix-core operands
+    on the way (rows_quant.hip: ~4.25 bits/weight of HBM traffic instead of 16
+    — the decode-latency win quantization exists for).
+  * GPU, more (prefill): dequant kernel to a transient bf16 buffer +
     hipBLASLt.
   * CPU: reference dequant + F.linear (the numerics oracle).
 """
@@ -153,20 +153,37 @@ class QuantLinear(nn.Module):
             return out
         return self._dequant_cpu()
 
+    def _few_rows(self, x2: torch.Tensor, gated: bool):
+        """The extension where rows_quant.hip takes the product, or None. 9
+        rows and more used to be a product in x's own type, which may be
+        differentiated: those stay where that is asked for."""
+        if not x2.is_cuda or not 0 < x2.shape[0] <= 64:
+            return None
+        if x2.shape[0] > 8 and (x2.dtype != torch.bfloat16
+                                or not ops.inference_only(x2)):
+            return None
+        from substratus_amd import _C
+        ok = _C.quant_rows_ok(x2.shape[0], self.out_features,
+                              self.in_features, self.quant, gated)
+        return _C if ok else None
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
         m = x2.shape[0]
-        if x.is_cuda and m <= 8:
+        ext = self._few_rows(x2, False)
+        if ext is not None:
+            y = torch.empty(m, self.out_features, dtype=torch.bfloat16,
+                            device=x.device)
+            ext.quant_rows(y, x2.contiguous().bfloat16(), self.scales,
+                           self.qs, self.quant, False)
+            y = y.to(x.dtype)
+        elif x.is_cuda and m <= 8 and not self.quant.endswith("_K"):
             from substratus_amd import _C
             y = torch.empty(m, self.out_features, dtype=torch.bfloat16,
                             device=x.device)
-            if self.quant.endswith("_K"):
-                _C.quant_gemv_k(y, x2.contiguous().bfloat16(), self.scales,
-                                self.qs, self.quant == "q6_K")
-            else:
-                _C.quant_gemv(y, x2.contiguous().bfloat16(), self.scales,
-                              self.qs, self.quant == "q8_0")
+            _C.quant_gemv(y, x2.contiguous().bfloat16(), self.scales,
+                          self.qs, self.quant == "q8_0")
             y = y.to(x.dtype)
         else:
             w = self.dequant_weight().to(x.dtype)
@@ -177,7 +194,16 @@ class QuantLinear(nn.Module):
 
     def gated(self, x: torch.Tensor) -> torch.Tensor:
         """silu(first half of the outputs) * second half."""
-        return ops.silu_mul(self(x))
+        x2 = x.reshape(-1, self.in_features)
+        ext = self._few_rows(x2, True) if self.bias is None and \
+            x.dtype == torch.bfloat16 else None
+        if ext is None:
+            return ops.silu_mul(self(x))
+        y = torch.empty(x2.shape[0], self.out_features // 2,
+                        dtype=torch.bfloat16, device=x.device)
+        ext.quant_rows(y, x2.contiguous(), self.scales, self.qs, self.quant,
+                       True)
+        return y.reshape(*x.shape[:-1], self.out_features // 2)
 
 
 def quantize_model(model: nn.Module, quant: str) -> nn.Module:

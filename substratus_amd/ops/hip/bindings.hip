@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
+#include "rows_quant.h"
+
 typedef __hip_bfloat16 bf16_t;
 
 // launchers (defined in the .hip translation units)
@@ -39,7 +41,6 @@ void launch_quant_gemv(bf16_t*, const bf16_t*, const void*, const unsigned char*
 bool rows_gemm_takes(int, int, int, bool);
 void launch_rows_gemm(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, int, int, int, long, long, bool, hipStream_t);
 void launch_dequant(bf16_t*, const void*, const unsigned char*, long, int, bool, hipStream_t);
-void launch_quant_gemv_k(bf16_t*, const bf16_t*, const void*, const unsigned char*, int, int, int, bool, hipStream_t);
 void launch_dequant_k(bf16_t*, const void*, const unsigned char*, int, int, bool, hipStream_t);
 int decode_gemm_splitk(int, int);
 bool decode_gemm_supported(int, int, int);
@@ -410,17 +411,49 @@ void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   post_launch_check("rows_gemm");
 }
 
-void quant_gemv_k(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
-                  torch::Tensor qs, bool q6) {
+Quant quant_of(const std::string& name) {
+  if (name == "q4_0") return Quant::Q4_0;
+  if (name == "q8_0") return Quant::Q8_0;
+  if (name == "q4_K") return Quant::Q4_K;
+  TORCH_CHECK(name == "q6_K", "unknown quantization ", name);
+  return Quant::Q6_K;
+}
+
+bool quant_rows_ok(long m, long n, long k, const std::string& quant,
+                   bool gated) {
+  return rows_quant_takes((int)m, (int)n, (int)k, quant_of(quant), gated);
+}
+
+// y = x w^T of a quantized weight matrix, at most 64 rows of x; gated as above
+void quant_rows(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
+                torch::Tensor qs, const std::string& quant, bool gated) {
   check_bf16(y, "y"); check_bf16(x, "x");
   TORCH_CHECK(scales.scalar_type() == torch::kHalf, "scales must be fp16");
   TORCH_CHECK(qs.scalar_type() == torch::kByte, "qs must be uint8");
-  int m = x.size(0), k = x.size(1), n = y.size(1);
+  TORCH_CHECK(scales.is_contiguous() && qs.is_contiguous());
+  const Quant q = quant_of(quant);
+  const int m = x.size(0), k = x.size(1);
+  const int n = y.size(1) * (gated ? 2 : 1);
+  TORCH_CHECK(y.size(0) == m && qs.size(0) == n && scales.size(0) == n,
+              "quant_rows: shape mismatch");
+  TORCH_CHECK(rows_quant_takes(m, n, k, q, gated),
+              "quant_rows: unsupported shape ", m, "x", n, "x", k);
+  // what is not aligned to the kernel's loads is copied to where it is
+  if (!aligned16(x)) x = x.clone();
+  if (!aligned16(qs)) qs = qs.clone();
+  if (!aligned16(scales)) scales = scales.clone();
+  launch_rows_quant(bf(y), bfc(x), scales.data_ptr(),
+                    qs.data_ptr<unsigned char>(), m, n, k, q, gated,
+                    stream());
+  post_launch_check("quant_rows");
+}
+
+void quant_gemv_k(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
+                  torch::Tensor qs, bool q6) {
+  const int m = x.size(0), k = x.size(1);
   TORCH_CHECK(m >= 1 && m <= 8, "quant_gemv_k is the M<=8 decode path");
   TORCH_CHECK(k % 256 == 0, "K must be a multiple of 256 (K-quants)");
-  launch_quant_gemv_k(bf(y), bfc(x), scales.data_ptr(),
-                      qs.data_ptr<unsigned char>(), m, n, k, q6, stream());
-  post_launch_check("quant_gemv_k");
+  quant_rows(y, x, scales, qs, q6 ? "q6_K" : "q4_K", false);
 }
 
 void dequant_k(torch::Tensor out, torch::Tensor scales, torch::Tensor qs,
@@ -527,6 +560,10 @@ void quant_gemv(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
   int m = x.size(0), k = x.size(1), n = y.size(1);
   TORCH_CHECK(m >= 1 && m <= 8, "quant_gemv supports M in [1,8], got ", m);
   TORCH_CHECK(k % 32 == 0, "K must be a multiple of 32");
+  if (rows_quant_takes(m, n, k, q8 ? Quant::Q8_0 : Quant::Q4_0, false)) {
+    quant_rows(y, x, scales, qs, q8 ? "q8_0" : "q4_0", false);
+    return;
+  }
   launch_quant_gemv(bf(y), bfc(x), scales.data_ptr(),
                     qs.data_ptr<unsigned char>(), m, n, k, q8, stream());
   post_launch_check("quant_gemv");
@@ -595,6 +632,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wstream_ok", &wstream_ok);
   m.def("rows_gemm", &rows_gemm);
   m.def("rows_gemm_ok", &rows_gemm_ok);
+  m.def("quant_rows", &quant_rows);
+  m.def("quant_rows_ok", &quant_rows_ok);
   m.def("quant_gemv", &quant_gemv);
   m.def("dequant", &dequant);
   m.def("rms_norm", &rms_norm);

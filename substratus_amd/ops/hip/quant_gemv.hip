@@ -8,9 +8,11 @@
 //   qs:     q4_0 -> uint8 [N, K/2] (nibble i of byte b packs weights b and
 //           b+16 of the 32-block: llama.cpp layout), q8_0 -> int8 [N, K]
 //
-// quant_gemv (M <= 8, latency-bound decode): one wave per output row; each
-// lane owns blocks lane, lane+64, ... (scale 2 B + 16 B nibbles via uint4);
-// x read through L2 (it is re-read by every row — L2/L3 resident);
+// quant_gemv: one wave per output element row of one row of x, for what
+// rows_quant.hip does not take (k no multiple of 64) and q8_0 with a single
+// row of x, where that kernel's workgroups of 16 weight rows leave the chip
+// unevenly filled (N=5120: 9.4 us here, 11.1 there); each lane owns blocks
+// lane, lane+64, ... (scale 2 B + 16 B nibbles via uint4); x read through L2;
 // wave-reduced fp32 accumulation.
 //
 // dequant (prefill / large M): block-parallel expansion to bf16, then the
@@ -19,7 +21,7 @@
 
 typedef _Float16 f16_t;
 
-template <int M, bool Q8>
+template <bool Q8>
 __global__ __launch_bounds__(256)
 void quant_gemv_kernel(bf16_t* __restrict__ y,         // [M, N]
                        const bf16_t* __restrict__ x,   // [M, K]
@@ -28,115 +30,73 @@ void quant_gemv_kernel(bf16_t* __restrict__ y,         // [M, N]
                        int n, int k) {
   const int row = blockIdx.x * 4 + threadIdx.x / WAVE;  // 4 waves = 4 rows
   if (row >= n) return;
+  x += (long)blockIdx.y * k;
   const int lane = threadIdx.x % WAVE;
   const int nblocks = k / 32;
   const f16_t* srow = scales + (long)row * nblocks;
-  float acc[M];
-  #pragma unroll
-  for (int m = 0; m < M; ++m) acc[m] = 0.f;
+  float acc = 0.f;
 
   if (!Q8) {
-    // 2-deep software pipeline: block b+WAVE's qs/scale loads are issued
-    // before block b's dequant-dot. Tail handling is BRANCHLESS: indices
-    // clamp to the last block and a zero scale masks the redundant work —
-    // a per-lane `if (b < nblocks)` guard around the loads makes hipcc
-    // branch and drain vmcnt per iteration (guide §5 trap 4(c)), which
-    // measured SLOWER than no pipeline at all.
     const uint4* qrow = reinterpret_cast<const uint4*>(qs + (long)row * k / 2);
-    const int last = nblocks - 1;
-    int b = lane;
-    uint4 nib_c = qrow[min(b, last)];
-    float sv0 = (float)srow[min(b, last)];
-    float s_c = (b <= last) ? sv0 : 0.f;
-    const int iters = (nblocks + WAVE - 1) / WAVE;
-    for (int it = 0; it < iters; ++it, b += WAVE) {
-      const int bn = min(b + WAVE, last);
-      const uint4 nib_n = qrow[bn];
-      const float svn = (float)srow[bn];  // load always, select after
-      const float s_n = (b + WAVE <= last) ? svn : 0.f;
-      const int bcl = min(b, last);       // clamp x address for masked lanes
-      const unsigned int w[4] = {nib_c.x, nib_c.y, nib_c.z, nib_c.w};
-      // issue every row's x loads before any compute (per-m inline loads
-      // serialize the M>1 case: 0.94 TB/s vs 2.34 at M=1)
-      uint4 xall[M][4];
+    for (int b = lane; b < nblocks; b += WAVE) {
+      const uint4 nib = qrow[b];
+      const unsigned int w[4] = {nib.x, nib.y, nib.z, nib.w};
+      const uint4* xb = reinterpret_cast<const uint4*>(x + b * 32);
+      uint4 xv[4];
       #pragma unroll
-      for (int m = 0; m < M; ++m) {
-        const uint4* xb =
-            reinterpret_cast<const uint4*>(x + (long)m * k + bcl * 32);
-        #pragma unroll
-        for (int c = 0; c < 4; ++c) xall[m][c] = xb[c];
-      }
+      for (int c = 0; c < 4; ++c) xv[c] = xb[c];
+      float partial = 0.f;
       #pragma unroll
-      for (int m = 0; m < M; ++m) {
-        float partial = 0.f;
+      for (int c = 0; c < 4; ++c) {   // 4 bytes -> weights i..i+3, i+16..19
+        const uint4 lo4 = xv[c / 2], hi4 = xv[2 + c / 2];
+        const unsigned int xlo[2] = {c % 2 == 0 ? lo4.x : lo4.z,
+                                     c % 2 == 0 ? lo4.y : lo4.w};
+        const unsigned int xhi[2] = {c % 2 == 0 ? hi4.x : hi4.z,
+                                     c % 2 == 0 ? hi4.y : hi4.w};
         #pragma unroll
-        for (int c = 0; c < 4; ++c) {   // 4 bytes -> weights i..i+3, i+16..19
-          unsigned int word = w[c];
-          const uint4 xlo4 = xall[m][c >= 2 ? 1 : 0];
-          const uint4 xhi4 = xall[m][c >= 2 ? 3 : 2];
-          const unsigned int xlo[2] = {c % 2 == 0 ? xlo4.x : xlo4.z,
-                                       c % 2 == 0 ? xlo4.y : xlo4.w};
-          const unsigned int xhi[2] = {c % 2 == 0 ? xhi4.x : xhi4.z,
-                                       c % 2 == 0 ? xhi4.y : xhi4.w};
-          #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float lo = (float)((word >> (8 * j)) & 0xF) - 8.f;
-            const float hi = (float)((word >> (8 * j + 4)) & 0xF) - 8.f;
-            const float2 xl = unpack_bf16x2(xlo[j / 2]);
-            const float2 xh = unpack_bf16x2(xhi[j / 2]);
-            const float xv_lo = (j % 2 == 0) ? xl.x : xl.y;
-            const float xv_hi = (j % 2 == 0) ? xh.x : xh.y;
-            partial += lo * xv_lo + hi * xv_hi;
-          }
+        for (int j = 0; j < 4; ++j) {
+          const float lo = (float)((w[c] >> (8 * j)) & 0xF) - 8.f;
+          const float hi = (float)((w[c] >> (8 * j + 4)) & 0xF) - 8.f;
+          const float2 xl = unpack_bf16x2(xlo[j / 2]);
+          const float2 xh = unpack_bf16x2(xhi[j / 2]);
+          partial += lo * (j % 2 == 0 ? xl.x : xl.y) +
+                     hi * (j % 2 == 0 ? xh.x : xh.y);
         }
-        acc[m] += partial * s_c;
       }
-      nib_c = nib_n;
-      s_c = s_n;
+      acc += partial * (float)srow[b];
     }
   } else {
     const uint4* qrow = reinterpret_cast<const uint4*>(qs + (long)row * k);
     for (int b = lane; b < nblocks; b += WAVE) {
       const float s = (float)srow[b];
-      // 32 int8 = 2 × uint4
+      // 32 int8 = 2 x uint4
       const uint4 q0 = qrow[b * 2], q1 = qrow[b * 2 + 1];
       const unsigned int w[8] = {q0.x, q0.y, q0.z, q0.w,
                                  q1.x, q1.y, q1.z, q1.w};
-      uint4 xall8[M][4];
+      const uint4* xb = reinterpret_cast<const uint4*>(x + b * 32);
+      uint4 xv[4];
       #pragma unroll
-      for (int m = 0; m < M; ++m) {
-        const uint4* xb =
-            reinterpret_cast<const uint4*>(x + (long)m * k + b * 32);
-        #pragma unroll
-        for (int c = 0; c < 4; ++c) xall8[m][c] = xb[c];
-      }
+      for (int c = 0; c < 4; ++c) xv[c] = xb[c];
+      float partial = 0.f;
       #pragma unroll
-      for (int m = 0; m < M; ++m) {
-        float partial = 0.f;
+      for (int c = 0; c < 4; ++c) {
+        const unsigned int xs[4] = {xv[c].x, xv[c].y, xv[c].z, xv[c].w};
         #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const uint4 xv = xall8[m][c];
-          const unsigned int xs[4] = {xv.x, xv.y, xv.z, xv.w};
+        for (int j = 0; j < 2; ++j) {  // 2 words of 4 int8 per uint4-pair
+          const unsigned int word = w[c * 2 + j];
           #pragma unroll
-          for (int j = 0; j < 2; ++j) {  // 2 words of 4 int8 per uint4-pair
-            const unsigned int word = w[c * 2 + j];
-            #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const float qv = (float)(signed char)((word >> (8 * t)) & 0xFF);
-              const float2 xp = unpack_bf16x2(xs[j * 2 + t / 2]);
-              partial += qv * ((t % 2 == 0) ? xp.x : xp.y);
-            }
+          for (int t = 0; t < 4; ++t) {
+            const float qv = (float)(signed char)((word >> (8 * t)) & 0xFF);
+            const float2 xp = unpack_bf16x2(xs[j * 2 + t / 2]);
+            partial += qv * ((t % 2 == 0) ? xp.x : xp.y);
           }
         }
-        acc[m] += partial * s;
       }
+      acc += partial * s;
     }
   }
-  #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    float v = wave_sum(acc[m]);
-    if (lane == 0) y[(long)m * n + row] = f2bf(v);
-  }
+  const float v = wave_sum(acc);
+  if (lane == 0) y[(long)blockIdx.y * n + row] = f2bf(v);
 }
 
 // expand quantized rows to bf16 (prefill path feeds hipBLASLt)
@@ -172,32 +132,14 @@ __global__ void dequant_kernel(bf16_t* __restrict__ out,   // [N, K]
 void launch_quant_gemv(bf16_t* y, const bf16_t* x, const void* scales,
                        const unsigned char* qs, int m, int n, int k,
                        bool q8, hipStream_t stream) {
-  dim3 grid((n + 3) / 4);
+  dim3 grid((n + 3) / 4, m);
   dim3 block(256);
   const f16_t* sc = reinterpret_cast<const f16_t*>(scales);
-  // braces matter: torch's hipify rewrites <<<>>> and glues a bare `else`
-  // onto the launch otherwise
-  #define GEMV_CASE(MM)                                                   \
-    do {                                                                  \
-      if (q8) {                                                           \
-        quant_gemv_kernel<MM, true><<<grid, block, 0, stream>>>(          \
-            y, x, sc, qs, n, k);                                          \
-      } else {                                                            \
-        quant_gemv_kernel<MM, false><<<grid, block, 0, stream>>>(         \
-            y, x, sc, qs, n, k);                                          \
-      }                                                                   \
-    } while (0)
-  switch (m) {
-    case 1: GEMV_CASE(1); break;
-    case 2: GEMV_CASE(2); break;
-    case 3: GEMV_CASE(3); break;
-    case 4: GEMV_CASE(4); break;
-    case 5: GEMV_CASE(5); break;
-    case 6: GEMV_CASE(6); break;
-    case 7: GEMV_CASE(7); break;
-    case 8: GEMV_CASE(8); break;
+  if (q8) {
+    quant_gemv_kernel<true><<<grid, block, 0, stream>>>(y, x, sc, qs, n, k);
+  } else {
+    quant_gemv_kernel<false><<<grid, block, 0, stream>>>(y, x, sc, qs, n, k);
   }
-  #undef GEMV_CASE
 }
 
 void launch_dequant(bf16_t* out, const void* scales, const unsigned char* qs,

@@ -1,4 +1,5 @@
-// Pieces of products of a few rows with a weight matrix (rows_gemm.hip).
+// What products of a few rows with a weight matrix share (rows_gemm.hip for
+// bf16 weights, rows_quant.hip for GGUF blocks).
 #pragma once
 
 #include "common.h"

@@ -1,0 +1,447 @@
+// y = x w^T of up to 64 rows with a GGUF-quantized weight matrix [n, k], or,
+// of a matrix whose first half gates its second, silu(gate) * up. Weights as
+// models/quant.py lays them out:
+//   q4_0, q8_0   scales fp16 [n, k/32]; qs [n, k/2] nibbles (byte i of a block
+//                has weights i and i + 16), [n, k] int8
+//   q4_K         scales fp16 [n, k/128] (d and dmin of each 256); qs rows: a
+//                6-bit scale per 32, a 6-bit minimum per 32, nibbles (byte l
+//                of 64 weights has l and l + 32)
+//   q6_K         scales fp16 [n, k/256]; qs rows: low nibbles, high pairs of
+//                bits, an int8 scale per 16
+//
+// Bound by reading packed weights and by unpacking them. Unpacked they are
+// whole numbers, which bf16 holds exactly: 16 + nibble (or 64 + six bits, or
+// 128 + byte) takes one and-or of a shifted word, and the matrix cores
+// multiply it with x. The offset is taken off inside: a product of x with a
+// constant gives -offset * sum(x), where the weights' product begins, and with
+// minima those sums are needed anyway. One instruction's inner size is one
+// block, so its sum is scaled in 32 bits and added up, as in a loop over
+// blocks in 32-bit arithmetic.
+//
+// A workgroup takes 16 weight rows and MR rows of x; its waves share k. A
+// stage is 256 columns; weights, scales and x go straight to LDS with
+// consecutive lanes on consecutive bytes (see rows_gemm.hip), pieces permuted
+// by the row against bank conflicts. Few rows of x: P stages in flight per
+// wave; many: one, and more workgroups per CU instead.
+//
+// us on a MI355X, 15360 x 5120, 5120 x 5120, 27648 x 5120, 5120 x 13824, from
+// one wave per weight row in vector arithmetic (up to 8 rows of x), or from
+// unpacking to bf16 in memory and the library (more), to this kernel:
+//   q4_0  1 row   20.5  8.5 31.7 15.0 -> 14.4  7.3 21.4 14.8
+//         5 rows  55.0 21.5 95.3 47.8 -> 16.1  9.3 25.6 18.8
+//        24 rows  81.4 37.8  152 75.9 -> 28.1 15.3 45.8 33.4
+//   q8_0  5 rows  55.9 21.2 97.5 46.3 -> 22.8 12.1 36.5 25.0
+//        24 rows  82.5 38.8  155 78.9 -> 42.1 20.8 70.2 43.5
+//   q4_K  1 row   29.4 12.9 49.4 24.6 -> 15.7  8.5 24.9 22.1
+//         5 rows   115 47.7  196  111 -> 18.0 10.4 28.8 25.4
+//        24 rows  90.1 37.8  172 84.6 -> 30.7 16.8 50.2 39.9
+//   q6_K  1 row   32.7 13.3 57.5 26.8 -> 20.8 11.8 33.1 26.3
+//         5 rows   118 40.9  205 90.9 -> 23.1 13.0 37.4 29.0
+//        24 rows   523  196  946  479 -> 38.4 19.5 64.8 46.9
+// q8_0 with one row stays with the vector kernel (quant_gemv.hip): 20.5, 9.4,
+// 33.1, 19.3 there and 19.9, 11.1, 32.2, 23.8 here.
+#include "rows_gemm.h"
+#include "rows_quant.h"
+
+#include <type_traits>
+
+namespace {
+
+typedef _Float16 f16_t;
+using std::integral_constant;
+
+constexpr int COLS = 256;         // of a stage
+constexpr int TILE = 64;          // 16-byte pieces of 16 rows x 64 bytes
+
+DEV_INLINE short8 vec8(unsigned a, unsigned b, unsigned c, unsigned d) {
+  return __builtin_bit_cast(short8, (uint4v){a, b, c, d});
+}
+
+DEV_INLINE float half_of(unsigned u) {       // its low 16 bits
+  return (float)__builtin_bit_cast(f16_t, (unsigned short)(u & 0xffff));
+}
+
+DEV_INLINE float half_at(const uint4v& u, int i) {
+  return half_of(u[i >> 1] >> (16 * (i & 1)));
+}
+
+DEV_INLINE float byte_at(const uint4v& u, int i) {
+  return (float)((u[i >> 2] >> (8 * (i & 3))) & 0xff);
+}
+
+// Two 16-bit halves out of two words: the low ones, the high ones.
+DEV_INLINE unsigned low2(unsigned a, unsigned b) {
+  return __builtin_amdgcn_perm(b, a, 0x05040100);
+}
+DEV_INLINE unsigned high2(unsigned a, unsigned b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302);
+}
+
+// 16 + nibbles at bits 3 to 6 of eight bytes, as bf16. c16: two bf16 of 16.
+DEV_INLINE short8 unpack4(unsigned a, unsigned b, unsigned c16) {
+  auto two = [&](unsigned v, unsigned sel) {
+    return (__builtin_amdgcn_perm(v, v, sel) & 0x780078u) | c16;
+  };
+  return vec8(two(a, 0x0c010c00), two(a, 0x0c030c02), two(b, 0x0c010c00),
+              two(b, 0x0c030c02));
+}
+
+// 128 + eight signed bytes, as bf16: whole numbers below 256 are exact.
+DEV_INLINE short8 unpack8(const uint2v& v) {
+  unsigned o[4];
+  #pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const unsigned z = v[h] ^ 0x80808080u;
+    float f[4];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = (float)((z >> (8 * i)) & 0xff);
+    o[h * 2] = high2(__float_as_uint(f[0]), __float_as_uint(f[1]));
+    o[h * 2 + 1] = high2(__float_as_uint(f[2]), __float_as_uint(f[3]));
+  }
+  return vec8(o[0], o[1], o[2], o[3]);
+}
+
+template <int ME>
+DEV_INLINE void add_scaled(float4v& a, float s, const float4v& v) {
+  #pragma unroll
+  for (int e = 0; e < ME; ++e) a[e] += s * v[e];
+}
+
+// Tiles of 16 rows x 64 bytes in a stage, 16-byte scale rows, loads of both;
+// two bf16 of minus the offset of unpacked weights.
+template <Quant Q> struct Layout;
+template <> struct Layout<Quant::Q4_0> {
+  static constexpr int W = 2, S = 1, LOADS = 3;
+  static constexpr unsigned OFF = 0xC1C0C1C0u;        // -24
+};
+template <> struct Layout<Quant::Q8_0> {
+  static constexpr int W = 4, S = 1, LOADS = 5;
+  static constexpr unsigned OFF = 0xC300C300u;        // -128
+};
+template <> struct Layout<Quant::Q4_K> {
+  static constexpr int W = 2, S = 2, LOADS = 4;
+  static constexpr unsigned OFF = 0xC180C180u;        // -16
+};
+template <> struct Layout<Quant::Q6_K> {
+  static constexpr int W = 3, S = 1, LOADS = 5;       // one to a register
+  static constexpr unsigned OFF = 0xC2C0C2C0u;        // -96
+};
+
+// MR: rows of x; ME: of every four, those that are there (MR 4 only); KW
+// waves share k, P stages are in flight in each
+template <Quant Q, int MR, int ME, int KW, int P, bool GATED>
+__global__ __launch_bounds__(KW * WAVE, 2)
+void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
+                       const f16_t* __restrict__ scales,
+                       const unsigned char* __restrict__ qs, int m, int n,
+                       int k) {
+  using L = Layout<Q>;
+  constexpr bool K_QUANT = Q == Quant::Q4_K || Q == Quant::Q6_K;
+  constexpr int FM = (MR + 15) / 16;
+  constexpr int XL = MR / 2;                     // loads of x, 4 rows x 256 B
+  constexpr int WS = L::W * TILE + L::S * 16;    // weights and scales
+  constexpr int STAGE = XL * 64 + WS;
+  constexpr int LOADS = XL + L::LOADS;
+  constexpr int BM = FM * 16, PAD = 1;
+  constexpr int RED = (KW * BM * (16 + PAD) + 3) / 4, RING = KW * P * STAGE;
+  __shared__ alignas(16) uint4v s_all[RING > RED ? RING : RED];
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE;
+  const int lo = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * (GATED ? 8 : 16);
+  x += (long)blockIdx.y * MR * k;
+  m -= blockIdx.y * MR;
+  const int nb = k / 32, all = (k + COLS - 1) / COLS;
+  const int c0 = all * wave / KW, c1 = all * (wave + 1) / KW;
+  const int steps = c1 - c0;
+  uint4v* ring = s_all + wave * P * STAGE;
+
+  // bytes of a row of weights, of scales
+  const long rb = Q == Quant::Q4_0 ? k / 2 : Q == Quant::Q8_0 ? k
+      : Q == Quant::Q4_K ? k / 16 + k / 2 : k / 16 * 13;
+  const long sb = !K_QUANT ? nb * 2 : Q == Quant::Q4_K ? k / 64 : k / 128;
+  // a lane loads 16 bytes of row lane / 4 of a tile, and a word of its scales
+  const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
+  const int word = lane & 3;
+  const unsigned char* sc = reinterpret_cast<const unsigned char*>(scales);
+  const unsigned char* wp = qs + weight_row<GATED>(n0, row, n) * rb;
+  const unsigned char* sp = sc + weight_row<GATED>(n0, row, n) * sb;
+  const unsigned char* dp = sc + weight_row<GATED>(n0, lo, n) * sb;
+  const char* xp[XL / 2];
+  #pragma unroll
+  for (int d = 0; d < XL / 2; ++d)
+    xp[d] = reinterpret_cast<const char*>(
+        x + (long)min(d * 4 + (lane >> 4), m - 1) * k);
+  unsigned short dreg[P];                        // q6_K: the stage's d
+  auto load = [&](int s, int c) {
+    uint4v* ws = ring + s * STAGE;
+    uint4v* ss = ws + L::W * TILE;
+    // past a row's last block: that block again, which nobody reads
+    if constexpr (Q == Quant::Q4_0) {
+      #pragma unroll
+      for (int t = 0; t < 2; ++t)
+        load_to_lds<16>(wp + min(c * 8 + t * 4 + piece, nb - 1) * 16,
+                        ws + t * TILE);
+      load_to_lds<4>(sp + min(c * 16 + word * 4, nb * 2 - 4), ss);
+    } else if constexpr (Q == Quant::Q8_0) {
+      #pragma unroll
+      for (int t = 0; t < 4; ++t)
+        load_to_lds<16>(wp + min(c * 256 + t * 64 + piece * 16, k - 16),
+                        ws + t * TILE);
+      load_to_lds<4>(sp + min(c * 16 + word * 4, nb * 2 - 4), ss);
+    } else if constexpr (Q == Quant::Q4_K) {
+      #pragma unroll
+      for (int t = 0; t < 2; ++t)
+        load_to_lds<16>(wp + k / 16 + c * 128 + t * 64 + piece * 16,
+                        ws + t * TILE);
+      // words: scales 0 to 3, 4 to 7, minima 0 to 3, 4 to 7
+      load_to_lds<4>(wp + (word & 2) * (k / 64) + c * 8 + (word & 1) * 4, ss);
+      load_to_lds<4>(dp + c * 4, ss + 16);
+    } else {
+      #pragma unroll
+      for (int t = 0; t < 2; ++t)
+        load_to_lds<16>(wp + c * 128 + t * 64 + piece * 16, ws + t * TILE);
+      load_to_lds<16>(wp + k / 2 + c * 64 + piece * 16, ws + 2 * TILE);
+      load_to_lds<4>(wp + k / 4 * 3 + c * 16 + word * 4, ss);
+      // two bytes only: words need not be aligned
+      dreg[s] = *reinterpret_cast<const unsigned short*>(dp + c * 2);
+    }
+    uint4v* xs = ws + WS;
+    #pragma unroll
+    for (int d = 0; d < XL; ++d) {
+      const int p = c * 32 + (d & 1) * 16 +
+                    (lo ^ ((lane >> 4) << 2) ^ ((d >> 1) & 3));
+      load_to_lds<16>(xp[d >> 1] + (long)min(p, k / 8 - 1) * 16, xs + d * 64);
+    }
+  };
+
+  unsigned c16 = 0x41804180u, c64 = 0x42804280u;
+  asm("" : "+v"(c16));       // in registers: an and-or has room for one literal
+  asm("" : "+v"(c64));
+  const short8 off = vec8(L::OFF, L::OFF, L::OFF, L::OFF);
+  const float4v zero = {0.f, 0.f, 0.f, 0.f};
+  // q4_0: lanes of the first 16 weights take low nibbles, the others high
+  // ones; rotated right by this they are at bits 3 to 6 of their bytes
+  const int turn = g >> 1 ? 1 : 29;
+  int xr[FM];                                    // the lane's rows of x
+  #pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int r = (j * 16 + lo) & (MR - 1);
+    xr[j] = (r >> 2) * 128 + (r & 3) * 16;
+  }
+  const int xsw = ((lo & 3) << 2) ^
+                  (((lo & (MR > 16 ? 15 : MR - 1)) >> 2) & 3);
+  const int wsw = (lo >> 2) & 3;
+  float4v acc[FM];
+  #pragma unroll
+  for (int j = 0; j < FM; ++j) acc[j] = zero;
+
+  auto use = [&](int s, int c, auto whole) {
+    const uint4v* ws = ring + s * STAGE + lo * 4;
+    const uint4v* ss = ring + s * STAGE + L::W * TILE;
+    const uint4v* xs = ring + s * STAGE + WS;
+    const uint4v sv = ss[lo];
+    float d = 0.f, dm = 0.f;
+    if constexpr (Q == Quant::Q4_K) {
+      const unsigned dd = reinterpret_cast<const unsigned*>(ss + 16)[lo];
+      d = half_of(dd);
+      dm = half_of(dd >> 16) * 0.0625f;          // sums of x come times -16
+    }
+    if constexpr (Q == Quant::Q6_K) d = half_of(dreg[s]);
+    #pragma unroll
+    for (int b = 0; b < COLS / 32; ++b) {
+      if (!decltype(whole)::value && c * 8 + b >= nb) break;
+      if constexpr (Q != Quant::Q6_K) {
+        // eight bytes with the lane's eight weights, k = 8 g on
+        const int at = Q == Quant::Q4_0 ? b & 3
+            : Q == Quant::Q8_0 ? (b & 1) * 2 + (g >> 1)
+                               : ((b >> 1) & 1) * 2 + (g >> 1);
+        const uint2v v = reinterpret_cast<const uint2v*>(
+            ws + (Q == Quant::Q8_0 ? b >> 1 : b >> 2) * TILE +
+            (at ^ wsw))[g & 1];
+        short8 wv;
+        if constexpr (Q == Quant::Q4_0)
+          wv = unpack4(__builtin_amdgcn_alignbit(v[0], v[0], turn),
+                       __builtin_amdgcn_alignbit(v[1], v[1], turn), c16);
+        else if constexpr (Q == Quant::Q8_0)
+          wv = unpack8(v);
+        else
+          wv = b & 1 ? unpack4(v[0] >> 1, v[1] >> 1, c16)
+                     : unpack4(v[0] << 3, v[1] << 3, c16);
+        const float scale = Q == Quant::Q4_K ? d * byte_at(sv, b)
+                                             : half_at(sv, b);
+        #pragma unroll
+        for (int j = 0; j < FM; ++j) {
+          const short8 xv = __builtin_bit_cast(
+              short8, xs[xr[j] + (b >> 2) * 64 + (((b * 4 + g) & 15) ^ xsw)]);
+          const float4v sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              xv, off, zero, 0, 0, 0);
+          add_scaled<ME>(acc[j], scale,
+                         __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                             xv, wv, sum, 0, 0, 0));
+          if constexpr (Q == Quant::Q4_K)
+            add_scaled<ME>(acc[j], dm * byte_at(sv, 8 + b), sum);
+        }
+      } else {
+        // a scale per 16 weights: instructions of inner size 16, even and odd
+        // bytes in turn
+        const int hf = b >> 2, quarter = b & 3;
+        const uint2v off4 = {L::OFF, L::OFF};
+        const short4v o4 = __builtin_bit_cast(short4v, off4);
+        #pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const unsigned v = reinterpret_cast<const unsigned*>(
+              ws + hf * TILE + (((quarter & 1) * 2 + h) ^ wsw))[g];
+          const unsigned hv = reinterpret_cast<const unsigned*>(
+              ws + 2 * TILE + ((hf * 2 + h) ^ wsw))[g];
+          unsigned o[2];
+          #pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const unsigned low = quarter < 2 ? (e ? v >> 7 : v << 1)
+                                             : (e ? v >> 11 : v >> 3);
+            const int up = 5 - 2 * quarter - 8 * e;
+            const unsigned high = up >= 0 ? hv << up : hv >> -up;
+            o[e] = ((low & 0x1E001Eu) | c64) | (high & 0x600060u);
+          }
+          const uint2v o2 = {o[0], o[1]};
+          const short4v wv = __builtin_bit_cast(short4v, o2);
+          const int si = hf * 8 + quarter * 2 + h;
+          const float scale = d * (float)(signed char)(
+              (sv[si >> 2] >> (8 * (si & 3))) & 0xff);
+          #pragma unroll
+          for (int j = 0; j < FM; ++j) {
+            const int p = b * 4 + h * 2 + (g >> 1);
+            const uint2v xw = reinterpret_cast<const uint2v*>(
+                xs + xr[j] + (p >> 4) * 64 + ((p & 15) ^ xsw))[g & 1];
+            const uint2v xe = {low2(xw[0], xw[1]), high2(xw[0], xw[1])};
+            const short4v xv = __builtin_bit_cast(short4v, xe);
+            const float4v sum = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                xv, o4, zero, 0, 0, 0);
+            add_scaled<ME>(acc[j], scale,
+                           __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                               xv, wv, sum, 0, 0, 0));
+          }
+        }
+      }
+    }
+  };
+
+  #pragma unroll
+  for (int s = 0; s < P; ++s)
+    if (s < steps) load(s, c0 + s);
+  int i = 0;
+  for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
+    #pragma unroll
+    for (int s = 0; s < P; ++s) {
+      wait_loads<(P - 1) * LOADS>();
+      use(s, c0 + i + s, integral_constant<bool, true>{});
+      wait_lds_reads();
+      load(s, c0 + i + s + P);
+    }
+  }
+  for (; i < steps; i += P) {               // the ring runs dry
+    #pragma unroll
+    for (int s = 0; s < P; ++s)
+      if (i + s < steps) {
+        if (i + s + P <= steps) wait_loads<(P - 1) * LOADS>();
+        else wait_loads<0>();
+        use(s, c0 + i + s, integral_constant<bool, K_QUANT>{});
+        if (i + s + P < steps) {
+          wait_lds_reads();
+          load(s, c0 + i + s + P);
+        }
+      }
+  }
+  __syncthreads();
+
+  // the waves' shares are added up
+  float* red = reinterpret_cast<float*>(s_all);
+  #pragma unroll
+  for (int j = 0; j < FM; ++j)
+    #pragma unroll
+    for (int e = 0; e < 4; ++e)
+      red[(wave * BM + j * 16 + g * 4 + e) * (16 + PAD) + lo] = acc[j][e];
+  __syncthreads();
+  y += (long)blockIdx.y * MR * (GATED ? n / 2 : n);
+  for (int i = threadIdx.x; i < BM * 16; i += KW * WAVE) {
+    const int r = i / 16, c = i % 16;
+    if (r >= m || r >= MR) break;
+    auto sum = [&](int c) {
+      float v = 0.f;
+      #pragma unroll
+      for (int q = 0; q < KW; ++q) v += red[(q * BM + r) * (16 + PAD) + c];
+      return v;
+    };
+    if constexpr (GATED) {
+      if (c < 8)
+        y[(long)r * (n / 2) + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
+    } else {
+      if (n0 + c < n) y[(long)r * n + n0 + c] = f2bf(sum(c));
+    }
+  }
+}
+
+}  // namespace
+
+// Blocks whose scales come in pairs (k a multiple of 64), or of 256.
+bool rows_quant_takes(int m, int n, int k, Quant q, bool gated) {
+  const int step = q == Quant::Q4_K || q == Quant::Q6_K ? 256 : 64;
+  return m >= 1 && m <= 64 && n >= 1 && k >= step && k % step == 0 &&
+         (!gated || n % 16 == 0) && (m > 1 || q != Quant::Q8_0);
+}
+
+void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
+                       const unsigned char* qs, int m, int n, int k, Quant q,
+                       bool gated, hipStream_t stream) {
+  const f16_t* sc = reinterpret_cast<const f16_t*>(scales);
+  auto go = [&](auto qc, auto mr, auto me, auto kw, auto p) {
+    constexpr Quant QQ = decltype(qc)::value;
+    constexpr int MR = decltype(mr)::value, ME = decltype(me)::value,
+                  KW = decltype(kw)::value, P = decltype(p)::value;
+    const dim3 grid((n + 15) / 16, (m + MR - 1) / MR), block(KW * WAVE);
+    if (gated) {
+      rows_quant_kernel<QQ, MR, ME, KW, P, true>
+          <<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k);
+    } else {
+      rows_quant_kernel<QQ, MR, ME, KW, P, false>
+          <<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k);
+    }
+  };
+  auto by_rows = [&](auto qc) {
+    constexpr Quant QQ = decltype(qc)::value;
+    constexpr integral_constant<int, 1> c1{};
+    constexpr integral_constant<int, 4> c4{};
+    constexpr integral_constant<int, 8> c8{};
+    constexpr integral_constant<int, 16> c16{};
+    constexpr integral_constant<int, 32> c32{};
+    // stages in flight for few rows: q6_K's are the largest
+    constexpr integral_constant<int, QQ == Quant::Q6_K ? 1 : 2> few{};
+    if (m == 1) {
+      if constexpr (QQ == Quant::Q4_0) go(qc, c4, c1, c8, c1);
+      else if constexpr (QQ != Quant::Q8_0) go(qc, c4, c1, c4, few);
+    } else if (m <= 4) {
+      go(qc, c4, c4, c4, few);
+    } else if (m <= 8) {
+      go(qc, c8, c4, c4, few);
+    } else if (m <= 16) {
+      go(qc, c16, c4, c4, c1);
+    } else {
+      go(qc, c32, c4, c4, c1);
+    }
+  };
+  switch (q) {
+    case Quant::Q4_0:
+      by_rows(integral_constant<Quant, Quant::Q4_0>{});
+      break;
+    case Quant::Q8_0:
+      by_rows(integral_constant<Quant, Quant::Q8_0>{});
+      break;
+    case Quant::Q4_K:
+      by_rows(integral_constant<Quant, Quant::Q4_K>{});
+      break;
+    case Quant::Q6_K:
+      by_rows(integral_constant<Quant, Quant::Q6_K>{});
+      break;
+  }
+}

@@ -1,10 +1,11 @@
-"""Products of a few rows (rows_gemm.hip) against 64 bits, at
+"""Products of a few rows (rows_gemm.hip, rows_quant.hip) against 64 bits, at
 the sizes where their tiles, stages and shares of the inner dimension end."""
 
 import pytest
 import torch
 
 from substratus_amd import ops
+from substratus_amd.models.quant import QuantLinear
 from substratus_amd.parallel.tp import Linear
 
 pytestmark = pytest.mark.gpu
@@ -96,16 +97,55 @@ def test_linear_keeps_gradients():
     assert xx.grad is not None
 
 
+# stages of 256 columns: fewer than waves, a last one in part (q4_0, q8_0), a
+# ring's rounds; row tiles of x: 4, 8, 16, 32, twice 32
+@pytest.mark.parametrize("quant", ["q4_0", "q8_0", "q4_K", "q6_K"])
+@pytest.mark.parametrize("m", [1, 2, 4, 5, 8, 9, 16, 17, 33, 64])
+@pytest.mark.parametrize("n,k", [(16, 256), (41, 512), (48, 2304),
+                                 (64, 4352), (32, 64), (64, 4544),
+                                 (48, 1056)])
+@torch.no_grad()
+def test_quant_rows(quant, m, n, k):
+    if quant.endswith("_K") and k % 256:
+        pytest.skip("blocks of 256")
+    torch.manual_seed(m * 10000 + n + k)
+    lin = Linear(k, n, device=DEV, dtype=torch.bfloat16)
+    lin.weight.normal_(0.0, 0.5)
+    ql = QuantLinear.from_linear(lin, quant)
+    w = ql._dequant_cpu().to(DEV)
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    # weights unpacked to bf16 on the way (more rows than the vector kernel
+    # takes, blocks in odd numbers) are themselves half a step off
+    unpacked = k % 64 and m > 8
+    got = ql(x)
+    want = x.double() @ w.double().T
+    room = x.double().abs() @ w.double().abs().T
+    slack = (2.0 ** -9 if unpacked else 2.0 ** -18) * room
+    assert bool(((got.double() - want).abs()
+                 <= 2.0 ** -8 * want.abs() + slack).all())
+    # a view of qs that does not begin on 16 bytes
+    odd = torch.empty(ql.qs.numel() + 1, dtype=torch.uint8, device=DEV)[1:]
+    ql.qs = odd.view(ql.qs.shape).copy_(ql.qs)
+    if not k % 64:
+        assert torch.equal(ql(x), got)
+    if n % 16 == 0:
+        y = ql.gated(x)
+        want = gated(want)
+        assert bool(((y.double() - want).abs() <= 2.0 ** -7 * want.abs()
+                     + 2.0 ** -6 * room.mean()).all())
+
+
 @torch.no_grad()
 def test_products_of_few_rows_in_a_graph():
     """Replays with other inputs, eager work between."""
     torch.manual_seed(3)
     lin = Linear(512, 96, device=DEV, dtype=torch.bfloat16)
     lin.weight.normal_()
+    ql = QuantLinear.from_linear(lin, "q4_0")
     x = torch.randn(3, 512, device=DEV).bfloat16()
 
     def step():
-        return lin(x), lin.gated(x)
+        return lin(x), lin.gated(x), ql(x), ql.gated(x)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
