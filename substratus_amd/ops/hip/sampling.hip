@@ -1,24 +1,99 @@
 // Fused sampling kernel (SURVEY.md §2.5 ledger item 5): temperature / top-k /
 // top-p + inverse-CDF draw, one workgroup per logits row.
 //
-// The row (V bf16, e.g. 32000 for llama2 = 62.5 KiB) is staged once into LDS
-// and every subsequent pass (max, top-k threshold search, top-p mass search,
-// CDF scan) runs from LDS — HBM is touched exactly once per row. top-k uses a
-// binary search on the value domain counting x >= t (monotone in t); top-p
-// finds the smallest threshold whose masked exp-mass reaches p·Z. Both avoid
-// any sort (sampling runs once per decode step; the passes are LDS-bound).
+// A row is read once, 16 bytes per load, and stays in registers as
+// exp(x/T - max): a thread has 8 consecutive logits of every 8192. Thresholds
+// are searched over the logits' own ordered bit patterns, so that 16 steps
+// (32-bit logits: 32) end on an exact logit: top-k counts what is not below
+// (one comparison per logit, a wave's count out of its mask), top-p adds it
+// up. A step costs one barrier.
+//
+// Bound by the chain of steps; one row occupies a CU. On a MI355X, 192 rows
+// of 32000, a quarter each greedy and top-k, half top-p: 32 us (292 us with
+// the row in LDS, 256 threads and 24 halvings of the value range per
+// threshold). 256 rows of 65024: 18 us greedy, 42 without thresholds, 69 to 88
+// with them (registers spill from 32768 logits on).
 #include "common.h"
 
-#define SBLOCK 256
+#define SBLOCK 1024
 #define SNW (SBLOCK / WAVE)
+#define SVEC 8                    // consecutive logits of a thread per round
+#define SROUND (SBLOCK * SVEC)
 
-// LDS budget: V values (bf16: <= 65536 -> 128 KiB) + scratch.
-extern __shared__ unsigned char s_raw[];  // [V] logits as they came
+namespace {
 
 DEV_INLINE float val(const bf16_t& v) { return bf2f(v); }
 DEV_INLINE float val(const float& v) { return v; }
 
-template <class T>
+// Ordered bit patterns: a <= b as floats just if key(a) <= key(b).
+template <class T> struct Key;
+template <> struct Key<bf16_t> {
+  static constexpr unsigned TOP = 0x8000u, ALL = 0xffffu;
+  DEV_INLINE static unsigned bits(float f) { return __float_as_uint(f) >> 16; }
+  DEV_INLINE static float number(unsigned b) { return __uint_as_float(b << 16); }
+};
+template <> struct Key<float> {
+  static constexpr unsigned TOP = 0x80000000u, ALL = 0xffffffffu;
+  DEV_INLINE static unsigned bits(float f) { return __float_as_uint(f); }
+  DEV_INLINE static float number(unsigned b) { return __uint_as_float(b); }
+};
+template <class T> DEV_INLINE unsigned key_of(float f) {
+  const unsigned b = Key<T>::bits(f);
+  return b & Key<T>::TOP ? Key<T>::ALL ^ b : b | Key<T>::TOP;
+}
+template <class T> DEV_INLINE float of_key(unsigned k) {
+  return Key<T>::number(k & Key<T>::TOP ? k ^ Key<T>::TOP : Key<T>::ALL ^ k);
+}
+
+// VEC: the row is whole 16-byte pieces, of which each is there or not.
+template <class T, bool VEC>
+DEV_INLINE void load8(const T* row, int at, int vocab, float v[SVEC]) {
+  constexpr int PER = 16 / sizeof(T);
+  #pragma unroll
+  for (int p = 0; p < SVEC; p += PER) {
+    if constexpr (VEC) {
+      const int from = at + p < vocab ? at + p : 0;
+      const uint4v u = *reinterpret_cast<const uint4v*>(row + from);
+      #pragma unroll
+      for (int j = 0; j < PER; ++j)
+        v[p + j] = at + p >= vocab ? -INFINITY
+            : sizeof(T) == 4 ? __uint_as_float(u[j % 4])
+            : __uint_as_float(j & 1 ? u[j / 2] & 0xffff0000u : u[j / 2] << 16);
+    } else {
+      #pragma unroll
+      for (int j = 0; j < PER; ++j)
+        v[p + j] = at + p + j < vocab ? val(row[at + p + j]) : -INFINITY;
+    }
+  }
+}
+
+// The sum over the workgroup, in all threads: one barrier, and the next call
+// takes the other half of the scratch.
+struct Totals {
+  float (*s)[SNW];
+  int turn = 0;
+  DEV_INLINE float add(float wave_total) {
+    float* t = s[turn ^= 1];
+    if ((threadIdx.x & (WAVE - 1)) == 0) t[threadIdx.x / WAVE] = wave_total;
+    __syncthreads();
+    float v = 0.f;
+    #pragma unroll
+    for (int i = 0; i < SNW; ++i) v += t[i];
+    return v;
+  }
+  DEV_INLINE float most(float wave_most) {
+    float* t = s[turn ^= 1];
+    if ((threadIdx.x & (WAVE - 1)) == 0) t[threadIdx.x / WAVE] = wave_most;
+    __syncthreads();
+    float v = t[0];
+    #pragma unroll
+    for (int i = 1; i < SNW; ++i) v = fmaxf(v, t[i]);
+    return v;
+  }
+};
+
+// NR: rounds of 8192 logits that cover the row
+template <class T, int NR, bool VEC>
 __global__ __launch_bounds__(SBLOCK)
 void softmax_sample_kernel(long* __restrict__ out,          // [B]
                            const T* __restrict__ logits,  // [B, V]
@@ -26,177 +101,217 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
                            const int* __restrict__ top_k,
                            const float* __restrict__ top_p,
                            const float* __restrict__ uniform, int vocab) {
-  __shared__ float scratch[SNW];
-  __shared__ float s_bcast;
+  __shared__ float s_tot[2][SNW];
+  __shared__ float s_part[NR][SNW];
+  __shared__ int s_idx[SNW];
   __shared__ int s_tok;
-  const int b = blockIdx.x;
-  T* s_vals = reinterpret_cast<T*>(s_raw);
+  Totals totals{s_tot};
+  const int b = blockIdx.x, tid = threadIdx.x;
+  const int wave = tid / WAVE, lane = tid % WAVE;
   const T* row = logits + (long)b * vocab;
   const float temp = temperature[b];
-  const int tid = threadIdx.x;
 
-  // ---- greedy: argmax without staging --------------------------------
+  // the largest logit; the smallest index of several. NaN is passed over.
+  float e[NR][SVEC];
+  float best = -INFINITY;
+  int besti = 0x7fffffff;
+  #pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int at = r * SROUND + tid * SVEC;
+    load8<T, VEC>(row, at, vocab, e[r]);
+    #pragma unroll
+    for (int j = 0; j < SVEC; ++j)
+      if (e[r][j] > best) { best = e[r][j]; besti = at + j; }
+  }
+
+  // ---- greedy ---------------------------------------------------------
   if (temp <= 0.f) {
-    float best = -INFINITY;
-    int besti = 0;
-    for (int i = tid; i < vocab; i += SBLOCK) {
-      float v = val(row[i]);
-      if (v > best || (v == best && i < besti)) { best = v; besti = i; }
-    }
-    // wave reduce (value, index) preferring smaller index on ties
     #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
-      float ov = __shfl_xor(best, off, WAVE);
-      int oi = __shfl_xor(besti, off, WAVE);
+      const float ov = __shfl_xor(best, off, WAVE);
+      const int oi = __shfl_xor(besti, off, WAVE);
       if (ov > best || (ov == best && oi < besti)) { best = ov; besti = oi; }
     }
-    __shared__ float wv[SNW];
-    __shared__ int wi[SNW];
-    if ((tid & (WAVE - 1)) == 0) { wv[tid / WAVE] = best; wi[tid / WAVE] = besti; }
+    if (lane == 0) { s_tot[0][wave] = best; s_idx[wave] = besti; }
     __syncthreads();
     if (tid == 0) {
       for (int w = 1; w < SNW; ++w)
-        if (wv[w] > wv[0] || (wv[w] == wv[0] && wi[w] < wi[0])) {
-          wv[0] = wv[w]; wi[0] = wi[w];
+        if (s_tot[0][w] > best || (s_tot[0][w] == best && s_idx[w] < besti)) {
+          best = s_tot[0][w];
+          besti = s_idx[w];
         }
-      out[b] = wi[0];
+      out[b] = besti < vocab ? besti : 0;
     }
     return;
   }
 
-  // ---- stage the ORIGINAL logits into LDS + row max -------------------
-  // (temperature is applied in fp32 at every read: staging pre-scaled bf16
-  // would re-quantize x/T and shift CDF boundaries vs the fp32 reference)
+  // temperature is applied in fp32, to the logits as they came
   const float inv_t = 1.f / temp;
-  float mx = -INFINITY;
-  for (int i = tid; i < vocab; i += SBLOCK) {
-    s_vals[i] = row[i];
-    mx = fmaxf(mx, val(s_vals[i]) * inv_t);
-  }
-  __syncthreads();
-  float m = block_max<SNW>(mx, scratch);
-  __syncthreads();
+  const float top = totals.most(wave_max(best));
+  const float m = top * inv_t;
+  auto weight = [&](float v) {       // NaN, and what is below all others: 0
+    const float x = v * inv_t, below = __expf(x - m);
+    return v == top ? 1.f : x < m ? below : 0.f;
+  };
+  #pragma unroll
+  for (int r = 0; r < NR; ++r)
+    #pragma unroll
+    for (int j = 0; j < SVEC; ++j) {
+      const int at = r * SROUND + tid * SVEC + j;
+      e[r][j] = at < vocab ? weight(e[r][j]) : -1.f;    // -1: not a token
+      // one after the other, or their parts take the registers of the row
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  const unsigned first = key_of<T>(-INFINITY), last = key_of<T>(top);
+  // the largest key whose logits and all above them satisfy enough(their
+  // weight's threshold)
+  auto search = [&](auto enough) {
+    unsigned lo = first, hi = last + 1;     // holds at lo, not at hi
+    while (hi - lo > 1) {
+      const unsigned mid = lo + (hi - lo) / 2;
+      if (enough(weight(of_key<T>(mid)))) lo = mid; else hi = mid;
+    }
+    return lo;
+  };
+  auto sum_from = [&](float t) {
+    float s = 0.f;
+    #pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      #pragma unroll
+      for (int j = 0; j < SVEC; ++j) s += e[r][j] >= t ? e[r][j] : 0.f;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return totals.add(wave_sum(s));
+  };
 
-  // ---- top-k: binary search threshold on value domain -----------------
-  float thresh = -INFINITY;
+  // ---- top-k: as many largest as are no more than k with all their equals,
+  // ---- the largest and its equals in any case
+  float thresh = 0.f;
   const int k = top_k[b];
   if (k > 0 && k < vocab) {
-    float lo = m - 64.f, hi = m;  // exp(-64) underflows anyway
-    for (int it = 0; it < 24; ++it) {
-      float mid = 0.5f * (lo + hi);
-      int cnt = 0;
-      for (int i = tid; i < vocab; i += SBLOCK) {
-        if (val(s_vals[i]) * inv_t >= mid) ++cnt;
+    const unsigned more = search([&](float t) {
+      int n = 0;
+      #pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        #pragma unroll
+        for (int j = 0; j < SVEC; ++j)
+          n += __popcll(__ballot(e[r][j] >= t));
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __syncthreads();
-      int total = (int)block_sum<SNW>((float)cnt, scratch);
-      __syncthreads();
-      if (total > k) lo = mid; else hi = mid;
-    }
-    // lo converges to v_{k+1} (count>k), hi to just above it (count<=k):
-    // x >= hi keeps exactly the top-k values, ties at v_k included.
-    thresh = hi;
+      return totals.add((float)n) > (float)k;
+    });
+    thresh = weight(of_key<T>(min(more + 1, last)));
   }
 
-  // ---- exp-sum over kept values ---------------------------------------
-  float zs = 0.f;
-  for (int i = tid; i < vocab; i += SBLOCK) {
-    float v = val(s_vals[i]) * inv_t;
-    if (v >= thresh) zs += __expf(v - m);
-  }
-  __syncthreads();
-  float z = block_sum<SNW>(zs, scratch);
-  __syncthreads();
-
-  // ---- top-p: binary search the prob-mass threshold -------------------
+  // ---- top-p: the fewest largest weights with that share ----------------
   const float p_target = top_p[b];
   if (p_target > 0.f && p_target < 1.f) {
-    float lo = thresh == -INFINITY ? m - 64.f : thresh, hi = m;
-    for (int it = 0; it < 24; ++it) {
-      float mid = 0.5f * (lo + hi);
-      float ms = 0.f;
-      for (int i = tid; i < vocab; i += SBLOCK) {
-        float v = val(s_vals[i]) * inv_t;
-        if (v >= mid && v >= thresh) ms += __expf(v - m);
-      }
-      __syncthreads();
-      float mass = block_sum<SNW>(ms, scratch);
-      __syncthreads();
-      if (mass >= p_target * z) lo = mid; else hi = mid;
-    }
-    thresh = fmaxf(thresh, lo);
-    // recompute z over the kept set
-    float zs2 = 0.f;
-    for (int i = tid; i < vocab; i += SBLOCK) {
-      float v = val(s_vals[i]) * inv_t;
-      if (v >= thresh) zs2 += __expf(v - m);
-    }
-    __syncthreads();
-    z = block_sum<SNW>(zs2, scratch);
-    __syncthreads();
+    const float goal = p_target * sum_from(thresh);
+    const float low = thresh;
+    thresh = fmaxf(low, weight(of_key<T>(search([&](float t) {
+      return t < low || sum_from(t) >= goal;
+    }))));
   }
 
-  // ---- inverse-CDF draw ------------------------------------------------
-  const float r = uniform[b] * z;
-  // per-thread chunk sums in token order: thread t owns [t*chunk, (t+1)*chunk)
-  const int chunk = (vocab + SBLOCK - 1) / SBLOCK;
-  const int beg = tid * chunk, end = min(beg + chunk, vocab);
-  float csum = 0.f;
-  for (int i = beg; i < end; ++i) {
-    float v = val(s_vals[i]) * inv_t;
-    if (v >= thresh) csum += __expf(v - m);
+  // ---- inverse-CDF draw, in token order ---------------------------------
+  float mine[NR];
+  #pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    mine[r] = 0.f;
+    #pragma unroll
+    for (int j = 0; j < SVEC; ++j)
+      mine[r] += e[r][j] >= thresh ? e[r][j] : 0.f;
+    const float t = wave_sum(mine[r]);
+    if (lane == 0) s_part[r][wave] = t;
+    __builtin_amdgcn_sched_barrier(0);
   }
-  // exclusive prefix over the 256 per-thread sums (via LDS, simple scan)
-  __shared__ float pre[SBLOCK + 1];
-  pre[tid + 1] = csum;
-  if (tid == 0) pre[0] = 0.f;
+  if (tid == 0) s_tok = -1;
   __syncthreads();
-  if (tid == 0) {
-    for (int i = 1; i <= SBLOCK; ++i) pre[i] += pre[i - 1];
-    s_tok = -1;
+  float z = 0.f;
+  for (int q = 0; q < NR * SNW; ++q) z += s_part[q / SNW][q % SNW];
+  const float goal = uniform[b] * z;
+  float before = 0.f;
+  int part = -1;              // round and wave in which the sum reaches goal
+  #pragma unroll 8
+  for (int q = 0; q < NR * SNW; ++q) {
+    const float t = s_part[q / SNW][q % SNW];
+    if (part < 0) {
+      if (before + t > goal) part = q; else before += t;
+    }
   }
-  __syncthreads();
-  // the thread whose [pre[tid], pre[tid+1]) straddles r walks its chunk
-  if (r >= pre[tid] && r < pre[tid + 1]) {
-    float acc = pre[tid];
-    int sel = -1;
-    for (int i = beg; i < end; ++i) {
-      float v = val(s_vals[i]) * inv_t;
-      if (v >= thresh) {
-        acc += __expf(v - m);
-        if (acc > r) { sel = i; break; }
+  #pragma unroll
+  for (int r = 0; r < NR; ++r)
+    if (part == r * SNW + wave) {
+      float upto = mine[r];     // with the lanes before
+      #pragma unroll
+      for (int off = 1; off < WAVE; off <<= 1) {
+        const float o = __shfl_up(upto, off, WAVE);
+        if (lane >= off) upto += o;
+      }
+      const float end = before + upto;
+      const unsigned long long over = __ballot(end > goal);
+      const int who = over ? __ffsll(over) - 1 : WAVE - 1;
+      if (lane == who) {
+        float acc = end - mine[r];
+        int sel = -1;
+        #pragma unroll
+        for (int j = 0; j < SVEC; ++j)
+          if (e[r][j] >= thresh) {
+            // the lane's last one where rounding leaves the sum short
+            if (sel < 0 || acc <= goal) sel = r * SROUND + tid * SVEC + j;
+            acc += e[r][j];
+          }
+        s_tok = sel;
       }
     }
-    if (sel >= 0) s_tok = sel;
+  __syncthreads();
+  if (s_tok >= 0) {
+    if (tid == 0) out[b] = s_tok;
+    return;
   }
+  // rounding at the very end (goal ~ z): the last token that may be drawn
+  int kept = -1;
+  #pragma unroll
+  for (int r = 0; r < NR; ++r)
+    #pragma unroll
+    for (int j = 0; j < SVEC; ++j)
+      if (e[r][j] >= thresh) kept = r * SROUND + tid * SVEC + j;
+  #pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    kept = max(kept, __shfl_xor(kept, off, WAVE));
+  if (lane == 0) s_idx[wave] = kept;
   __syncthreads();
   if (tid == 0) {
-    int sel = s_tok;
-    if (sel < 0) {
-      // numerical edge (r ~ z): fall back to the last kept token
-      for (int i = vocab - 1; i >= 0; --i) {
-        if (val(s_vals[i]) * inv_t >= thresh) { sel = i; break; }
-      }
-    }
-    out[b] = sel < 0 ? 0 : sel;
+    for (int w = 1; w < SNW; ++w) kept = max(kept, s_idx[w]);
+    out[b] = max(kept, 0);
   }
 }
 
 template <class T>
-static void launch(long* out, const T* logits, const float* temperature,
-                   const int* top_k, const float* top_p, const float* uniform,
-                   int bsz, int vocab, hipStream_t stream) {
-  size_t lds = (size_t)vocab * sizeof(T);
-  static size_t max_opted = 0;
-  if (lds > 65536 && lds > max_opted) {  // opt in to >64 KiB dynamic LDS
-    (void)hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&softmax_sample_kernel<T>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    max_opted = lds;
-  }
-  softmax_sample_kernel<T><<<dim3(bsz), dim3(SBLOCK), lds, stream>>>(
-      out, logits, temperature, top_k, top_p, uniform, vocab);
+void launch(long* out, const T* logits, const float* temperature,
+            const int* top_k, const float* top_p, const float* uniform,
+            int bsz, int vocab, hipStream_t stream) {
+  const bool vec = vocab * sizeof(T) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(logits) % 16 == 0;
+  auto go = [&](auto nr) {
+    constexpr int NR = decltype(nr)::value;
+    if (vec) {
+      softmax_sample_kernel<T, NR, true>
+          <<<dim3(bsz), dim3(SBLOCK), 0, stream>>>(
+              out, logits, temperature, top_k, top_p, uniform, vocab);
+    } else {
+      softmax_sample_kernel<T, NR, false>
+          <<<dim3(bsz), dim3(SBLOCK), 0, stream>>>(
+              out, logits, temperature, top_k, top_p, uniform, vocab);
+    }
+  };
+  if (vocab <= SROUND) go(std::integral_constant<int, 1>{});
+  else if (vocab <= 4 * SROUND) go(std::integral_constant<int, 4>{});
+  else if (vocab <= 7 * SROUND) go(std::integral_constant<int, 7>{});
+  else go(std::integral_constant<int, 10>{});
 }
+
+}  // namespace
 
 void launch_softmax_sample(long* out, const bf16_t* logits,
                            const float* temperature, const int* top_k,

@@ -1,0 +1,85 @@
+"""The sampling kernel against 64 bits: which tokens may be drawn, and which
+one a number in [0, 1) stands for, at sizes where its rounds and loads end."""
+
+import pytest
+import torch
+
+from substratus_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def draw(logits, t, k, p, u):
+    """(tokens that may be drawn, cumulated weights in token order, draw)."""
+    x = logits.double() / t
+    x = x.nan_to_num(nan=-torch.inf, posinf=torch.inf, neginf=-torch.inf)
+    w = torch.where(x == x.max(), 1.0, torch.exp(x - x.max()))
+    keep = ~logits.isnan()
+    if 0 < k < len(x):      # equals go together, the largest in any case
+        below = x.topk(k + 1).values[-1]
+        keep &= (x > below) | (x == x.max())
+    if 0 < p < 1:
+        goal = p * w[keep].sum()
+        by_size, at = w.masked_fill(~keep, 0).sort(descending=True)
+        n = int((by_size.cumsum(0) < goal * (1 - 1e-6)).sum())
+        keep &= w >= by_size[min(n, len(x) - 1)] * (1 - 1e-9)
+    w = w.masked_fill(~keep, 0)
+    return keep, w.cumsum(0), u * w.sum()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1, 7, 8, 1000, 8191, 8192, 8200, 32769,
+                                   39936, 50257, 57352, 79872])
+def test_draws(vocab, dtype):
+    if vocab * dtype.itemsize > 156 * 1024:
+        pytest.skip("refused: larger than a workgroup's memory")
+    torch.manual_seed(vocab)
+    settings = [(1.0, 0, 1.0), (0.7, 1, 1.0), (0.9, 40, 1.0), (1.3, 0, 0.9),
+                (0.5, 30, 0.5), (1.0, vocab - 1, 0.999), (2.0, 5000, 0.3)]
+    n = 8 * len(settings)
+    logits = (torch.randn(n, vocab, device=DEV) * 3).to(dtype)
+    u = torch.rand(n, device=DEV)
+    u[0], u[1] = 0.0, 1.0 - 2.0 ** -24
+    t, k, p = (torch.tensor([settings[i % len(settings)][j]
+                             for i in range(n)], device=DEV)
+               for j in range(3))
+    got = ops.softmax_sample(logits, t, k.int(), p, u).tolist()
+    for i in range(n):
+        keep, cum, goal = draw(logits[i].cpu(), float(t[i]), int(k[i]),
+                               float(p[i]), float(u[i]))
+        a = got[i]
+        assert 0 <= a < vocab and bool(keep[a])
+        # 32-bit sums of weights: 2^-24 per addend, of which a thread has at
+        # most 80 in a row and partial sums a few hundred
+        slack = 2e-5 * float(cum[-1])
+        assert float(cum[a]) >= float(goal) - slack
+        assert a == 0 or float(cum[a - 1]) <= float(goal) + slack
+
+
+def test_rows_that_are_not_ordinary():
+    """The smallest index of several largest; NaN and -inf are never drawn;
+    an infinite logit always is; rows of one value."""
+    v = 20000
+    rows = torch.randn(6, v, device=DEV).bfloat16()
+    rows[0, 5000] = rows[0, 12345] = 50.0
+    rows[1] = -torch.inf
+    rows[1, 17] = 1.0
+    rows[2, ::2] = torch.nan
+    rows[3, 777] = torch.inf
+    rows[4] = 3.0
+    rows[5, 1:] = -torch.inf
+    for temp in (0.0, 0.8):
+        t = torch.full((6,), temp, device=DEV)
+        for k, p in ((0, 1.0), (3, 1.0), (0, 0.5)):
+            got = ops.softmax_sample(
+                rows, t, torch.full((6,), k, device=DEV).int(),
+                torch.full((6,), p, device=DEV),
+                torch.full((6,), 0.4, device=DEV)).tolist()
+            assert got[0] == 5000 if temp == 0 else got[0] in (5000, 12345)
+            assert got[1] == 17 and got[2] % 2 == 1 and got[3] == 777
+            assert got[5] == 0
+            if temp == 0:
+                assert got[4] == 0
+            elif p == 1:
+                assert abs(got[4] - 0.4 * v) <= 1
