@@ -24,6 +24,8 @@
 // int32; seq_lens [B] int32 counts INCLUDING the current token.
 #include "common.h"
 
+#include <algorithm>
+
 #define BS 16   // tokens per KV block
 #define NW 4    // waves per workgroup
 
@@ -883,19 +885,32 @@ void paged_attn_reduce_kernel(bf16_t* __restrict__ out,      // [B, HQ, D]
   const int qh = blockIdx.y;
   const int lane = threadIdx.x;
   const long base = ((long)b * hq + qh) * nsplit;
-  float M = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, part_ml[(base + s) * 2]);
-  float L = 0.f;
+  // nsplit <= 16: a lane has a share's maximum and sum; the shares' rows are
+  // loaded together (7.1 us one after the other, 4.5 so, 16 heads x 16)
+  float pm = -INFINITY, pl = 0.f;
+  if (lane < nsplit) {
+    pm = part_ml[(base + lane) * 2];
+    pl = part_ml[(base + lane) * 2 + 1];
+  }
+  float v[16][DPL];
+  #pragma unroll
+  for (int s = 0; s < 16; ++s)
+    #pragma unroll
+    for (int j = 0; j < DPL; ++j)
+      v[s][j] = part_o[(base + min(s, nsplit - 1)) * D + lane * DPL + j];
+  const float M = wave_max(pm);
+  const float f = pm == -INFINITY ? 0.f : __expf(pm - M);
+  const float L = wave_sum(f * pl);
   float o[DPL];
   #pragma unroll
   for (int j = 0; j < DPL; ++j) o[j] = 0.f;
-  for (int s = 0; s < nsplit; ++s) {
-    const float pm = part_ml[(base + s) * 2];
-    const float f = (pm == -INFINITY) ? 0.f : __expf(pm - M);
-    L += f * part_ml[(base + s) * 2 + 1];
-    const float* po = part_o + (base + s) * D;
-    #pragma unroll
-    for (int j = 0; j < DPL; ++j) o[j] += f * po[lane * DPL + j];
+  #pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    const float fs = __shfl(f, s, WAVE);
+    if (s < nsplit) {
+      #pragma unroll
+      for (int j = 0; j < DPL; ++j) o[j] += fs * v[s][j];
+    }
   }
   const float invl = (L > 0.f) ? 1.f / L : 0.f;
   bf16_t* orow = out + ((long)b * hq + qh) * D;
@@ -907,23 +922,26 @@ void paged_attn_reduce_kernel(bf16_t* __restrict__ out,      // [B, HQ, D]
   }
 }
 
-int paged_attn_nsplit(int bsz, int hq, int hkv, int d) {
+// attention_decode_group.hip
+bool attn_group_takes(int hq, int hkv, int d, long q_ld, const void* q,
+                      const void* kc, const void* vc);
+void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
+                       const bf16_t* vc, const int* block_table,
+                       const int* seq_lens, int bsz, int hq, int hkv, int d,
+                       int max_blocks, float scale, long q_ld, int nsplit,
+                       float* part_o, float* part_ml, hipStream_t stream);
+
+int paged_attn_nsplit(int bsz, int hq, int hkv, int d, int max_blocks) {
   // flash-decoding split factor: fill >=1024 workgroups (256 CUs x 4
   // resident WGs) when the (B, Hkv, group-chunk) grid alone is too small
   // (llama2-70b at TP=8: B x 1 x 1). Shape-only -> hipGraph-stable.
-  const int group = hq / hkv;
-  int gchunks;
-  if (gqa_hpw(hq, hkv, d) > 0) {
-    gchunks = 1;                       // whole group lives in one block
-  } else {
-    const int gc = (group % 8 == 0) ? 8 : 1;
-    gchunks = (group + gc - 1) / gc;
-  }
-  const long base = (long)bsz * hkv * gchunks;
+  const long base = (long)bsz * hkv * ((hq / hkv + 15) / 16);
   if (base >= 1024) return 1;
   int ns = (int)((1024 + base - 1) / base);
   if (ns > 16) ns = 16;
-  return ns;
+  // four waves of a workgroup take a page each: no more shares than the
+  // longest sequence that the table has room for has pages for
+  return std::max(1, std::min(ns, (max_blocks + NW - 1) / NW));
 }
 
 void launch_paged_attn_decode(bf16_t* out, const bf16_t* q,
@@ -936,11 +954,17 @@ void launch_paged_attn_decode(bf16_t* out, const bf16_t* q,
   const int group = hq / hkv;
   const int hpw = gqa_hpw(hq, hkv, d);
   dim3 block(NW * WAVE);
-  if (hpw > 0) {
+  // SUB_DECODE_GQA=scalar, or anything else: the older kernels, which a cache
+  // of fp8 takes
+  static const char* ge = getenv("SUB_DECODE_GQA");
+  if (!kv8 && !ge && attn_group_takes(hq, hkv, d, q_rstride, q, k_cache,
+                                       v_cache)) {
+    launch_attn_group(out, q, reinterpret_cast<const bf16_t*>(k_cache),
+                      reinterpret_cast<const bf16_t*>(v_cache), block_table,
+                      seq_lens, bsz, hq, hkv, d, max_blocks, scale, q_rstride,
+                      nsplit, part_o, part_ml, stream);
+  } else if (hpw > 0) {
     dim3 grid(bsz, hkv, nsplit);
-    // default: the MFMA variant (group on the M dim); SUB_DECODE_GQA=scalar
-    // selects the scalar LDS-staged kernel for A/B measurement
-    static const char* ge = getenv("SUB_DECODE_GQA");
     static const bool scalar_gqa = ge && ge[0] == 's';
     if (!scalar_gqa) {
       #define LAUNCHM(DD, K8) \
