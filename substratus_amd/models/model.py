@@ -27,6 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..ops import train as train_ops
 from ..parallel.comm import state
 from ..parallel.tp import ColumnParallelLinear, Linear, RowParallelLinear
 from .config import ModelConfig
@@ -212,87 +213,40 @@ class Block(nn.Module):
         return h + self._mlp(self.norm2(h, self.eps))
 
     # -- train (dense, differentiable) --------------------------------------
-    def forward_train(self, h: torch.Tensor, cos: torch.Tensor,
-                      sin: torch.Tensor) -> torch.Tensor:
-        cfg = self.cfg
-        if self.norm1.rms:
-            y = F.rms_norm(h.float(), (cfg.hidden_size,),
-                           self.norm1.weight.float(), self.eps).to(h.dtype)
-        else:
-            y = F.layer_norm(h.float(), (cfg.hidden_size,),
-                             self.norm1.weight.float(),
-                             self.norm1.bias.float(), self.eps).to(h.dtype)
-        b, s, _ = y.shape
-        d = cfg.head_dim
-        q, k, v = self.wqkv(y).split(
-            [self.n_heads * d, self.n_kv_heads * d, self.n_kv_heads * d], dim=-1)
-        if (h.is_cuda and h.dtype == torch.bfloat16
-                and ops.flash_attn_train_available(d)):
-            # first-party MFMA flash fwd+bwd (attention_prefill.hip /
-            # attention_bwd.hip): BSHD layout end-to-end — no transposes,
-            # no GQA head materialization, no torch-SDPA/aotriton on the
-            # trainer hot path
-            q = q.view(b, s, self.n_heads, d)
-            k = k.view(b, s, self.n_kv_heads, d)
-            v = v.view(b, s, self.n_kv_heads, d)
-            if self.rope_theta > 0:
-                q = _rope_train(q, cos, sin, bshd=True)
-                k = _rope_train(k, cos, sin, bshd=True)
-            a = ops.flash_attn_train(q, k, v, self.scale)
-            a = a.reshape(b, s, self.n_heads * d)
-        else:
-            q = q.view(b, s, self.n_heads, d).transpose(1, 2)
-            k = k.view(b, s, self.n_kv_heads, d).transpose(1, 2)
-            v = v.view(b, s, self.n_kv_heads, d).transpose(1, 2)
-            if self.rope_theta > 0:
-                q = _rope_train(q, cos, sin)
-                k = _rope_train(k, cos, sin)
-            if self.n_kv_heads != self.n_heads:
-                rep = self.n_heads // self.n_kv_heads
-                k = k.repeat_interleave(rep, dim=1)
-                v = v.repeat_interleave(rep, dim=1)
-            a = F.scaled_dot_product_attention(q, k, v, is_causal=True)
-            a = a.transpose(1, 2).reshape(b, s, self.n_heads * d)
-        attn_out = self.wo(a)
+    def forward_train(self, h: torch.Tensor, deltas: tuple,
+                      cos: Optional[torch.Tensor],
+                      sin: Optional[torch.Tensor]) -> tuple:
+        """(h, deltas): the residual stream and what is still to be added to
+        it, which the next norm does; the same is returned."""
+        y, h = train_ops.add_norm(h, deltas, self.norm1.weight,
+                                  self.norm1.bias, self.eps)
+        if self.rope_theta <= 0:
+            cos = sin = None
+        attn_out = self.wo(train_ops.attend(
+            self.wqkv(y), cos, sin, self.n_heads, self.n_kv_heads,
+            self.scale))
         if self.parallel_attn:
             if self.parallel_norms:
-                y_mlp = F.layer_norm(h.float(), (cfg.hidden_size,),
-                                     self.norm2.weight.float(),
-                                     self.norm2.bias.float(),
-                                     self.eps).to(h.dtype)
-            else:
-                y_mlp = y
-            return h + attn_out + self._mlp_train(y_mlp)
-        h = h + attn_out
-        if self.norm2.rms:
-            y2 = F.rms_norm(h.float(), (cfg.hidden_size,),
-                            self.norm2.weight.float(), self.eps).to(h.dtype)
-        else:
-            y2 = F.layer_norm(h.float(), (cfg.hidden_size,),
-                              self.norm2.weight.float(),
-                              self.norm2.bias.float(), self.eps).to(h.dtype)
-        return h + self._mlp_train(y2)
+                y, _ = train_ops.add_norm(h, (), self.norm2.weight,
+                                          self.norm2.bias, self.eps)
+            return h, (attn_out, self._mlp_train(y))
+        y, h = train_ops.add_norm(h, (attn_out,), self.norm2.weight,
+                                  self.norm2.bias, self.eps)
+        return h, (self._mlp_train(y),)
+
+    def whole_train(self, h: torch.Tensor, cos: Optional[torch.Tensor],
+                    sin: Optional[torch.Tensor]) -> torch.Tensor:
+        """forward_train with its additions done, so that one tensor is kept
+        between recomputed blocks."""
+        h, deltas = self.forward_train(h, (), cos, sin)
+        for d in deltas:
+            h = h + d
+        return h
 
     def _mlp_train(self, y: torch.Tensor) -> torch.Tensor:
         if self.cfg.activation == "silu":
-            gu = self.w_gateup(y)
-            g, u = gu.chunk(2, dim=-1)
-            return self.w_down(F.silu(g) * u)
+            return self.w_down(train_ops.silu_mul(self.w_gateup(y)))
         return self.w_down(F.gelu(self.w_up(y), approximate="tanh"))
-
-
-def _rope_train(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                bshd: bool = False) -> torch.Tensor:
-    # x: [B, H, S, D] (or [B, S, H, D] when bshd); cos/sin: [S, D/2]
-    d = x.shape[-1]
-    x1, x2 = x[..., : d // 2], x[..., d // 2:]
-    if bshd:
-        c = cos[None, :, None, :]
-        s = sin[None, :, None, :]
-    else:
-        c = cos[None, None, :, :]
-        s = sin[None, None, :, :]
-    return torch.cat([x1 * c - x2 * s, x2 * c + x1 * s], dim=-1).to(x.dtype)
 
 
 class CausalLM(nn.Module):
@@ -407,18 +361,14 @@ class CausalLM(nn.Module):
             cos, sin = cos.to(h.device), sin.to(h.device)
         else:
             cos = sin = None
+        deltas = ()
         for blk in self.blocks:
             if self.gradient_checkpointing and h.requires_grad is not False \
                     and torch.is_grad_enabled():
                 h = torch.utils.checkpoint.checkpoint(
-                    blk.forward_train, h, cos, sin, use_reentrant=False)
+                    blk.whole_train, h, cos, sin, use_reentrant=False)
             else:
-                h = blk.forward_train(h, cos, sin)
-        if self.final_norm.rms:
-            h = F.rms_norm(h.float(), (self.cfg.hidden_size,),
-                           self.final_norm.weight.float(), self.eps).to(h.dtype)
-        else:
-            h = F.layer_norm(h.float(), (self.cfg.hidden_size,),
-                             self.final_norm.weight.float(),
-                             self.final_norm.bias.float(), self.eps).to(h.dtype)
-        return self._logits(h)
+                h, deltas = blk.forward_train(h, deltas, cos, sin)
+        y, _ = train_ops.add_norm(h, deltas, self.final_norm.weight,
+                                  self.final_norm.bias, self.eps)
+        return self._logits(y)

@@ -32,6 +32,13 @@ bool attn_bwd_supported(int);
 void launch_attn_prefill_probe(int, bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, int, int, int, int, float, hipStream_t);
 void launch_mfma_probe(float*, const bf16_t*, const bf16_t*, hipStream_t);
 void launch_mfma32_probe(float*, const bf16_t*, const bf16_t*, hipStream_t);
+bool train_norm_takes(int);
+int train_norm_shares(long);
+void launch_add_norm_fwd(bf16_t*, bf16_t*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, long, int, float, bool, hipStream_t);
+void launch_add_norm_bwd(bf16_t*, bf16_t*, bf16_t*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const bf16_t*, long, int, bool, hipStream_t);
+void launch_rope_split(bf16_t*, bf16_t*, bf16_t*, const bf16_t*, const float*, const float*, long, int, int, int, int, hipStream_t);
+void launch_rope_join(bf16_t*, const bf16_t*, const float*, const float*, const float*, const float*, long, int, int, int, int, hipStream_t);
+void launch_silu_mul_bwd(bf16_t*, const bf16_t*, const bf16_t*, long, int, hipStream_t);
 void launch_softmax_sample(long*, const bf16_t*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
 void launch_softmax_sample(long*, const float*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
 void launch_cross_entropy(float*, bf16_t*, const bf16_t*, const long*, long, int, long, float, hipStream_t);
@@ -89,6 +96,124 @@ bool aligned16(const torch::Tensor& t) {
 void post_launch_check(const char* op) {
   hipError_t e = hipGetLastError();
   TORCH_CHECK(e == hipSuccess, op, ": HIP launch failed: ", hipGetErrorString(e));
+}
+
+// bf16, contiguous, of n elements and on 16-byte boundaries
+void check_rows(const torch::Tensor& t, long n, const char* name) {
+  check_bf16(t, name);
+  TORCH_CHECK(t.numel() == n, name, " has ", t.numel(), " elements, not ", n);
+  TORCH_CHECK(aligned16(t), name, " must be on a 16-byte boundary");
+}
+
+void check_rows32(const torch::Tensor& t, long n, const char* name) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat &&
+                  t.is_contiguous() && aligned16(t) && t.numel() == n,
+              name, " must be ", n, " contiguous floats on GPU");
+}
+
+// y = norm(h + d1 + d2), sum = h + d1 + d2 (d1, d2 and with them sum may be
+// absent; without bias it is RMS)
+void add_norm_fwd(torch::Tensor y, c10::optional<torch::Tensor> sum,
+                  torch::Tensor stats, torch::Tensor h,
+                  c10::optional<torch::Tensor> d1,
+                  c10::optional<torch::Tensor> d2, torch::Tensor w,
+                  c10::optional<torch::Tensor> b, double eps) {
+  const long n = h.numel(), hidden = w.numel();
+  TORCH_CHECK(n > 0 && train_norm_takes(hidden) && n % hidden == 0,
+              "width ", hidden, " not taken");
+  check_rows(y, n, "y"); check_rows(h, n, "h"); check_rows(w, hidden, "w");
+  TORCH_CHECK(d1.has_value() == sum.has_value() && (d1 || !d2), "operands");
+  if (d1) { check_rows(*d1, n, "d1"); check_rows(*sum, n, "sum"); }
+  if (d2) check_rows(*d2, n, "d2");
+  if (b) check_rows(*b, hidden, "b");
+  check_rows32(stats, 2 * (n / hidden), "stats");
+  launch_add_norm_fwd(bf(y), sum ? bf(*sum) : nullptr,
+                      stats.data_ptr<float>(), bfc(h), d1 ? bfc(*d1) : nullptr,
+                      d2 ? bfc(*d2) : nullptr, bfc(w), b ? bfc(*b) : nullptr,
+                      n / hidden, hidden, (float)eps, !b, stream());
+  post_launch_check("add_norm_fwd");
+}
+
+// db tells LayerNorm from RMS
+void add_norm_bwd(torch::Tensor dh, torch::Tensor dw,
+                  c10::optional<torch::Tensor> db, torch::Tensor dy,
+                  c10::optional<torch::Tensor> dres, torch::Tensor x,
+                  torch::Tensor stats, torch::Tensor w) {
+  const long n = x.numel(), hidden = w.numel();
+  TORCH_CHECK(n > 0 && train_norm_takes(hidden) && n % hidden == 0,
+              "width ", hidden, " not taken");
+  check_rows(dh, n, "dh"); check_rows(dy, n, "dy"); check_rows(x, n, "x");
+  check_rows(w, hidden, "w"); check_rows(dw, hidden, "dw");
+  if (dres) check_rows(*dres, n, "dres");
+  if (db) check_rows(*db, hidden, "db");
+  check_rows32(stats, 2 * (n / hidden), "stats");
+  auto shares = torch::empty(
+      {(db ? 2 : 1) * train_norm_shares(n / hidden) * hidden},
+      stats.options());
+  launch_add_norm_bwd(bf(dh), bf(dw), db ? bf(*db) : nullptr,
+                      shares.data_ptr<float>(), bfc(dy),
+                      dres ? bfc(*dres) : nullptr, bfc(x),
+                      stats.data_ptr<float>(), bfc(w), n / hidden, hidden,
+                      !db, stream());
+  post_launch_check("add_norm_bwd");
+}
+
+void check_angles(const c10::optional<torch::Tensor>& c,
+                  const c10::optional<torch::Tensor>& s, long rows,
+                  long length, long d) {
+  // a head's threads have to divide a workgroup's
+  TORCH_CHECK(d == 16 || d == 32 || d == 64 || d == 128 || d == 256,
+              "head_dim ", d, " not taken");
+  TORCH_CHECK(rows > 0 && length > 0 && rows % length == 0, "rows");
+  TORCH_CHECK(c.has_value() == s.has_value(), "angles");
+  if (c) {
+    check_rows32(*c, length * (d / 2), "cos");
+    check_rows32(*s, length * (d / 2), "sin");
+  }
+}
+
+// qkv rows into q, k, v, turned by the angles of row % length (none: copied)
+void rope_split(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                torch::Tensor qkv, c10::optional<torch::Tensor> c,
+                c10::optional<torch::Tensor> s, long length) {
+  TORCH_CHECK(q.dim() == 3 && k.dim() == 3, "q, k are [rows, heads, d]");
+  const long rows = q.size(0), hq = q.size(1), hkv = k.size(1), d = q.size(2);
+  check_angles(c, s, rows, length, d);
+  check_rows(q, rows * hq * d, "q"); check_rows(k, rows * hkv * d, "k");
+  check_rows(v, rows * hkv * d, "v");
+  check_rows(qkv, rows * (hq + 2 * hkv) * d, "qkv");
+  launch_rope_split(bf(q), bf(k), bf(v), bfc(qkv),
+                    c ? c->data_ptr<float>() : nullptr,
+                    s ? s->data_ptr<float>() : nullptr, rows, length, hq, hkv,
+                    d, stream());
+  post_launch_check("rope_split");
+}
+
+void rope_join(torch::Tensor dqkv, torch::Tensor dq, torch::Tensor dk,
+               torch::Tensor dv, c10::optional<torch::Tensor> c,
+               c10::optional<torch::Tensor> s, long length) {
+  TORCH_CHECK(dq.dim() == 3 && dk.dim() == 3, "q, k are [rows, heads, d]");
+  const long rows = dq.size(0), hq = dq.size(1), hkv = dk.size(1);
+  const long d = dq.size(2);
+  check_angles(c, s, rows, length, d);
+  check_rows(dq, rows * hq * d, "dq");
+  check_rows32(dk, rows * hkv * d, "dk");
+  check_rows32(dv, rows * hkv * d, "dv");
+  check_rows(dqkv, rows * (hq + 2 * hkv) * d, "dqkv");
+  launch_rope_join(bf(dqkv), bfc(dq), dk.data_ptr<float>(),
+                   dv.data_ptr<float>(), c ? c->data_ptr<float>() : nullptr,
+                   s ? s->data_ptr<float>() : nullptr, rows, length, hq, hkv,
+                   d, stream());
+  post_launch_check("rope_join");
+}
+
+void silu_mul_bwd(torch::Tensor dx, torch::Tensor dy, torch::Tensor x) {
+  const long f = x.size(-1) / 2, n = x.numel();
+  TORCH_CHECK(n > 0 && f % 8 == 0 && x.size(-1) == 2 * f,
+              "width must be a multiple of 16");
+  check_rows(x, n, "x"); check_rows(dx, n, "dx"); check_rows(dy, n / 2, "dy");
+  launch_silu_mul_bwd(bf(dx), bfc(dy), bfc(x), n / (2 * f), f, stream());
+  post_launch_check("silu_mul_bwd");
 }
 
 void rms_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w, double eps) {
@@ -636,6 +761,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quant_rows_ok", &quant_rows_ok);
   m.def("quant_gemv", &quant_gemv);
   m.def("dequant", &dequant);
+  m.def("add_norm_fwd", &add_norm_fwd);
+  m.def("add_norm_bwd", &add_norm_bwd);
+  m.def("train_norm_takes", &train_norm_takes);
+  m.def("rope_split", &rope_split);
+  m.def("rope_join", &rope_join);
+  m.def("silu_mul_bwd", &silu_mul_bwd);
   m.def("rms_norm", &rms_norm);
   m.def("rms_norm_residual", &rms_norm_residual);
   m.def("layer_norm", &layer_norm);
