@@ -387,6 +387,43 @@ def adamw_step(param: torch.Tensor, grad: torch.Tensor, exp_avg: torch.Tensor,
                    eps, weight_decay, step, grad_scale)
 
 
+def _steady(tensors, dtype: torch.dtype) -> bool:
+    return all(t.is_cuda and t.device == tensors[0].device
+               and t.dtype == dtype and t.is_contiguous()
+               and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def grad_norm(grads: list[torch.Tensor]) -> torch.Tensor:
+    """2-norm of all gradients as one vector, a scalar where they are."""
+    if grads and _steady(grads, torch.bfloat16):
+        return _dispatch(grads[0]).grad_norm(grads)
+    norms = torch._foreach_norm(grads, 2.0)
+    return torch.linalg.vector_norm(torch.stack(norms))
+
+
+def adamw_steps(params: list[torch.Tensor], grads: list[torch.Tensor],
+                exp_avgs: list[torch.Tensor], exp_avg_sqs: list[torch.Tensor],
+                lr: float, beta1: float, beta2: float, eps: float,
+                weight_decay: float, step: int, grad_scale: float = 1.0,
+                norm: Optional[torch.Tensor] = None,
+                clip: float = 0.0) -> None:
+    """adamw_step of several tensors. With a norm the gradients are scaled by
+    min(1, clip / (norm + 1e-6)) besides, on the GPU without a wait for it."""
+    if (params and _steady(params + grads, torch.bfloat16)
+            and _steady([*exp_avgs, *exp_avg_sqs], torch.float32)
+            and (norm is None or grad_scale == 1.0 and norm.is_cuda
+                 and norm.dtype == torch.float32)):
+        _dispatch(params[0]).adamw_steps(
+            params, grads, exp_avgs, exp_avg_sqs, lr, beta1, beta2, eps,
+            weight_decay, step, grad_scale, norm, clip)
+        return
+    if norm is not None:
+        grad_scale *= min(1.0, clip / (float(norm) + 1e-6))
+    for p, g, m, v in zip(params, grads, exp_avgs, exp_avg_sqs):
+        adamw_step(p, g, m, v, lr, beta1, beta2, eps, weight_decay, step,
+                   grad_scale)
+
+
 # ---- weight-streaming decode GEMM (ops/hip/wstream_gemm.hip) -------------
 
 def wstream_repack(w: torch.Tensor) -> torch.Tensor:

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
+#include "optimizer.h"
 #include "rows_quant.h"
 
 typedef __hip_bfloat16 bf16_t;
@@ -41,8 +42,10 @@ void launch_rope_join(bf16_t*, const bf16_t*, const float*, const float*, const 
 void launch_silu_mul_bwd(bf16_t*, const bf16_t*, const bf16_t*, long, int, hipStream_t);
 void launch_softmax_sample(long*, const bf16_t*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
 void launch_softmax_sample(long*, const float*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
-void launch_cross_entropy(float*, bf16_t*, const bf16_t*, const long*, long, int, long, float, hipStream_t);
-void launch_adamw(bf16_t*, const bf16_t*, float*, float*, long, float, float, float, float, float, int, float, hipStream_t);
+void launch_cross_entropy(float*, bf16_t*, const bf16_t*, const long*, long, int, long, float*, hipStream_t);
+void launch_adamw(const std::vector<OptTensor>&, float, float, float, float, float, int, float, const float*, double, hipStream_t);
+long grad_norm_shares(const std::vector<OptTensor>&);
+void launch_grad_norm(float*, float*, const std::vector<OptTensor>&, hipStream_t);
 void launch_adamw_f32(float*, const float*, float*, float*, long, float, float, float, float, float, int, float, hipStream_t);
 void launch_quant_gemv(bf16_t*, const bf16_t*, const void*, const unsigned char*, int, int, int, bool, hipStream_t);
 bool rows_gemm_takes(int, int, int, bool);
@@ -593,6 +596,50 @@ void dequant_k(torch::Tensor out, torch::Tensor scales, torch::Tensor qs,
   post_launch_check("dequant_k");
 }
 
+// The same of several bf16 tensors, their gradients scaled by
+// min(1, clip / (norm + 1e-6)) where a norm on the device is given.
+void adamw_steps(std::vector<torch::Tensor> ps, std::vector<torch::Tensor> gs,
+                 std::vector<torch::Tensor> ms, std::vector<torch::Tensor> vs,
+                 double lr, double beta1, double beta2, double eps, double wd,
+                 long step, double gscale, c10::optional<torch::Tensor> norm,
+                 double clip) {
+  std::vector<OptTensor> all;
+  TORCH_CHECK(gs.size() == ps.size() && ms.size() == ps.size() &&
+              vs.size() == ps.size(), "as many of each");
+  for (size_t i = 0; i < ps.size(); ++i) {
+    const long n = ps[i].numel();
+    check_bf16(ps[i], "parameter");
+    check_rows(gs[i], n, "gradient");
+    check_rows32(ms[i], n, "moment");
+    check_rows32(vs[i], n, "moment");
+    TORCH_CHECK(aligned16(ps[i]), "parameter must be on a 16-byte boundary");
+    all.push_back({ps[i].data_ptr(), gs[i].data_ptr(),
+                   ms[i].data_ptr<float>(), vs[i].data_ptr<float>(), n, 0});
+  }
+  if (norm) check_rows32(*norm, 1, "norm");
+  launch_adamw(all, (float)lr, (float)beta1, (float)beta2, (float)eps,
+               (float)wd, (int)step, (float)gscale,
+               norm ? norm->data_ptr<float>() : nullptr, clip, stream());
+  post_launch_check("adamw_steps");
+}
+
+// The 2-norm of all tensors as one vector, in 32 bits on the device.
+torch::Tensor grad_norm(std::vector<torch::Tensor> gs) {
+  TORCH_CHECK(!gs.empty(), "no gradients");
+  std::vector<OptTensor> all;
+  for (auto& g : gs) {
+    check_rows(g, g.numel(), "gradient");
+    all.push_back({nullptr, g.data_ptr(), nullptr, nullptr, g.numel(), 0});
+  }
+  auto opts = gs[0].options().dtype(torch::kFloat);
+  auto norm = torch::empty({}, opts);
+  auto shares = torch::empty({grad_norm_shares(all)}, opts);
+  launch_grad_norm(norm.data_ptr<float>(), shares.data_ptr<float>(), all,
+                   stream());
+  post_launch_check("grad_norm");
+  return norm;
+}
+
 torch::Tensor mfma32_probe(torch::Tensor a, torch::Tensor b) {
   check_bf16(a, "a"); check_bf16(b, "b");
   TORCH_CHECK(a.size(0) == 32 && a.size(1) == 16 &&
@@ -646,11 +693,13 @@ void cross_entropy_fwd_bwd(torch::Tensor loss, torch::Tensor dlogits,
   long rows = logits.size(0);
   int vocab = logits.size(1);
   TORCH_CHECK(vocab % 8 == 0, "vocab must be a multiple of 8");
-  long nvalid = (targets != ignore_index).sum().item<long>();
-  float inv = nvalid > 0 ? 1.f / (float)nvalid : 0.f;
+  TORCH_CHECK(targets.is_cuda() && targets.numel() == rows,
+              "targets: one of each row, on GPU");
+  targets = targets.contiguous();
+  auto nvalid = torch::empty({1}, loss.options());
   launch_cross_entropy(loss.data_ptr<float>(), bf(dlogits), bfc(logits),
                        targets.data_ptr<long>(), rows, vocab, ignore_index,
-                       inv, stream());
+                       nvalid.data_ptr<float>(), stream());
   post_launch_check("cross_entropy_fwd_bwd");
 }
 
@@ -663,9 +712,10 @@ void adamw_step(torch::Tensor p, torch::Tensor g, torch::Tensor m,
   TORCH_CHECK(g.numel() == n && m.numel() == n && v.numel() == n);
   if (p.scalar_type() == torch::kBFloat16) {
     TORCH_CHECK(g.scalar_type() == torch::kBFloat16);
-    launch_adamw(bf(p), bfc(g), m.data_ptr<float>(), v.data_ptr<float>(), n,
+    launch_adamw({{p.data_ptr(), g.data_ptr(), m.data_ptr<float>(),
+                   v.data_ptr<float>(), n, 0}},
                  (float)lr, (float)beta1, (float)beta2, (float)eps, (float)wd,
-                 (int)step, (float)gscale, stream());
+                 (int)step, (float)gscale, nullptr, 0., stream());
   } else {
     TORCH_CHECK(p.scalar_type() == torch::kFloat && g.scalar_type() == torch::kFloat);
     launch_adamw_f32(p.data_ptr<float>(), g.data_ptr<float>(),
@@ -789,4 +839,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("softmax_sample", &softmax_sample);
   m.def("cross_entropy_fwd_bwd", &cross_entropy_fwd_bwd);
   m.def("adamw_step", &adamw_step);
+  m.def("adamw_steps", &adamw_steps);
+  m.def("grad_norm", &grad_norm);
 }

@@ -16,7 +16,8 @@ void cross_entropy_kernel(float* __restrict__ loss,       // [1]
                           bf16_t* __restrict__ dlogits,   // [N, V]
                           const bf16_t* __restrict__ logits,
                           const long* __restrict__ targets,  // [N]
-                          int vocab, long ignore_index, float inv_nvalid) {
+                          int vocab, long ignore_index,
+                          const float* __restrict__ nvalid) {
   __shared__ float scratch[CNW];
   const long row = blockIdx.x;
   const long tgt = targets[row];
@@ -24,6 +25,7 @@ void cross_entropy_kernel(float* __restrict__ loss,       // [1]
   bf16_t* drow = dlogits + row * vocab;
   const int tid = threadIdx.x;
   const bool valid = tgt != ignore_index;
+  const float inv_nvalid = *nvalid > 0.f ? 1.f / *nvalid : 0.f;
 
   // pass 1: online max + exp-sum
   float m = -INFINITY, s = 0.f;
@@ -82,10 +84,31 @@ void cross_entropy_kernel(float* __restrict__ loss,       // [1]
   }
 }
 
+// Targets that count, by one workgroup: the host does not have to wait for the
+// forward to end before it launches what follows.
+__global__ __launch_bounds__(1024) void count_kernel(
+    float* __restrict__ nvalid, const long* __restrict__ targets, long rows,
+    long ignore_index) {
+  __shared__ int part[1024 / WAVE];
+  int n = 0;
+  for (long i = threadIdx.x; i < rows; i += 1024)
+    n += targets[i] != ignore_index;
+  #pragma unroll
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, WAVE);
+  if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 1024 / WAVE; ++i) n += part[i];
+    *nvalid = (float)n;
+  }
+}
+
 void launch_cross_entropy(float* loss, bf16_t* dlogits, const bf16_t* logits,
                           const long* targets, long rows, int vocab,
-                          long ignore_index, float inv_nvalid,
+                          long ignore_index, float* nvalid,
                           hipStream_t stream) {
+  count_kernel<<<dim3(1), dim3(1024), 0, stream>>>(nvalid, targets, rows,
+                                                   ignore_index);
   cross_entropy_kernel<<<dim3(rows), dim3(CBLOCK), 0, stream>>>(
-      loss, dlogits, logits, targets, vocab, ignore_index, inv_nvalid);
+      loss, dlogits, logits, targets, vocab, ignore_index, nvalid);
 }

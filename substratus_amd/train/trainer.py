@@ -77,15 +77,16 @@ class AdamWState:
         self.step_num = 0
 
     def step(self, cfg: TrainConfig, grad_scale: float = 1.0,
-             lr: Optional[float] = None) -> None:
+             lr: Optional[float] = None,
+             norm: Optional[torch.Tensor] = None) -> None:
+        """norm: of the gradients, to clip them to cfg.grad_clip."""
         self.step_num += 1
         lr = cfg.lr if lr is None else lr
-        for p, m, v in zip(self.params, self.m, self.v):
-            if p.grad is None:
-                continue
-            ops.adamw_step(p.data, p.grad, m, v, lr, cfg.beta1, cfg.beta2,
-                           cfg.eps, cfg.weight_decay, self.step_num,
-                           grad_scale)
+        given = [(p.data, p.grad, m, v) for p, m, v in
+                 zip(self.params, self.m, self.v) if p.grad is not None]
+        ops.adamw_steps(*([t[i] for t in given] for i in range(4)), lr,
+                        cfg.beta1, cfg.beta2, cfg.eps, cfg.weight_decay,
+                        self.step_num, grad_scale, norm, cfg.grad_clip)
 
     def zero_grad(self) -> None:
         for p in self.params:
@@ -102,6 +103,30 @@ class AdamWState:
             dst.copy_(src.to(device))
         for dst, src in zip(self.v, sd["v"]):
             dst.copy_(src.to(device))
+
+
+class _Values:
+    """Scalars on their way to the host."""
+
+    def __init__(self, scalars: list[torch.Tensor]):
+        self.host, self.event = scalars, None
+        if scalars[0].is_cuda:
+            self.host = torch.empty(len(scalars), dtype=scalars[0].dtype,
+                                    pin_memory=True)
+            for i, t in enumerate(scalars):
+                self.host[i].copy_(t, non_blocking=True)
+            self.event = torch.cuda.Event()
+            self.after()
+
+    def after(self) -> None:
+        """read() waits for all that is queued by now."""
+        if self.event is not None:
+            self.event.record()
+
+    def read(self) -> list[float]:
+        if self.event is not None:
+            self.event.synchronize()
+        return [float(t) for t in self.host]
 
 
 class Trainer:
@@ -175,9 +200,11 @@ class Trainer:
             logits = self.model.forward_train(inputs)
             flat = logits.reshape(-1, logits.shape[-1])
             loss, dlogits = ops.cross_entropy_fwd_bwd(flat.detach(), targets)
-            flat.backward(gradient=dlogits / len(chunks))
-            losses.append(float(loss))
-        loss = sum(losses) / len(losses)
+            flat.backward(gradient=dlogits / len(chunks)
+                          if len(chunks) > 1 else dlogits)
+            losses.append(loss)
+        # what follows is queued before the host waits for these
+        losses = _Values(losses)
         lr = self.lr_at(self.global_step + 1)
         if self.use_zero:
             self.zero.finalize()
@@ -190,22 +217,21 @@ class Trainer:
             self.zero.zero_grad()
         else:
             self.buckets.finalize()
-            gscale = 1.0
+            norm = None
             if self.cfg.grad_clip > 0:
                 # norm only; the clip SCALE is folded into the fused AdamW
                 # kernel's gradient read (saves a foreach_mul pass over
                 # every grad — ~10 ms/step at falcon-7b scale)
-                grads = [p.grad for p in self.opt.params
-                         if p.grad is not None]
-                norms = torch._foreach_norm(grads, 2.0)
-                total = torch.linalg.vector_norm(torch.stack(norms))
-                gscale = min(1.0, self.cfg.grad_clip / (float(total) + 1e-6))
-            self.opt.step(self.cfg, grad_scale=gscale, lr=lr)
+                norm = ops.grad_norm([p.grad for p in self.opt.params
+                                      if p.grad is not None])
+                losses.after()
+            self.opt.step(self.cfg, lr=lr, norm=norm)
             self.opt.zero_grad()
         self.global_step += 1
         self.tokens_seen += (tokens.shape[0] * (tokens.shape[1] - 1) *
                              max(self.st.dp_size, 1))
-        return float(loss)
+        losses = losses.read()
+        return sum(losses) / len(losses)
 
     # ---------------------------------------------------------- checkpoints
     def save_checkpoint(self, step: Optional[int] = None) -> str:
