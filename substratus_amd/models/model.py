@@ -144,11 +144,13 @@ class Block(nn.Module):
         overlaps the leader's compute. forward_decode drives this
         generator to completion, so single-stream numerics are by
         construction identical."""
-        qkv = self.wqkv(y)
+        cache = ops.Cache(positions, k_cache, v_cache, slots, self.rope_theta)
+        q = self.wqkv.heads(y, cache)
+        qkv = self.wqkv(y) if q is None else None
         yield
-        q, k, v = self._split_qkv(qkv)
-        q = ops.rope_kv_append(q, k, v, positions, k_cache, v_cache, slots,
-                               self.rope_theta)
+        if q is None:
+            q, k, v = self._split_qkv(qkv)
+            q = ops.rope_kv_append(q, k, v, *cache)
         a = ops.paged_attn_decode(q, k_cache, v_cache, block_table, seq_lens,
                                   self.scale)
         yield

@@ -205,6 +205,22 @@ class QuantLinear(nn.Module):
                        True)
         return y.reshape(*x.shape[:-1], self.out_features // 2)
 
+    def heads(self, x: torch.Tensor,
+              cache: ops.Cache) -> Optional[torch.Tensor]:
+        """ops.rope_kv_append of the outputs in the same kernel, or None."""
+        x2 = x.reshape(-1, self.in_features)
+        n = self.out_features
+        ext = self._few_rows(x2, True) if self.bias is None and \
+            x.dtype == torch.bfloat16 and cache.takes(x, n) else None
+        if ext is None:
+            return None
+        hkv, d = cache.k.shape[1], cache.k.shape[3]
+        q = torch.empty(x2.shape[0], n // d - 2 * hkv, d,
+                        dtype=torch.bfloat16, device=x.device)
+        ext.quant_heads(q, x2.contiguous(), self.scales, self.qs, self.quant,
+                        *cache)
+        return q
+
 
 def quantize_model(model: nn.Module, quant: str) -> nn.Module:
     """Swap every projection Linear (wqkv/wo/w_gateup/w_up/w_down, lm_head)

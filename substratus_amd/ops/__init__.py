@@ -10,7 +10,7 @@ the parity oracle for the GPU tests.
 from __future__ import annotations
 
 import os
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -332,6 +332,48 @@ def linear_gated(x: torch.Tensor, weight: torch.Tensor,
     y = rows.new_empty(rows.shape[0], n)
     ext.rows_gemm(y, rows, weight, bias, True)
     return y if x.dim() == 2 else y.view(*x.shape[:-1], n)
+
+
+class Cache(NamedTuple):
+    """What rope_kv_append is told besides the heads: where their tokens are
+    and go."""
+    positions: torch.Tensor
+    k: torch.Tensor
+    v: torch.Tensor
+    slots: torch.Tensor
+    theta: float
+
+    def takes(self, x: torch.Tensor, n: int) -> bool:
+        """Whether a product of x with n columns may write it: shapes, types
+        and places as its kernel reads them. What is not, rope_kv_append
+        copies or refuses."""
+        hkv, d = self.k.shape[1], self.k.shape[-1]
+        return (self.k.dim() == 4 and self.k.shape == self.v.shape
+                and self.k.dtype == self.v.dtype
+                and self.k.dtype in (torch.bfloat16, torch.float8_e4m3fn)
+                and d % 16 == 0 and n % d == 0 and n > 2 * hkv * d
+                and all(t.device == x.device and t.is_contiguous()
+                        for t in self[:4])
+                and all(t.dtype == torch.int32
+                        and t.numel() == x.numel() // x.shape[-1]
+                        for t in (self.positions, self.slots))
+                and plain_tensors(*self[:4]))
+
+
+def linear_heads(x: torch.Tensor, weight: torch.Tensor,
+                 bias: Optional[torch.Tensor],
+                 cache: Cache) -> Optional[torch.Tensor]:
+    """rope_kv_append of F.linear's columns as heads, in one kernel: the
+    rotated queries, or None where it is not made for that."""
+    few = _few_rows(x, weight, bias, True)
+    n = weight.shape[0]
+    if few is None or not cache.takes(x, n):
+        return None
+    rows, ext = few
+    hkv, d = cache.k.shape[1], cache.k.shape[3]
+    q = rows.new_empty(rows.shape[0], n // d - 2 * hkv, d)
+    ext.rows_heads(q, rows, weight, bias, *cache)
+    return q
 
 
 def silu_mul(x: torch.Tensor) -> torch.Tensor:

@@ -49,7 +49,6 @@ void launch_grad_norm(float*, float*, const std::vector<OptTensor>&, hipStream_t
 void launch_adamw_f32(float*, const float*, float*, float*, long, float, float, float, float, float, int, float, hipStream_t);
 void launch_quant_gemv(bf16_t*, const bf16_t*, const void*, const unsigned char*, int, int, int, bool, hipStream_t);
 bool rows_gemm_takes(int, int, int, bool);
-void launch_rows_gemm(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, int, int, int, long, long, bool, hipStream_t);
 void launch_dequant(bf16_t*, const void*, const unsigned char*, long, int, bool, hipStream_t);
 void launch_dequant_k(bf16_t*, const void*, const unsigned char*, int, int, bool, hipStream_t);
 int decode_gemm_splitk(int, int);
@@ -515,18 +514,42 @@ bool rows_gemm_ok(long m, long n, long k, bool gated) {
   return rows_gemm_takes((int)m, (int)n, (int)k, gated);
 }
 
-void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, bool gated) {
+// Where the columns of a projection of heads go: queries to q [rows, hq, d],
+// keys and values to the paged caches.
+Heads heads_of(const torch::Tensor& q, const torch::Tensor& positions,
+               const torch::Tensor& k_cache, const torch::Tensor& v_cache,
+               const torch::Tensor& slots, double theta) {
+  check_bf16(q, "q");
+  TORCH_CHECK(q.dim() == 3 && q.size(2) % 16 == 0, "q must be [rows, hq, d]");
+  const bool kv8 = cache_kv8(k_cache, "k");
+  TORCH_CHECK(cache_kv8(v_cache, "v") == kv8, "cache dtypes must match");
+  TORCH_CHECK(k_cache.is_cuda() && v_cache.is_cuda() &&
+              k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              k_cache.dim() == 4 && k_cache.sizes() == v_cache.sizes() &&
+              k_cache.size(3) == q.size(2), "cache shape");
+  for (const auto& t : {positions, slots})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kInt &&
+                t.is_contiguous() && t.numel() == q.size(0),
+                "positions and slots must be an int32 of each row");
+  return {positions.data_ptr<int>(), slots.data_ptr<int>(),
+          k_cache.data_ptr(), v_cache.data_ptr(), (int)q.size(1),
+          (int)k_cache.size(1), (int)q.size(2), (int)k_cache.size(2),
+          theta > 0. ? logf((float)theta) : 0.f, theta > 0., kv8};
+}
+
+void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+                  c10::optional<torch::Tensor> bias, bool gated,
+                  const Heads* heads) {
   check_bf16(y, "y"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
               x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0,
               "x must be bf16 rows that begin on 16-byte pieces");
   const int m = x.size(0), k = x.size(1), n = w.size(0);
-  TORCH_CHECK(w.dim() == 2 && w.size(1) == k && y.dim() == 2 &&
-              y.size(0) == m && y.size(1) == (gated ? n / 2 : n),
-              "rows_gemm: shape mismatch");
-  TORCH_CHECK(rows_gemm_takes(m, n, k, gated), "rows_gemm: unsupported shape ",
-              m, "x", n, "x", k);
+  const int cols = heads ? n - 2 * heads->hkv * heads->d : gated ? n / 2 : n;
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == k && y.size(0) == m &&
+              y.numel() == (long)m * cols, "rows_gemm: shape mismatch");
+  TORCH_CHECK(rows_gemm_takes(m, n, k, gated || heads),
+              "rows_gemm: unsupported shape ", m, "x", n, "x", k);
   TORCH_CHECK(aligned16(x) && aligned16(w), "rows_gemm: misaligned operand");
   const bf16_t* bp = nullptr;
   if (bias.has_value()) {
@@ -534,9 +557,24 @@ void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
     TORCH_CHECK(bias->numel() == n, "bias size");
     bp = bfc(*bias);
   }
-  launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0),
-                   y.stride(0), gated, stream());
+  launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols,
+                   gated, heads, stream());
   post_launch_check("rows_gemm");
+}
+
+void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias, bool gated) {
+  rows_gemm_to(y, x, w, bias, gated, nullptr);
+}
+
+// A projection of heads with rope_kv_append of what comes out: rotated queries
+// in q, keys and values in the caches.
+void rows_heads(torch::Tensor q, torch::Tensor x, torch::Tensor w,
+                c10::optional<torch::Tensor> bias, torch::Tensor positions,
+                torch::Tensor k_cache, torch::Tensor v_cache,
+                torch::Tensor slots, double theta) {
+  const Heads heads = heads_of(q, positions, k_cache, v_cache, slots, theta);
+  rows_gemm_to(q, x, w, bias, false, &heads);
 }
 
 Quant quant_of(const std::string& name) {
@@ -552,28 +590,43 @@ bool quant_rows_ok(long m, long n, long k, const std::string& quant,
   return rows_quant_takes((int)m, (int)n, (int)k, quant_of(quant), gated);
 }
 
-// y = x w^T of a quantized weight matrix, at most 64 rows of x; gated as above
-void quant_rows(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
-                torch::Tensor qs, const std::string& quant, bool gated) {
+void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
+                   torch::Tensor qs, const std::string& quant, bool gated,
+                   const Heads* heads) {
   check_bf16(y, "y"); check_bf16(x, "x");
   TORCH_CHECK(scales.scalar_type() == torch::kHalf, "scales must be fp16");
   TORCH_CHECK(qs.scalar_type() == torch::kByte, "qs must be uint8");
   TORCH_CHECK(scales.is_contiguous() && qs.is_contiguous());
   const Quant q = quant_of(quant);
-  const int m = x.size(0), k = x.size(1);
-  const int n = y.size(1) * (gated ? 2 : 1);
-  TORCH_CHECK(y.size(0) == m && qs.size(0) == n && scales.size(0) == n,
-              "quant_rows: shape mismatch");
-  TORCH_CHECK(rows_quant_takes(m, n, k, q, gated),
+  const int m = x.size(0), k = x.size(1), n = qs.size(0);
+  const int cols = heads ? n - 2 * heads->hkv * heads->d : gated ? n / 2 : n;
+  TORCH_CHECK(y.size(0) == m && y.numel() == (long)m * cols &&
+              scales.size(0) == n, "quant_rows: shape mismatch");
+  TORCH_CHECK(rows_quant_takes(m, n, k, q, gated || heads),
               "quant_rows: unsupported shape ", m, "x", n, "x", k);
   // what is not aligned to the kernel's loads is copied to where it is
   if (!aligned16(x)) x = x.clone();
   if (!aligned16(qs)) qs = qs.clone();
   if (!aligned16(scales)) scales = scales.clone();
   launch_rows_quant(bf(y), bfc(x), scales.data_ptr(),
-                    qs.data_ptr<unsigned char>(), m, n, k, q, gated,
+                    qs.data_ptr<unsigned char>(), m, n, k, q, gated, heads,
                     stream());
   post_launch_check("quant_rows");
+}
+
+// y = x w^T of a quantized weight matrix, at most 64 rows of x; gated as above
+void quant_rows(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
+                torch::Tensor qs, const std::string& quant, bool gated) {
+  quant_rows_to(y, x, scales, qs, quant, gated, nullptr);
+}
+
+// rows_heads of a quantized weight matrix
+void quant_heads(torch::Tensor q, torch::Tensor x, torch::Tensor scales,
+                 torch::Tensor qs, const std::string& quant,
+                 torch::Tensor positions, torch::Tensor k_cache,
+                 torch::Tensor v_cache, torch::Tensor slots, double theta) {
+  const Heads heads = heads_of(q, positions, k_cache, v_cache, slots, theta);
+  quant_rows_to(q, x, scales, qs, quant, false, &heads);
 }
 
 void quant_gemv_k(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
@@ -806,6 +859,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wstream_gemm", &wstream_gemm);
   m.def("wstream_ok", &wstream_ok);
   m.def("rows_gemm", &rows_gemm);
+  m.def("rows_heads", &rows_heads);
+  m.def("quant_heads", &quant_heads);
   m.def("rows_gemm_ok", &rows_gemm_ok);
   m.def("quant_rows", &quant_rows);
   m.def("quant_rows_ok", &quant_rows_ok);

@@ -34,14 +34,94 @@ DEV_INLINE void wait_lds_reads() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
+// What becomes of a workgroup's 16 columns.
+//   PLAIN  they are stored
+//   GATED  eight gate another eight, which begin half a matrix later
+//   HEADS  of a fused projection of query, key and value heads: eight are
+//          rotated with another eight, half a head later; queries are stored,
+//          keys and values go to the paged cache
+enum class Columns { PLAIN, GATED, HEADS };
+
+// For HEADS: what launch_rope_kv_append takes.
+struct Heads {
+  const int* positions;
+  const int* slots;
+  void* k_cache;              // [blocks, hkv, block_size, d]
+  void* v_cache;
+  int hq, hkv, d, block_size;
+  float ln_theta;
+  bool turned;                // else keys and queries stay as they are
+  bool kv8;                   // the cache is fp8
+};
+
+// A workgroup's first column, and how much later its second eight are.
+template <Columns C>
+DEV_INLINE int first_column(const Heads& heads) {
+  const int at = blockIdx.x * (C == Columns::PLAIN ? 16 : 8);
+  if constexpr (C == Columns::HEADS) {
+    const int half = heads.d / 2;
+    return at + at / half * half;
+  }
+  return at;
+}
+
+template <Columns C>
+DEV_INLINE int second_half(int n, const Heads& heads) {
+  return C == Columns::HEADS ? heads.d / 2 : n / 2;
+}
+
 // The weight row behind row r of the 16 that a workgroup from column n0 on
-// multiplies. Gated: eight of the gates, then the same eight of what they
-// gate, whose rows begin halfway.
-template <bool GATED>
-DEV_INLINE int weight_row(int n0, int r, int n) {
-  if constexpr (GATED) return n0 + (r & 7) + (r >> 3) * (n / 2);
+// multiplies.
+template <Columns C>
+DEV_INLINE int weight_row(int n0, int r, int n, int half) {
+  if constexpr (C != Columns::PLAIN) return n0 + (r & 7) + (r >> 3) * half;
   return min(n0 + r, n - 1);
 }
+
+// A pair of a head's columns of row r: what rope_kv_append_kernel (rope.hip)
+// does with them after their product is rounded.
+DEV_INLINE void finish_heads(bf16_t* y, long y_ld, const Heads& heads, int r,
+                             int col, float a, float b) {
+  const int half = heads.d / 2, j = col % heads.d;
+  int head = col / heads.d;
+  float x1 = bf2f(f2bf(a)), x2 = bf2f(f2bf(b));
+  if (heads.turned && head < heads.hq + heads.hkv) {
+    float s, c;
+    const float pos = (float)heads.positions[r];
+    const float inv_freq = __expf(-(float)j / (float)half * heads.ln_theta);
+    __sincosf(pos * inv_freq, &s, &c);
+    const float r1 = x1 * c - x2 * s;
+    x2 = x2 * c + x1 * s;
+    x1 = r1;
+  }
+  if (head < heads.hq) {
+    y[r * y_ld + col] = f2bf(x1);
+    y[r * y_ld + col + half] = f2bf(x2);
+    return;
+  }
+  head -= heads.hq;
+  const bool key = head < heads.hkv;
+  if (!key) head -= heads.hkv;
+  const int slot = heads.slots[r];
+  const long at = (((long)(slot / heads.block_size) * heads.hkv + head) *
+                       heads.block_size + slot % heads.block_size) *
+                      heads.d + j;
+  void* cache = key ? heads.k_cache : heads.v_cache;
+  if (heads.kv8) {
+    unsigned char* to = reinterpret_cast<unsigned char*>(cache) + at;
+    to[0] = f32_to_fp8(x1);
+    to[half] = f32_to_fp8(x2);
+  } else {
+    bf16_t* to = reinterpret_cast<bf16_t*>(cache) + at;
+    to[0] = f2bf(x1);
+    to[half] = f2bf(x2);
+  }
+}
+
+void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
+                      const bf16_t* bias, int m, int n, int k, long x_ld,
+                      long y_ld, bool gated, const Heads* heads,
+                      hipStream_t stream);
 
 DEV_INLINE float silu_times(float g, float u) {
   return g / (1.f + __expf(-g)) * u;

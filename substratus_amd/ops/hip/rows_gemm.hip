@@ -1,6 +1,7 @@
 // y = x w^T + bias of at most 16 rows with a bf16 weight matrix [n, k], as
 // single tokens of a small batch need it; or, of a matrix whose first half
-// gates its second, silu(gate) * up.
+// gates its second, silu(gate) * up; or, of a projection of heads, rotated
+// queries, with keys and values appended to the cache.
 //
 // Bound by reading the weights once. A workgroup takes 16 weight rows; its
 // four waves share k. A wave's loads go straight to LDS, 16 rows x 64
@@ -33,17 +34,17 @@ constexpr int STAGE = U * 2 * TILE;
 constexpr int LOADS = U * 2;      // of a stage
 constexpr int PAD = 4;
 
-template <bool GATED>
+template <Columns C>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       const bf16_t* __restrict__ w,
                       const bf16_t* __restrict__ bias, int m, int n, int k,
-                      long x_ld, long y_ld) {
+                      long x_ld, long y_ld, Heads heads) {
   __shared__ alignas(16) uint4 s_all[KW * P * STAGE];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
   const int lo = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (GATED ? 8 : 16);
+  const int n0 = first_column<C>(heads), half = second_half<C>(n, heads);
   const int chunks = k / 32;
   const int c0 = chunks * wave / KW, c1 = chunks * (wave + 1) / KW;
   const int steps = (c1 - c0 + U - 1) / U;
@@ -52,7 +53,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   // a lane loads 16 bytes of row lane / 4 of a tile
   const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
   const char* wp = reinterpret_cast<const char*>(
-      w + (long)weight_row<GATED>(n0, row, n) * k) + piece * 16;
+      w + (long)weight_row<C>(n0, row, n, half) * k) + piece * 16;
   const char* xp = reinterpret_cast<const char*>(
       x + min(row, m - 1) * x_ld) + piece * 16;
   auto load = [&](int s, int i) {
@@ -117,11 +118,13 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     float v = 0.f;
     #pragma unroll
     for (int q = 0; q < KW; ++q) v += red[(q * 16 + r) * (16 + PAD) + c];
-    if (bias != nullptr) v += bf2f(bias[weight_row<GATED>(n0, c, n)]);
+    if (bias != nullptr) v += bf2f(bias[weight_row<C>(n0, c, n, half)]);
     return v;
   };
-  if constexpr (GATED) {
+  if constexpr (C == Columns::GATED) {
     if (c < 8) y[r * y_ld + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
+  } else if constexpr (C == Columns::HEADS) {
+    if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
   } else {
     if (n0 + c < n) y[r * y_ld + n0 + c] = f2bf(sum(c));
   }
@@ -135,15 +138,15 @@ bool rows_gemm_takes(int m, int n, int k, bool gated) {
          (!gated || n % 16 == 0);
 }
 
+// heads: null, or what is done with the columns instead of storing them (n is
+// a multiple of 16 then, like gated's)
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
-                      long y_ld, bool gated, hipStream_t stream) {
-  if (gated) {
-    rows_gemm_kernel<true><<<dim3(n / 16), dim3(KW * WAVE), 0, stream>>>(
-        y, x, w, bias, m, n, k, x_ld, y_ld);
-  } else {
-    rows_gemm_kernel<false>
-        <<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
-            y, x, w, bias, m, n, k, x_ld, y_ld);
-  }
+                      long y_ld, bool gated, const Heads* heads,
+                      hipStream_t stream) {
+  auto kernel = heads ? rows_gemm_kernel<Columns::HEADS>
+                : gated ? rows_gemm_kernel<Columns::GATED>
+                        : rows_gemm_kernel<Columns::PLAIN>;
+  kernel<<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
+      y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{});
 }

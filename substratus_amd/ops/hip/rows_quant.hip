@@ -1,5 +1,7 @@
 // y = x w^T of up to 64 rows with a GGUF-quantized weight matrix [n, k], or,
-// of a matrix whose first half gates its second, silu(gate) * up. Weights as
+// of a matrix whose first half gates its second, silu(gate) * up, or, of a
+// projection of heads, rotated queries, with keys and values appended to the
+// cache. Weights as
 // models/quant.py lays them out:
 //   q4_0, q8_0   scales fp16 [n, k/32]; qs [n, k/2] nibbles (byte i of a block
 //                has weights i and i + 16), [n, k] int8
@@ -40,7 +42,6 @@
 //        24 rows   523  196  946  479 -> 38.4 19.5 64.8 46.9
 // q8_0 with one row stays with the vector kernel (quant_gemv.hip): 20.5, 9.4,
 // 33.1, 19.3 there and 19.9, 11.1, 32.2, 23.8 here.
-#include "rows_gemm.h"
 #include "rows_quant.h"
 
 #include <type_traits>
@@ -129,12 +130,12 @@ template <> struct Layout<Quant::Q6_K> {
 
 // MR: rows of x; ME: of every four, those that are there (MR 4 only); KW
 // waves share k, P stages are in flight in each
-template <Quant Q, int MR, int ME, int KW, int P, bool GATED>
+template <Quant Q, int MR, int ME, int KW, int P, Columns C>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                        const f16_t* __restrict__ scales,
                        const unsigned char* __restrict__ qs, int m, int n,
-                       int k) {
+                       int k, Heads heads) {
   using L = Layout<Q>;
   constexpr bool K_QUANT = Q == Quant::Q4_K || Q == Quant::Q6_K;
   constexpr int FM = (MR + 15) / 16;
@@ -149,7 +150,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
   const int lo = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (GATED ? 8 : 16);
+  const int n0 = first_column<C>(heads), half = second_half<C>(n, heads);
   x += (long)blockIdx.y * MR * k;
   m -= blockIdx.y * MR;
   const int nb = k / 32, all = (k + COLS - 1) / COLS;
@@ -165,9 +166,9 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
   const int word = lane & 3;
   const unsigned char* sc = reinterpret_cast<const unsigned char*>(scales);
-  const unsigned char* wp = qs + weight_row<GATED>(n0, row, n) * rb;
-  const unsigned char* sp = sc + weight_row<GATED>(n0, row, n) * sb;
-  const unsigned char* dp = sc + weight_row<GATED>(n0, lo, n) * sb;
+  const unsigned char* wp = qs + weight_row<C>(n0, row, n, half) * rb;
+  const unsigned char* sp = sc + weight_row<C>(n0, row, n, half) * sb;
+  const unsigned char* dp = sc + weight_row<C>(n0, lo, n, half) * sb;
   const char* xp[XL / 2];
   #pragma unroll
   for (int d = 0; d < XL / 2; ++d)
@@ -363,7 +364,13 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     for (int e = 0; e < 4; ++e)
       red[(wave * BM + j * 16 + g * 4 + e) * (16 + PAD) + lo] = acc[j][e];
   __syncthreads();
-  y += (long)blockIdx.y * MR * (GATED ? n / 2 : n);
+  const int y_ld = C == Columns::GATED ? n / 2
+      : C == Columns::HEADS ? heads.hq * heads.d : n;
+  y += (long)blockIdx.y * MR * y_ld;
+  if constexpr (C == Columns::HEADS) {
+    heads.positions += blockIdx.y * MR;
+    heads.slots += blockIdx.y * MR;
+  }
   for (int i = threadIdx.x; i < BM * 16; i += KW * WAVE) {
     const int r = i / 16, c = i % 16;
     if (r >= m || r >= MR) break;
@@ -373,11 +380,13 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       for (int q = 0; q < KW; ++q) v += red[(q * BM + r) * (16 + PAD) + c];
       return v;
     };
-    if constexpr (GATED) {
+    if constexpr (C == Columns::GATED) {
       if (c < 8)
-        y[(long)r * (n / 2) + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
+        y[(long)r * y_ld + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
+    } else if constexpr (C == Columns::HEADS) {
+      if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
     } else {
-      if (n0 + c < n) y[(long)r * n + n0 + c] = f2bf(sum(c));
+      if (n0 + c < n) y[(long)r * y_ld + n0 + c] = f2bf(sum(c));
     }
   }
 }
@@ -393,20 +402,19 @@ bool rows_quant_takes(int m, int n, int k, Quant q, bool gated) {
 
 void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
                        const unsigned char* qs, int m, int n, int k, Quant q,
-                       bool gated, hipStream_t stream) {
+                       bool gated, const Heads* heads, hipStream_t stream) {
   const f16_t* sc = reinterpret_cast<const f16_t*>(scales);
   auto go = [&](auto qc, auto mr, auto me, auto kw, auto p) {
     constexpr Quant QQ = decltype(qc)::value;
     constexpr int MR = decltype(mr)::value, ME = decltype(me)::value,
                   KW = decltype(kw)::value, P = decltype(p)::value;
     const dim3 grid((n + 15) / 16, (m + MR - 1) / MR), block(KW * WAVE);
-    if (gated) {
-      rows_quant_kernel<QQ, MR, ME, KW, P, true>
-          <<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k);
-    } else {
-      rows_quant_kernel<QQ, MR, ME, KW, P, false>
-          <<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k);
-    }
+    auto kernel =
+        heads ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::HEADS>
+        : gated ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::GATED>
+                : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN>;
+    kernel<<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k,
+                                       heads ? *heads : Heads{});
   };
   auto by_rows = [&](auto qc) {
     constexpr Quant QQ = decltype(qc)::value;

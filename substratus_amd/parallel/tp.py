@@ -16,6 +16,7 @@ first-party (the reference's data plane is external — SURVEY.md §0).
 from __future__ import annotations
 
 import math
+from typing import Optional
 
 import torch
 import torch.nn as nn
@@ -53,6 +54,12 @@ class Linear(nn.Module):
         """silu(first half of the outputs) * second half."""
         y = ops.linear_gated(x, self.weight, self.bias)
         return ops.silu_mul(self(x)) if y is None else y
+
+
+    def heads(self, x: torch.Tensor,
+              cache: ops.Cache) -> Optional[torch.Tensor]:
+        """ops.rope_kv_append of the outputs in the same kernel, or None."""
+        return ops.linear_heads(x, self.weight, self.bias, cache)
 
 
 class ColumnParallelLinear(Linear):
