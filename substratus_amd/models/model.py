@@ -40,17 +40,20 @@ def _norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
     return ops.layer_norm(x, weight, bias, eps)
 
 
-def fused_norm_residual(delta: torch.Tensor, h: torch.Tensor,
-                        norm: "NormParams",
+def fused_norm_residual(deltas: tuple, h: torch.Tensor, norm: "NormParams",
                         eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """y = norm(h + delta), h = h + delta — fused on the RMSNorm path so the
-    hidden state makes one HBM round trip per norm (profiles/
-    serve_decode_r01_baseline.txt: unfused residual adds were ~2.2 ms of a
-    10.3 ms decode step)."""
-    if norm.rms:
-        return ops.rms_norm_residual(delta, h, norm.weight, eps)
-    h = h + delta
-    return norm(h, eps), h
+    """y = norm(h + deltas), h = h + deltas — fused so the hidden state makes
+    one HBM round trip per norm (profiles/serve_decode_r01_baseline.txt:
+    unfused residual adds were ~2.2 ms of a 10.3 ms decode step). RMSNorm of
+    one delta works in place on h."""
+    if norm.rms and len(deltas) == 1:
+        return ops.rms_norm_residual(deltas[0], h, norm.weight, eps)
+    got = train_ops.fused_add_norm(h, deltas, norm.weight, norm.bias, eps)
+    if got is None:
+        for d in deltas:
+            h = h + d
+        got = norm(h, eps), h
+    return got
 
 
 class NormParams(nn.Module):
@@ -161,13 +164,13 @@ class Block(nn.Module):
             if self.cfg.activation == "silu":
                 a = self.w_gateup.gated(mlp_in)
                 yield
-                out = attn_out + self.w_down(a)
+                out = self.w_down(a)
             else:
                 u = self.w_up(mlp_in)
                 yield
-                out = attn_out + self.w_down(ops.gelu(u))
-            return out, h
-        y2, h = fused_norm_residual(attn_out, h, self.norm2, self.eps)
+                out = self.w_down(ops.gelu(u))
+            return (attn_out, out), h
+        y2, h = fused_norm_residual((attn_out,), h, self.norm2, self.eps)
         if self.cfg.activation == "silu":
             a = self.w_gateup.gated(y2)
             yield
@@ -176,16 +179,16 @@ class Block(nn.Module):
             u = self.w_up(y2)
             yield
             out = self.w_down(ops.gelu(u))
-        return out, h
+        return (out,), h
 
     def forward_decode(self, y: torch.Tensor, h: torch.Tensor,
                        positions: torch.Tensor,
                        k_cache: torch.Tensor, v_cache: torch.Tensor,
                        slots: torch.Tensor, block_table: torch.Tensor,
-                       seq_lens: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+                       seq_lens: torch.Tensor) -> tuple[tuple, torch.Tensor]:
         """y: normalized input (this block's norm1 already applied by the
         caller's fused residual+norm); h: the residual stream. Returns
-        (delta, h) where delta is this block's output to be added by the
+        (deltas, h) where deltas are this block's outputs to be added by the
         NEXT norm's fused residual."""
         gen = self.decode_ops(y, h, positions, k_cache, v_cache, slots,
                               block_table, seq_lens)
@@ -196,23 +199,25 @@ class Block(nn.Module):
                 return e.value
 
     # -- prefill ------------------------------------------------------------
-    def forward_prefill(self, h: torch.Tensor, positions: torch.Tensor,
-                        seq_start: torch.Tensor, k_cache: torch.Tensor,
-                        v_cache: torch.Tensor, slots: torch.Tensor) -> torch.Tensor:
-        y = self.norm1(h, self.eps)
-        q, k, v = self._split_qkv(self.wqkv(y))
-        # rope_kv_append rotates q AND k in place (k also lands rotated in
-        # the paged cache); the dense varlen attention consumes them directly
-        k = k.contiguous()
-        q = ops.rope_kv_append(q, k, v, positions, k_cache, v_cache, slots,
-                               self.rope_theta)
-        a = ops.attn_prefill(q, k, v, seq_start, self.scale)
+    def forward_prefill(self, h: torch.Tensor, deltas: tuple,
+                        positions: torch.Tensor, seq_start: torch.Tensor,
+                        k_cache: torch.Tensor, v_cache: torch.Tensor,
+                        slots: torch.Tensor,
+                        max_len: Optional[int]) -> tuple:
+        """(h, deltas): the residual stream and what is still to be added to
+        it, which the next norm does; the same is returned."""
+        y, h = fused_norm_residual(deltas, h, self.norm1, self.eps)
+        q, k, v = ops.rope_split_append(
+            self.wqkv(y), self.n_heads, self.n_kv_heads,
+            ops.Cache(positions, k_cache, v_cache, slots, self.rope_theta))
+        a = ops.attn_prefill(q, k, v, seq_start, self.scale, max_len)
         attn_out = self.wo(a.reshape(a.shape[0], -1))
         if self.parallel_attn:
-            mlp_in = self.norm2(h, self.eps) if self.parallel_norms else y
-            return h + attn_out + self._mlp(mlp_in)
-        h = h + attn_out
-        return h + self._mlp(self.norm2(h, self.eps))
+            if self.parallel_norms:
+                y = self.norm2(h, self.eps)
+            return h, (attn_out, self._mlp(y))
+        y, h = fused_norm_residual((attn_out,), h, self.norm2, self.eps)
+        return h, (self._mlp(y),)
 
     # -- train (dense, differentiable) --------------------------------------
     def forward_train(self, h: torch.Tensor, deltas: tuple,
@@ -313,12 +318,12 @@ class CausalLM(nn.Module):
         y = self.blocks[0].norm1(h, self.eps)
         yield
         for i, (blk, (kc, vc)) in enumerate(zip(self.blocks, kv_caches)):
-            delta, h = yield from blk.decode_ops(y, h, positions, kc, vc,
+            deltas, h = yield from blk.decode_ops(y, h, positions, kc, vc,
                                                  slots, block_table,
                                                  seq_lens)
             nxt = (self.blocks[i + 1].norm1 if i + 1 < len(self.blocks)
                    else self.final_norm)
-            y, h = fused_norm_residual(delta, h, nxt, self.eps)
+            y, h = fused_norm_residual(deltas, h, nxt, self.eps)
             yield
         return self._logits(y)
 
@@ -343,11 +348,15 @@ class CausalLM(nn.Module):
         h = self.embed_tokens(tokens)
         if self.cfg.learned_pos_emb:
             h = h + self.embed_positions(positions.long())
+        max_len = ops.longest(seq_start) if h.is_cuda else None
+        deltas = ()
         for blk, (kc, vc) in zip(self.blocks, kv_caches):
-            h = blk.forward_prefill(h, positions, seq_start, kc, vc, slots)
+            h, deltas = blk.forward_prefill(h, deltas, positions, seq_start,
+                                            kc, vc, slots, max_len)
         last = (seq_start[1:] - 1).long()
-        h = self.final_norm(h[last], self.eps)
-        return self._logits(h)
+        y, _ = fused_norm_residual(tuple(d[last] for d in deltas), h[last],
+                                   self.final_norm, self.eps)
+        return self._logits(y)
 
     # -- train ---------------------------------------------------------------
     def forward_train(self, tokens: torch.Tensor) -> torch.Tensor:

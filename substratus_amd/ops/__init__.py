@@ -126,13 +126,21 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor,
     return out
 
 
+def longest(seq_start: torch.Tensor) -> int:
+    return int((seq_start[1:] - seq_start[:-1]).max())
+
+
 def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
-                 seq_start: torch.Tensor, scale: float) -> torch.Tensor:
+                 seq_start: torch.Tensor, scale: float,
+                 max_len: Optional[int] = None) -> torch.Tensor:
+    """max_len: of the sequences, where the caller knows it; the host waits
+    for it otherwise."""
     ext = _dispatch(q)
     if ext is None:
         return ref.attn_prefill(q, k, v, seq_start, scale)
     out = torch.empty_like(q)
-    max_len = int((seq_start[1:] - seq_start[:-1]).max())
+    if max_len is None:
+        max_len = longest(seq_start)
     if os.environ.get("SUB_ATTN_V5", "1") != "0":
         # V5: 8-wave swapped-QK^T in-register-softmax structure —
         # 293-516 TF vs V4's 167-250 (scripts/microbench.py --which attnv5)
@@ -358,6 +366,28 @@ class Cache(NamedTuple):
                         and t.numel() == x.numel() // x.shape[-1]
                         for t in (self.positions, self.slots))
                 and plain_tensors(*self[:4]))
+
+
+def rope_split_append(qkv: torch.Tensor, hq: int, hkv: int, cache: Cache
+                      ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(q, k, v), each [rows, heads, d], of fused rows; rope_kv_append of
+    them."""
+    n, d = qkv.shape[0], qkv.shape[1] // (hq + 2 * hkv)
+    if (qkv.is_cuda and qkv.dtype == torch.bfloat16 and qkv.is_contiguous()
+            and qkv.numel() > 0 and cache.takes(qkv, qkv.shape[1])
+            and cache.k.shape[1] == hkv and d in (16, 32, 64, 128)
+            and all(t.data_ptr() % 16 == 0 for t in (qkv, cache.k, cache.v))
+            and inference_only(qkv)):
+        q = qkv.new_empty(n, hq, d)
+        k, v = (qkv.new_empty(n, hkv, d) for _ in range(2))
+        _dispatch(qkv).rope_split_append(q, k, v, qkv, *cache)
+        return q, k, v
+    q, k, v = (t.view(n, -1, d)
+               for t in qkv.split([hq * d, hkv * d, hkv * d], dim=-1))
+    # rope_kv_append rotates q AND k in place (k also lands rotated in
+    # the paged cache); the dense varlen attention consumes them directly
+    k = k.contiguous()
+    return rope_kv_append(q, k, v, *cache), k, v
 
 
 def linear_heads(x: torch.Tensor, weight: torch.Tensor,

@@ -17,6 +17,7 @@ void launch_layer_norm(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, lon
 void launch_silu_mul(bf16_t*, const bf16_t*, long, int, hipStream_t);
 void launch_gelu(bf16_t*, const bf16_t*, long, hipStream_t);
 void launch_rope_kv_append(bf16_t*, bf16_t*, const bf16_t*, const int*, void*, void*, const int*, int, int, int, int, int, float, bool, long, long, long, hipStream_t);
+void launch_rope_split_append(bf16_t*, bf16_t*, bf16_t*, const bf16_t*, const int*, void*, void*, const int*, long, int, int, int, int, float, bool, hipStream_t);
 void launch_paged_attn_decode(bf16_t*, const bf16_t*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, long, int, float*, float*, bool, hipStream_t);
 int paged_attn_nsplit(int, int, int, int, int);
 bool paged_attn_decode_supported(int, int);
@@ -537,6 +538,25 @@ Heads heads_of(const torch::Tensor& q, const torch::Tensor& positions,
           theta > 0. ? logf((float)theta) : 0.f, theta > 0., kv8};
 }
 
+// rope_kv_append of fused rows qkv, whose heads come out as rows of their own
+void rope_split_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                       torch::Tensor qkv, torch::Tensor positions,
+                       torch::Tensor k_cache, torch::Tensor v_cache,
+                       torch::Tensor slots, double theta) {
+  const Heads h = heads_of(q, positions, k_cache, v_cache, slots, theta);
+  const long rows = q.size(0), kv = rows * h.hkv * h.d;
+  TORCH_CHECK(rows > 0 && 256 % (h.d / 16) == 0 && h.d <= 128,
+              "head_dim ", h.d, " not taken");
+  check_rows(q, rows * h.hq * h.d, "q");
+  check_rows(k, kv, "k"); check_rows(v, kv, "v");
+  check_rows(qkv, q.numel() + 2 * kv, "qkv");
+  TORCH_CHECK(aligned16(k_cache) && aligned16(v_cache), "misaligned cache");
+  launch_rope_split_append(bf(q), bf(k), bf(v), bfc(qkv), h.positions,
+                           h.k_cache, h.v_cache, h.slots, rows, h.hq, h.hkv,
+                           h.d, h.block_size, (float)theta, h.kv8, stream());
+  post_launch_check("rope_split_append");
+}
+
 void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> bias, bool gated,
                   const Heads* heads) {
@@ -860,6 +880,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wstream_ok", &wstream_ok);
   m.def("rows_gemm", &rows_gemm);
   m.def("rows_heads", &rows_heads);
+  m.def("rope_split_append", &rope_split_append);
   m.def("quant_heads", &quant_heads);
   m.def("rows_gemm_ok", &rows_gemm_ok);
   m.def("quant_rows", &quant_rows);

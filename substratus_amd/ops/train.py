@@ -101,11 +101,10 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-def add_norm(h: torch.Tensor, deltas: Sequence[torch.Tensor],
-             weight: torch.Tensor, bias: Optional[torch.Tensor],
-             eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """(norm(h + deltas), h + deltas): LayerNorm, without bias RMSNorm, over
-    the last dimension, in 32 bits."""
+def fused_add_norm(h: torch.Tensor, deltas: Sequence[torch.Tensor],
+                   weight: torch.Tensor, bias: Optional[torch.Tensor],
+                   eps: float) -> Optional[tuple]:
+    """add_norm where train_rows.hip takes it, or None."""
     if (len(deltas) <= 2 and _whole(h, weight, bias, *deltas)
             and h.shape[-1:] == weight.shape
             and (bias is None or bias.shape == weight.shape)
@@ -115,8 +114,19 @@ def add_norm(h: torch.Tensor, deltas: Sequence[torch.Tensor],
             and _load_ext().train_norm_takes(weight.numel())):
         out = _AddNorm.apply(eps, weight, bias, h, *deltas)
         return out if deltas else (out, h)
-    h = _add(h, deltas)
-    return _norm(h, weight, bias, eps), h
+    return None
+
+
+def add_norm(h: torch.Tensor, deltas: Sequence[torch.Tensor],
+             weight: torch.Tensor, bias: Optional[torch.Tensor],
+             eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """(norm(h + deltas), h + deltas): LayerNorm, without bias RMSNorm, over
+    the last dimension, in 32 bits."""
+    got = fused_add_norm(h, deltas, weight, bias, eps)
+    if got is None:
+        h = _add(h, deltas)
+        got = _norm(h, weight, bias, eps), h
+    return got
 
 
 # ----------------------------------------------------------------- attention
