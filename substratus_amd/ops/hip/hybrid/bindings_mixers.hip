@@ -362,7 +362,8 @@ void run_gla(const Gla<T>& a, const Tensor& state, int entries,
     if (seq_start && !recurrent &&
         gla_chunk_supported(a.dim, a.vdim, a.rank) &&
         max_len * a.ld * 2 < 0x7ffffff0 - (1 << 20)) {
-      const int nseg = gla_chunk_segments(entries, a.heads, max_len);
+      const int nseg =
+          gla_chunk_segments(entries, a.heads, a.dim, a.vdim, max_len);
       Tensor ws, wd;
       if (nseg > 1) {
         ws = torch::empty({entries, nseg, a.heads, a.dim, a.vdim},

@@ -44,6 +44,6 @@ template <class T>
 void launch_gla_recurrent(const Gla<T>&, int entries, hipStream_t);
 
 bool gla_chunk_supported(int dim, int vdim, int rank);
-int gla_chunk_segments(int entries, int heads, int max_len);
+int gla_chunk_segments(int entries, int heads, int dim, int vdim, int max_len);
 void launch_gla_chunk(const Gla<bf16_t>&, int entries, int max_len, int nseg,
                       float* ws, float* ws_decay, hipStream_t);

@@ -32,6 +32,7 @@
 #include "chunk.h"
 #include "gla.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -523,12 +524,30 @@ bool gla_chunk_supported(int dim, int vdim, int rank) {
   return dim <= 256 && vdim <= 32 * MAXW && rank <= MAXRANK;
 }
 
-// Segments per portion: enough workgroups for two per CU, segments of at
-// least 256 tokens.
-int gla_chunk_segments(int entries, int heads, int max_len) {
-  int n = 1;
-  while ((long)entries * heads * n < 512 && max_len >= n * 2 * 256) n *= 2;
-  return n;
+// Segments per portion. A segment is a serial chain of chunks, and a chunk
+// takes a workgroup 10 us (dim 128, MI355X) and 4 more in the pass before it,
+// whatever else runs, up to a workgroup per CU; two per CU take a third longer
+// each. Segments cost that pass, 14 us of launches, and their states' way
+// through memory four times. us, 16 heads of 128, one segment per 256 tokens
+// (as many as 512 workgroups) -> the number that takes least by this:
+//   portions of 900, 700, 500, 300   203 -> 100    one of 2000   211 -> 74
+//   one of 250    81 -> 47           one of 1000   204 -> 61     8000   220 -> 165
+//   16 of 300    106 (120 in two segments each)    8 of 120    48 (59)
+int gla_chunk_segments(int entries, int heads, int dim, int vdim,
+                       int max_len) {
+  const double width = 0.3 + 0.7 * dim / 128.;
+  const long pairs = (long)entries * heads;
+  auto cost = [&](long n) {
+    const long chunks = (max_len + n * C - 1) / (n * C);
+    const double busy = std::max(1., pairs * n / 256. * 0.66);
+    const double chain = chunks * width * busy * (n > 1 ? 14.5 : 10.5);
+    return n == 1 ? chain
+                  : chain + 14. + pairs * n * dim * vdim * (16. / 6e6);
+  };
+  int best = 1;
+  for (int n = 2; pairs * n < 1024 && max_len >= n * C; n *= 2)
+    if (cost(n) < cost(best)) best = n;
+  return best;
 }
 
 void launch_gla_chunk(const Gla<bf16_t>& a, int entries, int max_len, int nseg,
