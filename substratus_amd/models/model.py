@@ -285,7 +285,7 @@ class CausalLM(nn.Module):
 
     def _logits(self, y: torch.Tensor) -> torch.Tensor:
         if self.lm_head is None:
-            return F.linear(y, self.embed_tokens.weight)
+            return ops.linear(y, self.embed_tokens.weight)
         return self.lm_head(y)  # module call: works for Linear AND QuantLinear
 
     @torch.no_grad()

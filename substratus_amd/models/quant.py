@@ -18,7 +18,6 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import ops
 from .gguf import (QK, QK_K, Q4_K_BLOCK_BYTES, Q6_K_BLOCK_BYTES,
@@ -187,7 +186,7 @@ class QuantLinear(nn.Module):
             y = y.to(x.dtype)
         else:
             w = self.dequant_weight().to(x.dtype)
-            y = F.linear(x2, w)
+            y = ops.linear(x2, w)
         if self.bias is not None:
             y = y + self.bias
         return y.reshape(*shape[:-1], self.out_features)

@@ -280,12 +280,89 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
     return x, ext
 
 
+def _tile_gemm(a: torch.Tensor, b: torch.Tensor,
+               bias: Optional[torch.Tensor] = None, a_flipped: bool = False,
+               b_flipped: bool = False) -> Optional[torch.Tensor]:
+    """a b^T + bias on tile_gemm.hip, a stored as [k, m] and b as [k, n] where
+    flipped, or None where it does not take them or does not pay."""
+    ext = _load_ext()
+    m, k = a.shape[::-1] if a_flipped else a.shape
+    n = b.shape[1 if b_flipped else 0]
+    if (ext is None or not all(
+            t.is_cuda and t.device == a.device and t.dtype == torch.bfloat16
+            and t.stride(1) == 1 and t.data_ptr() % 16 == 0 for t in (a, b))
+            or not ext.tile_gemm_good(m, n, k, a.stride(0), b.stride(0),
+                                      a_flipped, b_flipped)):
+        return None
+    if bias is not None and not (
+            bias.device == a.device and bias.dtype == torch.bfloat16
+            and bias.is_contiguous() and bias.shape == (n,)
+            and bias.data_ptr() % 16 == 0):
+        return None
+    return ext.tile_gemm(a, b, bias, a_flipped, b_flipped)
+
+
+class _Linear(torch.autograd.Function):
+    """F.linear of rows, each product where it is faster."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        ctx.save_for_backward(x, weight)
+        y = _tile_gemm(x, weight, bias)
+        return torch.nn.functional.linear(x, weight, bias) if y is None else y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        dx = dw = db = None
+        # gradients that can be differentiated again are torch's
+        own = not torch.is_grad_enabled()
+        if own and ctx.needs_input_grad[0]:
+            dx = _tile_gemm(dy, weight, b_flipped=True)
+        if own and ctx.needs_input_grad[1]:
+            dw = _tile_gemm(dy, x, a_flipped=True, b_flipped=True)
+        if dx is None and ctx.needs_input_grad[0]:
+            dx = dy @ weight
+        if dw is None and ctx.needs_input_grad[1]:
+            dw = dy.t() @ x
+        if ctx.needs_input_grad[2]:
+            db = dy.sum(0)
+        return dx, dw, db
+
+
+def _many_rows(x: torch.Tensor, weight: torch.Tensor,
+               bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """F.linear of 256 rows and more, or None where torch's is as good."""
+    given = [t for t in (x, weight, bias) if t is not None]
+    if not (x.is_cuda and weight.dim() == 2 and weight.shape[0] >= 256
+            and x.dim() >= 2 and x.shape[-1] == weight.shape[1] > 0
+            and x.numel() >= 256 * x.shape[-1]
+            and all(t.device == x.device and t.dtype == torch.bfloat16
+                    for t in given)
+            and _load_ext() is not None and plain_tensors(*given)):
+        return None
+    rows = x.reshape(-1, x.shape[-1])
+    if torch.is_grad_enabled() and any(t.requires_grad for t in given):
+        m, k, n = *rows.shape, weight.shape[0]
+        good = _load_ext().tile_gemm_good
+        if not (good(m, n, k, k, k, False, False)
+                or good(m, k, n, n, k, False, True)
+                or good(n, k, m, n, k, True, True)):
+            return None
+        y = _Linear.apply(rows, weight, bias)
+    else:
+        y = _tile_gemm(rows, weight, bias)
+    return y if y is None or x.dim() == 2 else \
+        y.view(*x.shape[:-1], weight.shape[0])
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """F.linear. Up to 16 rows of bf16 without gradients take the kernel that
-    streams weights at the memory's rate (rows_gemm.hip). SUB_MGEMM=1 routes
-    decode shapes of 256 rows and more to the 256x256 glds GEMM
-    (mfma_gemm.hip).
+    streams weights at the memory's rate (rows_gemm.hip), products of 256 rows
+    and more the one for the matrix cores (tile_gemm.hip) where that is the
+    faster one, in a backward as well. SUB_MGEMM=1 routes decode shapes of 256
+    rows and more to the 256x256 glds GEMM (mfma_gemm.hip).
 
     The latter is NOT on by default: the round-3 measurement
     (profiles/mgemm_r02.md) shows hipBLASLt's MT192/MT256 solutions at 1.3-4.1
@@ -302,7 +379,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
     if (os.environ.get("SUB_MGEMM") != "1" or x.dtype != torch.bfloat16
             or torch.is_grad_enabled() and (
                 x.requires_grad or weight.requires_grad)):
-        return torch.nn.functional.linear(x, weight, bias)
+        y = _many_rows(x, weight, bias)
+        return torch.nn.functional.linear(x, weight, bias) if y is None else y
     ext = _dispatch(x)
     if ext is None:
         return torch.nn.functional.linear(x, weight, bias)

@@ -1,0 +1,515 @@
+// out = a b^T + bias of bf16 matrices of many rows, with either operand as it
+// is or flipped: the products of prompts, and of a training step's forward and
+// backward, which need no transposed copy.
+//
+// Bound by the matrix cores if they are kept busy. A workgroup of eight waves
+// takes 256 x 256 outputs, a wave 128 x 64 of them, 64 of the inner dimension
+// at a time. Two waves share a SIMD. One multiplies while the other reads its
+// next operands from LDS and starts loads from memory; a barrier later they
+// change places (without this turn-taking 1.10 instead of 1.33 PFLOP/s at
+// 4096^3). For that a step of 64 is cut into four phases of a 64 x 32
+// quadrant, 16 matrix instructions each:
+//
+//   phase  1         2         3         4
+//   reads  a low     b high    a high    b low of the next step
+//   takes  low low   low high  high high high low
+//
+// Loads go straight to LDS, a quarter of a step per phase, into the place that
+// the phase before has read, two steps ahead: 112 KB are in flight, and every
+// phase waits for all but the last 12 loads of its thread.
+//
+// LDS holds per step and half of an operand (a region of 128 rows) lines of 128
+// bytes of a row, or, of a flipped operand, lines of 256 bytes of one place of
+// the inner dimension, which transposing reads turn. 16-byte pieces are
+// permuted within their line against bank conflicts: on the way in, by what a
+// lane loads, since what is loaded directly lands in the order of lanes.
+//
+// A chip of 256 CUs takes 256 tiles at a time. Tiles left over from that share
+// the CUs along the inner dimension and leave 32-bit sums to a second kernel.
+//
+// TFLOP/s on a MI355X, the library -> this, m x n x k:
+//   neither flipped  4165 x 12288 x 4096  1045 -> 1343   (a prompt's products)
+//                    4165 x 4096 x 11008   665 -> 1369
+//                    4096 x 18176 x 4544  1130 -> 1420
+//                    4096 x 4096 x 4096   1411 -> 1369   8192^3 1570 -> 1534
+//   b flipped        4096 x 4544 x 18176   693 -> 1325   (gradient of inputs)
+//                    4096 x 4544 x 65024   652 -> 1340
+//   both flipped     18176 x 4544 x 4096  1011 -> 1280   (of weights)
+//                    65024 x 4544 x 4096  1091 -> 1260
+// A workgroup's first loads and last stores are some 4 us; workgroups that go
+// on to a next tile by themselves, with its loads under way, were no faster.
+#include "tile_gemm.h"
+
+#include <algorithm>
+#include <type_traits>
+
+#include "rows_gemm.h"
+
+namespace {
+
+constexpr int TILE = 256, STEP = 64;
+constexpr int THREADS = 512;
+constexpr int REGION = 1024;          // 16-byte pieces of 128 rows x 64
+constexpr int LINES = 4;              // tile rows that an XCD takes side by side
+
+// 32-bit raw buffers of 2 GB; what is past their end reads as zero
+constexpr int RAW = 0x00020000;
+constexpr unsigned PAST = 0xfffffff0u;
+
+DEV_INLINE void barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+DEV_INLINE unsigned lds_address(const void* p) {
+  return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+
+DEV_INLINE short8 join(uint2v a, uint2v b) {
+  return __builtin_bit_cast(short8, (uint4v){a[0], a[1], b[0], b[1]});
+}
+
+// Transposing reads of two, or four, fragments of 16 rows x 64, at `AT` bytes
+// past the fragments' addresses, and the wait for them. (The compiler's own
+// form waits for all direct loads first.)
+template <int AT>
+DEV_INLINE void read_flipped2(short8 (&f)[2][2], unsigned p) {
+  uint2v r[8];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8 offset:%9\n\t"
+      "ds_read_b64_tr_b16 %1, %8 offset:%10\n\t"
+      "ds_read_b64_tr_b16 %2, %8 offset:%11\n\t"
+      "ds_read_b64_tr_b16 %3, %8 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %4, %8 offset:%13\n\t"
+      "ds_read_b64_tr_b16 %5, %8 offset:%14\n\t"
+      "ds_read_b64_tr_b16 %6, %8 offset:%15\n\t"
+      "ds_read_b64_tr_b16 %7, %8 offset:%16\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]),
+        "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+      : "v"(p), "i"(AT), "i"(AT + 1024), "i"(AT + 8), "i"(AT + 1032),
+        "i"(AT + 8192), "i"(AT + 9216), "i"(AT + 8200), "i"(AT + 9224)
+      : "memory");
+  #pragma unroll
+  for (int q = 0; q < 2; ++q)
+    #pragma unroll
+    for (int i = 0; i < 2; ++i)
+      f[i][q] = join(r[q * 4 + i * 2], r[q * 4 + i * 2 + 1]);
+}
+
+template <int AT>
+DEV_INLINE void read_flipped4(short8 (&f)[4][2], unsigned p0, unsigned p1,
+                              unsigned p2, unsigned p3) {
+  uint2v r[16];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %16 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %1, %16 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %2, %17 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %3, %17 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %4, %18 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %5, %18 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %6, %19 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %7, %19 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %8, %16 offset:%22\n\t"
+      "ds_read_b64_tr_b16 %9, %16 offset:%23\n\t"
+      "ds_read_b64_tr_b16 %10, %17 offset:%22\n\t"
+      "ds_read_b64_tr_b16 %11, %17 offset:%23\n\t"
+      "ds_read_b64_tr_b16 %12, %18 offset:%22\n\t"
+      "ds_read_b64_tr_b16 %13, %18 offset:%23\n\t"
+      "ds_read_b64_tr_b16 %14, %19 offset:%22\n\t"
+      "ds_read_b64_tr_b16 %15, %19 offset:%23\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]),
+        "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7]), "=&v"(r[8]), "=&v"(r[9]),
+        "=&v"(r[10]), "=&v"(r[11]), "=&v"(r[12]), "=&v"(r[13]),
+        "=&v"(r[14]), "=&v"(r[15])
+      : "v"(p0), "v"(p1), "v"(p2), "v"(p3), "i"(AT), "i"(AT + 1024),
+        "i"(AT + 8192), "i"(AT + 9216)
+      : "memory");
+  #pragma unroll
+  for (int q = 0; q < 2; ++q)
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
+      f[i][q] = join(r[q * 8 + i * 2], r[q * 8 + i * 2 + 1]);
+}
+
+// Where a tile begins: LINES rows of tiles by columns. The last tiles reach
+// back instead of over the matrix' end; what two of them have is the same.
+DEV_INLINE void tile_of(const TileGemm& g, const TilePlan& p, int tile,
+                        int& m0, int& n0) {
+  const int per = LINES * p.tiles_n, first = tile / per * LINES;
+  const int lines = min(p.tiles_m - first, LINES);
+  m0 = min((first + tile % per % lines) * TILE, g.m - TILE);
+  n0 = min(tile % per / lines * TILE, g.n - TILE);
+}
+
+// Steps come in pairs, one for each half of LDS; past the end they are zeros.
+__host__ __device__ inline int pairs_of(long k) {
+  return (int)((k + 2 * STEP - 1) / (2 * STEP));
+}
+
+// A piece of work: a tile, or a share of one along the inner dimension.
+struct Item {
+  int m0, n0, t0, t1;
+  int share;                      // -1: the whole tile
+};
+
+DEV_INLINE Item item_of(const TileGemm& g, const TilePlan& p, int id) {
+  const int pairs = pairs_of(g.k);
+  Item it;
+  it.t0 = 0;
+  it.t1 = 2 * pairs;
+  it.share = id - p.whole;
+  int tile;
+  if (it.share < 0) {
+    // an XCD, which has every eighth workgroup, takes a run of tiles
+    const int q = p.whole / 8, r = p.whole % 8, xcd = id % 8;
+    tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + id / 8;
+    it.share = -1;
+  } else {
+    const int part = it.share % p.split;
+    tile = p.whole + it.share / p.split;
+    it.t0 = 2 * (int)((long)pairs * part / p.split);
+    it.t1 = 2 * (int)((long)pairs * (part + 1) / p.split);
+    if (p.split == 1) it.share = -1;
+  }
+  tile_of(g, p, tile, it.m0, it.n0);
+  return it;
+}
+
+// Eight outputs of one row.
+DEV_INLINE void store(const TileGemm& g, int row, int col, float4v v,
+                      float4v w) {
+  *reinterpret_cast<uint4*>(g.out + (long)row * g.n + col) =
+      make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
+                 pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3]));
+}
+
+DEV_INLINE float4v bias_of(const TileGemm& g, int col) {
+  if (g.bias == nullptr) return (float4v){0.f, 0.f, 0.f, 0.f};
+  const uint2 u = *reinterpret_cast<const uint2*>(g.bias + col);
+  const float2 x = unpack_bf16x2(u.x), y = unpack_bf16x2(u.y);
+  return (float4v){x.x, x.y, y.x, y.y};
+}
+
+// How the pieces of a region's row r are permuted.
+DEV_INLINE int a_key(int r) { return r & 7; }
+DEV_INLINE int b_key(int r) { return (r & 3) | (r >> 1 & 4); }
+
+// The row and first column of a thread's eight outputs: accumulators (i, 2j)
+// and (i, 2j + 1), whose fragments' rows are interleaved by fours for that.
+DEV_INLINE int out_row(int tid, int i) {
+  return (tid >> 8) * 128 + (i >> 2) * 64 + (i & 3) * 16 + (tid & 15);
+}
+DEV_INLINE int out_col(int tid, int j) {
+  return (tid >> 6 & 3) * 64 + j * 32 + (tid >> 4 & 3) * 8;
+}
+
+template <bool FA, bool FB>
+__global__ __launch_bounds__(THREADS, 2)
+void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
+  // [two steps][a low, a high, b low, b high]
+  __shared__ alignas(1024) uint4 s[2 * 4 * REGION];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, lo = lane & 15, gr = lane >> 4;
+  const int wm = wave >> 2, wn = wave & 3;
+  const Item it = item_of(g, plan, blockIdx.x);
+
+  // Loads: a wave has two KB of a region. Of rows: 8 lines of 128 bytes a KB,
+  // of a flipped operand 4 of 256. off: from the low region's first byte on.
+  unsigned off[2][2];
+  const int piece_f = lane & 15, piece_r = lane & 7;
+  #pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int r = (wave * 2 + p) * 8 + (lane >> 3);
+    const int line = (wave * 2 + p) * 4 + (lane >> 4);
+    const int qa = piece_f ^ ((line & 3) << 1);
+    const int qb = piece_f ^ ((line & 3) << 2);
+    off[0][p] = FA
+        ? (unsigned)(line * g.a_ld + (qa >> 3) * 128 + (qa & 7) * 8) * 2u
+        : (unsigned)(((r >> 6) * 128 + (r & 63)) * g.a_ld) * 2u +
+              (piece_r ^ a_key(r)) * 16;
+    off[1][p] = FB
+        ? (unsigned)(line * g.b_ld + (qb >> 2) * 64 + (qb & 3) * 8) * 2u
+        : (unsigned)(((r >> 5) * 64 + (r & 31)) * g.b_ld) * 2u +
+              (piece_r ^ b_key(r)) * 16;
+  }
+  const long a_step = (FA ? g.a_ld : 1) * STEP * 2;
+  const long b_step = (FB ? g.b_ld : 1) * STEP * 2;
+  const int a_high = (FA ? 1 : g.a_ld) * 64 * 2;
+  const int b_high = (FB ? 1 : g.b_ld) * 32 * 2;
+  // What is loaded, two steps ahead of what is multiplied: by buffer loads,
+  // whose only vector operand is the offset.
+  int lt = it.t0;
+  const char* la = reinterpret_cast<const char*>(
+      g.a + it.m0 * (FA ? 1 : g.a_ld)) + lt * a_step;
+  const char* lb = reinterpret_cast<const char*>(
+      g.b + it.n0 * (FB ? 1 : g.b_ld)) + lt * b_step;
+  // WHOLE: the step is known to be one of the inner dimension's whole ones
+  auto load = [&](auto whole, int buf, int region) {
+    const auto from = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(region < 2 ? la : lb), 0, 0x80000000u, RAW);
+    const int high = region & 1 ? (region < 2 ? a_high : b_high) : 0;
+    uint4* to = s + (buf * 4 + region) * REGION + wave * 128;
+    #pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      unsigned o = off[region >> 1][p];
+      if constexpr (!decltype(whole)::value) {
+        const int r = (wave * 2 + p) * 8 + (lane >> 3);
+        const int at = (region < 2 ? FA : FB)
+            ? (wave * 2 + p) * 4 + (lane >> 4)
+            : (piece_r ^ (region < 2 ? a_key(r) : b_key(r))) * 8;
+        if (at >= g.k - lt * STEP) o = PAST;
+      }
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          from, (__attribute__((address_space(3))) unsigned int*)(to + p * 64),
+          16, o, high, 0, 0);
+    }
+  };
+  auto advance = [&]() {
+    ++lt;
+    la += a_step;
+    lb += b_step;
+  };
+
+  float4v acc[8][4];
+  short8 af[4][2], bl[2][2][2], bh[2][2];
+
+  // flipped: a lane's place in a transposing read of the first fragment
+  const int place16 = ((gr * 8 + (lo >> 2)) * 16) * 16;
+  const unsigned base = lds_address(s);
+  const unsigned at_a = base + place16 + (lo & 1) * 8 +
+      (((wm * 8 + ((lo & 3) >> 1)) ^ ((lo >> 2) << 1)) * 16);
+  const unsigned at_b = base + place16 +
+      (((wn * 4 + (lo & 3)) ^ ((lo >> 2) << 2)) * 16);
+  auto read_a = [&](auto buf, auto half) {
+    constexpr int BUF = decltype(buf)::value, H = decltype(half)::value;
+    if constexpr (FA) {
+      const unsigned p = at_a + BUF * 4 * REGION * 16;
+      read_flipped4<H * REGION * 16>(af, p, p ^ 32, p ^ 64, p ^ 96);
+    } else {
+      const uint4* r = s + (BUF * 4 + H) * REGION + (wm * 64 + lo) * 8;
+      #pragma unroll
+      for (int i = 0; i < 4; ++i)
+        #pragma unroll
+        for (int q = 0; q < 2; ++q)
+          af[i][q] = *reinterpret_cast<const short8*>(
+              r + i * 128 + ((q * 4 + gr) ^ (lo & 7)));
+    }
+  };
+  auto read_b = [&](auto buf, auto half, short8 (&f)[2][2]) {
+    constexpr int BUF = decltype(buf)::value, H = decltype(half)::value;
+    if constexpr (FB) {
+      const unsigned p = at_b + BUF * 4 * REGION * 16;
+      read_flipped2<(2 + H) * REGION * 16>(f, p);
+    } else {
+      const uint4* r = s + (BUF * 4 + 2 + H) * REGION +
+                       (wn * 32 + (lo >> 2) * 8 + (lo & 3)) * 8;
+      #pragma unroll
+      for (int i = 0; i < 2; ++i)
+        #pragma unroll
+        for (int q = 0; q < 2; ++q)
+          f[i][q] = *reinterpret_cast<const short8*>(
+              r + i * 32 + ((q * 4 + gr) ^ (lo & 7)));
+    }
+  };
+  // the phase's reads are done, and so are the loads of the next one's
+  auto turn = [&]() {
+    wait_lds_reads();
+    wait_loads<12>();
+    barrier();
+  };
+  auto take = [&](int i0, int j0, const short8 (&f)[2][2]) {
+    #pragma unroll
+    for (int q = 0; q < 2; ++q)
+      #pragma unroll
+      for (int i = 0; i < 4; ++i)
+        #pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i0 + i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              f[j][q], af[i][q], acc[i0 + i][j0 + j], 0, 0, 0);
+    barrier();
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, 0> low{};
+  constexpr integral_constant<int, 1> high{};
+  auto step = [&](auto buf, auto whole) {
+    constexpr int B = decltype(buf)::value;
+    constexpr integral_constant<int, B ^ 1> other{};
+    read_a(buf, low);
+    load(whole, B, 2);
+    turn();
+    take(0, 0, bl[B]);
+    read_b(buf, high, bh);
+    load(whole, B, 0);
+    turn();
+    take(0, 2, bh);
+    read_a(buf, high);
+    load(whole, B, 3);
+    turn();
+    take(4, 2, bh);
+    read_b(other, low, bl[B ^ 1]);
+    load(whole, B, 1);
+    advance();
+    turn();
+    take(4, 0, bl[B]);
+  };
+  constexpr std::true_type whole{};
+  constexpr std::false_type any{};
+
+  #pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    load(any, t, 2);
+    load(any, t, 0);
+    load(any, t, 3);
+    load(any, t, 1);
+    advance();
+  }
+  #pragma unroll
+  for (int i = 0; i < 8; ++i)
+    #pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
+  wait_loads<12>();
+  barrier();
+  read_b(low, low, bl[0]);
+  wait_lds_reads();
+  barrier();
+  if (wm == 1) barrier();         // half of the waves run half a phase behind
+  const int pairs = (it.t1 - it.t0) / 2;
+  // pairs whose loads, a pair ahead, are all of whole steps
+  const int hot = min(pairs - 1, (g.k / STEP - it.t0) / 2 - 1);
+  int t = 0;
+  #pragma unroll 1
+  for (; t < hot; ++t) {
+    step(low, whole);
+    step(high, whole);
+  }
+  #pragma unroll 1
+  for (; t < pairs; ++t) {        // loads past the end are zeros
+    step(low, any);
+    step(high, any);
+  }
+  if (wm == 0) barrier();
+  wait_loads<0>();                // no load outlives its workgroup's LDS
+
+  const int tid = threadIdx.x;
+  if (it.share >= 0) {
+    float4v* to = shares + (long)it.share * (32 * THREADS) + tid;
+    #pragma unroll
+    for (int i = 0; i < 8; ++i)
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) to[(i * 4 + j) * THREADS] = acc[i][j];
+    return;
+  }
+  float4v add[4];
+  #pragma unroll
+  for (int j = 0; j < 4; ++j)
+    add[j] = bias_of(g, it.n0 + out_col(tid, j >> 1) + (j & 1) * 4);
+  #pragma unroll
+  for (int i = 0; i < 8; ++i)
+    #pragma unroll
+    for (int j = 0; j < 2; ++j)
+      store(g, it.m0 + out_row(tid, i), it.n0 + out_col(tid, j),
+            acc[i][2 * j] + add[2 * j], acc[i][2 * j + 1] + add[2 * j + 1]);
+}
+
+// The shares of the tiles left over are added up, a sixteenth of a tile per
+// workgroup.
+__global__ __launch_bounds__(THREADS)
+void tile_sum_kernel(TileGemm g, TilePlan plan,
+                     const float4v* __restrict__ shares) {
+  int m0, n0;
+  tile_of(g, plan, plan.whole + blockIdx.x, m0, n0);
+  const int tid = threadIdx.x;
+  const float4v* from = shares +
+      (long)blockIdx.x * plan.split * (32 * THREADS) + tid;
+  float4v v[2];
+  const int i = blockIdx.y >> 1, j = blockIdx.y & 1;
+  const int col = n0 + out_col(tid, j);
+  #pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int at = (i * 4 + j * 2 + e) * THREADS;
+    v[e] = from[at];
+    #pragma unroll 4
+    for (int p = 1; p < plan.split; ++p)
+      v[e] += from[(long)p * 32 * THREADS + at];
+    v[e] += bias_of(g, col + e * 4);
+  }
+  store(g, m0 + out_row(tid, i), col, v[0], v[1]);
+}
+
+}  // namespace
+
+// A tile's offsets within an operand fit 32 bits, 16-byte pieces of it lie
+// within a row.
+bool tile_gemm_takes(long m, long n, long k, long a_ld, long b_ld,
+                     bool a_flipped, bool b_flipped) {
+  auto fits = [&](long rows, long ld, bool flipped) {
+    return ld % 8 == 0 && (flipped ? rows % 8 == 0 && ld >= rows
+                                   : k % 8 == 0 && ld >= k) &&
+           ld < (1L << 21);
+  };
+  return m >= TILE && n >= TILE && k > STEP && n % 8 == 0 &&
+         m < (1L << 30) && n < (1L << 30) && k < (1L << 30) &&
+         fits(m, a_ld, a_flipped) && fits(n, b_ld, b_flipped);
+}
+
+TilePlan tile_gemm_plan(long m, long n, long k) {
+  TilePlan p;
+  p.tiles_m = (int)((m + TILE - 1) / TILE);
+  p.tiles_n = (int)((n + TILE - 1) / TILE);
+  const long tiles = (long)p.tiles_m * p.tiles_n;
+  const long steps = 2 * pairs_of(k);
+  const long rest = tiles % 256, rounds = tiles / 256;
+  // us on a MI355X: a step of a tile 1.5, a round's beginning and end 5, the
+  // sum of shares 5 and their way through memory
+  const double full = rounds * (steps * 1.5 + 5.);
+  p.whole = (int)tiles;
+  p.split = 1;
+  p.us = full + (rest ? steps * 1.5 + 5. : 0.);
+  for (int s = 2; rest && rest * s <= 256 && steps / s >= 4; ++s) {
+    const double us = full + (steps + s - 1) / s * 1.5 + 10. +
+                      rest * s * (0.262144 * 2 / 5.);
+    if (us < p.us) {
+      p.us = us;
+      p.whole = (int)(tiles - rest);
+      p.split = s;
+    }
+  }
+  return p;
+}
+
+// Whether the library's product would take longer. What it takes is no smooth
+// function of sizes; on a MI355X, planned PFLOP/s and what this one gains:
+//   neither flipped   below 0.9: 0.75 to 1.18 times as fast, mostly slower
+//                     (2048 x 4096 x 4096: 0.81, 0.85); above: 0.94 to 2.06
+//                     (4165 x 4096 x 11008: 1.19, 2.06; 4096 x 18176 x 4544:
+//                     1.25, 1.26; 2331 x 32000 x 2048: 1.15, 0.96); whole tiles
+//                     in whole rounds, which need neither split nor reach back:
+//                     0.95 to 0.99
+//   b flipped         0.39 to 0.57: 0.87 to 0.96; from 0.7: 1.02 to 2.05
+//   both flipped      0.39: 0.90; from 0.7: 1.00 to 1.41
+bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped) {
+  const TilePlan p = tile_gemm_plan(m, n, k);
+  const double rate = 2e-9 * m * n * k / p.us;        // PFLOP/s
+  if (a_flipped || b_flipped) return rate >= 0.7;
+  const bool even = m % TILE == 0 && n % TILE == 0 &&
+                    (long)p.tiles_m * p.tiles_n % 256 == 0;
+  return rate >= 0.9 && !even;
+}
+
+void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,
+                      hipStream_t stream) {
+  float4v* sh = reinterpret_cast<float4v*>(shares);
+  const dim3 grid(plan.whole + plan.rest() * plan.split);
+  auto kernel = g.a_flipped
+      ? (g.b_flipped ? tile_gemm_kernel<true, true>
+                     : tile_gemm_kernel<true, false>)
+      : (g.b_flipped ? tile_gemm_kernel<false, true>
+                     : tile_gemm_kernel<false, false>);
+  kernel<<<grid, dim3(THREADS), 0, stream>>>(g, plan, sh);
+  if (plan.split > 1)
+    tile_sum_kernel<<<dim3(plan.rest(), 16), dim3(THREADS), 0, stream>>>(
+        g, plan, sh);
+}

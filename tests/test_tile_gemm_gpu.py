@@ -1,0 +1,92 @@
+"""Products of many rows (tile_gemm.hip) against 64 bits: either operand
+flipped, at the ends of tiles, of steps of 64 of the inner dimension and of
+their pairs, with tiles that are left over from a round."""
+
+import pytest
+import torch
+
+from substratus_amd import _C, ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def close(got, a, b, bias=None):
+    """Half a bf16 step (2^-9), and 32-bit sums in any order (2^-18 of the sum
+    of magnitudes for some thousands of addends)."""
+    want = a.double() @ b.double().T
+    room = 2.0 ** -18 * (a.double().abs() @ b.double().abs().T)
+    if bias is not None:
+        want = want + bias.double()
+    assert got.dtype == torch.bfloat16 and got.shape == want.shape
+    off = (got.double() - want).abs()
+    assert bool((off <= 2.0 ** -8 * want.abs() + room + 1e-30).all())
+
+
+def operand(rows, k, flipped, pad):
+    shape = (k, rows) if flipped else (rows, k)
+    whole = torch.full((shape[0], shape[1] + pad), torch.nan, device=DEV)
+    whole[:, :shape[1]] = torch.randn(shape, device=DEV)
+    return whole.bfloat16()[:, :shape[1]]       # what is beside is no number
+
+
+# the inner dimension: two steps at least; within a pair, whole, one over
+@pytest.mark.parametrize("k", [72, 128, 136, 192, 248, 1096])
+@pytest.mark.parametrize("m,n", [(256, 256), (264, 256), (256, 1000),
+                                 (776, 520)])
+@pytest.mark.parametrize("fa", [False, True])
+@pytest.mark.parametrize("fb", [False, True])
+def test_tile_gemm(m, n, k, fa, fb):
+    torch.manual_seed(m + n + k)
+    inner = k + 3 if fa and fb else k           # lines of any number
+    a, b = operand(m, inner, fa, 8), operand(n, inner, fb, 16)
+    bias = torch.randn(n, device=DEV).bfloat16() if k % 3 == 0 else None
+    got = _C.tile_gemm(a, b, bias, fa, fb)
+    close(got, a.T if fa else a, b.T if fb else b, bias)
+
+
+@pytest.mark.parametrize("m,n,k,fa,fb", [
+    (1000, 1024, 4544, False, False),           # all shared
+    (4360, 4104, 1032, False, True),            # a round, and some
+    (2304, 8192, 520, True, True)])
+def test_rounds(m, n, k, fa, fb):
+    a, b = operand(m, k, fa, 0), operand(n, k, fb, 0)
+    got = _C.tile_gemm(a, b, None, fa, fb)
+    close(got, a.T if fa else a, b.T if fb else b)
+    assert torch.equal(got, _C.tile_gemm(a, b, None, fa, fb))
+
+
+def test_rows_of_any_number():
+    """Rows that are not flipped need not come in eights."""
+    a, b = operand(321, 192, False, 0), operand(264, 192, False, 0)
+    close(_C.tile_gemm(a, b, None, False, False), a, b)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_gradients(bias):
+    """ops.linear at a size where all three products pay."""
+    torch.manual_seed(5)
+    x = torch.randn(2, 1001, 4096, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(8192, 4096, device=DEV) / 64).bfloat16() \
+        .requires_grad_()
+    bs = torch.randn(8192, device=DEV).bfloat16().requires_grad_() \
+        if bias else None
+    y = ops.linear(x, w, bs)
+    dy = torch.randn(2, 1001, 8192, device=DEV).bfloat16()
+    rows, drows = x.detach().view(-1, 4096), dy.view(-1, 8192)
+    close(y.detach().view(-1, 8192), rows, w.detach(),
+          None if bs is None else bs.detach())
+    inputs = [t for t in (x, w, bs) if t is not None]
+    got = torch.autograd.grad(y, inputs, dy, retain_graph=True)
+    close(got[0].view(-1, 4096), drows, w.detach().T)
+    close(got[1], drows.T, rows.T)
+    if bias:
+        assert torch.equal(got[2], drows.sum(0))
+    # gradients that are no rows, and gradients of gradients
+    g, = torch.autograd.grad(y.sum(), x, retain_graph=True)
+    close(g.view(-1, 4096), torch.ones_like(drows), w.detach().T)
+    first, = torch.autograd.grad(y, x, dy, create_graph=True)
+    again, = torch.autograd.grad(first.float().sum(), w)
+    want = torch.nn.functional.linear(x, w, bs)
+    first, = torch.autograd.grad(want, x, dy, create_graph=True)
+    assert torch.equal(again, torch.autograd.grad(first.float().sum(), w)[0])
