@@ -56,6 +56,14 @@ def fused_norm_residual(deltas: tuple, h: torch.Tensor, norm: "NormParams",
     return got
 
 
+def normed_product(lin: Linear, deltas: tuple, h: torch.Tensor,
+                   norm: "NormParams", eps: float, **how):
+    """(lin of norm(h + deltas), h + deltas) in one kernel, or None."""
+    if not norm.rms or len(deltas) != 1:
+        return None
+    return lin.normed(deltas[0], h, norm.weight, eps, **how)
+
+
 class NormParams(nn.Module):
     def __init__(self, size: int, rms: bool, device=None, dtype=None):
         super().__init__()
@@ -128,28 +136,40 @@ class Block(nn.Module):
         return (q.view(n, self.n_heads, d), k.view(n, self.n_kv_heads, d),
                 v.view(n, self.n_kv_heads, d))
 
-    def _mlp(self, y: torch.Tensor) -> torch.Tensor:
+    def _mlp_up(self, y: torch.Tensor) -> torch.Tensor:
         if self.cfg.activation == "silu":
-            return self.w_down(self.w_gateup.gated(y))
-        return self.w_down(ops.gelu(self.w_up(y)))
+            return self.w_gateup.gated(y)
+        return ops.gelu(self.w_up(y))
+
+    def _mlp(self, y: torch.Tensor) -> torch.Tensor:
+        return self.w_down(self._mlp_up(y))
 
     # -- decode -------------------------------------------------------------
-    def decode_ops(self, y: torch.Tensor, h: torch.Tensor,
+    def decode_ops(self, h: torch.Tensor, deltas: tuple,
                    positions: torch.Tensor,
                    k_cache: torch.Tensor, v_cache: torch.Tensor,
                    slots: torch.Tensor, block_table: torch.Tensor,
                    seq_lens: torch.Tensor):
         """Generator form of the decode block: yields after each op group
-        (qkv GEMM | rope+attention | o GEMM | up GEMM | down GEMM) so the
-        dual-stream runner (serve/graph_runner.py) can interleave two
+        (norm + qkv GEMM | rope+attention | o GEMM | up GEMM | down GEMM) so
+        the dual-stream runner (serve/graph_runner.py) can interleave two
         half-batches op-by-op — the trailing half's GEMMs re-read weights
         the leading half just streamed (LLC-hot) while its attention
         overlaps the leader's compute. forward_decode drives this
         generator to completion, so single-stream numerics are by
-        construction identical."""
+        construction identical.
+
+        h: the residual stream, deltas: what is still to be added to it, which
+        this block's first norm does; the same is returned."""
         cache = ops.Cache(positions, k_cache, v_cache, slots, self.rope_theta)
-        q = self.wqkv.heads(y, cache)
-        qkv = self.wqkv(y) if q is None else None
+        got = None if self.parallel_attn else normed_product(
+            self.wqkv, deltas, h, self.norm1, self.eps, cache=cache)
+        if got is not None:
+            q, h = got
+        else:
+            y, h = fused_norm_residual(deltas, h, self.norm1, self.eps)
+            q = self.wqkv.heads(y, cache)
+            qkv = self.wqkv(y) if q is None else None
         yield
         if q is None:
             q, k, v = self._split_qkv(qkv)
@@ -160,43 +180,22 @@ class Block(nn.Module):
         attn_out = self.wo(a.reshape(a.shape[0], -1))
         yield
         if self.parallel_attn:
-            mlp_in = self.norm2(h, self.eps) if self.parallel_norms else y
-            if self.cfg.activation == "silu":
-                a = self.w_gateup.gated(mlp_in)
-                yield
-                out = self.w_down(a)
-            else:
-                u = self.w_up(mlp_in)
-                yield
-                out = self.w_down(ops.gelu(u))
-            return (attn_out, out), h
-        y2, h = fused_norm_residual((attn_out,), h, self.norm2, self.eps)
+            if self.parallel_norms:
+                y = self.norm2(h, self.eps)
+            up = self._mlp_up(y)
+            yield
+            return h, (attn_out, self.w_down(up))
+        got = None
         if self.cfg.activation == "silu":
-            a = self.w_gateup.gated(y2)
-            yield
-            out = self.w_down(a)
+            got = normed_product(self.w_gateup, (attn_out,), h, self.norm2,
+                                 self.eps, gated=True)
+        if got is not None:
+            up, h = got
         else:
-            u = self.w_up(y2)
-            yield
-            out = self.w_down(ops.gelu(u))
-        return (out,), h
-
-    def forward_decode(self, y: torch.Tensor, h: torch.Tensor,
-                       positions: torch.Tensor,
-                       k_cache: torch.Tensor, v_cache: torch.Tensor,
-                       slots: torch.Tensor, block_table: torch.Tensor,
-                       seq_lens: torch.Tensor) -> tuple[tuple, torch.Tensor]:
-        """y: normalized input (this block's norm1 already applied by the
-        caller's fused residual+norm); h: the residual stream. Returns
-        (deltas, h) where deltas are this block's outputs to be added by the
-        NEXT norm's fused residual."""
-        gen = self.decode_ops(y, h, positions, k_cache, v_cache, slots,
-                              block_table, seq_lens)
-        while True:
-            try:
-                next(gen)
-            except StopIteration as e:
-                return e.value
+            y, h = fused_norm_residual((attn_out,), h, self.norm2, self.eps)
+            up = self._mlp_up(y)
+        yield
+        return h, (self.w_down(up),)
 
     # -- prefill ------------------------------------------------------------
     def forward_prefill(self, h: torch.Tensor, deltas: tuple,
@@ -313,18 +312,20 @@ class CausalLM(nn.Module):
         h = self.embed_tokens(tokens)
         if self.cfg.learned_pos_emb:
             h = h + self.embed_positions(positions.long())
-        # fused residual+norm chain: each block's output delta is added to
-        # the residual stream inside the NEXT norm kernel
-        y = self.blocks[0].norm1(h, self.eps)
-        yield
-        for i, (blk, (kc, vc)) in enumerate(zip(self.blocks, kv_caches)):
-            deltas, h = yield from blk.decode_ops(y, h, positions, kc, vc,
-                                                 slots, block_table,
-                                                 seq_lens)
-            nxt = (self.blocks[i + 1].norm1 if i + 1 < len(self.blocks)
-                   else self.final_norm)
-            y, h = fused_norm_residual(deltas, h, nxt, self.eps)
+        # each block's outputs are added to the residual stream inside the
+        # NEXT norm
+        deltas = ()
+        for blk, (kc, vc) in zip(self.blocks, kv_caches):
+            h, deltas = yield from blk.decode_ops(h, deltas, positions, kc,
+                                                  vc, slots, block_table,
+                                                  seq_lens)
             yield
+        if self.lm_head is not None:
+            got = normed_product(self.lm_head, deltas, h, self.final_norm,
+                                 self.eps)
+            if got is not None:
+                return got[0]
+        y, _ = fused_norm_residual(deltas, h, self.final_norm, self.eps)
         return self._logits(y)
 
     def forward_decode(self, tokens: torch.Tensor, positions: torch.Tensor,

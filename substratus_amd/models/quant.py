@@ -213,12 +213,28 @@ class QuantLinear(nn.Module):
             x.dtype == torch.bfloat16 and cache.takes(x, n) else None
         if ext is None:
             return None
-        hkv, d = cache.k.shape[1], cache.k.shape[3]
-        q = torch.empty(x2.shape[0], n // d - 2 * hkv, d,
-                        dtype=torch.bfloat16, device=x.device)
+        q = x2.new_empty(*ops._columns(x2.shape[0], n, False, cache))
         ext.quant_heads(q, x2.contiguous(), self.scales, self.qs, self.quant,
                         *cache)
         return q
+
+    def normed(self, delta: torch.Tensor, h: torch.Tensor,
+               norm: torch.Tensor, eps: float, gated: bool = False,
+               cache: Optional[ops.Cache] = None):
+        """(the outputs for RMSNorm of h + delta, h + delta), gated or appended
+        as above, in the same kernel, or None."""
+        if self.bias is not None or not ops.norm_goes_in(delta, h, norm):
+            return None
+        n = self.out_features
+        ext = self._few_rows(h, gated or cache is not None)
+        if ext is None or cache is not None and not cache.takes(h, n):
+            return None
+        y = h.new_empty(*ops._columns(h.shape[0], n, gated, cache))
+        total = torch.empty_like(h)
+        ext.quant_normed(y, total, delta, h, norm, eps, self.scales, self.qs,
+                         self.quant, gated,
+                         *(cache or (None,) * 4 + (0.0,)))
+        return y, total
 
 
 def quantize_model(model: nn.Module, quant: str) -> nn.Module:

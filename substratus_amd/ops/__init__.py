@@ -478,10 +478,50 @@ def linear_heads(x: torch.Tensor, weight: torch.Tensor,
     if few is None or not cache.takes(x, n):
         return None
     rows, ext = few
-    hkv, d = cache.k.shape[1], cache.k.shape[3]
-    q = rows.new_empty(rows.shape[0], n // d - 2 * hkv, d)
+    q = rows.new_empty(*_columns(rows.shape[0], n, False, cache))
     ext.rows_heads(q, rows, weight, bias, *cache)
     return q
+
+
+def norm_goes_in(delta: torch.Tensor, h: torch.Tensor,
+                 norm: torch.Tensor) -> bool:
+    """Whether a product may make its rows itself, as the RMSNorm of
+    h + delta. Up to 4 rows of 8192 numbers in all: every workgroup makes them
+    for itself."""
+    ext = _load_ext()
+    return (ext is not None and h.dim() == 2 and h.shape == delta.shape
+            and norm.shape == h.shape[1:] and h.numel() > 0
+            and ext.norm_rows_take(*h.shape)
+            and all(t.is_cuda and t.device == h.device
+                    and t.dtype == torch.bfloat16 and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (delta, h, norm))
+            and inference_only(delta, h, norm))
+
+
+def linear_normed(delta: torch.Tensor, h: torch.Tensor, norm: torch.Tensor,
+                  eps: float, weight: torch.Tensor,
+                  bias: Optional[torch.Tensor], gated: bool = False,
+                  cache: Optional[Cache] = None):
+    """(what becomes of F.linear of norm(h + delta), h + delta) in one kernel,
+    or None where it is not made for that: the product, gated as
+    linear_gated's, or with a cache linear_heads' queries."""
+    if not norm_goes_in(delta, h, norm):
+        return None
+    few = _few_rows(h, weight, bias, gated or cache is not None)
+    m, n = h.shape[0], weight.shape[0]
+    if few is None or cache is not None and not cache.takes(h, n):
+        return None
+    y, total = h.new_empty(*_columns(m, n, gated, cache)), torch.empty_like(h)
+    few[1].rows_normed(y, total, delta, h, norm, eps, weight, bias, gated,
+                       *(cache or (None,) * 4 + (0.0,)))
+    return y, total
+
+
+def _columns(m: int, n: int, gated: bool, cache: Optional[Cache]) -> tuple:
+    if cache is None:
+        return m, n // 2 if gated else n
+    d = cache.k.shape[3]
+    return m, n // d - 2 * cache.k.shape[1], d
 
 
 def silu_mul(x: torch.Tensor) -> torch.Tensor:

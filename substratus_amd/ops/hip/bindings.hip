@@ -560,7 +560,7 @@ void rope_split_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 
 void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> bias, bool gated,
-                  const Heads* heads) {
+                  const Heads* heads, const NormOf* norm = nullptr) {
   check_bf16(y, "y"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
               x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0,
@@ -579,7 +579,7 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
     bp = bfc(*bias);
   }
   launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols,
-                   gated, heads, stream());
+                   gated, heads, norm, stream());
   post_launch_check("rows_gemm");
 }
 
@@ -649,7 +649,7 @@ bool quant_rows_ok(long m, long n, long k, const std::string& quant,
 
 void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
                    torch::Tensor qs, const std::string& quant, bool gated,
-                   const Heads* heads) {
+                   const Heads* heads, const NormOf* norm = nullptr) {
   check_bf16(y, "y"); check_bf16(x, "x");
   TORCH_CHECK(scales.scalar_type() == torch::kHalf, "scales must be fp16");
   TORCH_CHECK(qs.scalar_type() == torch::kByte, "qs must be uint8");
@@ -667,7 +667,7 @@ void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
   if (!aligned16(scales)) scales = scales.clone();
   launch_rows_quant(bf(y), bfc(x), scales.data_ptr(),
                     qs.data_ptr<unsigned char>(), m, n, k, q, gated, heads,
-                    stream());
+                    norm, stream());
   post_launch_check("quant_rows");
 }
 
@@ -675,6 +675,57 @@ void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
 void quant_rows(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
                 torch::Tensor qs, const std::string& quant, bool gated) {
   quant_rows_to(y, x, scales, qs, quant, gated, nullptr);
+}
+
+// The products above of RMS(h + delta) weight as x; sum = h + delta. Heads
+// where a cache is given.
+NormOf norm_of(const torch::Tensor& sum, const torch::Tensor& delta,
+               const torch::Tensor& h, const torch::Tensor& weight,
+               double eps) {
+  const long k = weight.numel();
+  TORCH_CHECK(h.dim() == 2 && h.size(1) == k && h.size(0) > 0 &&
+              norm_rows_take(h.size(0), k), "normed rows: unsupported shape");
+  check_rows(weight, k, "norm weight");
+  check_rows(h, h.numel(), "h"); check_rows(delta, h.numel(), "delta");
+  check_rows(sum, h.numel(), "sum");
+  return {bfc(delta), bfc(h), bfc(weight),
+          const_cast<bf16_t*>(bfc(sum)), (float)eps};
+}
+
+struct Where {
+  c10::optional<torch::Tensor> positions, k_cache, v_cache, slots;
+  double theta;
+  Heads heads;
+  const Heads* of(const torch::Tensor& q) {
+    if (!positions) return nullptr;
+    heads = heads_of(q, *positions, *k_cache, *v_cache, *slots, theta);
+    return &heads;
+  }
+};
+
+void rows_normed(torch::Tensor y, torch::Tensor sum, torch::Tensor delta,
+                 torch::Tensor h, torch::Tensor norm, double eps,
+                 torch::Tensor w, c10::optional<torch::Tensor> bias,
+                 bool gated, c10::optional<torch::Tensor> positions,
+                 c10::optional<torch::Tensor> k_cache,
+                 c10::optional<torch::Tensor> v_cache,
+                 c10::optional<torch::Tensor> slots, double theta) {
+  Where where{positions, k_cache, v_cache, slots, theta};
+  const NormOf of = norm_of(sum, delta, h, norm, eps);
+  rows_gemm_to(y, h, w, bias, gated, where.of(y), &of);
+}
+
+void quant_normed(torch::Tensor y, torch::Tensor sum, torch::Tensor delta,
+                  torch::Tensor h, torch::Tensor norm, double eps,
+                  torch::Tensor scales, torch::Tensor qs,
+                  const std::string& quant, bool gated,
+                  c10::optional<torch::Tensor> positions,
+                  c10::optional<torch::Tensor> k_cache,
+                  c10::optional<torch::Tensor> v_cache,
+                  c10::optional<torch::Tensor> slots, double theta) {
+  Where where{positions, k_cache, v_cache, slots, theta};
+  const NormOf of = norm_of(sum, delta, h, norm, eps);
+  quant_rows_to(y, h, scales, qs, quant, gated, where.of(y), &of);
 }
 
 // rows_heads of a quantized weight matrix
@@ -919,6 +970,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_gemm", &tile_gemm);
   m.def("tile_gemm_good", &tile_gemm_good);
   m.def("rows_heads", &rows_heads);
+  m.def("rows_normed", &rows_normed);
+  m.def("quant_normed", &quant_normed);
+  m.def("norm_rows_take", &norm_rows_take);
   m.def("rope_split_append", &rope_split_append);
   m.def("quant_heads", &quant_heads);
   m.def("rows_gemm_ok", &rows_gemm_ok);

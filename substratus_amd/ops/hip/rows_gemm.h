@@ -70,6 +70,102 @@ DEV_INLINE int second_half(int n, const Heads& heads) {
   return C == Columns::HEADS ? heads.d / 2 : n / 2;
 }
 
+// x as the norm of a sum, made by the product itself: RMS of h + delta, which
+// the first workgroup stores in sum. A row's 1/deviation only scales its
+// results, so a workgroup multiplies (h + delta) * weight, rounded like a
+// normed row, and scales at the end; it sums squares meanwhile. On a MI355X, us
+// of a decode step with a launch for each norm -> in the products: 737 -> 688
+// (1 row, 16 layers of 2048), 630 -> 614 (1 row, 8 layers of 5120, q4_0). Every
+// workgroup makes all of x: more than 8192 numbers of it would take LDS from
+// other workgroups.
+struct NormOf {
+  const bf16_t *delta, *h, *weight;
+  bf16_t* sum;
+  float eps;
+};
+
+constexpr int NORM_ROWS = 4;            // of x, at most
+constexpr int NORM_PIECES = 1024;       // 16-byte pieces of x in LDS, at most
+
+// A thread's pieces of h + delta on their way, loaded before a workgroup's
+// first weights so that their wait is not the weights'. A row of x in LDS is
+// a piece longer than k, against bank conflicts.
+template <int THREADS>
+struct NormRows {
+  static constexpr int PER = (NORM_PIECES + THREADS - 1) / THREADS;
+  uint4 h[PER], d[PER], w[PER];
+
+  DEV_INLINE void load(const NormOf& n, int m, int k) {
+    const int row = k / 8, all = m * row;
+    #pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int p = min((int)threadIdx.x + i * THREADS, all - 1);
+      h[i] = reinterpret_cast<const uint4*>(n.h)[p];
+      d[i] = reinterpret_cast<const uint4*>(n.delta)[p];
+      w[i] = reinterpret_cast<const uint4*>(n.weight)[p % row];
+    }
+  }
+
+  // x to LDS, and each wave's sum of squares of every row
+  DEV_INLINE void put(const NormOf& n, int m, int k, uint4* x,
+                      float (*squares)[NORM_ROWS]) {
+    const int row = k / 8, all = m * row;
+    float ss[NORM_ROWS] = {0.f, 0.f, 0.f, 0.f};
+    #pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int p = (int)threadIdx.x + i * THREADS;
+      if (p >= all) break;
+      const unsigned a[4] = {h[i].x, h[i].y, h[i].z, h[i].w};
+      const unsigned b[4] = {d[i].x, d[i].y, d[i].z, d[i].w};
+      const unsigned c[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+      unsigned s[4], o[4];
+      float q = 0.f;
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float2 x0 = unpack_bf16x2(a[j]), x1 = unpack_bf16x2(b[j]);
+        s[j] = pack_bf16x2(x0.x + x1.x, x0.y + x1.y);
+        const float2 v = unpack_bf16x2(s[j]), g = unpack_bf16x2(c[j]);
+        q += v.x * v.x + v.y * v.y;
+        o[j] = pack_bf16x2(v.x * g.x, v.y * g.y);
+      }
+      const int r = p / row;
+      #pragma unroll
+      for (int e = 0; e < NORM_ROWS; ++e) ss[e] += r == e ? q : 0.f;
+      x[p + r] = make_uint4(o[0], o[1], o[2], o[3]);
+      if (blockIdx.x == 0)
+        reinterpret_cast<uint4*>(n.sum)[p] = make_uint4(s[0], s[1], s[2],
+                                                        s[3]);
+    }
+    #pragma unroll
+    for (int e = 0; e < NORM_ROWS; ++e) ss[e] = wave_sum(ss[e]);
+    if (threadIdx.x % WAVE == 0) {
+      #pragma unroll
+      for (int e = 0; e < NORM_ROWS; ++e)
+        squares[threadIdx.x / WAVE][e] = ss[e];
+    }
+  }
+};
+
+template <int WAVES>
+DEV_INLINE float norm_scale(const float (*squares)[NORM_ROWS], int r, int k,
+                            float eps) {
+  float s = 0.f;
+  #pragma unroll
+  for (int w = 0; w < WAVES; ++w) s += squares[w][r];
+  return rsqrtf(s / (float)k + eps);
+}
+
+// LDS is written by all waves, and no load has to have arrived.
+DEV_INLINE void lds_barrier() {
+  wait_lds_reads();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+inline bool norm_rows_take(long m, long k) {
+  return m <= NORM_ROWS && k % 8 == 0 && m * (k / 8) <= NORM_PIECES;
+}
+
 // The weight row behind row r of the 16 that a workgroup from column n0 on
 // multiplies.
 template <Columns C>
@@ -121,7 +217,7 @@ DEV_INLINE void finish_heads(bf16_t* y, long y_ld, const Heads& heads, int r,
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
                       long y_ld, bool gated, const Heads* heads,
-                      hipStream_t stream);
+                      const NormOf* norm, hipStream_t stream);
 
 DEV_INLINE float silu_times(float g, float u) {
   return g / (1.f + __expf(-g)) * u;

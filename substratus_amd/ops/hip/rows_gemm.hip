@@ -24,23 +24,34 @@
 // two operand tiles of x per wave, the library is the faster one.
 #include "rows_gemm.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int KW = 4;             // waves, which share k
 constexpr int P = 4;              // stages in flight
 constexpr int U = 2;              // 32-column chunks of a stage
 constexpr int TILE = 64;          // 16-byte pieces of 16 rows x 32 columns
-constexpr int STAGE = U * 2 * TILE;
-constexpr int LOADS = U * 2;      // of a stage
 constexpr int PAD = 4;
 
-template <Columns C>
+template <Columns C, bool NORM>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       const bf16_t* __restrict__ w,
                       const bf16_t* __restrict__ bias, int m, int n, int k,
-                      long x_ld, long y_ld, Heads heads) {
-  __shared__ alignas(16) uint4 s_all[KW * P * STAGE];
+                      long x_ld, long y_ld, Heads heads,
+                      NormOf norm) {
+  // (normed x does not go through the ring)
+  constexpr int STAGE = U * (NORM ? 1 : 2) * TILE;
+  constexpr int LOADS = U * (NORM ? 1 : 2);
+  constexpr int RING = KW * P * STAGE;
+  // one array: beside a second one the compiler guards every LDS read against
+  // the direct loads in flight, and waits for them
+  __shared__ alignas(16)
+      uint4 s_all[RING + (NORM ? NORM_PIECES + NORM_ROWS + KW : 0)];
+  uint4* s_x = s_all + RING;
+  auto squares = reinterpret_cast<float (*)[NORM_ROWS]>(
+      s_x + NORM_PIECES + NORM_ROWS);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
   const int lo = lane & 15, g = lane >> 4;
@@ -61,8 +72,9 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     for (int u = 0; u < U; ++u) {
       // a stage may be half of one: then its last chunk comes twice
       const unsigned at = (unsigned)min(c0 + i * U + u, c1 - 1) * 64;
-      load_to_lds<16>(wp + at, ring + s * STAGE + u * 2 * TILE);
-      load_to_lds<16>(xp + at, ring + s * STAGE + (u * 2 + 1) * TILE);
+      uint4* to = ring + s * STAGE + u * (NORM ? 1 : 2) * TILE;
+      load_to_lds<16>(wp + at, to);
+      if constexpr (!NORM) load_to_lds<16>(xp + at, to + TILE);
     }
   };
   const int at = lo * 4 + (g ^ ((lo >> 2) & 3));
@@ -71,9 +83,12 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     short8 wf[U], xf[U];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint4* t = ring + s * STAGE + u * 2 * TILE + at;
+      const uint4* t = ring + s * STAGE + u * (NORM ? 1 : 2) * TILE + at;
       wf[u] = *reinterpret_cast<const short8*>(t);
-      xf[u] = *reinterpret_cast<const short8*>(t + TILE);
+      xf[u] = *reinterpret_cast<const short8*>(
+          NORM ? s_x + min(lo, m - 1) * (k / 8 + 1) +
+                     min(c0 + i * U + u, c1 - 1) * 4 + g
+               : t + TILE);
     }
     if (more) {
       wait_lds_reads();
@@ -85,9 +100,15 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0,
                                                       0);
   };
+  NormRows<KW * WAVE> rows;
+  if constexpr (NORM) rows.load(norm, m, k);
   #pragma unroll
   for (int s = 0; s < P; ++s)
     if (s < steps) load(s, s);
+  if constexpr (NORM) {
+    rows.put(norm, m, k, s_x, squares);
+    lds_barrier();
+  }
   int i = 0;
   for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
     #pragma unroll
@@ -114,10 +135,12 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   __syncthreads();
   const int r = threadIdx.x / 16, c = threadIdx.x % 16;
   if (r >= m) return;
+  const float scale = NORM ? norm_scale<KW>(squares, r, k, norm.eps) : 1.f;
   auto sum = [&](int c) {
     float v = 0.f;
     #pragma unroll
     for (int q = 0; q < KW; ++q) v += red[(q * 16 + r) * (16 + PAD) + c];
+    if constexpr (NORM) v *= scale;
     if (bias != nullptr) v += bf2f(bias[weight_row<C>(n0, c, n, half)]);
     return v;
   };
@@ -143,10 +166,15 @@ bool rows_gemm_takes(int m, int n, int k, bool gated) {
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
                       long y_ld, bool gated, const Heads* heads,
-                      hipStream_t stream) {
-  auto kernel = heads ? rows_gemm_kernel<Columns::HEADS>
-                : gated ? rows_gemm_kernel<Columns::GATED>
-                        : rows_gemm_kernel<Columns::PLAIN>;
+                      const NormOf* norm, hipStream_t stream) {
+  auto pick = [&](auto normed) {
+    constexpr bool N = decltype(normed)::value;
+    return heads ? rows_gemm_kernel<Columns::HEADS, N>
+           : gated ? rows_gemm_kernel<Columns::GATED, N>
+                   : rows_gemm_kernel<Columns::PLAIN, N>;
+  };
+  auto kernel = norm ? pick(std::true_type{}) : pick(std::false_type{});
   kernel<<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
-      y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{});
+      y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{},
+      norm ? *norm : NormOf{});
 }

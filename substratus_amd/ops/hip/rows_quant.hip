@@ -130,22 +130,28 @@ template <> struct Layout<Quant::Q6_K> {
 
 // MR: rows of x; ME: of every four, those that are there (MR 4 only); KW
 // waves share k, P stages are in flight in each
-template <Quant Q, int MR, int ME, int KW, int P, Columns C>
+template <Quant Q, int MR, int ME, int KW, int P, Columns C, bool NORM>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                        const f16_t* __restrict__ scales,
                        const unsigned char* __restrict__ qs, int m, int n,
-                       int k, Heads heads) {
+                       int k, Heads heads, NormOf norm) {
   using L = Layout<Q>;
   constexpr bool K_QUANT = Q == Quant::Q4_K || Q == Quant::Q6_K;
   constexpr int FM = (MR + 15) / 16;
-  constexpr int XL = MR / 2;                     // loads of x, 4 rows x 256 B
+  // loads of x, 4 rows x 256 B (normed x does not go through the ring)
+  constexpr int XL = NORM ? 0 : MR / 2;
   constexpr int WS = L::W * TILE + L::S * 16;    // weights and scales
   constexpr int STAGE = XL * 64 + WS;
   constexpr int LOADS = XL + L::LOADS;
   constexpr int BM = FM * 16, PAD = 1;
   constexpr int RED = (KW * BM * (16 + PAD) + 3) / 4, RING = KW * P * STAGE;
-  __shared__ alignas(16) uint4v s_all[RING > RED ? RING : RED];
+  constexpr int BEFORE = RING > RED ? RING : RED;
+  __shared__ alignas(16)
+      uint4v s_all[BEFORE + (NORM ? NORM_PIECES + NORM_ROWS + KW : 0)];
+  uint4v* s_x = s_all + BEFORE;
+  auto squares = reinterpret_cast<float (*)[NORM_ROWS]>(
+      s_x + NORM_PIECES + NORM_ROWS);
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
@@ -169,7 +175,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const unsigned char* wp = qs + weight_row<C>(n0, row, n, half) * rb;
   const unsigned char* sp = sc + weight_row<C>(n0, row, n, half) * sb;
   const unsigned char* dp = sc + weight_row<C>(n0, lo, n, half) * sb;
-  const char* xp[XL / 2];
+  const char* xp[XL / 2 + 1];
   #pragma unroll
   for (int d = 0; d < XL / 2; ++d)
     xp[d] = reinterpret_cast<const char*>(
@@ -234,6 +240,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const int xsw = ((lo & 3) << 2) ^
                   (((lo & (MR > 16 ? 15 : MR - 1)) >> 2) & 3);
   const int wsw = (lo >> 2) & 3;
+  const uint4v* x_row = s_x + min(lo & (MR - 1), m - 1) * (k / 8 + 1);
   float4v acc[FM];
   #pragma unroll
   for (int j = 0; j < FM; ++j) acc[j] = zero;
@@ -275,7 +282,9 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
         #pragma unroll
         for (int j = 0; j < FM; ++j) {
           const short8 xv = __builtin_bit_cast(
-              short8, xs[xr[j] + (b >> 2) * 64 + (((b * 4 + g) & 15) ^ xsw)]);
+              short8, NORM ? x_row[c * 32 + b * 4 + g]
+                           : xs[xr[j] + (b >> 2) * 64 +
+                                (((b * 4 + g) & 15) ^ xsw)]);
           const float4v sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               xv, off, zero, 0, 0, 0);
           add_scaled<ME>(acc[j], scale,
@@ -314,7 +323,8 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
           for (int j = 0; j < FM; ++j) {
             const int p = b * 4 + h * 2 + (g >> 1);
             const uint2v xw = reinterpret_cast<const uint2v*>(
-                xs + xr[j] + (p >> 4) * 64 + ((p & 15) ^ xsw))[g & 1];
+                NORM ? x_row + c * 32 + p
+                     : xs + xr[j] + (p >> 4) * 64 + ((p & 15) ^ xsw))[g & 1];
             const uint2v xe = {low2(xw[0], xw[1]), high2(xw[0], xw[1])};
             const short4v xv = __builtin_bit_cast(short4v, xe);
             const float4v sum = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
@@ -328,9 +338,15 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     }
   };
 
+  NormRows<KW * WAVE> rows;
+  if constexpr (NORM) rows.load(norm, m, k);
   #pragma unroll
   for (int s = 0; s < P; ++s)
     if (s < steps) load(s, c0 + s);
+  if constexpr (NORM) {
+    rows.put(norm, m, k, reinterpret_cast<uint4*>(s_x), squares);
+    lds_barrier();
+  }
   int i = 0;
   for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
     #pragma unroll
@@ -374,10 +390,13 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   for (int i = threadIdx.x; i < BM * 16; i += KW * WAVE) {
     const int r = i / 16, c = i % 16;
     if (r >= m || r >= MR) break;
+    const float scale =
+        NORM ? norm_scale<KW>(squares, r, k, norm.eps) : 1.f;
     auto sum = [&](int c) {
       float v = 0.f;
       #pragma unroll
       for (int q = 0; q < KW; ++q) v += red[(q * BM + r) * (16 + PAD) + c];
+      if constexpr (NORM) v *= scale;
       return v;
     };
     if constexpr (C == Columns::GATED) {
@@ -402,19 +421,27 @@ bool rows_quant_takes(int m, int n, int k, Quant q, bool gated) {
 
 void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
                        const unsigned char* qs, int m, int n, int k, Quant q,
-                       bool gated, const Heads* heads, hipStream_t stream) {
+                       bool gated, const Heads* heads, const NormOf* norm,
+                       hipStream_t stream) {
   const f16_t* sc = reinterpret_cast<const f16_t*>(scales);
   auto go = [&](auto qc, auto mr, auto me, auto kw, auto p) {
     constexpr Quant QQ = decltype(qc)::value;
     constexpr int MR = decltype(mr)::value, ME = decltype(me)::value,
                   KW = decltype(kw)::value, P = decltype(p)::value;
     const dim3 grid((n + 15) / 16, (m + MR - 1) / MR), block(KW * WAVE);
-    auto kernel =
-        heads ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::HEADS>
-        : gated ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::GATED>
-                : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN>;
+    auto pick = [&](auto normed) {
+      constexpr bool N = decltype(normed)::value;
+      return heads ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::HEADS, N>
+             : gated ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::GATED, N>
+                     : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN,
+                                         N>;
+    };
+    auto kernel = pick(std::false_type{});
+    if constexpr (MR == NORM_ROWS)
+      if (norm) kernel = pick(std::true_type{});
     kernel<<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k,
-                                       heads ? *heads : Heads{});
+                                       heads ? *heads : Heads{},
+                                       norm ? *norm : NormOf{});
   };
   auto by_rows = [&](auto qc) {
     constexpr Quant QQ = decltype(qc)::value;

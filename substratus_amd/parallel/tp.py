@@ -62,6 +62,15 @@ class Linear(nn.Module):
         return ops.linear_heads(x, self.weight, self.bias, cache)
 
 
+    def normed(self, delta: torch.Tensor, h: torch.Tensor,
+               norm: torch.Tensor, eps: float, gated: bool = False,
+               cache: Optional[ops.Cache] = None):
+        """(the outputs for RMSNorm of h + delta, h + delta), gated or appended
+        as above, in the same kernel, or None."""
+        return ops.linear_normed(delta, h, norm, eps, self.weight, self.bias,
+                                 gated, cache)
+
+
 class ColumnParallelLinear(Linear):
     """Output features sharded across TP ranks; output stays sharded."""
 
