@@ -279,14 +279,16 @@ void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
                          const float* __restrict__ lse,
                          const float* __restrict__ delta,
                          const int* __restrict__ seq_start,
-                         int hq, int hkv, float scale) {
+                         int hq, int hkv, int most, float scale) {
   constexpr int DC32 = D / 32;
   constexpr int DC16 = D / 16;
   const int s = blockIdx.x;
-  const int head = blockIdx.y;
   const int tile = blockIdx.z;
   const int grp = hq / hkv;
-  const int kvh = head / grp;
+  const int per = (grp + most - 1) / most;     // workgroups of a group
+  const int kvh = blockIdx.y / per;
+  const int head0 = kvh * grp + blockIdx.y % per * most;
+  const int head1 = min(head0 + most, (kvh + 1) * grp);
   const int base = seq_start[s];
   const int n = seq_start[s + 1] - base;
   const int kv0_tile = tile * BW_TILE;
@@ -335,7 +337,7 @@ void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
   const int qc_first = kv0_tile / BW_CH;   // BW_TILE == BW_CH: = tile
   const int nqchunks = (n + BW_CH - 1) / BW_CH;
 
-  {
+  for (int head = head0; head < head1; ++head) {
     for (int qc = qc_first; qc < nqchunks; ++qc) {
       const int qbase = qc * BW_CH;
       // ---- stage Q and dO, both layouts --------------------------------
@@ -455,7 +457,7 @@ void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
       const int kpos = kv0 + lhi * 4 + i;
       if (kpos >= n) continue;
       const long roff = (long)(base + kpos) * krow_stride + (long)kvh * D;
-      if (grp == 1) {
+      if (per == 1) {
         #pragma unroll
         for (int c = 0; c < DC16; ++c) {
           dk[roff + c * 16 + llo] = dk_acc[c][i];
@@ -489,6 +491,19 @@ void launch_attn_bwd_delta(float* delta, const bf16_t* dout,
         delta, dout, out, rows);
 }
 
+// Query heads of a group whose shares of dK and dV a workgroup adds up in
+// registers before its atomic additions, which a head at a time are a third of
+// the time at 71 heads on one. More of them leave too few workgroups. us of the
+// backward on a MI355X with 1, 2, 4 heads (2 x 2048: sequences x length):
+//   1 x 1024, 71 on 1 of 64   132  155  246     2 x 2048   740  633  677
+//   8 x 2048, the same       2697 2331 2233    16 x 512    564  470  419
+//   8 x 512, 32 on 8 of 128   291  221  239     2 x 2048   616  553  766
+//   8 x 2048, the same       2401 2232 2126     2 x 512     89  115  180
+int attn_bwd_heads(int num_seqs, int max_len, int hq, int hkv) {
+  const long all = (long)num_seqs * hq * ((max_len + BW_TILE - 1) / BW_TILE);
+  return min(all >= 8192 ? 4 : all >= 2048 ? 2 : 1, hq / hkv);
+}
+
 void launch_attn_bwd(bf16_t* dq, float* dk, float* dv, const bf16_t* q,
                      const bf16_t* k, const bf16_t* v, const bf16_t* dout,
                      const float* lse, const float* delta,
@@ -498,25 +513,25 @@ void launch_attn_bwd(bf16_t* dq, float* dk, float* dv, const bf16_t* q,
   const int tiles = (max_len + BW_TILE - 1) / BW_TILE;
   dim3 block(BW_WAVES * WAVE);
   dim3 grid_q(num_seqs, hq, tiles);
-  dim3 grid_kv(num_seqs, hq, tiles);
+  const int most = attn_bwd_heads(num_seqs, max_len, hq, hkv);
+  const int grp = hq / hkv;
+  dim3 grid_kv(num_seqs, hkv * ((grp + most - 1) / most), tiles);
   if (d == 128) {
     attnbwd::attn_bwd_dq_kernel<128><<<grid_q, block, 0, stream>>>(
         dq, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
     attnbwd::attn_bwd_dkv_kernel<128><<<grid_kv, block, 0, stream>>>(
-        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
+        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, most, scale);
   } else if (d == 64) {
     attnbwd::attn_bwd_dq_kernel<64><<<grid_q, block, 0, stream>>>(
         dq, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
     attnbwd::attn_bwd_dkv_kernel<64><<<grid_kv, block, 0, stream>>>(
-        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
+        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, most, scale);
   }
 }
 
 bool attn_bwd_supported(int d) { return d == 128 || d == 64; }
 
-// dkv alone (the mixed-dispatch backward pairs the V5 dq kernel with THIS
-// dkv: the V5-structure dkv measured 2.3x SLOWER — 2104 vs 918 us/call on
-// falcon MQA — despite winning on dq/fwd; see attention_v5.hip STATUS)
+// dkv alone: the V5 dq kernel is paired with this one where it is the faster
 void launch_attn_bwd_dkv_only(float* dk, float* dv, const bf16_t* q,
                               const bf16_t* k, const bf16_t* v,
                               const bf16_t* dout, const float* lse,
@@ -525,11 +540,13 @@ void launch_attn_bwd_dkv_only(float* dk, float* dv, const bf16_t* q,
                               int d, float scale, hipStream_t stream) {
   const int tiles = (max_len + BW_TILE - 1) / BW_TILE;
   dim3 block(BW_WAVES * WAVE);
-  dim3 grid_kv(num_seqs, hq, tiles);
+  const int most = attn_bwd_heads(num_seqs, max_len, hq, hkv);
+  const int grp = hq / hkv;
+  dim3 grid_kv(num_seqs, hkv * ((grp + most - 1) / most), tiles);
   if (d == 128)
     attnbwd::attn_bwd_dkv_kernel<128><<<grid_kv, block, 0, stream>>>(
-        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
+        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, most, scale);
   else
     attnbwd::attn_bwd_dkv_kernel<64><<<grid_kv, block, 0, stream>>>(
-        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
+        dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, most, scale);
 }

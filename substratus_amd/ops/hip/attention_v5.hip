@@ -328,14 +328,11 @@ bool attn_v5_supported(int d) { return d == 128 || d == 64; }
 
 namespace attnv5 {
 
-// STATUS of the V5 backward pair: dq_v5 WINS (393 vs 504 us/call on the
-// falcon MQA train shape) and is the default; dkv_v5 below is correct but
-// measured 2.3x SLOWER than the 16-row dkv (2104 vs 918 us/call) despite
-// the same structure winning on fwd/dq — its four chains (S, dP, dV, dK)
-// push the packing/tr16 VALU volume past what the removed P round-trip
-// buys, and occupancy drops to 3 waves/SIMD. Kept behind
-// SUB_ATTN_DKV_V5=1 as a measured negative result; the shipped backward
-// is delta + dq_v5 + 16-row dkv (bindings attn_train_bwd_v5).
+// Of the backward, dq takes this structure throughout (393 us against 504 per
+// call, 71 heads on one). dkv takes it for long sequences only: its four chains
+// (S, dP, dV, dK) push the packing/tr16 VALU volume past what the removed P
+// round-trip buys, and occupancy drops to 3 waves/SIMD (the rule and both sides
+// measured: attn_train_bwd_v5 in bindings.hip).
 
 // ---------------------------------------------------------------- dq V5
 // Per wave ONE 32-row q block (like the forward): Q and dO register-
@@ -535,7 +532,7 @@ namespace attnv5 {
 // lse/delta come per C-ROW from an LDS-staged slice), P and dS packed
 // in-register to B-fragments, dV^T = dO^T·P and dK^T = Q^T·dS accumulated
 // transposed (per-lane key-scalar epilogue; GQA heads atomically add into
-// the fp32 dk/dv buffers, grid is per Q head like the 16-row dkv).
+// the fp32 dk/dv buffers, some of them per workgroup like the 16-row dkv).
 template <int D, bool NOATOMIC = false>  // NOATOMIC: timing-only probe
 __global__ __launch_bounds__(V5_WAVES * WAVE)
 void attn_bwd_dkv_v5_kernel(float* __restrict__ dk,       // [T, HKV, D] f32
@@ -547,14 +544,16 @@ void attn_bwd_dkv_v5_kernel(float* __restrict__ dk,       // [T, HKV, D] f32
                             const float* __restrict__ lse,
                             const float* __restrict__ delta,
                             const int* __restrict__ seq_start,
-                            int hq, int hkv, float scale) {
+                            int hq, int hkv, int most, float scale) {
   constexpr int KK = D / 16;
   constexpr int DC = D / 32;
   const int s = blockIdx.x;
-  const int head = blockIdx.y;
   const int tile = blockIdx.z;
   const int grp = hq / hkv;
-  const int kvh = head / grp;
+  const int per = (grp + most - 1) / most;     // workgroups of a group
+  const int kvh = blockIdx.y / per;
+  const int head0 = kvh * grp + blockIdx.y % per * most;
+  const int head1 = min(head0 + most, (kvh + 1) * grp);
   const int base = seq_start[s];
   const int n = seq_start[s + 1] - base;
   const int kv0_tile = tile * V5_QTILE;
@@ -602,6 +601,7 @@ void attn_bwd_dkv_v5_kernel(float* __restrict__ dk,       // [T, HKV, D] f32
   if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256)
     __builtin_amdgcn_s_setprio(1);
 
+  for (int head = head0; head < head1; ++head)
   for (int qc = qc_first; qc < nqchunks; ++qc) {
     const int qbase = qc * V5_KCHUNK;
     {
@@ -727,7 +727,7 @@ void attn_bwd_dkv_v5_kernel(float* __restrict__ dk,       // [T, HKV, D] f32
       #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int d = c * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-        if (NOATOMIC || grp == 1) {
+        if (NOATOMIC || per == 1) {
           dk[roff + d] = dk_t[c][r];
           dv[roff + d] = dv_t[c][r];
         } else {
@@ -741,6 +741,8 @@ void attn_bwd_dkv_v5_kernel(float* __restrict__ dk,       // [T, HKV, D] f32
 
 }  // namespace attnv5
 
+int attn_bwd_heads(int, int, int, int);
+
 void launch_attn_bwd_dkv_v5(float* dk, float* dv, const bf16_t* q,
                             const bf16_t* k, const bf16_t* v,
                             const bf16_t* dout, const float* lse,
@@ -748,7 +750,8 @@ void launch_attn_bwd_dkv_v5(float* dk, float* dv, const bf16_t* q,
                             int num_seqs, int max_len, int hq, int hkv,
                             int d, float scale, hipStream_t stream) {
   const int tiles = (max_len + V5_QTILE - 1) / V5_QTILE;
-  dim3 grid(num_seqs, hq, tiles);
+  const int most = attn_bwd_heads(num_seqs, max_len, hq, hkv);
+  dim3 grid(num_seqs, hkv * ((hq / hkv + most - 1) / most), tiles);
   dim3 block(V5_WAVES * WAVE);
   const char* na = getenv("SUB_DKV_NOATOMIC");   // timing-only probe
   const bool noat = na && na[0] == '1';
@@ -756,17 +759,17 @@ void launch_attn_bwd_dkv_v5(float* dk, float* dv, const bf16_t* q,
     if (noat)
       attnv5::attn_bwd_dkv_v5_kernel<128, true><<<grid, block, 0,
           stream>>>(dk, dv, q, k, v, dout, lse, delta, seq_start, hq,
-                    hkv, scale);
+                    hkv, most, scale);
     else
       attnv5::attn_bwd_dkv_v5_kernel<128><<<grid, block, 0, stream>>>(
-          dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
+          dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, most, scale);
   } else {
     if (noat)
       attnv5::attn_bwd_dkv_v5_kernel<64, true><<<grid, block, 0,
           stream>>>(dk, dv, q, k, v, dout, lse, delta, seq_start, hq,
-                    hkv, scale);
+                    hkv, most, scale);
     else
       attnv5::attn_bwd_dkv_v5_kernel<64><<<grid, block, 0, stream>>>(
-          dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, scale);
+          dk, dv, q, k, v, dout, lse, delta, seq_start, hq, hkv, most, scale);
   }
 }

@@ -32,6 +32,7 @@ void launch_attn_bwd_dkv_only(float*, float*, const bf16_t*, const bf16_t*, cons
 void launch_attn_bwd_delta(float*, const bf16_t*, const bf16_t*, long, int, hipStream_t);
 void launch_attn_bwd(bf16_t*, float*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int*, int, int, int, int, int, float, hipStream_t);
 bool attn_bwd_supported(int);
+int attn_bwd_heads(int, int, int, int);
 void launch_attn_prefill_probe(int, bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, int, int, int, int, float, hipStream_t);
 void launch_mfma_probe(float*, const bf16_t*, const bf16_t*, hipStream_t);
 void launch_mfma32_probe(float*, const bf16_t*, const bf16_t*, hipStream_t);
@@ -446,12 +447,16 @@ void attn_train_bwd_v5(torch::Tensor dq, torch::Tensor dk,
                         lse.data_ptr<float>(), delta.data_ptr<float>(),
                         seq_start.data_ptr<int>(), num_seqs, (int)max_len,
                         hq, hkv, d, (float)scale, stream());
-  // dkv dispatch by GQA group size: the V5-structure dkv WINS at grp==1
-  // (llama MHA: 1010 vs 1113 us) but loses 2x under MQA/GQA — its fewer,
-  // wider blocks collide harder on the per-kv-row atomic adds (falcon
-  // 71:1: 2477 vs 918 us). SUB_ATTN_DKV_V5=0/1 overrides.
+  // dkv: the V5 structure's 256-row tiles and 32-row blocks pay for long
+  // sequences only. us of the backward on a MI355X, 16 rows a wave and V5:
+  // 32 heads of 128, 16 x 512 533, 742; 4 x 2048 1176, 1179; 1 x 4096 1037,
+  // 1001; 2 x 8192 8245, 6583. On 8 heads, 1 x 4096 1000, 1272; 2 x 8192 7719,
+  // 6343. SUB_ATTN_DKV_V5=0/1 overrides.
   const char* e = getenv("SUB_ATTN_DKV_V5");
-  const bool use_v5 = e ? (e[0] == '1') : (hq == hkv);
+  const bool use_v5 = e ? (e[0] == '1')
+      : hq == hkv ? max_len >= 4096
+                  : max_len >= 8192 &&
+                        attn_bwd_heads(num_seqs, max_len, hq, hkv) >= 4;
   if (use_v5)
     launch_attn_bwd_dkv_v5(dk.data_ptr<float>(), dv.data_ptr<float>(),
                            bfc(q), bfc(k), bfc(v), bfc(dout),

@@ -1,0 +1,35 @@
+"""The backward of grouped heads at the numbers of heads that a workgroup adds
+up (one, two, four; groups that they do not divide) against 64 bits."""
+
+import pytest
+import torch
+
+from substratus_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("b,s,hq,hkv,d", [
+    (1, 70, 3, 1, 64), (16, 128, 71, 1, 64), (32, 70, 192, 64, 64),
+    (64, 65, 66, 22, 64), (16, 100, 64, 16, 128), (16, 200, 71, 1, 64)])
+def test_heads(b, s, hq, hkv, d):
+    torch.manual_seed(b * s)
+    q, k, v = (torch.randn(b, s, h, d, device=DEV).bfloat16()
+               .requires_grad_() for h in (hq, hkv, hkv))
+    dout = torch.randn(b, s, hq, d, device=DEV).bfloat16()
+    out = ops.flash_attn_train(q, k, v, d ** -0.5)
+    got = torch.autograd.grad(out, (q, k, v), dout)
+    at = [t.detach()[-1:].float().requires_grad_() for t in (q, k, v)]
+    kk, vv = (t.repeat_interleave(hq // hkv, 2).transpose(1, 2)
+              for t in at[1:])
+    sc = (at[0].transpose(1, 2).double() @ kk.double().mT) * d ** -0.5
+    mask = torch.ones(s, s, device=DEV, dtype=torch.bool).tril()
+    p = torch.softmax(sc.masked_fill(~mask, -torch.inf), -1)
+    want = torch.autograd.grad((p @ vv.double()).transpose(1, 2), at,
+                               dout[-1:].double())
+    # weights and their gradients enter the products as bf16: 2^-9 each, and
+    # results are rounded once
+    for g, w in zip(got, want):
+        off = (g[-1:].double() - w.double()).norm() / w.double().norm()
+        assert float(off) < 2.0 ** -7, float(off)
