@@ -282,9 +282,11 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
 
 def _tile_gemm(a: torch.Tensor, b: torch.Tensor,
                bias: Optional[torch.Tensor] = None, a_flipped: bool = False,
-               b_flipped: bool = False) -> Optional[torch.Tensor]:
+               b_flipped: bool = False,
+               gated: bool = False) -> Optional[torch.Tensor]:
     """a b^T + bias on tile_gemm.hip, a stored as [k, m] and b as [k, n] where
-    flipped, or None where it does not take them or does not pay."""
+    flipped, gated as linear_gated's, or None where it does not take them or
+    does not pay."""
     ext = _load_ext()
     m, k = a.shape[::-1] if a_flipped else a.shape
     n = b.shape[1 if b_flipped else 0]
@@ -292,14 +294,14 @@ def _tile_gemm(a: torch.Tensor, b: torch.Tensor,
             t.is_cuda and t.device == a.device and t.dtype == torch.bfloat16
             and t.stride(1) == 1 and t.data_ptr() % 16 == 0 for t in (a, b))
             or not ext.tile_gemm_good(m, n, k, a.stride(0), b.stride(0),
-                                      a_flipped, b_flipped)):
+                                      a_flipped, b_flipped, gated)):
         return None
     if bias is not None and not (
             bias.device == a.device and bias.dtype == torch.bfloat16
             and bias.is_contiguous() and bias.shape == (n,)
             and bias.data_ptr() % 16 == 0):
         return None
-    return ext.tile_gemm(a, b, bias, a_flipped, b_flipped)
+    return ext.tile_gemm(a, b, bias, a_flipped, b_flipped, gated)
 
 
 class _Linear(torch.autograd.Function):
@@ -331,8 +333,10 @@ class _Linear(torch.autograd.Function):
 
 
 def _many_rows(x: torch.Tensor, weight: torch.Tensor,
-               bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    """F.linear of 256 rows and more, or None where torch's is as good."""
+               bias: Optional[torch.Tensor],
+               gated: bool = False) -> Optional[torch.Tensor]:
+    """F.linear of 256 rows and more, or None where torch's is as good; or what
+    linear_gated makes of it, without gradients."""
     given = [t for t in (x, weight, bias) if t is not None]
     if not (x.is_cuda and weight.dim() == 2 and weight.shape[0] >= 256
             and x.dim() >= 2 and x.shape[-1] == weight.shape[1] > 0
@@ -343,17 +347,19 @@ def _many_rows(x: torch.Tensor, weight: torch.Tensor,
         return None
     rows = x.reshape(-1, x.shape[-1])
     if torch.is_grad_enabled() and any(t.requires_grad for t in given):
+        if gated:
+            return None
         m, k, n = *rows.shape, weight.shape[0]
         good = _load_ext().tile_gemm_good
-        if not (good(m, n, k, k, k, False, False)
-                or good(m, k, n, n, k, False, True)
-                or good(n, k, m, n, k, True, True)):
+        if not (good(m, n, k, k, k, False, False, False)
+                or good(m, k, n, n, k, False, True, False)
+                or good(n, k, m, n, k, True, True, False)):
             return None
         y = _Linear.apply(rows, weight, bias)
     else:
-        y = _tile_gemm(rows, weight, bias)
+        y = _tile_gemm(rows, weight, bias, gated=gated)
     return y if y is None or x.dim() == 2 else \
-        y.view(*x.shape[:-1], weight.shape[0])
+        y.view(*x.shape[:-1], y.shape[1])
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor,
@@ -412,7 +418,7 @@ def linear_gated(x: torch.Tensor, weight: torch.Tensor,
     None where it is not made for that."""
     few = _few_rows(x, weight, bias, True)
     if few is None:
-        return None
+        return _many_rows(x, weight, bias, True)
     rows, ext = few
     n = weight.shape[0] // 2
     y = rows.new_empty(rows.shape[0], n)

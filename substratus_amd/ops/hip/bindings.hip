@@ -594,10 +594,10 @@ void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
 }
 
 // a b^T + bias for operands of many rows as they are stored: a [m, k], or [k, m]
-// if flipped; b [n, k], or [k, n].
+// if flipped; b [n, k], or [k, n]. gated: silu(first half) * second half.
 torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
                         c10::optional<torch::Tensor> bias, bool a_flipped,
-                        bool b_flipped) {
+                        bool b_flipped, bool gated) {
   for (const auto& t : {a, b})
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
                     t.dim() == 2 && t.stride(1) == 1 && aligned16(t),
@@ -606,17 +606,17 @@ torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
   const long n = b.size(b_flipped);
   TORCH_CHECK(b.size(!b_flipped) == k, "inner dimensions differ");
   TORCH_CHECK(tile_gemm_takes(m, n, k, a.stride(0), b.stride(0), a_flipped,
-                              b_flipped),
+                              b_flipped, gated),
               "tile_gemm: unsupported shape ", m, "x", n, "x", k);
   if (bias) check_rows(*bias, n, "bias");
   const TilePlan plan = tile_gemm_plan(m, n, k);
-  auto out = torch::empty({m, n}, a.options());
+  auto out = torch::empty({m, gated ? n / 2 : n}, a.options());
   torch::Tensor shares;
   if (plan.shares())
     shares = torch::empty({plan.shares()}, a.options().dtype(torch::kFloat));
   launch_tile_gemm({bf(out), bfc(a), bfc(b), bias ? bfc(*bias) : nullptr,
                     (int)m, (int)n, (int)k, a.stride(0), b.stride(0),
-                    a_flipped, b_flipped},
+                    a_flipped, b_flipped, gated},
                    plan, plan.shares() ? shares.data_ptr<float>() : nullptr,
                    stream());
   post_launch_check("tile_gemm");
@@ -624,9 +624,9 @@ torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
 }
 
 bool tile_gemm_good(long m, long n, long k, long a_ld, long b_ld,
-                    bool a_flipped, bool b_flipped) {
-  return tile_gemm_takes(m, n, k, a_ld, b_ld, a_flipped, b_flipped) &&
-         tile_gemm_pays(m, n, k, a_flipped, b_flipped);
+                    bool a_flipped, bool b_flipped, bool gated) {
+  return tile_gemm_takes(m, n, k, a_ld, b_ld, a_flipped, b_flipped, gated) &&
+         tile_gemm_pays(m, n, k, a_flipped, b_flipped, gated);
 }
 
 // A projection of heads with rope_kv_append of what comes out: rotated queries
@@ -972,7 +972,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wstream_gemm", &wstream_gemm);
   m.def("wstream_ok", &wstream_ok);
   m.def("rows_gemm", &rows_gemm);
-  m.def("tile_gemm", &tile_gemm);
+  m.def("tile_gemm", &tile_gemm, py::arg("a"), py::arg("b"), py::arg("bias"),
+        py::arg("a_flipped"), py::arg("b_flipped"), py::arg("gated") = false);
   m.def("tile_gemm_good", &tile_gemm_good);
   m.def("rows_heads", &rows_heads);
   m.def("rows_normed", &rows_normed);

@@ -22,11 +22,14 @@ struct TileGemm {
   int m, n, k;
   long a_ld, b_ld;
   bool a_flipped, b_flipped;
+  // the first n / 2 columns gate the others: out [m, n / 2] = silu(gate) * up
+  bool gated;
 };
 
 bool tile_gemm_takes(long m, long n, long k, long a_ld, long b_ld,
-                     bool a_flipped, bool b_flipped);
+                     bool a_flipped, bool b_flipped, bool gated);
 TilePlan tile_gemm_plan(long m, long n, long k);
-bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped);
+bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped,
+                    bool gated);
 void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,
                       hipStream_t stream);

@@ -1,6 +1,7 @@
 // out = a b^T + bias of bf16 matrices of many rows, with either operand as it
 // is or flipped: the products of prompts, and of a training step's forward and
-// backward, which need no transposed copy.
+// backward, which need no transposed copy. Or, of a matrix b whose first half
+// gates its second, silu(gate) * up: a tile has 128 columns of either then.
 //
 // Bound by the matrix cores if they are kept busy. A workgroup of eight waves
 // takes 256 x 256 outputs, a wave 128 x 64 of them, 64 of the inner dimension
@@ -136,12 +137,14 @@ DEV_INLINE void read_flipped4(short8 (&f)[4][2], unsigned p0, unsigned p1,
 
 // Where a tile begins: LINES rows of tiles by columns. The last tiles reach
 // back instead of over the matrix' end; what two of them have is the same.
+template <bool GATED>
 DEV_INLINE void tile_of(const TileGemm& g, const TilePlan& p, int tile,
                         int& m0, int& n0) {
   const int per = LINES * p.tiles_n, first = tile / per * LINES;
   const int lines = min(p.tiles_m - first, LINES);
   m0 = min((first + tile % per % lines) * TILE, g.m - TILE);
-  n0 = min(tile % per / lines * TILE, g.n - TILE);
+  const int wide = GATED ? TILE / 2 : TILE;
+  n0 = min(tile % per / lines * wide, (GATED ? g.n / 2 : g.n) - wide);
 }
 
 // Steps come in pairs, one for each half of LDS; past the end they are zeros.
@@ -155,6 +158,7 @@ struct Item {
   int share;                      // -1: the whole tile
 };
 
+template <bool GATED>
 DEV_INLINE Item item_of(const TileGemm& g, const TilePlan& p, int id) {
   const int pairs = pairs_of(g.k);
   Item it;
@@ -174,14 +178,14 @@ DEV_INLINE Item item_of(const TileGemm& g, const TilePlan& p, int id) {
     it.t1 = 2 * (int)((long)pairs * (part + 1) / p.split);
     if (p.split == 1) it.share = -1;
   }
-  tile_of(g, p, tile, it.m0, it.n0);
+  tile_of<GATED>(g, p, tile, it.m0, it.n0);
   return it;
 }
 
 // Eight outputs of one row.
-DEV_INLINE void store(const TileGemm& g, int row, int col, float4v v,
-                      float4v w) {
-  *reinterpret_cast<uint4*>(g.out + (long)row * g.n + col) =
+DEV_INLINE void store(const TileGemm& g, int width, int row, int col,
+                      float4v v, float4v w) {
+  *reinterpret_cast<uint4*>(g.out + (long)row * width + col) =
       make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
                  pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3]));
 }
@@ -206,7 +210,23 @@ DEV_INLINE int out_col(int tid, int j) {
   return (tid >> 6 & 3) * 64 + j * 32 + (tid >> 4 & 3) * 8;
 }
 
-template <bool FA, bool FB>
+// The first of a thread's four columns of accumulator j.
+template <bool GATED>
+DEV_INLINE int col_of(const TileGemm& g, int n0, int tid, int j) {
+  if constexpr (GATED)
+    return n0 + (tid >> 6 & 3) * 32 + (tid >> 4 & 3) * 8 + (j & 1) * 4 +
+           (j >> 1) * (g.n / 2);
+  return n0 + out_col(tid, j >> 1) + (j & 1) * 4;
+}
+
+DEV_INLINE float4v gate(float4v a, float4v u) {
+  float4v v;
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = silu_times(a[e], u[e]);
+  return v;
+}
+
+template <bool FA, bool FB, bool GATED>
 __global__ __launch_bounds__(THREADS, 2)
 void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   // [two steps][a low, a high, b low, b high]
@@ -214,7 +234,8 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE, lo = lane & 15, gr = lane >> 4;
   const int wm = wave >> 2, wn = wave & 3;
-  const Item it = item_of(g, plan, blockIdx.x);
+  static_assert(!GATED || !FB);
+  const Item it = item_of<GATED>(g, plan, blockIdx.x);
 
   // Loads: a wave has two KB of a region. Of rows: 8 lines of 128 bytes a KB,
   // of a flipped operand 4 of 256. off: from the low region's first byte on.
@@ -232,13 +253,13 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
               (piece_r ^ a_key(r)) * 16;
     off[1][p] = FB
         ? (unsigned)(line * g.b_ld + (qb >> 2) * 64 + (qb & 3) * 8) * 2u
-        : (unsigned)(((r >> 5) * 64 + (r & 31)) * g.b_ld) * 2u +
+        : (unsigned)((GATED ? r : (r >> 5) * 64 + (r & 31)) * g.b_ld) * 2u +
               (piece_r ^ b_key(r)) * 16;
   }
   const long a_step = (FA ? g.a_ld : 1) * STEP * 2;
   const long b_step = (FB ? g.b_ld : 1) * STEP * 2;
   const int a_high = (FA ? 1 : g.a_ld) * 64 * 2;
-  const int b_high = (FB ? 1 : g.b_ld) * 32 * 2;
+  const int b_high = (FB ? 1 : g.b_ld) * (GATED ? g.n / 2 : 32) * 2;
   // What is loaded, two steps ahead of what is multiplied: by buffer loads,
   // whose only vector operand is the offset.
   int lt = it.t0;
@@ -402,41 +423,58 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
       for (int j = 0; j < 4; ++j) to[(i * 4 + j) * THREADS] = acc[i][j];
     return;
   }
+  const int n = GATED ? g.n / 2 : g.n;
   float4v add[4];
   #pragma unroll
   for (int j = 0; j < 4; ++j)
-    add[j] = bias_of(g, it.n0 + out_col(tid, j >> 1) + (j & 1) * 4);
+    add[j] = bias_of(g, col_of<GATED>(g, it.n0, tid, j));
   #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < 8; ++i) {
+    const int row = it.m0 + out_row(tid, i);
     #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      store(g, it.m0 + out_row(tid, i), it.n0 + out_col(tid, j),
-            acc[i][2 * j] + add[2 * j], acc[i][2 * j + 1] + add[2 * j + 1]);
+    for (int j = 0; j < 4; ++j) acc[i][j] += add[j];
+    if constexpr (GATED) {
+      store(g, n, row, col_of<true>(g, it.n0, tid, 0),
+            gate(acc[i][0], acc[i][2]), gate(acc[i][1], acc[i][3]));
+    } else {
+      #pragma unroll
+      for (int j = 0; j < 2; ++j)
+        store(g, n, row, it.n0 + out_col(tid, j), acc[i][2 * j],
+              acc[i][2 * j + 1]);
+    }
+  }
 }
 
-// The shares of the tiles left over are added up, a sixteenth of a tile per
+// The shares of the tiles left over are added up, an eighth of a tile per
 // workgroup.
+template <bool GATED>
 __global__ __launch_bounds__(THREADS)
 void tile_sum_kernel(TileGemm g, TilePlan plan,
                      const float4v* __restrict__ shares) {
   int m0, n0;
-  tile_of(g, plan, plan.whole + blockIdx.x, m0, n0);
-  const int tid = threadIdx.x;
+  tile_of<GATED>(g, plan, plan.whole + blockIdx.x, m0, n0);
+  const int tid = threadIdx.x, i = blockIdx.y;
   const float4v* from = shares +
-      (long)blockIdx.x * plan.split * (32 * THREADS) + tid;
-  float4v v[2];
-  const int i = blockIdx.y >> 1, j = blockIdx.y & 1;
-  const int col = n0 + out_col(tid, j);
+      (long)blockIdx.x * plan.split * (32 * THREADS) + i * 4 * THREADS + tid;
+  float4v v[4];
   #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int at = (i * 4 + j * 2 + e) * THREADS;
-    v[e] = from[at];
-    #pragma unroll 4
-    for (int p = 1; p < plan.split; ++p)
-      v[e] += from[(long)p * 32 * THREADS + at];
-    v[e] += bias_of(g, col + e * 4);
+  for (int j = 0; j < 4; ++j) v[j] = from[j * THREADS];
+  #pragma unroll 4
+  for (int p = 1; p < plan.split; ++p)
+    #pragma unroll
+    for (int j = 0; j < 4; ++j)
+      v[j] += from[(long)p * 32 * THREADS + j * THREADS];
+  #pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] += bias_of(g, col_of<GATED>(g, n0, tid, j));
+  const int row = m0 + out_row(tid, i);
+  if constexpr (GATED) {
+    store(g, g.n / 2, row, col_of<true>(g, n0, tid, 0), gate(v[0], v[2]),
+          gate(v[1], v[3]));
+  } else {
+    #pragma unroll
+    for (int j = 0; j < 2; ++j)
+      store(g, g.n, row, n0 + out_col(tid, j), v[2 * j], v[2 * j + 1]);
   }
-  store(g, m0 + out_row(tid, i), col, v[0], v[1]);
 }
 
 }  // namespace
@@ -444,7 +482,10 @@ void tile_sum_kernel(TileGemm g, TilePlan plan,
 // A tile's offsets within an operand fit 32 bits, 16-byte pieces of it lie
 // within a row.
 bool tile_gemm_takes(long m, long n, long k, long a_ld, long b_ld,
-                     bool a_flipped, bool b_flipped) {
+                     bool a_flipped, bool b_flipped, bool gated) {
+  if (gated && (a_flipped || b_flipped || n % 16 != 0 ||
+                (n / 2 + TILE) * b_ld * 2 >= (1L << 31)))
+    return false;
   auto fits = [&](long rows, long ld, bool flipped) {
     return ld % 8 == 0 && (flipped ? rows % 8 == 0 && ld >= rows
                                    : k % 8 == 0 && ld >= k) &&
@@ -490,26 +531,31 @@ TilePlan tile_gemm_plan(long m, long n, long k) {
 //                     0.95 to 0.99
 //   b flipped         0.39 to 0.57: 0.87 to 0.96; from 0.7: 1.02 to 2.05
 //   both flipped      0.39: 0.90; from 0.7: 1.00 to 1.41
-bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped) {
+//   gated             from 0.9 on, even ones too: the pass that gates them
+//                     is a tenth of the product
+bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped,
+                    bool gated) {
   const TilePlan p = tile_gemm_plan(m, n, k);
   const double rate = 2e-9 * m * n * k / p.us;        // PFLOP/s
   if (a_flipped || b_flipped) return rate >= 0.7;
   const bool even = m % TILE == 0 && n % TILE == 0 &&
                     (long)p.tiles_m * p.tiles_n % 256 == 0;
-  return rate >= 0.9 && !even;
+  return rate >= 0.9 && (gated || !even);
 }
 
 void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,
                       hipStream_t stream) {
   float4v* sh = reinterpret_cast<float4v*>(shares);
   const dim3 grid(plan.whole + plan.rest() * plan.split);
-  auto kernel = g.a_flipped
-      ? (g.b_flipped ? tile_gemm_kernel<true, true>
-                     : tile_gemm_kernel<true, false>)
-      : (g.b_flipped ? tile_gemm_kernel<false, true>
-                     : tile_gemm_kernel<false, false>);
+  auto kernel = g.gated ? tile_gemm_kernel<false, false, true>
+      : g.a_flipped
+          ? (g.b_flipped ? tile_gemm_kernel<true, true, false>
+                         : tile_gemm_kernel<true, false, false>)
+          : (g.b_flipped ? tile_gemm_kernel<false, true, false>
+                         : tile_gemm_kernel<false, false, false>);
   kernel<<<grid, dim3(THREADS), 0, stream>>>(g, plan, sh);
-  if (plan.split > 1)
-    tile_sum_kernel<<<dim3(plan.rest(), 16), dim3(THREADS), 0, stream>>>(
-        g, plan, sh);
+  if (plan.split > 1) {
+    auto sum = g.gated ? tile_sum_kernel<true> : tile_sum_kernel<false>;
+    sum<<<dim3(plan.rest(), 8), dim3(THREADS), 0, stream>>>(g, plan, sh);
+  }
 }

@@ -56,6 +56,24 @@ def test_rounds(m, n, k, fa, fb):
     assert torch.equal(got, _C.tile_gemm(a, b, None, fa, fb))
 
 
+@pytest.mark.parametrize("m,f,k", [(256, 128, 72), (300, 136, 192),
+                                   (1000, 512, 4544), (4360, 2056, 1032)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gated(m, f, k, bias):
+    torch.manual_seed(m)
+    a = operand(m, k, False, 8)
+    b = (operand(2 * f, k, False, 0) / k ** 0.5).bfloat16()
+    bs = torch.randn(2 * f, device=DEV).bfloat16() if bias else None
+    got = _C.tile_gemm(a, b, bs, False, False, True)
+    y = a.double() @ b.double().T + (0 if bs is None else bs.double())
+    g, u = y.chunk(2, 1)
+    want = torch.nn.functional.silu(g) * u
+    # half a step of the result; 32-bit sums before, slopes of at most 1.1
+    room = 2.0 ** -17 * (g.abs() + 1) * (u.abs() + 1)
+    assert bool(((got.double() - want).abs() <=
+                 2.0 ** -8 * want.abs() + room).all())
+
+
 def test_rows_of_any_number():
     """Rows that are not flipped need not come in eights."""
     a, b = operand(321, 192, False, 0), operand(264, 192, False, 0)
