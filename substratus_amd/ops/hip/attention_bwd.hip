@@ -262,12 +262,28 @@ void attn_bwd_dq_kernel(bf16_t* __restrict__ dq,        // [T, HQ, D]
 }
 
 // ------------------------------------------------------------------ dkv
-// Grid (num_seqs, HQ, kv-tiles) — one block per Q HEAD so MQA/GQA keep the
-// full grid parallelism of the dq kernel (a per-kv-head grid with an
-// in-kernel group loop was 13x slower on falcon's 71:1 MQA: 71x fewer
-// blocks AND Q/dO re-staged serially per head). dK/dV accumulate across
-// the group's heads with fp32 unsafeAtomicAdd (hardware
-// global_atomic_add_f32); grp==1 skips the atomic.
+// Grid (num_seqs, HQ / some, kv-tiles) — some heads of a group per block
+// (attn_bwd_heads), the same K and V rows throughout; all of a group's heads
+// in one were 13x slower on falcon's 71:1 MQA. dK/dV accumulate across blocks
+// with fp32 unsafeAtomicAdd (hardware global_atomic_add_f32); one block alone
+// stores.
+//
+// Scores on the diagonal only are compared by position, and dS is scaled at
+// the end: us of the backward, 1 x 4096, 32 heads on 8 of 128: 1000 -> 858.
+
+// Where a chunk's log-sums and deltas are staged: LDS, 5 % faster than loads by
+// each lane, unless it is full. Of head size 128 a byte more would leave a CU
+// one workgroup (20 % slower).
+template <int D>
+DEV_INLINE float* stats_of() {
+  if constexpr (D == 64) {
+    __shared__ float stats[2 * BW_CH];
+    return stats;
+  } else {
+    return nullptr;
+  }
+}
+
 template <int D>
 __global__ __launch_bounds__(BW_WAVES * WAVE)
 void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
@@ -333,6 +349,7 @@ void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
   __shared__ short dst_img[BW_WAVES][BW_CH / 32][2][16][16];
 
   constexpr int NSC = BW_CH / 16;
+  float* stats = stats_of<D>();
   const float scale2 = scale * LOG2E;
   const int qc_first = kv0_tile / BW_CH;   // BW_TILE == BW_CH: = tile
   const int nqchunks = (n + BW_CH - 1) / BW_CH;
@@ -364,6 +381,22 @@ void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
           *reinterpret_cast<uint4*>(&do_img[c][ks][sel][r][off]) = d4;
         }
       }
+      // log-sums and deltas of the queries that this lane has columns of
+      float lse_q[NSC], dlt_q[NSC];
+      if (stats != nullptr) {
+        if (threadIdx.x < BW_CH) {
+          const long row = base + min(qbase + (int)threadIdx.x, n - 1);
+          stats[threadIdx.x] = lse[row * hq + head];
+          stats[BW_CH + threadIdx.x] = delta[row * hq + head];
+        }
+      } else {
+        #pragma unroll
+        for (int sc = 0; sc < NSC; ++sc) {
+          const long row = base + min(qbase + sc * 16 + llo, n - 1);
+          lse_q[sc] = lse[row * hq + head];
+          dlt_q[sc] = delta[row * hq + head];
+        }
+      }
       __syncthreads();
 
       if (wave_live) {
@@ -382,20 +415,25 @@ void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
             dptf = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 va[c], *reinterpret_cast<const short8*>(&db4), dptf, 0, 0, 0);
           }
-          // P^T and dS^T, causal-masked, C layout [kv row i][q col llo]
+          if (stats != nullptr) {
+            lse_q[sc] = stats[sc * 16 + llo];
+            dlt_q[sc] = stats[BW_CH + sc * 16 + llo];
+          }
+          // P^T and dS^T (the scale comes at the end), C layout
+          // [kv row i][q col llo]; positions are compared at the edges only
           const int qpos = qbase + sc * 16 + llo;
-          const int qcl = min(qpos, n - 1);
-          const float lse_q = lse[(long)(base + qcl) * hq + head];
-          const float dlt_q = delta[(long)(base + qcl) * hq + head];
+          const bool all = qbase + sc * 16 >= kv0 + 15 &&
+                           qbase + sc * 16 + 15 < n;      // uniform
           float ptv[4], dstv[4];
           #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int kpos = kv0 + lhi * 4 + i;
-            const bool live = (qpos < n) && (kpos < n) && (qpos >= kpos);
-            const float p =
-                live ? __builtin_amdgcn_exp2f(stf[i] * scale2 - lse_q) : 0.f;
+            float x = fmaf(stf[i], scale2, -lse_q[sc]);
+            if (!all && (qpos >= n || kpos >= n || qpos < kpos))
+              x = -INFINITY;
+            const float p = __builtin_amdgcn_exp2f(x);
             ptv[i] = p;
-            dstv[i] = p * (dptf[i] - dlt_q) * scale;
+            dstv[i] = p * (dptf[i] - dlt_q[sc]);
           }
           const int qk = qrow & 31;
           const int sel = (qk % 8) >= 4, r = (qk / 8) * 4 + (qk % 4);
@@ -460,13 +498,13 @@ void attn_bwd_dkv_kernel(float* __restrict__ dk,        // [T, HKV, D] f32
       if (per == 1) {
         #pragma unroll
         for (int c = 0; c < DC16; ++c) {
-          dk[roff + c * 16 + llo] = dk_acc[c][i];
+          dk[roff + c * 16 + llo] = dk_acc[c][i] * scale;
           dv[roff + c * 16 + llo] = dv_acc[c][i];
         }
       } else {
         #pragma unroll
         for (int c = 0; c < DC16; ++c) {
-          unsafeAtomicAdd(&dk[roff + c * 16 + llo], dk_acc[c][i]);
+          unsafeAtomicAdd(&dk[roff + c * 16 + llo], dk_acc[c][i] * scale);
           unsafeAtomicAdd(&dv[roff + c * 16 + llo], dv_acc[c][i]);
         }
       }
@@ -492,13 +530,13 @@ void launch_attn_bwd_delta(float* delta, const bf16_t* dout,
 }
 
 // Query heads of a group whose shares of dK and dV a workgroup adds up in
-// registers before its atomic additions, which a head at a time are a third of
-// the time at 71 heads on one. More of them leave too few workgroups. us of the
-// backward on a MI355X with 1, 2, 4 heads (2 x 2048: sequences x length):
-//   1 x 1024, 71 on 1 of 64   132  155  246     2 x 2048   740  633  677
-//   8 x 2048, the same       2697 2331 2233    16 x 512    564  470  419
-//   8 x 512, 32 on 8 of 128   291  221  239     2 x 2048   616  553  766
-//   8 x 2048, the same       2401 2232 2126     2 x 512     89  115  180
+// registers before its atomic additions, a tenth to a quarter of the time a
+// head at a time. More of them leave too few workgroups. us of the backward on
+// a MI355X with 1, 2, 4 heads (2 x 2048: sequences x length):
+//   1 x 1024, 71 on 1 of 64   125  144  227     2 x 2048   656  593  619
+//   8 x 2048, the same       2387 2234 2182    16 x 512    539  479  430
+//   8 x 512, 32 on 8 of 128   272  214  230     2 x 2048   532  480  663
+//   8 x 2048, the same       2143 2025 1934     2 x 512     86  107  165
 int attn_bwd_heads(int num_seqs, int max_len, int hq, int hkv) {
   const long all = (long)num_seqs * hq * ((max_len + BW_TILE - 1) / BW_TILE);
   return min(all >= 8192 ? 4 : all >= 2048 ? 2 : 1, hq / hkv);

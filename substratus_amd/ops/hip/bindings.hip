@@ -447,16 +447,17 @@ void attn_train_bwd_v5(torch::Tensor dq, torch::Tensor dk,
                         lse.data_ptr<float>(), delta.data_ptr<float>(),
                         seq_start.data_ptr<int>(), num_seqs, (int)max_len,
                         hq, hkv, d, (float)scale, stream());
-  // dkv: the V5 structure's 256-row tiles and 32-row blocks pay for long
-  // sequences only. us of the backward on a MI355X, 16 rows a wave and V5:
-  // 32 heads of 128, 16 x 512 533, 742; 4 x 2048 1176, 1179; 1 x 4096 1037,
-  // 1001; 2 x 8192 8245, 6583. On 8 heads, 1 x 4096 1000, 1272; 2 x 8192 7719,
-  // 6343. SUB_ATTN_DKV_V5=0/1 overrides.
+  // dkv: the V5 structure's 256-row tiles and 32-row blocks pay where there
+  // are enough of them. us of the backward on a MI355X, 16 rows a wave and V5:
+  // 32 heads of 128, 4 x 1024 314, 339; 4 x 2048 1149, 1026; 2 x 8192 7057,
+  // 5666. On 8 heads, 2 x 2048 480, 634; 8 x 2048 1934, 1657; 1 x 4096 858,
+  // 1088; 1 x 8192 3294, 3000. 71 heads on one of 64, 8 x 2048 2182, 2473;
+  // 2 x 8192 7718, 6003. SUB_ATTN_DKV_V5=0/1 overrides.
   const char* e = getenv("SUB_ATTN_DKV_V5");
+  const bool many = d == 128 &&
+      attn_bwd_heads(num_seqs, max_len, hq, hkv) >= 4;
   const bool use_v5 = e ? (e[0] == '1')
-      : hq == hkv ? max_len >= 4096
-                  : max_len >= 8192 &&
-                        attn_bwd_heads(num_seqs, max_len, hq, hkv) >= 4;
+      : max_len >= (hq == hkv || many ? 2048 : 8192);
   if (use_v5)
     launch_attn_bwd_dkv_v5(dk.data_ptr<float>(), dv.data_ptr<float>(),
                            bfc(q), bfc(k), bfc(v), bfc(dout),

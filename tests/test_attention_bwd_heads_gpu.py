@@ -33,3 +33,24 @@ def test_heads(b, s, hq, hkv, d):
     for g, w in zip(got, want):
         off = (g[-1:].double() - w.double()).norm() / w.double().norm()
         assert float(off) < 2.0 ** -7, float(off)
+
+
+@pytest.mark.parametrize("scale", [0.125, 0.0, -0.2])
+@pytest.mark.parametrize("lens", [[1, 63, 64, 65], [255, 256, 257], [600]])
+def test_forward(lens, scale):
+    """Rows on both sides of the diagonal's chunks, scales of any sign."""
+    torch.manual_seed(sum(lens))
+    ss = torch.tensor([0] + lens).cumsum(0).int()
+    q, k, v = (torch.randn(sum(lens), h, 64, device=DEV).bfloat16()
+               for h in (4, 2, 2))
+    got = ops.attn_prefill(q, k, v, ss.to(DEV), scale)
+    for lo, hi in zip(ss[:-1].tolist(), ss[1:].tolist()):
+        qq, kk, vv = (t[lo:hi].double().transpose(0, 1) for t in (
+            q, *(t.repeat_interleave(2, 1) for t in (k, v))))
+        mask = torch.ones(hi - lo, hi - lo, device=DEV,
+                          dtype=torch.bool).tril()
+        p = torch.softmax((torch.matmul(qq, kk.mT.contiguous()) * scale)
+                          .masked_fill(~mask, -torch.inf), -1)
+        want = torch.matmul(p, vv).transpose(0, 1)
+        off = (got[lo:hi].double() - want).norm() / want.norm()
+        assert float(off) < 2.0 ** -7, float(off)   # bf16 weights and results
