@@ -29,16 +29,16 @@
 // us on a MI355X, 15360 x 5120, 5120 x 5120, 27648 x 5120, 5120 x 13824, from
 // one wave per weight row in vector arithmetic (up to 8 rows of x), or from
 // unpacking to bf16 in memory and the library (more), to this kernel:
-//   q4_0  1 row   20.5  8.5 31.7 15.0 -> 14.4  7.3 21.4 14.8
-//         5 rows  55.0 21.5 95.3 47.8 -> 16.1  9.3 25.6 18.8
+//   q4_0  1 row   20.5  8.5 31.7 15.0 -> 12.7  7.0 21.8 14.4
+//         5 rows  55.0 21.5 95.3 47.8 -> 13.7  7.9 22.6 16.3
 //        24 rows  81.4 37.8  152 75.9 -> 28.1 15.3 45.8 33.4
-//   q8_0  5 rows  55.9 21.2 97.5 46.3 -> 22.8 12.1 36.5 25.0
+//   q8_0  5 rows  55.9 21.2 97.5 46.3 -> 23.7 12.7 38.3 26.6
 //        24 rows  82.5 38.8  155 78.9 -> 42.1 20.8 70.2 43.5
-//   q4_K  1 row   29.4 12.9 49.4 24.6 -> 15.7  8.5 24.9 22.1
-//         5 rows   115 47.7  196  111 -> 18.0 10.4 28.8 25.4
+//   q4_K  1 row   29.4 12.9 49.4 24.6 -> 13.6  7.6 22.9 17.0
+//         5 rows   115 47.7  196  111 -> 16.3  8.8 26.6 19.9
 //        24 rows  90.1 37.8  172 84.6 -> 30.7 16.8 50.2 39.9
-//   q6_K  1 row   32.7 13.3 57.5 26.8 -> 20.8 11.8 33.1 26.3
-//         5 rows   118 40.9  205 90.9 -> 23.1 13.0 37.4 29.0
+//   q6_K  1 row   32.7 13.3 57.5 26.8 -> 21.4 11.6 31.9 26.6
+//         5 rows   118 40.9  205 90.9 -> 23.4 13.0 34.4 29.1
 //        24 rows   523  196  946  479 -> 38.4 19.5 64.8 46.9
 // q8_0 with one row stays with the vector kernel (quant_gemv.hip): 20.5, 9.4,
 // 33.1, 19.3 there and 19.9, 11.1, 32.2, 23.8 here.
@@ -450,15 +450,32 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
     constexpr integral_constant<int, 8> c8{};
     constexpr integral_constant<int, 16> c16{};
     constexpr integral_constant<int, 32> c32{};
-    // stages in flight for few rows: q6_K's are the largest
-    constexpr integral_constant<int, QQ == Quant::Q6_K ? 1 : 2> few{};
+    // Stages in flight for few rows: q6_K's are the largest, q4_0's unpacking
+    // pays for none. Little more than a workgroup per CU: eight waves share k
+    // instead of four, since a wave's chain of stages is what takes the time.
+    // us on a MI355X, 4096 x 14336, 5120 x 13824, four waves -> eight: q4_0 5
+    // rows 15.5, 18.9 -> 12.1, 16.3; q4_K 1 row 13.1, 17.1 -> 10.6, 16.5, 5
+    // rows 15.1, 20.0 -> 13.3, 19.4; q6_K 1 row 23.0, 28.1 -> 16.7, 25.9.
+    // 27648 x 5120, q4_0 5 rows: two stages in flight 26.0, one 22.7; eight
+    // waves 24.8.
+    constexpr bool ONE = QQ == Quant::Q6_K || QQ == Quant::Q4_0;
+    constexpr integral_constant<int, ONE ? 1 : 2> some{};
+    constexpr integral_constant<int, QQ == Quant::Q8_0 ? 4 : 8> waves{};
+    const bool thin = n <= 384 * 16;
     if (m == 1) {
-      if constexpr (QQ == Quant::Q4_0) go(qc, c4, c1, c8, c1);
-      else if constexpr (QQ != Quant::Q8_0) go(qc, c4, c1, c4, few);
+      if constexpr (QQ == Quant::Q4_0) {
+        go(qc, c4, c1, c8, c1);
+      } else if constexpr (QQ != Quant::Q8_0) {
+        if (thin) go(qc, c4, c1, waves, some);
+        else go(qc, c4, c1, c4, some);
+      }
     } else if (m <= 4) {
-      go(qc, c4, c4, c4, few);
+      if (thin) go(qc, c4, c4, waves, some);
+      else go(qc, c4, c4, c4, some);
     } else if (m <= 8) {
-      go(qc, c8, c4, c4, few);
+      constexpr integral_constant<int, QQ == Quant::Q8_0 ? 2 : 1> one{};
+      if (thin) go(qc, c8, c4, waves, one);
+      else go(qc, c8, c4, c4, some);
     } else if (m <= 16) {
       go(qc, c16, c4, c4, c1);
     } else {
