@@ -363,7 +363,7 @@ class CausalLM(nn.Module):
     def forward_train(self, tokens: torch.Tensor) -> torch.Tensor:
         """tokens: [B, S] -> logits [B, S, V], differentiable."""
         b, s = tokens.shape
-        h = self.embed_tokens(tokens)
+        h = train_ops.lookup(tokens, self.embed_tokens)
         pos = torch.arange(s, device=tokens.device)
         if self.cfg.learned_pos_emb:
             h = h + self.embed_positions(pos)

@@ -42,6 +42,7 @@ void launch_add_norm_fwd(bf16_t*, bf16_t*, float*, const bf16_t*, const bf16_t*,
 void launch_add_norm_bwd(bf16_t*, bf16_t*, bf16_t*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const bf16_t*, long, int, bool, hipStream_t);
 void launch_rope_split(bf16_t*, bf16_t*, bf16_t*, const bf16_t*, const float*, const float*, long, int, int, int, int, hipStream_t);
 void launch_rope_join(bf16_t*, const bf16_t*, const float*, const float*, const float*, const float*, long, int, int, int, int, hipStream_t);
+void launch_lookup_bwd(bf16_t*, const bf16_t*, const long*, int, long, int, hipStream_t);
 void launch_silu_mul_bwd(bf16_t*, const bf16_t*, const bf16_t*, long, int, hipStream_t);
 void launch_softmax_sample(long*, const bf16_t*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
 void launch_softmax_sample(long*, const float*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
@@ -210,6 +211,19 @@ void rope_join(torch::Tensor dqkv, torch::Tensor dq, torch::Tensor dk,
                    s ? s->data_ptr<float>() : nullptr, rows, length, hq, hkv,
                    d, stream());
   post_launch_check("rope_join");
+}
+
+// dw, zero before, gets the sums of dy's rows at tokens, which are rows of dw.
+void lookup_bwd(torch::Tensor dw, torch::Tensor dy, torch::Tensor tokens) {
+  const long n = tokens.numel(), hidden = dw.size(1);
+  TORCH_CHECK(dw.dim() == 2 && n > 0 && n < (1L << 30) &&
+              train_norm_takes(hidden), "width ", hidden, " not taken");
+  TORCH_CHECK(tokens.is_cuda() && tokens.scalar_type() == torch::kLong &&
+              tokens.is_contiguous(), "tokens must be int64 on GPU");
+  check_rows(dw, dw.numel(), "dw"); check_rows(dy, n * hidden, "dy");
+  launch_lookup_bwd(bf(dw), bfc(dy), tokens.data_ptr<long>(), n, dw.size(0),
+                    hidden, stream());
+  post_launch_check("lookup_bwd");
 }
 
 void silu_mul_bwd(torch::Tensor dx, torch::Tensor dy, torch::Tensor x) {
@@ -993,6 +1007,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_split", &rope_split);
   m.def("rope_join", &rope_join);
   m.def("silu_mul_bwd", &silu_mul_bwd);
+  m.def("lookup_bwd", &lookup_bwd);
   m.def("rms_norm", &rms_norm);
   m.def("rms_norm_residual", &rms_norm_residual);
   m.def("layer_norm", &layer_norm);

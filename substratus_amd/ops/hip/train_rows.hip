@@ -369,6 +369,58 @@ __global__ __launch_bounds__(BLOCK) void silu_mul_bwd_kernel(
   }
 }
 
+// Gradient of a lookup, whose rows are zero already. A workgroup per token: the
+// first one of a number adds up the rows of all of them, in their order. It
+// looks through all tokens for that, which is less than sorting them up to
+// some thousands (MI355X: 3 x 777 tokens of 32000 x 2048 154 us by torch's
+// kernels, 11 by this; 2 x 2048 of 65024 x 4544 142, 31).
+template <int CAP>
+__global__ __launch_bounds__(BLOCK) void lookup_bwd_kernel(
+    bf16_t* __restrict__ dw, const bf16_t* __restrict__ dy,
+    const long* __restrict__ tokens, int n, long rows, int hidden) {
+  __shared__ unsigned long long same[NWAVES];
+  const int i = blockIdx.x, tid = threadIdx.x;
+  const long t = tokens[i];
+  if (t < 0 || t >= rows) return;
+  bool before = false;
+  for (int j = tid; j < i; j += BLOCK) before |= tokens[j] == t;
+  if (__syncthreads_or(before)) return;
+  const int nvec = hidden / 8;
+  float sum[CAP][8];
+  #pragma unroll
+  for (int c = 0; c < CAP; ++c)
+    #pragma unroll
+    for (int e = 0; e < 8; ++e) sum[c][e] = 0.f;
+  for (int j0 = i; j0 < n; j0 += BLOCK) {
+    const int j = j0 + tid;
+    const unsigned long long mine =
+        __ballot(j < n && tokens[min(j, n - 1)] == t);
+    if (tid % WAVE == 0) same[tid / WAVE] = mine;
+    __syncthreads();
+    for (int w = 0; w < NWAVES; ++w)
+      for (unsigned long long m = same[w]; m; m &= m - 1) {
+        const long row = j0 + w * WAVE + __builtin_ctzll(m);
+        const uint4* v = reinterpret_cast<const uint4*>(dy + row * hidden);
+        #pragma unroll
+        for (int c = 0; c < CAP; ++c) {
+          const int at = tid + c * BLOCK;
+          if (at >= nvec) break;
+          float f[8];
+          unpack8(v[at], f);
+          #pragma unroll
+          for (int e = 0; e < 8; ++e) sum[c][e] += f[e];
+        }
+      }
+    __syncthreads();
+  }
+  uint4* out = reinterpret_cast<uint4*>(dw + t * hidden);
+  #pragma unroll
+  for (int c = 0; c < CAP; ++c) {
+    const int at = tid + c * BLOCK;
+    if (at < nvec) out[at] = pack8(sum[c]);
+  }
+}
+
 template <class F>
 void by_width(int hidden, F go) {
   const int cap = (hidden / 8 + BLOCK - 1) / BLOCK;
@@ -444,4 +496,12 @@ void launch_silu_mul_bwd(bf16_t* dx, const bf16_t* dy, const bf16_t* x,
   const int most = (f / 8 + BLOCK - 1) / BLOCK;
   silu_mul_bwd_kernel<<<dim3(rows, std::min(most, 4)), dim3(BLOCK), 0,
                         stream>>>(dx, dy, x, f);
+}
+
+void launch_lookup_bwd(bf16_t* dw, const bf16_t* dy, const long* tokens,
+                       int n, long rows, int hidden, hipStream_t stream) {
+  by_width(hidden, [&](auto cap) {
+    lookup_bwd_kernel<decltype(cap)::value>
+        <<<dim3(n), dim3(BLOCK), 0, stream>>>(dw, dy, tokens, n, rows, hidden);
+  });
 }

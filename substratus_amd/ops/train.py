@@ -40,6 +40,45 @@ def _whole(*tensors: Optional[torch.Tensor]) -> bool:
                and t.numel() > 0 and t.data_ptr() % 16 == 0 for t in given)
 
 
+# -------------------------------------------------------------------- lookup
+
+class _Lookup(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, tokens, weight):
+        tokens = tokens.contiguous()
+        ctx.save_for_backward(tokens, weight)
+        return F.embedding(tokens, weight)
+
+    @staticmethod
+    def backward(ctx, dy):
+        tokens, weight = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return None, _again(lambda w: F.embedding(tokens, w), (weight,),
+                                dy)[0]
+        dw = torch.zeros_like(weight)
+        _load_ext().lookup_bwd(dw, _aligned(dy), tokens)
+        return None, dw
+
+
+def lookup(tokens: torch.Tensor, table: torch.nn.Embedding) -> torch.Tensor:
+    """table(tokens). Up to 8192 of them on the GPU get their gradients from a
+    kernel of their own."""
+    w = table.weight
+    if (type(table) is torch.nn.Embedding and table.padding_idx is None
+            and table.max_norm is None and not table.sparse
+            and not table.scale_grad_by_freq
+            and not torch.nn.modules.module._has_any_global_hook()
+            and not any((table._forward_hooks, table._forward_pre_hooks,
+                         table._backward_hooks, table._backward_pre_hooks))
+            and w.requires_grad and torch.is_grad_enabled() and _whole(w)
+            and tokens.dtype == torch.int64 and tokens.device == w.device
+            and 0 < tokens.numel() <= 8192
+            and plain_tensors(tokens, w) and _load_ext() is not None
+            and _load_ext().train_norm_takes(w.shape[1])):
+        return _Lookup.apply(tokens, w)
+    return table(tokens)
+
+
 # --------------------------------------------------------------------- norms
 
 def _add(h: torch.Tensor, deltas: Sequence[torch.Tensor]) -> torch.Tensor:

@@ -118,3 +118,30 @@ def test_silu_mul(rows, f):
     # the slope is a difference of terms near 1 around its zero
     near(dx, dw, torch.cat([x.detach()[:, f:] * dy, dy], 1).abs().double()
          * 16)
+
+
+@pytest.mark.parametrize("n,rows,width", [(1, 5, 8), (255, 3, 64),
+                                          (257, 1000, 2056), (3000, 40, 2048),
+                                          (8192, 9, 72), (700, 5000, 8192)])
+def test_lookup(n, rows, width):
+    """Numbers that come once, often and on both sides of a workgroup."""
+    torch.manual_seed(n)
+    table = torch.nn.Embedding(rows, width, device=DEV,
+                               dtype=torch.bfloat16)
+    tokens = torch.randint(rows, (2, n), device=DEV)[:, :(n + 1) // 2]
+    out = train.lookup(tokens, table)
+    assert out.grad_fn.name().startswith("_Lookup")
+    assert torch.equal(out, table(tokens))
+    dy = rand(*out.shape, seed=2)
+    got, = torch.autograd.grad(out, table.weight, dy)
+    want = torch.zeros(rows, width, device=DEV, dtype=torch.float64)
+    size = want.clone()
+    flat = dy.reshape(-1, width).double()
+    want.index_add_(0, tokens.reshape(-1), flat)
+    size.index_add_(0, tokens.reshape(-1), flat.abs())
+    near(got, want, size)
+    assert torch.equal(got, torch.autograd.grad(
+        train.lookup(tokens, table), table.weight, dy)[0])
+    table.register_forward_hook(lambda *a: None)
+    assert not train.lookup(tokens, table).grad_fn.name().startswith(
+        "_Lookup")
