@@ -11,14 +11,15 @@
 // Bound by the chain of steps; one row occupies a CU. On a MI355X, 192 rows
 // of 32000, a quarter each greedy and top-k, half top-p: 32 us (292 us with
 // the row in LDS, 256 threads and 24 halvings of the value range per
-// threshold). 256 rows of 65024: 18 us greedy, 42 without thresholds, 69 to 88
-// with them (registers spill from 32768 logits on).
+// threshold). 256 rows of 65024: 27 us greedy, 89 without thresholds, 123
+// with them as above (87, 133, 594); registers spill from 32768 logits on.
 #include "common.h"
 
 #define SBLOCK 1024
 #define SNW (SBLOCK / WAVE)
 #define SVEC 8                    // consecutive logits of a thread per round
 #define SROUND (SBLOCK * SVEC)
+#define RUNS 256                  // runs of tokens that a draw's edges are of
 
 namespace {
 
@@ -102,7 +103,6 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
                            const float* __restrict__ top_p,
                            const float* __restrict__ uniform, int vocab) {
   __shared__ float s_tot[2][SNW];
-  __shared__ float s_part[NR][SNW];
   __shared__ int s_idx[SNW];
   __shared__ int s_tok;
   Totals totals{s_tot};
@@ -214,56 +214,99 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   }
 
   // ---- inverse-CDF draw, in token order ---------------------------------
-  float mine[NR];
-  #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    mine[r] = 0.f;
+  // Which token a number falls to depends on how sums are rounded: about every
+  // two-hundredth draw from thousands of tokens lies that close to an edge. So
+  // that a row and a number keep their token, the sum is that of 256 threads
+  // over every 256th token, the edges those of 256 runs of tokens, added up
+  // from left to right, as they always were (2 us of the 32 above).
+  constexpr bool KEPT = NR <= 4;      // weights fit LDS; else made again, out
+  constexpr int RAW = KEPT || sizeof(T) == 4    // of logits where those do
+      ? 1 : NR * SROUND < 77824 ? NR * SROUND : 77824;
+  __shared__ float s_w[KEPT ? NR * SROUND : 1];
+  __shared__ T s_raw[RAW];
+  __shared__ float s_run[RUNS];
+  if constexpr (KEPT) {
     #pragma unroll
-    for (int j = 0; j < SVEC; ++j)
-      mine[r] += e[r][j] >= thresh ? e[r][j] : 0.f;
-    const float t = wave_sum(mine[r]);
-    if (lane == 0) s_part[r][wave] = t;
-    __builtin_amdgcn_sched_barrier(0);
+    for (int r = 0; r < NR; ++r) {
+      float4 w[2];
+      float* f = reinterpret_cast<float*>(w);
+      #pragma unroll
+      for (int j = 0; j < SVEC; ++j) f[j] = e[r][j] >= thresh ? e[r][j] : 0.f;
+      float4* to = reinterpret_cast<float4*>(s_w + r * SROUND + tid * SVEC);
+      to[0] = w[0];
+      to[1] = w[1];
+    }
+  } else if constexpr (RAW > 1) {
+    #pragma unroll 8
+    for (int i = tid; i < min(vocab, RAW); i += SBLOCK) s_raw[i] = row[i];
   }
   if (tid == 0) s_tok = -1;
   __syncthreads();
-  float z = 0.f;
-  for (int q = 0; q < NR * SNW; ++q) z += s_part[q / SNW][q % SNW];
-  const float goal = uniform[b] * z;
-  float before = 0.f;
-  int part = -1;              // round and wave in which the sum reaches goal
-  #pragma unroll 8
-  for (int q = 0; q < NR * SNW; ++q) {
-    const float t = s_part[q / SNW][q % SNW];
-    if (part < 0) {
-      if (before + t > goal) part = q; else before += t;
+  auto kept_weight = [&](int i) {
+    if constexpr (KEPT) {
+      return s_w[i];
+    } else {
+      const float w =
+          weight(val(RAW > 1 && i < RAW ? s_raw[i] : row[i]));
+      return w >= thresh ? w : 0.f;
+    }
+  };
+  const int run = (vocab + RUNS - 1) / RUNS;
+  if (tid < RUNS) {
+    float sum = 0.f;
+    #pragma unroll 16
+    for (int i = tid; i < vocab; i += RUNS) sum += kept_weight(i);
+    sum = wave_sum(sum);
+    if (lane == 0) s_tot[0][wave] = sum;
+  } else if (tid < 2 * RUNS) {
+    const int from = (tid - RUNS) * run, end = min(from + run, vocab);
+    float sum = 0.f;
+    #pragma unroll 16
+    for (int i = from; i < end; ++i) sum += kept_weight(i);
+    s_run[tid - RUNS] = sum;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float z = 0.f;
+    #pragma unroll
+    for (int q = 0; q < RUNS / WAVE; ++q) z += s_tot[0][q];
+    const float goal = uniform[b] * z;
+    constexpr int EACH = RUNS / WAVE;
+    float mine[EACH], edge[EACH], before = 0.f, upto = 0.f;
+    #pragma unroll
+    for (int q = 0; q < EACH; ++q) mine[q] = s_run[lane * EACH + q];
+    for (int l = 0; l < WAVE; ++l) {
+      if (lane == l) before = upto;
+      #pragma unroll
+      for (int q = 0; q < EACH; ++q) {
+        upto += __uint_as_float(
+            __builtin_amdgcn_readlane(__float_as_uint(mine[q]), l));
+        if (lane == l) edge[q] = upto;
+      }
+    }
+    #pragma unroll
+    for (int q = 0; q < EACH; ++q) {
+      if (goal >= before && goal < edge[q]) {
+        const int from = (lane * EACH + q) * run;
+        const int end = min(from + run, vocab);
+        float acc = before;
+        int sel = -1;
+        for (int i = from; i < end && sel < 0; i += 8) {
+          float w[8];
+          #pragma unroll
+          for (int j = 0; j < 8; ++j)
+            w[j] = i + j < end ? kept_weight(i + j) : 0.f;
+          #pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            acc += w[j];
+            if (sel < 0 && w[j] > 0.f && acc > goal) sel = i + j;
+          }
+        }
+        if (sel >= 0) s_tok = sel;
+      }
+      before = edge[q];
     }
   }
-  #pragma unroll
-  for (int r = 0; r < NR; ++r)
-    if (part == r * SNW + wave) {
-      float upto = mine[r];     // with the lanes before
-      #pragma unroll
-      for (int off = 1; off < WAVE; off <<= 1) {
-        const float o = __shfl_up(upto, off, WAVE);
-        if (lane >= off) upto += o;
-      }
-      const float end = before + upto;
-      const unsigned long long over = __ballot(end > goal);
-      const int who = over ? __ffsll(over) - 1 : WAVE - 1;
-      if (lane == who) {
-        float acc = end - mine[r];
-        int sel = -1;
-        #pragma unroll
-        for (int j = 0; j < SVEC; ++j)
-          if (e[r][j] >= thresh) {
-            // the lane's last one where rounding leaves the sum short
-            if (sel < 0 || acc <= goal) sel = r * SROUND + tid * SVEC + j;
-            acc += e[r][j];
-          }
-        s_tok = sel;
-      }
-    }
   __syncthreads();
   if (s_tok >= 0) {
     if (tid == 0) out[b] = s_tok;
