@@ -42,9 +42,8 @@ def parse_args():
     p.add_argument("--prompt-len", type=int, default=512)
     p.add_argument("--micro-batch", type=int, default=16,
                    help="per-GPU micro batch (train mode; 16 is the "
-                        "measured 1xMI355X sweet spot — 20.5k tok/s vs "
-                        "18.3k at mb4; mb32 exceeds 288 GB without "
-                        "gradient checkpointing)")
+                        "measured 1xMI355X sweet spot, 24.8k tok/s; mb32 "
+                        "exceeds 288 GB without gradient checkpointing)")
     p.add_argument("--seq-len", type=int, default=None)
     p.add_argument("--prefill-chunk", type=int, default=None,
                    help="max packed prefill tokens per step (default: "
