@@ -250,15 +250,29 @@ def inference_only(*tensors: torch.Tensor) -> bool:
     return plain_tensors(*tensors)
 
 
+def _rows_gemm_pays(numel: int, n: int, k: int) -> bool:
+    """Whether a product of numel / k rows is faster by rows_gemm.hip than by
+    the library. Up to 16 rows always: it reads the weights once. Then every
+    workgroup, 16 columns, reads all rows as well, which costs less than the
+    library's few tiles where there is no more than a workgroup per CU. us, the
+    library's and ours:
+        32 x 4096 x 4096    14.2  12.7     48 x 4096 x 4096    14.0  15.2
+        32 x 6144 x 4096    16.7  22.2     64 x 4096 x 2048    12.2  10.6
+        24 x 2048 x 5632    11.8  12.4     64 x 6144 x 2048    13.4  18.2
+    """
+    return numel <= 16 * k or n <= 4096 and (
+        k <= 4096 and numel <= 32 * k or k <= 2048 and numel <= 64 * k)
+
+
 def _few_rows(x: torch.Tensor, weight: torch.Tensor,
               bias: Optional[torch.Tensor], gated: bool):
     """(x as rows, extension) where the product goes to rows_gemm.hip, or
-    None. From 17 rows on the library is as fast or faster (28 x 4096 x 4096:
-    13.3 us there, 12.9 here; 28 x 22016 x 4096: 43.6, 47.6)."""
+    None."""
     if not (x.is_cuda and weight.is_cuda and x.device == weight.device
             and x.dtype == weight.dtype == torch.bfloat16 and x.dim() >= 1
             and weight.dim() == 2 and x.shape[-1] == weight.shape[1]
-            and 0 < x.numel() <= 16 * x.shape[-1]):
+            and x.numel() > 0
+            and _rows_gemm_pays(x.numel(), *weight.shape)):
         return None
     if bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_cuda
                                  and bias.is_contiguous()
@@ -364,10 +378,10 @@ def _many_rows(x: torch.Tensor, weight: torch.Tensor,
 
 def linear(x: torch.Tensor, weight: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """F.linear. Up to 16 rows of bf16 without gradients take the kernel that
-    streams weights at the memory's rate (rows_gemm.hip), products of 256 rows
-    and more the one for the matrix cores (tile_gemm.hip) where that is the
-    faster one, in a backward as well. SUB_MGEMM=1 routes decode shapes of 256
+    """F.linear. Up to 16 rows of bf16 without gradients, or up to 64 with a
+    matrix of few rows, take the kernel that streams weights at the memory's
+    rate (rows_gemm.hip), products of 256 rows and more the one for the matrix
+    cores (tile_gemm.hip) where that is the faster one, in a backward as well. SUB_MGEMM=1 routes decode shapes of 256
     rows and more to the 256x256 glds GEMM (mfma_gemm.hip).
 
     The latter is NOT on by default: the round-3 measurement

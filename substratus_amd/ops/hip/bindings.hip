@@ -530,7 +530,7 @@ long mfma_gemm_pick_splitk(long m, long n, long k) {
   return mfma_gemm_splitk((int)m, (int)n, (int)k);
 }
 
-// y = x w^T + bias, at most 16 rows of x; gated: y has half the columns,
+// y = x w^T + bias, at most 64 rows of x; gated: y has half the columns,
 // silu(first half) * second half
 bool rows_gemm_ok(long m, long n, long k, bool gated) {
   return rows_gemm_takes((int)m, (int)n, (int)k, gated);

@@ -1,4 +1,4 @@
-// y = x w^T + bias of at most 16 rows with a bf16 weight matrix [n, k], as
+// y = x w^T + bias of at most 64 rows with a bf16 weight matrix [n, k], as
 // single tokens of a small batch need it; or, of a matrix whose first half
 // gates its second, silu(gate) * up; or, of a projection of heads, rotated
 // queries, with keys and values appended to the cache.
@@ -20,8 +20,17 @@
 //   1 x 11264 x 2048   16.1 -> 10.2    8 x 22016 x 4096   52.8 -> 35.9
 //   1 x 2048 x 5632    11.2 -> 7.4     8 x 4096 x 11008   37.7 -> 19.5
 // (5.0 to 5.4 TB/s where the matrix is large). 8 and 16 waves, or 32 rows of
-// weights, are slower: fewer workgroups per CU. With 28 rows of x and more,
-// two operand tiles of x per wave, the library is the faster one.
+// weights, are slower: fewer workgroups per CU.
+//
+// With 17 to 64 rows a wave has two to four operand tiles of x, and every
+// workgroup reads all of x: that, not the weights, then sets the pace, so it
+// pays for matrices of few rows only, of which the library's tiles make too
+// few workgroups.
+//   20 x 3072 x 2048   11.8 -> 6.4     48 x 3072 x 2048   11.7 -> 8.5
+//   32 x 2048 x 2048   11.2 -> 6.5     64 x 2048 x 2048   11.6 -> 9.9
+//   32 x 4096 x 4096   14.2 -> 12.7    64 x 2304 x 768    7.2 -> 4.4
+// Four stages in flight instead of two, and eight waves, are 2 to 10% slower
+// at these.
 #include "rows_gemm.h"
 
 #include <type_traits>
@@ -29,12 +38,12 @@
 namespace {
 
 constexpr int KW = 4;             // waves, which share k
-constexpr int P = 4;              // stages in flight
 constexpr int U = 2;              // 32-column chunks of a stage
 constexpr int TILE = 64;          // 16-byte pieces of 16 rows x 32 columns
 constexpr int PAD = 4;
 
-template <Columns C, bool NORM>
+// FM: tiles of 16 rows of x; P: stages in flight
+template <Columns C, bool NORM, int FM, int P>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       const bf16_t* __restrict__ w,
@@ -42,8 +51,10 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       long x_ld, long y_ld, Heads heads,
                       NormOf norm) {
   // (normed x does not go through the ring)
-  constexpr int STAGE = U * (NORM ? 1 : 2) * TILE;
-  constexpr int LOADS = U * (NORM ? 1 : 2);
+  static_assert(!NORM || FM == 1);
+  constexpr int TILES = NORM ? 1 : 1 + FM;       // of a chunk of 32 columns
+  constexpr int STAGE = U * TILES * TILE;
+  constexpr int LOADS = U * TILES;
   constexpr int RING = KW * P * STAGE;
   // one array: beside a second one the compiler guards every LDS read against
   // the direct loads in flight, and waits for them
@@ -65,30 +76,41 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
   const char* wp = reinterpret_cast<const char*>(
       w + (long)weight_row<C>(n0, row, n, half) * k) + piece * 16;
-  const char* xp = reinterpret_cast<const char*>(
-      x + min(row, m - 1) * x_ld) + piece * 16;
+  const char* xp[FM];
+  #pragma unroll
+  for (int f = 0; f < FM; ++f)
+    xp[f] = reinterpret_cast<const char*>(
+        x + min(f * 16 + row, m - 1) * x_ld) + piece * 16;
   auto load = [&](int s, int i) {
     #pragma unroll
     for (int u = 0; u < U; ++u) {
       // a stage may be half of one: then its last chunk comes twice
       const unsigned at = (unsigned)min(c0 + i * U + u, c1 - 1) * 64;
-      uint4* to = ring + s * STAGE + u * (NORM ? 1 : 2) * TILE;
+      uint4* to = ring + s * STAGE + u * TILES * TILE;
       load_to_lds<16>(wp + at, to);
-      if constexpr (!NORM) load_to_lds<16>(xp + at, to + TILE);
+      if constexpr (!NORM) {
+        #pragma unroll
+        for (int f = 0; f < FM; ++f)
+          load_to_lds<16>(xp[f] + at, to + (1 + f) * TILE);
+      }
     }
   };
   const int at = lo * 4 + (g ^ ((lo >> 2) & 3));
-  float4v acc = {0.f, 0.f, 0.f, 0.f};
+  float4v acc[FM];
+  #pragma unroll
+  for (int f = 0; f < FM; ++f) acc[f] = (float4v){0.f, 0.f, 0.f, 0.f};
   auto step = [&](int s, int i, bool more) {
-    short8 wf[U], xf[U];
+    short8 wf[U], xf[U][FM];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint4* t = ring + s * STAGE + u * (NORM ? 1 : 2) * TILE + at;
+      const uint4* t = ring + s * STAGE + u * TILES * TILE + at;
       wf[u] = *reinterpret_cast<const short8*>(t);
-      xf[u] = *reinterpret_cast<const short8*>(
-          NORM ? s_x + min(lo, m - 1) * (k / 8 + 1) +
-                     min(c0 + i * U + u, c1 - 1) * 4 + g
-               : t + TILE);
+      #pragma unroll
+      for (int f = 0; f < FM; ++f)
+        xf[u][f] = *reinterpret_cast<const short8*>(
+            NORM ? s_x + min(lo, m - 1) * (k / 8 + 1) +
+                       min(c0 + i * U + u, c1 - 1) * 4 + g
+                 : t + (1 + f) * TILE);
     }
     if (more) {
       wait_lds_reads();
@@ -96,9 +118,12 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     }
     #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (c0 + i * U + u < c1)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0,
-                                                      0);
+      if (c0 + i * U + u < c1) {
+        #pragma unroll
+        for (int f = 0; f < FM; ++f)
+          acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              wf[u], xf[u][f], acc[f], 0, 0, 0);
+      }
   };
   NormRows<KW * WAVE> rows;
   if constexpr (NORM) rows.load(norm, m, k);
@@ -129,27 +154,32 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   __syncthreads();
 
   // the waves' shares are added up; a lane has four columns of one row
+  constexpr int ROWS = FM * 16;
+  static_assert(KW * ROWS * (16 + PAD) <= RING * 4);
   float* red = reinterpret_cast<float*>(s_all);
-  *reinterpret_cast<float4v*>(&red[(wave * 16 + lo) * (16 + PAD) + g * 4]) =
-      acc;
+  #pragma unroll
+  for (int f = 0; f < FM; ++f)
+    *reinterpret_cast<float4v*>(
+        &red[(wave * ROWS + f * 16 + lo) * (16 + PAD) + g * 4]) = acc[f];
   __syncthreads();
-  const int r = threadIdx.x / 16, c = threadIdx.x % 16;
-  if (r >= m) return;
-  const float scale = NORM ? norm_scale<KW>(squares, r, k, norm.eps) : 1.f;
-  auto sum = [&](int c) {
-    float v = 0.f;
-    #pragma unroll
-    for (int q = 0; q < KW; ++q) v += red[(q * 16 + r) * (16 + PAD) + c];
-    if constexpr (NORM) v *= scale;
-    if (bias != nullptr) v += bf2f(bias[weight_row<C>(n0, c, n, half)]);
-    return v;
-  };
-  if constexpr (C == Columns::GATED) {
-    if (c < 8) y[r * y_ld + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
-  } else if constexpr (C == Columns::HEADS) {
-    if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
-  } else {
-    if (n0 + c < n) y[r * y_ld + n0 + c] = f2bf(sum(c));
+  const int c = threadIdx.x % 16;
+  for (int r = threadIdx.x / 16; r < m; r += KW * 4) {
+    const float scale = NORM ? norm_scale<KW>(squares, r, k, norm.eps) : 1.f;
+    auto sum = [&](int c) {
+      float v = 0.f;
+      #pragma unroll
+      for (int q = 0; q < KW; ++q) v += red[(q * ROWS + r) * (16 + PAD) + c];
+      if constexpr (NORM) v *= scale;
+      if (bias != nullptr) v += bf2f(bias[weight_row<C>(n0, c, n, half)]);
+      return v;
+    };
+    if constexpr (C == Columns::GATED) {
+      if (c < 8) y[r * y_ld + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
+    } else if constexpr (C == Columns::HEADS) {
+      if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
+    } else {
+      if (n0 + c < n) y[r * y_ld + n0 + c] = f2bf(sum(c));
+    }
   }
 }
 
@@ -157,7 +187,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
 
 // Rows begin on 16-byte pieces; offsets within a row fit 32 bits.
 bool rows_gemm_takes(int m, int n, int k, bool gated) {
-  return m >= 1 && m <= 16 && n >= 1 && k >= 32 && k % 32 == 0 &&
+  return m >= 1 && m <= 64 && n >= 1 && k >= 32 && k % 32 == 0 &&
          (!gated || n % 16 == 0);
 }
 
@@ -167,14 +197,24 @@ void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
                       long y_ld, bool gated, const Heads* heads,
                       const NormOf* norm, hipStream_t stream) {
-  auto pick = [&](auto normed) {
+  auto launch = [&](auto normed, auto tiles, auto stages) {
     constexpr bool N = decltype(normed)::value;
-    return heads ? rows_gemm_kernel<Columns::HEADS, N>
-           : gated ? rows_gemm_kernel<Columns::GATED, N>
-                   : rows_gemm_kernel<Columns::PLAIN, N>;
+    constexpr int F = decltype(tiles)::value, S = decltype(stages)::value;
+    auto kernel = heads ? rows_gemm_kernel<Columns::HEADS, N, F, S>
+                  : gated ? rows_gemm_kernel<Columns::GATED, N, F, S>
+                          : rows_gemm_kernel<Columns::PLAIN, N, F, S>;
+    kernel<<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
+        y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{},
+        norm ? *norm : NormOf{});
   };
-  auto kernel = norm ? pick(std::true_type{}) : pick(std::false_type{});
-  kernel<<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
-      y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{},
-      norm ? *norm : NormOf{});
+  using std::integral_constant;
+  constexpr integral_constant<int, 1> one{};
+  constexpr integral_constant<int, 2> two{};
+  constexpr integral_constant<int, 3> three{};
+  constexpr integral_constant<int, 4> four{};
+  if (norm) launch(std::true_type{}, one, four);
+  else if (m <= 16) launch(std::false_type{}, one, four);
+  else if (m <= 32) launch(std::false_type{}, two, two);
+  else if (m <= 48) launch(std::false_type{}, three, two);
+  else launch(std::false_type{}, four, two);
 }

@@ -67,8 +67,8 @@ def test_heads(kind, m, hq, hkv, d, k, bias, theta, fp8):
 def test_heads_refused():
     """What the kernel does not read goes the general way."""
     lin = projection("dense", 64, 6 * 64, False)
-    x = torch.randn(17, 64, device=DEV).bfloat16()
-    pos = torch.arange(17, device=DEV).int()
+    x = torch.randn(65, 64, device=DEV).bfloat16()
+    pos = torch.arange(65, device=DEV).int()
     k, v = (torch.zeros(17, 1, 16, 64, device=DEV).bfloat16()
             for _ in range(2))
     ok = ops.Cache(pos[:4], k, v, pos[:4], 1e4)
