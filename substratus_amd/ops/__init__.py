@@ -351,27 +351,27 @@ def _many_rows(x: torch.Tensor, weight: torch.Tensor,
                gated: bool = False) -> Optional[torch.Tensor]:
     """F.linear of 256 rows and more, or None where torch's is as good; or what
     linear_gated makes of it, without gradients."""
-    given = [t for t in (x, weight, bias) if t is not None]
     if not (x.is_cuda and weight.dim() == 2 and weight.shape[0] >= 256
             and x.dim() >= 2 and x.shape[-1] == weight.shape[1] > 0
-            and x.numel() >= 256 * x.shape[-1]
-            and all(t.device == x.device and t.dtype == torch.bfloat16
-                    for t in given)
-            and _load_ext() is not None and plain_tensors(*given)):
+            and x.numel() >= 256 * x.shape[-1] and _load_ext() is not None):
         return None
-    rows = x.reshape(-1, x.shape[-1])
-    if torch.is_grad_enabled() and any(t.requires_grad for t in given):
-        if gated:
-            return None
-        m, k, n = *rows.shape, weight.shape[0]
-        good = _load_ext().tile_gemm_good
-        if not (good(m, n, k, k, k, False, False, False)
-                or good(m, k, n, n, k, False, True, False)
-                or good(n, k, m, n, k, True, True, False)):
-            return None
-        y = _Linear.apply(rows, weight, bias)
-    else:
-        y = _tile_gemm(rows, weight, bias, gated=gated)
+    # sizes first, which cost a microsecond: a step of a few hundred rows has
+    # dozens of products that stay with torch's
+    n, k = weight.shape
+    m, good = x.numel() // k, _load_ext().tile_gemm_good
+    given = [t for t in (x, weight, bias) if t is not None]
+    asked = torch.is_grad_enabled() and any(t.requires_grad for t in given)
+    if asked and gated or not (
+            good(m, n, k, k, k, False, False, gated)
+            or asked and (good(m, k, n, n, k, False, True, False)
+                          or good(n, k, m, n, k, True, True, False))):
+        return None
+    if not (all(t.device == x.device and t.dtype == torch.bfloat16
+                for t in given) and plain_tensors(*given)):
+        return None
+    rows = x.reshape(-1, k)
+    y = _Linear.apply(rows, weight, bias) if asked else \
+        _tile_gemm(rows, weight, bias, gated=gated)
     return y if y is None or x.dim() == 2 else \
         y.view(*x.shape[:-1], y.shape[1])
 
