@@ -384,7 +384,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
     cores (tile_gemm.hip) where that is the faster one, in a backward as well. SUB_MGEMM=1 routes decode shapes of 256
     rows and more to the 256x256 glds GEMM (mfma_gemm.hip).
 
-    The latter is NOT on by default: the round-3 measurement
+    The latter is NOT on by default: measurement
     (profiles/mgemm_r02.md) shows hipBLASLt's MT192/MT256 solutions at 1.3-4.1
     TB/s of weight stream on the llama2-7b decode shapes vs our kernel's
     1.0-2.25 — the library's measured rates reach the ceiling measured for a
