@@ -374,9 +374,13 @@ class CausalLM(nn.Module):
         else:
             cos = sin = None
         deltas = ()
+        recompute = self.gradient_checkpointing and torch.is_grad_enabled()
         for blk in self.blocks:
-            if self.gradient_checkpointing and h.requires_grad is not False \
-                    and torch.is_grad_enabled():
+            if recompute:       # what a block left is a part of the one tensor
+                for d in deltas:
+                    h = h + d
+                deltas = ()
+            if recompute and h.requires_grad:
                 h = torch.utils.checkpoint.checkpoint(
                     blk.whole_train, h, cos, sin, use_reentrant=False)
             else:

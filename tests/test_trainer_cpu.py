@@ -4,6 +4,7 @@ checkpoint/resume, and 2-process DDP gradient parity over gloo
 
 import json
 import os
+from dataclasses import replace
 
 import pytest
 import torch
@@ -306,3 +307,33 @@ def test_grad_accum_matches_full_batch(tmp_path):
     for k in params[1]:
         torch.testing.assert_close(params[1][k], params[2][k],
                                    atol=1e-5, rtol=1e-4)
+
+
+@pytest.mark.parametrize("name", ["llama-tiny", "falcon-tiny",
+                                  "falcon40-tiny", "opt"])
+def test_recomputed_blocks_of_frozen_embeddings(name):
+    """The first block's input needs no gradient then, so it is not recomputed
+    and leaves its outputs to the next block, which is."""
+    cfg = replace(get_config("opt-125m"), vocab_size=512, hidden_size=64,
+                  num_layers=3, num_heads=4, num_kv_heads=4,
+                  intermediate_size=128) if name == "opt" else \
+        replace(get_config(name), num_layers=3)
+    model = CausalLM(cfg, dtype=torch.float32)
+    model.init_random(3)
+    for table in (model.embed_tokens, getattr(model, "embed_positions", None)):
+        if table is not None:
+            table.weight.requires_grad_(False)
+    tokens = torch.randint(0, 512, (2, 17),
+                           generator=torch.Generator().manual_seed(5))
+    results, calls = [], []
+    for blk in model.blocks:
+        blk.wqkv.register_forward_pre_hook(lambda *_: calls.append(0))
+    for model.gradient_checkpointing in (False, True):
+        calls.clear()
+        logits = model.forward_train(tokens)
+        grads = torch.autograd.grad(logits.square().sum(),
+                                    list(model.blocks.parameters()))
+        results.append((logits, *grads))
+    assert len(calls) == 2 * cfg.num_layers - 1     # all but the first again
+    for a, b in zip(*results):
+        torch.testing.assert_close(a, b)
