@@ -83,3 +83,26 @@ def test_rows_that_are_not_ordinary():
                 assert got[4] == 0
             elif p == 1:
                 assert abs(got[4] - 0.4 * v) <= 1
+
+
+@pytest.mark.parametrize("k,p", [(0, 1.0), (2, 1.0), (0, 0.9)])
+@pytest.mark.parametrize("temp", [0.6, 0.7, 0.9, 1.3])
+def test_neighbouring_numbers_share_the_draws(temp, k, p):
+    """Two logits a unit of the last place apart weigh the same but for 1e-6,
+    also where they are equal once divided by the temperature."""
+    n, vocab = 64, 3000
+    g = torch.Generator().manual_seed(1)
+    low = torch.rand(n, generator=g) * 25 + 5
+    top = torch.nextafter(low, torch.tensor(100.0))
+    assert int((low * (1 / torch.tensor(temp)) ==
+                top * (1 / torch.tensor(temp))).sum()) > 0
+    rows = torch.full((n, vocab), -100.0)
+    first, second = 17, 2500
+    odd = torch.arange(n) % 2 == 1
+    rows[:, first] = torch.where(odd, top, low)
+    rows[:, second] = torch.where(odd, low, top)
+    of = lambda v, **how: torch.full((n,), v, device=DEV, **how)
+    for u, token in ((0.25, first), (0.75, second)):
+        got = ops.softmax_sample(rows.to(DEV), of(temp),
+                                 of(k, dtype=torch.int32), of(p), of(u))
+        assert got.tolist() == [token] * n
