@@ -583,7 +583,8 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   const Heads* heads, const NormOf* norm = nullptr) {
   check_bf16(y, "y"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
-              x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0,
+              x.dim() == 2 && x.stride(1) == 1 &&
+              (x.stride(0) % 8 == 0 || x.size(0) == 1),
               "x must be bf16 rows that begin on 16-byte pieces");
   const int m = x.size(0), k = x.size(1), n = w.size(0);
   const int cols = heads ? n - 2 * heads->hkv * heads->d : gated ? n / 2 : n;

@@ -81,6 +81,33 @@ def test_linear_forms_that_stay_with_the_library():
     assert ops.linear(x[:0].bfloat16(), w).shape == (0, 64)
 
 
+@torch.no_grad()
+def test_one_row_of_any_stride():
+    """The distance to a next row that is not there tells nothing."""
+    torch.manual_seed(2)
+    n, k, d = 64, 128, 16
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    norm = torch.ones(k, device=DEV).bfloat16()
+    delta = torch.randn(1, k, device=DEV).bfloat16()
+    kc, vc = (torch.zeros(1, 1, 16, d, device=DEV).bfloat16()
+              for _ in range(2))
+    at = torch.zeros(1, device=DEV, dtype=torch.int32)
+    cache = ops.Cache(at, kc, vc, at, 0.0)
+    for x in (torch.randn(2, 131, device=DEV).bfloat16()[:1, :k],
+              torch.randn(k, 1, device=DEV).bfloat16().t(),
+              torch.randn(k, device=DEV).bfloat16().as_strided((1, k), (3, 1))):
+        assert x.stride(0) % 8
+        close(ops.linear(x, w), x, w)
+        whole = x.clone(memory_format=torch.contiguous_format)
+        whole = whole.as_strided((1, k), (k, 1))
+        assert torch.equal(ops.linear_gated(x, w), ops.linear_gated(whole, w))
+        assert torch.equal(ops.linear_heads(x, w, None, cache),
+                           ops.linear_heads(whole, w, None, cache))
+        for a, b in zip(ops.linear_normed(delta, x, norm, 1e-5, w, None),
+                        ops.linear_normed(delta, whole, norm, 1e-5, w, None)):
+            assert torch.equal(a, b)
+
+
 def test_linear_keeps_gradients():
     w = torch.nn.Parameter(torch.randn(64, 128, device=DEV).bfloat16())
     x = torch.randn(3, 128, device=DEV).bfloat16()
