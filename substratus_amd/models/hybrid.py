@@ -26,7 +26,7 @@ import torch.nn as nn
 
 from ..ops import hybrid as ops, linear, linear_gated
 from ..parallel.comm import state
-from ..parallel.tp import Linear
+from ..parallel.tp import Linear, bare
 from ..serve.batch import StepBatch
 from .config import ModelConfig
 from .layers import (AttentionSpec, ConvAttentionSpec, DeltaSpec, GLASpec,
@@ -456,9 +456,10 @@ class HybridLayer(nn.Module):
     def feed_forward(self, y: torch.Tensor):
         if self.spec.moe:
             return self.experts(y)
-        h = linear_gated(y, self.w_gateup.weight)
+        lin = self.w_gateup
+        h = linear_gated(y, lin.weight, lin.bias) if bare(lin, Linear) else None
         if h is None:
-            h = ops.silu_mul(self.w_gateup(y))
+            h = ops.silu_mul(lin(y))
         return self.w_down(h)
 
 

@@ -29,7 +29,8 @@ import torch.nn.functional as F
 from .. import ops
 from ..ops import train as train_ops
 from ..parallel.comm import state
-from ..parallel.tp import ColumnParallelLinear, Linear, RowParallelLinear
+from ..parallel.tp import (ColumnParallelLinear, Linear, RowParallelLinear,
+                           bare)
 from .config import ModelConfig
 
 
@@ -46,9 +47,11 @@ def fused_norm_residual(deltas: tuple, h: torch.Tensor, norm: "NormParams",
     one HBM round trip per norm (profiles/serve_decode_r01_baseline.txt:
     unfused residual adds were ~2.2 ms of a 10.3 ms decode step). RMSNorm of
     one delta works in place on h."""
-    if norm.rms and len(deltas) == 1:
-        return ops.rms_norm_residual(deltas[0], h, norm.weight, eps)
-    got = train_ops.fused_add_norm(h, deltas, norm.weight, norm.bias, eps)
+    got = None
+    if bare(norm, NormParams):
+        if norm.rms and len(deltas) == 1:
+            return ops.rms_norm_residual(deltas[0], h, norm.weight, eps)
+        got = train_ops.fused_add_norm(h, deltas, norm.weight, norm.bias, eps)
     if got is None:
         for d in deltas:
             h = h + d
@@ -56,12 +59,29 @@ def fused_norm_residual(deltas: tuple, h: torch.Tensor, norm: "NormParams",
     return got
 
 
-def normed_product(lin: Linear, deltas: tuple, h: torch.Tensor,
+# Products with what follows them in one kernel: by methods of the module's own
+# class, since any module may stand where a projection was.
+
+def normed_product(lin: nn.Module, deltas: tuple, h: torch.Tensor,
                    norm: "NormParams", eps: float, **how):
     """(lin of norm(h + deltas), h + deltas) in one kernel, or None."""
-    if not norm.rms or len(deltas) != 1:
+    normed = getattr(type(lin), "normed", None)
+    if normed is None or len(deltas) != 1 or not bare(norm, NormParams) \
+            or not norm.rms:
         return None
-    return lin.normed(deltas[0], h, norm.weight, eps, **how)
+    return normed(lin, deltas[0], h, norm.weight, eps, **how)
+
+
+def heads_product(lin: nn.Module, y: torch.Tensor, cache: ops.Cache):
+    """ops.rope_kv_append of lin(y) in one kernel, or None."""
+    heads = getattr(type(lin), "heads", None)
+    return None if heads is None else heads(lin, y, cache)
+
+
+def gated_product(lin: nn.Module, y: torch.Tensor) -> torch.Tensor:
+    """ops.silu_mul(lin(y))"""
+    gated = getattr(type(lin), "gated", None)
+    return ops.silu_mul(lin(y)) if gated is None else gated(lin, y)
 
 
 class NormParams(nn.Module):
@@ -138,7 +158,7 @@ class Block(nn.Module):
 
     def _mlp_up(self, y: torch.Tensor) -> torch.Tensor:
         if self.cfg.activation == "silu":
-            return self.w_gateup.gated(y)
+            return gated_product(self.w_gateup, y)
         return ops.gelu(self.w_up(y))
 
     def _mlp(self, y: torch.Tensor) -> torch.Tensor:
@@ -168,7 +188,7 @@ class Block(nn.Module):
             q, h = got
         else:
             y, h = fused_norm_residual(deltas, h, self.norm1, self.eps)
-            q = self.wqkv.heads(y, cache)
+            q = heads_product(self.wqkv, y, cache)
             qkv = self.wqkv(y) if q is None else None
         yield
         if q is None:
@@ -349,6 +369,8 @@ class CausalLM(nn.Module):
         h = self.embed_tokens(tokens)
         if self.cfg.learned_pos_emb:
             h = h + self.embed_positions(positions.long())
+        elif not bare(self.embed_tokens, nn.Embedding):
+            h = h.clone()       # added to in place, and a hook may keep it
         max_len = ops.longest(seq_start) if h.is_cuda else None
         deltas = ()
         for blk, (kc, vc) in zip(self.blocks, kv_caches):

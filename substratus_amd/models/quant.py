@@ -20,6 +20,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from ..parallel.tp import bare
 from .gguf import (QK, QK_K, Q4_K_BLOCK_BYTES, Q6_K_BLOCK_BYTES,
                    QUANT_CODECS, _pack_scale_min_k4, _unpack_scale_min_k4,
                    dequantize_q4_0, dequantize_q8_0, quantize_q4_0,
@@ -195,7 +196,7 @@ class QuantLinear(nn.Module):
         """silu(first half of the outputs) * second half."""
         x2 = x.reshape(-1, self.in_features)
         ext = self._few_rows(x2, True) if self.bias is None and \
-            x.dtype == torch.bfloat16 else None
+            x.dtype == torch.bfloat16 and bare(self, QuantLinear) else None
         if ext is None:
             return ops.silu_mul(self(x))
         y = torch.empty(x2.shape[0], self.out_features // 2,
@@ -210,7 +211,8 @@ class QuantLinear(nn.Module):
         x2 = x.reshape(-1, self.in_features)
         n = self.out_features
         ext = self._few_rows(x2, True) if self.bias is None and \
-            x.dtype == torch.bfloat16 and cache.takes(x, n) else None
+            x.dtype == torch.bfloat16 and bare(self, QuantLinear) and \
+            cache.takes(x, n) else None
         if ext is None:
             return None
         q = x2.new_empty(*ops._columns(x2.shape[0], n, False, cache))
@@ -223,7 +225,8 @@ class QuantLinear(nn.Module):
                cache: Optional[ops.Cache] = None):
         """(the outputs for RMSNorm of h + delta, h + delta), gated or appended
         as above, in the same kernel, or None."""
-        if self.bias is not None or not ops.norm_goes_in(delta, h, norm):
+        if self.bias is not None or not bare(self, QuantLinear) or \
+                not ops.norm_goes_in(delta, h, norm):
             return None
         n = self.out_features
         ext = self._few_rows(h, gated or cache is not None)

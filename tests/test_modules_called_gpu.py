@@ -1,0 +1,146 @@
+"""A projection or norm that is more than its class's forward (hooks, a
+subclass, another module in its place) is called, not passed by for a kernel
+that reads its weights. Each here doubles what comes out, which doubled weights
+do as well."""
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+import torch.nn as nn
+
+from substratus_amd.models import CausalLM, get_config
+from substratus_amd.models.hybrid import HybridLayer
+from substratus_amd.models.quant import QuantLinear, quantize_model
+from substratus_amd.parallel.tp import Linear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+class Adapter(nn.Module):
+    """What it is not asked for itself, the module inside is."""
+
+    def __init__(self, inside):
+        super().__init__()
+        self.inside = inside
+
+    def forward(self, *a):
+        return 2 * self.inside(*a)
+
+    def __getattr__(self, name):
+        try:
+            return super().__getattr__(name)
+        except AttributeError:
+            return getattr(self.inside, name)
+
+
+def doubled(parent, name, how):
+    mod = getattr(parent, name)
+    kind = type(mod)
+    if how == "weights":
+        for t in ("weight", "scales", "bias"):
+            if getattr(mod, t, None) is not None:
+                getattr(mod, t).data.mul_(2)
+    elif how == "hook":
+        mod.register_forward_hook(lambda m, a, y: 2 * y)
+    elif how == "subclass":
+        mod.__class__ = type("Doubled", (kind,), {
+            "forward": lambda self, *a: 2 * kind.forward(self, *a)})
+    elif how == "instance":
+        mod.forward = lambda *a: 2 * kind.forward(mod, *a)
+    elif how == "adapter":
+        setattr(parent, name, Adapter(mod))
+
+
+def passes(name, how, quant, rows):
+    """Logits of a prompt and of a step after it."""
+    model = CausalLM(get_config("llama-tiny"), device=DEV,
+                     dtype=torch.bfloat16)
+    model.init_random(7)
+    if quant:
+        quantize_model(model, quant)
+    for parent in (model, *model.blocks):
+        if name in parent._modules:
+            doubled(parent, name, how)
+    hkv, d = model.n_kv_heads, model.cfg.head_dim
+    caches = [tuple(torch.zeros(rows, hkv, 16, d, device=DEV).bfloat16()
+                    for _ in range(2)) for _ in model.blocks]
+    n, at = 6, torch.arange(rows, device=DEV, dtype=torch.int32)
+    place = torch.arange(n, device=DEV, dtype=torch.int32)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    tokens = torch.randint(0, 512, (rows, n + 1), generator=g, device=DEV)
+    prompt = model.forward_prefill(
+        tokens[:, :n].reshape(-1), place.repeat(rows),
+        torch.arange(rows + 1, device=DEV, dtype=torch.int32) * n, caches,
+        (at[:, None] * 16 + place).reshape(-1))
+    step = model.forward_decode(
+        tokens[:, n], torch.full_like(at, n), caches, at * 16 + n,
+        at[:, None].contiguous(), torch.full_like(at, n + 1))
+    return prompt.double(), step.double()
+
+
+@pytest.mark.parametrize("quant", ["", "q4_0"])
+@pytest.mark.parametrize("how", ["hook", "subclass", "instance", "adapter"])
+@pytest.mark.parametrize("name", ["wqkv", "w_gateup", "lm_head", "norm2",
+                                  "final_norm"])
+@torch.no_grad()
+def test_called(name, how, quant):
+    if how == "adapter" and "norm" in name:
+        how = "hook"
+    for rows in (1, 5):
+        got = passes(name, how, quant, rows)
+        want = passes(name, "weights", quant, rows)
+        other = passes(name, "", quant, rows)
+        for a, b, c in zip(got, want, other):
+            # the same numbers, rounded to bf16 at some other places
+            assert float((a - b).norm()) <= 0.02 * float(b.norm())
+            assert float((a - c).norm()) > 0.1 * float(b.norm())
+
+
+@pytest.mark.parametrize("how", ["hook", "subclass", "instance", "adapter",
+                                 "quant"])
+@pytest.mark.parametrize("rows", [3, 40])
+@torch.no_grad()
+def test_unlike_layers(how, rows):
+    torch.manual_seed(rows)
+
+    def out(how):
+        torch.manual_seed(2)
+        layer = HybridLayer.__new__(HybridLayer)
+        nn.Module.__init__(layer)
+        layer.spec = SimpleNamespace(moe=None)
+        layer.w_gateup, layer.w_down = (
+            Linear(a, b, bias=True, device=DEV, dtype=torch.bfloat16)
+            for a, b in ((128, 256), (128, 128)))
+        for p in layer.parameters():
+            p.normal_(0, 0.2)
+        if how == "quant":
+            layer.w_gateup = QuantLinear.from_linear(layer.w_gateup, "q8_0")
+        else:
+            doubled(layer, "w_gateup", how)
+        return layer.feed_forward(x).double()
+
+    x = torch.randn(rows, 128, device=DEV).bfloat16()
+    got = out(how)
+    want = out("" if how == "quant" else "weights")
+    assert float((got - want).norm()) <= 0.02 * float(want.norm())
+
+
+@torch.no_grad()
+def test_embeddings_kept_by_a_hook():
+    """A prompt's residual stream is added up in place, in its own tensor."""
+    model = CausalLM(get_config("llama-tiny"), device=DEV,
+                     dtype=torch.bfloat16)
+    model.init_random(7)
+    kept = []
+    model.embed_tokens.register_forward_hook(
+        lambda m, a, y: kept.append(y))
+    cache = [tuple(torch.zeros(1, model.n_kv_heads, 16, 64,
+                               device=DEV).bfloat16() for _ in range(2))
+             for _ in model.blocks]
+    tokens = torch.arange(8, device=DEV)
+    at = torch.arange(8, device=DEV, dtype=torch.int32)
+    model.forward_prefill(tokens, at, torch.tensor([0, 8], device=DEV).int(),
+                          cache, at)
+    assert torch.equal(kept[0], model.embed_tokens.weight[tokens])
