@@ -13,6 +13,8 @@ import os
 from typing import NamedTuple, Optional
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import ref
 
@@ -229,17 +231,37 @@ def flash_attn_train_available(d: int) -> bool:
 _GEMM_WS: dict = {}
 
 
+# called for every product of a step: names looked up once
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+_STRIDED = torch.strided
+_batched = torch._C._functorch.is_legacy_batchedtensor
+_transforms = torch._C._are_functorch_transforms_active
+_tracing_state = torch._C._get_tracing_state
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_functions = torch._C._len_torch_function_stack
+_autocast = torch.is_autocast_enabled
+_compiling = torch.compiler.is_compiling
+_forward_ad = torch.autograd.forward_ad
+
+
+def _function_modes() -> bool:
+    """Whether a mode is to see calls of torch's functions (other than a device
+    for new tensors)."""
+    return any(type(m) is not DeviceContext
+               for m in _get_current_function_mode_stack())
+
+
 def plain_tensors(*tensors: Optional[torch.Tensor]) -> bool:
-    """No transform, trace, autocast or dispatch mode that expects torch's own
-    ops, no tensor subclass."""
-    if any(type(t) not in (torch.Tensor, torch.nn.Parameter)
-           for t in tensors if t is not None):
-        return False
-    return not (torch.is_autocast_enabled("cuda")
-                or torch.compiler.is_compiling()
-                or torch._C._are_functorch_transforms_active()
-                or torch._C._len_torch_dispatch_stack()
-                or torch.autograd.forward_ad._current_level >= 0)
+    """No transform, trace, autocast, function or dispatch mode that expects
+    torch's own ops, no tensor subclass, batch of tensors or sparse layout."""
+    for t in tensors:
+        if t is not None and (type(t) not in _TENSORS
+                              or t.layout is not _STRIDED or _batched(t)):
+            return False
+    return not (_compiling() or _autocast("cuda")
+                or _tracing_state() is not None or _transforms()
+                or _dispatch_modes() or _functions() and _function_modes()
+                or _forward_ad._current_level >= 0)
 
 
 def inference_only(*tensors: torch.Tensor) -> bool:
@@ -332,7 +354,7 @@ class _Linear(torch.autograd.Function):
         x, weight = ctx.saved_tensors
         dx = dw = db = None
         # gradients that can be differentiated again are torch's
-        own = not torch.is_grad_enabled()
+        own = not torch.is_grad_enabled() and plain_tensors(dy, x, weight)
         if own and ctx.needs_input_grad[0]:
             dx = _tile_gemm(dy, weight, b_flipped=True)
         if own and ctx.needs_input_grad[1]:
@@ -390,6 +412,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
     1.0-2.25 — the library's measured rates reach the ceiling measured for a
     deep-pipelined schedule on this chip (~1.33-1.47 PF). The kernel stays for
     measurement and as the base for a future counted-vmcnt schedule."""
+    if not isinstance(x, torch.Tensor):         # a symbolic trace's stand-in
+        return torch.nn.functional.linear(x, weight, bias)
     few = _few_rows(x, weight, bias, False)
     if few is not None:
         rows, ext = few

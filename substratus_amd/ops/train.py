@@ -4,7 +4,8 @@ follows, attention from the fused projection on, the gated activation.
 Each op has a general form in torch's own ops, which every device, type and
 transform gets, and a form on train_rows.hip's kernels for what a bf16 step on
 the GPU calls. Both give gradients that can be differentiated again: where a
-graph of the gradients is asked for, the backward is the general form's.
+graph of the gradients is asked for, or a transform runs, the backward is the
+general form's.
 """
 
 from __future__ import annotations
@@ -31,6 +32,11 @@ def _again(form: Callable, inputs: Sequence, dy: torch.Tensor) -> list:
                 for t in at]
 
 
+def _values_only(*grads: Optional[torch.Tensor]) -> bool:
+    """Whether a backward may take its kernels for these."""
+    return not torch.is_grad_enabled() and plain_tensors(*grads)
+
+
 def _whole(*tensors: Optional[torch.Tensor]) -> bool:
     """Contiguous bf16 on one GPU and 16-byte boundaries, as the kernels read
     them."""
@@ -52,7 +58,7 @@ class _Lookup(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         tokens, weight = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if not _values_only(dy):
             return None, _again(lambda w: F.embedding(tokens, w), (weight,),
                                 dy)[0]
         dw = torch.zeros_like(weight)
@@ -120,7 +126,7 @@ class _AddNorm(torch.autograd.Function):
         x, stats, weight, bias = ctx.saved_tensors
         if dy is None:
             return None, None, None, *[dsum] * (1 + ctx.n)
-        if torch.is_grad_enabled():
+        if not _values_only(dy, dsum):
             dw, db, dh = _again(
                 lambda w, b, x: _norm(x, w, b, ctx.eps), (weight, bias, x),
                 dy)
@@ -274,7 +280,7 @@ class _SiluMul(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         gu, = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if not _values_only(dy):
             return _again(_silu_mul, (gu,), dy)[0]
         dx = torch.empty_like(gu)
         _load_ext().silu_mul_bwd(dx, _aligned(dy), gu)
