@@ -254,11 +254,13 @@ def _function_modes() -> bool:
 def plain_tensors(*tensors: Optional[torch.Tensor]) -> bool:
     """No transform, trace, autocast, function or dispatch mode that expects
     torch's own ops, no tensor subclass, batch of tensors or sparse layout."""
+    if _compiling():        # first: a compiler does not know the others
+        return False
     for t in tensors:
         if t is not None and (type(t) not in _TENSORS
                               or t.layout is not _STRIDED or _batched(t)):
             return False
-    return not (_compiling() or _autocast("cuda")
+    return not (_autocast("cuda")
                 or _tracing_state() is not None or _transforms()
                 or _dispatch_modes() or _functions() and _function_modes()
                 or _forward_ad._current_level >= 0)
@@ -375,7 +377,8 @@ def _many_rows(x: torch.Tensor, weight: torch.Tensor,
     linear_gated makes of it, without gradients."""
     if not (x.is_cuda and weight.dim() == 2 and weight.shape[0] >= 256
             and x.dim() >= 2 and x.shape[-1] == weight.shape[1] > 0
-            and x.numel() >= 256 * x.shape[-1] and _load_ext() is not None):
+            and x.numel() >= 256 * x.shape[-1] and not _compiling()
+            and _load_ext() is not None):
         return None
     # sizes first, which cost a microsecond: a step of a few hundred rows has
     # dozens of products that stay with torch's

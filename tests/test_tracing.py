@@ -62,6 +62,19 @@ def test_symbolic_trace():
     assert torch.equal(graph(x), lin(x))
 
 
+def test_compiled():
+    """As one graph, without a break."""
+    w = torch.randn(16, 32)
+
+    def fn(x):
+        assert not ops.plain_tensors(x, w)
+        return train.silu_mul(ops.linear(x, w))
+    x = torch.randn(3, 32)
+    want = train.silu_mul(ops.linear(x, w))
+    got = torch.compile(fn, backend="eager", fullgraph=True)(x)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,k", [(3, 2048), (40, 2048), (1024, 11008)])
 @torch.no_grad()
@@ -77,6 +90,10 @@ def test_traced_products(rows, k):
     with Seen() as mode:
         lin(x)
     assert F.linear in mode.calls
+    compiled = torch.compile(lambda t: lin(t), backend="eager",
+                             fullgraph=True)
+    assert float((compiled(other).double() - want).norm()) <= \
+        2.0 ** -8 * float(want.norm())
 
 
 @pytest.mark.gpu
