@@ -204,6 +204,10 @@ class _FlashAttnTrain(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out, lse, seq_start = ctx.saved_tensors
+        if torch.is_grad_enabled() or not plain_tensors(dout):
+            from .train import attention_again
+            return *attention_again(q, k, v, dout, ctx.max_len,
+                                    ctx.scale), None, None, None
         dq, dk32, dv32 = _flash_bwd(q, k, v, out, dout.contiguous(), lse,
                                     seq_start, ctx.max_len, ctx.scale)
         return dq, dk32.to(k.dtype), dv32.to(v.dtype), None, None, None
@@ -217,8 +221,8 @@ def flash_attn_train(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     seq_start = torch.arange(0, (b + 1) * s, s, dtype=torch.int32,
                              device=q.device)
     out = _FlashAttnTrain.apply(
-        q.reshape(b * s, hq, d), k.reshape(b * s, k.shape[2], d),
-        v.reshape(b * s, v.shape[2], d), seq_start, s, scale)
+        *(t.reshape(b * s, -1, d).contiguous() for t in (q, k, v)),
+        seq_start, s, scale)
     return out.view(b, s, hq, d)
 
 

@@ -210,12 +210,35 @@ def _attend(qkv, cos, sin, hq: int, hkv: int, scale: float) -> torch.Tensor:
     return a.transpose(1, 2).reshape(b, s, hq * d)
 
 
+def _attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, s: int,
+               scale: float) -> torch.Tensor:
+    """Causal attention of sequences of s rows, rows of heads to rows of
+    heads, in 32-bit steps that can be differentiated any number of times."""
+    hq, d = q.shape[1:]
+    q32, k32, v32 = (
+        t.view(-1, s, *t.shape[1:]).transpose(1, 2).float()
+        .repeat_interleave(hq // t.shape[1], dim=1) for t in (q, k, v))
+    scores = q32 @ k32.transpose(2, 3).contiguous() * scale
+    later = torch.ones(s, s, dtype=torch.bool, device=q.device).triu(1)
+    a = scores.masked_fill(later, -torch.inf).softmax(-1) @ v32
+    return a.transpose(1, 2).reshape(-1, hq, d).to(q.dtype)
+
+
+def attention_again(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                    dout: torch.Tensor, s: int, scale: float) -> list:
+    """Gradients of attention as a part of the graph."""
+    return _again(lambda *t: _attention(*t, s, scale), (q, k, v),
+                  dout.reshape(q.shape))
+
+
 class _Attend(torch.autograd.Function):
     """From rows of a fused projection to rows of heads: split and rotation in
-    one kernel either way around the attention's own."""
+    one kernel either way around the attention's own. Split rows are outputs as
+    well, which nobody else sees: so they are kept as a part of the graph."""
 
     @staticmethod
     def forward(ctx, qkv, cos, sin, hq, hkv, scale):
+        ctx.set_materialize_grads(False)
         b, s, width = qkv.shape
         d = width // (hq + 2 * hkv)
         q = qkv.new_empty(b * s, hq, d)
@@ -226,18 +249,27 @@ class _Attend(torch.autograd.Function):
         out, lse = _flash_fwd(q, k, v, seq_start, s, scale)
         ctx.save_for_backward(q, k, v, out, lse, seq_start, cos, sin)
         ctx.scale, ctx.shape = scale, qkv.shape
-        return out.view(b, s, hq * d)
+        return out.view(b, s, hq * d), q, k, v
 
     @staticmethod
-    def backward(ctx, dout):
-        # like flash_attn_train's, a constant where a graph is asked for
+    def backward(ctx, dout, *dsplit):
         q, k, v, out, lse, seq_start, cos, sin = ctx.saved_tensors
-        s = ctx.shape[1]
-        dq, dk, dv = _flash_bwd(q, k, v, out, _aligned(dout).view_as(out),
-                                lse, seq_start, s, ctx.scale)
-        dqkv = q.new_empty(ctx.shape)
-        _load_ext().rope_join(dqkv, dq, dk, dv, cos, sin, s)
-        return dqkv, None, None, None, None, None
+        b, s, width = ctx.shape
+        if dout is not None and _values_only(dout) and not any(
+                t is not None for t in dsplit):
+            dq, dk, dv = _flash_bwd(q, k, v, out, _aligned(dout).view_as(out),
+                                    lse, seq_start, s, ctx.scale)
+            dqkv = q.new_empty(ctx.shape)
+            _load_ext().rope_join(dqkv, dq, dk, dv, cos, sin, s)
+            return dqkv, None, None, None, None, None
+        parts = [torch.zeros_like(t) for t in (q, k, v)] if dout is None \
+            else attention_again(q, k, v, dout, s, ctx.scale)
+        parts = [(t if g is None else t + g).view(b, s, -1, q.shape[2])
+                 for t, g in zip(parts, dsplit)]
+        if cos is not None:         # turned back
+            parts[:2] = (rope(t, cos, -sin, bshd=True) for t in parts[:2])
+        return torch.cat([t.reshape(b, s, -1) for t in parts], -1), \
+            None, None, None, None, None
 
 
 def _angles(t: Optional[torch.Tensor], s: int, d: int,
@@ -258,7 +290,7 @@ def attend(qkv: torch.Tensor, cos: Optional[torch.Tensor],
                     for t in (cos, sin))
             and plain_tensors(qkv, cos, sin)
             and flash_attn_train_available(d)):
-        return _Attend.apply(qkv, cos, sin, hq, hkv, scale)
+        return _Attend.apply(qkv, cos, sin, hq, hkv, scale)[0]
     return _attend(qkv, cos, sin, hq, hkv, scale)
 
 

@@ -133,5 +133,5 @@ def test_batches_of_gradients():
         for i in range(2):
             one = torch.autograd.grad(out, given, dy[i], retain_graph=True)
             for a, c in zip(got, one):
-                a, c = a[i].double(), c.double()
+                a, c = a[i].detach().double(), c.detach().double()
                 assert float((a - c).norm()) <= 0.01 * float(c.norm())

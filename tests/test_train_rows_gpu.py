@@ -105,6 +105,58 @@ def test_attend(b, s, hq, hkv, d, turned):
         assert off <= 1.02 * most + 2.0 ** -12
 
 
+@pytest.mark.parametrize("b,s,hq,hkv,d", [(2, 33, 4, 1, 64),
+                                          (1, 20, 2, 2, 128)])
+@pytest.mark.parametrize("turned", [True, False])
+@pytest.mark.parametrize("fused", [True, False])
+def test_attend_again(b, s, hq, hkv, d, turned, fused):
+    """Gradients of gradients, and batches of gradients, of the attention and
+    of what is around it."""
+    qkv = rand(b, s, (hq + 2 * hkv) * d).requires_grad_()
+    dout = rand(b, s, hq * d, seed=1).requires_grad_()
+    cos = sin = None
+    if turned:
+        a = torch.arange(s, device=DEV)[:, None] * 0.9 ** torch.arange(
+            d // 2, device=DEV)
+        cos, sin = a.cos(), a.sin()
+    form = train.attend if fused else train._attend
+
+    def twice(form, qkv, dout, cos, sin):
+        out = form(qkv, cos, sin, hq, hkv, d ** -0.5)
+        one, = torch.autograd.grad(out, qkv, dout, create_graph=True)
+        weigh = torch.linspace(-1, 1, one.numel(), device=one.device)
+        return one, *torch.autograd.grad(
+            (one * weigh.view_as(one).to(one.dtype)).float().square().sum(),
+            (qkv, dout))
+
+    def exact(qkv, cos, sin, hq, hkv, scale):
+        q, k, v = (t.view(b, s, -1, d).transpose(1, 2) for t in qkv.split(
+            [hq * d, hkv * d, hkv * d], -1))
+        if cos is not None:
+            q, k = train.rope(q, cos, sin), train.rope(k, cos, sin)
+        k, v = (t.repeat_interleave(hq // hkv, 1) for t in (k, v))
+        later = torch.ones(s, s, dtype=torch.bool).triu(1)
+        a = (q @ k.mT * scale).masked_fill(later, -torch.inf).softmax(-1) @ v
+        return a.transpose(1, 2).reshape(b, s, hq * d)
+
+    got = twice(form, qkv, dout, cos, sin)
+    want = twice(exact, *(t if t is None else
+                          t.detach().double().cpu().requires_grad_(
+                              t.requires_grad)
+                          for t in (qkv, dout, cos, sin)))
+    for g, w in zip(got, want):     # bf16 between the steps
+        g, w = g.detach().double().cpu(), w.detach()
+        assert float((g - w).norm()) <= 0.03 * float(w.norm())
+    out = form(qkv, cos, sin, hq, hkv, d ** -0.5)
+    many = torch.stack([dout.detach(), 2 * dout.detach()])
+    both, = torch.autograd.grad(out, qkv, many, is_grads_batched=True,
+                                retain_graph=True)
+    alone, = torch.autograd.grad(out, qkv, dout)
+    for i in range(2):
+        assert float((both[i].float() - (i + 1) * alone.float()).norm()) <= \
+            0.02 * float((i + 1) * alone.float().norm())
+
+
 @pytest.mark.parametrize("rows,f", [(1, 8), (3, 2056), (700, 5632)])
 def test_silu_mul(rows, f):
     x = (4 * rand(rows, 2 * f)).detach().requires_grad_()
