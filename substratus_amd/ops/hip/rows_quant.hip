@@ -12,12 +12,15 @@
 //                bits, an int8 scale per 16
 //
 // Bound by reading packed weights and by unpacking them. Unpacked they are
-// whole numbers, which bf16 holds exactly: 16 + nibble (or 64 + six bits, or
-// 128 + byte) takes one and-or of a shifted word, and the matrix cores
-// multiply it with x. The offset is taken off inside: a product of x with a
-// constant gives -offset * sum(x), where the weights' product begins, and with
-// minima those sums are needed anyway. One instruction's inner size is one
-// block, so its sum is scaled in 32 bits and added up, as in a loop over
+// whole numbers, which bf16 holds exactly, and the matrix cores multiply them
+// with x as they are, so that a block's 32-bit sum holds nothing that is taken
+// off again (an offset, which is cheap to unpack with, would cost its last bits
+// where x is large, and make an infinite x no number). Four bits are bytes that
+// count as small 8-bit floating-point numbers, of which one operation converts
+// two; six bits go to the top of their bytes, which are then 4 times the number
+// with a sign, and are converted like eight bits one by one. Minima need the
+// sums of x, which a product with ones gives. One instruction's inner size is
+// one block, so its sum is scaled in 32 bits and added up, as in a loop over
 // blocks in 32-bit arithmetic.
 //
 // A workgroup takes 16 weight rows and MR rows of x; its waves share k. A
@@ -29,17 +32,20 @@
 // us on a MI355X, 15360 x 5120, 5120 x 5120, 27648 x 5120, 5120 x 13824, from
 // one wave per weight row in vector arithmetic (up to 8 rows of x), or from
 // unpacking to bf16 in memory and the library (more), to this kernel:
-//   q4_0  1 row   20.5  8.5 31.7 15.0 -> 12.7  7.0 21.8 14.4
-//         5 rows  55.0 21.5 95.3 47.8 -> 13.7  7.9 22.6 16.3
-//        24 rows  81.4 37.8  152 75.9 -> 28.1 15.3 45.8 33.4
-//   q8_0  5 rows  55.9 21.2 97.5 46.3 -> 23.7 12.7 38.3 26.6
-//        24 rows  82.5 38.8  155 78.9 -> 42.1 20.8 70.2 43.5
-//   q4_K  1 row   29.4 12.9 49.4 24.6 -> 13.6  7.6 22.9 17.0
-//         5 rows   115 47.7  196  111 -> 16.3  8.8 26.6 19.9
-//        24 rows  90.1 37.8  172 84.6 -> 30.7 16.8 50.2 39.9
-//   q6_K  1 row   32.7 13.3 57.5 26.8 -> 21.4 11.6 31.9 26.6
-//         5 rows   118 40.9  205 90.9 -> 23.4 13.0 34.4 29.1
-//        24 rows   523  196  946  479 -> 38.4 19.5 64.8 46.9
+//   q4_0  1 row   20.5  8.5 31.7 15.0 -> 12.9  7.2 20.9 15.3
+//         5 rows  55.0 21.5 95.3 47.8 -> 14.1  7.7 22.9 16.9
+//        24 rows  81.4 37.8  152 75.9 -> 23.5 12.5 38.7 26.5
+//   q8_0  5 rows  55.9 21.2 97.5 46.3 -> 22.2 11.9 36.0 25.7
+//        24 rows  82.5 38.8  155 78.9 -> 40.6 20.7 69.9 43.6
+//   q4_K  1 row   29.4 12.9 49.4 24.6 -> 12.8  7.3 21.4 16.1
+//         5 rows   115 47.7  196  111 -> 15.5  8.6 24.8 18.6
+//        24 rows  90.1 37.8  172 84.6 -> 25.9 15.1 43.2 31.4
+//   q6_K  1 row   32.7 13.3 57.5 26.8 -> 20.6 11.0 29.9 25.8
+//         5 rows   118 40.9  205 90.9 -> 22.4 12.1 31.4 28.6
+//        24 rows   523  196  946  479 -> 35.7 18.8 51.9 44.1
+// (4-bit numbers with an offset of 24 or 16, which one operation unpacked, took
+// 12.6 7.0 20.4 14.4 and 13.3 7.4 22.2 16.6 for one row, 27.5 14.1 50.0 33.3
+// and 28.5 14.3 51.2 35.7 for 24.)
 // q8_0 with one row stays with the vector kernel (quant_gemv.hip): 20.5, 9.4,
 // 33.1, 19.3 there and 19.9, 11.1, 32.2, 23.8 here.
 #include "rows_quant.h"
@@ -70,36 +76,18 @@ DEV_INLINE float byte_at(const uint4v& u, int i) {
   return (float)((u[i >> 2] >> (8 * (i & 3))) & 0xff);
 }
 
-// Two 16-bit halves out of two words: the low ones, the high ones.
-DEV_INLINE unsigned low2(unsigned a, unsigned b) {
-  return __builtin_amdgcn_perm(b, a, 0x05040100);
-}
+// The high halves of two words.
 DEV_INLINE unsigned high2(unsigned a, unsigned b) {
   return __builtin_amdgcn_perm(b, a, 0x07060302);
 }
 
-// 16 + nibbles at bits 3 to 6 of eight bytes, as bf16. c16: two bf16 of 16.
-DEV_INLINE short8 unpack4(unsigned a, unsigned b, unsigned c16) {
-  auto two = [&](unsigned v, unsigned sel) {
-    return (__builtin_amdgcn_perm(v, v, sel) & 0x780078u) | c16;
-  };
-  return vec8(two(a, 0x0c010c00), two(a, 0x0c030c02), two(b, 0x0c010c00),
-              two(b, 0x0c030c02));
-}
-
-// 128 + eight signed bytes, as bf16: whole numbers below 256 are exact.
-DEV_INLINE short8 unpack8(const uint2v& v) {
-  unsigned o[4];
+// Four signed bytes as bf16, which holds whole numbers up to 256.
+DEV_INLINE uint2v unpack4(unsigned v) {
+  float f[4];
   #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const unsigned z = v[h] ^ 0x80808080u;
-    float f[4];
-    #pragma unroll
-    for (int i = 0; i < 4; ++i) f[i] = (float)((z >> (8 * i)) & 0xff);
-    o[h * 2] = high2(__float_as_uint(f[0]), __float_as_uint(f[1]));
-    o[h * 2 + 1] = high2(__float_as_uint(f[2]), __float_as_uint(f[3]));
-  }
-  return vec8(o[0], o[1], o[2], o[3]);
+  for (int i = 0; i < 4; ++i) f[i] = (float)(signed char)(v >> (8 * i) & 0xff);
+  return {high2(__float_as_uint(f[0]), __float_as_uint(f[1])),
+          high2(__float_as_uint(f[2]), __float_as_uint(f[3]))};
 }
 
 template <int ME>
@@ -108,24 +96,55 @@ DEV_INLINE void add_scaled(float4v& a, float s, const float4v& v) {
   for (int e = 0; e < ME; ++e) a[e] += s * v[e];
 }
 
+// Four numbers of 4 exponent and 3 mantissa bits as 512 times what they are, in
+// bf16: one operation converts two. As such numbers bytes below 16 are 0 to 15
+// times 2^-9.
+DEV_INLINE uint2v unpack_small(unsigned v) {
+  return {__builtin_bit_cast(
+              unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.f,
+                                                                  false)),
+          __builtin_bit_cast(
+              unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.f,
+                                                                  true))};
+}
+
+// Bytes n below 16 as such numbers of n - 8: 0x88 - n or n - 8. A selector of
+// 8 and more gives 0 or 255, by the table's own signs below 12, so each half of
+// the table undoes what the other one gives there.
+DEV_INLINE unsigned minus8(unsigned n) {
+  return __builtin_amdgcn_perm(0x7E7D7C84u, 0x7A798788u, n) ^
+         __builtin_amdgcn_perm(0xF8F9FA04u, 0x030201FFu, n ^ 0x08080808u);
+}
+
+// One result by weights and not by their two parts, whose sums are infinite
+// with opposite signs where x is.
+DEV_INLINE float dot_q4k(const bf16_t* x, const unsigned char* row,
+                         const f16_t* d, int k) {
+  float s = 0.f;
+  for (int i = 0; i < k; ++i) {
+    const unsigned b = row[k / 16 + i / 64 * 32 + i % 32];
+    const float w = (float)d[i / 256 * 2] * (float)row[i / 32] *
+                        (float)(i & 32 ? b >> 4 : b & 15) -
+                    (float)d[i / 256 * 2 + 1] * (float)row[k / 32 + i / 32];
+    s += w * bf2f(x[i]);
+  }
+  return s;
+}
+
 // Tiles of 16 rows x 64 bytes in a stage, 16-byte scale rows, loads of both;
-// two bf16 of minus the offset of unpacked weights.
+// how many times the number unpacked weights are.
 template <Quant Q> struct Layout;
 template <> struct Layout<Quant::Q4_0> {
-  static constexpr int W = 2, S = 1, LOADS = 3;
-  static constexpr unsigned OFF = 0xC1C0C1C0u;        // -24
+  static constexpr int W = 2, S = 1, LOADS = 3, TIMES = 1;
 };
 template <> struct Layout<Quant::Q8_0> {
-  static constexpr int W = 4, S = 1, LOADS = 5;
-  static constexpr unsigned OFF = 0xC300C300u;        // -128
+  static constexpr int W = 4, S = 1, LOADS = 5, TIMES = 1;
 };
 template <> struct Layout<Quant::Q4_K> {
-  static constexpr int W = 2, S = 2, LOADS = 4;
-  static constexpr unsigned OFF = 0xC180C180u;        // -16
+  static constexpr int W = 2, S = 2, LOADS = 4, TIMES = 1;
 };
 template <> struct Layout<Quant::Q6_K> {
-  static constexpr int W = 3, S = 1, LOADS = 5;       // one to a register
-  static constexpr unsigned OFF = 0xC2C0C2C0u;        // -96
+  static constexpr int W = 3, S = 1, LOADS = 5, TIMES = 4;   // one to a register
 };
 
 // MR: rows of x; ME: of every four, those that are there (MR 4 only); KW
@@ -223,14 +242,10 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     }
   };
 
-  unsigned c16 = 0x41804180u, c64 = 0x42804280u;
-  asm("" : "+v"(c16));       // in registers: an and-or has room for one literal
-  asm("" : "+v"(c64));
-  const short8 off = vec8(L::OFF, L::OFF, L::OFF, L::OFF);
+  const short8 ones = vec8(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
   const float4v zero = {0.f, 0.f, 0.f, 0.f};
-  // q4_0: lanes of the first 16 weights take low nibbles, the others high
-  // ones; rotated right by this they are at bits 3 to 6 of their bytes
-  const int turn = g >> 1 ? 1 : 29;
+  // q4_0: lanes of the first 16 weights take low nibbles, the others high ones
+  const int down = g >> 1 ? 4 : 0;
   int xr[FM];                                    // the lane's rows of x
   #pragma unroll
   for (int j = 0; j < FM; ++j) {
@@ -253,85 +268,89 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     float d = 0.f, dm = 0.f;
     if constexpr (Q == Quant::Q4_K) {
       const unsigned dd = reinterpret_cast<const unsigned*>(ss + 16)[lo];
-      d = half_of(dd);
-      dm = half_of(dd >> 16) * 0.0625f;          // sums of x come times -16
+      d = half_of(dd) / L::TIMES;
+      dm = -half_of(dd >> 16);
     }
-    if constexpr (Q == Quant::Q6_K) d = half_of(dreg[s]);
+    if constexpr (Q == Quant::Q6_K) d = half_of(dreg[s]) / L::TIMES;
+    // the lane's eight weights of a block, k = 8 g on, out of eight bytes
+    auto weights = [&](int b) {
+      const int at = Q == Quant::Q4_0 ? b & 3
+          : Q == Quant::Q8_0 ? (b & 1) * 2 + (g >> 1)
+                             : ((b >> 1) & 1) * 2 + (g >> 1);
+      const uint2v v = reinterpret_cast<const uint2v*>(
+          ws + (Q == Quant::Q8_0 ? b >> 1 : b >> 2) * TILE +
+          (at ^ wsw))[g & 1];
+      uint2v w[2];
+      #pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if constexpr (Q == Quant::Q4_0)
+          w[h] = unpack_small(minus8(v[h] >> down & 0x0F0F0F0Fu));
+        else if constexpr (Q == Quant::Q8_0)
+          w[h] = unpack4(v[h]);
+        else
+          w[h] = unpack_small((b & 1 ? v[h] >> 4 : v[h]) & 0x0F0F0F0Fu);
+      }
+      return vec8(w[0][0], w[0][1], w[1][0], w[1][1]);
+    };
     #pragma unroll
     for (int b = 0; b < COLS / 32; ++b) {
       if (!decltype(whole)::value && c * 8 + b >= nb) break;
       if constexpr (Q != Quant::Q6_K) {
-        // eight bytes with the lane's eight weights, k = 8 g on
-        const int at = Q == Quant::Q4_0 ? b & 3
-            : Q == Quant::Q8_0 ? (b & 1) * 2 + (g >> 1)
-                               : ((b >> 1) & 1) * 2 + (g >> 1);
-        const uint2v v = reinterpret_cast<const uint2v*>(
-            ws + (Q == Quant::Q8_0 ? b >> 1 : b >> 2) * TILE +
-            (at ^ wsw))[g & 1];
-        short8 wv;
-        if constexpr (Q == Quant::Q4_0)
-          wv = unpack4(__builtin_amdgcn_alignbit(v[0], v[0], turn),
-                       __builtin_amdgcn_alignbit(v[1], v[1], turn), c16);
-        else if constexpr (Q == Quant::Q8_0)
-          wv = unpack8(v);
-        else
-          wv = b & 1 ? unpack4(v[0] >> 1, v[1] >> 1, c16)
-                     : unpack4(v[0] << 3, v[1] << 3, c16);
-        const float scale = Q == Quant::Q4_K ? d * byte_at(sv, b)
-                                             : half_at(sv, b);
+        // two blocks at a time: the second's work is done while the first's
+        // products are on their way
+        if (b & 1) continue;
+        const short8 wv[2] = {weights(b), weights(b + 1)};
         #pragma unroll
         for (int j = 0; j < FM; ++j) {
-          const short8 xv = __builtin_bit_cast(
-              short8, NORM ? x_row[c * 32 + b * 4 + g]
-                           : xs[xr[j] + (b >> 2) * 64 +
-                                (((b * 4 + g) & 15) ^ xsw)]);
-          const float4v sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              xv, off, zero, 0, 0, 0);
-          add_scaled<ME>(acc[j], scale,
-                         __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                             xv, wv, sum, 0, 0, 0));
-          if constexpr (Q == Quant::Q4_K)
-            add_scaled<ME>(acc[j], dm * byte_at(sv, 8 + b), sum);
+          float4v p[2], sums[2];
+          #pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const short8 xv = __builtin_bit_cast(
+                short8, NORM ? x_row[c * 32 + (b + t) * 4 + g]
+                             : xs[xr[j] + (b >> 2) * 64 +
+                                  ((((b + t) * 4 + g) & 15) ^ xsw)]);
+            p[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, wv[t], zero, 0,
+                                                           0, 0);
+            if constexpr (Q == Quant::Q4_K)
+              sums[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  xv, ones, zero, 0, 0, 0);
+          }
+          #pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            add_scaled<ME>(acc[j], Q == Quant::Q4_K ? d * byte_at(sv, b + t)
+                                                    : half_at(sv, b + t),
+                           p[t]);
+            if constexpr (Q == Quant::Q4_K)
+              add_scaled<ME>(acc[j], dm * byte_at(sv, 8 + b + t), sums[t]);
+          }
         }
       } else {
-        // a scale per 16 weights: instructions of inner size 16, even and odd
-        // bytes in turn
+        // a scale per 16 weights: instructions of inner size 16
         const int hf = b >> 2, quarter = b & 3;
-        const uint2v off4 = {L::OFF, L::OFF};
-        const short4v o4 = __builtin_bit_cast(short4v, off4);
         #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const unsigned v = reinterpret_cast<const unsigned*>(
               ws + hf * TILE + (((quarter & 1) * 2 + h) ^ wsw))[g];
           const unsigned hv = reinterpret_cast<const unsigned*>(
               ws + 2 * TILE + ((hf * 2 + h) ^ wsw))[g];
-          unsigned o[2];
-          #pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const unsigned low = quarter < 2 ? (e ? v >> 7 : v << 1)
-                                             : (e ? v >> 11 : v >> 3);
-            const int up = 5 - 2 * quarter - 8 * e;
-            const unsigned high = up >= 0 ? hv << up : hv >> -up;
-            o[e] = ((low & 0x1E001Eu) | c64) | (high & 0x600060u);
-          }
-          const uint2v o2 = {o[0], o[1]};
-          const short4v wv = __builtin_bit_cast(short4v, o2);
+          const unsigned low = (quarter < 2 ? v << 2 : v >> 2) & 0x3C3C3C3Cu;
+          const unsigned high = hv << (6 - 2 * quarter) & 0xC0C0C0C0u;
+          const short4v wv = __builtin_bit_cast(
+              short4v, unpack4((low | high) ^ 0x80808080u));
           const int si = hf * 8 + quarter * 2 + h;
           const float scale = d * (float)(signed char)(
               (sv[si >> 2] >> (8 * (si & 3))) & 0xff);
           #pragma unroll
           for (int j = 0; j < FM; ++j) {
             const int p = b * 4 + h * 2 + (g >> 1);
-            const uint2v xw = reinterpret_cast<const uint2v*>(
-                NORM ? x_row + c * 32 + p
-                     : xs + xr[j] + (p >> 4) * 64 + ((p & 15) ^ xsw))[g & 1];
-            const uint2v xe = {low2(xw[0], xw[1]), high2(xw[0], xw[1])};
-            const short4v xv = __builtin_bit_cast(short4v, xe);
-            const float4v sum = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                xv, o4, zero, 0, 0, 0);
+            const short4v xv = __builtin_bit_cast(
+                short4v, reinterpret_cast<const uint2v*>(
+                    NORM ? x_row + c * 32 + p
+                         : xs + xr[j] + (p >> 4) * 64 +
+                               ((p & 15) ^ xsw))[g & 1]);
             add_scaled<ME>(acc[j], scale,
                            __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                               xv, wv, sum, 0, 0, 0));
+                               xv, wv, zero, 0, 0, 0));
           }
         }
       }
@@ -396,6 +415,11 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       float v = 0.f;
       #pragma unroll
       for (int q = 0; q < KW; ++q) v += red[(q * BM + r) * (16 + PAD) + c];
+      if constexpr (Q == Quant::Q4_K && !NORM)
+        if (v != v) {
+          const long at = weight_row<C>(n0, c, n, half);
+          v = dot_q4k(x + (long)r * k, qs + at * rb, scales + at * (sb / 2), k);
+        }
       if constexpr (NORM) v *= scale;
       return v;
     };
@@ -457,15 +481,14 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
     // rows 15.5, 18.9 -> 12.1, 16.3; q4_K 1 row 13.1, 17.1 -> 10.6, 16.5, 5
     // rows 15.1, 20.0 -> 13.3, 19.4; q6_K 1 row 23.0, 28.1 -> 16.7, 25.9.
     // 27648 x 5120, q4_0 5 rows: two stages in flight 26.0, one 22.7; eight
-    // waves 24.8.
+    // waves 24.8. q4_0 1 row, 5120 x 13824 17.4 -> 15.2, 15360 x 5120 12.9 ->
+    // 13.1.
     constexpr bool ONE = QQ == Quant::Q6_K || QQ == Quant::Q4_0;
     constexpr integral_constant<int, ONE ? 1 : 2> some{};
     constexpr integral_constant<int, QQ == Quant::Q8_0 ? 4 : 8> waves{};
     const bool thin = n <= 384 * 16;
     if (m == 1) {
-      if constexpr (QQ == Quant::Q4_0) {
-        go(qc, c4, c1, c8, c1);
-      } else if constexpr (QQ != Quant::Q8_0) {
+      if constexpr (QQ != Quant::Q8_0) {
         if (thin) go(qc, c4, c1, waves, some);
         else go(qc, c4, c1, c4, some);
       }

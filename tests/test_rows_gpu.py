@@ -162,6 +162,59 @@ def test_quant_rows(quant, m, n, k):
                      + 2.0 ** -6 * room.mean()).all())
 
 
+def one_column(ql, quant, at, number):
+    """Every row's number of column `at`, and its minimum 0."""
+    k, qs = ql.in_features, ql.qs
+    if quant == "q8_0":
+        qs[:, at] = number & 255
+    elif quant == "q4_0":
+        byte = at // 32 * 16 + at % 16
+        high = at % 32 >= 16
+        qs[:, byte] = qs[:, byte] & (15 if high else 240) | \
+            number + 8 << 4 * high
+    elif quant == "q4_K":
+        byte, high = k // 16 + at // 64 * 32 + at % 32, at % 64 >= 32
+        qs[:, byte] = qs[:, byte] & (15 if high else 240) | \
+            number << 4 * high
+        qs[:, k // 32 + at // 32] = 0
+    else:
+        block, half, l = at // 256, at % 256 // 128, at % 128
+        low, high = block * 128 + half * 64 + l % 64, l >= 64
+        qs[:, low] = qs[:, low] & (15 if high else 240) | \
+            (number + 32 & 15) << 4 * high
+        pair, turn = k // 2 + block * 64 + half * 32 + l % 32, l // 32 * 2
+        qs[:, pair] = qs[:, pair] & (255 - (3 << turn)) | \
+            (number + 32 >> 4) << turn
+
+
+@pytest.mark.parametrize("quant", ["q4_0", "q8_0", "q4_K", "q6_K"])
+@pytest.mark.parametrize("m", [2, 5, 16, 33])
+@pytest.mark.parametrize("at", [3, 501, 767])
+@torch.no_grad()
+def test_quant_outliers(quant, m, at):
+    """What weights of zero meet leaves nothing behind, however large; what is
+    infinite is infinite, by the sign of its weight."""
+    torch.manual_seed(m + at)
+    n, k = 48, 1024
+    lin = Linear(k, n, device=DEV, dtype=torch.bfloat16)
+    lin.weight.normal_(0.0, 0.5)
+    ql = QuantLinear.from_linear(lin, quant)
+    one_column(ql, quant, at, 0)
+    w = ql._dequant_cpu().to(DEV).double()
+    assert not bool(w[:, at].any())
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    x[:, at] = 2.0 ** 24
+    want = x.double() @ w.T
+    room = x.double().abs() @ w.abs().T
+    assert bool(((ql(x).double() - want).abs()
+                 <= 2.0 ** -8 * want.abs() + 2.0 ** -18 * room).all())
+    one_column(ql, quant, at, 5)
+    x[:, at] = torch.inf
+    w = ql._dequant_cpu().to(DEV)[:, at]
+    assert bool((w != 0).all())
+    assert torch.equal(ql(x).float(), (w * torch.inf).expand(m, n))
+
+
 @torch.no_grad()
 def test_products_of_few_rows_in_a_graph():
     """Replays with other inputs, eager work between."""
