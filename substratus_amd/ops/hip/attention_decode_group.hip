@@ -17,12 +17,13 @@
 // share a chunk of 32 keys with a barrier (groups of 4, 8, 16) or a wave per
 // head (others) to this one:
 //   64 sequences of 625 to 2500 keys, 32 heads on 8 of 128   148 -> 94 (4.4 TB/s)
-//   256 of 150 to 600, the same                              127 -> 84
-//   1 of 4000, the same                                     28.5 -> 12.2
+//   256 of 150 to 600, the same                              127 -> 85
+//   1 of 4000, the same                                     28.5 -> 12.3
 //   32 of 250 to 1000, 128 heads on 8 of 64                 28.8 -> 16.9
-//   128 of 300 to 1200, 71 heads on 1 of 64                  206 -> 26
+//   128 of 300 to 1200, 71 heads on 1 of 64                  206 -> 28
 // Four waves (one workgroup per CU): 96, 98, 10.9, 20.4, 25; one: 95, 86, 14.8,
-// 17.9, 27. Weights as bf16 high and low parts cost nothing beside the loads.
+// 17.9, 27, with weights in two bf16 parts. Three, which keep all their bits,
+// cost 1 % (the last shape 6 %).
 #include "rows_gemm.h"
 
 namespace {
@@ -180,16 +181,20 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
       #pragma unroll
       for (int t = 0; t < DT; ++t) o[t] *= keep;
     }
-    // weights as high and low parts, so they keep 16 bits
-    uint4v hi, low;
+    // weights as three parts, which hold all of their 24 bits
+    short8 parts[3];
     #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      hi[e] = pack2(p[2 * e], p[2 * e + 1]);
-      const float2 b = unpack_bf16x2(hi[e]);
-      low[e] = pack2(p[2 * e] - b.x, p[2 * e + 1] - b.y);
+    for (int w = 0; w < 3; ++w) {
+      uint4v u;
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        u[e] = pack2(p[2 * e], p[2 * e + 1]);
+        const float2 b = unpack_bf16x2(u[e]);
+        p[2 * e] -= b.x;
+        p[2 * e + 1] -= b.y;
+      }
+      parts[w] = __builtin_bit_cast(short8, u);
     }
-    const short8 ph = __builtin_bit_cast(short8, hi);
-    const short8 pl = __builtin_bit_cast(short8, low);
     // a cache's own values past the last key may be anything, and times a
     // weight of zero still be no number
     if (key0 + CH > n) {
@@ -215,10 +220,10 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
         const uint4v w = {r[2 * t][0], r[2 * t][1], r[2 * t + 1][0],
                           r[2 * t + 1][1]};
         const short8 vt = __builtin_bit_cast(short8, w);
-        o[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            vt, ph, o[t0 + t], 0, 0, 0);
-        o[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            vt, pl, o[t0 + t], 0, 0, 0);
+        #pragma unroll
+        for (int w = 0; w < 3; ++w)
+          o[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              vt, parts[w], o[t0 + t], 0, 0, 0);
       }
     }
   };

@@ -43,7 +43,33 @@ def test_groups(hq, hkv, d, contexts):
                   for t in (k, v))
         s = torch.matmul(kk, q[i].double()[:, :, None])[..., 0] * d ** -0.5
         want = torch.matmul(torch.softmax(s, 1)[:, None], vv)[:, 0]
-        # half a bf16 step of the result; weights keep 16 bits, scores' 32-bit
-        # sums are off by less
+        # half a bf16 step of the result; weights and scores are 32-bit numbers
         room = 2.0 ** -8 * want.abs() + 2.0 ** -14 * vv.abs().amax(1)
         assert bool(((got[i].double() - want).abs() <= room).all())
+
+
+@pytest.mark.parametrize("group", [3, 4, 8, 17])
+def test_weights_keep_their_bits(group):
+    """Two values that nearly cancel, so that what is left of a result is as
+    small as what 16 bits leave out of a weight."""
+    torch.manual_seed(group)
+    n, hkv, d = 16, 4, 64
+    q = (torch.randn(n, hkv * group, d, device=DEV) * 0.3).bfloat16()
+    k, v = (torch.zeros(n, hkv, 16, d, device=DEV).bfloat16()
+            for _ in range(2))
+    k[:, :, :2] = torch.randn(n, hkv, 2, d, device=DEV).bfloat16() * 0.3
+    first = q.view(n, hkv, group, d)[:, :, 0].double()
+    s = (k[:, :, :2].double() * first[:, :, None]).sum(-1) * d ** -0.5
+    a, b = torch.softmax(s, -1)[..., None].unbind(2)      # [n, hkv, 1]
+    some = (1 + torch.rand(256, n, hkv, d, device=DEV)).bfloat16().double()
+    against = -(some * a / b).bfloat16().double()
+    best = (some * a + against * b).abs().argmin(0, keepdim=True)
+    v[:, :, 0], v[:, :, 1] = (t.gather(0, best)[0] for t in (some, against))
+    got = ops.paged_attn_decode(
+        q, k, v, torch.arange(n, device=DEV, dtype=torch.int32)[:, None]
+        .contiguous(), torch.full((n,), 2, device=DEV, dtype=torch.int32),
+        d ** -0.5).view(n, hkv, group, d)[:, :, 0].double()
+    want = v[:, :, 0].double() * a + v[:, :, 1].double() * b
+    # 32-bit scores and exponentials: some 2^-23 of either product, about 1
+    off = (got - want).abs() - 2.0 ** -8 * want.abs()
+    assert float(off.max()) <= 2.0 ** -20
