@@ -931,17 +931,37 @@ void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
                        int max_blocks, float scale, long q_ld, int nsplit,
                        float* part_o, float* part_ml, hipStream_t stream);
 
-int paged_attn_nsplit(int bsz, int hq, int hkv, int d, int max_blocks) {
-  // flash-decoding split factor: fill >=1024 workgroups (256 CUs x 4
-  // resident WGs) when the (B, Hkv, group-chunk) grid alone is too small
-  // (llama2-70b at TP=8: B x 1 x 1). Shape-only -> hipGraph-stable.
-  const long base = (long)bsz * hkv * ((hq / hkv + 15) / 16);
+// Whether the grouped kernel takes a call. SUB_DECODE_GQA=scalar, or anything
+// else: the older kernels, which a cache of fp8 takes.
+bool paged_attn_grouped(int hq, int hkv, int d, long q_ld, const void* q,
+                        const void* kc, const void* vc, bool kv8) {
+  static const char* ge = getenv("SUB_DECODE_GQA");
+  return !kv8 && !ge && attn_group_takes(hq, hkv, d, q_ld, q, kc, vc);
+}
+
+// Flash-decoding shares: enough for 1024 workgroups (256 CUs x 4 resident ones)
+// where the grid alone is too small (llama2-70b at TP=8: B x 1 x 1), but no more
+// than the longest sequence that the table has room for has steps for. By shapes
+// only, so that a captured graph holds them. What a workgroup takes is its
+// kernel's: 16 heads, 4 pages a step (grouped); all of a group of 4, 8 or 16, 2
+// pages; 8 heads or one, 4 pages. With 16 heads and 4 pages counted for all of
+// them, fp8 caches took, us -> by this:
+//   71 heads on one of 64, 64 and 200 sequences of 150 keys  27.2 -> 20.2, 66.4
+//   -> 53.1; 24 on 2 of 64, the same  13.5 -> 9.9, 34.3 -> 25.0
+//   32 on 8 of 128, 1 and 16 sequences of 150 keys  11.1 -> 8.3, 14.0 -> 11.1
+// Two shares of one step each are no faster than one of both and a merge less:
+// 128 on 8 of 64, 16 sequences of 64 keys  8.2, 6.4.
+int paged_attn_nsplit(int bsz, int hq, int hkv, int d, int max_blocks,
+                      bool grouped) {
+  const int group = hq / hkv;
+  const bool whole = !grouped && gqa_hpw(hq, hkv, d) > 0;
+  const int heads = grouped ? 16 : whole ? group : group % 8 == 0 ? 8 : 1;
+  const int pages = whole ? 2 : 4;
+  const long base = (long)bsz * hkv * ((group + heads - 1) / heads);
   if (base >= 1024) return 1;
-  int ns = (int)((1024 + base - 1) / base);
-  if (ns > 16) ns = 16;
-  // four waves of a workgroup take a page each: no more shares than the
-  // longest sequence that the table has room for has pages for
-  return std::max(1, std::min(ns, (max_blocks + NW - 1) / NW));
+  const int ns = (int)std::min((1024 + base - 1) / base, 16L);
+  const int steps = (max_blocks + pages - 1) / pages;
+  return whole && steps < 3 ? 1 : std::max(1, std::min(ns, steps));
 }
 
 void launch_paged_attn_decode(bf16_t* out, const bf16_t* q,
@@ -950,21 +970,18 @@ void launch_paged_attn_decode(bf16_t* out, const bf16_t* q,
                               int bsz, int hq, int hkv, int d, int max_blocks,
                               int block_size, float scale, long q_rstride,
                               int nsplit, float* part_o, float* part_ml,
-                              bool kv8, hipStream_t stream) {
+                              bool kv8, bool grouped, hipStream_t stream) {
   const int group = hq / hkv;
   const int hpw = gqa_hpw(hq, hkv, d);
   dim3 block(NW * WAVE);
-  // SUB_DECODE_GQA=scalar, or anything else: the older kernels, which a cache
-  // of fp8 takes
-  static const char* ge = getenv("SUB_DECODE_GQA");
-  if (!kv8 && !ge && attn_group_takes(hq, hkv, d, q_rstride, q, k_cache,
-                                       v_cache)) {
+  if (grouped) {
     launch_attn_group(out, q, reinterpret_cast<const bf16_t*>(k_cache),
                       reinterpret_cast<const bf16_t*>(v_cache), block_table,
                       seq_lens, bsz, hq, hkv, d, max_blocks, scale, q_rstride,
                       nsplit, part_o, part_ml, stream);
   } else if (hpw > 0) {
     dim3 grid(bsz, hkv, nsplit);
+    static const char* ge = getenv("SUB_DECODE_GQA");
     static const bool scalar_gqa = ge && ge[0] == 's';
     if (!scalar_gqa) {
       #define LAUNCHM(DD, K8) \
