@@ -73,3 +73,10 @@ def test_weights_keep_their_bits(group):
     # 32-bit scores and exponentials: some 2^-23 of either product, about 1
     off = (got - want).abs() - 2.0 ** -8 * want.abs()
     assert float(off.max()) <= 2.0 ** -20
+
+
+@pytest.mark.parametrize("shares", [2, 3, 4, 5, 8, 9, 12, 16])
+@pytest.mark.parametrize("d", [64, 128])
+def test_merged_shares(shares, d):
+    """As many shares as fill what the merge loads at once, and one more."""
+    test_groups(4, 2, d, [64 * shares - 71])
