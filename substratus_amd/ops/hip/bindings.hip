@@ -43,7 +43,7 @@ void launch_add_norm_fwd(bf16_t*, bf16_t*, float*, const bf16_t*, const bf16_t*,
 void launch_add_norm_bwd(bf16_t*, bf16_t*, bf16_t*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const bf16_t*, long, int, bool, hipStream_t);
 void launch_rope_split(bf16_t*, bf16_t*, bf16_t*, const bf16_t*, const float*, const float*, long, int, int, int, int, hipStream_t);
 void launch_rope_join(bf16_t*, const bf16_t*, const float*, const float*, const float*, const float*, long, int, int, int, int, hipStream_t);
-void launch_lookup_bwd(bf16_t*, const bf16_t*, const long*, int, long, int, hipStream_t);
+void launch_lookup_bwd(bf16_t*, unsigned char*, const bf16_t*, const long*, int, long, int, hipStream_t);
 void launch_silu_mul_bwd(bf16_t*, const bf16_t*, const bf16_t*, long, int, hipStream_t);
 void launch_softmax_sample(long*, const bf16_t*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
 void launch_softmax_sample(long*, const float*, const float*, const int*, const float*, const float*, int, int, hipStream_t);
@@ -222,8 +222,9 @@ void lookup_bwd(torch::Tensor dw, torch::Tensor dy, torch::Tensor tokens) {
   TORCH_CHECK(tokens.is_cuda() && tokens.scalar_type() == torch::kLong &&
               tokens.is_contiguous(), "tokens must be int64 on GPU");
   check_rows(dw, dw.numel(), "dw"); check_rows(dy, n * hidden, "dy");
-  launch_lookup_bwd(bf(dw), bfc(dy), tokens.data_ptr<long>(), n, dw.size(0),
-                    hidden, stream());
+  auto often = torch::empty({n}, tokens.options().dtype(torch::kByte));
+  launch_lookup_bwd(bf(dw), often.data_ptr<unsigned char>(), bfc(dy),
+                    tokens.data_ptr<long>(), n, dw.size(0), hidden, stream());
   post_launch_check("lookup_bwd");
 }
 

@@ -370,16 +370,27 @@ __global__ __launch_bounds__(BLOCK) void silu_mul_bwd_kernel(
 }
 
 // Gradient of a lookup, whose rows are zero already. A workgroup per token: the
-// first one of a number adds up the rows of all of them, in their order. It
-// looks through all tokens for that, which is less than sorting them up to
-// some thousands (MI355X: 3 x 777 tokens of 32000 x 2048 154 us by torch's
-// kernels, 11 by this; 2 x 2048 of 65024 x 4544 142, 31).
+// first one of a number adds up the rows of all of them, in their order, unless
+// there are more than OFTEN, which it leaves to the kernel after this one: a row
+// after the other takes 0.3 us. It looks through all tokens for them, which is
+// less than sorting them up to some thousands.
+// us on a MI355X, torch's kernels (without the zeros), the first one of these
+// alone, both; 2331 tokens of 32000 x 2048, 4096 of 65024 x 4544, 8192 of 32000 x
+// 2048:
+//   every number about as often           179   11  14   184   26  30   179   53   58
+//   the k-th most frequent 1/k as often   177   71  30   155  157  62   156  231   87
+//   half of them one number               193  339  34   177  956  89   235 1236  122
+//   one number only                       251  692  41   211 1767  72   329 2440  134
+constexpr int OFTEN = 32;
+
 template <int CAP>
 __global__ __launch_bounds__(BLOCK) void lookup_bwd_kernel(
-    bf16_t* __restrict__ dw, const bf16_t* __restrict__ dy,
-    const long* __restrict__ tokens, int n, long rows, int hidden) {
+    bf16_t* __restrict__ dw, unsigned char* __restrict__ often,
+    const bf16_t* __restrict__ dy, const long* __restrict__ tokens, int n,
+    long rows, int hidden) {
   __shared__ unsigned long long same[NWAVES];
   const int i = blockIdx.x, tid = threadIdx.x;
+  if (tid == 0) often[i] = 0;
   const long t = tokens[i];
   if (t < 0 || t >= rows) return;
   bool before = false;
@@ -391,12 +402,19 @@ __global__ __launch_bounds__(BLOCK) void lookup_bwd_kernel(
   for (int c = 0; c < CAP; ++c)
     #pragma unroll
     for (int e = 0; e < 8; ++e) sum[c][e] = 0.f;
+  int count = 0;
   for (int j0 = i; j0 < n; j0 += BLOCK) {
     const int j = j0 + tid;
     const unsigned long long mine =
         __ballot(j < n && tokens[min(j, n - 1)] == t);
     if (tid % WAVE == 0) same[tid / WAVE] = mine;
     __syncthreads();
+    #pragma unroll
+    for (int w = 0; w < NWAVES; ++w) count += __popcll(same[w]);
+    if (count > OFTEN) {
+      if (tid == 0) often[i] = 1;
+      return;
+    }
     for (int w = 0; w < NWAVES; ++w)
       for (unsigned long long m = same[w]; m; m &= m - 1) {
         const long row = j0 + w * WAVE + __builtin_ctzll(m);
@@ -418,6 +436,75 @@ __global__ __launch_bounds__(BLOCK) void lookup_bwd_kernel(
   for (int c = 0; c < CAP; ++c) {
     const int at = tid + c * BLOCK;
     if (at < nvec) out[at] = pack8(sum[c]);
+  }
+}
+
+// The numbers that come often: a workgroup for 64 columns of those whose first
+// tokens are a grid apart, eight threads a row, 32 rows at once.
+constexpr int SLICE = 64;
+
+__global__ __launch_bounds__(BLOCK) void lookup_bwd_often_kernel(
+    bf16_t* __restrict__ dw, const unsigned char* __restrict__ often,
+    const bf16_t* __restrict__ dy, const long* __restrict__ tokens, int n,
+    int hidden) {
+  constexpr int SLOTS = BLOCK / 8;
+  __shared__ unsigned long long mask[2][NWAVES];
+  __shared__ int list[BLOCK];
+  __shared__ float part[SLOTS][SLICE];
+  const int tid = threadIdx.x, wave = tid / WAVE, slot = tid / 8;
+  const int lane8 = tid % 8 * 8, col = blockIdx.y * SLICE + lane8;
+  const int grid = gridDim.x;
+  for (int i0 = blockIdx.x; i0 < n; i0 += grid * BLOCK) {
+    const long mine = i0 + (long)tid * grid;
+    const unsigned long long b = __ballot(mine < n && often[mine]);
+    if (tid % WAVE == 0) mask[0][wave] = b;
+    __syncthreads();
+    for (int w = 0; w < NWAVES; ++w)
+      for (unsigned long long m = mask[0][w]; m; m &= m - 1) {
+        const int i = i0 + (w * WAVE + __builtin_ctzll(m)) * grid;
+        const long t = tokens[i];
+        float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int j0 = i; j0 < n; j0 += BLOCK) {
+          const int j = j0 + tid;
+          const bool same = j < n && tokens[min(j, n - 1)] == t;
+          const unsigned long long all = __ballot(same);
+          if (tid % WAVE == 0) mask[1][wave] = all;
+          __syncthreads();
+          int before = 0, count = 0;
+          #pragma unroll
+          for (int q = 0; q < NWAVES; ++q) {
+            const int some = __popcll(mask[1][q]);
+            before += q < wave ? some : 0;
+            count += some;
+          }
+          if (same)
+            list[before + __popcll(all & ((1ull << (tid % WAVE)) - 1))] = j;
+          __syncthreads();
+          if (col < hidden) {
+            #pragma unroll 4
+            for (int r = slot; r < count; r += SLOTS) {
+              float f[8];
+              unpack8(*reinterpret_cast<const uint4*>(
+                          dy + (long)list[r] * hidden + col), f);
+              #pragma unroll
+              for (int e = 0; e < 8; ++e) sum[e] += f[e];
+            }
+          }
+          __syncthreads();
+        }
+        #pragma unroll
+        for (int e = 0; e < 8; ++e) part[slot][lane8 + e] = sum[e];
+        __syncthreads();
+        const int at = blockIdx.y * SLICE + tid;
+        if (tid < SLICE && at < hidden) {
+          float s = 0.f;
+          #pragma unroll
+          for (int q = 0; q < SLOTS; ++q) s += part[q][tid];
+          dw[t * hidden + at] = f2bf(s);
+        }
+        __syncthreads();
+      }
+    __syncthreads();
   }
 }
 
@@ -498,10 +585,17 @@ void launch_silu_mul_bwd(bf16_t* dx, const bf16_t* dy, const bf16_t* x,
                         stream>>>(dx, dy, x, f);
 }
 
-void launch_lookup_bwd(bf16_t* dw, const bf16_t* dy, const long* tokens,
-                       int n, long rows, int hidden, hipStream_t stream) {
+void launch_lookup_bwd(bf16_t* dw, unsigned char* often, const bf16_t* dy,
+                       const long* tokens, int n, long rows, int hidden,
+                       hipStream_t stream) {
   by_width(hidden, [&](auto cap) {
     lookup_bwd_kernel<decltype(cap)::value>
-        <<<dim3(n), dim3(BLOCK), 0, stream>>>(dw, dy, tokens, n, rows, hidden);
+        <<<dim3(n), dim3(BLOCK), 0, stream>>>(dw, often, dy, tokens, n, rows,
+                                              hidden);
   });
+  if (n > OFTEN)
+    lookup_bwd_often_kernel<<<dim3(std::min(n, 64),
+                                   (hidden + SLICE - 1) / SLICE),
+                              dim3(BLOCK), 0, stream>>>(dw, often, dy, tokens,
+                                                        n, hidden);
 }

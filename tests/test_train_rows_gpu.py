@@ -197,3 +197,28 @@ def test_lookup(n, rows, width):
     table.register_forward_hook(lambda *a: None)
     assert not train.lookup(tokens, table).grad_fn.name().startswith(
         "_Lookup")
+
+
+@pytest.mark.parametrize("width", [8, 72, 2056])
+def test_lookup_of_frequent_numbers(width):
+    """Numbers that come as often as one workgroup takes, and once more; a
+    number behind a workgroup's reach of others; one alone."""
+    g = torch.Generator().manual_seed(width)
+    counts = torch.tensor([31, 32, 33, 64, 65, 0, 1, 300, 257, 2])
+    for tokens in (torch.arange(10).repeat_interleave(counts),
+                   torch.arange(10).repeat_interleave(counts)[
+                       torch.randperm(785, generator=g)],
+                   torch.tensor([3] * 700), torch.tensor([9] * 8192)):
+        tokens = tokens.to(DEV)
+        table = torch.nn.Embedding(10, width, device=DEV,
+                                   dtype=torch.bfloat16)
+        out = train.lookup(tokens, table)
+        assert out.grad_fn.name().startswith("_Lookup")
+        dy = rand(len(tokens), width, seed=2)
+        got, = torch.autograd.grad(out, table.weight, dy)
+        want, size = (torch.zeros(10, width, device=DEV, dtype=torch.float64)
+                      .index_add_(0, tokens, t) for t in (
+                          dy.double(), dy.double().abs()))
+        near(got, want, size)
+        assert torch.equal(got, torch.autograd.grad(
+            train.lookup(tokens, table), table.weight, dy)[0])
