@@ -508,7 +508,7 @@ TilePlan tile_gemm_plan(long m, long n, long k) {
   const double full = rounds * (steps * 1.5 + 5.);
   p.whole = (int)tiles;
   p.split = 1;
-  p.us = full + (rest ? steps * 1.5 + 5. : 0.);
+  p.us = p.unshared = full + (rest ? steps * 1.5 + 5. : 0.);
   for (int s = 2; rest && rest * s <= 256 && steps / s >= 4; ++s) {
     const double us = full + (steps + s - 1) / s * 1.5 + 10. +
                       rest * s * (0.262144 * 2 / 5.);
@@ -521,26 +521,38 @@ TilePlan tile_gemm_plan(long m, long n, long k) {
   return p;
 }
 
-// Whether the library's product would take longer. What it takes is no smooth
-// function of sizes; on a MI355X, planned PFLOP/s and what this one gains:
-//   neither flipped   below 0.9: 0.75 to 1.18 times as fast, mostly slower
-//                     (2048 x 4096 x 4096: 0.81, 0.85); above: 0.94 to 2.06
-//                     (4165 x 4096 x 11008: 1.19, 2.06; 4096 x 18176 x 4544:
-//                     1.25, 1.26; 2331 x 32000 x 2048: 1.15, 0.96); whole tiles
-//                     in whole rounds, which need neither split nor reach back:
-//                     0.95 to 0.99
-//   b flipped         0.39 to 0.57: 0.87 to 0.96; from 0.7: 1.02 to 2.05
-//   both flipped      0.39: 0.90; from 0.7: 1.00 to 1.41
-//   gated             from 0.9 on, even ones too: the pass that gates them
-//                     is a tenth of the product
+// Whether the library's product would take longer. What that takes is no smooth
+// function of sizes, so this takes kinds of which next to none was measured to be
+// slower: products of 700 to 8192 rows with matrices of 768 to 50272 rows and
+// columns that come from memory, MI355X, by planned PFLOP/s; the library's time
+// over this one's:
+//   neither flipped   from 1.0 on, 162 products 0.985 to 1.90 and one 0.956 (3000
+//                     x 18176 x 4544), where one of these holds: the library's
+//                     tiles reach over the columns' end (2472 x 6160 x 2048
+//                     1.10; with few steps, 8192 x 50272 x 768, 0.92), sharing
+//                     is to gain a tenth (4165 x 4096 x 11008 1.85), or steps are
+//                     many, so that a tile's end, 5 us, counts for little (2331 x
+//                     5120 x 13824 1.46). Others: 0.90 to 1.43, more than half
+//                     of them below 1 (3000 x 32000 x 4096 0.90, 2464 x 6144 x
+//                     2048 0.94), below 1.0 from 0.90. Whole tiles in whole
+//                     rounds 0.96 to 1.04.
+//   b flipped         shared ones from 0.7 on, others from 1.1 on: 141 of 0.997
+//                     to 1.97. Others: 0.87 to 1.41 (2331 x 4096 x 22016 0.88)
+//   both flipped      0.39: 0.90; from 0.7 on 119 of 1.02 to 1.42
+//   gated             from 0.9 on 35 of 1.03 and more, whole rounds too: the
+//                     pass that gates them is a tenth of the product
 bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped,
                     bool gated) {
   const TilePlan p = tile_gemm_plan(m, n, k);
   const double rate = 2e-9 * m * n * k / p.us;        // PFLOP/s
-  if (a_flipped || b_flipped) return rate >= 0.7;
+  if (gated) return rate >= 0.9;
+  if (a_flipped) return rate >= 0.7;
+  if (b_flipped) return rate >= (p.split > 1 ? 0.7 : 1.1);
   const bool even = m % TILE == 0 && n % TILE == 0 &&
                     (long)p.tiles_m * p.tiles_n % 256 == 0;
-  return rate >= 0.9 && (gated || !even);
+  return rate >= 1.0 && !even &&
+         ((n % TILE != 0 && k >= 1024) || p.unshared >= 1.1 * p.us ||
+          k >= 4500);
 }
 
 void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,

@@ -84,25 +84,28 @@ def test_rows_of_any_number():
 def test_linear_gradients(bias):
     """ops.linear at a size where all three products pay."""
     torch.manual_seed(5)
-    x = torch.randn(2, 1001, 4096, device=DEV).bfloat16().requires_grad_()
-    w = (torch.randn(8192, 4096, device=DEV) / 64).bfloat16() \
-        .requires_grad_()
-    bs = torch.randn(8192, device=DEV).bfloat16().requires_grad_() \
+    t, k, n = 2082, 11008, 4096
+    assert all(_C.tile_gemm_good(*s, False) for s in (
+        (2 * t, n, k, k, k, False, False), (2 * t, k, n, n, k, False, True),
+        (n, k, 2 * t, n, k, True, True)))
+    x = torch.randn(2, t, k, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(n, k, device=DEV) / 64).bfloat16().requires_grad_()
+    bs = torch.randn(n, device=DEV).bfloat16().requires_grad_() \
         if bias else None
     y = ops.linear(x, w, bs)
-    dy = torch.randn(2, 1001, 8192, device=DEV).bfloat16()
-    rows, drows = x.detach().view(-1, 4096), dy.view(-1, 8192)
-    close(y.detach().view(-1, 8192), rows, w.detach(),
+    dy = torch.randn(2, t, n, device=DEV).bfloat16()
+    rows, drows = x.detach().view(-1, k), dy.view(-1, n)
+    close(y.detach().view(-1, n), rows, w.detach(),
           None if bs is None else bs.detach())
     inputs = [t for t in (x, w, bs) if t is not None]
     got = torch.autograd.grad(y, inputs, dy, retain_graph=True)
-    close(got[0].view(-1, 4096), drows, w.detach().T)
+    close(got[0].view(-1, k), drows, w.detach().T)
     close(got[1], drows.T, rows.T)
     if bias:
         assert torch.equal(got[2], drows.sum(0))
     # gradients that are no rows, and gradients of gradients
     g, = torch.autograd.grad(y.sum(), x, retain_graph=True)
-    close(g.view(-1, 4096), torch.ones_like(drows), w.detach().T)
+    close(g.view(-1, k), torch.ones_like(drows), w.detach().T)
     first, = torch.autograd.grad(y, x, dy, create_graph=True)
     again, = torch.autograd.grad(first.float().sum(), w)
     want = torch.nn.functional.linear(x, w, bs)

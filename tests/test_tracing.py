@@ -76,7 +76,7 @@ def test_compiled():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,k", [(3, 2048), (40, 2048), (1024, 11008)])
+@pytest.mark.parametrize("rows,k", [(3, 2048), (40, 2048), (4165, 11008)])
 @torch.no_grad()
 def test_traced_products(rows, k):
     lin = Linear(k, 4096, device="cuda", dtype=torch.bfloat16)
@@ -117,7 +117,7 @@ def test_batches_of_gradients():
 
     def leaf(*shape):
         return torch.randn(*shape, device="cuda").bfloat16().requires_grad_()
-    x, w = leaf(4096, 2048), leaf(2048, 2048)
+    x, w = leaf(4165, 11008), leaf(4096, 11008)
     h, d, n, b = leaf(5, 64), leaf(5, 64), leaf(64), leaf(64)
     table = torch.nn.Embedding(50, 64, device="cuda", dtype=torch.bfloat16)
     tokens = torch.randint(0, 50, (2, 9), device="cuda")
