@@ -351,7 +351,10 @@ class _Linear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, bias):
-        ctx.save_for_backward(x, weight)
+        # each gradient needs the other operand: a frozen weight's input is
+        # not kept
+        dx, dw, _ = ctx.needs_input_grad
+        ctx.save_for_backward(x if dw else None, weight if dx else None)
         y = _tile_gemm(x, weight, bias)
         return torch.nn.functional.linear(x, weight, bias) if y is None else y
 

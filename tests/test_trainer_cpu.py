@@ -337,3 +337,25 @@ def test_recomputed_blocks_of_frozen_embeddings(name):
     assert len(calls) == 2 * cfg.num_layers - 1     # all but the first again
     for a, b in zip(*results):
         torch.testing.assert_close(a, b)
+
+
+@pytest.mark.parametrize("frozen", ["none", "input", "weight"])
+def test_products_keep_what_their_gradients_need(frozen):
+    """As torch's own linear: an input is kept for its weight's gradient and a
+    weight for its input's."""
+    from substratus_amd.ops import _Linear
+    x, w = torch.randn(6, 4), torch.randn(5, 4)
+    x.requires_grad_(frozen != "input")
+    w.requires_grad_(frozen != "weight")
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(
+            lambda t: kept.append(t.shape) or t, lambda t: t):
+        y = _Linear.apply(x, w, None)
+    assert (x.shape in kept) == w.requires_grad
+    assert (w.shape in kept) == x.requires_grad
+    want = torch.nn.functional.linear(x, w)
+    given = [t for t in (x, w) if t.requires_grad]
+    dy = torch.randn_like(want)
+    for a, b in zip(torch.autograd.grad(y, given, dy),
+                    torch.autograd.grad(want, given, dy)):
+        torch.testing.assert_close(a, b)
