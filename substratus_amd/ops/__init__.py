@@ -302,7 +302,8 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
             and x.numel() > 0
             and _rows_gemm_pays(x.numel(), *weight.shape)):
         return None
-    if bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_cuda
+    if bias is not None and not (bias.dtype == torch.bfloat16
+                                 and bias.device == x.device
                                  and bias.is_contiguous()
                                  and bias.shape == weight.shape[:1]):
         return None

@@ -2,6 +2,7 @@
 // Validation lives here; kernels are thin and trusting.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
+#include <c10/core/DeviceGuard.h>
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
@@ -68,6 +69,8 @@ void launch_wstream_gemm(bf16_t*, const bf16_t*, const bf16_t*, float*, int, int
 
 namespace {
 
+// The current device's; of products and training ops, which torch's own do on
+// whatever device their operands are, the operands' (a guard in each).
 inline hipStream_t stream() {
   return at::cuda::getCurrentCUDAStream().stream();
 }
@@ -125,6 +128,7 @@ void add_norm_fwd(torch::Tensor y, c10::optional<torch::Tensor> sum,
                   c10::optional<torch::Tensor> d1,
                   c10::optional<torch::Tensor> d2, torch::Tensor w,
                   c10::optional<torch::Tensor> b, double eps) {
+  const c10::DeviceGuard guard(h.device());
   const long n = h.numel(), hidden = w.numel();
   TORCH_CHECK(n > 0 && train_norm_takes(hidden) && n % hidden == 0,
               "width ", hidden, " not taken");
@@ -146,6 +150,7 @@ void add_norm_bwd(torch::Tensor dh, torch::Tensor dw,
                   c10::optional<torch::Tensor> db, torch::Tensor dy,
                   c10::optional<torch::Tensor> dres, torch::Tensor x,
                   torch::Tensor stats, torch::Tensor w) {
+  const c10::DeviceGuard guard(x.device());
   const long n = x.numel(), hidden = w.numel();
   TORCH_CHECK(n > 0 && train_norm_takes(hidden) && n % hidden == 0,
               "width ", hidden, " not taken");
@@ -183,6 +188,7 @@ void check_angles(const c10::optional<torch::Tensor>& c,
 void rope_split(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                 torch::Tensor qkv, c10::optional<torch::Tensor> c,
                 c10::optional<torch::Tensor> s, long length) {
+  const c10::DeviceGuard guard(qkv.device());
   TORCH_CHECK(q.dim() == 3 && k.dim() == 3, "q, k are [rows, heads, d]");
   const long rows = q.size(0), hq = q.size(1), hkv = k.size(1), d = q.size(2);
   check_angles(c, s, rows, length, d);
@@ -199,6 +205,7 @@ void rope_split(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 void rope_join(torch::Tensor dqkv, torch::Tensor dq, torch::Tensor dk,
                torch::Tensor dv, c10::optional<torch::Tensor> c,
                c10::optional<torch::Tensor> s, long length) {
+  const c10::DeviceGuard guard(dqkv.device());
   TORCH_CHECK(dq.dim() == 3 && dk.dim() == 3, "q, k are [rows, heads, d]");
   const long rows = dq.size(0), hq = dq.size(1), hkv = dk.size(1);
   const long d = dq.size(2);
@@ -216,6 +223,7 @@ void rope_join(torch::Tensor dqkv, torch::Tensor dq, torch::Tensor dk,
 
 // dw, zero before, gets the sums of dy's rows at tokens, which are rows of dw.
 void lookup_bwd(torch::Tensor dw, torch::Tensor dy, torch::Tensor tokens) {
+  const c10::DeviceGuard guard(dw.device());
   const long n = tokens.numel(), hidden = dw.size(1);
   TORCH_CHECK(dw.dim() == 2 && n > 0 && n < (1L << 30) &&
               train_norm_takes(hidden), "width ", hidden, " not taken");
@@ -229,6 +237,7 @@ void lookup_bwd(torch::Tensor dw, torch::Tensor dy, torch::Tensor tokens) {
 }
 
 void silu_mul_bwd(torch::Tensor dx, torch::Tensor dy, torch::Tensor x) {
+  const c10::DeviceGuard guard(x.device());
   const long f = x.size(-1) / 2, n = x.numel();
   TORCH_CHECK(n > 0 && f % 8 == 0 && x.size(-1) == 2 * f,
               "width must be a multiple of 16");
@@ -273,6 +282,7 @@ void layer_norm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor x) {
+  const c10::DeviceGuard guard(x.device());
   check_bf16(out, "out"); check_bf16(x, "x");
   int f = out.size(-1);
   TORCH_CHECK(x.size(-1) == 2 * f, "x last dim must be 2*out last dim");
@@ -586,6 +596,7 @@ void rope_split_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> bias, bool gated,
                   const Heads* heads, const NormOf* norm = nullptr) {
+  const c10::DeviceGuard guard(x.device());
   check_bf16(y, "y"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
               x.dim() == 2 && x.stride(1) == 1 &&
@@ -619,6 +630,7 @@ void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
 torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
                         c10::optional<torch::Tensor> bias, bool a_flipped,
                         bool b_flipped, bool gated) {
+  const c10::DeviceGuard guard(a.device());
   for (const auto& t : {a, b})
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
                     t.dim() == 2 && t.stride(1) == 1 && aligned16(t),
@@ -676,6 +688,7 @@ bool quant_rows_ok(long m, long n, long k, const std::string& quant,
 void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
                    torch::Tensor qs, const std::string& quant, bool gated,
                    const Heads* heads, const NormOf* norm = nullptr) {
+  const c10::DeviceGuard guard(x.device());
   check_bf16(y, "y"); check_bf16(x, "x");
   TORCH_CHECK(scales.scalar_type() == torch::kHalf, "scales must be fp16");
   TORCH_CHECK(qs.scalar_type() == torch::kByte, "qs must be uint8");
@@ -791,8 +804,10 @@ void adamw_steps(std::vector<torch::Tensor> ps, std::vector<torch::Tensor> gs,
                  long step, double gscale, c10::optional<torch::Tensor> norm,
                  double clip) {
   std::vector<OptTensor> all;
-  TORCH_CHECK(gs.size() == ps.size() && ms.size() == ps.size() &&
-              vs.size() == ps.size(), "as many of each");
+  TORCH_CHECK(!ps.empty() && gs.size() == ps.size() &&
+              ms.size() == ps.size() && vs.size() == ps.size(),
+              "as many of each");
+  const c10::DeviceGuard guard(ps[0].device());
   for (size_t i = 0; i < ps.size(); ++i) {
     const long n = ps[i].numel();
     check_bf16(ps[i], "parameter");
@@ -813,6 +828,7 @@ void adamw_steps(std::vector<torch::Tensor> ps, std::vector<torch::Tensor> gs,
 // The 2-norm of all tensors as one vector, in 32 bits on the device.
 torch::Tensor grad_norm(std::vector<torch::Tensor> gs) {
   TORCH_CHECK(!gs.empty(), "no gradients");
+  const c10::DeviceGuard guard(gs[0].device());
   std::vector<OptTensor> all;
   for (auto& g : gs) {
     check_rows(g, g.numel(), "gradient");
@@ -874,6 +890,7 @@ void softmax_sample(torch::Tensor out, torch::Tensor logits,
 void cross_entropy_fwd_bwd(torch::Tensor loss, torch::Tensor dlogits,
                            torch::Tensor logits, torch::Tensor targets,
                            long ignore_index) {
+  const c10::DeviceGuard guard(logits.device());
   check_bf16(dlogits, "dlogits"); check_bf16(logits, "logits");
   TORCH_CHECK(loss.scalar_type() == torch::kFloat, "loss must be fp32");
   TORCH_CHECK(targets.scalar_type() == torch::kLong, "targets must be int64");

@@ -110,6 +110,7 @@ class _Values:
 
     def __init__(self, scalars: list[torch.Tensor]):
         self.host, self.event = scalars, None
+        self.device = scalars[0].device
         if scalars[0].is_cuda:
             self.host = torch.empty(len(scalars), dtype=scalars[0].dtype,
                                     pin_memory=True)
@@ -121,7 +122,7 @@ class _Values:
     def after(self) -> None:
         """read() waits for all that is queued by now."""
         if self.event is not None:
-            self.event.record()
+            self.event.record(torch.cuda.current_stream(self.device))
 
     def read(self) -> list[float]:
         if self.event is not None:
