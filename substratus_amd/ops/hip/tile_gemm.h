@@ -11,7 +11,6 @@ struct TilePlan {
   // floats of the shares
   long shares() const { return split > 1 ? (long)rest() * split * 65536 : 0; }
   double us;                      // what it is to take
-  double unshared;                // the same with split 1
 };
 
 // out [m, n] = a b^T + bias, all bf16 and sums in 32 bits. An operand has its

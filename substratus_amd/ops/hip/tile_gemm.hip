@@ -508,7 +508,7 @@ TilePlan tile_gemm_plan(long m, long n, long k) {
   const double full = rounds * (steps * 1.5 + 5.);
   p.whole = (int)tiles;
   p.split = 1;
-  p.us = p.unshared = full + (rest ? steps * 1.5 + 5. : 0.);
+  p.us = full + (rest ? steps * 1.5 + 5. : 0.);
   for (int s = 2; rest && rest * s <= 256 && steps / s >= 4; ++s) {
     const double us = full + (steps + s - 1) / s * 1.5 + 10. +
                       rest * s * (0.262144 * 2 / 5.);
@@ -522,37 +522,36 @@ TilePlan tile_gemm_plan(long m, long n, long k) {
 }
 
 // Whether the library's product would take longer. What that takes is no smooth
-// function of sizes, so this takes kinds of which next to none was measured to be
-// slower: products of 700 to 8192 rows with matrices of 768 to 50272 rows and
-// columns that come from memory, MI355X, by planned PFLOP/s; the library's time
-// over this one's:
-//   neither flipped   from 1.0 on, 162 products 0.985 to 1.90 and one 0.956 (3000
-//                     x 18176 x 4544), where one of these holds: the library's
-//                     tiles reach over the columns' end (2472 x 6160 x 2048
-//                     1.10; with few steps, 8192 x 50272 x 768, 0.92), sharing
-//                     is to gain a tenth (4165 x 4096 x 11008 1.85), or steps are
-//                     many, so that a tile's end, 5 us, counts for little (2331 x
-//                     5120 x 13824 1.46). Others: 0.90 to 1.43, more than half
-//                     of them below 1 (3000 x 32000 x 4096 0.90, 2464 x 6144 x
-//                     2048 0.94), below 1.0 from 0.90. Whole tiles in whole
-//                     rounds 0.96 to 1.04.
-//   b flipped         shared ones from 0.7 on, others from 1.1 on: 141 of 0.997
-//                     to 1.97. Others: 0.87 to 1.41 (2331 x 4096 x 22016 0.88)
-//   both flipped      0.39: 0.90; from 0.7 on 119 of 1.02 to 1.42
+// function of sizes; by itself it is often a few percent faster, but it writes
+// past the caches, and the pass that reads the results pays for it (2331 x 32000
+// x 2048 0.97, a step's loss after it 90 us instead of 73). So this goes by the
+// product and a pass that reads its results together, less that pass: the
+// library's time over this one's, MI355X, weights that come from memory, 1024 to
+// 8192 rows, matrices of 2048 to 32000 rows and columns, by planned PFLOP/s:
+//   neither flipped   from 0.9 on 158 products of 0.97 to 1.98 (three of 3000
+//                     rows and more x 32000, whose results no cache holds,
+//                     below 0.99; 2331 x 32000 x 2048 1.05, 4096 x 18176 x 4544
+//                     1.25); by themselves 0.92 to 1.9. Whole tiles in whole
+//                     rounds, 1.01 to 1.09, stay with the library: by themselves
+//                     0.94 to 1.0
+//   b flipped         shared ones from 0.7 on, others from 0.9 on where tiles
+//                     take more than three quarters of their rounds' CUs: 155 of
+//                     0.98 to 2.48. Others: 0.86 to 1.69 (2331 x 4096 x 22016,
+//                     160 tiles, 0.86)
+//   both flipped      0.39: 0.90; from 0.7 on 119 of 1.02 to 1.42 by themselves
 //   gated             from 0.9 on 35 of 1.03 and more, whole rounds too: the
 //                     pass that gates them is a tenth of the product
 bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped,
                     bool gated) {
   const TilePlan p = tile_gemm_plan(m, n, k);
   const double rate = 2e-9 * m * n * k / p.us;        // PFLOP/s
-  if (gated) return rate >= 0.9;
+  const long tiles = (long)p.tiles_m * p.tiles_n;
+  const long places = (tiles + 255) / 256 * 256;
   if (a_flipped) return rate >= 0.7;
-  if (b_flipped) return rate >= (p.split > 1 ? 0.7 : 1.1);
-  const bool even = m % TILE == 0 && n % TILE == 0 &&
-                    (long)p.tiles_m * p.tiles_n % 256 == 0;
-  return rate >= 1.0 && !even &&
-         ((n % TILE != 0 && k >= 1024) || p.unshared >= 1.1 * p.us ||
-          k >= 4500);
+  if (b_flipped)
+    return p.split > 1 ? rate >= 0.7 : rate >= 0.9 && 4 * tiles > 3 * places;
+  const bool even = m % TILE == 0 && n % TILE == 0 && tiles == places;
+  return rate >= 0.9 && (gated || !even);
 }
 
 void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,
