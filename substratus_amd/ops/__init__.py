@@ -235,39 +235,22 @@ def flash_attn_train_available(d: int) -> bool:
 _GEMM_WS: dict = {}
 
 
-# called for every product of a step: names looked up once
-_TENSORS = (torch.Tensor, torch.nn.Parameter)
-_STRIDED = torch.strided
-_batched = torch._C._functorch.is_legacy_batchedtensor
-_transforms = torch._C._are_functorch_transforms_active
-_tracing_state = torch._C._get_tracing_state
-_dispatch_modes = torch._C._len_torch_dispatch_stack
-_functions = torch._C._len_torch_function_stack
-_autocast = torch.is_autocast_enabled
 _compiling = torch.compiler.is_compiling
-_forward_ad = torch.autograd.forward_ad
-
-
-def _function_modes() -> bool:
-    """Whether a mode is to see calls of torch's functions (other than a device
-    for new tensors)."""
-    return any(type(m) is not DeviceContext
-               for m in _get_current_function_mode_stack())
 
 
 def plain_tensors(*tensors: Optional[torch.Tensor]) -> bool:
     """No transform, trace, autocast, function or dispatch mode that expects
-    torch's own ops, no tensor subclass, batch of tensors or sparse layout."""
+    torch's own ops, no tensor subclass, batch of tensors, dual number or
+    sparse layout; and there are kernels to ask for."""
     if _compiling():        # first: a compiler does not know the others
         return False
-    for t in tensors:
-        if t is not None and (type(t) not in _TENSORS
-                              or t.layout is not _STRIDED or _batched(t)):
-            return False
-    return not (_autocast("cuda")
-                or _tracing_state() is not None or _transforms()
-                or _dispatch_modes() or _functions() and _function_modes()
-                or _forward_ad._current_level >= 0)
+    ext = _load_ext()
+    if ext is None:
+        return False
+    state = ext.plain_tensors(*tensors)
+    # function modes: one that only gives new tensors a device sees nothing
+    return state == 2 or state == 1 and all(
+        type(m) is DeviceContext for m in _get_current_function_mode_stack())
 
 
 def inference_only(*tensors: torch.Tensor) -> bool:

@@ -1,7 +1,12 @@
 // Python bindings for the CDNA4 HIP kernel library (substratus_amd._C).
 // Validation lives here; kernels are thin and trusting.
 #include <torch/extension.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/cuda/CUDAContext.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/core/DeviceGuard.h>
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
@@ -106,6 +111,32 @@ bool aligned16(const torch::Tensor& t) {
 void post_launch_check(const char* op) {
   hipError_t e = hipGetLastError();
   TORCH_CHECK(e == hipSuccess, op, ": HIP launch failed: ", hipGetErrorString(e));
+}
+
+// Whether values are all that is asked of an op on these (None among them): 2; 1
+// but for function modes; 0. Asked for every product and by every backward: 0.7
+// us here, 1.4 (6.5 the first time in a thread) in Python.
+int plain_tensors(const py::args& tensors) {
+  using c10::DispatchKey;
+  constexpr c10::DispatchKeySet wrapped({
+      DispatchKey::Python, DispatchKey::Batched, DispatchKey::FuncTorchBatched,
+      DispatchKey::FuncTorchGradWrapper, DispatchKey::Functionalize});
+  for (const auto& o : tensors) {
+    if (o.is_none()) continue;
+    if (!THPVariable_CheckExact(o.ptr())) return 0;
+    const at::Tensor& t = THPVariable_Unpack(o.ptr());
+    if (t.layout() != at::kStrided || t.key_set().has_any(wrapped) ||
+        (t.key_set().has(DispatchKey::ADInplaceOrView) &&
+         t._fw_grad(0).defined()))
+      return 0;
+  }
+  if (at::autocast::is_autocast_enabled(at::kCUDA) ||
+      torch::jit::tracer::isTracing() ||
+      c10::impl::tls_is_dispatch_key_included(
+          DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+      c10::impl::TorchDispatchModeTLS::any_modes_set())
+    return 0;
+  return at::impl::PythonTorchFunctionTLS::stack_len() > 0 ? 1 : 2;
 }
 
 // bf16, contiguous, of n elements and on 16-byte boundaries
@@ -1037,6 +1068,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul", &silu_mul);
   m.def("gelu_tanh", &gelu_tanh);
   m.def("rope_kv_append", &rope_kv_append);
+  m.def("plain_tensors", &plain_tensors);
   m.def("paged_attn_nsplit", &paged_attn_nsplit);
   m.def("paged_attn_decode", &paged_attn_decode);
   m.def("attn_prefill", &attn_prefill);
