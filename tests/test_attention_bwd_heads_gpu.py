@@ -35,6 +35,25 @@ def test_heads(b, s, hq, hkv, d):
         assert float(off) < 2.0 ** -7, float(off)
 
 
+@pytest.mark.parametrize("b,s,hq,hkv,d", [
+    (1, 31, 8, 8, 64), (2, 33, 4, 4, 128), (1, 65, 3, 1, 64),
+    (2, 255, 2, 1, 128), (1, 300, 5, 5, 64), (16, 128, 71, 1, 64),
+    (64, 65, 66, 22, 64), (32, 257, 71, 1, 64), (16, 255, 64, 8, 128),
+    (33, 256, 64, 8, 128)])
+def test_long_form(b, s, hq, hkv, d, monkeypatch):
+    """The keys' and values' kernel for long sequences, at its edges: 32 rows
+    of a wave, 64 of a chunk, 256 of a tile."""
+    monkeypatch.setenv("SUB_ATTN_DKV_V5", "1")
+    test_heads(b, s, hq, hkv, d)
+
+
+@pytest.mark.parametrize("b,s,hq,hkv,d", [
+    (1, 2049, 4, 4, 64), (1, 2111, 3, 3, 128), (1, 8200, 2, 1, 64)])
+def test_long(b, s, hq, hkv, d):
+    """Lengths from which that kernel is taken."""
+    test_heads(b, s, hq, hkv, d)
+
+
 @pytest.mark.parametrize("scale", [0.125, 0.0, -0.2])
 @pytest.mark.parametrize("lens", [[1, 63, 64, 65], [255, 256, 257], [600]])
 def test_forward(lens, scale):

@@ -27,13 +27,13 @@ def made(kind, k, n, bias):
 # stages of 64 and 256 columns for 4 or 8 waves, parts of them, the most that
 # fits; rows up to four
 @pytest.mark.parametrize("kind,m,k,n,bias", [
-    ("dense", 1, 32, 16, True), ("dense", 1, 8192, 48, False),
+    ("dense", 1, 32, 48, True), ("dense", 1, 8192, 48, False),
     ("dense", 2, 4096, 160, True), ("dense", 3, 1056, 96, False),
     ("dense", 4, 2048, 256, True), ("q4_0", 1, 5120, 96, False),
-    ("q4_0", 3, 320, 64, False), ("q8_0", 2, 448, 32, False),
-    ("q4_K", 1, 2560, 64, False), ("q4_K", 4, 2048, 32, False),
+    ("q4_0", 3, 320, 64, False), ("q8_0", 2, 448, 48, False),
+    ("q4_K", 1, 2560, 64, False), ("q4_K", 4, 2048, 48, False),
     ("q6_K", 1, 256, 64, False), ("q6_K", 2, 1024, 48, False)])
-@pytest.mark.parametrize("how", ["plain", "gated", "heads"])
+@pytest.mark.parametrize("how", ["plain", "gated", "heads", "turned heads"])
 @torch.no_grad()
 def test_normed(kind, m, k, n, bias, how):
     torch.manual_seed(m * k + n)
@@ -42,13 +42,12 @@ def test_normed(kind, m, k, n, bias, how):
     norm = (1 + 0.3 * torch.randn(k, device=DEV)).bfloat16()
     d, hkv = 16, 1
     cache = None
-    if how == "heads":
-        if n < 4 * d or n % d:
-            return
+    if "heads" in how:
         kc, vc = (torch.zeros(m, hkv, 16, d, device=DEV).bfloat16()
                   for _ in range(2))
         at = torch.arange(m, device=DEV).int()
-        cache = ops.Cache(at * 3, kc, vc, at * 16 + 5, 0.0)
+        cache = ops.Cache(at * 3, kc, vc, at * 16 + 5,
+                          1e4 if "turned" in how else 0.0)
     got = lin.normed(delta, h, norm, 1e-5, how == "gated", cache)
     assert got is not None
     y, total = got
@@ -60,6 +59,18 @@ def test_normed(kind, m, k, n, bias, how):
     if how == "gated":
         want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
         other = ops.silu_mul(other)
+    elif how == "turned heads":
+        plain = lin.normed(delta, h, norm, 1e-5)[0].view(m, -1, d)
+        caches = [torch.zeros_like(kc) for _ in range(2)]
+        q = ops.rope_kv_append(
+            *(t.contiguous() for t in plain.split([n // d - 2, 1, 1], 1)),
+            cache.positions, *caches, cache.slots, 1e4)
+        # one rounding of the same 32-bit numbers, whose last bits may differ
+        for a, b in ((y, q), (kc, caches[0]), (vc, caches[1])):
+            a, b = a.float().view(-1), b.float().view(-1)
+            assert bool(((a - b).abs() <=
+                         2.0 ** -7 * b.abs() + 2.0 ** -20).all())
+        return
     elif how == "heads":
         assert torch.equal(y.view(m, -1), lin.normed(
             delta, h, norm, 1e-5)[0][:, :n - 2 * d])
