@@ -149,13 +149,13 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   const float inv_t = 1.f / temp;
   const float top = totals.most(wave_max(best));
   const float m = top * inv_t;
-  // NaN, and what is below all others: 0. A logit below the largest may be
-  // equal to it once scaled (of neighbours in 32 bits about a tenth are): 1,
-  // unless both went past the largest number
+  // NaN, and what went past the largest number beside the largest logit: 0. A
+  // logit below the largest may be equal to it once scaled (of neighbours in 32
+  // bits about a tenth are), and weighs as much then.
+  const float past = m == -INFINITY ? m : INFINITY;
   auto weight = [&](float v) {
     const float x = v * inv_t, below = __expf(x - m);
-    return v == top || (x == m && fabsf(m) < INFINITY) ? 1.f
-        : x < m ? below : 0.f;
+    return v == top ? 1.f : x < past ? below : 0.f;
   };
   #pragma unroll
   for (int r = 0; r < NR; ++r)
