@@ -397,8 +397,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
     """F.linear. Up to 16 rows of bf16 without gradients, or up to 64 with a
     matrix of few rows, take the kernel that streams weights at the memory's
     rate (rows_gemm.hip), products of 256 rows and more the one for the matrix
-    cores (tile_gemm.hip) where that is the faster one, in a backward as well. SUB_MGEMM=1 routes decode shapes of 256
-    rows and more to the 256x256 glds GEMM (mfma_gemm.hip).
+    cores (tile_gemm.hip) where that is the faster one, in a backward as well.
+    SUB_MGEMM=1 routes decode shapes of 256 rows and more to the 256x256 glds
+    GEMM (mfma_gemm.hip).
 
     The latter is NOT on by default: measurement
     (profiles/mgemm_r02.md) shows hipBLASLt's MT192/MT256 solutions at 1.3-4.1

@@ -9,7 +9,7 @@
 // (rows x width, launches of everything, us of everything but products,
 // attention and update):
 //   4096 x 4544, 71 heads on 1 of 64, LayerNorm   502 -> 238, 6950 -> 3900
-//   2331 x 2048, 16 heads on 4 of 128, RMS, gated  496 -> 194, 3350 -> 1190
+//   2331 x 2048, 16 heads of 128, RMS, gated       496 -> 194, 3350 -> 1190
 // At 4096 x 4544 the norm of two additions takes 33 us (5.6 TB/s), its
 // backward 38 and 9 for the sum of shares, split and join 14 and 16.
 #include <algorithm>
