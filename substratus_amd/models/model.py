@@ -1,7 +1,6 @@
 """Unified decoder-only transformer for the llama / falcon / opt families.
 
-One implementation serves all model configs the reference's examples name
-(SURVEY.md §2.5): llama2-7b/13b/70b (RMSNorm + RoPE + GQA + SwiGLU),
+One implementation serves all model configs the reference's examples name: llama2-7b/13b/70b (RMSNorm + RoPE + GQA + SwiGLU),
 falcon-7b-instruct (LayerNorm + RoPE + MQA + parallel attn/MLP + GELU),
 facebook/opt-125m (LayerNorm + learned positions + GELU).
 
@@ -13,8 +12,7 @@ Three execution paths:
     torch SDPA; loss/gradients via the fused cross-entropy kernel)
 
 Tensor-parallel: heads are sharded column-parallel for QKV, row-parallel for
-the output/down projections (2 RCCL all-reduces per layer — SURVEY.md §2.5
-ledger items 9).
+the output/down projections (2 RCCL all-reduces per layer).
 """
 
 from __future__ import annotations

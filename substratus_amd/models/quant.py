@@ -1,4 +1,4 @@
-"""Quantized linear layers for GGUF serving (SURVEY.md §2.5: the llama.cpp
+"""Quantized linear layers for GGUF serving (the llama.cpp
 serving path rebuilt first-party).
 
 QuantLinear keeps weights resident as repacked GGUF blocks — fp16 scales

@@ -1,5 +1,4 @@
-// Paged-KV decode attention (SURVEY.md §2.5 ledger item 1) — the serving hot
-// kernel: per sequence and KV head, softmax(q·K^T/√d)·V over a block-paged
+// Paged-KV decode attention — the serving hot kernel: per sequence and KV head, softmax(q·K^T/√d)·V over a block-paged
 // cache, one new token per sequence.
 //
 // Decode at batch B is HBM-bound on the K/V stream (e.g. llama2-7b @ctx 512,

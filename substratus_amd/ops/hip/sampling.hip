@@ -1,4 +1,4 @@
-// Fused sampling kernel (SURVEY.md §2.5 ledger item 5): temperature / top-k /
+// Fused sampling kernel: temperature / top-k /
 // top-p + inverse-CDF draw, one workgroup per logits row.
 //
 // A row is read once, 16 bytes per load, and stays in registers as

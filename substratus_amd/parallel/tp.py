@@ -3,14 +3,14 @@
 Column-parallel: weight rows (output features) sharded; no comm on forward.
 Row-parallel: weight cols (input features) sharded; one all-reduce on forward.
 Per transformer layer the server does 2 all-reduces (post-attention o_proj and
-post-MLP down_proj) — SURVEY.md §2.5 ledger item 9. On 8×MI355X the xGMI
+post-MLP down_proj). On 8×MI355X the xGMI
 topology is 7 p2p links/GPU, so for the small latency-sensitive decode
 all-reduces RCCL's one-shot algorithm is preferred (RCCL chooses by size; we
 keep tensors contiguous and per-step message counts minimal).
 
 Reference behavioral contract: multi-GPU Server Pods request amd.com/gpu: N
 (reference api/v1/common_types.go:102-107); the parallelism itself is new,
-first-party (the reference's data plane is external — SURVEY.md §0).
+first-party (the reference's data plane is external).
 """
 
 from __future__ import annotations

@@ -1,5 +1,5 @@
 """Trainer — replaces the reference's external
-`substratusai/model-trainer-huggingface` image (SURVEY.md §2.5).
+`substratusai/model-trainer-huggingface` image.
 
 Container contract (reference docs/container-contract.md + examples/
 llama2-7b/finetuned-model.yaml:10-21): base model RO at /content/model,
@@ -262,8 +262,7 @@ class Trainer:
 
     def maybe_resume(self) -> int:
         """Resume from the newest checkpoint-{N} under artifacts_dir
-        (reference behavior: training-level resume is the trainer's job —
-        SURVEY.md §5 'Checkpoint / resume')."""
+        (reference behavior: training-level resume is the trainer's job)."""
         if not self.cfg.resume or not os.path.isdir(self.cfg.artifacts_dir):
             return 0
         ckpts = []

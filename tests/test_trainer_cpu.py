@@ -1,6 +1,5 @@
 """Trainer CPU tests: fused-CE gradient path vs torch autograd, loss descent,
-checkpoint/resume, and 2-process DDP gradient parity over gloo
-(multi-GPU paths are covered by multi-process CPU tests)."""
+checkpoint/resume, and 2-process DDP gradient parity over gloo."""
 
 import json
 import os
