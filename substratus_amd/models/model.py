@@ -1,6 +1,7 @@
 """Unified decoder-only transformer for the llama / falcon / opt families.
 
-One implementation serves all model configs the reference's examples name: llama2-7b/13b/70b (RMSNorm + RoPE + GQA + SwiGLU),
+One implementation serves all model configs the reference's examples name:
+llama2-7b/13b/70b (RMSNorm + RoPE + GQA + SwiGLU),
 falcon-7b-instruct (LayerNorm + RoPE + MQA + parallel attn/MLP + GELU),
 facebook/opt-125m (LayerNorm + learned positions + GELU).
 
