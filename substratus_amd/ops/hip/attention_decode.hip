@@ -1,5 +1,5 @@
-// Paged-KV decode attention — the serving hot kernel: per sequence and KV head, softmax(q·K^T/√d)·V over a block-paged
-// cache, one new token per sequence.
+// Paged-KV decode attention — the serving hot kernel: per sequence and KV head,
+// softmax(q·K^T/√d)·V over a block-paged cache, one new token per sequence.
 //
 // Decode at batch B is HBM-bound on the K/V stream (e.g. llama2-7b @ctx 512,
 // B=64: ~16 GB of KV per step vs 13.5 GB of weights). Structure:
