@@ -1,5 +1,8 @@
-// Paged-KV decode attention — the serving hot kernel: per sequence and KV head,
-// softmax(q·K^T/√d)·V over a block-paged cache, one new token per sequence.
+// Paged-KV decode attention of grouped heads — per sequence and KV head,
+// softmax(q·K^T/√d)·V over a block-paged cache, one new token per sequence —
+// and the choice of the kernel that takes a call. Heads by themselves:
+// attention_decode_heads.hip; groups over an aligned bf16 cache:
+// attention_decode_group.hip.
 //
 // Decode at batch B is HBM-bound on the K/V stream (e.g. llama2-7b @ctx 512,
 // B=64: ~16 GB of KV per step vs 13.5 GB of weights). Structure:
@@ -863,7 +866,8 @@ void paged_attn_decode_mfma_kernel(
 }
 
 // GQA heads-per-wave for the LDS-staged decode variant; 0 = use the
-// register-tiled kernel (MHA group 1, falcon's prime group 71, d oddballs).
+// register-tiled kernel (other groups of a multiple of 8), or a head at a time
+// (attention_decode_heads.hip).
 static inline int gqa_hpw(int hq, int hkv, int d) {
   if (d != 64 && d != 128) return 0;
   const int group = hq / hkv;
@@ -933,6 +937,16 @@ void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
                        int max_blocks, float scale, long q_ld, int nsplit,
                        float* part_o, float* part_ml, hipStream_t stream);
 
+// attention_decode_heads.hip
+void attn_heads_plan(int bsz, int hq, int d, int max_blocks, int& waves,
+                     int& nsplit);
+void launch_attn_heads(bf16_t* out, const bf16_t* q, const void* kc,
+                       const void* vc, const int* block_table,
+                       const int* seq_lens, int bsz, int hq, int hkv, int d,
+                       int max_blocks, float scale, long q_ld, int waves,
+                       int nsplit, float* part_o, float* part_ml, bool kv8,
+                       hipStream_t stream);
+
 // Whether the grouped kernel takes a call. SUB_DECODE_GQA=scalar, or anything
 // else: the older kernels, which a cache of fp8 takes.
 bool paged_attn_grouped(int hq, int hkv, int d, long q_ld, const void* q,
@@ -941,7 +955,7 @@ bool paged_attn_grouped(int hq, int hkv, int d, long q_ld, const void* q,
   return !kv8 && !ge && attn_group_takes(hq, hkv, d, q_ld, q, kc, vc);
 }
 
-// Flash-decoding shares: enough for 1024 workgroups (256 CUs x 4 resident ones)
+// Flash-decoding shares of workgroups of two or four waves: enough for 1024 workgroups (256 CUs x 4 resident ones)
 // where the grid alone is too small (llama2-70b at TP=8: B x 1 x 1), but no more
 // than the longest sequence that the table has room for has steps for. By shapes
 // only, so that a captured graph holds them. What a workgroup takes is its
@@ -966,13 +980,26 @@ int paged_attn_nsplit(int bsz, int hq, int hkv, int d, int max_blocks,
   return whole && steps < 3 ? 1 : std::max(1, std::min(ns, steps));
 }
 
+// The same for the kernel that takes a call. waves: 0, or those of a workgroup
+// for a single head where no kernel takes several of a group together.
+int paged_attn_plan(int bsz, int hq, int hkv, int d, int max_blocks,
+                    bool grouped, int& waves) {
+  waves = 0;
+  int nsplit;
+  if (grouped || gqa_hpw(hq, hkv, d) > 0 || hq / hkv % 8 == 0)
+    return paged_attn_nsplit(bsz, hq, hkv, d, max_blocks, grouped);
+  attn_heads_plan(bsz, hq, d, max_blocks, waves, nsplit);
+  return nsplit;
+}
+
 void launch_paged_attn_decode(bf16_t* out, const bf16_t* q,
                               const void* k_cache, const void* v_cache,
                               const int* block_table, const int* seq_lens,
                               int bsz, int hq, int hkv, int d, int max_blocks,
                               int block_size, float scale, long q_rstride,
                               int nsplit, float* part_o, float* part_ml,
-                              bool kv8, bool grouped, hipStream_t stream) {
+                              bool kv8, bool grouped, int waves,
+                              hipStream_t stream) {
   const int group = hq / hkv;
   const int hpw = gqa_hpw(hq, hkv, d);
   dim3 block(NW * WAVE);
@@ -981,6 +1008,10 @@ void launch_paged_attn_decode(bf16_t* out, const bf16_t* q,
                       reinterpret_cast<const bf16_t*>(v_cache), block_table,
                       seq_lens, bsz, hq, hkv, d, max_blocks, scale, q_rstride,
                       nsplit, part_o, part_ml, stream);
+  } else if (waves > 0) {
+    launch_attn_heads(out, q, k_cache, v_cache, block_table, seq_lens, bsz, hq,
+                      hkv, d, max_blocks, scale, q_rstride, waves, nsplit,
+                      part_o, part_ml, kv8, stream);
   } else if (hpw > 0) {
     dim3 grid(bsz, hkv, nsplit);
     static const char* ge = getenv("SUB_DECODE_GQA");
@@ -1022,29 +1053,16 @@ void launch_paged_attn_decode(bf16_t* out, const bf16_t* q,
     #undef LAUNCHG
     }
   } else {
-  // GC=8 when the GQA group tiles evenly by 8 but the LDS path is out
-  // (non-power-of-two d); GC=1 otherwise (MHA group=1; falcon's prime
-  // group=71 — its MQA KV is tiny and L3-resident, so per-head K
-  // re-reads are cheap).
-  const int gc = (group % 8 == 0) ? 8 : 1;
-  const int gchunks = (group + gc - 1) / gc;
-  dim3 grid(bsz, hkv, gchunks * nsplit);
-  #define LAUNCH(DD, GG, K8) \
-    paged_attn_decode_kernel<DD, GG, K8><<<grid, block, 0, stream>>>( \
-        out, q, k_cache, v_cache, block_table, seq_lens, hq, hkv, \
-        max_blocks, scale, q_rstride, nsplit, part_o, part_ml)
-  if (!kv8) {
-    if (d == 128 && gc == 8) LAUNCH(128, 8, false);
-    else if (d == 128) LAUNCH(128, 1, false);
-    else if (d == 64 && gc == 8) LAUNCH(64, 8, false);
-    else if (d == 64) LAUNCH(64, 1, false);
-  } else {
-    if (d == 128 && gc == 8) LAUNCH(128, 8, true);
-    else if (d == 128) LAUNCH(128, 1, true);
-    else if (d == 64 && gc == 8) LAUNCH(64, 8, true);
-    else if (d == 64) LAUNCH(64, 1, true);
-  }
-  #undef LAUNCH
+    // groups of a multiple of 8 other than 8 and 16, over an fp8 cache or
+    // unaligned operands
+    dim3 grid(bsz, hkv, group / 8 * nsplit);
+    auto kernel = kv8 ? (d == 128 ? paged_attn_decode_kernel<128, 8, true>
+                                  : paged_attn_decode_kernel<64, 8, true>)
+                      : (d == 128 ? paged_attn_decode_kernel<128, 8, false>
+                                  : paged_attn_decode_kernel<64, 8, false>);
+    kernel<<<grid, block, 0, stream>>>(
+        out, q, k_cache, v_cache, block_table, seq_lens, hq, hkv, max_blocks,
+        scale, q_rstride, nsplit, part_o, part_ml);
   }
   if (nsplit > 1) {
     auto merge = [&](auto shares) {

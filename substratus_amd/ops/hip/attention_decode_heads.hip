@@ -1,0 +1,312 @@
+// Paged decode attention, a workgroup per query head and share of a sequence:
+// heads that share no keys, and grouped ones over an fp8 cache for which no
+// other kernel is made (head sizes 64 and 128).
+//
+// Bound by the K/V stream, or with few sequences by the chain of loads to its
+// end. A row of K or V is 16 (head size 64: 8) lanes wide, in either the same
+// eight elements a lane, so a score that those lanes have added up is where its
+// weight is needed: lanes of a row keep a softmax of their own, and nothing
+// leaves registers before the end. Both of a step's panels and the next step's
+// are in flight, page numbers two steps ahead.
+//
+// Eight waves share a sequence, whose results are merged through LDS. us of a
+// captured call, second kernel included where there is one, from a kernel that
+// waited for V after its scores and took shares of four waves each (max. keys):
+//   1 sequence of 150, 16 heads of 128      6.8 -> 4.2
+//   1 of 800, 40 heads                      9.0 -> 8.0
+//   8 of 900, 32 heads                     22.7 -> 17.5 (4.7 TB/s)
+//   5 of 1100, 40 heads                    23.0 -> 17.8
+//   256 of 620, 32 heads                    261 -> 254  (6.5 TB/s)
+//   30 of 700, 12 heads of 64              16.8 -> 11.6
+//   40 of 800, fp8, 71 heads on 1 of 64    48.2 -> 27.9
+#include "common.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace {
+
+constexpr int PAGE = 16;
+constexpr int PIECES = 4;         // of K, or V, that a lane has of a step
+constexpr float LOG2E = 1.44269504088896340736f;
+
+// Eight elements of a row.
+template <bool KV8> struct Piece;
+template <> struct Piece<false> {
+  uint4v u;
+  DEV_INLINE void load(const char* p) { u = nt_load_u4(p); }
+  DEV_INLINE void clear() { u = (uint4v){0, 0, 0, 0}; }
+  DEV_INLINE void unpack(float (&f)[8]) const {
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float2 v = unpack_bf16x2(u[i]);
+      f[2 * i] = v.x;
+      f[2 * i + 1] = v.y;
+    }
+  }
+};
+template <> struct Piece<true> {
+  uint2v u;
+  DEV_INLINE void load(const char* p) { u = nt_load_u2(p); }
+  DEV_INLINE void clear() { u = (uint2v){0, 0}; }
+  DEV_INLINE void unpack(float (&f)[8]) const {
+    #pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      f[4 * i] = fp8_to_f32<0>(u[i]);
+      f[4 * i + 1] = fp8_to_f32<1>(u[i]);
+      f[4 * i + 2] = fp8_to_f32<2>(u[i]);
+      f[4 * i + 3] = fp8_to_f32<3>(u[i]);
+    }
+  }
+};
+
+// v plus another lane's, by a data-parallel move
+template <int CTRL>
+DEV_INLINE float plus(float v) {
+  return v + __uint_as_float(__builtin_amdgcn_update_dpp(
+      0u, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
+// The sum over a row's lanes, in all of them: exchanges within pairs, fours,
+// eights and sixteens.
+template <int LANES>
+DEV_INLINE float row_sum(float v) {
+  v = plus<0xb1>(v);                      // quad_perm 1 0 3 2
+  v = plus<0x4e>(v);                      // quad_perm 2 3 0 1
+  v = plus<0x141>(v);                     // row_half_mirror
+  if constexpr (LANES == 16) v = plus<0x140>(v);    // row_mirror
+  return v;
+}
+
+template <int D, bool KV8, int WAVES>
+__global__ __launch_bounds__(WAVES * WAVE, 4)
+void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
+                       const bf16_t* __restrict__ q,
+                       const char* __restrict__ kc,    // [NB, HKV, 16, D]
+                       const char* __restrict__ vc,
+                       const int* __restrict__ block_table,  // [B, max_blocks]
+                       const int* __restrict__ seq_lens,
+                       int hq, int hkv, int max_blocks, float scale,
+                       long q_ld, int nsplit,
+                       float* __restrict__ part_o,   // [B, HQ, NS, D]
+                       float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
+  constexpr int LANES = D / 8;                   // of a row
+  constexpr int ROWS = WAVE / LANES;             // of a piece of all lanes
+  constexpr int KEYS = PIECES * ROWS;            // of a step
+  constexpr int SIZE = KV8 ? 1 : 2;
+  const int b = blockIdx.x, head = blockIdx.y, split = blockIdx.z;
+  const int kvh = head / (hq / hkv);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, row = lane / LANES, at = lane % LANES;
+  const int* bt = block_table + (long)b * max_blocks;
+
+  // steps of KEYS keys, one page or two, by turns with other waves
+  constexpr int PAGES = KEYS / PAGE;
+  const int first = split * WAVES + wave, stride = nsplit * WAVES;
+  auto page_of = [&](int step, int p) {
+    return max_blocks > 0 ? bt[min(step * PAGES + p, max_blocks - 1)] : 0;
+  };
+  int page[PAGES], next[PAGES];
+  #pragma unroll
+  for (int p = 0; p < PAGES; ++p) {
+    page[p] = page_of(first, p);
+    next[p] = page_of(first + stride, p);
+  }
+  const int n = seq_lens[b];
+  const int steps = (n + KEYS - 1) / KEYS;
+
+  float qf[8];
+  {
+    const uint4v u = *reinterpret_cast<const uint4v*>(
+        q + (long)b * q_ld + (long)head * D + at * 8);
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float2 v = unpack_bf16x2(u[i]);
+      qf[2 * i] = v.x * (scale * LOG2E);
+      qf[2 * i + 1] = v.y * (scale * LOG2E);
+    }
+  }
+  struct Panels { Piece<KV8> k[PIECES], v[PIECES]; };
+  const long own = (long)kvh * PAGE * D * SIZE + (row * D + at * 8) * SIZE;
+  const long page_size = (long)hkv * PAGE * D * SIZE;
+  auto load = [&](Panels& x, int step, const int (&pages)[PAGES]) {
+    #pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int p = i * ROWS / PAGE;
+      // a step's second page may be past the last one: the first again
+      const bool there = p == 0 || step * PAGES + p < (n + PAGE - 1) / PAGE;
+      x.k[i].load(kc + (there ? pages[p] : pages[0]) * page_size + own +
+                  i * ROWS % PAGE * D * SIZE);
+    }
+    #pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int p = i * ROWS / PAGE;
+      const bool there = p == 0 || step * PAGES + p < (n + PAGE - 1) / PAGE;
+      x.v[i].load(vc + (there ? pages[p] : pages[0]) * page_size + own +
+                  i * ROWS % PAGE * D * SIZE);
+    }
+  };
+  float m = -INFINITY, l = 0.f, acc[8];
+  #pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] = 0.f;
+  auto use = [&](Panels& x, int step) {
+    const int key = step * KEYS + row;
+    float s[PIECES], most = m;
+    #pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      float k[8];
+      x.k[i].unpack(k);
+      float v = qf[0] * k[0];
+      #pragma unroll
+      for (int j = 1; j < 8; ++j) v = fmaf(qf[j], k[j], v);
+      v = row_sum<LANES>(v);
+      s[i] = key + i * ROWS < n ? v : -INFINITY;
+      most = fmaxf(most, s[i]);
+    }
+    // no key yet: its weights are zeros, not differences of infinities
+    const float base = most == -INFINITY ? 0.f : most;
+    const float keep = __builtin_amdgcn_exp2f(m - base);
+    m = most;
+    l *= keep;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] *= keep;
+    // a cache's own values past the last key may be no numbers
+    if ((step + 1) * KEYS > n) {
+      #pragma unroll
+      for (int i = 0; i < PIECES; ++i)
+        if (key + i * ROWS >= n) x.v[i].clear();
+    }
+    #pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const float w = __builtin_amdgcn_exp2f(s[i] - base);
+      float v[8];
+      x.v[i].unpack(v);
+      l += w;
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] = fmaf(w, v[j], acc[j]);
+    }
+  };
+  Panels a, c;
+  auto turn = [&](int step) {
+    #pragma unroll
+    for (int p = 0; p < PAGES; ++p) next[p] = page_of(step, p);
+  };
+  if (first < steps) load(a, first, page);
+  for (int t = first; t < steps; t += 2 * stride) {
+    if (t + stride < steps) {
+      load(c, t + stride, next);
+      turn(t + 2 * stride);
+    }
+    use(a, t);
+    if (t + stride >= steps) break;
+    if (t + 2 * stride < steps) {
+      load(a, t + 2 * stride, next);
+      turn(t + 3 * stride);
+    }
+    use(c, t + stride);
+  }
+
+  // the rows' softmaxes become one a wave, and the waves' one
+  __shared__ float s_o[WAVES][D], s_m[WAVES], s_l[WAVES];
+  float most = m;
+  #pragma unroll
+  for (int off = LANES; off < WAVE; off *= 2)
+    most = fmaxf(most, __shfl_xor(most, off, WAVE));
+  const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - most);
+  l *= f;
+  #pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] *= f;
+  #pragma unroll
+  for (int off = LANES; off < WAVE; off *= 2) {
+    l += __shfl_xor(l, off, WAVE);
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] += __shfl_xor(acc[j], off, WAVE);
+  }
+  if (row == 0) {
+    #pragma unroll
+    for (int j = 0; j < 8; j += 4)
+      *reinterpret_cast<float4*>(&s_o[wave][at * 8 + j]) =
+          make_float4(acc[j], acc[j + 1], acc[j + 2], acc[j + 3]);
+    if (at == 0) { s_m[wave] = most; s_l[wave] = l; }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x >= D / 2) return;
+  float M = -INFINITY, L = 0.f, o0 = 0.f, o1 = 0.f;
+  #pragma unroll
+  for (int w = 0; w < WAVES; ++w) M = fmaxf(M, s_m[w]);
+  const int d = threadIdx.x * 2;
+  #pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const float e =
+        s_m[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[w] - M);
+    L += e * s_l[w];
+    o0 += e * s_o[w][d];
+    o1 += e * s_o[w][d + 1];
+  }
+  const long h = (long)b * hq + head;
+  if (nsplit == 1) {
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    *reinterpret_cast<unsigned*>(out + h * D + d) =
+        pack_bf16x2(o0 * inv, o1 * inv);
+  } else {
+    const long part = h * nsplit + split;
+    *reinterpret_cast<float2*>(part_o + part * D + d) = make_float2(o0, o1);
+    if (d == 0) {
+      // the merging kernel's maxima are natural logarithms
+      part_ml[part * 2] = M / LOG2E;
+      part_ml[part * 2 + 1] = L;
+    }
+  }
+}
+
+}  // namespace
+
+// Waves of a workgroup, and workgroups that share a sequence: by shapes only, so
+// that a captured graph holds them. A CU reads some 55 GB/s, so a step of a head
+// by itself takes 0.15 us, and merging 2.4 us more than one launch: the line is
+// where shares win that back, which they do less the more heads there are to
+// keep the chip busy. MI355X, us alone, 8 shares, 16 shares, by heads in all:
+//   keys of 128       16                  40                  96
+//   400         6.6  6.6  6.7       6.9  7.0  7.3       7.3  8.7 11.0
+//   800        10.4  6.8  6.9      10.7  8.0  8.5      11.4 11.1 13.0
+//   1600       17.7  8.4  7.4      18.6 10.8 10.9      19.8 15.2 17.0
+//   4000       39.3 11.5 10.5      41.3 20.4 18.8      47.9 30.9 30.0
+// and 128 heads of 1600 keys 20.2 18.9 21.7; 160 of 1100 17.8 and 18.7 (4).
+// Eight waves or four alone: 256 x 32 heads of 620 keys 254, 258; 40 x 71 of
+// 800 keys of 64 in fp8, 25 steps, 29.0, 27.9.
+void attn_heads_plan(int bsz, int hq, int d, int max_blocks, int& waves,
+                     int& nsplit) {
+  const long heads = (long)bsz * hq;
+  const int pages = PIECES * WAVE * 8 / d / PAGE;          // of a step
+  const long steps = (max_blocks + pages - 1) / pages;
+  waves = heads >= 1024 && steps < 32 ? 4 : 8;
+  nsplit = heads < 170 && steps * (170 - heads) > 20 * 170
+               ? steps > 128 ? 16 : 8 : 1;
+}
+
+void launch_attn_heads(bf16_t* out, const bf16_t* q, const void* kc,
+                       const void* vc, const int* block_table,
+                       const int* seq_lens, int bsz, int hq, int hkv, int d,
+                       int max_blocks, float scale, long q_ld, int waves,
+                       int nsplit, float* part_o, float* part_ml, bool kv8,
+                       hipStream_t stream) {
+  const dim3 grid(bsz, hq, nsplit);
+  auto go = [&](auto dim, auto fp8, auto w) {
+    constexpr int W = decltype(w)::value;
+    attn_heads_kernel<decltype(dim)::value, decltype(fp8)::value, W>
+        <<<grid, dim3(W * WAVE), 0, stream>>>(
+            out, q, reinterpret_cast<const char*>(kc),
+            reinterpret_cast<const char*>(vc), block_table, seq_lens, hq, hkv,
+            max_blocks, scale, q_ld, nsplit, part_o, part_ml);
+  };
+  auto sized = [&](auto dim, auto fp8) {
+    if (waves == 8) go(dim, fp8, std::integral_constant<int, 8>());
+    else go(dim, fp8, std::integral_constant<int, 4>());
+  };
+  auto typed = [&](auto dim) {
+    if (kv8) sized(dim, std::true_type());
+    else sized(dim, std::false_type());
+  };
+  if (d == 128) typed(std::integral_constant<int, 128>());
+  else typed(std::integral_constant<int, 64>());
+}

@@ -25,9 +25,10 @@ void launch_silu_mul(bf16_t*, const bf16_t*, long, int, hipStream_t);
 void launch_gelu(bf16_t*, const bf16_t*, long, hipStream_t);
 void launch_rope_kv_append(bf16_t*, bf16_t*, const bf16_t*, const int*, void*, void*, const int*, int, int, int, int, int, float, bool, long, long, long, hipStream_t);
 void launch_rope_split_append(bf16_t*, bf16_t*, bf16_t*, const bf16_t*, const int*, void*, void*, const int*, long, int, int, int, int, float, bool, hipStream_t);
-void launch_paged_attn_decode(bf16_t*, const bf16_t*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, long, int, float*, float*, bool, bool, hipStream_t);
+void launch_paged_attn_decode(bf16_t*, const bf16_t*, const void*, const void*, const int*, const int*, int, int, int, int, int, int, float, long, int, float*, float*, bool, bool, int, hipStream_t);
 bool paged_attn_grouped(int, int, int, long, const void*, const void*, const void*, bool);
 int paged_attn_nsplit(int, int, int, int, int, bool);
+int paged_attn_plan(int, int, int, int, int, bool, int&);
 bool paged_attn_decode_supported(int, int);
 void launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, int, int, int, int, int, float, hipStream_t, float*);
 bool attn_prefill_supported(int);
@@ -380,7 +381,9 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   const bool grouped = paged_attn_grouped(
       hq, hkv, d, q.stride(0), q.data_ptr(), k_cache.data_ptr(),
       v_cache.data_ptr(), kv8);
-  const int nsplit = paged_attn_nsplit(bsz, hq, hkv, d, max_blocks, grouped);
+  int waves;
+  const int nsplit = paged_attn_plan(bsz, hq, hkv, d, max_blocks, grouped,
+                                     waves);
   float *po = nullptr, *pml = nullptr;
   torch::Tensor part_o, part_ml;
   if (nsplit > 1) {
@@ -395,7 +398,7 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
                            block_table.data_ptr<int>(),
                            seq_lens.data_ptr<int>(), bsz, hq, hkv, d,
                            max_blocks, block_size, (float)scale, q.stride(0),
-                           nsplit, po, pml, kv8, grouped, stream());
+                           nsplit, po, pml, kv8, grouped, waves, stream());
   post_launch_check("paged_attn_decode");
 }
 
