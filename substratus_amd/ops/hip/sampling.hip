@@ -3,16 +3,19 @@
 //
 // A row is read once, 16 bytes per load, and stays in registers as
 // exp(x/T - max): a thread has 8 consecutive logits of every 8192. Thresholds
-// are searched over the logits' own ordered bit patterns, so that 16 steps
-// (32-bit logits: 32) end on an exact logit: top-k counts what is not below
-// (one comparison per logit, a wave's count out of its mask), top-p adds it
-// up. A step costs one barrier.
+// are searched over the logits' own ordered bit patterns, by interpolation: top-k
+// counts what is not below (one comparison per logit, a wave's count out of its
+// mask), top-p adds it up. A step costs one barrier.
 //
-// Bound by the chain of steps; one row occupies a CU. On a MI355X, 192 rows
-// of 32000, a quarter each greedy and top-k, half top-p: 32 us (292 us with
-// the row in LDS, 256 threads and 24 halvings of the value range per
-// threshold). 256 rows of 65024: 27 us greedy, 89 without thresholds, 123
-// with them as above (87, 133, 594); registers spill from 32768 logits on.
+// Bound by the chain of steps; one row occupies a CU. us on a MI355X, from 16
+// (32) halvings a threshold, weights past 32768 made again for the draw and one
+// lane going through a run:
+//                                    greedy    no threshold  top-k 40  top-p .92
+//   192 x 32000                    5.6 -> 5.6  16.6 -> 11.5  28.5 22.7 32.3 20.9
+//   64 x 50272                     7.1 -> 6.4  54.7 -> 16.7  78.1 30.5 75.9 29.2
+//   256 x 65024                   17.7 -> 9.8  83.6 -> 35.0   118 53.6  109 48.6
+//   192 x 32000 in 32 bits         5.7 -> 5.8  16.6 -> 11.9  40.0 22.7 45.4 38.3
+// (the last but one is short of registers for ten rounds of eight weights).
 #include "common.h"
 
 #define SBLOCK 1024
@@ -20,53 +23,70 @@
 #define SVEC 8                    // consecutive logits of a thread per round
 #define SROUND (SBLOCK * SVEC)
 #define RUNS 256                  // runs of tokens that a draw's edges are of
+#define LIST 64                   // weights that share 16 bits of a logit
+#define SEG 320                   // tokens of a run, at most
 
 namespace {
 
 DEV_INLINE float val(const bf16_t& v) { return bf2f(v); }
 DEV_INLINE float val(const float& v) { return v; }
 
-// Ordered bit patterns: a <= b as floats just if key(a) <= key(b).
-template <class T> struct Key;
-template <> struct Key<bf16_t> {
-  static constexpr unsigned TOP = 0x8000u, ALL = 0xffffu;
-  DEV_INLINE static unsigned bits(float f) { return __float_as_uint(f) >> 16; }
-  DEV_INLINE static float number(unsigned b) { return __uint_as_float(b << 16); }
-};
-template <> struct Key<float> {
-  static constexpr unsigned TOP = 0x80000000u, ALL = 0xffffffffu;
-  DEV_INLINE static unsigned bits(float f) { return __float_as_uint(f); }
-  DEV_INLINE static float number(unsigned b) { return __uint_as_float(b); }
-};
-template <class T> DEV_INLINE unsigned key_of(float f) {
-  const unsigned b = Key<T>::bits(f);
-  return b & Key<T>::TOP ? Key<T>::ALL ^ b : b | Key<T>::TOP;
+// The high halves of ordered bit patterns: a <= b as floats means that key16(a)
+// <= key16(b), of bf16 numbers just then. And the least number that has one.
+DEV_INLINE unsigned key16_of(float f) {
+  const unsigned b = __float_as_uint(f);
+  return (b & 0x80000000u ? ~b : b | 0x80000000u) >> 16;
 }
-template <class T> DEV_INLINE float of_key(unsigned k) {
-  return Key<T>::number(k & Key<T>::TOP ? k ^ Key<T>::TOP : Key<T>::ALL ^ k);
+template <class T> DEV_INLINE float number16(unsigned k) {
+  const unsigned u = k << 16;
+  // (of negative numbers the one whose other bits are set, as keys count)
+  return __uint_as_float(u & 0x80000000u ? u ^ 0x80000000u
+                         : sizeof(T) == 4 ? ~u : ~u & 0xffff0000u);
 }
 
-// VEC: the row is whole 16-byte pieces, of which each is there or not.
-template <class T, bool VEC>
-DEV_INLINE void load8(const T* row, int at, int vocab, float v[SVEC]) {
-  constexpr int PER = 16 / sizeof(T);
-  #pragma unroll
-  for (int p = 0; p < SVEC; p += PER) {
+// Eight logits as they are stored: half the registers of their numbers, if of
+// 16 bits. Past the row's end: -inf.
+template <class T> struct Eight {
+  static constexpr int WORDS = SVEC * sizeof(T) / 4;
+  unsigned w[WORDS];
+
+  // VEC: the row is whole 16-byte pieces, of which each is there or not.
+  template <bool VEC>
+  DEV_INLINE void load(const T* row, int at, int vocab) {
+    constexpr int PER = 16 / sizeof(T);
+    constexpr unsigned NONE = sizeof(T) == 4 ? 0xff800000u : 0xff80ff80u;
     if constexpr (VEC) {
-      const int from = at + p < vocab ? at + p : 0;
-      const uint4v u = *reinterpret_cast<const uint4v*>(row + from);
       #pragma unroll
-      for (int j = 0; j < PER; ++j)
-        v[p + j] = at + p >= vocab ? -INFINITY
-            : sizeof(T) == 4 ? __uint_as_float(u[j % 4])
-            : __uint_as_float(j & 1 ? u[j / 2] & 0xffff0000u : u[j / 2] << 16);
+      for (int p = 0; p < SVEC; p += PER) {
+        const uint4v u = *reinterpret_cast<const uint4v*>(
+            row + (at + p < vocab ? at + p : 0));
+        #pragma unroll
+        for (int i = 0; i < 4; ++i)
+          w[p / PER * 4 + i] = at + p < vocab ? u[i] : NONE;
+      }
     } else {
       #pragma unroll
-      for (int j = 0; j < PER; ++j)
-        v[p + j] = at + p + j < vocab ? val(row[at + p + j]) : -INFINITY;
+      for (int i = 0; i < WORDS; ++i) {
+        if constexpr (sizeof(T) == 4) {
+          w[i] = at + i < vocab ? __float_as_uint(val(row[at + i])) : NONE;
+        } else {
+          unsigned half[2];
+          #pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int from = at + i * 2 + j;
+            half[j] = from < vocab
+                ? __float_as_uint(val(row[from])) >> 16 : NONE >> 16;
+          }
+          w[i] = half[0] | half[1] << 16;
+        }
+      }
     }
   }
-}
+  DEV_INLINE float operator[](int j) const {
+    if constexpr (sizeof(T) == 4) return __uint_as_float(w[j]);
+    return __uint_as_float(j & 1 ? w[j / 2] & 0xffff0000u : w[j / 2] << 16);
+  }
+};
 
 // The sum over the workgroup, in all threads: one barrier, and the next call
 // takes the other half of the scratch.
@@ -93,6 +113,11 @@ struct Totals {
   }
 };
 
+// What the wave has written to LDS may be read by all of its lanes.
+DEV_INLINE void wait_lds() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
 // NR: rounds of 8192 logits that cover the row
 template <class T, int NR, bool VEC>
 __global__ __launch_bounds__(SBLOCK)
@@ -112,16 +137,19 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   const float temp = temperature[b];
 
   // the largest logit; the smallest index of several. NaN is passed over.
-  float e[NR][SVEC];
-  float best = -INFINITY;
+  Eight<T> raw[NR];
+  float best = -INFINITY, least = INFINITY;
   int besti = 0x7fffffff;
   #pragma unroll
   for (int r = 0; r < NR; ++r) {
     const int at = r * SROUND + tid * SVEC;
-    load8<T, VEC>(row, at, vocab, e[r]);
+    raw[r].template load<VEC>(row, at, vocab);
     #pragma unroll
-    for (int j = 0; j < SVEC; ++j)
-      if (e[r][j] > best) { best = e[r][j]; besti = at + j; }
+    for (int j = 0; j < SVEC; ++j) {
+      const float v = raw[r][j];
+      if (v > best) { best = v; besti = at + j; }
+      least = fminf(least, v > -INFINITY ? v : INFINITY);
+    }
   }
 
   // ---- greedy ---------------------------------------------------------
@@ -157,26 +185,15 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
     const float x = v * inv_t, below = __expf(x - m);
     return v == top ? 1.f : x < past ? below : 0.f;
   };
+  float e[NR][SVEC];
   #pragma unroll
   for (int r = 0; r < NR; ++r)
     #pragma unroll
     for (int j = 0; j < SVEC; ++j) {
-      const int at = r * SROUND + tid * SVEC + j;
-      e[r][j] = at < vocab ? weight(e[r][j]) : -1.f;    // -1: not a token
-      // one after the other, or their parts take the registers of the row
-      __builtin_amdgcn_sched_barrier(0);
+      e[r][j] = weight(raw[r][j]);      // past the row's end: as of -inf
+      // a few at a time, or their parts take the registers of the row
+      if (j % (NR <= 4 ? 4 : 1) == 0) __builtin_amdgcn_sched_barrier(0);
     }
-  const unsigned first = key_of<T>(-INFINITY), last = key_of<T>(top);
-  // the largest key whose logits and all above them satisfy enough(their
-  // weight's threshold)
-  auto search = [&](auto enough) {
-    unsigned lo = first, hi = last + 1;     // holds at lo, not at hi
-    while (hi - lo > 1) {
-      const unsigned mid = lo + (hi - lo) / 2;
-      if (enough(weight(of_key<T>(mid)))) lo = mid; else hi = mid;
-    }
-    return lo;
-  };
   auto sum_from = [&](float t) {
     float s = 0.f;
     #pragma unroll
@@ -187,34 +204,167 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
     }
     return totals.add(wave_sum(s));
   };
+  auto count_from = [&](float t) {
+    int n = 0;
+    #pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      #pragma unroll
+      for (int j = 0; j < SVEC; ++j) n += __popcll(__ballot(e[r][j] >= t));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return totals.add((float)n);
+  };
+
+  // Two of the 65536 keys of 16 bits between which a threshold lies:
+  // measure(weight) holds at lo, not at hi. They are neighbours, or the tokens
+  // from lo on, less those from hi on, are no more than LIST. A step's key is where a line
+  // between what was measured at either end, by logits, meets the goal, every
+  // third one half way, by logits or by keys (so that it ends). An end that
+  // stays is moved half way to the goal. 5 to 7 steps on average, 13 at most,
+  // for 32000 logits of one to five units' deviation.
+  const unsigned first = key16_of(-INFINITY), last = key16_of(top);
+  struct Measured { bool holds; float f, n; };
+  struct Ends { unsigned lo, hi; float above; };   // tokens from hi on
+  constexpr float MANY = 1e9f;
+  auto search = [&](auto measure, float goal, float xl, float fl, float fh) {
+    unsigned lo = first, hi = last + 1;
+    float xh = top, nl = MANY, nh = 0.f;
+    int side = 0;
+    for (int turn = 0; hi - lo > 1 && nl - nh > (float)LIST; turn = turn == 5 ? 0 : turn + 1) {
+      unsigned mid = lo + (hi - lo) / 2;
+      if (turn != 5) {
+        const float x = turn == 2
+            ? (xl + xh) * 0.5f
+            : xl + (xh - xl) * (fl - goal) * __builtin_amdgcn_rcpf(fl - fh);
+        mid = min(max(key16_of(x), lo + 1), hi - 1);
+      }
+      const float x = number16<T>(mid);
+      const Measured got = measure(weight(x));
+      if (got.holds) {
+        lo = mid;
+        xl = x;
+        fl = got.f;
+        nl = got.n;
+        if (side == 1) fh = goal + (fh - goal) * 0.5f;
+        side = 1;
+      } else {
+        hi = mid;
+        xh = x;
+        fh = got.f;
+        nh = got.n;
+        if (side == 2) fl = goal + (fl - goal) * 0.5f;
+        side = 2;
+      }
+    }
+    return Ends{lo, hi, nh};
+  };
+  // The weights between low and high, sorted out by the first wave's lanes: a
+  // lane has one (0: none), how many there are of that and more, and their sum.
+  // pick(those) in all threads, or -1 where there are more than LIST.
+  __shared__ float s_list[LIST], s_pick;
+  __shared__ int s_listed;
+  auto between = [&](float low, float high, auto pick) {
+    if (tid == 0) s_listed = 0;
+    __syncthreads();
+    #pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      #pragma unroll
+      for (int j = 0; j < SVEC; ++j)
+        if (e[r][j] >= low && e[r][j] < high) {
+          const int at = atomicAdd(&s_listed, 1);
+          if (at < LIST) s_list[at] = e[r][j];
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    const int listed = s_listed;
+    if (listed > LIST) return -1.f;
+    if (wave == 0) {
+      const float w = lane < listed ? s_list[lane] : 0.f;
+      float n = 0.f, sum = 0.f;
+      #pragma unroll 4
+      for (int i = 0; i < listed; ++i) {
+        const float other = __uint_as_float(
+            __builtin_amdgcn_readlane(__float_as_uint(w), i));
+        n += other >= w ? 1.f : 0.f;
+        sum += other >= w ? other : 0.f;
+      }
+      const float picked = pick(w, n, sum);
+      if (lane == 0) s_pick = picked;
+    }
+    __syncthreads();
+    return s_pick;
+  };
+  // the last weight of [low, high) where holds is true, by halves of its bits
+  auto halves = [&](auto holds, float low, float high) {
+    unsigned lo = __float_as_uint(low), hi = __float_as_uint(high);
+    while (hi - lo > 1) {
+      const unsigned mid = lo + (hi - lo) / 2;
+      if (holds(__uint_as_float(mid))) lo = mid; else hi = mid;
+    }
+    return __uint_as_float(lo);
+  };
+  constexpr bool EXACT = sizeof(T) == 2;        // 16 bits are all of them
 
   // ---- top-k: as many largest as are no more than k with all their equals,
-  // ---- the largest and its equals in any case
-  float thresh = 0.f;
+  // ---- the largest and its equals in any case. Measured: tokens' logarithm
+  float thresh = 0.f, floor = -INFINITY;
   const int k = top_k[b];
   if (k > 0 && k < vocab) {
-    const unsigned more = search([&](float t) {
-      int n = 0;
-      #pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        #pragma unroll
-        for (int j = 0; j < SVEC; ++j)
-          n += __popcll(__ballot(e[r][j] >= t));
-        __builtin_amdgcn_sched_barrier(0);
+    const float from =
+        fmaxf(-totals.most(wave_max(-least)), top - 60.f * temp);
+    const Ends at = search([&](float t) {
+      const float n = count_from(t);
+      return Measured{n > (float)k, __logf(fmaxf(n, 0.5f)), n};
+    }, __logf((float)k + 0.5f), from, __logf((float)vocab), __logf(0.5f));
+    if (EXACT && at.hi - at.lo == 1) {
+      floor = number16<T>(min(at.hi, last));
+      thresh = weight(floor);
+    } else {
+      floor = number16<T>(at.lo);
+      const float low = weight(floor), high = weight(number16<T>(at.hi));
+      // the smallest that are kept
+      float t = between(low, high, [&](float w, float n, float) {
+        return -wave_max(w > 0.f && at.above + n <= (float)k ? -w : -high);
+      });
+      if (t < 0.f) {
+        t = halves([&](float t) { return count_from(t) > (float)k; }, low,
+                   high);
+        t = __uint_as_float(__float_as_uint(t) + 1);
       }
-      return totals.add((float)n) > (float)k;
-    });
-    thresh = weight(of_key<T>(min(more + 1, last)));
+      thresh = fminf(t, 1.f);
+    }
   }
 
-  // ---- top-p: the fewest largest weights with that share ----------------
+  // ---- top-p: the fewest largest weights with that share. Measured: the
+  // ---- logarithm of what is left out, which a goal's share of the tokens at
+  // ---- most has if each weighs no more than at the first key
   const float p_target = top_p[b];
   if (p_target > 0.f && p_target < 1.f) {
-    const float goal = p_target * sum_from(thresh);
-    const float low = thresh;
-    thresh = fmaxf(low, weight(of_key<T>(search([&](float t) {
-      return t < low || sum_from(t) >= goal;
-    }))));
+    const float all = sum_from(thresh), goal = p_target * all;
+    const float out = all - goal, low = thresh;
+    auto enough = [&](float t) { return t < low || sum_from(t) >= goal; };
+    const unsigned lo = search([&](float t) {
+      if (t < low) return Measured{true, __logf(out) - 2.f, MANY};
+      const float s = sum_from(t);
+      return Measured{s >= goal, __logf(fmaxf(all - s, 1e-3f * out)),
+                      s >= goal ? MANY : 0.f};
+    }, __logf(out), fmaxf(floor, top - __logf((float)vocab / out) * temp),
+       __logf(out) - 2.f, __logf(all)).lo;
+    thresh = fmaxf(low, weight(number16<T>(lo)));
+    if constexpr (!EXACT) {
+      const float high = weight(number16<T>(lo + 1)), above = sum_from(high);
+      // a sum in another order may be off by its last bits
+      const float start = thresh;
+      const float t = between(start, high, [&](float w, float, float sum) {
+        return wave_max(w > 0.f && above + sum >= goal ? w : start);
+      });
+      if (t < 0.f || !enough(t) ||
+          enough(__uint_as_float(__float_as_uint(t) + 1)))
+        thresh = fmaxf(low, halves(enough, thresh, high));
+      else
+        thresh = fmaxf(low, t);
+    }
   }
 
   // ---- inverse-CDF draw, in token order ---------------------------------
@@ -222,53 +372,46 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   // two-hundredth draw from thousands of tokens lies that close to an edge. So
   // that a row and a number keep their token, the sum is that of 256 threads
   // over every 256th token, the edges those of 256 runs of tokens, added up
-  // from left to right, as they always were (2 us of the 32 above).
-  constexpr bool KEPT = NR <= 4;      // weights fit LDS; else made again, out
-  constexpr int RAW = KEPT || sizeof(T) == 4    // of logits where those do
-      ? 1 : NR * SROUND < 77824 ? NR * SROUND : 77824;
-  __shared__ float s_w[KEPT ? NR * SROUND : 1];
-  __shared__ T s_raw[RAW];
-  __shared__ float s_run[RUNS];
-  if constexpr (KEPT) {
+  // from left to right, as they always were.
+  constexpr int PART = NR < 4 ? NR : 4;     // rounds whose weights fit LDS
+  __shared__ alignas(16) float s_w[PART * SROUND];
+  __shared__ alignas(16) float s_run[RUNS];
+  __shared__ alignas(16) float s_one[SEG];
+  const int run = (vocab + RUNS - 1) / RUNS;
+  const int from = (tid - RUNS) * run;
+  float sum = 0.f;
+  #pragma unroll
+  for (int r0 = 0; r0 < NR; r0 += PART) {
+    if (r0 > 0) __syncthreads();
     #pragma unroll
-    for (int r = 0; r < NR; ++r) {
+    for (int r = r0; r < NR && r < r0 + PART; ++r) {
       float4 w[2];
       float* f = reinterpret_cast<float*>(w);
       #pragma unroll
       for (int j = 0; j < SVEC; ++j) f[j] = e[r][j] >= thresh ? e[r][j] : 0.f;
-      float4* to = reinterpret_cast<float4*>(s_w + r * SROUND + tid * SVEC);
+      float4* to =
+          reinterpret_cast<float4*>(s_w + (r - r0) * SROUND + tid * SVEC);
       to[0] = w[0];
       to[1] = w[1];
     }
-  } else if constexpr (RAW > 1) {
-    #pragma unroll 8
-    for (int i = tid; i < min(vocab, RAW); i += SBLOCK) s_raw[i] = row[i];
-  }
-  if (tid == 0) s_tok = -1;
-  __syncthreads();
-  auto kept_weight = [&](int i) {
-    if constexpr (KEPT) {
-      return s_w[i];
-    } else {
-      const float w =
-          weight(val(RAW > 1 && i < RAW ? s_raw[i] : row[i]));
-      return w >= thresh ? w : 0.f;
+    __syncthreads();
+    const int base = r0 * SROUND, end = min(vocab, base + PART * SROUND);
+    if (tid < RUNS) {
+      #pragma unroll 16
+      for (int i = base + tid; i < end; i += RUNS) sum += s_w[i - base];
+    } else if (tid < 2 * RUNS) {
+      const int stop = min(from + run, end);
+      #pragma unroll 16
+      for (int i = max(from, base); i < stop; ++i) sum += s_w[i - base];
     }
-  };
-  const int run = (vocab + RUNS - 1) / RUNS;
+  }
   if (tid < RUNS) {
-    float sum = 0.f;
-    #pragma unroll 16
-    for (int i = tid; i < vocab; i += RUNS) sum += kept_weight(i);
     sum = wave_sum(sum);
     if (lane == 0) s_tot[0][wave] = sum;
   } else if (tid < 2 * RUNS) {
-    const int from = (tid - RUNS) * run, end = min(from + run, vocab);
-    float sum = 0.f;
-    #pragma unroll 16
-    for (int i = from; i < end; ++i) sum += kept_weight(i);
     s_run[tid - RUNS] = sum;
   }
+  if (tid == 0) s_tok = -1;
   __syncthreads();
   if (wave == 0) {
     float z = 0.f;
@@ -276,39 +419,59 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
     for (int q = 0; q < RUNS / WAVE; ++q) z += s_tot[0][q];
     const float goal = uniform[b] * z;
     constexpr int EACH = RUNS / WAVE;
-    float mine[EACH], edge[EACH], before = 0.f, upto = 0.f;
-    #pragma unroll
-    for (int q = 0; q < EACH; ++q) mine[q] = s_run[lane * EACH + q];
+    static_assert(EACH == 4);
+    // edges from left to right: every lane goes over all of them, and keeps
+    // what there is before its four
+    float before = 0.f, upto = 0.f;
+    #pragma unroll 8
     for (int l = 0; l < WAVE; ++l) {
-      if (lane == l) before = upto;
-      #pragma unroll
-      for (int q = 0; q < EACH; ++q) {
-        upto += __uint_as_float(
-            __builtin_amdgcn_readlane(__float_as_uint(mine[q]), l));
-        if (lane == l) edge[q] = upto;
-      }
+      const float4 x = reinterpret_cast<const float4*>(s_run)[l];
+      before = lane == l ? upto : before;
+      upto = upto + x.x + x.y + x.z + x.w;
     }
+    int hit = -1;
+    float acc = 0.f;
     #pragma unroll
     for (int q = 0; q < EACH; ++q) {
-      if (goal >= before && goal < edge[q]) {
-        const int from = (lane * EACH + q) * run;
-        const int end = min(from + run, vocab);
-        float acc = before;
-        int sel = -1;
-        for (int i = from; i < end && sel < 0; i += 8) {
-          float w[8];
-          #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            w[j] = i + j < end ? kept_weight(i + j) : 0.f;
-          #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            acc += w[j];
-            if (sel < 0 && w[j] > 0.f && acc > goal) sel = i + j;
+      const float edge = before + s_run[lane * EACH + q];
+      const unsigned long long here = __ballot(goal >= before && goal < edge);
+      if (here) {
+        const int l = __ffsll(here) - 1;
+        hit = l * EACH + q;
+        acc = __shfl(before, l, WAVE);
+      }
+      before = edge;
+    }
+    if (hit >= 0) {
+      // the run's weights, and how many of its sums the goal is not below
+      const int first = hit * run, end = min(first + run, vocab);
+      for (int i = lane; i < SEG; i += WAVE) {
+        float w = 0.f;
+        if (first + i < end) {
+          if constexpr (NR <= PART) {
+            w = s_w[first + i];
+          } else {
+            w = weight(val(row[first + i]));
+            w = w >= thresh ? w : 0.f;
           }
         }
-        if (sel >= 0) s_tok = sel;
+        s_one[i] = w;
       }
-      before = edge[q];
+      wait_lds();
+      int n = 0;
+      for (int i = 0; i < run && acc <= goal; i += 16) {
+        float4 w[4];
+        #pragma unroll
+        for (int j = 0; j < 4; ++j)
+          w[j] = reinterpret_cast<const float4*>(s_one + i)[j];
+        const float* f = reinterpret_cast<const float*>(w);
+        #pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          acc += f[j];
+          n += acc <= goal ? 1 : 0;
+        }
+      }
+      if (lane == 0 && first + n < end) s_tok = first + n;
     }
   }
   __syncthreads();
@@ -318,11 +481,8 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   }
   // rounding at the very end (goal ~ z): the last token that may be drawn
   int kept = -1;
-  #pragma unroll
-  for (int r = 0; r < NR; ++r)
-    #pragma unroll
-    for (int j = 0; j < SVEC; ++j)
-      if (e[r][j] >= thresh) kept = r * SROUND + tid * SVEC + j;
+  for (int i = tid; i < vocab; i += SBLOCK)
+    if (weight(val(row[i])) >= thresh) kept = i;
   #pragma unroll
   for (int off = 32; off > 0; off >>= 1)
     kept = max(kept, __shfl_xor(kept, off, WAVE));

@@ -106,3 +106,38 @@ def test_neighbouring_numbers_share_the_draws(temp, k, p):
         got = ops.softmax_sample(rows.to(DEV), of(temp),
                                  of(k, dtype=torch.int32), of(p), of(u))
         assert got.tolist() == [token] * n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k,p", [(3, 1.0), (200, 1.0), (0, 0.6), (500, 0.97)])
+@pytest.mark.parametrize("kind", ["close", "equal", "steps", "below zero"])
+def test_thresholds_among_like_weights(dtype, k, p, kind):
+    """Many logits that share their upper 16 bits, or all of them, where a
+    threshold lies: more, and fewer, than are sorted out at once."""
+    n, vocab = 24, 9000
+    g = torch.Generator().manual_seed(k + vocab)
+    x = torch.randn(n, vocab, generator=g)
+    if kind == "close":
+        x = 4 + x * 1e-3
+    elif kind == "equal":
+        x = torch.where(torch.rand(n, vocab, generator=g) < 0.01, 5.0, 3.0)
+    elif kind == "steps":
+        # a step's 1000 to 3600 tokens are 3e-5 apart, some 2^-20 of a logit
+        # near 4: weights of 32 bits still differ. (At 1e-4 a step they are
+        # not all told apart, and a threshold takes or leaves several.)
+        x = (x * 2).round() + torch.rand(n, vocab, generator=g) * 0.1
+    else:
+        x = -x.abs() * 8 - 0.1
+    x = x.to(dtype)
+    u = torch.rand(n, generator=g)
+    of = lambda v: torch.full((n,), v, device=DEV)
+    got = ops.softmax_sample(x.to(DEV), of(0.9), of(k).int(), of(p),
+                             u.to(DEV)).tolist()
+    for i in range(n):
+        keep, cum, goal = draw(x[i], 0.9, k, p, float(u[i]))
+        a = got[i]
+        # as above; a step of the sums may take or leave a weight at the edge
+        slack = 2e-5 * float(cum[-1])
+        assert bool(keep[a])
+        assert float(cum[a]) >= float(goal) - slack
+        assert a == 0 or float(cum[a - 1]) <= float(goal) + slack
