@@ -134,19 +134,21 @@ void moe_select_kernel(int* __restrict__ ids, float* __restrict__ weights,
 
 constexpr int SORT = 1024;      // threads, and most experts
 
-// inclusive sum over the workgroup
+// inclusive sum over the workgroup: of each wave by exchanges (ten rounds through
+// LDS took 1.5 us of 48 rows' 5.5)
 DEV_INLINE int scan(int v, int* s) {
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = 1; off < SORT; off <<= 1) {
-    const int add = (int)threadIdx.x >= off ? s[threadIdx.x - off] : 0;
-    __syncthreads();
-    s[threadIdx.x] += add;
-    __syncthreads();
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  #pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const int add = __shfl_up(v, off, WAVE);
+    if (lane >= off) v += add;
   }
-  const int r = s[threadIdx.x];
+  if (lane == WAVE - 1) s[wave] = v;
   __syncthreads();
-  return r;
+  #pragma unroll
+  for (int w = 0; w < SORT / WAVE; ++w) v += w < wave ? s[w] : 0;
+  __syncthreads();
+  return v;
 }
 
 __global__ __launch_bounds__(SORT)
@@ -154,7 +156,7 @@ void moe_sort_kernel(int* __restrict__ at, int* __restrict__ src,
                      int* __restrict__ start, int* __restrict__ tiles,
                      const int* __restrict__ ids, int n, int top, int experts,
                      int tile) {
-  __shared__ int s_n[SORT], s_scan[SORT];
+  __shared__ int s_n[SORT], s_scan[SORT / WAVE];
   const int t = threadIdx.x;
   s_n[t] = 0;
   __syncthreads();
