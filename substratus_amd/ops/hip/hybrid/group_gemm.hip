@@ -1,13 +1,21 @@
 // Grouped products (group_gemm.h) of few rows per group, and of any size:
 //
+//   rows     packed bf16 rows, up to 32 of a group: group_gemm_rows.hip.
 //   stream   bf16, few rows per group: bound by reading the weights once.
 //            Every wave takes a share of the inner dimension of a tile of
 //            rows and 64 columns (4 waves; 16 and 32 columns where there are
-//            few tiles; where the inner dimension is short, a share of the
-//            rows), with both operands going from memory
+//            few tiles; where the inner dimension is one step of loads, a
+//            share of the rows), with both operands going from memory
 //            straight into the matrix cores' registers (a fragment is 16
 //            consecutive bytes of a row, so nothing is gained by LDS); there
 //            is no barrier until the partial tiles are added up.
+//            us on a MI355X, 16 heads, from sharing the rows up to an inner
+//            size of 512, and what results are multiplied with fetched last:
+//              512 -> 128 each, gated: 48 rows 12.5 -> 5.6, 512 13.5 -> 9.9,
+//              1024 24.0 -> 16.0; 128 -> 512 with 64 copied: 6.8 -> 5.2, 19.0
+//              -> 13.9, 34.3 -> 25.0 (one block copied, element by element)
+//              48 x 256 x 2048, times a table's rows: 8.2 -> 6.4 (16 columns a
+//              workgroup instead of 32)
 //   any      float, and bf16 sizes whose rows are not 16-byte pieces.
 //
 // Weights are the first operand, so a lane ends up with four consecutive
@@ -61,6 +69,17 @@ void group_gemm_stream_kernel(GroupGemm<bf16_t, Y> a) {
   for (int i = 0; i < FN; ++i)
     #pragma unroll
     for (int j = 0; j < FM; ++j) acc[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
+
+  // the thread's four columns in the end: what they are multiplied with is on
+  // its way meanwhile
+  constexpr bool EARLY = KW > 1 && BM * BN / 4 <= KW * WAVE &&
+                         (ACT == Act::GATE || ACT == Act::SIDE);
+  const int er = t.r0 + threadIdx.x / (BN / 4),
+            en = n0 + threadIdx.x % (BN / 4) * 4;
+  const bool early = EARLY && a.quads && er < t.r1 && en < a.n;
+  float by[4] = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (EARLY)
+    if (early) act_operand<ACT, 4>(a, er, t.g, en, by);
 
   const int chunks = (a.k + KC - 1) / KC, shares = KW * a.splits,
             part = share * KW + (KW > 1 ? wave : 0);
@@ -121,11 +140,20 @@ void group_gemm_stream_kernel(GroupGemm<bf16_t, Y> a) {
       #pragma unroll
       for (int w = 0; w < KW; ++w)
         v += *reinterpret_cast<const float4v*>(&s_p[w][r][c]);
+      if constexpr (EARLY) {
+        if (a.quads) {
+          if (early) {
+            float f[4] = {v[0], v[1], v[2], v[3]};
+            act_with<ACT, true, 4>(f, by);
+            stv<4>(a.y + (long)er * a.y_ld + t.g * a.y_gs + en, f);
+          }
+          continue;
+        }
+      }
       store4<ACT>(a, t, t.r0 + r, n0 + c, v);
     }
   }
-  if (a.tail && blockIdx.x == 0)
-    copy_tail(a, t, threadIdx.x, KW * RW * WAVE);
+  if (a.tail) copy_tail(a, t, threadIdx.x, KW * RW * WAVE);
 }
 
 // 32 x 32 outputs per workgroup, 2 x 2 per thread, operands through LDS.
@@ -175,7 +203,7 @@ void group_gemm_any_kernel(GroupGemm<T, Y> a) {
         st1(a.y + (long)r * a.y_ld + t.g * a.y_gs + n, acc[i][j]);
       }
     }
-  if (a.tail && blockIdx.x == 0) copy_tail(a, t, threadIdx.x, 256);
+  if (a.tail) copy_tail(a, t, threadIdx.x, 256);
 }
 
 // rows of both operands are whole, aligned 16-byte pieces
@@ -224,6 +252,17 @@ bool by_quads(const GroupGemm<T, Y>& a) {
 }
 
 template <class T, class Y>
+bool by_eights(const GroupGemm<T, Y>& a) {
+  auto ok = [](const void* p) {
+    return reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  };
+  return sizeof(T) == 2 && sizeof(Y) == 2 && a.tail % 8 == 0 &&
+         a.n % 8 == 0 && a.k % 8 == 0 && a.x_ld % 8 == 0 &&
+         a.x_gs % 8 == 0 && a.y_ld % 8 == 0 && a.y_gs % 8 == 0 && ok(a.x) &&
+         ok(a.y);
+}
+
+template <class T, class Y>
 int group_gemm_splits(const GroupGemm<T, Y>& a) {
   if constexpr (std::is_same_v<T, bf16_t>) {
     if (!pieces(a) || a.tiles != nullptr || a.groups != 1) return 1;
@@ -240,6 +279,7 @@ void launch_group_gemm(const GroupGemm<T, Y>& given, int tile,
                        hipStream_t stream) {
   GroupGemm<T, Y> a = given;
   a.quads = by_quads(a);
+  a.tail_eights = by_eights(a);
   const bool packed = a.tiles != nullptr, split = a.splits > 1;
   const int gz = packed ? 1 : split ? a.splits : a.groups;
   if (split) tile = 16;
@@ -254,7 +294,12 @@ void launch_group_gemm(const GroupGemm<T, Y>& given, int tile,
         launch_group_gemm_tile(a, tile, stream);
         return;
       }
-      const bool flat = !packed && a.k <= 512 && tile == 64;
+      if (group_gemm_rows_takes(a, tile)) {
+        launch_group_gemm_rows(a, tile, stream);
+        return;
+      }
+      // an inner size of one step of loads: waves share the rows instead
+      const bool flat = !packed && a.k <= 4 * KC && tile == 64;
       auto groups = [&](int bn) {
         return (long)((a.n + bn - 1) / bn) *
                (packed ? a.max_tiles : (a.m + tile - 1) / tile) * gz;
@@ -277,6 +322,8 @@ void launch_group_gemm(const GroupGemm<T, Y>& given, int tile,
       constexpr std::integral_constant<int, 16> c16{};
       if (split) go(c1, c2, c4, c1);
       else if (flat) go(c1, c4, c1, c4);
+      else if (tile == 16 && groups(32) < 128 && a.k >= 1024)
+        go(c1, c1, c16, c1);
       else if (tile == 16 && groups(64) < 256 && a.k >= 1024)
         go(c1, c2, c16, c1);
       else if (tile == 16) go(c1, c4, c4, c1);

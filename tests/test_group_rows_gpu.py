@@ -1,0 +1,81 @@
+"""Grouped products of few rows: ends of stages, rings, tiles and columns, tails
+copied by pieces, gates fetched ahead, against the products in 64 bits."""
+
+import pytest
+import torch
+
+from substratus_amd.ops import hybrid as ops
+from test_hybrid_ops_gpu import close, rand
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+@pytest.mark.parametrize("tile", [16, 32])
+@pytest.mark.parametrize("k,n,act", [(128, 16, "none"), (160, 44, "gelu"),
+                                     (1056, 24, "silu"), (2080, 72, "none"),
+                                     (2048, 8, "gelu")])
+def test_experts_of_few_rows(tile, k, n, act):
+    counts = [1, 15, 0, 16, 17, 31, 32, 33, 2]
+    total, e = sum(counts), len(counts)
+    g = torch.Generator().manual_seed(k + n)
+    ids = torch.repeat_interleave(torch.arange(e), torch.tensor(counts))
+    ids = ids[torch.randperm(total, generator=g)].int()[:, None].contiguous()
+    x = rand(total, k, seed=1, dtype=BF16)
+    w = rand(e, n, k, seed=2, dtype=BF16, scale=k ** -0.5)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    at, src = torch.empty(total, 1, **i32), torch.empty(total, **i32)
+    start = torch.empty(e + 1, **i32)
+    tiles = torch.empty(1 + 2 * ((total + tile - 1) // tile + e), **i32)
+    ext = ops._ext()
+    ext.moe_sort(at, src, start, tiles, ids.cuda(), tile)
+    assert start.tolist() == torch.tensor([0] + counts).cumsum(0).tolist()
+    cols = n // 2 if act == "silu" else n
+    out = torch.full((total, cols), 9.0, dtype=BF16, device="cuda")
+    ext.expert_linear(out, x.cuda(), w.cuda(), src, start, tiles, tile, act,
+                      0.0)
+    want = torch.empty(total, cols, dtype=torch.float64)
+    for i in range(e):
+        r = ids[:, 0] == i
+        y = x[r].double() @ w[i].double().T
+        if act == "gelu":
+            y = torch.nn.functional.gelu(y)
+        if act == "silu":           # columns are gate and up in turn
+            y = torch.nn.functional.silu(y[:, ::2]) * y[:, 1::2]
+        want[r] = y
+    close(out[at[:, 0].long()], want.float(), BF16)
+
+
+@pytest.mark.parametrize("rows", [1, 16, 48, 65, 300])
+@pytest.mark.parametrize("k,n,tail,each", [(512, 128, 0, True),
+                                           (512, 72, 0, False),
+                                           (128, 512, 64, None),
+                                           (256, 40, 24, True),
+                                           (128, 64, 12, None)])
+def test_heads_of_few_rows(rows, k, n, tail, each):
+    heads = 3
+    x = rand(rows, heads * (k + tail), seed=1, dtype=BF16)
+    w = rand(heads, n, k, seed=2, dtype=BF16, scale=k ** -0.5)
+    gate = None if each is None else rand(
+        rows, heads * n if each else heads, seed=3, dtype=BF16)
+    v = x.view(rows, heads, k + tail)
+    got = ops.head_linear(v.cuda(), w.cuda(),
+                          None if gate is None else gate.cuda(), tail)
+    want = torch.einsum("rhk,hnk->rhn", v[..., :k].double(), w.double())
+    if gate is not None:
+        want *= torch.sigmoid(gate.double().view(rows, heads, -1))
+    close(got[..., :n], want.float(), BF16)
+    assert torch.equal(got[..., n:].cpu(), v[..., k:])
+
+
+@pytest.mark.parametrize("rows", [1, 17, 48])
+def test_side_gate_of_few_columns(rows):
+    y = rand(rows, 1088, seed=1, dtype=BF16)
+    w = rand(40, 1088, seed=2, dtype=BF16, scale=1088 ** -0.5)
+    table = rand(50, 80, seed=3, dtype=BF16)
+    tok = torch.randint(0, 50, (rows,), dtype=torch.int32)
+    got = ops.side_gate(y.cuda(), w.cuda(), tok.cuda(), table.cuda(), 40)
+    want = torch.nn.functional.gelu(y.double() @ w.double().T,
+                                    approximate="tanh") \
+        * table[tok.long(), 40:].double()
+    close(got, want.float(), BF16)
