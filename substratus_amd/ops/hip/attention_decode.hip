@@ -982,11 +982,25 @@ int paged_attn_nsplit(int bsz, int hq, int hkv, int d, int max_blocks,
 
 // The same for the kernel that takes a call. waves: 0, or those of a workgroup
 // for a single head where no kernel takes several of a group together.
+// Grouped heads: two workgroups fit a CU, and no more shares than let each have
+// one. us, MI355X, heads on key heads, keys at most, from 1024 workgroups to this
+// (shares):
+//   64 sequences, 32 on 8 of 128, 2500   89.4 -> 83.9 (2, 1)    600  32.5 -> 26.5
+//   24, the same, 2500                   47.3 -> 43.0 (6, 2)
+//   64, 64 on 8, 1500                    62.0 -> 55.3 (2, 1)
+//   16, 64 on 8, 2000                    30.3 -> 26.3 (8, 4)
+//   40, 128 on 8 of 64, 800              19.8 -> 18.1 (4, 1)
+//   8, 32 on 8, 4000                     30.1 -> 26.1 (16, 8)
 int paged_attn_plan(int bsz, int hq, int hkv, int d, int max_blocks,
                     bool grouped, int& waves) {
   waves = 0;
   int nsplit;
-  if (grouped || gqa_hpw(hq, hkv, d) > 0 || hq / hkv % 8 == 0)
+  if (grouped) {
+    const long base = (long)bsz * hkv * ((hq / hkv + 15) / 16);
+    return std::min(paged_attn_nsplit(bsz, hq, hkv, d, max_blocks, true),
+                    (int)std::max(512 / std::max(base, 1L), 1L));
+  }
+  if (gqa_hpw(hq, hkv, d) > 0 || hq / hkv % 8 == 0)
     return paged_attn_nsplit(bsz, hq, hkv, d, max_blocks, grouped);
   attn_heads_plan(bsz, hq, d, max_blocks, waves, nsplit);
   return nsplit;
