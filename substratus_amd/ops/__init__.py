@@ -282,8 +282,14 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
     if not (x.is_cuda and weight.is_cuda and x.device == weight.device
             and x.dtype == weight.dtype == torch.bfloat16 and x.dim() >= 1
             and weight.dim() == 2 and x.shape[-1] == weight.shape[1]
-            and x.numel() > 0
-            and _rows_gemm_pays(x.numel(), *weight.shape)):
+            and x.numel() > 0):
+        return None
+    n, k = weight.shape
+    # larger matrices' rows by mid_gemm.hip, in the same call
+    if not (_rows_gemm_pays(x.numel(), n, k)
+            or x.numel() <= 256 * k and not _compiling()
+            and _load_ext() is not None
+            and _load_ext().mid_gemm_good(x.numel() // k, n, k, gated)):
         return None
     if bias is not None and not (bias.dtype == torch.bfloat16
                                  and bias.device == x.device
@@ -294,7 +300,6 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
     ext = _load_ext()
     if ext is None or not inference_only(*given):
         return None
-    n, k = weight.shape
     if x.dim() != 2:
         x = x.reshape(-1, k)
     if not (ext.rows_gemm_ok(x.shape[0], n, k, gated)
@@ -396,7 +401,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """F.linear. Up to 16 rows of bf16 without gradients, or up to 64 with a
     matrix of few rows, take the kernel that streams weights at the memory's
-    rate (rows_gemm.hip), products of 256 rows and more the one for the matrix
+    rate (rows_gemm.hip), up to 256 rows the one for tiles of them where the
+    library's are too few (mid_gemm.hip), products of 256 rows and more the one for the matrix
     cores (tile_gemm.hip) where that is the faster one, in a backward as well.
     SUB_MGEMM=1 routes decode shapes of 256 rows and more to the 256x256 glds
     GEMM (mfma_gemm.hip).

@@ -13,6 +13,7 @@
 
 #include "optimizer.h"
 #include "rows_quant.h"
+#include "mid_gemm.h"
 #include "tile_gemm.h"
 
 typedef __hip_bfloat16 bf16_t;
@@ -579,10 +580,15 @@ long mfma_gemm_pick_splitk(long m, long n, long k) {
   return mfma_gemm_splitk((int)m, (int)n, (int)k);
 }
 
-// y = x w^T + bias, at most 64 rows of x; gated: y has half the columns,
-// silu(first half) * second half
+// y = x w^T + bias, at most 64 rows of x, or up to 256 where that is faster than
+// the library; gated: y has half the columns, silu(first half) * second half
+bool mid_gemm_good(long m, long n, long k, bool paired) {
+  return mid_gemm_takes(m, n, k, paired) && mid_gemm_pays(m, n, k, paired);
+}
+
 bool rows_gemm_ok(long m, long n, long k, bool gated) {
-  return rows_gemm_takes((int)m, (int)n, (int)k, gated);
+  return mid_gemm_good(m, n, k, gated) ||
+         rows_gemm_takes((int)m, (int)n, (int)k, gated);
 }
 
 // Where the columns of a projection of heads go: queries to q [rows, hq, d],
@@ -640,7 +646,8 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const int cols = heads ? n - 2 * heads->hkv * heads->d : gated ? n / 2 : n;
   TORCH_CHECK(w.dim() == 2 && w.size(1) == k && y.size(0) == m &&
               y.numel() == (long)m * cols, "rows_gemm: shape mismatch");
-  TORCH_CHECK(rows_gemm_takes(m, n, k, gated || heads),
+  const bool many = norm == nullptr && mid_gemm_good(m, n, k, gated || heads);
+  TORCH_CHECK(many || rows_gemm_takes(m, n, k, gated || heads),
               "rows_gemm: unsupported shape ", m, "x", n, "x", k);
   TORCH_CHECK(aligned16(x) && aligned16(w), "rows_gemm: misaligned operand");
   const bf16_t* bp = nullptr;
@@ -649,8 +656,20 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
     TORCH_CHECK(bias->numel() == n, "bias size");
     bp = bfc(*bias);
   }
-  launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols,
-                   gated, heads, norm, stream());
+  if (many) {
+    const MidPlan plan = mid_gemm_plan(m, n, k);
+    torch::Tensor part;
+    if (plan.shares(m, n))
+      part = torch::empty({plan.shares(m, n)},
+                          x.options().dtype(torch::kFloat));
+    launch_mid_gemm({bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols},
+                    plan, heads, gated,
+                    plan.shares(m, n) ? part.data_ptr<float>() : nullptr,
+                    stream());
+  } else {
+    launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols,
+                     gated, heads, norm, stream());
+  }
   post_launch_check("rows_gemm");
 }
 
@@ -1054,6 +1073,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_split_append", &rope_split_append);
   m.def("quant_heads", &quant_heads);
   m.def("rows_gemm_ok", &rows_gemm_ok);
+  m.def("mid_gemm_good", &mid_gemm_good);
   m.def("quant_rows", &quant_rows);
   m.def("quant_rows_ok", &quant_rows_ok);
   m.def("quant_gemv", &quant_gemv);

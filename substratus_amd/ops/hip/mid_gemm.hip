@@ -1,0 +1,339 @@
+// y = x w^T + bias of 17 to 256 rows with a bf16 weight matrix [n, k], as decode
+// steps of larger batches and short prompts need it; or silu(gate) * up of a
+// matrix whose first half gates its second; or, of a projection of heads, rotated
+// queries, with keys and values appended to the cache (rows_gemm.h).
+//
+// Bound by reading the weights once and the rows of x once per workgroup: tiles
+// are about as wide as they are high, so that either is half of it, and as many
+// workgroups as CUs share the inner dimension, whose 32-bit sums a second kernel
+// adds up. Stages of 64 columns go straight to LDS, up to 96 KB in flight per CU.
+// A load takes 8 rows x 128 bytes: with 16 rows x 64 bytes every cache line came
+// twice, 128 x 4544 x 18176 in 64 us instead of 51. Four waves that shared the
+// inner dimension instead, without barriers, were no faster at either; nor are
+// more stages in flight, or operands read half a stage ahead (a CU takes in some
+// 38 GB/s as it is).
+//
+// us on a MI355X, from the library's product to this one:
+//   rows     n x k: 4096 x 4096    4096 x 11008   4544 x 18176   8192 x 8192
+//   17              13.6 -> 11.7    32.5 -> 22.6   117 -> 35.8   31.4 -> 34.6
+//   64              15.1 -> 13.2    34.8 -> 25.9   156 -> 40.9   33.9 -> 36.1
+//   128             24.5 -> 17.0    59.9 -> 31.9   151 -> 51.1   49.1 -> 44.8
+//   192             33.1 -> 20.7    81.4 -> 39.6   123 -> 69.4   64.7 -> 53.7
+//   256             23.0 -> 24.0    50.2 -> 44.1   143 -> 77.6   77.2 -> 60.7
+#include "mid_gemm.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace {
+
+constexpr int WAVES = 4;
+constexpr int STEP = 64;          // columns of a stage
+constexpr int TILE = 128;         // 16-byte pieces of 16 rows x 64 columns
+
+DEV_INLINE void barrier() {
+  wait_lds_reads();
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Weight tile t's first column, and how much later its second eight are.
+template <Columns C>
+DEV_INLINE int column_of(int t, const Heads& heads) {
+  if constexpr (C == Columns::PLAIN) return t * 16;
+  const int at = t * 8;
+  if constexpr (C == Columns::HEADS) {
+    const int half = heads.d / 2;
+    return at + at / half * half;
+  }
+  return at;
+}
+
+// Four columns c to c + 3 of tile t, row r, and, unless they are stored as they
+// are, the four that go with them, eight later in the tile.
+template <Columns C>
+DEV_INLINE void finish(const MidGemm& a, const Heads& heads, int r, int t, int c,
+                       float4v u, float4v v) {
+  const int n0 = column_of<C>(t, heads), half = C == Columns::HEADS
+      ? heads.d / 2 : a.n / 2;
+  if constexpr (C == Columns::PLAIN) {
+    const int col = n0 + c;
+    if (col >= a.n) return;
+    if (a.bias != nullptr) {
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) u[e] += bf2f(a.bias[min(col + e, a.n - 1)]);
+    }
+    bf16_t* to = a.y + r * a.y_ld + col;
+    if (a.quads) {
+      *reinterpret_cast<uint2*>(to) =
+          make_uint2(pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]));
+      return;
+    }
+    #pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < a.n) to[e] = f2bf(u[e]);
+    return;
+  }
+  if (a.bias != nullptr) {
+    #pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      u[e] += bf2f(a.bias[n0 + c + e]);
+      v[e] += bf2f(a.bias[n0 + c + e + half]);
+    }
+  }
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if constexpr (C == Columns::GATED)
+      a.y[r * a.y_ld + n0 + c + e] = f2bf(silu_times(u[e], v[e]));
+    else
+      finish_heads(a.y, a.y_ld, heads, r, n0 + c + e, u[e], v[e]);
+  }
+}
+
+// F: tiles of 16 rows of x, N: of weights; P stages of 64 columns of both in LDS
+template <Columns C, int F, int N, int P>
+__global__ __launch_bounds__(WAVES * WAVE, (N + F) * 2 * P <= 80 ? 2 : 1)
+void mid_gemm_kernel(MidGemm a, Heads heads, float* __restrict__ part) {
+  constexpr int STAGE = (N + F) * TILE;
+  constexpr int LOADS = (N + F) * 2 / WAVES;     // a wave's, of a stage
+  static_assert((N + F) % 2 == 0);
+  // waves share rows of x, too, where there are enough
+  constexpr int WM = F >= 4 ? 2 : 1;
+  constexpr int WN = WAVES / WM, FW = F / WM, NW = N / WN;
+  static_assert(FW * WM == F && NW * WN == N);
+  __shared__ alignas(16) uint4 s_all[P * STAGE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, lo = lane & 15, g = lane >> 4;
+  const int wm = wave % WM, wn = wave / WM;
+  // blocks of rows of the same columns go to the same XCD, which has every
+  // eighth workgroup
+  const int cols = gridDim.x / a.blocks;
+  const int q = blockIdx.x / (8 * a.blocks), rest = min(cols - q * 8, 8);
+  const int in = blockIdx.x - q * 8 * a.blocks;
+  const int ct = q * 8 + in % rest, r0 = in / rest * F * 16;
+  const int last = (a.n + 15) / 16 - 1;
+  const int all = (a.k + STEP - 1) / STEP;
+  const int i0 = (int)((long)all * blockIdx.y / gridDim.y);
+  const int steps = (int)((long)all * (blockIdx.y + 1) / gridDim.y) - i0;
+
+  // A load is 8 rows x 128 bytes, whole cache lines (64 of 16 rows each: lines
+  // came twice, 35 % slower). A row's pieces are permuted by the row against
+  // bank conflicts.
+  const char* from[LOADS];
+  int piece[LOADS];
+  #pragma unroll
+  for (int l = 0; l < LOADS; ++l) {
+    const int id = wave * LOADS + l, t = id / 2;
+    const int row = id % 2 * 8 + lane / 8;
+    const int n0 = column_of<C>(min(ct * N + min(t, N - 1), last), heads);
+    const int half = C == Columns::HEADS ? heads.d / 2 : a.n / 2;
+    const bf16_t* p = t < N
+        ? a.w + (long)weight_row<C>(n0, row, a.n, half) * a.k
+        : a.x + min(r0 + (t - N) * 16 + row, a.m - 1) * a.x_ld;
+    piece[l] = (lane % 8) ^ (row >> 1 & 7);
+    from[l] = reinterpret_cast<const char*>(p + (long)i0 * STEP);
+  }
+  const int over = a.k / 8 - i0 * 8 - 1;         // a row's last piece from here
+  auto load = [&](int i) {
+    uint4* to = s_all + i % P * STAGE + wave * LOADS * 64;
+    #pragma unroll
+    for (int l = 0; l < LOADS; ++l)
+      load_to_lds<16>(from[l] + min(i * 8 + piece[l], over) * 16, to + l * 64);
+  };
+  float4v acc[NW][FW];
+  #pragma unroll
+  for (int j = 0; j < NW; ++j)
+    #pragma unroll
+    for (int f = 0; f < FW; ++f) acc[j][f] = (float4v){0.f, 0.f, 0.f, 0.f};
+  auto use = [&](int i) {
+    const uint4* s = s_all + i % P * STAGE + lo * 8;
+    #pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int at = (c * 4 + g) ^ (lo >> 1);
+      short8 wf[NW], xf[FW];
+      #pragma unroll
+      for (int j = 0; j < NW; ++j)
+        wf[j] = *reinterpret_cast<const short8*>(s + (wn * NW + j) * TILE + at);
+      #pragma unroll
+      for (int f = 0; f < FW; ++f)
+        xf[f] = *reinterpret_cast<const short8*>(
+            s + (N + wm * FW + f) * TILE + at);
+      if (c == 1 && (i0 + i) * STEP + STEP > a.k) break;   // half a step's
+      #pragma unroll
+      for (int j = 0; j < NW; ++j)
+        #pragma unroll
+        for (int f = 0; f < FW; ++f)
+          acc[j][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              wf[j], xf[f], acc[j][f], 0, 0, 0);
+    }
+  };
+  #pragma unroll
+  for (int i = 0; i < P - 1; ++i)
+    if (i < steps) load(i);
+  int i = 0;
+  for (; i + P - 1 < steps; ++i) {
+    wait_loads<(P - 2) * LOADS>();  // this step's, of all waves; and all have
+    barrier();                      // read what the next load takes the place of
+    load(i + P - 1);
+    use(i);
+  }
+  for (; i < steps; ++i) {
+    wait_loads<0>();
+    barrier();
+    use(i);
+  }
+
+  #pragma unroll
+  for (int f = 0; f < FW; ++f) {
+    const int r = r0 + (wm * FW + f) * 16 + lo;
+    #pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      const int t = ct * N + wn * NW + j;
+      const bool there = r < a.m && t <= last;
+      if (gridDim.y > 1) {
+        if (there)
+          *reinterpret_cast<float4v*>(
+              part + ((long)blockIdx.y * a.m + r) * (last + 1) * 16 + t * 16 +
+              g * 4) = acc[j][f];
+        continue;
+      }
+      float4v other = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (C != Columns::PLAIN)
+        #pragma unroll
+        for (int e = 0; e < 4; ++e)
+          other[e] = __shfl_xor(acc[j][f][e], 32, WAVE);
+      if (there && (C == Columns::PLAIN || g < 2))
+        finish<C>(a, heads, r, t, g * 4, acc[j][f], other);
+    }
+  }
+}
+
+// Workgroups' shares of the inner dimension, added up.
+template <Columns C>
+__global__ __launch_bounds__(256)
+void mid_sum_kernel(MidGemm a, Heads heads, const float* __restrict__ part,
+                    int splits) {
+  constexpr int PER = C == Columns::PLAIN ? 4 : 2;
+  const int tiles = (a.n + 15) / 16;
+  const long id = (long)blockIdx.x * 256 + threadIdx.x;
+  const int r = id / (tiles * PER), e = id % (tiles * PER);
+  if (r >= a.m) return;
+  const int t = e / PER, c = e % PER * 4;
+  const long step = (long)a.m * tiles * 16;
+  const float* p = part + (long)r * tiles * 16 + t * 16 + c;
+  float4v u = {0.f, 0.f, 0.f, 0.f}, v = u;
+  #pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    u += *reinterpret_cast<const float4v*>(p + s * step);
+    if constexpr (C != Columns::PLAIN)
+      v += *reinterpret_cast<const float4v*>(p + s * step + 8);
+  }
+  finish<C>(a, heads, r, t, c, u, v);
+}
+
+}  // namespace
+
+bool mid_gemm_takes(long m, long n, long k, bool paired) {
+  return m >= 1 && m <= 256 && n >= 16 && k >= STEP && k % 32 == 0 &&
+         n < (1L << 24) && k < (1L << 24) && (!paired || n % 16 == 0);
+}
+
+// The tiles and shares that take least: some 5 us of launch and first loads, the
+// weights at 5.3 TB/s, a stage of a CU at 38 GB/s, and the sums' kernel and way
+// through memory. Within a seventh of what 900 products were measured to take.
+MidPlan mid_gemm_plan(long m, long n, long k) {
+  MidPlan best{};
+  best.us = 1e30;
+  const long steps = (k + STEP - 1) / STEP;
+  const long blocks = (m + 127) / 128, per = (m + blocks - 1) / blocks;
+  const int rows = per <= 32 ? 32 : per <= 64 ? 64 : per <= 96 ? 96 : 128;
+  const double weights = n * k * 2 / 5.3e6;
+  for (int tiles = 4; tiles <= 8; tiles += 4) {
+    const long groups = (n + tiles * 16 - 1) / (tiles * 16) * blocks;
+    for (int s = 1; s <= 16 && s <= steps; ++s) {
+      const long rounds = (groups * s + 255) / 256;
+      const double load = rounds * ((steps + s - 1) / s) *
+                          ((tiles + rows / 16) * 2.048 / 38.);
+      const double sum = s > 1 ? 3. + s * m * n * 8 / 7e6 : 0.;
+      const double us = 4.5 + std::max(weights, load) + sum;
+      if (us < best.us) best = {rows, tiles, s, us};
+    }
+  }
+  return best;
+}
+
+// Whether the library's product would take longer, whose tiles are few or waste
+// the chip where matrices are not wide. Its time over this one's, MI355X, 11 row
+// counts x 14 widths x 7 inner sizes (a paired one saves it a launch, too):
+//   inner size 18176               10240 and less 1.02 to 4, 12288 0.75 to 1.5
+//   17 to 32 rows                  up to 5120 x from 5120 on 1.0 to 2.9, but for
+//                                  4096 x 8192 (0.80 to 0.87); 6144 0.84 to 1.4,
+//                                  8192 0.79 to 0.96
+//   48, 64                         3072 to 6144 x from 4096 on 0.95 to 2.0, 8192
+//                                  0.82 to 1.1, 9216 and 10240 1.04 to 1.2
+//   96, 128                        3072 to 10240 x from 4096 on 1.04 to 1.9 (8192
+//                                  x 8192 0.91, 1.05)
+//   160, 192                       3072 to 5120 x from 4096 on 0.87 to 2.3, 6144
+//                                  and 8192 x from 5120 on 0.99 to 1.3, 9216 0.8
+//   224, 256                       4672 to 8192 x from 4096 on 1.0 to 1.8, 4096 x
+//                                  from 11008 on 1.1, to 8192 0.95
+//   2048 and 2304                  x from 5632 on 1.02 to 2.4, 4096 0.6 to 1.1
+//   768 and 1024                   x 11008 0.97 to 2.9, 8192 0.8 to 1.2
+//   12288                          0.71 to 1.03, 0.85 to 1.2 x 2048
+bool mid_gemm_pays(long m, long n, long k, bool paired) {
+  if (m <= 16 || m > 256 || n > 10240)
+    return paired && m > 16 && m <= 40 && n <= 16384 && k >= 4096;
+  if (k >= 16384) return true;
+  if (paired && (k >= 4096 || (k >= 2048 && n >= 3072))) return true;
+  if (n < 2048) return k >= 11008;
+  if (n < 3072) return k >= 5632;
+  if (k < 4096) return false;
+  if (m <= 40)
+    return n <= 5120 && k >= 4544 && !(n % 4096 == 0 && k % 4096 == 0);
+  if (m <= 96) return n <= 6144 || k >= 11008 || (m <= 64 ? n >= 9216
+                                                         : n != 8192);
+  if (m <= 128) return true;
+  if (m <= 192) return n >= 4096 && n <= 5120 ? true : n <= 8192 && k >= 5120;
+  return n <= 8192 && (n >= 4544 || k >= (n == 4096 ? 11008 : 5120));
+}
+
+void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
+                     const Heads* heads, bool gated, float* part,
+                     hipStream_t stream) {
+  MidGemm a = given;
+  a.blocks = (a.m + plan.rows - 1) / plan.rows;
+  a.quads = a.n % 4 == 0 && a.y_ld % 4 == 0 &&
+            reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+  const Heads h = heads ? *heads : Heads{};
+  const int tiles = (a.n + 15) / 16;
+  auto launch = [&](auto f, auto n, auto p) {
+    constexpr int F = decltype(f)::value, N = decltype(n)::value,
+                  P = decltype(p)::value;
+    auto kernel = heads ? mid_gemm_kernel<Columns::HEADS, F, N, P>
+                  : gated ? mid_gemm_kernel<Columns::GATED, F, N, P>
+                          : mid_gemm_kernel<Columns::PLAIN, F, N, P>;
+    kernel<<<dim3((tiles + N - 1) / N * a.blocks, plan.splits), WAVES * WAVE,
+             0, stream>>>(a, h, part);
+  };
+  using std::integral_constant;
+  auto wide = [&](auto f) {
+    constexpr int F = decltype(f)::value;
+    constexpr integral_constant<int, 4> c4{};
+    constexpr integral_constant<int, 8> c8{};
+    if (plan.tiles == 4) launch(f, c4, integral_constant<int, F == 2 ? 6 : F <= 4 ? 5 : F == 6 ? 4 : 3>{});
+    else launch(f, c8, integral_constant<int, F == 2 ? 4 : F == 4 ? 3 : F == 6 ? 5 : 4>{});
+  };
+  if (plan.rows == 32) wide(integral_constant<int, 2>{});
+  else if (plan.rows == 64) wide(integral_constant<int, 4>{});
+  else if (plan.rows == 96) wide(integral_constant<int, 6>{});
+  else wide(integral_constant<int, 8>{});
+  if (plan.splits > 1) {
+    auto sum = heads ? mid_sum_kernel<Columns::HEADS>
+               : gated ? mid_sum_kernel<Columns::GATED>
+                       : mid_sum_kernel<Columns::PLAIN>;
+    const long quads = (long)a.m * tiles * (heads || gated ? 2 : 4);
+    sum<<<dim3((quads + 255) / 256), 256, 0, stream>>>(a, h, part,
+                                                       plan.splits);
+  }
+}

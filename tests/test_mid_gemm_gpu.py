@@ -1,0 +1,117 @@
+"""Products of 17 to 256 rows (mid_gemm.hip) against 64 bits: tiles of rows and
+columns that are partly there, halves of stages, rings that are not filled,
+shares of the inner dimension; gated columns and heads."""
+
+import pytest
+import torch
+
+from substratus_amd import _C, ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def near(got, prod, room):
+    # half a bf16 step of the result, and 32-bit sums whose order is free
+    off = (got.double() - prod).abs()
+    assert bool((off <= 2.0 ** -8 * prod.abs() + room + 1e-30).all())
+
+
+def operands(m, n, k):
+    torch.manual_seed(m * 10000 + n + k)
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    x = torch.randn(m, k + 64, device=DEV).bfloat16()[:, 32:32 + k]
+    prod = x.double() @ w.double().T
+    # 2^-24 per addend, errors that partly cancel
+    return x, w, prod, 2.0 ** -18 * (x.double().abs() @ w.double().abs().T)
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 64, 65, 96, 97, 128, 129, 192, 193,
+                               256])
+@pytest.mark.parametrize("n,k", [(16, 16416), (100, 16384), (3076, 5152),
+                                 (4600, 4544), (2050, 11040)])
+@torch.no_grad()
+def test_rows(m, n, k):
+    if not _C.mid_gemm_good(m, n, k, False):
+        pytest.skip("the library's")
+    x, w, prod, room = operands(m, n, k)
+    b = torch.randn(n, device=DEV).bfloat16()
+    assert ops._few_rows(x, w, b, False) is not None
+    near(ops.linear(x, w), prod, room)
+    near(ops.linear(x, w, b), prod + b.double(), room)
+    assert torch.equal(ops.linear(x, w), ops.linear(x, w))
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 48, 4096), (70, 4112, 2080),
+                                   (256, 320, 4128)])
+@torch.no_grad()
+def test_gated(m, n, k):
+    assert _C.mid_gemm_good(m, n, k, True)
+    x, w, prod, room = operands(m, n, k)
+    x, prod, room = x * 0.03125, prod * 0.03125, room * 0.03125
+    g, u = prod.chunk(2, 1)
+    rg, ru = room.chunk(2, 1)
+    want = torch.nn.functional.silu(g) * u
+    off = (ops.linear_gated(x, w).double() - want).abs()
+    # a gate's error reaches the product by silu's slope, at most 1.1
+    assert bool((off <= 2.0 ** -8 * want.abs() + 1e-6
+                 + 1.1 * (rg * u.abs() + ru * g.abs())).all())
+
+
+@pytest.mark.parametrize("m,hq,hkv,d,k", [(17, 3, 1, 64, 4096),
+                                          (100, 4, 2, 128, 4128),
+                                          (256, 24, 12, 64, 2048),
+                                          (130, 2, 1, 16, 4096)])
+@pytest.mark.parametrize("theta", [0.0, 10000.0])
+@torch.no_grad()
+def test_heads(m, hq, hkv, d, k, theta):
+    n = (hq + 2 * hkv) * d
+    assert _C.mid_gemm_good(m, n, k, True)
+    x, w, _, _ = operands(m, n, k)
+    x, b = x * 0.03125, torch.randn(n, device=DEV).bfloat16()
+    pages = (m + 15) // 16 + 2
+    made = []
+    for fused in (True, False):
+        kc, vc = (torch.zeros(pages, hkv, 16, d, device=DEV).bfloat16()
+                  for _ in range(2))
+        g = torch.Generator().manual_seed(m)
+        slots = torch.randperm(pages * 16, generator=g)[:m].int().to(DEV)
+        positions = torch.randint(0, 3000, (m,), generator=g).int().to(DEV)
+        cache = ops.Cache(positions, kc, vc, slots, theta)
+        if fused:
+            q = ops.linear_heads(x, w, b, cache)
+        else:
+            y = ops.linear(x, w, b)
+            q, kk, v = y.split([hq * d, hkv * d, hkv * d], 1)
+            q = ops.rope_kv_append(
+                q.reshape(m, hq, d).contiguous(),
+                kk.reshape(m, hkv, d).contiguous(),
+                v.reshape(m, hkv, d).contiguous(), *cache)
+        made.append((q, kc, vc))
+    for got, want in zip(*made):
+        # sums in another order may round to the next bf16 number before a turn
+        off = (got.float() - want.float()).abs()
+        assert bool((off <= 2.0 ** -6 * want.float().abs().amax()).all())
+        assert float((got.float() - want.float()).norm()) <= \
+            2.0 ** -8 * float(want.float().norm())
+        assert torch.equal(got == 0, want == 0)
+
+
+@torch.no_grad()
+def test_in_a_graph():
+    """Sums of shares come from memory of the graph's own."""
+    m, n, k = 40, 4600, 4544
+    x, w, prod, room = operands(m, n, k)
+    ops.linear(x, w)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.linear(x, w)
+    for i in range(3):
+        x.mul_(-1)
+        prod = -prod
+        graph.replay()
+        other = ops.linear(x, w)
+        torch.cuda.synchronize()
+        near(y, prod, room)
+        assert torch.equal(y, other)
