@@ -208,7 +208,7 @@ template <class Y>
 void launch_group_gemm_tile(const GroupGemm<bf16_t, Y>&, int tile,
                             hipStream_t);
 
-// Packed rows, up to 32 of a group (group_gemm_rows.hip).
+// Packed rows, up to 64 of a group (group_gemm_rows.hip).
 template <class Y>
 bool group_gemm_rows_takes(const GroupGemm<bf16_t, Y>&, int tile);
 template <class Y>

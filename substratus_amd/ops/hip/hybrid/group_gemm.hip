@@ -1,6 +1,6 @@
 // Grouped products (group_gemm.h) of few rows per group, and of any size:
 //
-//   rows     packed bf16 rows, up to 32 of a group: group_gemm_rows.hip.
+//   rows     packed bf16 rows, up to 64 of a group: group_gemm_rows.hip.
 //   stream   bf16, few rows per group: bound by reading the weights once.
 //            Every wave takes a share of the inner dimension of a tile of
 //            rows and 64 columns (4 waves; 16 and 32 columns where there are

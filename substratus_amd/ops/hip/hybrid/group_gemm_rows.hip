@@ -1,23 +1,22 @@
 // Grouped products (group_gemm.h) of packed rows, few to a group: experts of a
-// decode step, up to 32 rows of one in a tile.
+// decode step, up to 64 rows of one in a tile.
 //
 // Bound by reading the weights once. A workgroup has 16 of a matrix' rows (tiles
-// of 16 rows of x) or 32 (tiles of up to 32), and its four waves share the inner
-// dimension; a wave's loads go straight to LDS, 16 rows x 64 contiguous bytes
-// with consecutive lanes on consecutive pieces (loaded in the order of the matrix
-// operands every lane is a cache lookup of its own). A stage is 64 columns of the
-// weights and of the 16 or 32 rows that a tile really has.
+// of 16 rows of x) or 32, and its four waves share the inner dimension; a wave's
+// loads go straight to LDS, 8 rows x 128 contiguous bytes with consecutive lanes
+// on consecutive pieces (loaded in the order of the matrix operands every lane is
+// a cache lookup of its own; 16 rows x 64 bytes are half cache lines, and 48 rows
+// take 37.3 us instead of 35.1). A stage is 64 columns of the weights and of the
+// 16 to 64 rows that a tile really has.
 //
 // us on a MI355X, 32 experts, 6 a row, 2048 -> 1408 and back, from operands loaded
 // in their own order to this:
-//   1 row     14.4 -> 10.3 (3.4 TB/s)    13.0 -> 9.9
-//   10 rows   35.4 -> 31.4 (5.3)         35.8 -> 34.1
-//   48 rows   41.1 -> 37.3 (5.0)         42.5 -> 38.8
-//   64 rows   42.0 -> 39.0
-//   100 rows  43.4 -> 43.7
-// Tiles of 48 and 64 rows read more of x than of weights and are no faster so
-// (128 rows 49.3, 50.6): those stay with the other kernel. 48 rows, 16 and 64
-// columns a workgroup: 38.0 43.7, 41.3 39.4.
+//   1 row     14.4 -> 10.4 (3.3 TB/s)    13.0 -> 10.2
+//   10 rows   35.4 -> 32.2 (5.2)         35.8 -> 34.1
+//   48 rows   41.1 -> 35.1 (5.3)         42.5 -> 34.0
+//   128 rows  49.3 -> 38.4 (4.8)         50.0 -> 38.8
+//   300 rows  62.9 -> 55.4               65.0 -> 53.9
+//   500 rows  89.0 -> 73.3               86.2 -> 71.8
 #include "../rows_gemm.h"
 #include "group_gemm.h"
 
@@ -27,56 +26,64 @@ constexpr int KW = 4;             // waves, which share k
 constexpr int TILE = 64;          // 16-byte pieces of 16 rows x 32 columns
 constexpr int PAD = 4;
 constexpr int KC = 32;
+constexpr int U = 2;              // chunks of a stage
 
-// How rows are taken: F tiles of 16 with N of the weights', U chunks a stage, P
-// stages in flight.
-template <int F_, int N_, int U_, int P_> struct How {
-  static constexpr int F = F_, N = N_, U = U_, P = P_;
+// How rows are taken: F tiles of 16 with N of the weights', P stages in flight.
+template <int F_, int N_, int P_> struct How {
+  static constexpr int F = F_, N = N_, P = P_;
   static constexpr int PIECES = KW * P * U * (N + F) * TILE;     // of LDS
 };
 
 template <class H, Act ACT, class Y>
 DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
                               uint4* s_all) {
-  constexpr int F = H::F, N = H::N, U = H::U, P = H::P;
+  constexpr int F = H::F, N = H::N, P = H::P;
   constexpr int TILES = N + F, STAGE = U * TILES * TILE, LOADS = U * TILES;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE, lo = lane & 15, g = lane >> 4;
+  // shares begin on whole cache lines
   const int n0 = blockIdx.x * N * 16, chunks = a.k / KC;
-  const int c0 = chunks * wave / KW, c1 = chunks * (wave + 1) / KW;
+  const int pairs = (chunks + 1) / 2;
+  const int c0 = pairs * wave / KW * 2;
+  const int c1 = min(pairs * (wave + 1) / KW * 2, chunks);
   const int steps = (c1 - c0 + U - 1) / U;
   uint4* ring = s_all + wave * P * STAGE;
 
-  // a lane loads 16 bytes of row lane / 4 of a tile, permuted by the row
-  // against bank conflicts
-  const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
-  const char* wp[N];
+  // a load is 8 rows x 128 bytes: of a tile's row lane / 8, or eight later.
+  // Pieces are permuted by the row against bank conflicts.
+  const char *wp[N][2], *xp[F][2];
+  int piece[2];
   #pragma unroll
-  for (int f = 0; f < N; ++f)
-    wp[f] = reinterpret_cast<const char*>(
-        a.w + ((long)t.g * a.n + min(n0 + f * 16 + row, a.n - 1)) * a.k) +
-        piece * 16;
-  const char* xp[F];
-  #pragma unroll
-  for (int f = 0; f < F; ++f) {
-    const int r = min(t.r0 + f * 16 + row, t.r1 - 1);
-    xp[f] = reinterpret_cast<const char*>(
-        a.x + (long)(a.src != nullptr ? a.src[r] : r) * a.x_ld) + piece * 16;
-  }
-  auto load = [&](int s, int i) {
+  for (int h = 0; h < 2; ++h) {
+    const int row = h * 8 + (lane >> 3);
+    piece[h] = (lane & 7) ^ (row >> 1);
     #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // a stage may be half of one: then its last chunk comes twice
-      const unsigned at = (unsigned)min(c0 + i * U + u, c1 - 1) * 64;
-      uint4* to = ring + s * STAGE + u * TILES * TILE;
+    for (int f = 0; f < N; ++f)
+      wp[f][h] = reinterpret_cast<const char*>(
+          a.w + ((long)t.g * a.n + min(n0 + f * 16 + row, a.n - 1)) * a.k +
+          c0 * KC);
+    #pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const int r = min(t.r0 + f * 16 + row, t.r1 - 1);
+      xp[f][h] = reinterpret_cast<const char*>(
+          a.x + (long)(a.src != nullptr ? a.src[r] : r) * a.x_ld + c0 * KC);
+    }
+  }
+  const int end = (c1 - c0) * 4 - 1;             // the share's last piece
+  auto load = [&](int s, int i) {
+    uint4* to = ring + s * STAGE;
+    #pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // a stage may be half of one: then its last piece comes again
+      const unsigned at = (unsigned)min(i * 8 + piece[h], end) * 16;
       #pragma unroll
-      for (int f = 0; f < N; ++f) load_to_lds<16>(wp[f] + at, to + f * TILE);
+      for (int f = 0; f < N; ++f)
+        load_to_lds<16>(wp[f][h] + at, to + (f * 2 + h) * TILE);
       #pragma unroll
       for (int f = 0; f < F; ++f)
-        load_to_lds<16>(xp[f] + at, to + (N + f) * TILE);
+        load_to_lds<16>(xp[f][h] + at, to + ((N + f) * 2 + h) * TILE);
     }
   };
-  const int at = lo * 4 + (g ^ ((lo >> 2) & 3));
   float4v acc[N][F];
   #pragma unroll
   for (int j = 0; j < N; ++j)
@@ -86,13 +93,13 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
     short8 wf[U][N], xf[U][F];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint4* p = ring + s * STAGE + u * TILES * TILE + at;
+      const uint4* p = ring + s * STAGE + lo * 8 + ((u * 4 + g) ^ (lo >> 1));
       #pragma unroll
       for (int f = 0; f < N; ++f)
-        wf[u][f] = *reinterpret_cast<const short8*>(p + f * TILE);
+        wf[u][f] = *reinterpret_cast<const short8*>(p + f * 2 * TILE);
       #pragma unroll
       for (int f = 0; f < F; ++f)
-        xf[u][f] = *reinterpret_cast<const short8*>(p + (N + f) * TILE);
+        xf[u][f] = *reinterpret_cast<const short8*>(p + (N + f) * 2 * TILE);
     }
     if (more) {
       wait_lds_reads();
@@ -157,19 +164,28 @@ template <class Y, Act ACT, int MAX>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void group_gemm_rows_kernel(GroupGemm<bf16_t, Y> a) {
   constexpr int N = MAX == 1 ? 1 : 2;
-  using One = std::conditional_t<MAX == 1, How<1, N, 2, 4>, How<1, N, 2, 3>>;
-  using Two = How<2, N, 2, 2>;
+  using One = std::conditional_t<MAX == 1, How<1, N, 4>, How<1, N, 3>>;
+  using Two = How<2, N, 2>;
   // one array: beside a second one the compiler guards every LDS read against
   // the direct loads in flight, and waits for them
-  __shared__ alignas(16)
-      uint4 s_all[MAX > 1 && Two::PIECES > One::PIECES ? Two::PIECES
-                                                        : One::PIECES];
+  using Three = How<3, N, 2>;
+  using Four = How<4, N, 1>;
+  constexpr int LARGEST = MAX > 2 ? Three::PIECES : One::PIECES;
+  __shared__ alignas(16) uint4 s_all[LARGEST];
+  static_assert(MAX == 1 || Two::PIECES <= LARGEST);
   const Tile t = tile_of(a, blockIdx.y, 0, MAX * 16);
   if (t.r1 <= t.r0) return;
-  if (MAX == 1 || t.r1 - t.r0 <= 16)             // rows that there are
+  const int tiles = (t.r1 - t.r0 + 15) / 16;     // of the rows there are
+  if (MAX == 1 || tiles == 1) {
     rows_of_group<One, ACT>(a, t, s_all);
-  else if constexpr (MAX > 1)
-    rows_of_group<Two, ACT>(a, t, s_all);
+  } else if constexpr (MAX > 1) {
+    if (MAX == 2 || tiles == 2) {
+      rows_of_group<Two, ACT>(a, t, s_all);
+    } else if constexpr (MAX > 2) {
+      if (tiles == 3) rows_of_group<Three, ACT>(a, t, s_all);
+      else rows_of_group<Four, ACT>(a, t, s_all);
+    }
+  }
 }
 
 }  // namespace
@@ -177,7 +193,7 @@ void group_gemm_rows_kernel(GroupGemm<bf16_t, Y> a) {
 // Pieces of rows are known to be aligned; stages are of whole chunks.
 template <class Y>
 bool group_gemm_rows_takes(const GroupGemm<bf16_t, Y>& a, int tile) {
-  return a.tiles != nullptr && tile <= 32 && a.k % KC == 0 && a.k >= 4 * KC &&
+  return a.tiles != nullptr && tile <= 64 && a.k % KC == 0 && a.k >= 4 * KC &&
          a.tail == 0;
 }
 
@@ -187,7 +203,8 @@ void launch_group_gemm_rows(const GroupGemm<bf16_t, Y>& a, int tile,
   by_act(a.act, [&](auto act) {
     constexpr Act ACT = decltype(act)::value;
     auto kernel = tile == 16 ? group_gemm_rows_kernel<Y, ACT, 1>
-                             : group_gemm_rows_kernel<Y, ACT, 2>;
+                  : tile == 32 ? group_gemm_rows_kernel<Y, ACT, 2>
+                               : group_gemm_rows_kernel<Y, ACT, 4>;
     const int wide = tile == 16 ? 16 : 32;
     kernel<<<dim3((a.n + wide - 1) / wide, a.max_tiles), KW * WAVE, 0, stream>>>(a);
   });

@@ -11,12 +11,12 @@ pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
 
 
-@pytest.mark.parametrize("tile", [16, 32])
+@pytest.mark.parametrize("tile", [16, 32, 64])
 @pytest.mark.parametrize("k,n,act", [(128, 16, "none"), (160, 44, "gelu"),
                                      (1056, 24, "silu"), (2080, 72, "none"),
                                      (2048, 8, "gelu")])
 def test_experts_of_few_rows(tile, k, n, act):
-    counts = [1, 15, 0, 16, 17, 31, 32, 33, 2]
+    counts = [1, 15, 0, 16, 17, 31, 32, 33, 2, 48, 49, 64, 65]
     total, e = sum(counts), len(counts)
     g = torch.Generator().manual_seed(k + n)
     ids = torch.repeat_interleave(torch.arange(e), torch.tensor(counts))
