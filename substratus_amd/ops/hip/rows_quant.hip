@@ -28,10 +28,20 @@
 // consecutive lanes on consecutive bytes (see rows_gemm.hip), pieces permuted
 // by the row against bank conflicts. Few rows of x: P stages in flight per
 // wave; many: one, and more workgroups per CU instead.
+// A load takes 8 rows x 128 bytes of weights, where 16 x 64 asked for every
+// line twice. q6_K keeps the halves: a row is half a line more than whole ones,
+// and what a stage asks for is four kinds of pieces, of which two are less than
+// a line. us, weights not in a cache, 15360 x 5120, 5120 x 5120, 27648 x 5120,
+// 5120 x 13824, 12288 x 4096, 4096 x 11008, halves -> lines:
+//   q4_0  1 row   14.2 7.2 23.2 16.8 10.0 10.9 -> 14.1 7.4 21.8 16.5 10.3 9.5
+//   q8_0  3 rows  20.8 10.7 33.5 24.1 13.8 13.1 -> 19.4 10.3 31.6 22.5 12.8 13
+//   q4_K  5 rows  18.2 8.6 30.0 24.9 11.6 12.6 -> 17.8 8.7 29.1 23.8 11.5 12.2
+//   q6_K  5 rows  5120 x 5120 11.9 -> 15.3, 24 rows 15360 x 5120 35.6 -> 39.2
 //
-// us on a MI355X, 15360 x 5120, 5120 x 5120, 27648 x 5120, 5120 x 13824, from
-// one wave per weight row in vector arithmetic (up to 8 rows of x), or from
-// unpacking to bf16 in memory and the library (more), to this kernel:
+// us on a MI355X with weights partly in a cache, before that, 15360 x 5120,
+// 5120 x 5120, 27648 x 5120, 5120 x 13824, from one wave per weight row in
+// vector arithmetic (up to 8 rows of x), or from unpacking to bf16 in memory and
+// the library (more), to this kernel:
 //   q4_0  1 row   20.5  8.5 31.7 15.0 -> 12.9  7.2 20.9 15.3
 //         5 rows  55.0 21.5 95.3 47.8 -> 14.1  7.7 22.9 16.9
 //        24 rows  81.4 37.8  152 75.9 -> 23.5 12.5 38.7 26.5
@@ -187,9 +197,18 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const long rb = Q == Quant::Q4_0 ? k / 2 : Q == Quant::Q8_0 ? k
       : Q == Quant::Q4_K ? k / 16 + k / 2 : k / 16 * 13;
   const long sb = !K_QUANT ? nb * 2 : Q == Quant::Q4_K ? k / 64 : k / 128;
-  // a lane loads 16 bytes of row lane / 4 of a tile, and a word of its scales
+  // a lane loads 16 bytes of row lane / 4 of a tile, and a word of its scales;
+  // of lines of 128 bytes, of row lane / 8 or eight later
   const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
   const int word = lane & 3;
+  const unsigned char* pair[2];
+  int in_pair[2];
+  #pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = h * 8 + (lane >> 3);
+    in_pair[h] = (lane & 7) ^ (r >> 1);
+    pair[h] = qs + weight_row<C>(n0, r, n, half) * rb;
+  }
   const unsigned char* sc = reinterpret_cast<const unsigned char*>(scales);
   const unsigned char* wp = qs + weight_row<C>(n0, row, n, half) * rb;
   const unsigned char* sp = sc + weight_row<C>(n0, row, n, half) * sb;
@@ -207,19 +226,20 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     if constexpr (Q == Quant::Q4_0) {
       #pragma unroll
       for (int t = 0; t < 2; ++t)
-        load_to_lds<16>(wp + min(c * 8 + t * 4 + piece, nb - 1) * 16,
+        load_to_lds<16>(pair[t] + min(c * 8 + in_pair[t], nb - 1) * 16,
                         ws + t * TILE);
       load_to_lds<4>(sp + min(c * 16 + word * 4, nb * 2 - 4), ss);
     } else if constexpr (Q == Quant::Q8_0) {
       #pragma unroll
       for (int t = 0; t < 4; ++t)
-        load_to_lds<16>(wp + min(c * 256 + t * 64 + piece * 16, k - 16),
+        load_to_lds<16>(pair[t & 1] + min(c * 256 + (t >> 1) * 128 +
+                                              in_pair[t & 1] * 16, k - 16),
                         ws + t * TILE);
       load_to_lds<4>(sp + min(c * 16 + word * 4, nb * 2 - 4), ss);
     } else if constexpr (Q == Quant::Q4_K) {
       #pragma unroll
       for (int t = 0; t < 2; ++t)
-        load_to_lds<16>(wp + k / 16 + c * 128 + t * 64 + piece * 16,
+        load_to_lds<16>(pair[t] + k / 16 + c * 128 + in_pair[t] * 16,
                         ws + t * TILE);
       // words: scales 0 to 3, 4 to 7, minima 0 to 3, 4 to 7
       load_to_lds<4>(wp + (word & 2) * (k / 64) + c * 8 + (word & 1) * 4, ss);
@@ -254,14 +274,15 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   }
   const int xsw = ((lo & 3) << 2) ^
                   (((lo & (MR > 16 ? 15 : MR - 1)) >> 2) & 3);
-  const int wsw = (lo >> 2) & 3;
+  const int wsw = Q == Quant::Q6_K ? lo >> 2 : lo >> 1;
   const uint4v* x_row = s_x + min(lo & (MR - 1), m - 1) * (k / 8 + 1);
   float4v acc[FM];
   #pragma unroll
   for (int j = 0; j < FM; ++j) acc[j] = zero;
 
   auto use = [&](int s, int c, auto whole) {
-    const uint4v* ws = ring + s * STAGE + lo * 4;
+    const uint4v* ws = ring + s * STAGE;
+    const uint4v* row = ws + lo * (Q == Quant::Q6_K ? 4 : 8);
     const uint4v* ss = ring + s * STAGE + L::W * TILE;
     const uint4v* xs = ring + s * STAGE + WS;
     const uint4v sv = ss[lo];
@@ -277,9 +298,12 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       const int at = Q == Quant::Q4_0 ? b & 3
           : Q == Quant::Q8_0 ? (b & 1) * 2 + (g >> 1)
                              : ((b >> 1) & 1) * 2 + (g >> 1);
+      // four blocks of q8_0 are a line
+      const int line = Q == Quant::Q8_0 ? (b >> 2) * 2 * TILE : 0;
+      const int in = Q == Quant::Q8_0 ? (b >> 1 & 1) * 4 + at
+                                      : (b >> 2) * 4 + at;
       const uint2v v = reinterpret_cast<const uint2v*>(
-          ws + (Q == Quant::Q8_0 ? b >> 1 : b >> 2) * TILE +
-          (at ^ wsw))[g & 1];
+          row + line + (in ^ wsw))[g & 1];
       uint2v w[2];
       #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -330,9 +354,9 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
         #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const unsigned v = reinterpret_cast<const unsigned*>(
-              ws + hf * TILE + (((quarter & 1) * 2 + h) ^ wsw))[g];
+              row + hf * TILE + (((quarter & 1) * 2 + h) ^ wsw))[g];
           const unsigned hv = reinterpret_cast<const unsigned*>(
-              ws + 2 * TILE + ((hf * 2 + h) ^ wsw))[g];
+              row + 2 * TILE + ((hf * 2 + h) ^ wsw))[g];
           const unsigned low = (quarter < 2 ? v << 2 : v >> 2) & 0x3C3C3C3Cu;
           const unsigned high = hv << (6 - 2 * quarter) & 0xC0C0C0C0u;
           const short4v wv = __builtin_bit_cast(
@@ -485,11 +509,13 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
     // 13.1.
     constexpr bool ONE = QQ == Quant::Q6_K || QQ == Quant::Q4_0;
     constexpr integral_constant<int, ONE ? 1 : 2> some{};
+    constexpr integral_constant<int, QQ == Quant::Q6_K ? 1 : 2> one_row{};
     constexpr integral_constant<int, QQ == Quant::Q8_0 ? 4 : 8> waves{};
     const bool thin = n <= 384 * 16;
     if (m == 1) {
       if constexpr (QQ != Quant::Q8_0) {
-        if (thin) go(qc, c4, c1, waves, some);
+        // q4_0, 4096 x 11008: one stage in flight 11.5 us, two 9.6
+        if (thin) go(qc, c4, c1, waves, one_row);
         else go(qc, c4, c1, c4, some);
       }
     } else if (m <= 4) {
