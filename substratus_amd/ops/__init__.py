@@ -177,12 +177,8 @@ def _flash_bwd(q, k, v, out, dout, lse, seq_start, max_len, scale):
     dk32 = torch.zeros(k.shape, dtype=torch.float32, device=k.device)
     dv32 = torch.zeros(v.shape, dtype=torch.float32, device=v.device)
     delta = torch.empty_like(lse)
-    if os.environ.get("SUB_ATTN_V5", "1") != "0":
-        ext.attn_train_bwd_v5(dq, dk32, dv32, q, k, v, out, dout, lse,
-                              delta, seq_start, max_len, scale)
-    else:
-        ext.attn_train_bwd(dq, dk32, dv32, q, k, v, out, dout, lse,
-                           delta, seq_start, max_len, scale)
+    ext.attn_train_bwd(dq, dk32, dv32, q, k, v, out, dout, lse, delta,
+                       seq_start, max_len, scale)
     return dq, dk32, dv32
 
 

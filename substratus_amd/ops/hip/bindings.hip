@@ -35,13 +35,10 @@ void launch_attn_prefill(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, c
 bool attn_prefill_supported(int);
 void launch_attn_v5(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, int, int, int, int, int, float, hipStream_t, float*);
 bool attn_v5_supported(int);
-void launch_attn_bwd_dq_v5(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int*, int, int, int, int, int, float, hipStream_t);
-void launch_attn_bwd_dkv_v5(float*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int*, int, int, int, int, int, float, hipStream_t);
-void launch_attn_bwd_dkv_only(float*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int*, int, int, int, int, int, float, hipStream_t);
+void launch_attn_bwd_dq(bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int*, int, int, int, int, int, float, hipStream_t);
+void launch_attn_bwd_dkv(float*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int*, int, int, int, int, int, float, hipStream_t);
 void launch_attn_bwd_delta(float*, const bf16_t*, const bf16_t*, long, int, hipStream_t);
-void launch_attn_bwd(bf16_t*, float*, float*, const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const float*, const float*, const int*, int, int, int, int, int, float, hipStream_t);
 bool attn_bwd_supported(int);
-int attn_bwd_heads(int, int, int, int);
 void launch_attn_prefill_probe(int, bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*, const int*, int, int, int, int, float, hipStream_t);
 void launch_mfma_probe(float*, const bf16_t*, const bf16_t*, hipStream_t);
 void launch_mfma32_probe(float*, const bf16_t*, const bf16_t*, hipStream_t);
@@ -480,63 +477,16 @@ void attn_train_bwd(torch::Tensor dq, torch::Tensor dk, torch::Tensor dv,
   TORCH_CHECK(hq % hkv == 0, "hq must be divisible by hkv");
   launch_attn_bwd_delta(delta.data_ptr<float>(), bfc(dout), bfc(out),
                         (long)q.size(0) * hq, d, stream());
-  launch_attn_bwd(bf(dq), dk.data_ptr<float>(), dv.data_ptr<float>(),
-                  bfc(q), bfc(k), bfc(v), bfc(dout),
-                  lse.data_ptr<float>(), delta.data_ptr<float>(),
-                  seq_start.data_ptr<int>(), num_seqs, (int)max_len, hq,
-                  hkv, d, (float)scale, stream());
+  launch_attn_bwd_dq(bf(dq), bfc(q), bfc(k), bfc(v), bfc(dout),
+                     lse.data_ptr<float>(), delta.data_ptr<float>(),
+                     seq_start.data_ptr<int>(), num_seqs, (int)max_len, hq,
+                     hkv, d, (float)scale, stream());
+  launch_attn_bwd_dkv(dk.data_ptr<float>(), dv.data_ptr<float>(), bfc(q),
+                      bfc(k), bfc(v), bfc(dout), lse.data_ptr<float>(),
+                      delta.data_ptr<float>(), seq_start.data_ptr<int>(),
+                      num_seqs, (int)max_len, hq, hkv, d, (float)scale,
+                      stream());
   post_launch_check("attn_train_bwd");
-}
-void attn_train_bwd_v5(torch::Tensor dq, torch::Tensor dk,
-                       torch::Tensor dv, torch::Tensor q, torch::Tensor k,
-                       torch::Tensor v, torch::Tensor out,
-                       torch::Tensor dout, torch::Tensor lse,
-                       torch::Tensor delta, torch::Tensor seq_start,
-                       long max_len, double scale) {
-  check_bf16(dq, "dq");
-  TORCH_CHECK(dk.scalar_type() == torch::kFloat &&
-              dv.scalar_type() == torch::kFloat, "dk/dv f32");
-  check_bf16(q, "q"); check_bf16(k, "k"); check_bf16(v, "v");
-  check_bf16(out, "out"); check_bf16(dout, "dout");
-  TORCH_CHECK(lse.scalar_type() == torch::kFloat &&
-              delta.scalar_type() == torch::kFloat, "lse/delta f32");
-  TORCH_CHECK(seq_start.scalar_type() == torch::kInt, "seq_start int32");
-  int hq = q.size(1), d = q.size(2), hkv = k.size(1);
-  int num_seqs = seq_start.size(0) - 1;
-  TORCH_CHECK(attn_v5_supported(d), "unsupported head_dim ", d);
-  TORCH_CHECK(hq % hkv == 0, "hq must be divisible by hkv");
-  launch_attn_bwd_delta(delta.data_ptr<float>(), bfc(dout), bfc(out),
-                        (long)q.size(0) * hq, d, stream());
-  launch_attn_bwd_dq_v5(bf(dq), bfc(q), bfc(k), bfc(v), bfc(dout),
-                        lse.data_ptr<float>(), delta.data_ptr<float>(),
-                        seq_start.data_ptr<int>(), num_seqs, (int)max_len,
-                        hq, hkv, d, (float)scale, stream());
-  // dkv: the V5 structure's 256-row tiles and 32-row blocks pay where there
-  // are enough of them. us of the backward on a MI355X, 16 rows a wave and V5:
-  // 32 heads of 128, 4 x 1024 314, 339; 4 x 2048 1149, 1026; 2 x 8192 7057,
-  // 5666. On 8 heads, 2 x 2048 480, 634; 8 x 2048 1934, 1657; 1 x 4096 858,
-  // 1088; 1 x 8192 3294, 3000. 71 heads on one of 64, 8 x 2048 2182, 2473;
-  // 2 x 8192 7718, 6003. SUB_ATTN_DKV_V5=0/1 overrides.
-  const char* e = getenv("SUB_ATTN_DKV_V5");
-  const bool many = d == 128 &&
-      attn_bwd_heads(num_seqs, max_len, hq, hkv) >= 4;
-  const bool use_v5 = e ? (e[0] == '1')
-      : max_len >= (hq == hkv || many ? 2048 : 8192);
-  if (use_v5)
-    launch_attn_bwd_dkv_v5(dk.data_ptr<float>(), dv.data_ptr<float>(),
-                           bfc(q), bfc(k), bfc(v), bfc(dout),
-                           lse.data_ptr<float>(), delta.data_ptr<float>(),
-                           seq_start.data_ptr<int>(), num_seqs,
-                           (int)max_len, hq, hkv, d, (float)scale,
-                           stream());
-  else
-    launch_attn_bwd_dkv_only(dk.data_ptr<float>(), dv.data_ptr<float>(),
-                             bfc(q), bfc(k), bfc(v), bfc(dout),
-                             lse.data_ptr<float>(), delta.data_ptr<float>(),
-                             seq_start.data_ptr<int>(), num_seqs,
-                             (int)max_len, hq, hkv, d, (float)scale,
-                             stream());
-  post_launch_check("attn_train_bwd_v5");
 }
 
 
@@ -1100,7 +1050,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quant_gemv_k", &quant_gemv_k);
   m.def("mfma32_probe", &mfma32_probe);
   m.def("attn_v5", &attn_v5);
-  m.def("attn_train_bwd_v5", &attn_train_bwd_v5);
   m.def("dequant_k", &dequant_k);
   m.def("mfma_gemm_pick_splitk", &mfma_gemm_pick_splitk);
   m.def("attn_train_bwd", &attn_train_bwd);
