@@ -1,4 +1,4 @@
-"""The backward of packed sequences at the edges of its tiles: 32 keys or queries
+"""Forward and backward of packed sequences at the edges of its tiles: 32 keys or queries
 of a wave, 64 taken at a time (32 keys of 128 columns), 128 of a workgroup."""
 
 import pytest
@@ -11,15 +11,15 @@ DEV = "cuda"
 
 
 def reference(q, k, v, dout, scale):
-    """Gradients of one sequence, in 64 bits."""
+    """Output and gradients of one sequence, in 64 bits."""
     q, k, v = (t.double().requires_grad_() for t in (q, k, v))
     group = q.shape[1] // k.shape[1]
     kk, vv = (t.repeat_interleave(group, 1).transpose(0, 1) for t in (k, v))
     sc = (q.transpose(0, 1) @ kk.mT) * scale
     mask = torch.ones(sc.shape[-2:], dtype=torch.bool).tril()
     p = torch.softmax(sc.masked_fill(~mask, -torch.inf), -1)
-    return torch.autograd.grad((p @ vv).transpose(0, 1), (q, k, v),
-                               dout.double())
+    out = (p @ vv).transpose(0, 1)
+    return out.detach(), *torch.autograd.grad(out, (q, k, v), dout.double())
 
 
 @pytest.mark.parametrize("scale", [None, -0.2])
@@ -28,7 +28,7 @@ def reference(q, k, v, dout, scale):
 @pytest.mark.parametrize("lens", [[1, 31, 32, 33], [64, 65, 63, 2],
                                   [127, 128, 129], [96, 0, 97, 160],
                                   [255, 257], [513]])
-def test_backward(lens, hq, hkv, d, scale):
+def test_packed(lens, hq, hkv, d, scale):
     scale = d ** -0.5 if scale is None else scale
     g = torch.Generator().manual_seed(sum(lens) + hq + d)
     n = sum(lens)
@@ -41,7 +41,7 @@ def test_backward(lens, hq, hkv, d, scale):
     out, lse = ops._flash_fwd(*dev[:3], starts_dev, max(lens), scale)
     got = ops._flash_bwd(*dev[:3], out, dev[3], lse, starts_dev, max(lens),
                          scale)
-    want = [torch.zeros(t.shape, dtype=torch.float64) for t in (q, k, v)]
+    want = [torch.zeros(t.shape, dtype=torch.float64) for t in (q, q, k, v)]
     for a, b in zip(starts[:-1], starts[1:]):
         if a < b:
             for w, r in zip(want, reference(q[a:b], k[a:b], v[a:b],
@@ -49,6 +49,6 @@ def test_backward(lens, hq, hkv, d, scale):
                 w[a:b] = r
     # weights and their gradients enter the products as bf16: 2^-9 each; the
     # outputs that Delta is made from and the results are rounded once
-    for x, w in zip(got, want):
+    for x, w in zip((out, *got), want):
         off = (x.cpu().double() - w).norm() / w.norm()
         assert float(off) < 2.0 ** -7, float(off)
