@@ -259,13 +259,13 @@ def inference_only(*tensors: torch.Tensor) -> bool:
 
 def _rows_gemm_pays(numel: int, n: int, k: int) -> bool:
     """Whether a product of numel / k rows is faster by rows_gemm.hip than by
-    the library. Up to 16 rows always: it reads the weights once. Then every
+    the library, wherever the question is asked (the extension knows more of
+    them). Up to 16 rows always: it reads the weights once. Then every
     workgroup, 16 columns, reads all rows as well, which costs less than the
     library's few tiles where there is no more than a workgroup per CU. us, the
     library's and ours:
-        32 x 4096 x 4096    14.2  12.7     48 x 4096 x 4096    14.0  15.2
-        32 x 6144 x 4096    16.7  22.2     64 x 4096 x 2048    12.2  10.6
-        24 x 2048 x 5632    11.8  12.4     64 x 6144 x 2048    13.4  18.2
+        32 x 4096 x 4096    13.4  10.3     48 x 4096 x 4096    13.7  12.6
+        64 x 4096 x 2048    12.2   8.5     64 x 6144 x 2048    13.2  13.7
     """
     return numel <= 16 * k or n <= 4096 and (
         k <= 4096 and numel <= 32 * k or k <= 2048 and numel <= 64 * k)
@@ -281,11 +281,11 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
             and x.numel() > 0):
         return None
     n, k = weight.shape
-    # larger matrices' rows by mid_gemm.hip, in the same call
+    # more of them, and larger matrices' rows by mid_gemm.hip, in the same call
     if not (_rows_gemm_pays(x.numel(), n, k)
             or x.numel() <= 256 * k and not _compiling()
             and _load_ext() is not None
-            and _load_ext().mid_gemm_good(x.numel() // k, n, k, gated)):
+            and _load_ext().few_rows_good(x.numel() // k, n, k, gated)):
         return None
     if bias is not None and not (bias.dtype == torch.bfloat16
                                  and bias.device == x.device

@@ -59,6 +59,7 @@ void launch_grad_norm(float*, float*, const std::vector<OptTensor>&, hipStream_t
 void launch_adamw_f32(float*, const float*, float*, float*, long, float, float, float, float, float, int, float, hipStream_t);
 void launch_quant_gemv(bf16_t*, const bf16_t*, const void*, const unsigned char*, int, int, int, bool, hipStream_t);
 bool rows_gemm_takes(int, int, int, bool);
+bool rows_gemm_pays(int, int, int, bool);
 void launch_dequant(bf16_t*, const void*, const unsigned char*, long, int, bool, hipStream_t);
 void launch_dequant_k(bf16_t*, const void*, const unsigned char*, int, int, bool, hipStream_t);
 int decode_gemm_splitk(int, int);
@@ -536,6 +537,16 @@ bool mid_gemm_good(long m, long n, long k, bool paired) {
   return mid_gemm_takes(m, n, k, paired) && mid_gemm_pays(m, n, k, paired);
 }
 
+bool rows_gemm_good(long m, long n, long k, bool paired) {
+  return rows_gemm_takes((int)m, (int)n, (int)k, paired) &&
+         rows_gemm_pays((int)m, (int)n, (int)k, paired);
+}
+
+// Whether the library's product of these few rows would take longer.
+bool few_rows_good(long m, long n, long k, bool paired) {
+  return rows_gemm_good(m, n, k, paired) || mid_gemm_good(m, n, k, paired);
+}
+
 bool rows_gemm_ok(long m, long n, long k, bool gated) {
   return mid_gemm_good(m, n, k, gated) ||
          rows_gemm_takes((int)m, (int)n, (int)k, gated);
@@ -596,7 +607,8 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const int cols = heads ? n - 2 * heads->hkv * heads->d : gated ? n / 2 : n;
   TORCH_CHECK(w.dim() == 2 && w.size(1) == k && y.size(0) == m &&
               y.numel() == (long)m * cols, "rows_gemm: shape mismatch");
-  const bool many = norm == nullptr && mid_gemm_good(m, n, k, gated || heads);
+  const bool many = norm == nullptr && !rows_gemm_good(m, n, k, gated || heads) &&
+                    mid_gemm_good(m, n, k, gated || heads);
   TORCH_CHECK(many || rows_gemm_takes(m, n, k, gated || heads),
               "rows_gemm: unsupported shape ", m, "x", n, "x", k);
   TORCH_CHECK(aligned16(x) && aligned16(w), "rows_gemm: misaligned operand");
@@ -1024,6 +1036,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quant_heads", &quant_heads);
   m.def("rows_gemm_ok", &rows_gemm_ok);
   m.def("mid_gemm_good", &mid_gemm_good);
+  m.def("few_rows_good", &few_rows_good);
   m.def("quant_rows", &quant_rows);
   m.def("quant_rows_ok", &quant_rows_ok);
   m.def("quant_gemv", &quant_gemv);

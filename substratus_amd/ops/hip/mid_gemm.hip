@@ -281,11 +281,15 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 //   2048 and 2304                  x from 5632 on 1.02 to 2.4, 4096 0.6 to 1.1
 //   768 and 1024                   x 11008 0.97 to 2.9, 8192 0.8 to 1.2
 //   12288                          0.71 to 1.03, 0.85 to 1.2 x 2048
+// Paired ones of 17 to 64 rows up to 16384 x from 2048 on 1.02 to 1.5, of more
+// rows x 2048 and 3072 only up to 4096 (1.2 to 1.5; 6144 and 8192 0.93 to 1.1).
 bool mid_gemm_pays(long m, long n, long k, bool paired) {
   if (m <= 16 || m > 256 || n > 10240)
-    return paired && m > 16 && m <= 40 && n <= 16384 && k >= 4096;
+    return paired && m > 16 && m <= 64 && n <= 16384 && k >= 2048;
   if (k >= 16384) return true;
-  if (paired && (k >= 4096 || (k >= 2048 && n >= 3072))) return true;
+  if (paired && (k >= 4096 ||
+                 (k >= 2048 && n >= 3072 && (m <= 64 || n <= 4608))))
+    return true;
   if (n < 2048) return k >= 11008;
   if (n < 3072) return k >= 5632;
   if (k < 4096) return false;

@@ -201,6 +201,26 @@ bool rows_gemm_takes(int m, int n, int k, bool gated) {
          (!gated || n % 16 == 0);
 }
 
+// Whether the library's product of 17 to 64 rows takes longer, and mid_gemm.hip's:
+// every workgroup, 16 columns, reads all rows here, which costs less than few
+// tiles, or shares and their sums, where there are not many columns or they are
+// short. us, the library, mid_gemm, this, MI355X, weights from memory (17 to 64
+// rows, 512 to 16384 x 768 to 5632 measured):
+//   17 rows   4096 x 4096 13.4 11.8 9.3     8192 x 3072 18.4 15.2 13.4
+//   32        8192 x 2048 13.6 12.2 10.3   12288 x 2048 15.8 14.2 14.7
+//   48        4096 x 4096 13.7 12.6 12.6    5120 x 2048 12.7 11.9 11.7
+//             8192 x 2048 14.3 12.7 12.3   10240 x 2048 16.2 15.7 16.6
+//   64        4096 x 3072 16.1 12.7 12.2    4096 x 4096 15.2 13.3 14.5
+//             8192 x 1024 12.0  9.1  8.7    8192 x 2048 14.0 13.4 14.1
+// paired: the library's needs a launch more, gated 17 x 8192 x 4096 18.7 20.4 15.3.
+bool rows_gemm_pays(int m, int n, int k, bool paired) {
+  if (m <= 16) return true;
+  if (n <= 4096) return k <= (m <= 48 || n <= 1024 ? 4096 : 3072);
+  if (n > 8192) return n <= 12288 && k <= 2048 && m <= 32;
+  if (k <= (m <= 48 ? 2048 : 1024)) return true;
+  return n > 6144 && m <= 32 && k <= (paired ? 4096 : 3072);
+}
+
 // heads: null, or what is done with the columns instead of storing them (n is
 // a multiple of 16 then, like gated's)
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,

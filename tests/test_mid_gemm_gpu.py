@@ -43,6 +43,7 @@ def test_rows(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(17, 48, 4096), (70, 4112, 2080),
+                                   (17, 48, 4128), (64, 11264, 2080),
                                    (256, 320, 4128)])
 @torch.no_grad()
 def test_gated(m, n, k):

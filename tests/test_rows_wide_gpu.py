@@ -53,6 +53,33 @@ def test_rows(m, n, k):
                      + 1.1 * (rg * u.abs() + ru * g.abs())).all())
 
 
+# where matrices are wide or inner sizes long: the last that go here, and the
+# first that go elsewhere
+@pytest.mark.parametrize("m,n,k", [(48, 4096, 4096), (49, 4096, 3072),
+                                   (64, 1024, 4096), (48, 8192, 2048),
+                                   (49, 8192, 1024), (32, 12288, 2048),
+                                   (32, 6160, 3072), (32, 6160, 4096)])
+@torch.no_grad()
+def test_larger(m, n, k):
+    for rows, cols, inner in ((m, n, k), (m + 1, n, k), (m, n + 16, k),
+                              (m, n, k + 32)):
+        torch.manual_seed(rows + cols + inner)
+        w = torch.randn(cols, inner, device=DEV).bfloat16()
+        x = torch.randn(rows, inner, device=DEV).bfloat16()
+        prod = x.double() @ w.double().T
+        room = 2.0 ** -18 * (x.double().abs() @ w.double().abs().T)
+        off = (ops.linear(x, w).double() - prod).abs()
+        assert bool((off <= 2.0 ** -8 * prod.abs() + room + 1e-30).all())
+        y = ops.linear_gated(x * 0.03125, w)
+        if y is not None:
+            g, u = (prod * 0.03125).chunk(2, 1)
+            rg, ru = (room * 0.03125).chunk(2, 1)
+            want = torch.nn.functional.silu(g) * u
+            off = (y.double() - want).abs()
+            assert bool((off <= 2.0 ** -8 * want.abs() + 1e-6
+                         + 1.1 * (rg * u.abs() + ru * g.abs())).all())
+
+
 @pytest.mark.parametrize("m,hq,hkv,d,k", [(17, 2, 1, 16, 32),
                                           (40, 4, 2, 128, 160),
                                           (64, 3, 1, 64, 2048)])
