@@ -83,6 +83,12 @@ def gated_product(lin: nn.Module, y: torch.Tensor) -> torch.Tensor:
     return ops.silu_mul(lin(y)) if gated is None else gated(lin, y)
 
 
+def gelu_product(lin: nn.Module, y: torch.Tensor) -> torch.Tensor:
+    """ops.gelu(lin(y))"""
+    gelu = getattr(type(lin), "gelu", None)
+    return ops.gelu(lin(y)) if gelu is None else gelu(lin, y)
+
+
 class NormParams(nn.Module):
     def __init__(self, size: int, rms: bool, device=None, dtype=None):
         super().__init__()
@@ -158,7 +164,7 @@ class Block(nn.Module):
     def _mlp_up(self, y: torch.Tensor) -> torch.Tensor:
         if self.cfg.activation == "silu":
             return gated_product(self.w_gateup, y)
-        return ops.gelu(self.w_up(y))
+        return gelu_product(self.w_up, y)
 
     def _mlp(self, y: torch.Tensor) -> torch.Tensor:
         return self.w_down(self._mlp_up(y))

@@ -398,8 +398,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
     """F.linear. Up to 16 rows of bf16 without gradients, or up to 64 with a
     matrix of few rows, take the kernel that streams weights at the memory's
     rate (rows_gemm.hip), up to 256 rows the one for tiles of them where the
-    library's are too few (mid_gemm.hip), products of 256 rows and more the one for the matrix
-    cores (tile_gemm.hip) where that is the faster one, in a backward as well.
+    library's are too few (mid_gemm.hip), products of 256 rows and more the one
+    for the matrix cores (tile_gemm.hip) where that is the faster one, in a
+    backward as well.
     SUB_MGEMM=1 routes decode shapes of 256 rows and more to the 256x256 glds
     GEMM (mfma_gemm.hip).
 
@@ -459,6 +460,20 @@ def linear_gated(x: torch.Tensor, weight: torch.Tensor,
     y = rows.new_empty(rows.shape[0], n)
     ext.rows_gemm(y, rows, weight, bias, True)
     return y if x.dim() == 2 else y.view(*x.shape[:-1], n)
+
+
+def linear_gelu(x: torch.Tensor, weight: torch.Tensor,
+                bias: Optional[torch.Tensor] = None
+                ) -> Optional[torch.Tensor]:
+    """gelu of F.linear, in one kernel and bit by bit the same, or None where
+    it is not made for that."""
+    few = _few_rows(x, weight, bias, False)
+    if few is None or x.numel() // x.shape[-1] * weight.shape[0] % 8:
+        return None
+    rows, ext = few
+    y = rows.new_empty(rows.shape[0], weight.shape[0])
+    ext.rows_gemm(y, rows, weight, bias, False, True)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], weight.shape[0])
 
 
 class Cache(NamedTuple):

@@ -36,12 +36,6 @@ __global__ void silu_mul_kernel(bf16_t* __restrict__ out,
   }
 }
 
-DEV_INLINE float gelu_tanh_f(float v) {
-  const float c = 0.7978845608028654f;  // sqrt(2/pi)
-  float inner = c * (v + 0.044715f * v * v * v);
-  return 0.5f * v * (1.f + tanhf(inner));
-}
-
 template <int BLOCK>
 __global__ void gelu_kernel(bf16_t* __restrict__ out,
                             const bf16_t* __restrict__ x, long n8) {
@@ -55,7 +49,7 @@ __global__ void gelu_kernel(bf16_t* __restrict__ out,
     unsigned int o[4];
     #pragma unroll
     for (int j = 0; j < 4; ++j)
-      o[j] = pack_bf16x2(gelu_tanh_f(f[j].x), gelu_tanh_f(f[j].y));
+      o[j] = pack_bf16x2(gelu_of(f[j].x), gelu_of(f[j].y));
     ov[i] = make_uint4(o[0], o[1], o[2], o[3]);
   }
 }

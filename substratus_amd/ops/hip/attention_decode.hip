@@ -955,7 +955,8 @@ bool paged_attn_grouped(int hq, int hkv, int d, long q_ld, const void* q,
   return !kv8 && !ge && attn_group_takes(hq, hkv, d, q_ld, q, kc, vc);
 }
 
-// Flash-decoding shares of workgroups of two or four waves: enough for 1024 workgroups (256 CUs x 4 resident ones)
+// Flash-decoding shares of workgroups of two or four waves: enough for 1024
+// workgroups (256 CUs x 4 resident ones)
 // where the grid alone is too small (llama2-70b at TP=8: B x 1 x 1), but no more
 // than the longest sequence that the table has room for has steps for. By shapes
 // only, so that a captured graph holds them. What a workgroup takes is its

@@ -532,7 +532,8 @@ long mfma_gemm_pick_splitk(long m, long n, long k) {
 }
 
 // y = x w^T + bias, at most 64 rows of x, or up to 256 where that is faster than
-// the library; gated: y has half the columns, silu(first half) * second half
+// the library; gated: y has half the columns, silu(first half) * second half;
+// gelu: gelu of rounded columns
 bool mid_gemm_good(long m, long n, long k, bool paired) {
   return mid_gemm_takes(m, n, k, paired) && mid_gemm_pays(m, n, k, paired);
 }
@@ -596,7 +597,8 @@ void rope_split_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 
 void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> bias, bool gated,
-                  const Heads* heads, const NormOf* norm = nullptr) {
+                  const Heads* heads, const NormOf* norm = nullptr,
+                  bool gelu = false) {
   const c10::DeviceGuard guard(x.device());
   check_bf16(y, "y"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
@@ -625,19 +627,20 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
       part = torch::empty({plan.shares(m, n)},
                           x.options().dtype(torch::kFloat));
     launch_mid_gemm({bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols},
-                    plan, heads, gated,
+                    plan, heads, gated, gelu,
                     plan.shares(m, n) ? part.data_ptr<float>() : nullptr,
                     stream());
   } else {
     launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols,
-                     gated, heads, norm, stream());
+                     gated, gelu, heads, norm, stream());
   }
   post_launch_check("rows_gemm");
 }
 
 void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, bool gated) {
-  rows_gemm_to(y, x, w, bias, gated, nullptr);
+               c10::optional<torch::Tensor> bias, bool gated, bool gelu) {
+  TORCH_CHECK(!gated || !gelu, "rows_gemm: one activation");
+  rows_gemm_to(y, x, w, bias, gated, nullptr, nullptr, gelu);
 }
 
 // a b^T + bias for operands of many rows as they are stored: a [m, k], or [k, m]
@@ -1024,7 +1027,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_gemm_ok", &decode_gemm_ok);
   m.def("wstream_gemm", &wstream_gemm);
   m.def("wstream_ok", &wstream_ok);
-  m.def("rows_gemm", &rows_gemm);
+  m.def("rows_gemm", &rows_gemm, py::arg("y"), py::arg("x"), py::arg("w"),
+        py::arg("bias"), py::arg("gated"), py::arg("gelu") = false);
   m.def("tile_gemm", &tile_gemm, py::arg("a"), py::arg("b"), py::arg("bias"),
         py::arg("a_flipped"), py::arg("b_flipped"), py::arg("gated") = false);
   m.def("tile_gemm_good", &tile_gemm_good);

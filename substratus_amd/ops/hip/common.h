@@ -103,6 +103,12 @@ DEV_INLINE float block_max(float v, float* scratch) {
   return m;
 }
 
+DEV_INLINE float gelu_of(float v) {
+  const float c = 0.7978845608028654f;  // sqrt(2/pi)
+  float inner = c * (v + 0.044715f * v * v * v);
+  return 0.5f * v * (1.f + tanhf(inner));
+}
+
 #define HIP_CHECK_KERNEL()                                            \
   do {                                                                \
     hipError_t e_ = hipGetLastError();                                \

@@ -14,7 +14,8 @@ struct MidGemm {
   bool quads;
 };
 
-// A workgroup's rows (32, 64, 96 or 128) and tiles of 16 columns (4 or 8), and the workgroups that share the inner dimension.
+// A workgroup's rows (32, 64, 96 or 128) and tiles of 16 columns (4 or 8), and
+// the workgroups that share the inner dimension.
 struct MidPlan {
   int rows, tiles, splits;
   double us;                      // what it is to take
@@ -27,4 +28,4 @@ bool mid_gemm_takes(long m, long n, long k, bool paired);
 MidPlan mid_gemm_plan(long m, long n, long k);
 bool mid_gemm_pays(long m, long n, long k, bool paired);
 void launch_mid_gemm(const MidGemm& a, const MidPlan& plan, const Heads* heads,
-                     bool gated, float* part, hipStream_t stream);
+                     bool gated, bool gelu, float* part, hipStream_t stream);

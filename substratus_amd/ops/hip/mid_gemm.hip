@@ -41,7 +41,7 @@ DEV_INLINE void barrier() {
 // Weight tile t's first column, and how much later its second eight are.
 template <Columns C>
 DEV_INLINE int column_of(int t, const Heads& heads) {
-  if constexpr (C == Columns::PLAIN) return t * 16;
+  if constexpr (!paired(C)) return t * 16;
   const int at = t * 8;
   if constexpr (C == Columns::HEADS) {
     const int half = heads.d / 2;
@@ -57,12 +57,16 @@ DEV_INLINE void finish(const MidGemm& a, const Heads& heads, int r, int t, int c
                        float4v u, float4v v) {
   const int n0 = column_of<C>(t, heads), half = C == Columns::HEADS
       ? heads.d / 2 : a.n / 2;
-  if constexpr (C == Columns::PLAIN) {
+  if constexpr (!paired(C)) {
     const int col = n0 + c;
     if (col >= a.n) return;
     if (a.bias != nullptr) {
       #pragma unroll
       for (int e = 0; e < 4; ++e) u[e] += bf2f(a.bias[min(col + e, a.n - 1)]);
+    }
+    if constexpr (C == Columns::GELU) {
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) u[e] = gelu_of(bf2f(f2bf(u[e])));
     }
     bf16_t* to = a.y + r * a.y_ld + col;
     if (a.quads) {
@@ -199,11 +203,11 @@ void mid_gemm_kernel(MidGemm a, Heads heads, float* __restrict__ part) {
         continue;
       }
       float4v other = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (C != Columns::PLAIN)
+      if constexpr (paired(C))
         #pragma unroll
         for (int e = 0; e < 4; ++e)
           other[e] = __shfl_xor(acc[j][f][e], 32, WAVE);
-      if (there && (C == Columns::PLAIN || g < 2))
+      if (there && (!paired(C) || g < 2))
         finish<C>(a, heads, r, t, g * 4, acc[j][f], other);
     }
   }
@@ -214,7 +218,7 @@ template <Columns C>
 __global__ __launch_bounds__(256)
 void mid_sum_kernel(MidGemm a, Heads heads, const float* __restrict__ part,
                     int splits) {
-  constexpr int PER = C == Columns::PLAIN ? 4 : 2;
+  constexpr int PER = paired(C) ? 2 : 4;
   const int tiles = (a.n + 15) / 16;
   const long id = (long)blockIdx.x * 256 + threadIdx.x;
   const int r = id / (tiles * PER), e = id % (tiles * PER);
@@ -226,7 +230,7 @@ void mid_sum_kernel(MidGemm a, Heads heads, const float* __restrict__ part,
   #pragma unroll 4
   for (int s = 0; s < splits; ++s) {
     u += *reinterpret_cast<const float4v*>(p + s * step);
-    if constexpr (C != Columns::PLAIN)
+    if constexpr (paired(C))
       v += *reinterpret_cast<const float4v*>(p + s * step + 8);
   }
   finish<C>(a, heads, r, t, c, u, v);
@@ -303,7 +307,7 @@ bool mid_gemm_pays(long m, long n, long k, bool paired) {
 }
 
 void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
-                     const Heads* heads, bool gated, float* part,
+                     const Heads* heads, bool gated, bool gelu, float* part,
                      hipStream_t stream) {
   MidGemm a = given;
   a.blocks = (a.m + plan.rows - 1) / plan.rows;
@@ -316,6 +320,7 @@ void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
                   P = decltype(p)::value;
     auto kernel = heads ? mid_gemm_kernel<Columns::HEADS, F, N, P>
                   : gated ? mid_gemm_kernel<Columns::GATED, F, N, P>
+                  : gelu ? mid_gemm_kernel<Columns::GELU, F, N, P>
                           : mid_gemm_kernel<Columns::PLAIN, F, N, P>;
     kernel<<<dim3((tiles + N - 1) / N * a.blocks, plan.splits), WAVES * WAVE,
              0, stream>>>(a, h, part);
@@ -335,6 +340,7 @@ void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
   if (plan.splits > 1) {
     auto sum = heads ? mid_sum_kernel<Columns::HEADS>
                : gated ? mid_sum_kernel<Columns::GATED>
+               : gelu ? mid_sum_kernel<Columns::GELU>
                        : mid_sum_kernel<Columns::PLAIN>;
     const long quads = (long)a.m * tiles * (heads || gated ? 2 : 4);
     sum<<<dim3((quads + 255) / 256), 256, 0, stream>>>(a, h, part,

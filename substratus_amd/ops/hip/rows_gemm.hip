@@ -188,7 +188,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     } else if constexpr (C == Columns::HEADS) {
       if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
     } else {
-      if (n0 + c < n) y[r * y_ld + n0 + c] = f2bf(sum(c));
+      if (n0 + c < n) y[r * y_ld + n0 + c] = stored<C>(sum(c));
     }
   }
 }
@@ -225,7 +225,7 @@ bool rows_gemm_pays(int m, int n, int k, bool paired) {
 // a multiple of 16 then, like gated's)
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
-                      long y_ld, bool gated, const Heads* heads,
+                      long y_ld, bool gated, bool gelu, const Heads* heads,
                       const NormOf* norm, hipStream_t stream) {
   auto launch = [&](auto normed, auto tiles, auto stages) {
     constexpr bool N = decltype(normed)::value;
@@ -233,6 +233,8 @@ void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
     auto kernel = heads ? rows_gemm_kernel<Columns::HEADS, N, F, S>
                   : gated ? rows_gemm_kernel<Columns::GATED, N, F, S>
                           : rows_gemm_kernel<Columns::PLAIN, N, F, S>;
+    if constexpr (!N)
+      if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S>;
     kernel<<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
         y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{},
         norm ? *norm : NormOf{});

@@ -68,6 +68,11 @@ class Linear(nn.Module):
             if bare(self, Linear) else None
         return ops.silu_mul(self(x)) if y is None else y
 
+    def gelu(self, x: torch.Tensor) -> torch.Tensor:
+        y = ops.linear_gelu(x, self.weight, self.bias) \
+            if bare(self, Linear) else None
+        return ops.gelu(self(x)) if y is None else y
+
     def heads(self, x: torch.Tensor,
               cache: ops.Cache) -> Optional[torch.Tensor]:
         """ops.rope_kv_append of the outputs in the same kernel, or None."""
