@@ -271,6 +271,8 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // the chip where matrices are not wide. Its time over this one's, MI355X, 11 row
 // counts x 14 widths x 7 inner sizes (a paired one saves it a launch, too):
 //   inner size 18176               10240 and less 1.02 to 4, 12288 0.75 to 1.5
+//   8192 x 28672, 32768            17 to 28 rows 0.81 to 0.91, 32 1.03 and 0.90,
+//                                  40 and more 1.05 to 1.95
 //   17 to 32 rows                  up to 5120 x from 5120 on 1.0 to 2.9, but for
 //                                  4096 x 8192 (0.80 to 0.87); 6144 0.84 to 1.4,
 //                                  8192 0.79 to 0.96
@@ -290,7 +292,7 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 bool mid_gemm_pays(long m, long n, long k, bool paired) {
   if (m <= 16 || m > 256 || n > 10240)
     return paired && m > 16 && m <= 64 && n <= 16384 && k >= 2048;
-  if (k >= 16384) return true;
+  if (k >= 16384) return paired || m > 32 || n < 8192 || k < 24576;
   if (paired && (k >= 4096 ||
                  (k >= 2048 && n >= 3072 && (m <= 64 || n <= 4608))))
     return true;

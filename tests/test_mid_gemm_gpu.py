@@ -98,6 +98,13 @@ def test_heads(m, hq, hkv, d, k, theta):
         assert torch.equal(got == 0, want == 0)
 
 
+def test_long_sums_of_few_rows():
+    """Wide matrices of the longest rows are the library's up to 32 rows."""
+    for m, n, k, want in ((32, 8192, 24576, False), (33, 8192, 24576, True),
+                          (32, 8176, 24576, True), (32, 8192, 24544, True)):
+        assert _C.mid_gemm_good(m, n, k, False) == want
+
+
 @torch.no_grad()
 def test_in_a_graph():
     """Sums of shares come from memory of the graph's own."""
