@@ -899,8 +899,7 @@ def bench_attn_v5():
 
 
 def bench_attn_bwd():
-    """Backward kernels old-vs-V5, interleaved (falcon MQA + llama
-    shapes) — the dkv_v5 slowdown diagnosis harness."""
+    """Attention's backward (falcon MQA + llama shapes)."""
     from substratus_amd import _C
     shapes = [("falcon", 4, 71, 1, 64, 2048), ("llama", 4, 32, 32, 128, 2048)]
     for name, B, hq, hkv, d, S in shapes:
@@ -920,14 +919,10 @@ def bench_attn_bwd():
         dk = torch.zeros(t, hkv, d, dtype=torch.float32, device="cuda")
         dv = torch.zeros_like(dk)
         delta = torch.empty_like(lse)
-        import os as _os
-        for tag, env in (("mixed", None), ("dkv_v5", "1")):
-            if env: _os.environ["SUB_ATTN_DKV_V5"] = env
-            else: _os.environ.pop("SUB_ATTN_DKV_V5", None)
-            dt = timeit(lambda: _C.attn_train_bwd_v5(
-                dq, dk, dv, q, k, v, out, do, lse, delta, ss, S, scale),
-                iters=20)
-            print(f"bwd {name} [{tag}]: {dt*1e6:.0f} us")
+        dt = timeit(lambda: _C.attn_train_bwd(
+            dq, dk, dv, q, k, v, out, do, lse, delta, ss, S, scale),
+            iters=20)
+        print(f"bwd {name}: {dt*1e6:.0f} us")
 
 
 def bench_mgemm(m=512):
