@@ -310,9 +310,10 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
 def _tile_gemm(a: torch.Tensor, b: torch.Tensor,
                bias: Optional[torch.Tensor] = None, a_flipped: bool = False,
                b_flipped: bool = False,
-               gated: bool = False) -> Optional[torch.Tensor]:
+               gated: bool = False,
+               gelu: bool = False) -> Optional[torch.Tensor]:
     """a b^T + bias on tile_gemm.hip, a stored as [k, m] and b as [k, n] where
-    flipped, gated as linear_gated's, or None where it does not take them or
+    flipped, gated as linear_gated's, its gelu, or None where it does not take them or
     does not pay."""
     ext = _load_ext()
     m, k = a.shape[::-1] if a_flipped else a.shape
@@ -328,7 +329,7 @@ def _tile_gemm(a: torch.Tensor, b: torch.Tensor,
             and bias.is_contiguous() and bias.shape == (n,)
             and bias.data_ptr() % 16 == 0):
         return None
-    return ext.tile_gemm(a, b, bias, a_flipped, b_flipped, gated)
+    return ext.tile_gemm(a, b, bias, a_flipped, b_flipped, gated, gelu)
 
 
 class _Linear(torch.autograd.Function):
@@ -364,9 +365,10 @@ class _Linear(torch.autograd.Function):
 
 def _many_rows(x: torch.Tensor, weight: torch.Tensor,
                bias: Optional[torch.Tensor],
-               gated: bool = False) -> Optional[torch.Tensor]:
+               gated: bool = False,
+               gelu: bool = False) -> Optional[torch.Tensor]:
     """F.linear of 256 rows and more, or None where torch's is as good; or what
-    linear_gated makes of it, without gradients."""
+    linear_gated or linear_gelu makes of it, without gradients."""
     if not (x.is_cuda and weight.dim() == 2 and weight.shape[0] >= 256
             and x.dim() >= 2 and x.shape[-1] == weight.shape[1] > 0
             and x.numel() >= 256 * x.shape[-1] and not _compiling()
@@ -378,7 +380,7 @@ def _many_rows(x: torch.Tensor, weight: torch.Tensor,
     m, good = x.numel() // k, _load_ext().tile_gemm_good
     given = [t for t in (x, weight, bias) if t is not None]
     asked = torch.is_grad_enabled() and any(t.requires_grad for t in given)
-    if asked and gated or not (
+    if asked and (gated or gelu) or not (
             good(m, n, k, k, k, False, False, gated)
             or asked and (good(m, k, n, n, k, False, True, False)
                           or good(n, k, m, n, k, True, True, False))):
@@ -388,7 +390,7 @@ def _many_rows(x: torch.Tensor, weight: torch.Tensor,
         return None
     rows = x.reshape(-1, k)
     y = _Linear.apply(rows, weight, bias) if asked else \
-        _tile_gemm(rows, weight, bias, gated=gated)
+        _tile_gemm(rows, weight, bias, gated=gated, gelu=gelu)
     return y if y is None or x.dim() == 2 else \
         y.view(*x.shape[:-1], y.shape[1])
 
@@ -468,6 +470,8 @@ def linear_gelu(x: torch.Tensor, weight: torch.Tensor,
     """gelu of F.linear, in one kernel and bit by bit the same, or None where
     it is not made for that."""
     few = _few_rows(x, weight, bias, False)
+    if few is None and os.environ.get("SUB_MGEMM") != "1":
+        return _many_rows(x, weight, bias, gelu=True)
     if few is None or x.numel() // x.shape[-1] * weight.shape[0] % 8:
         return None
     rows, ext = few

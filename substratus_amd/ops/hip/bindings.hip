@@ -647,7 +647,7 @@ void rows_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
 // if flipped; b [n, k], or [k, n]. gated: silu(first half) * second half.
 torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
                         c10::optional<torch::Tensor> bias, bool a_flipped,
-                        bool b_flipped, bool gated) {
+                        bool b_flipped, bool gated, bool gelu) {
   const c10::DeviceGuard guard(a.device());
   for (const auto& t : {a, b})
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
@@ -656,6 +656,8 @@ torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
   const long m = a.size(a_flipped), k = a.size(!a_flipped);
   const long n = b.size(b_flipped);
   TORCH_CHECK(b.size(!b_flipped) == k, "inner dimensions differ");
+  TORCH_CHECK(!gelu || !(gated || a_flipped || b_flipped),
+              "tile_gemm: gelu is of rows by rows, and the one activation");
   TORCH_CHECK(tile_gemm_takes(m, n, k, a.stride(0), b.stride(0), a_flipped,
                               b_flipped, gated),
               "tile_gemm: unsupported shape ", m, "x", n, "x", k);
@@ -667,7 +669,7 @@ torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
     shares = torch::empty({plan.shares()}, a.options().dtype(torch::kFloat));
   launch_tile_gemm({bf(out), bfc(a), bfc(b), bias ? bfc(*bias) : nullptr,
                     (int)m, (int)n, (int)k, a.stride(0), b.stride(0),
-                    a_flipped, b_flipped, gated},
+                    a_flipped, b_flipped, gated, gelu},
                    plan, plan.shares() ? shares.data_ptr<float>() : nullptr,
                    stream());
   post_launch_check("tile_gemm");
@@ -1030,7 +1032,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_gemm", &rows_gemm, py::arg("y"), py::arg("x"), py::arg("w"),
         py::arg("bias"), py::arg("gated"), py::arg("gelu") = false);
   m.def("tile_gemm", &tile_gemm, py::arg("a"), py::arg("b"), py::arg("bias"),
-        py::arg("a_flipped"), py::arg("b_flipped"), py::arg("gated") = false);
+        py::arg("a_flipped"), py::arg("b_flipped"), py::arg("gated") = false,
+        py::arg("gelu") = false);
   m.def("tile_gemm_good", &tile_gemm_good);
   m.def("rows_heads", &rows_heads);
   m.def("rows_normed", &rows_normed);

@@ -231,9 +231,9 @@ DEV_INLINE float silu_times(float g, float u) {
 
 // A column as it is stored. Rounded before its gelu, as gelu_kernel has it, so
 // the bits are that kernel's: a launch less. us, MI355X, product and gelu ->
-// one kernel: 1 x 3072 x 768 5.8 -> 3.4, 32 rows 6.8 -> 4.3, 64 rows 7.9 -> 5.6;
-// 1 x 18176 x 4544 34.0 -> 31.4, 16 rows 38.3 -> 35.7; 4 x 32768 x 8192 101.0 ->
-// 98.2.
+// one kernel: 1 x 3072 x 768 5.4 -> 3.4, 32 rows 6.4 -> 4.2, 64 rows 7.4 -> 5.3;
+// 1 x 18176 x 4544 33.4 -> 31.3, 16 rows 37.6 -> 35.4; 4 x 32768 x 8192 100.3 ->
+// 97.6.
 template <Columns C>
 DEV_INLINE bf16_t stored(float v) {
   return f2bf(C == Columns::GELU ? gelu_of(bf2f(f2bf(v))) : v);

@@ -24,6 +24,8 @@ struct TileGemm {
   bool a_flipped, b_flipped;
   // the first n / 2 columns gate the others: out [m, n / 2] = silu(gate) * up
   bool gated;
+  // out is the gelu of the rounded columns; of operands that are not flipped
+  bool gelu;
 };
 
 bool tile_gemm_takes(long m, long n, long k, long a_ld, long b_ld,

@@ -226,7 +226,17 @@ DEV_INLINE float4v gate(float4v a, float4v u) {
   return v;
 }
 
-template <bool FA, bool FB, bool GATED>
+// The gelu of rounded numbers, as gelu_kernel has it: a pass over memory less. us,
+// MI355X, 18176 x 4544, product and gelu -> one kernel: 700 rows 108.6 -> 105.9,
+// 2000 280.5 -> 266.3, 8000 996 -> 938.
+DEV_INLINE float4v gelu(float4v a) {
+  float4v v;
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = gelu_of(bf2f(f2bf(a[e])));
+  return v;
+}
+
+template <bool FA, bool FB, bool GATED, bool GELU = false>
 __global__ __launch_bounds__(THREADS, 2)
 void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   // [two steps][a low, a high, b low, b high]
@@ -433,6 +443,10 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
     const int row = it.m0 + out_row(tid, i);
     #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] += add[j];
+    if constexpr (GELU) {
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = gelu(acc[i][j]);
+    }
     if constexpr (GATED) {
       store(g, n, row, col_of<true>(g, it.n0, tid, 0),
             gate(acc[i][0], acc[i][2]), gate(acc[i][1], acc[i][3]));
@@ -447,7 +461,7 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
 
 // The shares of the tiles left over are added up, an eighth of a tile per
 // workgroup.
-template <bool GATED>
+template <bool GATED, bool GELU = false>
 __global__ __launch_bounds__(THREADS)
 void tile_sum_kernel(TileGemm g, TilePlan plan,
                      const float4v* __restrict__ shares) {
@@ -466,6 +480,10 @@ void tile_sum_kernel(TileGemm g, TilePlan plan,
       v[j] += from[(long)p * 32 * THREADS + j * THREADS];
   #pragma unroll
   for (int j = 0; j < 4; ++j) v[j] += bias_of(g, col_of<GATED>(g, n0, tid, j));
+  if constexpr (GELU) {
+    #pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = gelu(v[j]);
+  }
   const int row = m0 + out_row(tid, i);
   if constexpr (GATED) {
     store(g, g.n / 2, row, col_of<true>(g, n0, tid, 0), gate(v[0], v[2]),
@@ -559,6 +577,7 @@ void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,
   float4v* sh = reinterpret_cast<float4v*>(shares);
   const dim3 grid(plan.whole + plan.rest() * plan.split);
   auto kernel = g.gated ? tile_gemm_kernel<false, false, true>
+      : g.gelu ? tile_gemm_kernel<false, false, false, true>
       : g.a_flipped
           ? (g.b_flipped ? tile_gemm_kernel<true, true, false>
                          : tile_gemm_kernel<true, false, false>)
@@ -566,7 +585,9 @@ void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,
                          : tile_gemm_kernel<false, false, false>);
   kernel<<<grid, dim3(THREADS), 0, stream>>>(g, plan, sh);
   if (plan.split > 1) {
-    auto sum = g.gated ? tile_sum_kernel<true> : tile_sum_kernel<false>;
+    auto sum = g.gated ? tile_sum_kernel<true>
+               : g.gelu ? tile_sum_kernel<false, true>
+                        : tile_sum_kernel<false>;
     sum<<<dim3(plan.rest(), 8), dim3(THREADS), 0, stream>>>(g, plan, sh);
   }
 }
