@@ -71,6 +71,30 @@ def normed_product(lin: nn.Module, deltas: tuple, h: torch.Tensor,
     return normed(lin, deltas[0], h, norm.weight, eps, **how)
 
 
+def added_product(lin: nn.Module, x: torch.Tensor, h: torch.Tensor,
+                  norm: Optional["NormParams"]) -> tuple:
+    """(h + lin(x), what of norm's rows is there already), or h and what is
+    still to be added to it."""
+    added = getattr(type(lin), "added", None)
+    if added is not None and norm is not None and bare(norm, NormParams) \
+            and norm.rms:
+        got = added(lin, x, h, norm.weight)
+        if got is not None:
+            return got
+    return h, (lin(x),)
+
+
+def scaled_product(lin: nn.Module, deltas: tuple, h: torch.Tensor,
+                   norm: "NormParams", eps: float, **how):
+    """(lin of norm(h + deltas), h + deltas) in one kernel, or None, and what
+    is still to be added to h."""
+    if not isinstance(deltas, ops.Undivided):
+        return normed_product(lin, deltas, h, norm, eps, **how), deltas
+    scaled = getattr(type(lin), "scaled", None)
+    y = None if scaled is None else scaled(lin, deltas, eps, **how)
+    return None if y is None else (y, h), ()
+
+
 def heads_product(lin: nn.Module, y: torch.Tensor, cache: ops.Cache):
     """ops.rope_kv_append of lin(y) in one kernel, or None."""
     heads = getattr(type(lin), "heads", None)
@@ -174,7 +198,8 @@ class Block(nn.Module):
                    positions: torch.Tensor,
                    k_cache: torch.Tensor, v_cache: torch.Tensor,
                    slots: torch.Tensor, block_table: torch.Tensor,
-                   seq_lens: torch.Tensor):
+                   seq_lens: torch.Tensor,
+                   after: Optional[NormParams] = None):
         """Generator form of the decode block: yields after each op group
         (norm + qkv GEMM | rope+attention | o GEMM | up GEMM | down GEMM) so
         the dual-stream runner (serve/graph_runner.py) can interleave two
@@ -185,10 +210,13 @@ class Block(nn.Module):
         construction identical.
 
         h: the residual stream, deltas: what is still to be added to it, which
-        this block's first norm does; the same is returned."""
+        this block's first norm does, or ops.Undivided, what is there of that
+        norm already; the same is returned, the latter of the norm after."""
         cache = ops.Cache(positions, k_cache, v_cache, slots, self.rope_theta)
-        got = None if self.parallel_attn else normed_product(
-            self.wqkv, deltas, h, self.norm1, self.eps, cache=cache)
+        got = None
+        if not self.parallel_attn:
+            got, deltas = scaled_product(self.wqkv, deltas, h, self.norm1,
+                                         self.eps, cache=cache)
         if got is not None:
             q, h = got
         else:
@@ -202,25 +230,29 @@ class Block(nn.Module):
         a = ops.paged_attn_decode(q, k_cache, v_cache, block_table, seq_lens,
                                   self.scale)
         yield
-        attn_out = self.wo(a.reshape(a.shape[0], -1))
-        yield
+        a = a.reshape(a.shape[0], -1)
         if self.parallel_attn:
+            attn_out = self.wo(a)
+            yield
             if self.parallel_norms:
                 y = self.norm2(h, self.eps)
             up = self._mlp_up(y)
             yield
             return h, (attn_out, self.w_down(up))
+        silu = self.cfg.activation == "silu"
+        h, deltas = added_product(self.wo, a, h, self.norm2 if silu else None)
+        yield
         got = None
-        if self.cfg.activation == "silu":
-            got = normed_product(self.w_gateup, (attn_out,), h, self.norm2,
-                                 self.eps, gated=True)
+        if silu:
+            got, deltas = scaled_product(self.w_gateup, deltas, h, self.norm2,
+                                         self.eps, gated=True)
         if got is not None:
             up, h = got
         else:
-            y, h = fused_norm_residual((attn_out,), h, self.norm2, self.eps)
+            y, h = fused_norm_residual(deltas, h, self.norm2, self.eps)
             up = self._mlp_up(y)
         yield
-        return h, (self.w_down(up),)
+        return added_product(self.w_down, up, h, after)
 
     # -- prefill ------------------------------------------------------------
     def forward_prefill(self, h: torch.Tensor, deltas: tuple,
@@ -340,16 +372,20 @@ class CausalLM(nn.Module):
         # each block's outputs are added to the residual stream inside the
         # NEXT norm
         deltas = ()
-        for blk, (kc, vc) in zip(self.blocks, kv_caches):
+        norms = [getattr(blk, "norm1", None) for blk in self.blocks[1:]]
+        for blk, after, (kc, vc) in zip(
+                self.blocks, [*norms, self.final_norm], kv_caches):
             h, deltas = yield from blk.decode_ops(h, deltas, positions, kc,
                                                   vc, slots, block_table,
-                                                  seq_lens)
+                                                  seq_lens, after)
             yield
         if self.lm_head is not None:
-            got = normed_product(self.lm_head, deltas, h, self.final_norm,
-                                 self.eps)
+            got, deltas = scaled_product(self.lm_head, deltas, h,
+                                         self.final_norm, self.eps)
             if got is not None:
                 return got[0]
+        elif isinstance(deltas, ops.Undivided):
+            deltas = ()
         y, _ = fused_norm_residual(deltas, h, self.final_norm, self.eps)
         return self._logits(y)
 

@@ -240,6 +240,40 @@ class QuantLinear(nn.Module):
         return y, total
 
 
+    def added(self, x: torch.Tensor, h: torch.Tensor, norm: torch.Tensor):
+        """(h + the outputs, RMSNorm of that but for its division) in one
+        kernel, or None."""
+        if self.bias is not None or not bare(self, QuantLinear) or \
+                x.dim() != 2 or x.dtype != torch.bfloat16 or \
+                x.device != h.device or x.shape[1] != self.in_features or \
+                not ops.may_add(h, norm, x.shape[0], self.out_features):
+            return None
+        ext = self._few_rows(x, False)
+        if ext is None or not ops.inference_only(x):
+            return None
+        total, parts = ops.room_for_added(h)
+        ext.quant_added(parts.rows, total, parts.squares, x.contiguous(),
+                        self.scales, self.qs, self.quant, h, norm)
+        return total, parts
+
+    def scaled(self, x: ops.Undivided, eps: float, gated: bool = False,
+               cache: Optional[ops.Cache] = None) -> Optional[torch.Tensor]:
+        """The outputs for rows that are still to be divided, gated or appended
+        as above, in one kernel, or None."""
+        m, n = x.rows.shape[0], self.out_features
+        if self.bias is not None or not bare(self, QuantLinear) or \
+                x.rows.shape[1] != self.in_features or \
+                not ops.inference_only(x.rows):
+            return None
+        ext = self._few_rows(x.rows, gated or cache is not None)
+        if ext is None or cache is not None and not cache.takes(x.rows, n):
+            return None
+        y = x.rows.new_empty(*ops._columns(m, n, gated, cache))
+        ext.quant_scaled(y, *x, eps, self.scales, self.qs, self.quant, gated,
+                         *(cache or (None,) * 4 + (0.0,)))
+        return y
+
+
 def quantize_model(model: nn.Module, quant: str) -> nn.Module:
     """Swap every projection Linear (wqkv/wo/w_gateup/w_up/w_down, lm_head)
     for a QuantLinear; embeddings and norms stay bf16."""

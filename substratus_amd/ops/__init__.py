@@ -580,6 +580,64 @@ def linear_normed(delta: torch.Tensor, h: torch.Tensor, norm: torch.Tensor,
     return y, total
 
 
+class Undivided(NamedTuple):
+    """An RMSNorm's rows but for the division by their deviations: rounded
+    h * weight, and parts of every row's squares of h, [rows, n / 16] of 32
+    bits."""
+    rows: torch.Tensor
+    squares: torch.Tensor
+
+
+def may_add(h: torch.Tensor, norm: torch.Tensor, rows: int, n: int) -> bool:
+    """Whether a product of these rows and columns may be added to h, and make
+    the rows of the norm that follows."""
+    return (h.shape == (rows, n) and norm.shape == (n,) and n % 64 == 0
+            and all(t.is_cuda and t.device == h.device
+                    and t.dtype == torch.bfloat16 and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (h, norm))
+            and inference_only(h, norm))
+
+
+def room_for_added(h: torch.Tensor) -> tuple[torch.Tensor, Undivided]:
+    """Room for h + a product, and for its norm's rows."""
+    return torch.empty_like(h), Undivided(torch.empty_like(h), h.new_empty(
+        h.shape[0], h.shape[1] // 16, dtype=torch.float32))
+
+
+def linear_added(x: torch.Tensor, weight: torch.Tensor,
+                 bias: Optional[torch.Tensor], h: torch.Tensor,
+                 norm: torch.Tensor
+                 ) -> Optional[tuple[torch.Tensor, Undivided]]:
+    """(h + F.linear, RMSNorm of that by the weight norm, undivided) in one
+    kernel, or None where it is not made for that. Up to 16 rows: with more of
+    them the products that would take such rows are other kernels'."""
+    few = _few_rows(x, weight, bias, False)
+    if few is None or x.dim() != 2 or x.shape[0] > 16 \
+            or x.device != h.device \
+            or not may_add(h, norm, x.shape[0], weight.shape[0]):
+        return None
+    total, parts = room_for_added(h)
+    few[1].rows_added(parts.rows, total, parts.squares, few[0], weight, bias,
+                      h, norm)
+    return total, parts
+
+
+def linear_scaled(x: Undivided, eps: float, weight: torch.Tensor,
+                  bias: Optional[torch.Tensor], gated: bool = False,
+                  cache: Optional[Cache] = None) -> Optional[torch.Tensor]:
+    """What becomes of F.linear of x divided, gated as linear_gated's, or with a
+    cache linear_heads' queries; or None."""
+    few = _few_rows(x.rows, weight, bias, gated or cache is not None)
+    m, n = x.rows.shape[0], weight.shape[0]
+    if few is None or m > 16 \
+            or cache is not None and not cache.takes(x.rows, n):
+        return None
+    y = x.rows.new_empty(*_columns(m, n, gated, cache))
+    few[1].rows_scaled(y, *x, eps, weight, bias, gated,
+                       *(cache or (None,) * 4 + (0.0,)))
+    return y
+
+
 def _columns(m: int, n: int, gated: bool, cache: Optional[Cache]) -> tuple:
     if cache is None:
         return m, n // 2 if gated else n

@@ -604,7 +604,8 @@ void rope_split_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> bias, bool gated,
                   const Heads* heads, const NormOf* norm = nullptr,
-                  bool gelu = false) {
+                  bool gelu = false, const AddTo* add = nullptr,
+                  const Undivided* of = nullptr) {
   const c10::DeviceGuard guard(x.device());
   check_bf16(y, "y"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
@@ -615,7 +616,7 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const int cols = heads ? n - 2 * heads->hkv * heads->d : gated ? n / 2 : n;
   TORCH_CHECK(w.dim() == 2 && w.size(1) == k && y.size(0) == m &&
               y.numel() == (long)m * cols, "rows_gemm: shape mismatch");
-  const bool many = norm == nullptr && !rows_gemm_good(m, n, k, gated || heads) &&
+  const bool many = !(norm || add || of) && !rows_gemm_good(m, n, k, gated || heads) &&
                     mid_gemm_good(m, n, k, gated || heads);
   TORCH_CHECK(many || rows_gemm_takes(m, n, k, gated || heads),
               "rows_gemm: unsupported shape ", m, "x", n, "x", k);
@@ -638,7 +639,7 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     stream());
   } else {
     launch_rows_gemm(bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols,
-                     gated, gelu, heads, norm, stream());
+                     gated, gelu, heads, norm, add, of, stream());
   }
   post_launch_check("rows_gemm");
 }
@@ -707,7 +708,9 @@ bool quant_rows_ok(long m, long n, long k, const std::string& quant,
 
 void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
                    torch::Tensor qs, const std::string& quant, bool gated,
-                   const Heads* heads, const NormOf* norm = nullptr) {
+                   const Heads* heads, const NormOf* norm = nullptr,
+                   const AddTo* add = nullptr,
+                   const Undivided* of = nullptr) {
   const c10::DeviceGuard guard(x.device());
   check_bf16(y, "y"); check_bf16(x, "x");
   TORCH_CHECK(scales.scalar_type() == torch::kHalf, "scales must be fp16");
@@ -726,7 +729,7 @@ void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
   if (!aligned16(scales)) scales = scales.clone();
   launch_rows_quant(bf(y), bfc(x), scales.data_ptr(),
                     qs.data_ptr<unsigned char>(), m, n, k, q, gated, heads,
-                    norm, stream());
+                    norm, add, of, stream());
   post_launch_check("quant_rows");
 }
 
@@ -761,6 +764,76 @@ struct Where {
     return &heads;
   }
 };
+
+// A product that is added to the residual stream: total = h + its rows, y =
+// total * weight, and every row's squares in parts, one of 16 columns.
+AddTo add_of(const torch::Tensor& y, const torch::Tensor& total,
+             const torch::Tensor& squares, const torch::Tensor& h,
+             const torch::Tensor& weight) {
+  const long n = weight.numel();
+  TORCH_CHECK(h.dim() == 2 && h.size(1) == n && n % 64 == 0 &&
+              y.dim() == 2 && y.sizes() == h.sizes(), "added rows: shapes");
+  check_rows(weight, n, "norm weight");
+  check_rows(h, h.numel(), "h"); check_rows(total, h.numel(), "total");
+  TORCH_CHECK(squares.is_cuda() && squares.is_contiguous() &&
+              squares.scalar_type() == torch::kFloat &&
+              squares.numel() == h.size(0) * (n / 16), "squares");
+  return {bfc(h), bfc(weight), const_cast<bf16_t*>(bfc(total)),
+          squares.data_ptr<float>()};
+}
+
+// Rows x that are an RMSNorm's but for the division by its deviations.
+Undivided undivided_of(const torch::Tensor& x, const torch::Tensor& squares,
+                       double eps) {
+  TORCH_CHECK(x.dim() == 2 && squares.dim() == 2 && squares.is_cuda() &&
+              squares.is_contiguous() && aligned16(squares) &&
+              squares.scalar_type() == torch::kFloat &&
+              squares.size(0) == x.size(0) && squares.size(1) % 4 == 0,
+              "squares");
+  return {squares.data_ptr<float>(), (int)squares.size(1), (float)eps};
+}
+
+void rows_added(torch::Tensor y, torch::Tensor total, torch::Tensor squares,
+                torch::Tensor x, torch::Tensor w,
+                c10::optional<torch::Tensor> bias, torch::Tensor h,
+                torch::Tensor weight) {
+  const AddTo add = add_of(y, total, squares, h, weight);
+  rows_gemm_to(y, x, w, bias, false, nullptr, nullptr, false, &add);
+}
+
+void rows_scaled(torch::Tensor y, torch::Tensor x, torch::Tensor squares,
+                 double eps, torch::Tensor w,
+                 c10::optional<torch::Tensor> bias, bool gated,
+                 c10::optional<torch::Tensor> positions,
+                 c10::optional<torch::Tensor> k_cache,
+                 c10::optional<torch::Tensor> v_cache,
+                 c10::optional<torch::Tensor> slots, double theta) {
+  Where where{positions, k_cache, v_cache, slots, theta};
+  const Undivided of = undivided_of(x, squares, eps);
+  rows_gemm_to(y, x, w, bias, gated, where.of(y), nullptr, false, nullptr,
+               &of);
+}
+
+void quant_added(torch::Tensor y, torch::Tensor total, torch::Tensor squares,
+                 torch::Tensor x, torch::Tensor scales, torch::Tensor qs,
+                 const std::string& quant, torch::Tensor h,
+                 torch::Tensor weight) {
+  const AddTo add = add_of(y, total, squares, h, weight);
+  quant_rows_to(y, x, scales, qs, quant, false, nullptr, nullptr, &add);
+}
+
+void quant_scaled(torch::Tensor y, torch::Tensor x, torch::Tensor squares,
+                  double eps, torch::Tensor scales, torch::Tensor qs,
+                  const std::string& quant, bool gated,
+                  c10::optional<torch::Tensor> positions,
+                  c10::optional<torch::Tensor> k_cache,
+                  c10::optional<torch::Tensor> v_cache,
+                  c10::optional<torch::Tensor> slots, double theta) {
+  Where where{positions, k_cache, v_cache, slots, theta};
+  const Undivided of = undivided_of(x, squares, eps);
+  quant_rows_to(y, x, scales, qs, quant, gated, where.of(y), nullptr, nullptr,
+                &of);
+}
 
 void rows_normed(torch::Tensor y, torch::Tensor sum, torch::Tensor delta,
                  torch::Tensor h, torch::Tensor norm, double eps,
@@ -1038,6 +1111,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_heads", &rows_heads);
   m.def("rows_normed", &rows_normed);
   m.def("quant_normed", &quant_normed);
+  m.def("rows_added", &rows_added);
+  m.def("rows_scaled", &rows_scaled);
+  m.def("quant_added", &quant_added);
+  m.def("quant_scaled", &quant_scaled);
   m.def("norm_rows_take", &norm_rows_take);
   m.def("rope_split_append", &rope_split_append);
   m.def("quant_heads", &quant_heads);

@@ -41,7 +41,8 @@ DEV_INLINE void wait_lds_reads() {
 //   HEADS  of a fused projection of query, key and value heads: eight are
 //          rotated with another eight, half a head later; queries are stored,
 //          keys and values go to the paged cache
-enum class Columns { PLAIN, GATED, HEADS, GELU };
+//   ADDED  they are added to the residual stream (AddTo)
+enum class Columns { PLAIN, GATED, HEADS, GELU, ADDED };
 
 // Whether a workgroup has eight columns and another eight that go with them.
 constexpr bool paired(Columns c) {
@@ -76,7 +77,63 @@ DEV_INLINE int second_half(int n, const Heads& heads) {
   return C == Columns::HEADS ? heads.d / 2 : n / 2;
 }
 
-// x as the norm of a sum, made by the product itself: RMS of h + delta, which
+// What becomes of a product that is added to the residual stream h, whose RMSNorm
+// the next product takes: sum = h + the columns, rounded, y = sum * weight, and
+// each workgroup's part of every row's squares. A row's 1/deviation only scales
+// the results of that product, which adds the parts up while its first weights
+// are on their way (Undivided): no launch for the norm, and nothing of it is made
+// by every workgroup. us of a captured decode step on a MI355X, from a launch for
+// each norm of 5 rows and more, and NormOf's of fewer, to this: 890 -> 848 (8
+// rows, 8 layers of 4096), 685 -> 653 (5 rows, 6 layers of 5120, q4_K), 600 -> 568
+// (1 row, 8 layers of 5120, q4_0), 620 -> 617 (1 row, 16 layers of 2048).
+struct AddTo {
+  const bf16_t *h, *weight;     // [m, n], [n]
+  bf16_t* sum;                  // [m, n]
+  float* squares;               // [m, workgroups]
+};
+struct Undivided {
+  const float* squares;         // [m, parts], or null: nothing is divided
+  int parts;                    // a multiple of 4
+  float eps;
+};
+
+// A row's sum of squares for the 16 lanes that ask for it: what a lane adds up is
+// asked for behind a workgroup's first weights.
+struct RowSquares {
+  static constexpr int PER = 5;
+  float4 v[PER];
+  float rest;
+
+  DEV_INLINE void load(const Undivided& of, int r) {
+    const float* row = of.squares + (long)r * of.parts;
+    const int at = threadIdx.x % 16 * 4;
+    #pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (i * 64 < of.parts)
+        v[i] = *reinterpret_cast<const float4*>(
+            row + min(at + i * 64, of.parts - 4));
+    rest = 0.f;
+    for (int j = at + PER * 64; j < of.parts; j += 64) {
+      const float4 u = *reinterpret_cast<const float4*>(row + j);
+      rest += u.x + u.y + (u.z + u.w);
+    }
+  }
+  DEV_INLINE float sum(const Undivided& of) const {
+    const int at = threadIdx.x % 16 * 4;
+    float s = rest;
+    #pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (at + i * 64 < of.parts) s += v[i].x + v[i].y + (v[i].z + v[i].w);
+    return group16_sum(s);
+  }
+};
+
+DEV_INLINE float undivided_scale(const Undivided& of, float squares, int k) {
+  return rsqrtf(squares / (float)k + of.eps);
+}
+
+// x as the norm of a sum, made by the product itself, where what is added has to be
+// summed over ranks first: RMS of h + delta, which
 // the first workgroup stores in sum. A row's 1/deviation only scales its
 // results, so a workgroup multiplies (h + delta) * weight, rounded like a
 // normed row, and scales at the end; it sums squares meanwhile. On a MI355X, us
@@ -223,10 +280,25 @@ DEV_INLINE void finish_heads(bf16_t* y, long y_ld, const Heads& heads, int r,
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
                       long y_ld, bool gated, bool gelu, const Heads* heads,
-                      const NormOf* norm, hipStream_t stream);
+                      const NormOf* norm, const AddTo* add,
+                      const Undivided* of, hipStream_t stream);
 
 DEV_INLINE float silu_times(float g, float u) {
   return g / (1.f + __expf(-g)) * u;
+}
+
+// One of a row's 16 columns that a workgroup adds, the others in the lanes beside
+// it (past the last one h, weight and v are 0).
+DEV_INLINE void finish_added(const AddTo& add, bf16_t* y, long at, int r,
+                             bool there, float h, float weight, float v) {
+  const float s = bf2f(f2bf(h + bf2f(f2bf(v))));
+  if (there) {
+    add.sum[at] = f2bf(s);
+    y[at] = f2bf(s * weight);
+  }
+  const float squares = group16_sum(s * s);
+  if (threadIdx.x % 16 == 0)
+    add.squares[(long)r * gridDim.x + blockIdx.x] = squares;
 }
 
 // A column as it is stored. Rounded before its gelu, as gelu_kernel has it, so

@@ -50,8 +50,8 @@ __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       const bf16_t* __restrict__ w,
                       const bf16_t* __restrict__ bias, int m, int n, int k,
-                      long x_ld, long y_ld, Heads heads,
-                      NormOf norm) {
+                      long x_ld, long y_ld, Heads heads, NormOf norm,
+                      AddTo add, Undivided of) {
   // (normed x does not go through the ring)
   static_assert(!NORM || FM == 1);
   constexpr int TILES = NORM ? 1 : 1 + FM;       // of a chunk of 32 columns
@@ -135,11 +135,27 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
               wf[u], xf[u][f], acc[f], 0, 0, 0);
       }
   };
+  // a thread ends up with column c of rows from row on
+  const int c = threadIdx.x % 16, first = threadIdx.x / 16;
+  bf16_t h[FM], weight;
+  RowSquares parts[FM];
   NormRows<KW * WAVE> rows;
   if constexpr (NORM) rows.load(norm, m, k);
   #pragma unroll
   for (int s = 0; s < P; ++s)
     if (s < steps) load(s, s);
+  if constexpr (C == Columns::ADDED) {
+    const int at = min(n0 + c, n - 1);
+    #pragma unroll
+    for (int f = 0; f < FM; ++f)
+      h[f] = add.h[(long)min(first + f * 16, m - 1) * n + at];
+    weight = add.weight[at];
+  } else if (!NORM && of.squares != nullptr) {
+    // waited for at the end (added up here, 643 us instead of 616 for a step of
+    // 16 layers of 2048, one row)
+    #pragma unroll
+    for (int f = 0; f < FM; ++f) parts[f].load(of, min(first + f * 16, m - 1));
+  }
   if constexpr (NORM) {
     rows.put(norm, m, k, s_x, squares);
     lds_barrier();
@@ -172,14 +188,19 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     *reinterpret_cast<float4v*>(
         &red[(wave * ROWS + f * 16 + lo) * (16 + PAD) + g * 4]) = acc[f];
   __syncthreads();
-  const int c = threadIdx.x % 16;
-  for (int r = threadIdx.x / 16; r < m; r += KW * 4) {
-    const float scale = NORM ? norm_scale<KW>(squares, r, k, norm.eps) : 1.f;
+  #pragma unroll
+  for (int f = 0; f < FM; ++f) {
+    const int r = first + f * 16;
+    if (r >= m) break;
+    float scale = 1.f;
+    if constexpr (NORM) scale = norm_scale<KW>(squares, r, k, norm.eps);
+    else if (C != Columns::ADDED && of.squares != nullptr)
+      scale = undivided_scale(of, parts[f].sum(of), k);
     auto sum = [&](int c) {
       float v = 0.f;
       #pragma unroll
       for (int q = 0; q < KW; ++q) v += red[(q * ROWS + r) * (16 + PAD) + c];
-      if constexpr (NORM) v *= scale;
+      v *= scale;
       if (bias != nullptr) v += bf2f(bias[weight_row<C>(n0, c, n, half)]);
       return v;
     };
@@ -187,6 +208,10 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       if (c < 8) y[r * y_ld + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
     } else if constexpr (C == Columns::HEADS) {
       if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
+    } else if constexpr (C == Columns::ADDED) {
+      const bool there = n0 + c < n;
+      finish_added(add, y, r * y_ld + n0 + c, r, there, there ? bf2f(h[f]) : 0.f,
+                   bf2f(weight), there ? sum(c) : 0.f);
     } else {
       if (n0 + c < n) y[r * y_ld + n0 + c] = stored<C>(sum(c));
     }
@@ -226,18 +251,22 @@ bool rows_gemm_pays(int m, int n, int k, bool paired) {
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
                       long y_ld, bool gated, bool gelu, const Heads* heads,
-                      const NormOf* norm, hipStream_t stream) {
+                      const NormOf* norm, const AddTo* add,
+                      const Undivided* of, hipStream_t stream) {
   auto launch = [&](auto normed, auto tiles, auto stages) {
     constexpr bool N = decltype(normed)::value;
     constexpr int F = decltype(tiles)::value, S = decltype(stages)::value;
     auto kernel = heads ? rows_gemm_kernel<Columns::HEADS, N, F, S>
                   : gated ? rows_gemm_kernel<Columns::GATED, N, F, S>
                           : rows_gemm_kernel<Columns::PLAIN, N, F, S>;
-    if constexpr (!N)
+    if constexpr (!N) {
       if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S>;
+      if (add) kernel = rows_gemm_kernel<Columns::ADDED, N, F, S>;
+    }
     kernel<<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
         y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{},
-        norm ? *norm : NormOf{});
+        norm ? *norm : NormOf{}, add ? *add : AddTo{},
+        of ? *of : Undivided{});
   };
   using std::integral_constant;
   constexpr integral_constant<int, 1> one{};

@@ -10,4 +10,5 @@ bool rows_quant_takes(int m, int n, int k, Quant q, bool gated);
 void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
                        const unsigned char* qs, int m, int n, int k, Quant q,
                        bool gated, const Heads* heads, const NormOf* norm,
+                       const AddTo* add, const Undivided* of,
                        hipStream_t stream);

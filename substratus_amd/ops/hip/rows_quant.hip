@@ -164,7 +164,8 @@ __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                        const f16_t* __restrict__ scales,
                        const unsigned char* __restrict__ qs, int m, int n,
-                       int k, Heads heads, NormOf norm) {
+                       int k, Heads heads, NormOf norm, AddTo add,
+                       Undivided of) {
   using L = Layout<Q>;
   constexpr bool K_QUANT = Q == Quant::Q4_K || Q == Quant::Q6_K;
   constexpr int FM = (MR + 15) / 16;
@@ -381,11 +382,33 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     }
   };
 
+  // a thread ends up with column lo of every ROWSth row from first on
+  constexpr int ROWS = KW * WAVE / 16, PER = (BM + ROWS - 1) / ROWS;
+  const int first = threadIdx.x / 16, m_here = min(m, MR);
+  const int row0 = blockIdx.y * MR;
+  bf16_t h[PER], weight;
+  float row_squares[PER];
   NormRows<KW * WAVE> rows;
   if constexpr (NORM) rows.load(norm, m, k);
   #pragma unroll
   for (int s = 0; s < P; ++s)
     if (s < steps) load(s, c0 + s);
+  if constexpr (C == Columns::ADDED) {
+    const int at = min(n0 + lo, n - 1);
+    #pragma unroll
+    for (int f = 0; f < PER; ++f)
+      h[f] = add.h[(long)(row0 + min(first + f * ROWS, m_here - 1)) * n + at];
+    weight = add.weight[at];
+  } else if (!NORM && of.squares != nullptr) {
+    // added up here: kept until the end they take registers, and so workgroups of
+    // a CU (q4_0, one row, 8 layers of 5120: 568 us instead of 547)
+    #pragma unroll
+    for (int f = 0; f < PER; ++f) {
+      RowSquares parts;
+      parts.load(of, row0 + min(first + f * ROWS, m_here - 1));
+      row_squares[f] = parts.sum(of);
+    }
+  }
   if constexpr (NORM) {
     rows.put(norm, m, k, reinterpret_cast<uint4*>(s_x), squares);
     lds_barrier();
@@ -430,11 +453,18 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     heads.positions += blockIdx.y * MR;
     heads.slots += blockIdx.y * MR;
   }
-  for (int i = threadIdx.x; i < BM * 16; i += KW * WAVE) {
-    const int r = i / 16, c = i % 16;
-    if (r >= m || r >= MR) break;
-    const float scale =
-        NORM ? norm_scale<KW>(squares, r, k, norm.eps) : 1.f;
+  if constexpr (C == Columns::ADDED) {
+    add.sum += (long)row0 * y_ld;
+    add.squares += (long)row0 * gridDim.x;
+  }
+  #pragma unroll
+  for (int f = 0; f < PER; ++f) {
+    const int r = first + f * ROWS, c = lo;
+    if (r >= m_here) break;
+    float scale = 1.f;
+    if constexpr (NORM) scale = norm_scale<KW>(squares, r, k, norm.eps);
+    else if (C != Columns::ADDED && of.squares != nullptr)
+      scale = undivided_scale(of, row_squares[f], k);
     auto sum = [&](int c) {
       float v = 0.f;
       #pragma unroll
@@ -444,14 +474,18 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
           const long at = weight_row<C>(n0, c, n, half);
           v = dot_q4k(x + (long)r * k, qs + at * rb, scales + at * (sb / 2), k);
         }
-      if constexpr (NORM) v *= scale;
-      return v;
+      return v * scale;
     };
     if constexpr (C == Columns::GATED) {
       if (c < 8)
         y[(long)r * y_ld + n0 + c] = f2bf(silu_times(sum(c), sum(c + 8)));
     } else if constexpr (C == Columns::HEADS) {
       if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
+    } else if constexpr (C == Columns::ADDED) {
+      const bool there = n0 + c < n;
+      finish_added(add, y, (long)r * y_ld + n0 + c, r, there,
+                   there ? bf2f(h[f]) : 0.f,
+                   bf2f(weight), there ? sum(c) : 0.f);
     } else {
       if (n0 + c < n) y[(long)r * y_ld + n0 + c] = f2bf(sum(c));
     }
@@ -470,6 +504,7 @@ bool rows_quant_takes(int m, int n, int k, Quant q, bool gated) {
 void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
                        const unsigned char* qs, int m, int n, int k, Quant q,
                        bool gated, const Heads* heads, const NormOf* norm,
+                       const AddTo* add, const Undivided* of,
                        hipStream_t stream) {
   const f16_t* sc = reinterpret_cast<const f16_t*>(scales);
   auto go = [&](auto qc, auto mr, auto me, auto kw, auto p) {
@@ -484,12 +519,16 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
                      : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN,
                                          N>;
     };
-    auto kernel = pick(std::false_type{});
+    auto kernel = add ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::ADDED,
+                                          false>
+                      : pick(std::false_type{});
     if constexpr (MR == NORM_ROWS)
       if (norm) kernel = pick(std::true_type{});
     kernel<<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k,
                                        heads ? *heads : Heads{},
-                                       norm ? *norm : NormOf{});
+                                       norm ? *norm : NormOf{},
+                                       add ? *add : AddTo{},
+                                       of ? *of : Undivided{});
   };
   auto by_rows = [&](auto qc) {
     constexpr Quant QQ = decltype(qc)::value;

@@ -87,6 +87,19 @@ class Linear(nn.Module):
         return ops.linear_normed(delta, h, norm, eps, self.weight, self.bias,
                                  gated, cache) if bare(self, Linear) else None
 
+    def added(self, x: torch.Tensor, h: torch.Tensor, norm: torch.Tensor):
+        """(h + the outputs, RMSNorm of that but for its division) in one
+        kernel, or None."""
+        return ops.linear_added(x, self.weight, self.bias, h, norm) \
+            if bare(self, Linear) else None
+
+    def scaled(self, x: ops.Undivided, eps: float, gated: bool = False,
+               cache: Optional[ops.Cache] = None) -> Optional[torch.Tensor]:
+        """The outputs for rows that are still to be divided, gated or appended
+        as above, in one kernel, or None."""
+        return ops.linear_scaled(x, eps, self.weight, self.bias, gated,
+                                 cache) if bare(self, Linear) else None
+
 
 class ColumnParallelLinear(Linear):
     """Output features sharded across TP ranks; output stays sharded."""
@@ -123,3 +136,9 @@ class RowParallelLinear(Linear):
         if self.bias is not None:
             y = y + self.bias
         return y
+
+    def added(self, x: torch.Tensor, h: torch.Tensor, norm: torch.Tensor):
+        # (a bias would be rounded with the sum and not after it)
+        return ops.linear_added(x, self.weight, None, h, norm) \
+            if self.tp_world == 1 and self.bias is None \
+            and bare(self, RowParallelLinear) else None
