@@ -165,8 +165,7 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
         mx = fmaxf(mx, p[s * 4 + e]);
       }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    mx = across_from<16>(mx, Larger{});
     const float mn = fmaxf(m, mx);
     const float keep = __builtin_amdgcn_exp2f(m - mn);
     m = mn;
@@ -245,8 +244,7 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
   // merge: [wave][head][D + 2], the last two being maximum and sum
   float* red = reinterpret_cast<float*>(s_all);
   constexpr int LD = D + 4;
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
+  l = across_from<16>(l, Plus{});
   float* w = red + (wave * 16 + lo) * LD;
   #pragma unroll
   for (int t = 0; t < DT; ++t)

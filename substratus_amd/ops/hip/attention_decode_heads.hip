@@ -210,20 +210,14 @@ void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
 
   // the rows' softmaxes become one a wave, and the waves' one
   __shared__ float s_o[WAVES][D], s_m[WAVES], s_l[WAVES];
-  float most = m;
-  #pragma unroll
-  for (int off = LANES; off < WAVE; off *= 2)
-    most = fmaxf(most, __shfl_xor(most, off, WAVE));
+  const float most = across_from<LANES>(m, Larger{});
   const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - most);
   l *= f;
   #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] *= f;
+  l = across_from<LANES>(l, Plus{});
   #pragma unroll
-  for (int off = LANES; off < WAVE; off *= 2) {
-    l += __shfl_xor(l, off, WAVE);
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[j] += __shfl_xor(acc[j], off, WAVE);
-  }
+  for (int j = 0; j < 8; ++j) acc[j] = across_from<LANES>(acc[j], Plus{});
   if (row == 0) {
     #pragma unroll
     for (int j = 0; j < 8; j += 4)

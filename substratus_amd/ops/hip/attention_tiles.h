@@ -116,9 +116,7 @@ __global__ void attn_bwd_delta_kernel(float* __restrict__ delta,
       const float2 ov = unpack_bf16x2(op[i]);
       acc += dv.x * ov.x + dv.y * ov.y;
     }
-    #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-      acc += __shfl_xor(acc, off, WAVE);
+    acc = wave_sum(acc);
     if (lane == 0) delta[r] = acc;
   }
 }

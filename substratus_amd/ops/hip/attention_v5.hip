@@ -144,7 +144,7 @@ void attn_v5_kernel(bf16_t* __restrict__ out,      // [T, HQ, D]
           #pragma unroll
           for (int r = 0; r < 16; ++r) mraw = fmaxf(mraw, sacc[sc][r]);
       }
-      mraw = fmaxf(mraw, __shfl_xor(mraw, 32, WAVE));
+      mraw = across<32>(mraw, Larger{});
       const float mloc = mraw == -INFINITY ? mraw : mraw * scale2;
       constexpr float MOST = 8.f;
       float alpha = 1.f;
@@ -178,7 +178,7 @@ void attn_v5_kernel(bf16_t* __restrict__ out,      // [T, HQ, D]
       };
       if (edge || !__all(mloc != -INFINITY)) weigh(std::true_type{});
       else weigh(std::false_type{});
-      rowsum += __shfl_xor(rowsum, 32, WAVE);
+      rowsum = across<32>(rowsum, Plus{});
       l = l * alpha + rowsum;
       #pragma unroll
       for (int sc = 0; sc < STEP / 32; ++sc)

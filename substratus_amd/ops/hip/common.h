@@ -58,24 +58,89 @@ DEV_INLINE unsigned int pack_bf16x2(float lo, float hi) {
 }
 
 // --- wave-level reductions (64 lanes) -------------------------------------
-DEV_INLINE float wave_sum(float v) {
-  #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-  return v;
+// op, which is symmetric, of a lane's number and that of the lane OFF away: by
+// moves between registers, where __shfl_xor goes through LDS. 4 away only where
+// lanes 8 away have equal numbers (a row of 16 lanes turned by four). Lanes must
+// be there: all of a wave for 32 and 16, of a row of 16 for the others. ns of a
+// sum over a wave that waits for the one before it: 178 -> 52.
+template <int OFF, class Op>
+DEV_INLINE float across(float v, Op op) {
+  const unsigned u = __float_as_uint(v);
+  if constexpr (OFF == 32) {
+    const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return op(__uint_as_float(s[0]), __uint_as_float(s[1]));
+  } else if constexpr (OFF == 16) {
+    const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return op(__uint_as_float(s[0]), __uint_as_float(s[1]));
+  } else {
+    static_assert(OFF == 8 || OFF == 4 || OFF == 2 || OFF == 1);
+    constexpr int CTRL = OFF == 8 ? 0x128       // row_ror 8
+                       : OFF == 4 ? 0x124       // row_ror 4
+                       : OFF == 2 ? 0x4e        // quad_perm 2 3 0 1
+                                  : 0xb1;       // quad_perm 1 0 3 2
+    return op(v, __uint_as_float(__builtin_amdgcn_update_dpp(
+                     0u, u, CTRL, 0xf, 0xf, true)));
+  }
 }
 
-DEV_INLINE float wave_max(float v) {
-  #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, WAVE));
-  return v;
+// The number of the lane OFF away.
+template <int OFF>
+DEV_INLINE float from_lane(float v) {
+  const unsigned u = __float_as_uint(v);
+  if constexpr (OFF >= 16) {
+    static_assert(OFF == 32 || OFF == 16);
+    const bool up = threadIdx.x & OFF;
+    if constexpr (OFF == 32) {
+      const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      return __uint_as_float(up ? s[0] : s[1]);
+    } else {
+      const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      return __uint_as_float(up ? s[0] : s[1]);
+    }
+  } else if constexpr (OFF == 4) {              // 7 away, of which 3 back
+    const unsigned t =
+        __builtin_amdgcn_update_dpp(0u, u, 0x141, 0xf, 0xf, true);
+    return __uint_as_float(
+        __builtin_amdgcn_update_dpp(0u, t, 0x1b, 0xf, 0xf, true));
+  } else {
+    constexpr int CTRL = OFF == 8 ? 0x128 : OFF == 2 ? 0x4e : 0xb1;
+    static_assert(OFF == 8 || OFF == 2 || OFF == 1);
+    return __uint_as_float(
+        __builtin_amdgcn_update_dpp(0u, u, CTRL, 0xf, 0xf, true));
+  }
 }
 
-// Reduce within 16-lane groups (used by 16-lanes-per-token layouts).
-DEV_INLINE float group16_sum(float v) {
-  #pragma unroll
-  for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-  return v;
+struct Plus {
+  DEV_INLINE float operator()(float a, float b) const { return a + b; }
+};
+struct Larger {
+  DEV_INLINE float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+
+// Of the lanes FROM, 2 FROM and so on to 32 away, in this order.
+template <int FROM, class Op>
+DEV_INLINE float across_from(float v, Op op) {
+  static_assert(FROM == 8 || FROM == 16 || FROM == 32);
+  if constexpr (FROM == 8) v = across<8>(v, op);
+  if constexpr (FROM <= 16) v = across<16>(v, op);
+  return across<32>(v, op);
 }
+
+// Within 16-lane groups (used by 16-lanes-per-token layouts).
+template <class Op>
+DEV_INLINE float group16(float v, Op op) {
+  return across<1>(across<2>(across<4>(across<8>(v, op), op), op), op);
+}
+
+DEV_INLINE float group16_sum(float v) { return group16(v, Plus{}); }
+
+template <class Op>
+DEV_INLINE float wave_all(float v, Op op) {
+  return group16(across<16>(across<32>(v, op), op), op);
+}
+
+DEV_INLINE float wave_sum(float v) { return wave_all(v, Plus{}); }
+DEV_INLINE float wave_max(float v) { return wave_all(v, Larger{}); }
 
 // --- block-level reductions over NW waves via LDS --------------------------
 // Caller provides __shared__ float scratch[NW]; result valid in all threads.

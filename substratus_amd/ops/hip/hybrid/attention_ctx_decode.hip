@@ -137,8 +137,7 @@ void attn_ctx_decode_kernel(AttnCtx<bf16_t> a, int splits,
     const float dist = (float)(pos - kpos);
     #pragma unroll
     for (int g = 0; g < GQ; ++g) {
-      s[g] += __shfl_xor(s[g], 1, WAVE);
-      s[g] += __shfl_xor(s[g], 2, WAVE);
+      s[g] = across<2>(across<1>(s[g], Plus{}), Plus{});
       s[g] = a.cap > 0.f ? cap2 * tanh_exp2(s[g] * cscale) : s[g] * scale2;
       if (a.r1 != nullptr)
         s[g] -= r1[g] * __builtin_amdgcn_logf(1.f + r2[g] * dist);
@@ -147,10 +146,8 @@ void attn_ctx_decode_kernel(AttnCtx<bf16_t> a, int splits,
         continue;
       }
       s[g] = live ? s[g] + bn[g] : NEG;
-      float mx = s[g];
-      #pragma unroll
-      for (int off = 4; off < WAVE; off <<= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, off, WAVE));
+      const float mx = across<4>(across<8>(across<16>(
+          across<32>(s[g], Larger{}), Larger{}), Larger{}), Larger{});
       if (mx > m[g]) {                     // uniform over the wave
         const float keep = __builtin_amdgcn_exp2f(m[g] - mx);
         l[g] *= keep;
@@ -182,9 +179,7 @@ void attn_ctx_decode_kernel(AttnCtx<bf16_t> a, int splits,
   for (int g = 0; g < GQ; ++g) {
     #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      #pragma unroll
-      for (int off = CL; off < WAVE; off <<= 1)
-        acc[g][j] += __shfl_xor(acc[g][j], off, WAVE);
+      acc[g][j] = across_from<CL>(acc[g][j], Plus{});
       if (rg == 0) s_o[wave][g][col * 8 + j] = acc[g][j];
     }
     const float lt = wave_sum(l[g]) * 0.25f;

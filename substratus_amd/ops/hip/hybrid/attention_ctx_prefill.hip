@@ -240,7 +240,7 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
         for (int sc = 0; sc < CH / 32; ++sc)
           #pragma unroll
           for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sv[sc][r]);
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, WAVE));
+        mloc = across<32>(mloc, Larger{});
         // the running maximum moves only when a score exceeds it by 2^8
         if (!__all(mloc == -INFINITY || mloc - m <= 8.f)) {
           const float mn = fmaxf(m, mloc);
@@ -295,7 +295,7 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
           }
         }
       }
-      if constexpr (KIND != SIGMOID) l += sum + __shfl_xor(sum, 32, WAVE);
+      if constexpr (KIND != SIGMOID) l += across<32>(sum, Plus{});
     }
     if (it + 1 < part.n) stage_write(cur ^ 1);
     __syncthreads();

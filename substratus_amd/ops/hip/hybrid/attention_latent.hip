@@ -171,8 +171,7 @@ void attn_latent_kernel(AttnCtx<bf16_t> a, int entries, int splits,
             ? (acc[0][i] + acc[1][i]) * scale2 : -INFINITY;
         mx = fmaxf(mx, s[i]);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+      mx = across_from<16>(mx, Larger{});
       if (grp == 0) s_m[page][mine + lo] = mx;
     }
     lds_barrier();
@@ -255,8 +254,7 @@ void attn_latent_kernel(AttnCtx<bf16_t> a, int entries, int splits,
   }
 
   // sums of all waves' keys
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
+  l = across_from<16>(l, Plus{});
   if (scoring && grp == 0) s_m[page][mine + lo] = l;
   lds_barrier();
   #pragma unroll

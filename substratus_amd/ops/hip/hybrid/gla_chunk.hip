@@ -214,7 +214,7 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
         if (j > 0) b[r] += b[r - 1];
       }
       gs[g] = b[4 * g + 3];
-      og[g] = __shfl_xor(gs[g], 32, WAVE);
+      og[g] = from_lane<32>(gs[g]);
     }
     float before = 0.f;          // over the tokens ahead of each four
     #pragma unroll
@@ -414,17 +414,21 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
       float q[16];
       #pragma unroll
       for (int r = 0; r < 16; ++r) q[r] = col_ok ? o[r] * o[r] : 0.f;
-      #pragma unroll
-      for (int w = 8; w >= 1; w >>= 1) {
+      auto halve = [&](auto width) {
+        constexpr int w = decltype(width)::value;
+        const bool up = (lane & w) != 0;
         #pragma unroll
         for (int r = 0; r < w; ++r) {
-          const bool up = (lane & w) != 0;
           const float give = up ? q[r] : q[r + w];
-          q[r] = (up ? q[r + w] : q[r]) + __shfl_xor(give, w, WAVE);
+          q[r] = (up ? q[r + w] : q[r]) + from_lane<w>(give);
         }
-      }
+      };
+      halve(std::integral_constant<int, 8>{});
+      halve(std::integral_constant<int, 4>{});
+      halve(std::integral_constant<int, 2>{});
+      halve(std::integral_constant<int, 1>{});
       // lane now holds accumulator row lane & 15, over 16 of 32 columns
-      q[0] += __shfl_xor(q[0], 16, WAVE);
+      q[0] = across<16>(q[0], Plus{});
       if ((lane & 16) == 0) s.ssq[wave][crow(lane & 15)] = q[0];
     }
     __syncthreads();
