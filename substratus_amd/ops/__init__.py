@@ -582,8 +582,7 @@ def linear_normed(delta: torch.Tensor, h: torch.Tensor, norm: torch.Tensor,
 
 class Undivided(NamedTuple):
     """An RMSNorm's rows but for the division by their deviations: rounded
-    h * weight, and parts of every row's squares of h, [rows, n / 16] of 32
-    bits."""
+    h * weight, and sums of parts of every row's squares of h, in 32 bits."""
     rows: torch.Tensor
     squares: torch.Tensor
 
@@ -598,10 +597,11 @@ def may_add(h: torch.Tensor, norm: torch.Tensor, rows: int, n: int) -> bool:
             and inference_only(h, norm))
 
 
-def room_for_added(h: torch.Tensor) -> tuple[torch.Tensor, Undivided]:
+def room_for_added(h: torch.Tensor,
+                   parts: int) -> tuple[torch.Tensor, Undivided]:
     """Room for h + a product, and for its norm's rows."""
     return torch.empty_like(h), Undivided(torch.empty_like(h), h.new_empty(
-        h.shape[0], h.shape[1] // 16, dtype=torch.float32))
+        h.shape[0], parts, dtype=torch.float32))
 
 
 def linear_added(x: torch.Tensor, weight: torch.Tensor,
@@ -616,7 +616,8 @@ def linear_added(x: torch.Tensor, weight: torch.Tensor,
             or x.device != h.device \
             or not may_add(h, norm, x.shape[0], weight.shape[0]):
         return None
-    total, parts = room_for_added(h)
+    total, parts = room_for_added(h, few[1].rows_added_parts(
+        x.shape[0], *weight.shape))
     few[1].rows_added(parts.rows, total, parts.squares, few[0], weight, bias,
                       h, norm)
     return total, parts
@@ -626,10 +627,13 @@ def linear_scaled(x: Undivided, eps: float, weight: torch.Tensor,
                   bias: Optional[torch.Tensor], gated: bool = False,
                   cache: Optional[Cache] = None) -> Optional[torch.Tensor]:
     """What becomes of F.linear of x divided, gated as linear_gated's, or with a
-    cache linear_heads' queries; or None."""
+    cache linear_heads' queries; or None. Every 16 columns ask for all rows'
+    squares, so with more than 8 rows and as many columns as a large vocabulary
+    has a norm of its own costs less: a step of llama3-8b's first two layers
+    and 16 rows 448 us instead of 431."""
     few = _few_rows(x.rows, weight, bias, gated or cache is not None)
     m, n = x.rows.shape[0], weight.shape[0]
-    if few is None or m > 16 \
+    if few is None or m > 16 or m > 8 and n > 65536 \
             or cache is not None and not cache.takes(x.rows, n):
         return None
     y = x.rows.new_empty(*_columns(m, n, gated, cache))

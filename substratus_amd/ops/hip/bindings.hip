@@ -620,6 +620,7 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                     mid_gemm_good(m, n, k, gated || heads);
   TORCH_CHECK(many || rows_gemm_takes(m, n, k, gated || heads),
               "rows_gemm: unsupported shape ", m, "x", n, "x", k);
+  TORCH_CHECK(m <= 16 || !(add || of), "rows_gemm: too many rows");
   TORCH_CHECK(aligned16(x) && aligned16(w), "rows_gemm: misaligned operand");
   const bf16_t* bp = nullptr;
   if (bias.has_value()) {
@@ -723,6 +724,7 @@ void quant_rows_to(torch::Tensor y, torch::Tensor x, torch::Tensor scales,
               scales.size(0) == n, "quant_rows: shape mismatch");
   TORCH_CHECK(rows_quant_takes(m, n, k, q, gated || heads),
               "quant_rows: unsupported shape ", m, "x", n, "x", k);
+  TORCH_CHECK(m <= 8 || !(add || of), "quant_rows: too many rows");
   // what is not aligned to the kernel's loads is copied to where it is
   if (!aligned16(x)) x = x.clone();
   if (!aligned16(qs)) qs = qs.clone();
@@ -765,11 +767,21 @@ struct Where {
   }
 };
 
+// In how many parts a product that is added leaves a row's squares.
+long rows_added_parts(long m, long n, long k) {
+  return n / (rows_gemm_thin((int)m, (int)n, (int)k, false) ? 8 : 16);
+}
+
+long quant_added_parts(long m, long n, long k, const std::string& quant) {
+  return n / (rows_quant_thin((int)m, (int)n, (int)k, quant_of(quant), false)
+                  ? 8 : 16);
+}
+
 // A product that is added to the residual stream: total = h + its rows, y =
-// total * weight, and every row's squares in parts, one of 16 columns.
+// total * weight, and every row's squares in parts.
 AddTo add_of(const torch::Tensor& y, const torch::Tensor& total,
              const torch::Tensor& squares, const torch::Tensor& h,
-             const torch::Tensor& weight) {
+             const torch::Tensor& weight, long parts) {
   const long n = weight.numel();
   TORCH_CHECK(h.dim() == 2 && h.size(1) == n && n % 64 == 0 &&
               y.dim() == 2 && y.sizes() == h.sizes(), "added rows: shapes");
@@ -777,7 +789,7 @@ AddTo add_of(const torch::Tensor& y, const torch::Tensor& total,
   check_rows(h, h.numel(), "h"); check_rows(total, h.numel(), "total");
   TORCH_CHECK(squares.is_cuda() && squares.is_contiguous() &&
               squares.scalar_type() == torch::kFloat &&
-              squares.numel() == h.size(0) * (n / 16), "squares");
+              squares.numel() == h.size(0) * parts, "squares");
   return {bfc(h), bfc(weight), const_cast<bf16_t*>(bfc(total)),
           squares.data_ptr<float>()};
 }
@@ -797,7 +809,9 @@ void rows_added(torch::Tensor y, torch::Tensor total, torch::Tensor squares,
                 torch::Tensor x, torch::Tensor w,
                 c10::optional<torch::Tensor> bias, torch::Tensor h,
                 torch::Tensor weight) {
-  const AddTo add = add_of(y, total, squares, h, weight);
+  const AddTo add =
+      add_of(y, total, squares, h, weight,
+             rows_added_parts(x.size(0), w.size(0), w.size(1)));
   rows_gemm_to(y, x, w, bias, false, nullptr, nullptr, false, &add);
 }
 
@@ -818,7 +832,9 @@ void quant_added(torch::Tensor y, torch::Tensor total, torch::Tensor squares,
                  torch::Tensor x, torch::Tensor scales, torch::Tensor qs,
                  const std::string& quant, torch::Tensor h,
                  torch::Tensor weight) {
-  const AddTo add = add_of(y, total, squares, h, weight);
+  const AddTo add = add_of(y, total, squares, h, weight,
+                           quant_added_parts(x.size(0), qs.size(0),
+                                             x.size(1), quant));
   quant_rows_to(y, x, scales, qs, quant, false, nullptr, nullptr, &add);
 }
 
@@ -1112,6 +1128,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_normed", &rows_normed);
   m.def("quant_normed", &quant_normed);
   m.def("rows_added", &rows_added);
+  m.def("rows_added_parts", &rows_added_parts);
+  m.def("quant_added_parts", &quant_added_parts);
   m.def("rows_scaled", &rows_scaled);
   m.def("quant_added", &quant_added);
   m.def("quant_scaled", &quant_scaled);

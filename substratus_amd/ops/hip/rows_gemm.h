@@ -97,34 +97,33 @@ struct Undivided {
   float eps;
 };
 
-// A row's sum of squares for the 16 lanes that ask for it: what a lane adds up is
-// asked for behind a workgroup's first weights.
+// A row's sum of squares, by a wave. Asked for behind a workgroup's first weights.
+template <int PER>
 struct RowSquares {
-  static constexpr int PER = 5;
   float4 v[PER];
   float rest;
 
   DEV_INLINE void load(const Undivided& of, int r) {
     const float* row = of.squares + (long)r * of.parts;
-    const int at = threadIdx.x % 16 * 4;
+    const int at = threadIdx.x % WAVE * 4;
     #pragma unroll
     for (int i = 0; i < PER; ++i)
-      if (i * 64 < of.parts)
+      if (i * 256 < of.parts)
         v[i] = *reinterpret_cast<const float4*>(
-            row + min(at + i * 64, of.parts - 4));
+            row + min(at + i * 256, of.parts - 4));
     rest = 0.f;
-    for (int j = at + PER * 64; j < of.parts; j += 64) {
+    for (int j = at + PER * 256; j < of.parts; j += 256) {
       const float4 u = *reinterpret_cast<const float4*>(row + j);
       rest += u.x + u.y + (u.z + u.w);
     }
   }
   DEV_INLINE float sum(const Undivided& of) const {
-    const int at = threadIdx.x % 16 * 4;
+    const int at = threadIdx.x % WAVE * 4;
     float s = rest;
     #pragma unroll
     for (int i = 0; i < PER; ++i)
-      if (at + i * 64 < of.parts) s += v[i].x + v[i].y + (v[i].z + v[i].w);
-    return group16_sum(s);
+      if (at + i * 256 < of.parts) s += v[i].x + v[i].y + (v[i].z + v[i].w);
+    return wave_sum(s);
   }
 };
 
@@ -277,6 +276,7 @@ DEV_INLINE void finish_heads(bf16_t* y, long y_ld, const Heads& heads, int r,
   }
 }
 
+bool rows_gemm_thin(int m, int n, int k, bool paired);
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       const bf16_t* bias, int m, int n, int k, long x_ld,
                       long y_ld, bool gated, bool gelu, const Heads* heads,

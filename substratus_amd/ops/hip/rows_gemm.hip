@@ -44,8 +44,10 @@ constexpr int U = 2;              // 32-column chunks of a stage
 constexpr int TILE = 64;          // 16-byte pieces of 16 rows x 32 columns
 constexpr int PAD = 4;
 
-// FM: tiles of 16 rows of x; P: stages in flight
-template <Columns C, bool NORM, int FM, int P>
+// FM: tiles of 16 rows of x; P: stages in flight. THIN: a workgroup has eight
+// weight rows, and the other eight of an operand are the next 64 columns of the
+// same ones, beside those of x: the rows of x are eight at most then.
+template <Columns C, bool NORM, int FM, int P, bool THIN>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       const bf16_t* __restrict__ w,
@@ -54,6 +56,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       AddTo add, Undivided of) {
   // (normed x does not go through the ring)
   static_assert(!NORM || FM == 1);
+  static_assert(!THIN || (FM == 1 && !NORM && !paired(C)));
   constexpr int TILES = NORM ? 1 : 1 + FM;       // of a chunk of 32 columns
   constexpr int STAGE = U * TILES * TILE;
   constexpr int LOADS = U * TILES;
@@ -61,19 +64,22 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   // one array: beside a second one the compiler guards every LDS read against
   // the direct loads in flight, and waits for them
   __shared__ alignas(16)
-      uint4 s_all[RING + (NORM ? NORM_PIECES + NORM_ROWS + KW : 0)];
+      uint4 s_all[RING + (NORM ? NORM_PIECES + NORM_ROWS + KW
+                               : FM == 1 ? 4 : 0)];
   uint4* s_x = s_all + RING;
   auto squares = reinterpret_cast<float (*)[NORM_ROWS]>(
       s_x + NORM_PIECES + NORM_ROWS);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
   const int lo = lane & 15, g = lane >> 4;
-  const int n0 = first_column<C>(heads), half = second_half<C>(n, heads);
-  // shares begin on whole cache lines
-  const int chunks = k / 32, pairs = (chunks + 1) / 2;
-  const int c0 = pairs * wave / KW * 2;
-  const int c1 = min(pairs * (wave + 1) / KW * 2, chunks);
-  const int steps = (c1 - c0 + U - 1) / U;
+  const int n0 = THIN ? blockIdx.x * 8 : first_column<C>(heads);
+  const int half = second_half<C>(n, heads);
+  // shares begin on whole cache lines, of THIN on two
+  constexpr int LINES = THIN ? 2 : 1, CHUNKS = U * LINES;     // of a stage
+  const int chunks = k / 32, lines = (chunks + CHUNKS - 1) / CHUNKS;
+  const int c0 = lines * wave / KW * CHUNKS;
+  const int c1 = min(lines * (wave + 1) / KW * CHUNKS, chunks);
+  const int steps = (c1 - c0 + CHUNKS - 1) / CHUNKS;
   uint4* ring = s_all + wave * P * STAGE;
 
   // a load is 8 rows x 128 bytes: of a tile's row lane / 8, or eight later
@@ -82,14 +88,15 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   int piece[2];
   #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int r = h * 8 + row;
+    const int r = h * 8 + row, from = THIN ? row : r;
+    const int at = c0 * 32 + (THIN ? h * 64 : 0);
     piece[h] = (lane & 7) ^ (r >> 1);
     wp[h] = reinterpret_cast<const char*>(
-        w + (long)weight_row<C>(n0, r, n, half) * k + c0 * 32);
+        w + (long)weight_row<C>(n0, from, n, half) * k + at);
     #pragma unroll
     for (int f = 0; f < FM; ++f)
       xp[f][h] = reinterpret_cast<const char*>(
-          x + min(f * 16 + r, m - 1) * x_ld + c0 * 32);
+          x + min(f * 16 + from, m - 1) * x_ld + at);
   }
   const int end = (c1 - c0) * 4 - 1;             // the share's last piece
   auto load = [&](int s, int i) {
@@ -97,7 +104,8 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     #pragma unroll
     for (int h = 0; h < 2; ++h) {
       // a stage may be half of one: then its last piece comes again
-      const unsigned at = (unsigned)min(i * 8 + piece[h], end) * 16;
+      const unsigned at = THIN ? (unsigned)(i * 16 + piece[h]) * 16
+                               : (unsigned)min(i * 8 + piece[h], end) * 16;
       load_to_lds<16>(wp[h] + at, to + h * TILE);
       if constexpr (!NORM) {
         #pragma unroll
@@ -128,7 +136,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     }
     #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (c0 + i * U + u < c1) {
+      if (THIN || c0 + i * U + u < c1) {
         #pragma unroll
         for (int f = 0; f < FM; ++f)
           acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -138,7 +146,11 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   // a thread ends up with column c of rows from row on
   const int c = threadIdx.x % 16, first = threadIdx.x / 16;
   bf16_t h[FM], weight;
-  RowSquares parts[FM];
+  // rows that are still to be divided: a wave adds up the squares of every fourth
+  constexpr bool DIVIDES = FM == 1 && !NORM && C != Columns::ADDED;
+  const bool divided = DIVIDES && of.squares != nullptr;
+  float* row_squares = reinterpret_cast<float*>(s_all + RING);
+  RowSquares<2> parts[DIVIDES ? 16 / KW : 1];
   NormRows<KW * WAVE> rows;
   if constexpr (NORM) rows.load(norm, m, k);
   #pragma unroll
@@ -150,11 +162,13 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     for (int f = 0; f < FM; ++f)
       h[f] = add.h[(long)min(first + f * 16, m - 1) * n + at];
     weight = add.weight[at];
-  } else if (!NORM && of.squares != nullptr) {
+  }
+  if constexpr (DIVIDES) {
     // waited for at the end (added up here, 643 us instead of 616 for a step of
     // 16 layers of 2048, one row)
     #pragma unroll
-    for (int f = 0; f < FM; ++f) parts[f].load(of, min(first + f * 16, m - 1));
+    for (int i = 0; i < 16 / KW; ++i)
+      if (divided && wave + i * KW < m) parts[i].load(of, wave + i * KW);
   }
   if constexpr (NORM) {
     rows.put(norm, m, k, s_x, squares);
@@ -187,6 +201,14 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   for (int f = 0; f < FM; ++f)
     *reinterpret_cast<float4v*>(
         &red[(wave * ROWS + f * 16 + lo) * (16 + PAD) + g * 4]) = acc[f];
+  if constexpr (DIVIDES) {
+    #pragma unroll
+    for (int i = 0; i < 16 / KW; ++i)
+      if (divided && wave + i * KW < m) {
+        const float q = parts[i].sum(of);
+        if (lane == 0) row_squares[wave + i * KW] = q;
+      }
+  }
   __syncthreads();
   #pragma unroll
   for (int f = 0; f < FM; ++f) {
@@ -194,12 +216,14 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     if (r >= m) break;
     float scale = 1.f;
     if constexpr (NORM) scale = norm_scale<KW>(squares, r, k, norm.eps);
-    else if (C != Columns::ADDED && of.squares != nullptr)
-      scale = undivided_scale(of, parts[f].sum(of), k);
+    else if (divided) scale = undivided_scale(of, row_squares[r], k);
     auto sum = [&](int c) {
       float v = 0.f;
       #pragma unroll
-      for (int q = 0; q < KW; ++q) v += red[(q * ROWS + r) * (16 + PAD) + c];
+      for (int q = 0; q < KW; ++q) {
+        v += red[(q * ROWS + r) * (16 + PAD) + c];
+        if constexpr (THIN) v += red[(q * ROWS + r + 8) * (16 + PAD) + c + 8];
+      }
       v *= scale;
       if (bias != nullptr) v += bf2f(bias[weight_row<C>(n0, c, n, half)]);
       return v;
@@ -209,11 +233,12 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     } else if constexpr (C == Columns::HEADS) {
       if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
     } else if constexpr (C == Columns::ADDED) {
-      const bool there = n0 + c < n;
+      const bool there = (!THIN || c < 8) && n0 + c < n;
       finish_added(add, y, r * y_ld + n0 + c, r, there, there ? bf2f(h[f]) : 0.f,
                    bf2f(weight), there ? sum(c) : 0.f);
     } else {
-      if (n0 + c < n) y[r * y_ld + n0 + c] = stored<C>(sum(c));
+      if ((!THIN || c < 8) && n0 + c < n)
+        y[r * y_ld + n0 + c] = stored<C>(sum(c));
     }
   }
 }
@@ -246,6 +271,21 @@ bool rows_gemm_pays(int m, int n, int k, bool paired) {
   return n > 6144 && m <= 32 && k <= (paired ? 4096 : 3072);
 }
 
+// Whether a workgroup has eight weight rows instead of 16. A CU takes in some 45
+// GB/s, so the ones that have most of a matrix are what takes the time: eight rows
+// instead of 16 up to 2048, three times eight instead of two of 16 from 4096 to
+// 6144. (Between and past them it is as many rows either way, and x once more.) us,
+// MI355X, 16 -> eight, of one and eight rows:
+//   768 x 3072   4.6  5.2 ->  3.6  4.2     4608 x 18432  41.6 45.2 -> 34.8 40.7
+//   2048 x 2048  4.7  4.8 ->  4.1  4.2     5120 x 5120   13.7 15.3 -> 12.1 13.7
+//   2048 x 5632  8.6  8.4 ->  6.5  6.8     6144 x 2048    7.4  7.4 ->  7.2  7.4
+//   2560 x 10240  14 14.9 -> 13.5 16.4     6144 x 16384  44.7 47.2 -> 41.8 43.6
+//   3584 x 18944  26 27.1 -> 26.0 32.3
+bool rows_gemm_thin(int m, int n, int k, bool paired) {
+  return m <= 8 && !paired && (n <= 2048 || (n > 4096 && n <= 6144)) &&
+         k % 128 == 0;
+}
+
 // heads: null, or what is done with the columns instead of storing them (n is
 // a multiple of 16 then, like gated's)
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
@@ -253,29 +293,36 @@ void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       long y_ld, bool gated, bool gelu, const Heads* heads,
                       const NormOf* norm, const AddTo* add,
                       const Undivided* of, hipStream_t stream) {
-  auto launch = [&](auto normed, auto tiles, auto stages) {
-    constexpr bool N = decltype(normed)::value;
+  auto launch = [&](auto normed, auto tiles, auto stages, auto thin) {
+    constexpr bool N = decltype(normed)::value, T = decltype(thin)::value;
     constexpr int F = decltype(tiles)::value, S = decltype(stages)::value;
-    auto kernel = heads ? rows_gemm_kernel<Columns::HEADS, N, F, S>
-                  : gated ? rows_gemm_kernel<Columns::GATED, N, F, S>
-                          : rows_gemm_kernel<Columns::PLAIN, N, F, S>;
-    if constexpr (!N) {
-      if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S>;
-      if (add) kernel = rows_gemm_kernel<Columns::ADDED, N, F, S>;
+    auto kernel = rows_gemm_kernel<Columns::PLAIN, N, F, S, T>;
+    if constexpr (!T) {
+      if (heads) kernel = rows_gemm_kernel<Columns::HEADS, N, F, S, T>;
+      else if (gated) kernel = rows_gemm_kernel<Columns::GATED, N, F, S, T>;
     }
-    kernel<<<dim3((n + 15) / 16), dim3(KW * WAVE), 0, stream>>>(
+    if constexpr (!N) {
+      if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S, T>;
+      if (add) kernel = rows_gemm_kernel<Columns::ADDED, N, F, S, T>;
+    }
+    constexpr int ROWS = T ? 8 : 16;
+    kernel<<<dim3((n + ROWS - 1) / ROWS), dim3(KW * WAVE), 0, stream>>>(
         y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{},
         norm ? *norm : NormOf{}, add ? *add : AddTo{},
         of ? *of : Undivided{});
   };
   using std::integral_constant;
+  constexpr std::false_type no{};
+  constexpr std::true_type yes{};
   constexpr integral_constant<int, 1> one{};
   constexpr integral_constant<int, 2> two{};
   constexpr integral_constant<int, 3> three{};
   constexpr integral_constant<int, 4> four{};
-  if (norm) launch(std::true_type{}, one, four);
-  else if (m <= 16) launch(std::false_type{}, one, four);
-  else if (m <= 32) launch(std::false_type{}, two, two);
-  else if (m <= 48) launch(std::false_type{}, three, two);
-  else launch(std::false_type{}, four, two);
+  if (norm) launch(yes, one, four, no);
+  else if (rows_gemm_thin(m, n, k, gated || heads))
+    launch(no, one, four, yes);
+  else if (m <= 16) launch(no, one, four, no);
+  else if (m <= 32) launch(no, two, two, no);
+  else if (m <= 48) launch(no, three, two, no);
+  else launch(no, four, two, no);
 }

@@ -5,6 +5,7 @@
 
 enum class Quant { Q4_0, Q8_0, Q4_K, Q6_K };
 
+bool rows_quant_thin(int m, int n, int k, Quant q, bool paired);
 bool rows_quant_takes(int m, int n, int k, Quant q, bool gated);
 
 void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,

@@ -158,9 +158,18 @@ template <> struct Layout<Quant::Q6_K> {
 };
 
 // MR: rows of x; ME: of every four, those that are there (MR 4 only); KW
-// waves share k, P stages are in flight in each
-template <Quant Q, int MR, int ME, int KW, int P, Columns C, bool NORM>
-__global__ __launch_bounds__(KW * WAVE, 2)
+// waves share k, P stages are in flight in each. THIN: a workgroup has eight
+// weight rows, and the other eight of an operand are the next 256 columns of the
+// same ones, beside those of x (MR 8 at most): a stage is 512 columns.
+template <Quant Q, int MR, int ME, int KW, int P, Columns C, bool NORM,
+          bool THIN>
+// (one row: 80 registers at most, or what a stage needs before its turn takes 118
+// and a workgroup's place; 559 us instead of 549 for a step of 8 layers of 5120,
+// q4_0. With more rows of x the same costs a tenth, with q4_K's two stages in
+// flight up to 6 %.)
+__global__ __launch_bounds__(KW * WAVE, ME == 1 && !NORM &&
+                                                (Q == Quant::Q4_0 || THIN)
+                                            ? 6 : 2)
 void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                        const f16_t* __restrict__ scales,
                        const unsigned char* __restrict__ qs, int m, int n,
@@ -168,9 +177,13 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                        Undivided of) {
   using L = Layout<Q>;
   constexpr bool K_QUANT = Q == Quant::Q4_K || Q == Quant::Q6_K;
+  static_assert(!THIN || (MR <= 8 && !NORM && !paired(C) &&
+                          Q != Quant::Q6_K));
+  constexpr int HALVES = THIN ? 2 : 1, XW = 2 * HALVES;
   constexpr int FM = (MR + 15) / 16;
-  // loads of x, 4 rows x 256 B (normed x does not go through the ring)
-  constexpr int XL = NORM ? 0 : MR / 2;
+  // loads of x, 4 rows x 256 B, XW to a row (normed x does not go through the
+  // ring)
+  constexpr int XL = NORM ? 0 : MR / 4 * XW;
   constexpr int WS = L::W * TILE + L::S * 16;    // weights and scales
   constexpr int STAGE = XL * 64 + WS;
   constexpr int LOADS = XL + L::LOADS;
@@ -178,7 +191,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   constexpr int RED = (KW * BM * (16 + PAD) + 3) / 4, RING = KW * P * STAGE;
   constexpr int BEFORE = RING > RED ? RING : RED;
   __shared__ alignas(16)
-      uint4v s_all[BEFORE + (NORM ? NORM_PIECES + NORM_ROWS + KW : 0)];
+      uint4v s_all[BEFORE + (NORM ? NORM_PIECES + NORM_ROWS + KW : BM / 4)];
   uint4v* s_x = s_all + BEFORE;
   auto squares = reinterpret_cast<float (*)[NORM_ROWS]>(
       s_x + NORM_PIECES + NORM_ROWS);
@@ -186,10 +199,11 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
   const int lo = lane & 15, g = lane >> 4;
-  const int n0 = first_column<C>(heads), half = second_half<C>(n, heads);
+  const int n0 = THIN ? blockIdx.x * 8 : first_column<C>(heads);
+  const int half = second_half<C>(n, heads);
   x += (long)blockIdx.y * MR * k;
   m -= blockIdx.y * MR;
-  const int nb = k / 32, all = (k + COLS - 1) / COLS;
+  const int nb = k / 32, all = (k + COLS * HALVES - 1) / (COLS * HALVES);
   const int c0 = all * wave / KW, c1 = all * (wave + 1) / KW;
   const int steps = c1 - c0;
   uint4v* ring = s_all + wave * P * STAGE;
@@ -206,20 +220,27 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   int in_pair[2];
   #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int r = h * 8 + (lane >> 3);
+    const int r = h * 8 + (lane >> 3), from = THIN ? lane >> 3 : r;
     in_pair[h] = (lane & 7) ^ (r >> 1);
-    pair[h] = qs + weight_row<C>(n0, r, n, half) * rb;
+    pair[h] = qs + weight_row<C>(n0, from, n, half) * rb;
   }
   const unsigned char* sc = reinterpret_cast<const unsigned char*>(scales);
-  const unsigned char* wp = qs + weight_row<C>(n0, row, n, half) * rb;
-  const unsigned char* sp = sc + weight_row<C>(n0, row, n, half) * sb;
-  const unsigned char* dp = sc + weight_row<C>(n0, lo, n, half) * sb;
-  const char* xp[XL / 2 + 1];
+  // THIN: the half of a stage that rows 8 to 15 are
+  const int up = THIN ? row >> 3 : 0, lo_up = THIN ? lo >> 3 : 0;
+  const int row_w = THIN ? row & 7 : row, lo_w = THIN ? lo & 7 : lo;
+  const unsigned char* wp = qs + weight_row<C>(n0, row_w, n, half) * rb;
+  const unsigned char* sp = sc + weight_row<C>(n0, row_w, n, half) * sb;
+  const unsigned char* dp = sc + weight_row<C>(n0, lo_w, n, half) * sb;
+  const char* xp[XL / XW + 1];
   #pragma unroll
-  for (int d = 0; d < XL / 2; ++d)
+  for (int d = 0; d < XL / XW; ++d)
     xp[d] = reinterpret_cast<const char*>(
         x + (long)min(d * 4 + (lane >> 4), m - 1) * k);
   unsigned short dreg[P];                        // q6_K: the stage's d
+  // the 256 columns that a stage's half has, or the last ones again
+  auto of_stage = [&](int c, int h) {
+    return THIN ? min(c * 2 + h, k / 256 - 1) : c;
+  };
   auto load = [&](int s, int c) {
     uint4v* ws = ring + s * STAGE;
     uint4v* ss = ws + L::W * TILE;
@@ -227,24 +248,31 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     if constexpr (Q == Quant::Q4_0) {
       #pragma unroll
       for (int t = 0; t < 2; ++t)
-        load_to_lds<16>(pair[t] + min(c * 8 + in_pair[t], nb - 1) * 16,
+        load_to_lds<16>(pair[t] + min((c * HALVES + (THIN ? t : 0)) * 8 +
+                                          in_pair[t], nb - 1) * 16,
                         ws + t * TILE);
-      load_to_lds<4>(sp + min(c * 16 + word * 4, nb * 2 - 4), ss);
+      load_to_lds<4>(sp + min((c * HALVES + up) * 16 + word * 4, nb * 2 - 4),
+                     ss);
     } else if constexpr (Q == Quant::Q8_0) {
       #pragma unroll
       for (int t = 0; t < 4; ++t)
-        load_to_lds<16>(pair[t & 1] + min(c * 256 + (t >> 1) * 128 +
-                                              in_pair[t & 1] * 16, k - 16),
-                        ws + t * TILE);
-      load_to_lds<4>(sp + min(c * 16 + word * 4, nb * 2 - 4), ss);
+        load_to_lds<16>(
+            pair[t & 1] + min((c * HALVES + (THIN ? t & 1 : 0)) * 256 +
+                                  (t >> 1) * 128 + in_pair[t & 1] * 16,
+                              k - 16),
+            ws + t * TILE);
+      load_to_lds<4>(sp + min((c * HALVES + up) * 16 + word * 4, nb * 2 - 4),
+                     ss);
     } else if constexpr (Q == Quant::Q4_K) {
       #pragma unroll
       for (int t = 0; t < 2; ++t)
-        load_to_lds<16>(pair[t] + k / 16 + c * 128 + in_pair[t] * 16,
+        load_to_lds<16>(pair[t] + k / 16 + of_stage(c, THIN ? t : 0) * 128 +
+                            in_pair[t] * 16,
                         ws + t * TILE);
       // words: scales 0 to 3, 4 to 7, minima 0 to 3, 4 to 7
-      load_to_lds<4>(wp + (word & 2) * (k / 64) + c * 8 + (word & 1) * 4, ss);
-      load_to_lds<4>(dp + c * 4, ss + 16);
+      load_to_lds<4>(wp + (word & 2) * (k / 64) + of_stage(c, up) * 8 +
+                         (word & 1) * 4, ss);
+      load_to_lds<4>(dp + of_stage(c, lo_up) * 4, ss + 16);
     } else {
       #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -257,9 +285,9 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     uint4v* xs = ws + WS;
     #pragma unroll
     for (int d = 0; d < XL; ++d) {
-      const int p = c * 32 + (d & 1) * 16 +
-                    (lo ^ ((lane >> 4) << 2) ^ ((d >> 1) & 3));
-      load_to_lds<16>(xp[d >> 1] + (long)min(p, k / 8 - 1) * 16, xs + d * 64);
+      const int p = (c * XW + d % XW) * 16 +
+                    (lo ^ ((lane >> 4) << 2) ^ (d / XW & 3));
+      load_to_lds<16>(xp[d / XW] + (long)min(p, k / 8 - 1) * 16, xs + d * 64);
     }
   };
 
@@ -271,7 +299,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   #pragma unroll
   for (int j = 0; j < FM; ++j) {
     const int r = (j * 16 + lo) & (MR - 1);
-    xr[j] = (r >> 2) * 128 + (r & 3) * 16;
+    xr[j] = (r >> 2) * (XW * 64) + lo_up * 128 + (r & 3) * 16;
   }
   const int xsw = ((lo & 3) << 2) ^
                   (((lo & (MR > 16 ? 15 : MR - 1)) >> 2) & 3);
@@ -319,7 +347,10 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     };
     #pragma unroll
     for (int b = 0; b < COLS / 32; ++b) {
-      if (!decltype(whole)::value && c * 8 + b >= nb) break;
+      if (!decltype(whole)::value && c * HALVES * 8 + b >= nb) break;
+      // a stage's second half may have fewer blocks than its first, or none
+      const bool there = !THIN || decltype(whole)::value ||
+                         (c * 2 + lo_up) * 8 + b < nb;
       if constexpr (Q != Quant::Q6_K) {
         // two blocks at a time: the second's work is done while the first's
         // products are on their way
@@ -340,6 +371,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
               sums[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                   xv, ones, zero, 0, 0, 0);
           }
+          if (!there) continue;
           #pragma unroll
           for (int t = 0; t < 2; ++t) {
             add_scaled<ME>(acc[j], Q == Quant::Q4_K ? d * byte_at(sv, b + t)
@@ -385,9 +417,8 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   // a thread ends up with column lo of every ROWSth row from first on
   constexpr int ROWS = KW * WAVE / 16, PER = (BM + ROWS - 1) / ROWS;
   const int first = threadIdx.x / 16, m_here = min(m, MR);
-  const int row0 = blockIdx.y * MR;
   bf16_t h[PER], weight;
-  float row_squares[PER];
+  float* row_squares = reinterpret_cast<float*>(s_all + BEFORE);
   NormRows<KW * WAVE> rows;
   if constexpr (NORM) rows.load(norm, m, k);
   #pragma unroll
@@ -397,16 +428,16 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     const int at = min(n0 + lo, n - 1);
     #pragma unroll
     for (int f = 0; f < PER; ++f)
-      h[f] = add.h[(long)(row0 + min(first + f * ROWS, m_here - 1)) * n + at];
+      h[f] = add.h[(long)min(first + f * ROWS, m_here - 1) * n + at];
     weight = add.weight[at];
   } else if (!NORM && of.squares != nullptr) {
     // added up here: kept until the end they take registers, and so workgroups of
     // a CU (q4_0, one row, 8 layers of 5120: 568 us instead of 547)
-    #pragma unroll
-    for (int f = 0; f < PER; ++f) {
-      RowSquares parts;
-      parts.load(of, row0 + min(first + f * ROWS, m_here - 1));
-      row_squares[f] = parts.sum(of);
+    for (int r = wave; r < m_here; r += KW) {
+      RowSquares<3> parts;
+      parts.load(of, r);
+      const float q = parts.sum(of);
+      if (lane == 0) row_squares[r] = q;
     }
   }
   if constexpr (NORM) {
@@ -429,7 +460,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       if (i + s < steps) {
         if (i + s + P <= steps) wait_loads<(P - 1) * LOADS>();
         else wait_loads<0>();
-        use(s, c0 + i + s, integral_constant<bool, K_QUANT>{});
+        use(s, c0 + i + s, integral_constant<bool, K_QUANT && !THIN>{});
         if (i + s + P < steps) {
           wait_lds_reads();
           load(s, c0 + i + s + P);
@@ -453,10 +484,6 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     heads.positions += blockIdx.y * MR;
     heads.slots += blockIdx.y * MR;
   }
-  if constexpr (C == Columns::ADDED) {
-    add.sum += (long)row0 * y_ld;
-    add.squares += (long)row0 * gridDim.x;
-  }
   #pragma unroll
   for (int f = 0; f < PER; ++f) {
     const int r = first + f * ROWS, c = lo;
@@ -464,11 +491,14 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     float scale = 1.f;
     if constexpr (NORM) scale = norm_scale<KW>(squares, r, k, norm.eps);
     else if (C != Columns::ADDED && of.squares != nullptr)
-      scale = undivided_scale(of, row_squares[f], k);
+      scale = undivided_scale(of, row_squares[r], k);
     auto sum = [&](int c) {
       float v = 0.f;
       #pragma unroll
-      for (int q = 0; q < KW; ++q) v += red[(q * BM + r) * (16 + PAD) + c];
+      for (int q = 0; q < KW; ++q) {
+        v += red[(q * BM + r) * (16 + PAD) + c];
+        if constexpr (THIN) v += red[(q * BM + r + 8) * (16 + PAD) + c + 8];
+      }
       if constexpr (Q == Quant::Q4_K && !NORM)
         if (v != v) {
           const long at = weight_row<C>(n0, c, n, half);
@@ -482,12 +512,13 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     } else if constexpr (C == Columns::HEADS) {
       if (c < 8) finish_heads(y, y_ld, heads, r, n0 + c, sum(c), sum(c + 8));
     } else if constexpr (C == Columns::ADDED) {
-      const bool there = n0 + c < n;
+      const bool there = (!THIN || c < 8) && n0 + c < n;
       finish_added(add, y, (long)r * y_ld + n0 + c, r, there,
                    there ? bf2f(h[f]) : 0.f,
                    bf2f(weight), there ? sum(c) : 0.f);
     } else {
-      if (n0 + c < n) y[(long)r * y_ld + n0 + c] = f2bf(sum(c));
+      if ((!THIN || c < 8) && n0 + c < n)
+        y[(long)r * y_ld + n0 + c] = f2bf(sum(c));
     }
   }
 }
@@ -495,6 +526,24 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
 }  // namespace
 
 // Blocks whose scales come in pairs (k a multiple of 64), or of 256.
+// Whether a workgroup has eight weight rows instead of 16: where some CUs would have
+// two workgroups and others one, all have two or three half as large. Rows shorter
+// than 4096 are read too soon for that to matter, and x, which is read once more,
+// counts more from five rows on. us, MI355X, 16 -> eight, 5120 x
+// 5120, 5120 x 13824, 6144 x 16384 (4096 rows and fewer, q4_0 of one: 4096 x 11008
+// 9.5 -> 11.4; 5120 x 2048, 5 rows 4.9 -> 5.2):
+//   q4_0  1 row    7.7 15.9 19.2 ->  7.3 14.6 17.1
+//         5 rows   9.0 18.9 22.9 ->  8.7 17.1 20.7
+//   q8_0  3 rows   9.9 22.2 28.4 ->  9.8 20.7 25.9
+//         5 rows  10.8 23.1 28.3 -> 10.4 21.9 26.3
+//   q4_K  1 row    8.3 19.9 22.2 ->  7.6 15.9 18.9
+//         5 rows   9.6 23.3 25.7 ->  9.3 19.7 23.3
+bool rows_quant_thin(int m, int n, int k, Quant q, bool paired) {
+  return m <= 8 && !paired && n > 256 * 16 &&
+         n <= (m <= 4 ? 384 : 352) * 16 && k >= 4096 &&
+         q != Quant::Q6_K && (m > 1 || q != Quant::Q8_0);
+}
+
 bool rows_quant_takes(int m, int n, int k, Quant q, bool gated) {
   const int step = q == Quant::Q4_K || q == Quant::Q6_K ? 256 : 64;
   return m >= 1 && m <= 64 && n >= 1 && k >= step && k % step == 0 &&
@@ -507,23 +556,32 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
                        const AddTo* add, const Undivided* of,
                        hipStream_t stream) {
   const f16_t* sc = reinterpret_cast<const f16_t*>(scales);
-  auto go = [&](auto qc, auto mr, auto me, auto kw, auto p) {
+  auto go = [&](auto qc, auto mr, auto me, auto kw, auto p, auto t) {
     constexpr Quant QQ = decltype(qc)::value;
     constexpr int MR = decltype(mr)::value, ME = decltype(me)::value,
                   KW = decltype(kw)::value, P = decltype(p)::value;
-    const dim3 grid((n + 15) / 16, (m + MR - 1) / MR), block(KW * WAVE);
-    auto pick = [&](auto normed) {
-      constexpr bool N = decltype(normed)::value;
-      return heads ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::HEADS, N>
-             : gated ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::GATED, N>
-                     : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN,
-                                         N>;
-    };
+    constexpr bool THIN = decltype(t)::value;
+    constexpr int ROWS = THIN ? 8 : 16;
+    const dim3 grid((n + ROWS - 1) / ROWS, (m + MR - 1) / MR),
+        block(KW * WAVE);
     auto kernel = add ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::ADDED,
-                                          false>
-                      : pick(std::false_type{});
-    if constexpr (MR == NORM_ROWS)
-      if (norm) kernel = pick(std::true_type{});
+                                          false, THIN>
+                      : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN,
+                                          false, THIN>;
+    if constexpr (!THIN) {
+      auto pick = [&](auto normed) {
+        constexpr bool N = decltype(normed)::value;
+        return heads ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::HEADS, N,
+                                         false>
+               : gated ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::GATED,
+                                           N, false>
+                       : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN,
+                                           N, false>;
+      };
+      if (!add) kernel = pick(std::false_type{});
+      if constexpr (MR == NORM_ROWS)
+        if (norm) kernel = pick(std::true_type{});
+    }
     kernel<<<grid, block, 0, stream>>>(y, x, sc, qs, m, n, k,
                                        heads ? *heads : Heads{},
                                        norm ? *norm : NormOf{},
@@ -550,24 +608,42 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
     constexpr integral_constant<int, ONE ? 1 : 2> some{};
     constexpr integral_constant<int, QQ == Quant::Q6_K ? 1 : 2> one_row{};
     constexpr integral_constant<int, QQ == Quant::Q8_0 ? 4 : 8> waves{};
-    const bool thin = n <= 384 * 16;
-    if (m == 1) {
+    const bool few = n <= 384 * 16;
+    const bool thin = !norm && rows_quant_thin(m, n, k, QQ, gated || heads);
+    constexpr std::false_type no{};
+    constexpr std::true_type yes{};
+    constexpr bool CAN = QQ != Quant::Q6_K;
+    if (thin) {
+      if constexpr (CAN) {
+        // more waves, or stages in flight, of more rows: 5120 x 5120 of five, q4_0
+        // 8.7 us by four waves, 13.0 by eight, 14.3 with two stages
+        if constexpr (QQ != Quant::Q8_0) {
+          if (m == 1) go(qc, c4, c1, c8, c1, yes);
+          else if (m <= 4) go(qc, c4, c4, c4, c1, yes);
+          else go(qc, c8, c4, c4, c1, yes);
+        } else {
+          constexpr integral_constant<int, 2> c2{};
+          if (m <= 4) go(qc, c4, c4, c4, c1, yes);
+          else go(qc, c8, c4, c2, c2, yes);
+        }
+      }
+    } else if (m == 1) {
       if constexpr (QQ != Quant::Q8_0) {
         // q4_0, 4096 x 11008: one stage in flight 11.5 us, two 9.6
-        if (thin) go(qc, c4, c1, waves, one_row);
-        else go(qc, c4, c1, c4, some);
+        if (few) go(qc, c4, c1, waves, one_row, no);
+        else go(qc, c4, c1, c4, some, no);
       }
     } else if (m <= 4) {
-      if (thin) go(qc, c4, c4, waves, some);
-      else go(qc, c4, c4, c4, some);
+      if (few) go(qc, c4, c4, waves, some, no);
+      else go(qc, c4, c4, c4, some, no);
     } else if (m <= 8) {
       constexpr integral_constant<int, QQ == Quant::Q8_0 ? 2 : 1> one{};
-      if (thin) go(qc, c8, c4, waves, one);
-      else go(qc, c8, c4, c4, some);
+      if (few) go(qc, c8, c4, waves, one, no);
+      else go(qc, c8, c4, c4, some, no);
     } else if (m <= 16) {
-      go(qc, c16, c4, c4, c1);
+      go(qc, c16, c4, c4, c1, no);
     } else {
-      go(qc, c32, c4, c4, c1);
+      go(qc, c32, c4, c4, c1, no);
     }
   };
   switch (q) {
