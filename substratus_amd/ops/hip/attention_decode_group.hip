@@ -24,6 +24,7 @@
 // Four waves (one workgroup per CU): 96, 98, 10.9, 20.4, 25; one: 95, 86, 14.8,
 // 17.9, 27, with weights in two bf16 parts. Three, which keep all their bits,
 // cost 1 % (the last shape 6 %).
+#include "attention_order.h"
 #include "rows_gemm.h"
 
 namespace {
@@ -67,7 +68,7 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit,
+                       long q_ld, int nsplit, bool ordered,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
   constexpr int RC = D / 8;                      // 16-byte pieces of a row
@@ -79,9 +80,12 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
   // the direct loads in flight, and waits for them
   __shared__ alignas(16) uint4v s_all[NW * 2 * 2 * HALF];
 
-  const int b = blockIdx.x, split = blockIdx.z;
+  const int split = blockIdx.y;
+  const int b = ordered ? sequence_at(seq_lens, gridDim.z, max_blocks * PAGE,
+                                      blockIdx.z)
+                        : blockIdx.z;
   const int in_group = hq / hkv, parts = (in_group + 15) / 16;
-  const int kvh = blockIdx.y / parts, h0 = blockIdx.y % parts * 16;
+  const int kvh = blockIdx.x / parts, h0 = blockIdx.x % parts * 16;
   const int head0 = kvh * in_group + h0, heads = min(16, in_group - h0);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
@@ -298,15 +302,34 @@ void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
                        const int* seq_lens, int bsz, int hq, int hkv, int d,
                        int max_blocks, float scale, long q_ld, int nsplit,
                        float* part_o, float* part_ml, hipStream_t stream) {
+  if (bsz > MOST) {               // the others first
+    const long at = MOST;
+    launch_attn_group(out + at * hq * d, q + at * q_ld, kc, vc,
+                      block_table + at * max_blocks, seq_lens + at, bsz - MOST,
+                      hq, hkv, d, max_blocks, scale, q_ld, nsplit,
+                      part_o ? part_o + at * hq * nsplit * d : nullptr,
+                      part_ml ? part_ml + at * hq * nsplit * 2 : nullptr,
+                      stream);
+    bsz = MOST;
+  }
   const int parts = (hq / hkv + 15) / 16;
-  const dim3 grid(bsz, hkv * parts, nsplit), block(NW * WAVE);
+  // as in attention_decode_heads.hip; us, 32 heads on 8 of 128:
+  //   sequences x most keys    unlike          all            one
+  //   8 x 2500               20.9 -> 19.5   23.4 -> 22.8   17.0 -> 12.9
+  //   64 x 300               17.5 -> 17.2
+  //   64 x 2500              92.9 -> 85.0    127 -> 127    52.9 -> 35.8
+  //   256 x 2500              316 -> 291     461 -> 460    86.6 -> 64
+  const dim3 grid(hkv * parts, nsplit, bsz), block(NW * WAVE);
+  const bool ordered = orders_sequences(bsz, max_blocks, nsplit,
+                                        (long)bsz * hkv * parts * nsplit,
+                                        d == 128 ? 2 : 4);
   if (d == 128) {
     attn_group_kernel<128><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, part_o, part_ml);
+        q_ld, nsplit, ordered, part_o, part_ml);
   } else {
     attn_group_kernel<64><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, part_o, part_ml);
+        q_ld, nsplit, ordered, part_o, part_ml);
   }
 }

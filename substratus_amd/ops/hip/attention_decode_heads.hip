@@ -21,7 +21,7 @@
 //   256 of 620, 32 heads                    319 -> 316  (6.2 TB/s)
 //   30 of 700, 12 heads of 64              18.1 -> 13.8
 //   40 of 800, fp8, 71 heads on 1 of 64    49.0 -> 28.4
-#include "common.h"
+#include "attention_order.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -89,14 +89,17 @@ void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit,
+                       long q_ld, int nsplit, bool ordered,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
   constexpr int LANES = D / 8;                   // of a row
   constexpr int ROWS = WAVE / LANES;             // of a piece of all lanes
   constexpr int KEYS = PIECES * ROWS;            // of a step
   constexpr int SIZE = KV8 ? 1 : 2;
-  const int b = blockIdx.x, head = blockIdx.y, split = blockIdx.z;
+  const int head = blockIdx.x, split = blockIdx.y;
+  const int b = ordered ? sequence_at(seq_lens, gridDim.z, max_blocks * PAGE,
+                                      blockIdx.z)
+                        : blockIdx.z;
   const int kvh = head / (hq / hkv);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE, row = lane / LANES, at = lane % LANES;
@@ -302,14 +305,39 @@ void launch_attn_heads(bf16_t* out, const bf16_t* q, const void* kc,
                        int max_blocks, float scale, long q_ld, int waves,
                        int nsplit, float* part_o, float* part_ml, bool kv8,
                        hipStream_t stream) {
-  const dim3 grid(bsz, hq, nsplit);
+  if (bsz > MOST) {               // the others first
+    const long at = MOST;
+    launch_attn_heads(out + at * hq * d, q + at * q_ld, kc, vc,
+                      block_table + at * max_blocks, seq_lens + at, bsz - MOST,
+                      hq, hkv, d, max_blocks, scale, q_ld, waves, nsplit,
+                      part_o ? part_o + at * hq * nsplit * d : nullptr,
+                      part_ml ? part_ml + at * hq * nsplit * 2 : nullptr, kv8,
+                      stream);
+    bsz = MOST;
+  }
+  // a sequence's heads and shares next to each other: the sequence itself as the
+  // fastest put all heads of one on the same eighth of the chip where there are
+  // eight of them, and long ones last. us, MI355X, keys from a quarter of the most
+  // to all, all of them, one of them (the others' a twentieth), sequences first ->
+  // heads first, and in order from 1000 on:
+  //   heads x most keys        unlike          all            one
+  //   8 x 32 x 1000          19.7 -> 19.3   24.1 -> 24.3
+  //   64 x 32 x 300          39.2 -> 36.7
+  //   64 x 32 x 1000          119 -> 107     166 -> 170
+  //   64 x 32 x 2500          288 -> 261     410 -> 414     120 -> 46
+  //   256 x 32 x 1000         431 -> 423     669 -> 663
+  //   100 x 12 (64) x 2500   90.7 -> 82.2    122 -> 125    36.1 -> 22
+  const dim3 grid(hq, nsplit, bsz);
+  const bool ordered = orders_sequences(bsz, max_blocks, nsplit,
+                                        (long)bsz * hq * nsplit,
+                                        16 / waves);
   auto go = [&](auto dim, auto fp8, auto w) {
     constexpr int W = decltype(w)::value;
     attn_heads_kernel<decltype(dim)::value, decltype(fp8)::value, W>
         <<<grid, dim3(W * WAVE), 0, stream>>>(
             out, q, reinterpret_cast<const char*>(kc),
             reinterpret_cast<const char*>(vc), block_table, seq_lens, hq, hkv,
-            max_blocks, scale, q_ld, nsplit, part_o, part_ml);
+            max_blocks, scale, q_ld, nsplit, ordered, part_o, part_ml);
   };
   auto sized = [&](auto dim, auto fp8) {
     if (waves == 8) go(dim, fp8, std::integral_constant<int, 8>());

@@ -1,0 +1,67 @@
+"""Decode attention of more workgroups than the chip holds, which take sequences
+by length: each has its own keys, whatever the lengths are."""
+
+import pytest
+import torch
+
+from substratus_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# sequences of a part of a wave, of one, of two and of all four; all lengths
+# equal, none, the table's room; grouped heads and heads by themselves
+@pytest.mark.parametrize("batch", [2, 63, 64, 65, 129, 256, 257])
+@pytest.mark.parametrize("hq,hkv,d", [(64, 16, 64), (32, 8, 128), (64, 64, 64)])
+@pytest.mark.parametrize("how", ["unlike", "equal", "one", "none"])
+@torch.no_grad()
+def test_own_keys(batch, hq, hkv, d, how):
+    g = torch.Generator().manual_seed(batch + d)
+    room = 62 if batch < 100 else 60
+    most = room * 16
+    lens = torch.randint(1, most + 1, (batch,), generator=g)
+    if how == "equal":
+        lens[:] = most - 3
+    elif how == "one":
+        lens[:] = 5
+        lens[batch // 2] = most
+    elif how == "none":
+        lens[::3] = 0
+    # few pages, shared by sequences: what tells them apart is their order
+    kc, vc = (torch.randn(70, hkv, 16, d, device=DEV).bfloat16()
+              for _ in range(2))
+    table = torch.randint(0, 70, (batch, room), generator=g).int().to(DEV)
+    q = torch.randn(batch, hq, d, device=DEV).bfloat16()
+    n = lens.int().to(DEV)
+    out = ops.paged_attn_decode(q, kc, vc, table, n, d ** -0.5)
+    per = hq // hkv
+    for b in {0, 1, batch // 2, batch - 1, int(lens.argmax()),
+              int(lens.argmin())}:
+        if lens[b] == 0:
+            assert not out[b].any()
+            continue
+        k, v = (c[table[b].long()].transpose(0, 1).reshape(hkv, -1, d)
+                [:, :lens[b]].double().repeat_interleave(per, 0)
+                for c in (kc, vc))
+        s = torch.einsum("hd,hnd->hn", q[b].double(), k) * d ** -0.5
+        want = torch.einsum("hn,hnd->hd", s.softmax(-1), v)
+        # results are rounded to bf16, weights have 24 bits
+        assert float((out[b].double() - want).norm()) <= \
+            2.0 ** -8 * float(want.norm()), b
+
+
+@pytest.mark.parametrize("hq", [2, 4])
+@torch.no_grad()
+def test_more_sequences_than_a_grid_side(hq):
+    batch, d = 65535 + 9, 64
+    kc, vc = (torch.randn(50, 2, 16, d, device=DEV).bfloat16()
+              for _ in range(2))
+    table = torch.randint(0, 50, (batch, 1), device=DEV).int()
+    q = torch.randn(batch, hq, d, device=DEV).bfloat16()
+    n = torch.randint(1, 17, (batch,), device=DEV).int()
+    out = ops.paged_attn_decode(q, kc, vc, table, n, 0.125)
+    for part in (slice(0, 9), slice(batch - 18, batch)):
+        assert torch.equal(out[part], ops.paged_attn_decode(
+            q[part].contiguous(), kc, vc, table[part].contiguous(),
+            n[part].contiguous(), 0.125))
