@@ -7,17 +7,20 @@
 // counts what is not below (one comparison per logit, a wave's count out of its
 // mask), top-p adds it up. A step costs one barrier.
 //
-// Bound by the chain of steps; one row occupies a CU. us on a MI355X, from 16
-// (32) halvings a threshold, weights past 32768 made again for the draw and one
-// lane going through a run:
-//                                    greedy    no threshold  top-k 40  top-p .92
-//   192 x 32000                    6.3 -> 6.5  17.3 -> 12.6  29.7 23.4 33.3 22.4
-//   64 x 50272                     7.4 -> 6.8  56.4 -> 17.2  77.9 33.0 77.6 28.6
-//   256 x 65024                   20.8 -> 11.4 84.6 -> 35.3   120 57.8  112 48.8
-//   192 x 32000 in 32 bits         7.8 -> 8.0  18.7 -> 14.3  43.0 25.0 48.2 33.8
-//   256 x 1000                     4.7 -> 4.7   7.3 -> 6.9   14.0 14.8 17.6 17.4
-// (65024 tokens take the kernel of ten rounds of eight weights, which is short of
-// registers).
+// Thresholds of bf16 rows of more than 8192 tokens take no steps where they are among
+// the 512 largest numbers: the tokens of each of these are counted in LDS.
+//
+// Bound by vector arithmetic over a row, which one CU has: an operation on every
+// logit takes 0.2 us of 32000, its weight 1.5, a step of a search 0.7 to 1, the
+// draw's sums in order 5. us on a MI355X, from a search of 4 to 10 steps for every
+// threshold and the largest logit found number by number:
+//                     greedy      no threshold  top-k 40      top-p .92
+//   192 x 32000    6.8 ->  5.5   13.2 -> 12.7   23.5 -> 15.2  22.4 -> 17.1
+//   64 x 50272     7.2 ->  5.8   17.8 -> 16.5   33.7 -> 20.6  28.4 -> 22.2
+//   256 x 65024   11.7 ->  9.8   36.1 -> 25.6   57.4 -> 32.2  48.8 -> 34.4
+//   256 x 1000     4.9 ->  3.7    7.1 ->  6.7   15.1 -> 14.8  18.0 -> 15.5
+//   192 x 32000, logits of +-0.1, top-p .92     28.4 -> 25.9 (steps)
+//   192 x 32000 in 32 bits   8.1    14.5          24.6           30.7
 #include "common.h"
 
 #define SBLOCK 1024
@@ -27,6 +30,7 @@
 #define RUNS 256                  // runs of tokens that a draw's edges are of
 #define LIST 64                   // weights that share 16 bits of a logit
 #define SEG 320                   // tokens of a run, at most
+#define BINS 512                  // keys below the largest that are counted
 
 namespace {
 
@@ -117,6 +121,37 @@ struct Totals {
   }
 };
 
+typedef __attribute__((ext_vector_type(2))) short short2v;
+typedef __attribute__((ext_vector_type(2))) unsigned short ushort2v;
+
+// Two bf16 numbers as numbers of 16 bits in the same order: 0 is -inf, USUAL the
+// largest that is neither infinite nor NaN (which are above it, of either sign).
+// A number's key16_of less that of -inf.
+constexpr unsigned USUAL = 0xff00u;
+DEV_INLINE ushort2v order16(unsigned w) {
+  const short2v s = __builtin_bit_cast(short2v, w);
+  const unsigned k =
+      w ^ (__builtin_bit_cast(unsigned, (short2v)(s >> 15)) & 0x7fff7fffu);
+  return __builtin_bit_cast(ushort2v, k) - (unsigned short)0x807f;
+}
+
+// Before a lane: the sums of all lanes ahead of it, by moves to the next lane, the
+// second, fourth and eighth of a row, and of whole rows to those behind them.
+template <int CTRL, int ROWS>
+DEV_INLINE float moved(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(
+      0u, __float_as_uint(v), CTRL, ROWS, 0xf, true));
+}
+DEV_INLINE float sum_upto(float v) {             // a lane's own included
+  v += moved<0x111, 0xf>(v);
+  v += moved<0x112, 0xf>(v);
+  v += moved<0x114, 0xf>(v);
+  v += moved<0x118, 0xf>(v);
+  v += moved<0x142, 0xa>(v);                     // a row's last to the next row
+  v += moved<0x143, 0xc>(v);                     // lane 31 to the upper half
+  return v;
+}
+
 // What the wave has written to LDS may be read by all of its lanes.
 DEV_INLINE void wait_lds() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -140,23 +175,87 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   const T* row = logits + (long)b * vocab;
   const float temp = temperature[b];
 
+  // weights for the draw, and before that how many tokens have a key
+  constexpr int PART = NR < 4 ? NR : 4;     // rounds whose weights fit LDS
+  __shared__ alignas(16) float s_w[PART * SROUND];
+  int* bins = reinterpret_cast<int*>(s_w);
+  constexpr bool EXACT = sizeof(T) == 2;        // 16 bits are all of a logit
+  constexpr bool HALVED = EXACT && NR == 1;
+  constexpr bool COUNTED = EXACT && !HALVED;
+  if (COUNTED && tid < BINS) bins[tid] = 0;
+
   // the largest logit; the smallest index of several. NaN is passed over.
   Eight<T> raw[NR];
   float best = -INFINITY, least = INFINITY;
   int besti = 0x7fffffff;
+  auto look_at = [&](float v, int i) {
+    if (v > best) { best = v; besti = i; }
+    least = fminf(least, v > -INFINITY ? v : INFINITY);
+  };
+  // (read again: kept for the few rows that need it they are short of registers)
+  auto look = [&]() {
+    for (int i = tid; i < vocab; i += SBLOCK) look_at(val(row[i]), i);
+  };
   #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    const int at = r * SROUND + tid * SVEC;
-    raw[r].template load<VEC>(row, at, vocab);
+  for (int r = 0; r < NR; ++r)
+    raw[r].template load<VEC>(row, r * SROUND + tid * SVEC, vocab);
+  // Two numbers an operation where all of a row are finite or -inf, not all -inf:
+  // usual. (Of others each is looked at by itself.)
+  bool usual = false;
+  float top = -INFINITY;
+  unsigned mine = 0;
+  if constexpr (EXACT) {
+    ushort2v most = {0, 0};
     #pragma unroll
-    for (int j = 0; j < SVEC; ++j) {
-      const float v = raw[r][j];
-      if (v > best) { best = v; besti = at + j; }
-      least = fminf(least, v > -INFINITY ? v : INFINITY);
-    }
+    for (int r = 0; r < NR; ++r)
+      #pragma unroll
+      for (int i = 0; i < Eight<T>::WORDS; ++i)
+        most = __builtin_elementwise_max(most, order16(raw[r].w[i]));
+    mine = max((unsigned)most[0], (unsigned)most[1]);
+    top = totals.most(wave_max(
+        mine > USUAL ? INFINITY : number16<T>(mine + key16_of(-INFINITY))));
+    usual = top < INFINITY && top > -INFINITY;
+  }
+  if constexpr (EXACT) {
+    if (!usual) look();
+  } else {
+    #pragma unroll
+    for (int r = 0; r < NR; ++r)
+      #pragma unroll
+      for (int j = 0; j < SVEC; ++j)
+        look_at(raw[r][j], r * SROUND + tid * SVEC + j);
   }
 
   // ---- greedy ---------------------------------------------------------
+  if (temp <= 0.f && usual) {
+    if (tid == 0) s_tok = 0x7fffffff;
+    __syncthreads();
+    // zeros of either sign are equal, of other numbers a thread knows its largest
+    if (top == 0.f || mine + key16_of(-INFINITY) == key16_of(top)) {
+      // read again, which the compiler is not to know: the row kept for this takes
+      // registers from all that follows (256 x 65024, no threshold: 39 us for 26).
+      // Not one by one: that takes longer than they would.
+      int from = tid * SVEC;
+      if constexpr (VEC || NR > 4) asm volatile("" : "+v"(from));
+      Eight<T> again[NR];
+      #pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        if constexpr (VEC || NR > 4)
+          again[r].template load<VEC>(row, r * SROUND + from, vocab);
+        else
+          again[r] = raw[r];
+      }
+      #pragma unroll
+      for (int r = NR - 1; r >= 0; --r)
+        #pragma unroll
+        for (int j = SVEC - 1; j >= 0; --j)
+          if (again[r][j] == top) besti = r * SROUND + from + j;
+      if (besti < vocab) atomicMin(&s_tok, besti);
+    }
+    __syncthreads();
+    if (tid == 0) out[b] = s_tok;
+    return;
+  }
   if (temp <= 0.f) {
     #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -179,25 +278,73 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
 
   // temperature is applied in fp32, to the logits as they came
   const float inv_t = 1.f / temp;
-  const float top = totals.most(wave_max(best));
+  if (!usual) top = totals.most(wave_max(best));
   const float m = top * inv_t;
   // NaN, and what went past the largest number beside the largest logit: 0. A
   // logit below the largest may be equal to it once scaled (of neighbours in 32
   // bits about a tenth are), and weighs as much then.
   const float past = m == -INFINITY ? m : INFINITY;
   auto weight = [&](float v) {
-    const float x = v * inv_t, below = __expf(x - m);
+    const float x = v * inv_t, below = __expf(fmaf(v, inv_t, -m));
     return v == top ? 1.f : x < past ? below : 0.f;
   };
-  float e[NR][SVEC];
-  #pragma unroll
-  for (int r = 0; r < NR; ++r)
-    #pragma unroll
-    for (int j = 0; j < SVEC; ++j) {
-      e[r][j] = weight(raw[r][j]);      // past the row's end: as of -inf
-      // a few at a time, or their parts take the registers of the row
-      if (j % (NR <= 4 ? 4 : 1) == 0) __builtin_amdgcn_sched_barrier(0);
+  // of usual ones none is past the largest, and that is 1 as any is
+  const bool plain = usual && fabsf(m) < INFINITY;
+  const unsigned first = key16_of(-INFINITY), last = key16_of(top);
+  const int k = top_k[b];
+  const float p_target = top_p[b];
+  const bool some = k > 0 && k < vocab, share = p_target > 0.f &&
+                                                p_target < 1.f;
+  // Where 512 keys from the largest one down are enough, thresholds are found
+  // without steps: one pass counts the tokens of each, and every wave adds them up,
+  // eight keys a lane. (With few of a row's numbers within them, or not all usual,
+  // steps it is.) us, 192 x 32000, steps -> counts: top-k 40 23.7 -> 15.1, 2000
+  // 32.7 -> 15.0, top-p .92 22.3 -> 16.3.
+  constexpr int EACH_BIN = BINS / WAVE;
+  float tokens[EACH_BIN];
+  // (a share of a row whose 512th key still weighs half as much: not there)
+  const bool counted =
+      COUNTED && plain &&
+      (some || (share && weight(number16<T>(max(last, first + BINS) - BINS)) <
+                             0.5f));
+  if constexpr (COUNTED) {
+    if (counted) {
+      const unsigned topmost = last - first;
+      #pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        #pragma unroll
+        for (int i = 0; i < Eight<T>::WORDS; ++i) {
+          const ushort2v u = order16(raw[r].w[i]);
+          #pragma unroll
+          for (int j = 0; j < 2; ++j)
+            if (topmost - u[j] < (unsigned)BINS)
+              atomicAdd(&bins[topmost - u[j]], 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __syncthreads();
+      #pragma unroll
+      for (int j = 0; j < EACH_BIN; ++j)
+        tokens[j] = (float)bins[lane * EACH_BIN + j];
     }
+  }
+  auto key_at = [&](int i) { return (unsigned)max((int)last - i, (int)first); };
+
+  float e[NR][SVEC];
+  auto weigh = [&](auto by) {
+    #pragma unroll
+    for (int r = 0; r < NR; ++r)
+      #pragma unroll
+      for (int j = 0; j < SVEC; ++j) {
+        e[r][j] = by(raw[r][j]);        // past the row's end: as of -inf
+        // a few at a time, or their parts take the registers of the row
+        if (j % (NR <= 4 ? 4 : 1) == 0) __builtin_amdgcn_sched_barrier(0);
+      }
+  };
+  if (plain) weigh([&](float v) {
+    return v == top ? 1.f : __expf(fmaf(v, inv_t, -m));
+  });
+  else weigh(weight);
   auto sum_from = [&](float t) {
     float s = 0.f;
     #pragma unroll
@@ -231,12 +378,8 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   // much of a row, and top-p of that, fit it least.)
   // Up to 8192 logits of 16 bits cost less to halve than to list: us, 256 rows of
   // 1000, top-k 40, top-p .9, halved 14.2 17.9, by lines throughout 16.7 32.4.
-  constexpr bool EXACT = sizeof(T) == 2;        // 16 bits are all of them
-  constexpr bool HALVED = EXACT && NR == 1;
   constexpr float FEW = HALVED ? -1.f : LIST;
   constexpr float MANY = 1e9f;
-  const unsigned first = key16_of(-INFINITY), last = key16_of(top);
-  const int k = top_k[b];
   const bool large = NR == 1 || (k >= 1024 && k < vocab);
   struct Measured { bool holds; float f, n; };
   struct Ends { unsigned lo, hi; float above; };   // tokens from hi on
@@ -329,16 +472,50 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
     return key > last ? INFINITY : weight(number16<T>(key));
   };
 
+  // The first bin whose sum with those before it passes, or BINS. value(lane's
+  // j-th bin) is added up.
+  auto first_bin = [&](auto value, auto passes) {
+    float own[EACH_BIN], all = 0.f;
+    #pragma unroll
+    for (int j = 0; j < EACH_BIN; ++j) {
+      own[j] = value(j);
+      all += own[j];
+    }
+    float sum = sum_upto(all) - all;
+    int at = BINS;
+    #pragma unroll
+    for (int j = 0; j < EACH_BIN; ++j) {
+      sum += own[j];
+      if (at == BINS && passes(sum, j)) at = lane * EACH_BIN + j;
+    }
+    const unsigned long long any = __ballot(at < BINS);
+    return any ? __builtin_amdgcn_readlane(at, __ffsll(any) - 1) : BINS;
+  };
+
   // ---- top-k: as many largest as are no more than k with all their equals,
   // ---- the largest and its equals in any case. Measured: tokens
   float thresh = 0.f, floor = -INFINITY;
-  if (k > 0 && k < vocab) {
-    const float from = HALVED ? 0.f : fmaxf(
-        -totals.most(wave_max(-least)), top - 60.f * temp);
-    const Ends at = search(large ? 1 : 4, [&](float t) {
-      const float n = count_from(t);
-      return Measured{n > (float)k, fmaxf(n, 0.5f), n};
-    }, __logf((float)k + 0.5f), from, __logf((float)vocab), __logf(0.5f));
+  if (some) {
+    Ends at{};
+    int bin = BINS;
+    if (counted) {
+      bin = first_bin([&](int j) { return tokens[j]; },
+                      [&](float n, int) { return n > (float)k; });
+      at = Ends{key_at(bin), key_at(bin) + 1, 0.f};
+      // a key whose tokens weigh as much as the next one's counts with it
+      if (bin > 0 && bin < BINS &&
+          !(weight(number16<T>(at.lo)) < weight(number16<T>(at.hi))))
+        bin = BINS;
+    }
+    if (bin == BINS) {
+      if (usual) look();
+      const float from = HALVED ? 0.f : fmaxf(
+          -totals.most(wave_max(-least)), top - 60.f * temp);
+      at = search(large ? 1 : 4, [&](float t) {
+        const float n = count_from(t);
+        return Measured{n > (float)k, fmaxf(n, 0.5f), n};
+      }, __logf((float)k + 0.5f), from, __logf((float)vocab), __logf(0.5f));
+    }
     if (EXACT && at.hi - at.lo == 1) {
       floor = number16<T>(min(at.hi, last));
       thresh = weight(floor);
@@ -361,19 +538,30 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   // ---- top-p: the fewest largest weights with that share. Measured: what is
   // ---- left out, which a goal's share of the tokens at most has if each weighs
   // ---- no more than at the first key
-  const float p_target = top_p[b];
-  if (p_target > 0.f && p_target < 1.f) {
+  if (share) {
     const float all = sum_from(thresh), goal = p_target * all;
     const float out = all - goal, low = thresh;
     auto enough = [&](float t) { return t < low || sum_from(t) >= goal; };
     constexpr float LESS = 0.135f;              // than what is to be left out
-    const unsigned lo = search(large ? 1 : 8, [&](float t) {
-      if (t < low) return Measured{true, LESS * out, MANY};
-      const float s = sum_from(t);
-      return Measured{s >= goal, fmaxf(all - s, 1e-3f * out),
-                      s >= goal ? MANY : 0.f};
-    }, __logf(out), fmaxf(floor, top - __logf((float)vocab / out) * temp),
-       __logf(LESS * out), __logf(all)).lo;
+    unsigned lo = 0;
+    int bin = BINS;
+    if (counted) {
+      float w[EACH_BIN];
+      #pragma unroll
+      for (int j = 0; j < EACH_BIN; ++j)
+        w[j] = weight(number16<T>(key_at(lane * EACH_BIN + j)));
+      bin = first_bin([&](int j) { return tokens[j] * w[j]; },
+                      [&](float s, int j) { return w[j] < low || s >= goal; });
+      lo = key_at(bin);
+    }
+    if (bin == BINS)
+      lo = search(large ? 1 : 8, [&](float t) {
+        if (t < low) return Measured{true, LESS * out, MANY};
+        const float s = sum_from(t);
+        return Measured{s >= goal, fmaxf(all - s, 1e-3f * out),
+                        s >= goal ? MANY : 0.f};
+      }, __logf(out), fmaxf(floor, top - __logf((float)vocab / out) * temp),
+         __logf(LESS * out), __logf(all)).lo;
     thresh = fmaxf(low, weight(number16<T>(lo)));
     if constexpr (!EXACT) {
       const float high = weight_from(lo + 1), above = sum_from(high);
@@ -396,8 +584,6 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   // that a row and a number keep their token, the sum is that of 256 threads
   // over every 256th token, the edges those of 256 runs of tokens, added up
   // from left to right, as they always were.
-  constexpr int PART = NR < 4 ? NR : 4;     // rounds whose weights fit LDS
-  __shared__ alignas(16) float s_w[PART * SROUND];
   __shared__ alignas(16) float s_run[RUNS];
   __shared__ alignas(16) float s_one[SEG];
   const int run = (vocab + RUNS - 1) / RUNS;
@@ -405,7 +591,7 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   float sum = 0.f;
   #pragma unroll
   for (int r0 = 0; r0 < NR; r0 += PART) {
-    if (r0 > 0) __syncthreads();
+    if (r0 > 0 || counted) __syncthreads();     // (all have read the bins)
     #pragma unroll
     for (int r = r0; r < NR && r < r0 + PART; ++r) {
       float4 w[2];

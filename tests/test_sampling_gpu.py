@@ -206,3 +206,54 @@ def test_number_at_the_last_edge(dtype):
         torch.zeros(1, device=DEV).int(), torch.ones(1, device=DEV),
         torch.full((1,), 2.0, device=DEV))
     assert int(got) == 699
+
+
+@pytest.mark.parametrize("k", [1, 509, 510, 511, 512, 513, 600])
+@pytest.mark.parametrize("p", [1.0, 0.3, 0.9999])
+def test_thresholds_at_the_last_key_that_is_counted(k, p):
+    """One token for each of the numbers from 4 down, among others far below:
+    thresholds a little before and behind the 512th of them."""
+    n, vocab = 16, 9000
+    g = torch.Generator().manual_seed(k)
+    x = torch.full((n, vocab), -30.0).bfloat16()
+    bits = torch.tensor(4.0).bfloat16().view(torch.int16) - \
+        torch.arange(700, dtype=torch.int16)
+    at = torch.rand(n, vocab, generator=g).argsort(1)[:, :700]
+    x.scatter_(1, at, bits.view(torch.bfloat16).expand(n, -1))
+    x[::4, at[0, 0]] = -torch.inf
+    u = torch.rand(n, generator=g)
+    of = lambda v: torch.full((n,), v, device=DEV)
+    got = ops.softmax_sample(x.to(DEV), of(0.8), of(k).int(), of(p),
+                             u.to(DEV)).tolist()
+    for i in range(n):
+        keep, cum, goal = draw(x[i], 0.8, k, p, float(u[i]))
+        a = got[i]
+        slack = 2e-5 * float(cum[-1])
+        assert bool(keep[a])
+        assert float(cum[a]) >= float(goal) - slack
+        assert a == 0 or float(cum[a - 1]) <= float(goal) + slack
+
+
+def test_largest_of_rows_that_are_not_usual():
+    """The first of equals, zeros of either sign; NaN of either sign, infinities
+    and rows of nothing else beside usual ones."""
+    vocab = 20000
+    x = torch.full((8, vocab), -3.0)
+    x[0, 700], x[0, 15000] = -0.0, 0.0
+    x[1, 700], x[1, 15000] = 0.0, -0.0
+    x[2, 5], x[2, 9], x[2, 19999] = torch.nan, 7.0, 7.0
+    x[3, 5], x[3, 9] = -torch.nan, 2.0
+    x[4, 12345] = torch.inf
+    x[5] = -torch.inf
+    x[6] = torch.nan
+    x[7] = -torch.inf
+    x[7, 19998] = -2e38
+    x = x.bfloat16().to(DEV)
+    zeros = torch.zeros(8, device=DEV)
+    got = ops.softmax_sample(x, zeros, zeros.int(), zeros + 1, zeros)
+    assert got.tolist() == [700, 700, 9, 9, 12345, 0, 0, 19998]
+    # and as a draw that leaves one token
+    got = ops.softmax_sample(x, zeros + 1, zeros.int() + 1, zeros + 1,
+                             zeros + 0.5)
+    assert got[2:5].tolist() == [9, 9, 12345] or got[2] in (9, 19999)
+    assert got[7] == 19998 and got[0] in (700, 15000)
