@@ -46,8 +46,9 @@ constexpr int PAD = 4;
 
 // FM: tiles of 16 rows of x; P: stages in flight. THIN: a workgroup has eight
 // weight rows, and the other eight of an operand are the next 64 columns of the
-// same ones, beside those of x: the rows of x are eight at most then.
-template <Columns C, bool NORM, int FM, int P, bool THIN>
+// same ones, beside those of x: the rows of x are eight at most then. X8: of its 16
+// rows of x only eight are loaded.
+template <Columns C, bool NORM, int FM, int P, bool THIN, bool X8>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       const bf16_t* __restrict__ w,
@@ -57,9 +58,10 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   // (normed x does not go through the ring)
   static_assert(!NORM || FM == 1);
   static_assert(!THIN || (FM == 1 && !NORM && !paired(C)));
-  constexpr int TILES = NORM ? 1 : 1 + FM;       // of a chunk of 32 columns
-  constexpr int STAGE = U * TILES * TILE;
-  constexpr int LOADS = U * TILES;
+  static_assert(!X8 || (FM == 1 && !NORM && !THIN));
+  // of a stage, 8 rows x 64 columns
+  constexpr int LOADS = NORM ? U : X8 ? U + 1 : U + U * FM;
+  constexpr int STAGE = LOADS * TILE;
   constexpr int RING = KW * P * STAGE;
   // one array: beside a second one the compiler guards every LDS read against
   // the direct loads in flight, and waits for them
@@ -108,6 +110,8 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                                : (unsigned)min(i * 8 + piece[h], end) * 16;
       load_to_lds<16>(wp[h] + at, to + h * TILE);
       if constexpr (!NORM) {
+        if constexpr (X8)
+          if (h == 1) continue;
         #pragma unroll
         for (int f = 0; f < FM; ++f)
           load_to_lds<16>(xp[f][h] + at, to + (2 + f * 2 + h) * TILE);
@@ -128,6 +132,8 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
         xf[u][f] = *reinterpret_cast<const short8*>(
             NORM ? s_x + min(lo, m - 1) * (k / 8 + 1) +
                        min(c0 + i * U + u, c1 - 1) * 4 + g
+            : X8 ? ring + s * STAGE + 2 * TILE + (lo & 7) * 8 +
+                       ((u * 4 + g) ^ (lo >> 1 & 3))
                  : t + (2 + f * 2) * TILE);
     }
     if (more) {
@@ -293,17 +299,19 @@ void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
                       long y_ld, bool gated, bool gelu, const Heads* heads,
                       const NormOf* norm, const AddTo* add,
                       const Undivided* of, hipStream_t stream) {
-  auto launch = [&](auto normed, auto tiles, auto stages, auto thin) {
-    constexpr bool N = decltype(normed)::value, T = decltype(thin)::value;
+  auto launch = [&](auto normed, auto tiles, auto stages, auto thin,
+                    auto eight) {
+    constexpr bool N = decltype(normed)::value, T = decltype(thin)::value,
+                   X = decltype(eight)::value;
     constexpr int F = decltype(tiles)::value, S = decltype(stages)::value;
-    auto kernel = rows_gemm_kernel<Columns::PLAIN, N, F, S, T>;
+    auto kernel = rows_gemm_kernel<Columns::PLAIN, N, F, S, T, X>;
     if constexpr (!T) {
-      if (heads) kernel = rows_gemm_kernel<Columns::HEADS, N, F, S, T>;
-      else if (gated) kernel = rows_gemm_kernel<Columns::GATED, N, F, S, T>;
+      if (heads) kernel = rows_gemm_kernel<Columns::HEADS, N, F, S, T, X>;
+      else if (gated) kernel = rows_gemm_kernel<Columns::GATED, N, F, S, T, X>;
     }
     if constexpr (!N) {
-      if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S, T>;
-      if (add) kernel = rows_gemm_kernel<Columns::ADDED, N, F, S, T>;
+      if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S, T, X>;
+      if (add) kernel = rows_gemm_kernel<Columns::ADDED, N, F, S, T, X>;
     }
     constexpr int ROWS = T ? 8 : 16;
     kernel<<<dim3((n + ROWS - 1) / ROWS), dim3(KW * WAVE), 0, stream>>>(
@@ -318,11 +326,12 @@ void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
   constexpr integral_constant<int, 2> two{};
   constexpr integral_constant<int, 3> three{};
   constexpr integral_constant<int, 4> four{};
-  if (norm) launch(yes, one, four, no);
+  if (norm) launch(yes, one, four, no, no);
   else if (rows_gemm_thin(m, n, k, gated || heads))
-    launch(no, one, four, yes);
-  else if (m <= 16) launch(no, one, four, no);
-  else if (m <= 32) launch(no, two, two, no);
-  else if (m <= 48) launch(no, three, two, no);
-  else launch(no, four, two, no);
+    launch(no, one, four, yes, no);
+  else if (m <= 8) launch(no, one, four, no, yes);
+  else if (m <= 16) launch(no, one, four, no, no);
+  else if (m <= 32) launch(no, two, two, no, no);
+  else if (m <= 48) launch(no, three, two, no, no);
+  else launch(no, four, two, no, no);
 }
