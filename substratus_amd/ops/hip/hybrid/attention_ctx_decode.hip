@@ -239,27 +239,28 @@ void attn_ctx_merge_kernel(AttnCtx<bf16_t> a, int splits,
                            const float* __restrict__ part_ml) {
   const int h = blockIdx.x;
   const long b = blockIdx.y, at = (b * a.heads + h) * splits;
-  const int c = threadIdx.x * VEC;
-  if (c >= a.vdim) return;
+  const int c = threadIdx.x * VEC, lane = threadIdx.x % WAVE;
   const bool sig = a.wbias != nullptr;          // sums only, no part_ml
-  float M = sig ? 0.f : NEG;
-  for (int s = 0; s < splits && !sig; ++s)
-    M = fmaxf(M, part_ml[(at + s) * 2]);
-  float L = sig ? 1.f : 0.f, o[VEC];
-  if (a.sink != nullptr) {
-    const float s = a.sink[h] * LOG2E;
-    M = fmaxf(M, s);
-    L = __builtin_amdgcn_exp2f(s - M);
+  // a lane has a share's maximum and sum
+  float m = NEG, l = 0.f, L = sig ? 1.f : 0.f, o[VEC];
+  if (lane < splits && !sig) {
+    m = part_ml[(at + lane) * 2];
+    l = part_ml[(at + lane) * 2 + 1];
   }
+  const float sink = a.sink != nullptr ? a.sink[h] * LOG2E : NEG;
+  const float M = sig ? 0.f : fmaxf(wave_max(m), sink);
+  const float w = sig ? 1.f : __builtin_amdgcn_exp2f(m - M);
+  if (!sig) L = wave_sum(l * w);
+  if (a.sink != nullptr) L += __builtin_amdgcn_exp2f(sink - M);
+  if (c >= a.vdim) return;
   #pragma unroll
   for (int j = 0; j < VEC; ++j) o[j] = 0.f;
-  #pragma unroll 4
+  #pragma unroll 8
   for (int s = 0; s < splits; ++s) {
-    const float f =
-        sig ? 1.f : __builtin_amdgcn_exp2f(part_ml[(at + s) * 2] - M);
+    const float f = __uint_as_float(
+        __builtin_amdgcn_readlane(__float_as_uint(w), s));
     float p[VEC];
     ldv<VEC>(part_o + (at + s) * a.vdim + c, p);
-    if (!sig) L += part_ml[(at + s) * 2 + 1] * f;
     #pragma unroll
     for (int j = 0; j < VEC; ++j) o[j] += p[j] * f;
   }

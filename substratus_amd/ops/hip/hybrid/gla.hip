@@ -69,6 +69,9 @@ void gla_recurrent_kernel(Gla<T> a, int lpr) {
         continue;
       }
       float z = a.a2b[c];
+      // (one by one, every term would wait for its loads: us, MI355X, of a rank of
+      // 16, 1 and 24 tokens, 8 heads of 128 x 256 10.3 16.3 -> 9.5 15.5)
+      #pragma unroll 8
       for (int r = 0; r < a.rank; ++r)
         z += a.a2[(long)c * a.rank + r] * ld1(x + a.a_off + r);
       s_a[d] = expf(log_sigmoid_f(z) * a.inv_tau);

@@ -15,6 +15,7 @@
 namespace {
 
 constexpr int BLOCK = 256;
+constexpr int EARLY = 2;          // numbers of a thread that are loaded early
 
 template <class T>
 __global__ __launch_bounds__(BLOCK)
@@ -29,6 +30,22 @@ void latent_prepare_kernel(T* __restrict__ buf, long ld, int heads, int dim,
   __shared__ float scratch[2][BLOCK / WAVE];
   const long row = blockIdx.x;
   T* q = buf + row * ld;
+  // a thread's first pairs of queries and its part of the latent are on their way
+  // while the angles are made
+  T qu[EARLY], qv[EARLY], lv[EARLY];
+  auto pair = [&](int i) {
+    return q + (long)(i / half) * (dim + rot_dim) + dim + i % half;
+  };
+  #pragma unroll
+  for (int e = 0; e < EARLY; ++e) {
+    const int i = threadIdx.x + e * BLOCK;
+    if (i < heads * half) {
+      qu[e] = pair(i)[0];
+      qv[e] = pair(i)[half];
+    }
+    if (c_at >= 0 && i < rank) lv[e] = q[c_at + i];
+  }
+  const int slot = c_at >= 0 ? slots[row] : 0;
   const double pos = positions[row];
   for (int i = threadIdx.x; i < half; i += BLOCK) {
     double t = pos * turns[i];
@@ -39,14 +56,20 @@ void latent_prepare_kernel(T* __restrict__ buf, long ld, int heads, int dim,
     s_cs[2 * i + 1] = s;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < heads * half; i += BLOCK) {
-    const int h = i / half, j = i % half;
-    T* p = q + (long)h * (dim + rot_dim) + dim + j;
-    const float u = ld1(p), v = ld1(p + half);
+  auto turn = [&](int i, float u, float v) {
+    T* p = pair(i);
+    const int j = i % half;
     const float c = s_cs[2 * j], s = s_cs[2 * j + 1];
     st1(p, u * c - v * s);
     st1(p + half, v * c + u * s);
+  };
+  #pragma unroll
+  for (int e = 0; e < EARLY; ++e) {
+    const int i = threadIdx.x + e * BLOCK;
+    if (i < heads * half) turn(i, ld1(&qu[e]), ld1(&qv[e]));
   }
+  for (int i = threadIdx.x + EARLY * BLOCK; i < heads * half; i += BLOCK)
+    turn(i, ld1(pair(i)), ld1(pair(i) + half));
   if (q_norm != nullptr) {
     float ss = 0.f;
     for (int i = threadIdx.x; i < q_rank; i += BLOCK) {
@@ -61,14 +84,25 @@ void latent_prepare_kernel(T* __restrict__ buf, long ld, int heads, int dim,
   if (c_at < 0) return;
   const T* lat = q + c_at;
   float ss = 0.f;
-  for (int i = threadIdx.x; i < rank; i += BLOCK) {
+  #pragma unroll
+  for (int e = 0; e < EARLY; ++e)
+    if (threadIdx.x + e * BLOCK < rank) {
+      const float f = ld1(&lv[e]);
+      ss += f * f;
+    }
+  for (int i = threadIdx.x + EARLY * BLOCK; i < rank; i += BLOCK) {
     const float f = ld1(lat + i);
     ss += f * f;
   }
   ss = block_sum<BLOCK / WAVE>(ss, scratch[0]);
   const float inv = 1.f / sqrtf(ss / (float)rank + eps);
-  T* out = cache + (long)slots[row] * (rank + rot_dim);
-  for (int i = threadIdx.x; i < rank; i += BLOCK)
+  T* out = cache + (long)slot * (rank + rot_dim);
+  #pragma unroll
+  for (int e = 0; e < EARLY; ++e) {
+    const int i = threadIdx.x + e * BLOCK;
+    if (i < rank) st1(out + i, ld1(&lv[e]) * inv * norm[i]);
+  }
+  for (int i = threadIdx.x + EARLY * BLOCK; i < rank; i += BLOCK)
     st1(out + i, ld1(lat + i) * inv * norm[i]);
   for (int j = threadIdx.x; j < rot_dim; j += BLOCK) {
     const float x = ld1(lat + rank + j);

@@ -17,7 +17,8 @@
 
 enum Source { EMBED, ROW, PICKED };
 
-template <class T, int VEC, int BLOCK, Source SRC>
+// RCAP: vectors per thread, at most; the launcher checks the row
+template <class T, int VEC, int BLOCK, Source SRC, int RCAP>
 __global__ __launch_bounds__(BLOCK)
 void stream_norm_kernel(T* __restrict__ y, float* __restrict__ x,
                         const T* __restrict__ delta,     // [rows, width]
@@ -33,7 +34,6 @@ void stream_norm_kernel(T* __restrict__ y, float* __restrict__ x,
                         const float* __restrict__ w_pre, int width, int vocab,
                         float off, float eps, float out_scale,
                         float mult) {
-  constexpr int RCAP = 8;   // vectors per thread; the launcher checks the row
   __shared__ float scratch[2][BLOCK / WAVE];
   const long row = blockIdx.x;
   const int nvec = width / VEC;
@@ -152,18 +152,27 @@ static void launch(T* y, float* x, const T* delta, const int* at,
                    int max_pos, const float* w_post, const float* w_pre,
                    long rows, int width, int vocab, float off, float eps,
                    float out_scale, float mult, hipStream_t stream) {
-  auto go = [&](auto vec, auto block) {
+  auto go = [&](auto vec, auto block, auto cap) {
     constexpr int V = decltype(vec)::value, B = decltype(block)::value;
-    stream_norm_kernel<T, V, B, SRC><<<dim3(rows), dim3(B), 0, stream>>>(
+    stream_norm_kernel<T, V, B, SRC, decltype(cap)::value>
+        <<<dim3(rows), dim3(B), 0, stream>>>(
         y, x, delta, at, wt, picks, table, tokens, pos, positions, max_pos,
         w_post, w_pre, width, vocab, off, eps, out_scale, mult);
   };
   using std::integral_constant;
   auto by_block = [&](auto vec) {
     const int nvec = width / decltype(vec)::value;
-    if (nvec <= 128) go(vec, integral_constant<int, 64>{});
-    else if (nvec <= 256 * 8) go(vec, integral_constant<int, 256>{});
-    else go(vec, integral_constant<int, 1024>{});
+    // no more registers than a row needs: us, MI355X, eight vectors of a thread
+    // -> 48 x 1024 2.9 -> 2.5, 48 x 2048 3.5 -> 3.0, 2488 x 2048 18.3 -> 17.2,
+    // 2488 x 1024 11.4 -> 10.1. (A wave a row, without barriers: 5.9, 17.5, 10.2.)
+    constexpr integral_constant<int, 256> threads{};
+    if (nvec <= 128)
+      go(vec, integral_constant<int, 64>{}, integral_constant<int, 2>{});
+    else if (nvec <= 256) go(vec, threads, integral_constant<int, 1>{});
+    else if (nvec <= 512) go(vec, threads, integral_constant<int, 2>{});
+    else if (nvec <= 1024) go(vec, threads, integral_constant<int, 4>{});
+    else if (nvec <= 2048) go(vec, threads, integral_constant<int, 8>{});
+    else go(vec, integral_constant<int, 1024>{}, integral_constant<int, 8>{});
   };
   if (width % 4 == 0) by_block(integral_constant<int, 4>{});
   else by_block(integral_constant<int, 1>{});
