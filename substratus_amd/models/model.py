@@ -46,6 +46,8 @@ def fused_norm_residual(deltas: tuple, h: torch.Tensor, norm: "NormParams",
     one HBM round trip per norm (profiles/serve_decode_r01_baseline.txt:
     unfused residual adds were ~2.2 ms of a 10.3 ms decode step). RMSNorm of
     one delta works in place on h."""
+    if isinstance(deltas, ops.Normed):
+        return deltas.rows, h
     got = None
     if bare(norm, NormParams):
         if norm.rms and len(deltas) == 1:
@@ -72,15 +74,15 @@ def normed_product(lin: nn.Module, deltas: tuple, h: torch.Tensor,
 
 
 def added_product(lin: nn.Module, x: torch.Tensor, h: torch.Tensor,
-                  norm: Optional["NormParams"]) -> tuple:
+                  norm: Optional["NormParams"], eps: float) -> tuple:
     """(h + lin(x), what of norm's rows is there already), or h and what is
     still to be added to it."""
-    added = getattr(type(lin), "added", None)
-    if added is not None and norm is not None and bare(norm, NormParams) \
-            and norm.rms:
-        got = added(lin, x, h, norm.weight)
-        if got is not None:
-            return got
+    if norm is not None and bare(norm, NormParams) and norm.rms:
+        for name, more in ("added", ()), ("added_norm", (eps,)):
+            how = getattr(type(lin), name, None)
+            got = None if how is None else how(lin, x, h, norm.weight, *more)
+            if got is not None:
+                return got
     return h, (lin(x),)
 
 
@@ -88,6 +90,8 @@ def scaled_product(lin: nn.Module, deltas: tuple, h: torch.Tensor,
                    norm: "NormParams", eps: float, **how):
     """(lin of norm(h + deltas), h + deltas) in one kernel, or None, and what
     is still to be added to h."""
+    if isinstance(deltas, ops.Normed):
+        return None, deltas
     if not isinstance(deltas, ops.Undivided):
         return normed_product(lin, deltas, h, norm, eps, **how), deltas
     scaled = getattr(type(lin), "scaled", None)
@@ -210,8 +214,8 @@ class Block(nn.Module):
         construction identical.
 
         h: the residual stream, deltas: what is still to be added to it, which
-        this block's first norm does, or ops.Undivided, what is there of that
-        norm already; the same is returned, the latter of the norm after."""
+        this block's first norm does, or ops.Undivided or ops.Normed, what is
+        there of that norm already; the same is returned, of the norm after."""
         cache = ops.Cache(positions, k_cache, v_cache, slots, self.rope_theta)
         got = None
         if not self.parallel_attn:
@@ -240,7 +244,8 @@ class Block(nn.Module):
             yield
             return h, (attn_out, self.w_down(up))
         silu = self.cfg.activation == "silu"
-        h, deltas = added_product(self.wo, a, h, self.norm2 if silu else None)
+        h, deltas = added_product(self.wo, a, h,
+                                  self.norm2 if silu else None, self.eps)
         yield
         got = None
         if silu:
@@ -252,7 +257,7 @@ class Block(nn.Module):
             y, h = fused_norm_residual(deltas, h, self.norm2, self.eps)
             up = self._mlp_up(y)
         yield
-        return added_product(self.w_down, up, h, after)
+        return added_product(self.w_down, up, h, after, self.eps)
 
     # -- prefill ------------------------------------------------------------
     def forward_prefill(self, h: torch.Tensor, deltas: tuple,

@@ -272,9 +272,10 @@ def _rows_gemm_pays(numel: int, n: int, k: int) -> bool:
 
 
 def _few_rows(x: torch.Tensor, weight: torch.Tensor,
-              bias: Optional[torch.Tensor], gated: bool):
+              bias: Optional[torch.Tensor], gated: bool,
+              summed: bool = False):
     """(x as rows, extension) where the product goes to rows_gemm.hip, or
-    None."""
+    None. summed: only where the norm that follows adds up its shares."""
     if not (x.is_cuda and weight.is_cuda and x.device == weight.device
             and x.dtype == weight.dtype == torch.bfloat16 and x.dim() >= 1
             and weight.dim() == 2 and x.shape[-1] == weight.shape[1]
@@ -285,10 +286,12 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
         return None
     # more of them, and larger matrices' rows by mid_gemm.hip, in the same call; a
     # compiler would hold the number of rows to a side of 256
-    if not (_rows_gemm_pays(x.numel(), n, k)
-            or not _compiling() and x.numel() <= 256 * k
-            and _load_ext() is not None
-            and _load_ext().few_rows_good(x.numel() // k, n, k, gated)):
+    if _rows_gemm_pays(x.numel(), n, k):
+        if summed:
+            return None
+    elif _compiling() or x.numel() > 256 * k or _load_ext() is None or not (
+            _load_ext().mid_norm_good(x.numel() // k, n, k) if summed else
+            _load_ext().few_rows_good(x.numel() // k, n, k, gated)):
         return None
     if bias is not None and not (bias.dtype == torch.bfloat16
                                  and bias.device == x.device
@@ -301,7 +304,7 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor,
         return None
     if x.dim() != 2:
         x = x.reshape(-1, k)
-    if not (ext.rows_gemm_ok(x.shape[0], n, k, gated)
+    if not ((summed or ext.rows_gemm_ok(x.shape[0], n, k, gated))
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and x.stride(1) == 1 and x.data_ptr() % 16 == 0
             and (x.stride(0) % 8 == 0 and x.stride(0) >= k
@@ -621,6 +624,26 @@ def linear_added(x: torch.Tensor, weight: torch.Tensor,
     few[1].rows_added(parts.rows, total, parts.squares, few[0], weight, bias,
                       h, norm)
     return total, parts
+
+
+class Normed(NamedTuple):
+    """An RMSNorm's rows."""
+    rows: torch.Tensor
+
+
+def linear_added_norm(x: torch.Tensor, weight: torch.Tensor,
+                      bias: Optional[torch.Tensor], h: torch.Tensor,
+                      norm: torch.Tensor, eps: float
+                      ) -> Optional[tuple[torch.Tensor, Normed]]:
+    """(h + F.linear, RMSNorm of that by the weight norm), or None: where
+    workgroups share the product's sums, which the norm adds up."""
+    few = _few_rows(x, weight, bias, False, True)
+    if few is None or x.dim() != 2 or x.device != h.device \
+            or not may_add(h, norm, x.shape[0], weight.shape[0]):
+        return None
+    total, rows = torch.empty_like(h), torch.empty_like(h)
+    few[1].mid_normed(rows, total, few[0], weight, bias, h, norm, eps)
+    return total, Normed(rows)
 
 
 def linear_scaled(x: Undivided, eps: float, weight: torch.Tensor,

@@ -549,6 +549,13 @@ bool rows_gemm_good(long m, long n, long k, bool paired) {
          rows_gemm_pays((int)m, (int)n, (int)k, paired);
 }
 
+// Whether a product's shares are best added up by the norm that follows it.
+bool mid_norm_good(long m, long n, long k) {
+  return mid_norm_takes(m, n, k) && mid_gemm_pays(m, n, k, false, true) &&
+         !rows_gemm_good(m, n, k, false) &&
+         !tile_gemm_good(m, n, k, k, k, false, false, false);
+}
+
 // Whether the library's product of these few rows would take longer.
 bool few_rows_good(long m, long n, long k, bool paired) {
   return rows_gemm_good(m, n, k, paired) || mid_gemm_good(m, n, k, paired);
@@ -605,7 +612,8 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                   c10::optional<torch::Tensor> bias, bool gated,
                   const Heads* heads, const NormOf* norm = nullptr,
                   bool gelu = false, const AddTo* add = nullptr,
-                  const Undivided* of = nullptr) {
+                  const Undivided* of = nullptr,
+                  const MidNorm* after = nullptr) {
   const c10::DeviceGuard guard(x.device());
   check_bf16(y, "y"); check_bf16(w, "w");
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 &&
@@ -616,11 +624,13 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
   const int cols = heads ? n - 2 * heads->hkv * heads->d : gated ? n / 2 : n;
   TORCH_CHECK(w.dim() == 2 && w.size(1) == k && y.size(0) == m &&
               y.numel() == (long)m * cols, "rows_gemm: shape mismatch");
-  const bool many = !(norm || add || of) && !rows_gemm_good(m, n, k, gated || heads) &&
-                    mid_gemm_good(m, n, k, gated || heads);
+  const bool many = after || !(norm || add || of) &&
+                                 !rows_gemm_good(m, n, k, gated || heads) &&
+                                 mid_gemm_good(m, n, k, gated || heads);
   TORCH_CHECK(many || rows_gemm_takes(m, n, k, gated || heads),
               "rows_gemm: unsupported shape ", m, "x", n, "x", k);
   TORCH_CHECK(m <= 16 || !(add || of), "rows_gemm: too many rows");
+  TORCH_CHECK(!after || mid_norm_takes(m, n, k), "rows_gemm: no shares");
   TORCH_CHECK(aligned16(x) && aligned16(w), "rows_gemm: misaligned operand");
   const bf16_t* bp = nullptr;
   if (bias.has_value()) {
@@ -635,7 +645,7 @@ void rows_gemm_to(torch::Tensor y, torch::Tensor x, torch::Tensor w,
       part = torch::empty({plan.shares(m, n)},
                           x.options().dtype(torch::kFloat));
     launch_mid_gemm({bf(y), bfc(x), bfc(w), bp, m, n, k, x.stride(0), cols},
-                    plan, heads, gated, gelu,
+                    plan, heads, gated, gelu, after,
                     plan.shares(m, n) ? part.data_ptr<float>() : nullptr,
                     stream());
   } else {
@@ -813,6 +823,24 @@ void rows_added(torch::Tensor y, torch::Tensor total, torch::Tensor squares,
       add_of(y, total, squares, h, weight,
              rows_added_parts(x.size(0), w.size(0), w.size(1)));
   rows_gemm_to(y, x, w, bias, false, nullptr, nullptr, false, &add);
+}
+
+// A product that is added to the residual stream, total = h + its rows, and the
+// RMSNorm of that, y.
+void mid_normed(torch::Tensor y, torch::Tensor total, torch::Tensor x,
+                torch::Tensor w, c10::optional<torch::Tensor> bias,
+                torch::Tensor h, torch::Tensor weight, double eps) {
+  const long n = weight.numel();
+  TORCH_CHECK(h.dim() == 2 && h.size(1) == n && y.sizes() == h.sizes() &&
+              w.dim() == 2 && w.size(0) == n, "normed: shapes");
+  check_rows(weight, n, "norm weight");
+  check_rows(h, h.numel(), "h"); check_rows(total, h.numel(), "total");
+  check_rows(y, h.numel(), "y");
+  if (bias) check_rows(*bias, n, "bias");
+  const MidNorm after{bfc(h), bfc(weight), const_cast<bf16_t*>(bfc(total)),
+                      (float)eps};
+  rows_gemm_to(y, x, w, bias, false, nullptr, nullptr, false, nullptr, nullptr,
+               &after);
 }
 
 void rows_scaled(torch::Tensor y, torch::Tensor x, torch::Tensor squares,
@@ -1138,6 +1166,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quant_heads", &quant_heads);
   m.def("rows_gemm_ok", &rows_gemm_ok);
   m.def("mid_gemm_good", &mid_gemm_good);
+  m.def("mid_norm_good", &mid_norm_good);
+  m.def("mid_normed", &mid_normed);
   m.def("few_rows_good", &few_rows_good);
   m.def("quant_rows", &quant_rows);
   m.def("quant_rows_ok", &quant_rows_ok);

@@ -24,8 +24,18 @@ struct MidPlan {
   }
 };
 
+// What follows the sums of shares, where each row's are one workgroup's: total = h +
+// the product's row, y the RMSNorm of that.
+struct MidNorm {
+  const bf16_t *h, *weight;
+  bf16_t* total;
+  float eps;
+};
+
 bool mid_gemm_takes(long m, long n, long k, bool paired);
 MidPlan mid_gemm_plan(long m, long n, long k);
-bool mid_gemm_pays(long m, long n, long k, bool paired);
+bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed = false);
+bool mid_norm_takes(long m, long n, long k);
 void launch_mid_gemm(const MidGemm& a, const MidPlan& plan, const Heads* heads,
-                     bool gated, bool gelu, float* part, hipStream_t stream);
+                     bool gated, bool gelu, const MidNorm* norm, float* part,
+                     hipStream_t stream);

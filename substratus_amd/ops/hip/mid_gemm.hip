@@ -237,6 +237,60 @@ void mid_sum_kernel(MidGemm a, Heads heads, const float* __restrict__ part,
   finish<C>(a, heads, r, t, c, u, v);
 }
 
+// The same, of a whole row to a workgroup, which adds them to the residual stream
+// and makes the norm that follows of it: bound by a launch and its first loads, and
+// a norm of its own has both again, besides the row's way through memory. The row
+// is rounded as the product and the norm round it.
+template <int BLOCK, int QUADS>
+__global__ __launch_bounds__(BLOCK)
+void mid_norm_kernel(MidGemm a, MidNorm norm, const float* __restrict__ part,
+                     int splits) {
+  __shared__ float scratch[BLOCK / WAVE];
+  const int r = blockIdx.x, wide = (a.n + 15) / 16 * 16;
+  const long step = (long)a.m * wide, row = (long)r * a.n;
+  float4v keep[QUADS], w[QUADS];
+  float squares = 0.f;
+  auto quad = [](const bf16_t* p) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    const float2 x = unpack_bf16x2(u.x), y = unpack_bf16x2(u.y);
+    return (float4v){x.x, x.y, y.x, y.y};
+  };
+  #pragma unroll
+  for (int q = 0; q < QUADS; ++q) {
+    const int c = (q * BLOCK + threadIdx.x) * 4;
+    if (c >= a.n) break;
+    const float4v h = quad(norm.h + row + c);
+    w[q] = quad(norm.weight + c);
+    const float* p = part + (long)r * wide + c;
+    float4v u = {0.f, 0.f, 0.f, 0.f};
+    #pragma unroll 4
+    for (int s = 0; s < splits; ++s)
+      u += *reinterpret_cast<const float4v*>(p + s * step);
+    if (a.bias != nullptr) u += quad(a.bias + c);
+    #pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      u[e] = h[e] + bf2f(f2bf(u[e]));
+      squares += u[e] * u[e];
+    }
+    const uint2 to = make_uint2(pack_bf16x2(u[0], u[1]),
+                                pack_bf16x2(u[2], u[3]));
+    *reinterpret_cast<uint2*>(norm.total + row + c) = to;
+    const float2 x = unpack_bf16x2(to.x), y = unpack_bf16x2(to.y);
+    keep[q] = (float4v){x.x, x.y, y.x, y.y};
+  }
+  const float inv = rsqrtf(
+      block_sum<BLOCK / WAVE>(squares, scratch) / (float)a.n + norm.eps);
+  #pragma unroll
+  for (int q = 0; q < QUADS; ++q) {
+    const int c = (q * BLOCK + threadIdx.x) * 4;
+    if (c >= a.n) break;
+    const float4v v = keep[q];
+    *reinterpret_cast<uint2*>(a.y + row + c) = make_uint2(
+        pack_bf16x2(v[0] * inv * w[q][0], v[1] * inv * w[q][1]),
+        pack_bf16x2(v[2] * inv * w[q][2], v[3] * inv * w[q][3]));
+  }
+}
+
 }  // namespace
 
 bool mid_gemm_takes(long m, long n, long k, bool paired) {
@@ -290,7 +344,14 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 //   64 x 4096 x 11008  34 28 (39 27)     208 x 6144 x 4096    27  36 (24 37)
 //   64 x 4096 x 4096   15 13 (16 16)     224 x 5120 x 13824  111  62 (90 74)
 //   96 x 768 x 3072   7.8 10 (10 11)      80 x 10240 x 8192   75  42 (48 43)
-bool mid_gemm_pays(long m, long n, long k, bool paired) {
+// A norm that adds up the shares saves a launch, but for the steps above and short
+// products of few columns. Of 5578 products of those widths, each with the residual's
+// sum and its norm, as they were -> now: 1.07 times as fast on average (2048 to 14336
+// columns' inner sizes and 4096 rows 1.05 to 1.17 where the product was this one's,
+// 1.1 to 1.66 where it was the library's), 20 slower by more than 3 %, by 17 at most.
+// 64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
+// 128 x 5120 x 5120 35.7 -> 25.3, 256 x 4096 x 11008 47.2 -> 43.8.
+bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
   if (m <= 16 || m > 256 || k < (paired ? 1024 : 3072) ||
       (m > 96 && n > 12288))
     return false;
@@ -298,20 +359,28 @@ bool mid_gemm_pays(long m, long n, long k, bool paired) {
   const double inner = m > 128 ? 1.5e-3 + 1.7e-3 * few : .6e-3 + .6e-3 * few;
   const double work = n * k * 2 / 1e7 + k * inner + m * n * k * 2 / 2e9;
   const double library = (m > 128 ? 1. : 6.6) + work * (k % 256 ? 1.45 : 1.);
-  const double pass = !paired ? 0. : n >= 4096 && k >= 2048 ? 2. : 1.;
   const bool longer = m > 32 && m < 256 && n <= 10240 &&
                       k >= (m > 128 ? 12288 : 8192);
   const MidPlan plan = mid_gemm_plan(m, n, k);
   const long share = ((k + STEP - 1) / STEP + plan.splits - 1) / plan.splits;
   const bool in_step = m <= 128 && k % 8192 == 0 && share % 32 == 0;
+  const bool saved = normed && plan.splits > 1 && !in_step &&
+                     (m <= 64 || n >= 1536 || k > 4096);
+  const double pass = saved ? 3.5
+                      : !paired ? 0. : n >= 4096 && k >= 2048 ? 2. : 1.;
   const double ours = plan.us * (in_step ? 1.25 : 1.) -
                       (plan.splits > 1 ? 0. : 2.);
   return ours < library * (longer ? 1.2 : 1.) + pass;
 }
 
+bool mid_norm_takes(long m, long n, long k) {
+  return mid_gemm_takes(m, n, k, false) && n % 4 == 0 && n <= 16384 &&
+         mid_gemm_plan(m, n, k).splits > 1;
+}
+
 void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
-                     const Heads* heads, bool gated, bool gelu, float* part,
-                     hipStream_t stream) {
+                     const Heads* heads, bool gated, bool gelu,
+                     const MidNorm* norm, float* part, hipStream_t stream) {
   MidGemm a = given;
   a.blocks = (a.m + plan.rows - 1) / plan.rows;
   a.quads = a.n % 4 == 0 && a.y_ld % 4 == 0 &&
@@ -340,7 +409,14 @@ void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
   else if (plan.rows == 64) wide(integral_constant<int, 4>{});
   else if (plan.rows == 96) wide(integral_constant<int, 6>{});
   else wide(integral_constant<int, 8>{});
-  if (plan.splits > 1) {
+  if (norm) {
+    auto kernel = a.n <= 2048 ? mid_norm_kernel<512, 1>
+                  : a.n <= 4096 ? mid_norm_kernel<1024, 1>
+                  : a.n <= 8192 ? mid_norm_kernel<1024, 2>
+                                : mid_norm_kernel<1024, 4>;
+    const dim3 block(a.n <= 2048 ? 512 : 1024);
+    kernel<<<dim3(a.m), block, 0, stream>>>(a, *norm, part, plan.splits);
+  } else if (plan.splits > 1) {
     auto sum = heads ? mid_sum_kernel<Columns::HEADS>
                : gated ? mid_sum_kernel<Columns::GATED>
                : gelu ? mid_sum_kernel<Columns::GELU>

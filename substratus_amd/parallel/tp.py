@@ -93,6 +93,13 @@ class Linear(nn.Module):
         return ops.linear_added(x, self.weight, self.bias, h, norm) \
             if bare(self, Linear) else None
 
+    def added_norm(self, x: torch.Tensor, h: torch.Tensor,
+                   norm: torch.Tensor, eps: float):
+        """(h + the outputs, RMSNorm of that) by the kernels of the product,
+        or None."""
+        return ops.linear_added_norm(x, self.weight, self.bias, h, norm, eps) \
+            if bare(self, Linear) else None
+
     def scaled(self, x: ops.Undivided, eps: float, gated: bool = False,
                cache: Optional[ops.Cache] = None) -> Optional[torch.Tensor]:
         """The outputs for rows that are still to be divided, gated or appended
@@ -140,5 +147,11 @@ class RowParallelLinear(Linear):
     def added(self, x: torch.Tensor, h: torch.Tensor, norm: torch.Tensor):
         # (a bias would be rounded with the sum and not after it)
         return ops.linear_added(x, self.weight, None, h, norm) \
+            if self.tp_world == 1 and self.bias is None \
+            and bare(self, RowParallelLinear) else None
+
+    def added_norm(self, x: torch.Tensor, h: torch.Tensor,
+                   norm: torch.Tensor, eps: float):
+        return ops.linear_added_norm(x, self.weight, None, h, norm, eps) \
             if self.tp_world == 1 and self.bias is None \
             and bare(self, RowParallelLinear) else None
