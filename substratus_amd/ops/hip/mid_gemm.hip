@@ -10,17 +10,16 @@
 // (of one workgroup that has most of LDS, or of two). A load takes 8 rows x 128
 // bytes: with 16 rows x 64 bytes every cache line came twice, 128 x 4544 x 18176
 // in 64 us instead of 51. Four waves that shared the inner dimension instead,
-// without barriers, were no faster at either; nor are more stages in flight, or
-// operands read half a stage ahead (a CU takes in some
-// 38 GB/s as it is).
+// without barriers, were no faster at either; nor are more stages in flight,
+// operands read half a stage ahead, or 256 columns a workgroup.
 //
 // us on a MI355X, from the library's product to this one:
 //   rows     n x k: 4096 x 4096    4096 x 11008   4544 x 18176   8192 x 8192
-//   17              13.6 -> 11.7    32.5 -> 22.6   117 -> 35.8   31.4 -> 34.6
-//   64              15.1 -> 13.2    34.8 -> 25.9   156 -> 40.9   33.9 -> 36.1
-//   128             24.5 -> 17.0    59.9 -> 31.9   151 -> 51.1   49.1 -> 44.8
-//   192             33.1 -> 20.7    81.4 -> 39.6   123 -> 69.4   64.7 -> 53.7
-//   256             23.0 -> 24.0    50.2 -> 44.1   143 -> 77.6   77.2 -> 60.7
+//   17              13.1 -> 11.8    30.6 -> 21.3   117 -> 35.3   30.2 -> 29.9
+//   64              14.9 -> 13.3    34.2 -> 25.6   155 -> 40.9   33.2 -> 32.1
+//   128             24.3 -> 19.2    59.9 -> 31.1   150 -> 46.8   48.0 -> 39.0
+//   192             32.6 -> 21.4    81.1 -> 39.0   124 -> 70.9   64.8 -> 54.1
+//   256             22.4 -> 23.8    49.6 -> 43.8   142 -> 77.5   78.0 -> 60.2
 #include "mid_gemm.h"
 
 #include <algorithm>
@@ -96,8 +95,9 @@ DEV_INLINE void finish(const MidGemm& a, const Heads& heads, int r, int t, int c
   }
 }
 
-// F: tiles of 16 rows of x, N: of weights; P stages of 64 columns of both in LDS
-template <Columns C, int F, int N, int P>
+// F: tiles of 16 rows of x, N: of weights; P stages of 64 columns of both in LDS.
+// SPREAD: workgroups begin at different places of their shares
+template <Columns C, int F, int N, int P, bool SPREAD>
 __global__ __launch_bounds__(WAVES * WAVE, (N + F) * 2 * P <= 80 ? 2 : 1)
 void mid_gemm_kernel(MidGemm a, Heads heads, float* __restrict__ part) {
   constexpr int STAGE = (N + F) * TILE;
@@ -121,7 +121,13 @@ void mid_gemm_kernel(MidGemm a, Heads heads, float* __restrict__ part) {
   const int all = (a.k + STEP - 1) / STEP;
   const int i0 = (int)((long)all * blockIdx.y / gridDim.y);
   const int steps = (int)((long)all * (blockIdx.y + 1) / gridDim.y) - i0;
-
+  // Those of an XCD stay close to each other, so that rows of x come to its cache
+  // once (128 x 8192 x 28672 110 us, spread over the whole share 137).
+  const int first = SPREAD && steps > 0
+      ? (ct % 8 * 4 + ct / 8 * (a.m > 64 ? 1 : 3)) % steps : 0;
+  auto in_share = [&](int i) {
+    return SPREAD && i + first >= steps ? i + first - steps : i + first;
+  };
   // A load is 8 rows x 128 bytes, whole cache lines (64 of 16 rows each: lines
   // came twice, 35 % slower). A row's pieces are permuted by the row against
   // bank conflicts.
@@ -142,9 +148,10 @@ void mid_gemm_kernel(MidGemm a, Heads heads, float* __restrict__ part) {
   const int over = a.k / 8 - i0 * 8 - 1;         // a row's last piece from here
   auto load = [&](int i) {
     uint4* to = s_all + i % P * STAGE + wave * LOADS * 64;
+    const int at = in_share(i) * 8;
     #pragma unroll
     for (int l = 0; l < LOADS; ++l)
-      load_to_lds<16>(from[l] + min(i * 8 + piece[l], over) * 16, to + l * 64);
+      load_to_lds<16>(from[l] + min(at + piece[l], over) * 16, to + l * 64);
   };
   float4v acc[NW][FW];
   #pragma unroll
@@ -153,6 +160,7 @@ void mid_gemm_kernel(MidGemm a, Heads heads, float* __restrict__ part) {
     for (int f = 0; f < FW; ++f) acc[j][f] = (float4v){0.f, 0.f, 0.f, 0.f};
   auto use = [&](int i) {
     const uint4* s = s_all + i % P * STAGE + lo * 8;
+    const bool half = (i0 + in_share(i)) * STEP + STEP > a.k;
     #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int at = (c * 4 + g) ^ (lo >> 1);
@@ -164,7 +172,7 @@ void mid_gemm_kernel(MidGemm a, Heads heads, float* __restrict__ part) {
       for (int f = 0; f < FW; ++f)
         xf[f] = *reinterpret_cast<const short8*>(
             s + (N + wm * FW + f) * TILE + at);
-      if (c == 1 && (i0 + i) * STEP + STEP > a.k) break;   // half a step's
+      if (c == 1 && half) break;
       #pragma unroll
       for (int j = 0; j < NW; ++j)
         #pragma unroll
@@ -329,11 +337,13 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // begin on lines of 512 bytes. A paired product saves a launch and a pass. Where
 // matrices are wide and rows many the library has tiles for the chip, and sums of
 // few numbers cannot be shared. Long sums of more than 32 rows take it a fifth
-// longer at least, but for 256, which are whole tiles. Ours take a quarter longer
-// where shares begin on whole 4 KB of rows of a multiple of 16 KB, as then all CUs
-// read the same channels at a time (8192 x 8192 in four shares 37 to 45 us; 128 rows
-// of 8208 x 8192 in three 44, and the library 54); what nothing is shared of begins
-// and ends 2 us sooner (55 x 11264 x 2048, gated: 16 us, the library 21).
+// longer at least, but for 256, which are whole tiles. Of rows of a multiple of 4 KB
+// it takes a fifth longer in wide paired products, as its CUs all read the same of the
+// memory's channels (64 x 28672 x 4096 54.4 us, and 45.9 here; 32 x 22016 x 4096 46.1,
+// and 37.0; 64 x 57344 x 8192 182 and 176). Up to 96 rows whose shares begin on whole
+// 4 KB of rows of a multiple of 16 KB stay with it: of 8192 x 8192 32 to 40 us either
+// way, of 128 rows 48, and 39 here. What nothing is shared of begins and ends 2 us
+// sooner (55 x 11264 x 2048, gated: 16 us, the library 21).
 // Of 7795 products (17 to 256 rows, 250 to 20000 x 512 to 32768, an eighth of them
 // sizes of models, a quarter paired) this takes 0.75 of the library's time on
 // average, where 0.72 is the least of either; 30 take longer than the library's, by
@@ -344,8 +354,8 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 //   64 x 4096 x 11008  34 28 (39 27)     208 x 6144 x 4096    27  36 (24 37)
 //   64 x 4096 x 4096   15 13 (16 16)     224 x 5120 x 13824  111  62 (90 74)
 //   96 x 768 x 3072   7.8 10 (10 11)      80 x 10240 x 8192   75  42 (48 43)
-// A norm that adds up the shares saves a launch, but for the steps above and short
-// products of few columns. Of 5578 products of those widths, each with the residual's
+// A norm that adds up the shares saves a launch, but for short products of few
+// columns. Of 5578 products of those widths, each with the residual's
 // sum and its norm, as they were -> now: 1.07 times as fast on average (2048 to 14336
 // columns' inner sizes and 4096 rows 1.05 to 1.17 where the product was this one's,
 // 1.1 to 1.66 where it was the library's), 20 slower by more than 3 %, by 17 at most.
@@ -358,13 +368,15 @@ bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
   const double few = std::min(1., n / 4500.);
   const double inner = m > 128 ? 1.5e-3 + 1.7e-3 * few : .6e-3 + .6e-3 * few;
   const double work = n * k * 2 / 1e7 + k * inner + m * n * k * 2 / 2e9;
-  const double library = (m > 128 ? 1. : 6.6) + work * (k % 256 ? 1.45 : 1.);
+  const double library = (m > 128 ? 1. : 6.6) + work *
+      (k % 256 ? 1.45 : paired && k % 2048 == 0 ? 1.2 : 1.);
   const bool longer = m > 32 && m < 256 && n <= 10240 &&
                       k >= (m > 128 ? 12288 : 8192);
   const MidPlan plan = mid_gemm_plan(m, n, k);
   const long share = ((k + STEP - 1) / STEP + plan.splits - 1) / plan.splits;
-  const bool in_step = m <= 128 && k % 8192 == 0 && share % 32 == 0;
-  const bool saved = normed && plan.splits > 1 && !in_step &&
+  const bool in_step = !(paired || normed) && m <= 96 && k % 8192 == 0 &&
+                       share % 32 == 0;
+  const bool saved = normed && plan.splits > 1 &&
                      (m <= 64 || n >= 1536 || k > 4096);
   const double pass = saved ? 3.5
                       : !paired ? 0. : n >= 4096 && k >= 2048 ? 2. : 1.;
@@ -376,6 +388,20 @@ bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
 bool mid_norm_takes(long m, long n, long k) {
   return mid_gemm_takes(m, n, k, false) && n % 4 == 0 && n <= 16384 &&
          mid_gemm_plan(m, n, k).splits > 1;
+}
+
+// Whether workgroups begin at different places of the inner dimension. Where they all
+// read the same columns, and rows are a multiple of a large power of two of bytes, or
+// nearly, they meet at few of the memory's channels. us, from the start -> spread:
+// 64 x 8192 x 8192 40.8 -> 31.7, 64 x 28672 x 4096, gated, 53.2 -> 45.4, 64 x 57344 x
+// 8192, gated, 181 -> 176, 64 x 4096 x 14336 34.6 -> 30.1, 64 x 4096 x 11008 27.6 ->
+// 25.9, 128 x 8192 x 8192 45.2 -> 38.5, 128 x 22016 x 4096, gated, 56.5 -> 53.3. Rows
+// of other lengths, and many long ones, of which x is no longer read by all at the
+// same time, lose 2 to 6 %: 64 x 6656 x 17920 55.5 -> 57.1, 224 x 4544 x 18176 77.4 ->
+// 82.7, 160 x 8192 x 28672 158 -> 166.
+static bool mid_gemm_spreads(int m, int k) {
+  return k % 2048 == 0 && (m <= 64 || k <= 8192) ||
+         k % 256 == 0 && m <= 64 && k <= 12288;
 }
 
 void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
@@ -390,10 +416,15 @@ void launch_mid_gemm(const MidGemm& given, const MidPlan& plan,
   auto launch = [&](auto f, auto n, auto p) {
     constexpr int F = decltype(f)::value, N = decltype(n)::value,
                   P = decltype(p)::value;
-    auto kernel = heads ? mid_gemm_kernel<Columns::HEADS, F, N, P>
-                  : gated ? mid_gemm_kernel<Columns::GATED, F, N, P>
-                  : gelu ? mid_gemm_kernel<Columns::GELU, F, N, P>
-                          : mid_gemm_kernel<Columns::PLAIN, F, N, P>;
+    auto pick = [&](auto spread) {
+      constexpr bool S = decltype(spread)::value;
+      return heads ? mid_gemm_kernel<Columns::HEADS, F, N, P, S>
+             : gated ? mid_gemm_kernel<Columns::GATED, F, N, P, S>
+             : gelu ? mid_gemm_kernel<Columns::GELU, F, N, P, S>
+                    : mid_gemm_kernel<Columns::PLAIN, F, N, P, S>;
+    };
+    auto kernel = mid_gemm_spreads(a.m, a.k) ? pick(std::true_type{})
+                                             : pick(std::false_type{});
     kernel<<<dim3((tiles + N - 1) / N * a.blocks, plan.splits), WAVES * WAVE,
              0, stream>>>(a, h, part);
   };
