@@ -354,6 +354,13 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 //   64 x 4096 x 11008  34 28 (39 27)     208 x 6144 x 4096    27  36 (24 37)
 //   64 x 4096 x 4096   15 13 (16 16)     224 x 5120 x 13824  111  62 (90 74)
 //   96 x 768 x 3072   7.8 10 (10 11)      80 x 10240 x 8192   75  42 (48 43)
+// Of such rows the widest are taken by up to 64 in any case, up to inner sizes where
+// memory is all that either waits for (20 x 44032 x 16384 260 us, and 267 here; 32 x
+// 57344 x 8192, gated, 171 and 176): 20 x 32000 x 2048 33.4 us, and 26.1 here, 64 x
+// 32000 x 4096 61.6 and 50.7, 64 x 128256 x 4096 210 and 191, 48 x 29760 x 12288 174
+// and 130, 20 x 28672 x 4096, gated, 56.7 and 47.3. More rows lose what there is to
+// gain (96 x 48000 x 6144 146 and 143), or are two blocks, which read the weights
+// twice (130 x 32000 x 4096 65 and 93).
 // A norm that adds up the shares saves a launch, but for short products of few
 // columns. Of 5578 products of those widths, each with the residual's
 // sum and its norm, as they were -> now: 1.07 times as fast on average (2048 to 14336
@@ -362,9 +369,12 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // 64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
 // 128 x 5120 x 5120 35.7 -> 25.3, 256 x 4096 x 11008 47.2 -> 43.8.
 bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
-  if (m <= 16 || m > 256 || k < (paired ? 1024 : 3072) ||
+  if (m <= 16 || m > 256 || k < (paired ? 1024 : 2048) ||
       (m > 96 && n > 12288))
     return false;
+  if (m <= 64 && n >= 16000 && k % 2048 == 0 && k <= (paired ? 6144 : 12288))
+    return true;
+  if (!paired && k < 3072) return false;
   const double few = std::min(1., n / 4500.);
   const double inner = m > 128 ? 1.5e-3 + 1.7e-3 * few : .6e-3 + .6e-3 * few;
   const double work = n * k * 2 / 1e7 + k * inner + m * n * k * 2 / 2e9;
