@@ -239,7 +239,10 @@ void attn_ctx_merge_kernel(AttnCtx<bf16_t> a, int splits,
                            const float* __restrict__ part_ml) {
   const int h = blockIdx.x;
   const long b = blockIdx.y, at = (b * a.heads + h) * splits;
-  const int c = threadIdx.x * VEC, lane = threadIdx.x % WAVE;
+  // all lanes stay to the end, as they are read from
+  const int lane = threadIdx.x % WAVE;
+  const bool there = threadIdx.x * VEC < a.vdim;
+  const int c = there ? threadIdx.x * VEC : 0;
   const bool sig = a.wbias != nullptr;          // sums only, no part_ml
   // a lane has a share's maximum and sum
   float m = NEG, l = 0.f, L = sig ? 1.f : 0.f, o[VEC];
@@ -252,7 +255,6 @@ void attn_ctx_merge_kernel(AttnCtx<bf16_t> a, int splits,
   const float w = sig ? 1.f : __builtin_amdgcn_exp2f(m - M);
   if (!sig) L = wave_sum(l * w);
   if (a.sink != nullptr) L += __builtin_amdgcn_exp2f(sink - M);
-  if (c >= a.vdim) return;
   #pragma unroll
   for (int j = 0; j < VEC; ++j) o[j] = 0.f;
   #pragma unroll 8
@@ -268,6 +270,7 @@ void attn_ctx_merge_kernel(AttnCtx<bf16_t> a, int splits,
   if (a.gate != nullptr) f *= sigmoid_f(bf2f(a.gate[b * a.g_ld + h]));
   #pragma unroll
   for (int j = 0; j < VEC; ++j) o[j] *= f;
+  if (!there) return;
   bf16_t* out = a.out + b * a.out_ld + (long)h * a.vdim + c;
   if (a.quads) {
     stv<VEC>(out, o);
