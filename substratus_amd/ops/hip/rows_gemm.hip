@@ -17,11 +17,14 @@
 // meet no bank conflicts.
 //
 // us on a MI355X, from the library's product to this one:
-//   1 x 6144 x 2048    12.3 -> 7.1     8 x 12288 x 4096   28.2 -> 19.8
-//   1 x 2048 x 2048    10.8 -> 4.2     8 x 4096 x 4096    15.4 -> 8.0
-//   1 x 11264 x 2048   16.1 -> 10.2    8 x 22016 x 4096   52.8 -> 35.9
-//   1 x 2048 x 5632    11.2 -> 7.4     8 x 4096 x 11008   37.7 -> 19.5
-// (5.0 to 5.4 TB/s where the matrix is large). 8 and 16 waves, or 32 rows of
+//   1 x 6144 x 2048    12.3 -> 7.1     8 x 12288 x 4096   28.2 -> 18.5
+//   1 x 2048 x 2048    10.8 -> 3.6     8 x 4096 x 4096    15.4 -> 8.0
+//   1 x 11264 x 2048   16.1 -> 9.7     8 x 22016 x 4096   52.8 -> 33.1
+//   1 x 2048 x 5632    11.2 -> 6.2     8 x 4096 x 11008   37.7 -> 19.2
+// (5.0 to 5.8 TB/s where the matrix is large). Workgroups that begin at different
+// columns, as those of mid_gemm.hip, have the last in 17.0, 8 x 8192 x 8192 in 24.7
+// instead of 27.8, and the others as they are; but the arithmetic of their addresses
+// costs more than that in a decode step (llama2-7b, 8 layers, 8 rows: 827 -> 837 us). 8 and 16 waves, or 32 rows of
 // weights, are slower: fewer workgroups per CU.
 //
 // With 17 to 64 rows a wave has two to four operand tiles of x, and every
