@@ -20,11 +20,8 @@
 //   1 x 6144 x 2048    12.3 -> 7.1     8 x 12288 x 4096   28.2 -> 18.5
 //   1 x 2048 x 2048    10.8 -> 3.6     8 x 4096 x 4096    15.4 -> 8.0
 //   1 x 11264 x 2048   16.1 -> 9.7     8 x 22016 x 4096   52.8 -> 33.1
-//   1 x 2048 x 5632    11.2 -> 6.2     8 x 4096 x 11008   37.7 -> 19.2
-// (5.0 to 5.8 TB/s where the matrix is large). Workgroups that begin at different
-// columns, as those of mid_gemm.hip, have the last in 17.0, 8 x 8192 x 8192 in 24.7
-// instead of 27.8, and the others as they are; but the arithmetic of their addresses
-// costs more than that in a decode step (llama2-7b, 8 layers, 8 rows: 827 -> 837 us). 8 and 16 waves, or 32 rows of
+//   1 x 2048 x 5632    11.2 -> 6.2     8 x 4096 x 11008   37.7 -> 17.4
+// (5.0 to 5.8 TB/s where the matrix is large). 8 and 16 waves, or 32 rows of
 // weights, are slower: fewer workgroups per CU.
 //
 // With 17 to 64 rows a wave has two to four operand tiles of x, and every
@@ -50,8 +47,10 @@ constexpr int PAD = 4;
 // FM: tiles of 16 rows of x; P: stages in flight. THIN: a workgroup has eight
 // weight rows, and the other eight of an operand are the next 64 columns of the
 // same ones, beside those of x: the rows of x are eight at most then. X8: of its 16
-// rows of x only eight are loaded.
-template <Columns C, bool NORM, int FM, int P, bool THIN, bool X8>
+// rows of x only eight are loaded. SPREAD: workgroups begin at different places of
+// their shares.
+template <Columns C, bool NORM, int FM, int P, bool THIN, bool X8,
+          bool SPREAD = false>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                       const bf16_t* __restrict__ w,
@@ -86,6 +85,11 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const int c1 = min(lines * (wave + 1) / KW * CHUNKS, chunks);
   const int steps = (c1 - c0 + CHUNKS - 1) / CHUNKS;
   uint4* ring = s_all + wave * P * STAGE;
+  const int begin = SPREAD && steps > 0
+      ? (int)(blockIdx.x * 5 % (unsigned)steps) : 0;
+  auto in_share = [&](int i) {
+    return SPREAD && i + begin >= steps ? i + begin - steps : i + begin;
+  };
 
   // a load is 8 rows x 128 bytes: of a tile's row lane / 8, or eight later
   const int row = lane >> 3;
@@ -106,6 +110,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const int end = (c1 - c0) * 4 - 1;             // the share's last piece
   auto load = [&](int s, int i) {
     uint4* to = ring + s * STAGE;
+    i = in_share(i);
     #pragma unroll
     for (int h = 0; h < 2; ++h) {
       // a stage may be half of one: then its last piece comes again
@@ -125,6 +130,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   #pragma unroll
   for (int f = 0; f < FM; ++f) acc[f] = (float4v){0.f, 0.f, 0.f, 0.f};
   auto step = [&](int s, int i, bool more) {
+    const int at = in_share(i);
     short8 wf[U], xf[U][FM];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -134,7 +140,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       for (int f = 0; f < FM; ++f)
         xf[u][f] = *reinterpret_cast<const short8*>(
             NORM ? s_x + min(lo, m - 1) * (k / 8 + 1) +
-                       min(c0 + i * U + u, c1 - 1) * 4 + g
+                       min(c0 + at * U + u, c1 - 1) * 4 + g
             : X8 ? ring + s * STAGE + 2 * TILE + (lo & 7) * 8 +
                        ((u * 4 + g) ^ (lo >> 1 & 3))
                  : t + (2 + f * 2) * TILE);
@@ -145,7 +151,7 @@ void rows_gemm_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     }
     #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (THIN || c0 + i * U + u < c1) {
+      if (THIN || c0 + at * U + u < c1) {
         #pragma unroll
         for (int f = 0; f < FM; ++f)
           acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -295,6 +301,17 @@ bool rows_gemm_thin(int m, int n, int k, bool paired) {
          k % 128 == 0;
 }
 
+// Whether workgroups begin at different columns: all at the same they meet at few of
+// the memory's channels where rows are a multiple of 512 bytes. us: 8 x 4096 x 11008
+// 19.3 -> 17.4, 8 x 4096 x 8192 16.2 -> 13.7, 8 x 8192 x 8192 28.3 -> 25.4, 8 x 32000 x
+// 8192 95.9 -> 92.6; 1 x 9216 x 8448 30.8 -> 31.0. Longer rows are as fast or 1 to 2 %
+// slower (8 x 4096 x 14336 21.9 -> 22.3), and shorter ones gain less than the
+// arithmetic of the loads' addresses costs (a step of 8 rows and 8 layers of llama2-7b:
+// with all products like this 827 -> 837, with these alone 829 -> 816).
+static bool rows_gemm_spreads(int n, int k) {
+  return n >= 4096 && k >= 8192 && k < 12288 && k % 256 == 0;
+}
+
 // heads: null, or what is done with the columns instead of storing them (n is
 // a multiple of 16 then, like gated's)
 void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
@@ -316,6 +333,10 @@ void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
       if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S, T, X>;
       if (add) kernel = rows_gemm_kernel<Columns::ADDED, N, F, S, T, X>;
     }
+    if constexpr (!N && !T && F == 1)
+      if (!(heads || gated || gelu) && rows_gemm_spreads(n, k))
+        kernel = add ? rows_gemm_kernel<Columns::ADDED, N, F, S, T, X, true>
+                     : rows_gemm_kernel<Columns::PLAIN, N, F, S, T, X, true>;
     constexpr int ROWS = T ? 8 : 16;
     kernel<<<dim3((n + ROWS - 1) / ROWS), dim3(KW * WAVE), 0, stream>>>(
         y, x, w, bias, m, n, k, x_ld, y_ld, heads ? *heads : Heads{},

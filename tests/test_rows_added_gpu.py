@@ -35,7 +35,10 @@ def kept(x: torch.Tensor, h: torch.Tensor, norm: torch.Tensor, lin):
     # workgroups of eight weight rows, the last stage a part of one
     ("dense", 8, 4224, 4160, False), ("q4_0", 3, 4160, 4160, False),
     ("q4_0", 1, 4160, 6144, False), ("q8_0", 4, 4352, 4160, False),
-    ("q4_K", 5, 4352, 4160, False)])
+    ("q4_K", 5, 4352, 4160, False),
+    # workgroups that begin at different columns
+    ("dense", 1, 8448, 4160, False), ("dense", 8, 11008, 4160, False),
+    ("dense", 16, 8192, 4160, False)])
 @pytest.mark.parametrize("how", ["plain", "gated", "heads"])
 @torch.no_grad()
 def test_added_and_scaled(kind, m, k, n, bias, how):
