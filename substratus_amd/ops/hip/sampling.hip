@@ -288,8 +288,9 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
     const float x = v * inv_t, below = __expf(fmaf(v, inv_t, -m));
     return v == top ? 1.f : x < past ? below : 0.f;
   };
-  // of usual ones none is past the largest, and that is 1 as any is
-  const bool plain = usual && fabsf(m) < INFINITY;
+  // of usual ones none is past the largest, and that is 1 as any is (but at an
+  // infinite temperature -inf is no number once scaled)
+  const bool plain = usual && fabsf(m) < INFINITY && inv_t > 0.f;
   const unsigned first = key16_of(-INFINITY), last = key16_of(top);
   const int k = top_k[b];
   const float p_target = top_p[b];

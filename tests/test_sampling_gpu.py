@@ -257,3 +257,26 @@ def test_largest_of_rows_that_are_not_usual():
                              zeros + 0.5)
     assert got[2:5].tolist() == [9, 9, 12345] or got[2] in (9, 19999)
     assert got[7] == 19998 and got[0] in (700, 15000)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1000, 9000, 32000])
+@pytest.mark.parametrize("k,p", [(0, 1.0), (40, 1.0), (0, 0.9), (600, 0.3)])
+def test_infinite_temperature(vocab, dtype, k, p):
+    """All tokens but those of -inf, which are none whatever the temperature:
+    in masked rows and past a row's end."""
+    n = 16
+    g = torch.Generator().manual_seed(vocab)
+    x = (torch.randn(n, vocab, generator=g) * 3).to(dtype)
+    x[1::2, ::7] = -torch.inf
+    x[2::4, vocab // 3:] = -torch.inf
+    u = torch.rand(n, generator=g)
+    of = lambda v: torch.full((n,), v, device=DEV)
+    got = ops.softmax_sample(x.to(DEV), of(torch.inf), of(k).int(), of(p),
+                             u.to(DEV)).tolist()
+    for i in range(n):
+        keep, cum, goal = draw(x[i], torch.inf, k, p, float(u[i]))
+        # equal weights: whole numbers, and a number that is rounded once
+        assert bool(keep[got[i]])
+        assert float(cum[got[i]]) >= float(goal) * (1 - 1e-6)
+        assert float(cum[got[i]]) <= float(goal) * (1 + 1e-6) + 1
