@@ -68,7 +68,7 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit, bool ordered,
+                       long q_ld, int nsplit, int worth,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
   constexpr int RC = D / 8;                      // 16-byte pieces of a row
@@ -80,17 +80,23 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
   // the direct loads in flight, and waits for them
   __shared__ alignas(16) uint4v s_all[NW * 2 * 2 * HALF];
 
+  // worth: keys from which sequences are put in order, or 0
   const int split = blockIdx.y;
-  const int b = ordered ? sequence_at(seq_lens, gridDim.z, max_blocks * PAGE,
-                                      blockIdx.z)
-                        : blockIdx.z;
+  int b = blockIdx.z, n;
+  if (worth > 0) {
+    const int at_lane = length_at_lane(seq_lens, gridDim.z);
+    if (unlike_lengths(at_lane, max_blocks * PAGE, worth))
+      b = sequence_at(at_lane, gridDim.z, max_blocks * PAGE, b);
+    n = __builtin_amdgcn_readlane(at_lane, b);
+  } else {
+    n = __builtin_amdgcn_readfirstlane(seq_lens[b]);
+  }
   const int in_group = hq / hkv, parts = (in_group + 15) / 16;
   const int kvh = blockIdx.x / parts, h0 = blockIdx.x % parts * 16;
   const int head0 = kvh * in_group + h0, heads = min(16, in_group - h0);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
   const int lo = lane & 15, g = lane >> 4;
-  const int n = __builtin_amdgcn_readfirstlane(seq_lens[b]);
   const int pages = (n + PAGE - 1) / PAGE;
   const int chunks = (n + CH - 1) / CH;
   const int first = split * NW + wave, step = nsplit * NW;
@@ -314,22 +320,24 @@ void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
   }
   const int parts = (hq / hkv + 15) / 16;
   // as in attention_decode_heads.hip; us, 32 heads on 8 of 128:
-  //   sequences x most keys    unlike          all            one
-  //   8 x 2500               20.9 -> 19.5   23.4 -> 22.8   17.0 -> 12.9
-  //   64 x 300               17.5 -> 17.2
-  //   64 x 2500              92.9 -> 85.0    127 -> 127    52.9 -> 35.8
-  //   256 x 2500              316 -> 291     461 -> 460    86.6 -> 64
+  //   sequences x most keys    unlike          all            one (2500)
+  //   64 x 300               18.9 -> 19.5   23.4 -> 25.2
+  //   64 x 1500              54.4 -> 53.3   71.3 -> 74.6   50.9 -> 35.8
+  //   256 x 1500              184 -> 181     269 -> 281    84.1 -> 73.4
+  // and in order, of grouped heads too: 64 x 2500 unlike 94.6 -> 80.8, 40 x 2000
+  // 55.8 -> 49.5
   const dim3 grid(hkv * parts, nsplit, bsz), block(NW * WAVE);
-  const bool ordered = orders_sequences(bsz, max_blocks, nsplit,
-                                        (long)bsz * hkv * parts * nsplit,
-                                        d == 128 ? 2 : 4);
+  const int worth = orders_sequences(bsz, max_blocks, nsplit,
+                                     (long)bsz * hkv * parts * nsplit,
+                                     d == 128 ? 2 : 4)
+                        ? worth_ordering(nsplit) : 0;
   if (d == 128) {
     attn_group_kernel<128><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, ordered, part_o, part_ml);
+        q_ld, nsplit, worth, part_o, part_ml);
   } else {
     attn_group_kernel<64><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, ordered, part_o, part_ml);
+        q_ld, nsplit, worth, part_o, part_ml);
   }
 }

@@ -89,21 +89,22 @@ void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit, bool ordered,
+                       long q_ld, int nsplit, int worth,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
+  // worth: keys from which sequences are put in order, or 0
   constexpr int LANES = D / 8;                   // of a row
   constexpr int ROWS = WAVE / LANES;             // of a piece of all lanes
   constexpr int KEYS = PIECES * ROWS;            // of a step
   constexpr int SIZE = KV8 ? 1 : 2;
   const int head = blockIdx.x, split = blockIdx.y;
-  const int b = ordered ? sequence_at(seq_lens, gridDim.z, max_blocks * PAGE,
-                                      blockIdx.z)
-                        : blockIdx.z;
+  int b = blockIdx.z, at_lane = 0;
+  if (worth > 0) at_lane = length_at_lane(seq_lens, gridDim.z);
   const int kvh = head / (hq / hkv);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE, row = lane / LANES, at = lane % LANES;
   const int* bt = block_table + (long)b * max_blocks;
+  int n = seq_lens[b];
 
   // steps of KEYS keys, one page or two, by turns with other waves
   constexpr int PAGES = KEYS / PAGE;
@@ -112,12 +113,20 @@ void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
     return max_blocks > 0 ? bt[min(step * PAGES + p, max_blocks - 1)] : 0;
   };
   int page[PAGES], next[PAGES];
-  #pragma unroll
-  for (int p = 0; p < PAGES; ++p) {
-    page[p] = page_of(first, p);
-    next[p] = page_of(first + stride, p);
+  auto begin = [&]() {
+    #pragma unroll
+    for (int p = 0; p < PAGES; ++p) {
+      page[p] = page_of(first, p);
+      next[p] = page_of(first + stride, p);
+    }
+  };
+  begin();
+  if (worth > 0 && unlike_lengths(at_lane, max_blocks * PAGE, worth)) {
+    b = sequence_at(at_lane, gridDim.z, max_blocks * PAGE, b);
+    bt = block_table + (long)b * max_blocks;
+    n = __builtin_amdgcn_readlane(at_lane, b);
+    begin();
   }
-  const int n = seq_lens[b];
   const int steps = (n + KEYS - 1) / KEYS;
 
   float qf[8];
@@ -319,25 +328,24 @@ void launch_attn_heads(bf16_t* out, const bf16_t* q, const void* kc,
   // fastest put all heads of one on the same eighth of the chip where there are
   // eight of them, and long ones last. us, MI355X, keys from a quarter of the most
   // to all, all of them, one of them (the others' a twentieth), sequences first ->
-  // heads first, and in order from 1000 on:
+  // heads first:
   //   heads x most keys        unlike          all            one
-  //   8 x 32 x 1000          19.7 -> 19.3   24.1 -> 24.3
-  //   64 x 32 x 300          39.2 -> 36.7
-  //   64 x 32 x 1000          119 -> 107     166 -> 170
-  //   64 x 32 x 2500          288 -> 261     410 -> 414     120 -> 46
-  //   256 x 32 x 1000         431 -> 423     669 -> 663
-  //   100 x 12 (64) x 2500   90.7 -> 82.2    122 -> 125    36.1 -> 22
+  //   64 x 32 x 300          37.3 -> 34.8   49.9 -> 49.8
+  //   64 x 32 x 1500          168 -> 157     250 -> 259     118 -> 48 (2500)
+  //   256 x 12 (64) x 1500    119 -> 117     173 -> 175    54.6 -> 29 (2500)
+  // Long sequences before short ones (attention_order.h): 30 x 40 x 1100 unlike
+  // 74.7 -> 70.3, 64 x 32 x 2500 one 52.9 -> 47.6.
   const dim3 grid(hq, nsplit, bsz);
-  const bool ordered = orders_sequences(bsz, max_blocks, nsplit,
-                                        (long)bsz * hq * nsplit,
-                                        16 / waves);
+  const int worth = orders_sequences(bsz, max_blocks, nsplit,
+                                     (long)bsz * hq * nsplit, 16 / waves)
+                        ? worth_ordering(nsplit) : 0;
   auto go = [&](auto dim, auto fp8, auto w) {
     constexpr int W = decltype(w)::value;
     attn_heads_kernel<decltype(dim)::value, decltype(fp8)::value, W>
         <<<grid, dim3(W * WAVE), 0, stream>>>(
             out, q, reinterpret_cast<const char*>(kc),
             reinterpret_cast<const char*>(vc), block_table, seq_lens, hq, hkv,
-            max_blocks, scale, q_ld, nsplit, ordered, part_o, part_ml);
+            max_blocks, scale, q_ld, nsplit, worth, part_o, part_ml);
   };
   auto sized = [&](auto dim, auto fp8) {
     if (waves == 8) go(dim, fp8, std::integral_constant<int, 8>());

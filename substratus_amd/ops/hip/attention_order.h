@@ -3,67 +3,58 @@
 
 #include "common.h"
 
-constexpr int ORDERED = 256;      // sequences that are put in order, at most
+constexpr int ORDERED = WAVE;     // sequences that are put in order, at most
 constexpr int MOST = 65535;       // that a grid's last side takes
 
-// The sequence that is r-th by length, longest first, lengths counted in 256ths of
-// the keys that a table has room for; equal ones as they come. For all lanes of a
-// wave; bsz sequences, at most ORDERED, 0 <= r < bsz. Bit by bit: those that have
-// it are the longer ones of what is left.
-DEV_INLINE int sequence_at(const int* lens, int bsz, int room, int r) {
-  constexpr int PER = ORDERED / WAVE;
-  const int lane = threadIdx.x % WAVE;
-  const int shift = max(24 - __clz(max(room, 1)), 0);
-  int key[PER];
-  unsigned long long left[PER];
-  #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    key[i] = 0;
-    left[i] = 0;
-    if (i * WAVE < bsz) {
-      key[i] = min(lens[min(i * WAVE + lane, bsz - 1)] >> shift, 255);
-      left[i] = __ballot(i * WAVE + lane < bsz);
-    }
-  }
-  #pragma unroll
-  for (int bit = 7; bit >= 0; --bit) {
-    unsigned long long with[PER];
-    int many = 0;
-    #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      with[i] = 0;
-      if (i * WAVE < bsz) {
-        with[i] = left[i] & __ballot(key[i] >> bit & 1);
-        many += __popcll(with[i]);
-      }
-    }
-    const bool longer = r < many;
-    if (!longer) r -= many;
-    #pragma unroll
-    for (int i = 0; i < PER; ++i)
-      left[i] = longer ? with[i] : left[i] & ~with[i];
-  }
-  int at = 0;
-  #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int many = __popcll(left[i]);
-    if (r >= 0 && r < many) {
-      const int before = __builtin_amdgcn_mbcnt_hi(
-          (unsigned)(left[i] >> 32),
-          __builtin_amdgcn_mbcnt_lo((unsigned)left[i], 0));
-      at = i * WAVE - 1 + __ffsll(__ballot((left[i] >> lane & 1) &&
-                                           before == r));
-    }
-    r -= many;
-  }
-  return __builtin_amdgcn_readfirstlane(at);
+// A lane's sequence's length, of bsz sequences, at most ORDERED (the last one's in
+// lanes past it).
+DEV_INLINE int length_at_lane(const int* lens, int bsz) {
+  return lens[min((int)threadIdx.x % WAVE, bsz - 1)];
 }
 
-// Whether they are put in order: where not all workgroups fit the chip at once, so
-// that those of long sequences may be the last ones, and take long. Finding its
-// sequence costs a workgroup half a microsecond, a share of a thousand keys ten.
+// Lengths in 256ths of the keys that a table has room for.
+DEV_INLINE int coarse(int n, int room) {
+  return min(n >> max(24 - __clz(max(room, 1)), 0), 255);
+}
+
+// Whether putting sequences of these lengths in order pays: some are unlike others,
+// and the longest has more than `worth` keys.
+DEV_INLINE bool unlike_lengths(int n, int room, int worth) {
+  const int key = coarse(n, room);
+  return __ballot(n > worth) &&
+         __ballot(key != __builtin_amdgcn_readfirstlane(key));
+}
+
+// The sequence that is r-th by length, longest first, 0 <= r < bsz; equal ones as
+// they come. For all lanes of a wave. Bit by bit: those that have it are the longer
+// ones of what is left.
+DEV_INLINE int sequence_at(int n, int bsz, int room, int r) {
+  const int lane = threadIdx.x % WAVE, key = coarse(n, room);
+  unsigned long long left = __ballot(lane < bsz);
+  #pragma unroll
+  for (int bit = 7; bit >= 0; --bit) {
+    const unsigned long long with = left & __ballot(key >> bit & 1);
+    const int many = __popcll(with);
+    left = r < many ? with : left & ~with;
+    if (r >= many) r -= many;
+  }
+  const int before = __builtin_amdgcn_mbcnt_hi(
+      (unsigned)(left >> 32),
+      __builtin_amdgcn_mbcnt_lo((unsigned)left, 0));
+  return __ffsll(__ballot((left >> lane & 1) && before == r)) - 1;
+}
+
+// Whether workgroups look at the lengths: where not all of them fit the chip at once,
+// so that those of long sequences may be the last ones, and take long. Of up to 64
+// sequences a look is one load, of 256 four and their wait: at 100 keys in a table
+// of 4096, 256 x 12 x 64, 12.4 us without, 16.9 with (20.2 where they are put in
+// order whatever their lengths).
 inline bool orders_sequences(int bsz, int max_blocks, int nsplit,
                              long workgroups, int per_cu) {
   return bsz > 1 && bsz <= ORDERED && max_blocks >= 60L * nsplit &&
          workgroups > 256L * per_cu;
 }
+
+// Keys from which it pays: of a share of a thousand, finding the sequence takes half
+// a microsecond and the share ten.
+inline int worth_ordering(int nsplit) { return 960 * nsplit; }

@@ -1,5 +1,5 @@
-"""Decode attention of more workgroups than the chip holds, which take sequences
-by length: each has its own keys, whatever the lengths are."""
+"""Decode attention of more workgroups than the chip holds: each sequence has its
+own keys, whatever the lengths are."""
 
 import pytest
 import torch
@@ -28,7 +28,7 @@ def test_own_keys(batch, hq, hkv, d, how):
         lens[batch // 2] = most
     elif how == "none":
         lens[::3] = 0
-    # few pages, shared by sequences: what tells them apart is their order
+    # few pages, shared by sequences: what tells them apart is their tables
     kc, vc = (torch.randn(70, hkv, 16, d, device=DEV).bfloat16()
               for _ in range(2))
     table = torch.randint(0, 70, (batch, room), generator=g).int().to(DEV)
