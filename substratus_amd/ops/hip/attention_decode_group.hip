@@ -68,7 +68,7 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit, int worth,
+                       long q_ld, int nsplit, bool ordered,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
   constexpr int RC = D / 8;                      // 16-byte pieces of a row
@@ -80,19 +80,21 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
   // the direct loads in flight, and waits for them
   __shared__ alignas(16) uint4v s_all[NW * 2 * 2 * HALF];
 
-  // worth: keys from which sequences are put in order, or 0
-  const int split = blockIdx.y;
-  int b = blockIdx.z, n;
-  if (worth > 0) {
-    const int at_lane = length_at_lane(seq_lens, gridDim.z);
-    if (unlike_lengths(at_lane, max_blocks * PAGE, worth))
-      b = sequence_at(at_lane, gridDim.z, max_blocks * PAGE, b);
+  const int in_group = hq / hkv, parts = (in_group + 15) / 16;
+  int b = blockIdx.x, part = blockIdx.y, split = blockIdx.z, n;
+  if (ordered) {
+    const int bsz = gridDim.x, at_lane = length_at_lane(seq_lens, bsz);
+    if (unlike_lengths(at_lane, max_blocks * PAGE)) {
+      const Turn turn = turn_of(hkv * parts, nsplit);
+      part = turn.head;
+      split = turn.split;
+      b = sequence_at(at_lane, bsz, max_blocks * PAGE, turn.sequence);
+    }
     n = __builtin_amdgcn_readlane(at_lane, b);
   } else {
     n = __builtin_amdgcn_readfirstlane(seq_lens[b]);
   }
-  const int in_group = hq / hkv, parts = (in_group + 15) / 16;
-  const int kvh = blockIdx.x / parts, h0 = blockIdx.x % parts * 16;
+  const int kvh = part / parts, h0 = part % parts * 16;
   const int head0 = kvh * in_group + h0, heads = min(16, in_group - h0);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
@@ -308,36 +310,24 @@ void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
                        const int* seq_lens, int bsz, int hq, int hkv, int d,
                        int max_blocks, float scale, long q_ld, int nsplit,
                        float* part_o, float* part_ml, hipStream_t stream) {
-  if (bsz > MOST) {               // the others first
-    const long at = MOST;
-    launch_attn_group(out + at * hq * d, q + at * q_ld, kc, vc,
-                      block_table + at * max_blocks, seq_lens + at, bsz - MOST,
-                      hq, hkv, d, max_blocks, scale, q_ld, nsplit,
-                      part_o ? part_o + at * hq * nsplit * d : nullptr,
-                      part_ml ? part_ml + at * hq * nsplit * 2 : nullptr,
-                      stream);
-    bsz = MOST;
-  }
   const int parts = (hq / hkv + 15) / 16;
-  // as in attention_decode_heads.hip; us, 32 heads on 8 of 128:
-  //   sequences x most keys    unlike          all            one (2500)
-  //   64 x 300               18.9 -> 19.5   23.4 -> 25.2
-  //   64 x 1500              54.4 -> 53.3   71.3 -> 74.6   50.9 -> 35.8
-  //   256 x 1500              184 -> 181     269 -> 281    84.1 -> 73.4
-  // and in order, of grouped heads too: 64 x 2500 unlike 94.6 -> 80.8, 40 x 2000
-  // 55.8 -> 49.5
-  const dim3 grid(hkv * parts, nsplit, bsz), block(NW * WAVE);
-  const int worth = orders_sequences(bsz, max_blocks, nsplit,
-                                     (long)bsz * hkv * parts * nsplit,
-                                     d == 128 ? 2 : 4)
-                        ? worth_ordering(nsplit) : 0;
+  // sequences first, as parts of a group read the same keys (see
+  // attention_decode_heads.hip; us, 71 heads on 1, 200 x 516 keys, heads first 31.4,
+  // now 23.8; 64 x 32 on 8 x 1500, all of them, 83 and 76.5). Where a part is all of
+  // a group, long sequences before short ones, heads first then: 32 on 8, unlike, 64
+  // x 2500 89.6 -> 80.8, 40 x 2000 55.8 -> 49.4.
+  const dim3 grid(bsz, hkv * parts, nsplit), block(NW * WAVE);
+  const bool ordered =
+      parts == 1 && orders_sequences(bsz, max_blocks, nsplit,
+                                     (long)bsz * hkv * nsplit,
+                                     d == 128 ? 2 : 4);
   if (d == 128) {
     attn_group_kernel<128><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, worth, part_o, part_ml);
+        q_ld, nsplit, ordered, part_o, part_ml);
   } else {
     attn_group_kernel<64><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, worth, part_o, part_ml);
+        q_ld, nsplit, ordered, part_o, part_ml);
   }
 }

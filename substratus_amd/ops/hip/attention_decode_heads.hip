@@ -89,26 +89,30 @@ void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit, int worth,
+                       long q_ld, int nsplit, bool turned, bool ordered,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
-  // worth: keys from which sequences are put in order, or 0
+  // turned: workgroups take a sequence's heads in turn, the next sequence's from
+  // the next one on; or every sequence's first head, and so on
+  // ordered: long sequences first where lengths are unlike
   constexpr int LANES = D / 8;                   // of a row
   constexpr int ROWS = WAVE / LANES;             // of a piece of all lanes
   constexpr int KEYS = PIECES * ROWS;            // of a step
   constexpr int SIZE = KV8 ? 1 : 2;
-  const int head = blockIdx.x, split = blockIdx.y;
-  int b = blockIdx.z, at_lane = 0;
-  if (worth > 0) at_lane = length_at_lane(seq_lens, gridDim.z);
-  const int kvh = head / (hq / hkv);
+  const int bsz = turned ? gridDim.y : gridDim.x;
+  int b = turned ? blockIdx.y : blockIdx.x, split = blockIdx.z, at_lane = 0;
+  int head = turned ? (int)(blockIdx.x + blockIdx.y) % hq : blockIdx.y;
+  if (ordered) at_lane = length_at_lane(seq_lens, bsz);
+  const int group = hq / hkv;
+  int kvh = head / group;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE, row = lane / LANES, at = lane % LANES;
   const int* bt = block_table + (long)b * max_blocks;
-  int n = seq_lens[b];
 
   // steps of KEYS keys, one page or two, by turns with other waves
   constexpr int PAGES = KEYS / PAGE;
-  const int first = split * WAVES + wave, stride = nsplit * WAVES;
+  const int stride = nsplit * WAVES;
+  int first = split * WAVES + wave;
   auto page_of = [&](int step, int p) {
     return max_blocks > 0 ? bt[min(step * PAGES + p, max_blocks - 1)] : 0;
   };
@@ -121,10 +125,16 @@ void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
     }
   };
   begin();
-  if (worth > 0 && unlike_lengths(at_lane, max_blocks * PAGE, worth)) {
-    b = sequence_at(at_lane, gridDim.z, max_blocks * PAGE, b);
+  int n = seq_lens[b];
+  if (ordered && unlike_lengths(at_lane, max_blocks * PAGE)) {
+    const Turn turn = turn_of(hq, nsplit);
+    head = turn.head;
+    kvh = head / group;
+    split = turn.split;
+    b = sequence_at(at_lane, bsz, max_blocks * PAGE, turn.sequence);
     bt = block_table + (long)b * max_blocks;
     n = __builtin_amdgcn_readlane(at_lane, b);
+    first = split * WAVES + wave;
     begin();
   }
   const int steps = (n + KEYS - 1) / KEYS;
@@ -314,38 +324,37 @@ void launch_attn_heads(bf16_t* out, const bf16_t* q, const void* kc,
                        int max_blocks, float scale, long q_ld, int waves,
                        int nsplit, float* part_o, float* part_ml, bool kv8,
                        hipStream_t stream) {
-  if (bsz > MOST) {               // the others first
-    const long at = MOST;
-    launch_attn_heads(out + at * hq * d, q + at * q_ld, kc, vc,
-                      block_table + at * max_blocks, seq_lens + at, bsz - MOST,
-                      hq, hkv, d, max_blocks, scale, q_ld, waves, nsplit,
-                      part_o ? part_o + at * hq * nsplit * d : nullptr,
-                      part_ml ? part_ml + at * hq * nsplit * 2 : nullptr, kv8,
-                      stream);
-    bsz = MOST;
-  }
-  // a sequence's heads and shares next to each other: the sequence itself as the
-  // fastest put all heads of one on the same eighth of the chip where there are
-  // eight of them, and long ones last. us, MI355X, keys from a quarter of the most
-  // to all, all of them, one of them (the others' a twentieth), sequences first ->
-  // heads first:
-  //   heads x most keys        unlike          all            one
-  //   64 x 32 x 300          37.3 -> 34.8   49.9 -> 49.8
-  //   64 x 32 x 1500          168 -> 157     250 -> 259     118 -> 48 (2500)
-  //   256 x 12 (64) x 1500    119 -> 117     173 -> 175    54.6 -> 29 (2500)
-  // Long sequences before short ones (attention_order.h): 30 x 40 x 1100 unlike
-  // 74.7 -> 70.3, 64 x 32 x 2500 one 52.9 -> 47.6.
-  const dim3 grid(hq, nsplit, bsz);
-  const int worth = orders_sequences(bsz, max_blocks, nsplit,
-                                     (long)bsz * hq * nsplit, 16 / waves)
-                        ? worth_ordering(nsplit) : 0;
+  // Workgroups go to the eighths of the chip in turn. Sequences first, a sequence's
+  // heads come to the same eighth where there is a multiple of eight of them: keys
+  // that heads share, and their pages' addresses, come to its caches once. Heads
+  // first, an eighth reads its own eighth of all pages, and meets the others at few
+  // of the memory's channels where lengths are equal; turned by the sequence it does
+  // not, and a long sequence has all of the chip. So turned where heads share no keys
+  // and there are more than the chip holds at a time (four a CU). us, MI355X,
+  // sequences first, heads first, turned; keys from a quarter of the most to all, all
+  // of them, one of them (the others' a twentieth):
+  //   sequences x heads x keys      unlike         all            one (2500)
+  //   512 x 32 x 516                             698  764  660
+  //   256 x 32 x 516                             387  348  327
+  //   64 x 32 x 1500             168  157  158   250  259  239   118   48   48
+  //   256 x 12 x 1500 of 64      119  117  117   173  175  174    55   29   29
+  //   64 x 16 x 1500 of 64      47.1 44.5 43.8                    51   32   32
+  //   86 x 12 x 1500 of 64      42.6      44.5  67.2      68.2
+  //   16 x 32 x 900 (not turned) 35.6     37.2  31.4      31.3 (516)
+  //   64 x 71 on 1 x 516, fp8 (not turned)      33.7 37.3
+  // Long sequences before short ones, heads first then (attention_order.h): 30 x 40
+  // x 1100 unlike 74.7 -> 70.5, 64 x 71 on 1 x 1500, fp8, unlike 71.1 -> 61.5.
+  const bool turned = hq == hkv && (long)bsz * hq >= 1024 && bsz <= MOST;
+  const dim3 grid = turned ? dim3(hq, bsz, nsplit) : dim3(bsz, hq, nsplit);
+  const bool ordered = orders_sequences(bsz, max_blocks, nsplit,
+                                        (long)bsz * hq * nsplit, 16 / waves);
   auto go = [&](auto dim, auto fp8, auto w) {
     constexpr int W = decltype(w)::value;
     attn_heads_kernel<decltype(dim)::value, decltype(fp8)::value, W>
         <<<grid, dim3(W * WAVE), 0, stream>>>(
             out, q, reinterpret_cast<const char*>(kc),
             reinterpret_cast<const char*>(vc), block_table, seq_lens, hq, hkv,
-            max_blocks, scale, q_ld, nsplit, worth, part_o, part_ml);
+            max_blocks, scale, q_ld, nsplit, turned, ordered, part_o, part_ml);
   };
   auto sized = [&](auto dim, auto fp8) {
     if (waves == 8) go(dim, fp8, std::integral_constant<int, 8>());

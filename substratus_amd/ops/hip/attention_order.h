@@ -4,7 +4,8 @@
 #include "common.h"
 
 constexpr int ORDERED = WAVE;     // sequences that are put in order, at most
-constexpr int MOST = 65535;       // that a grid's last side takes
+constexpr int MOST = 65535;       // that a grid's second side takes
+constexpr int LONG = 960;         // keys from which their order matters
 
 // A lane's sequence's length, of bsz sequences, at most ORDERED (the last one's in
 // lanes past it).
@@ -18,10 +19,11 @@ DEV_INLINE int coarse(int n, int room) {
 }
 
 // Whether putting sequences of these lengths in order pays: some are unlike others,
-// and the longest has more than `worth` keys.
-DEV_INLINE bool unlike_lengths(int n, int room, int worth) {
+// and the longest is long. (Finding a sequence takes half a microsecond, a thousand
+// keys ten.)
+DEV_INLINE bool unlike_lengths(int n, int room) {
   const int key = coarse(n, room);
-  return __ballot(n > worth) &&
+  return __ballot(n > LONG) &&
          __ballot(key != __builtin_amdgcn_readfirstlane(key));
 }
 
@@ -44,6 +46,16 @@ DEV_INLINE int sequence_at(int n, int bsz, int room, int r) {
   return __ffsll(__ballot((left >> lane & 1) && before == r)) - 1;
 }
 
+// What a workgroup has where a sequence's heads come first, then its shares, then
+// other sequences.
+struct Turn {
+  int head, sequence, split;
+};
+DEV_INLINE Turn turn_of(int heads, int nsplit) {
+  const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  return {id % heads, id / (heads * nsplit), id / heads % nsplit};
+}
+
 // Whether workgroups look at the lengths: where not all of them fit the chip at once,
 // so that those of long sequences may be the last ones, and take long. Of up to 64
 // sequences a look is one load, of 256 four and their wait: at 100 keys in a table
@@ -54,7 +66,3 @@ inline bool orders_sequences(int bsz, int max_blocks, int nsplit,
   return bsz > 1 && bsz <= ORDERED && max_blocks >= 60L * nsplit &&
          workgroups > 256L * per_cu;
 }
-
-// Keys from which it pays: of a share of a thousand, finding the sequence takes half
-// a microsecond and the share ten.
-inline int worth_ordering(int nsplit) { return 960 * nsplit; }

@@ -28,6 +28,10 @@ def test_own_keys(batch, hq, hkv, d, how):
         lens[batch // 2] = most
     elif how == "none":
         lens[::3] = 0
+    check(batch, hq, hkv, d, room, lens, g)
+
+
+def check(batch, hq, hkv, d, room, lens, g):
     # few pages, shared by sequences: what tells them apart is their tables
     kc, vc = (torch.randn(70, hkv, 16, d, device=DEV).bfloat16()
               for _ in range(2))
@@ -51,6 +55,19 @@ def test_own_keys(batch, hq, hkv, d, how):
             2.0 ** -8 * float(want.norm()), b
 
 
+# long and short ones in a table with room for more, in shares or not
+@pytest.mark.parametrize("batch,hq,hkv,d,room,most", [
+    (40, 32, 8, 128, 256, 2000), (33, 128, 8, 64, 256, 4096),
+    (64, 32, 8, 128, 157, 961), (64, 32, 8, 128, 256, 960),
+    (40, 71, 71, 64, 300, 1500), (64, 71, 1, 64, 120, 1900)])
+@torch.no_grad()
+def test_shares_in_order(batch, hq, hkv, d, room, most):
+    g = torch.Generator().manual_seed(batch + d)
+    lens = torch.randint(1, most + 1, (batch,), generator=g)
+    lens[batch // 3] = most
+    check(batch, hq, hkv, d, room, lens, g)
+
+
 @pytest.mark.parametrize("hq", [2, 4])
 @torch.no_grad()
 def test_more_sequences_than_a_grid_side(hq):
@@ -65,3 +82,36 @@ def test_more_sequences_than_a_grid_side(hq):
         assert torch.equal(out[part], ops.paged_attn_decode(
             q[part].contiguous(), kc, vc, table[part].contiguous(),
             n[part].contiguous(), 0.125))
+
+
+# about 1024 heads, where a sequence's come in turn; heads that share keys or not;
+# as many sequences as a grid's second side takes
+@pytest.mark.parametrize("batch,hq,hkv,d", [
+    (63, 16, 16, 64), (64, 16, 16, 64), (65, 16, 16, 64), (85, 12, 12, 64),
+    (86, 12, 12, 64), (1024, 1, 1, 128), (25, 41, 41, 128), (40, 71, 1, 64),
+    (64, 96, 2, 128), (65535, 2, 2, 64)])
+@pytest.mark.parametrize("fp8", [False, True])
+@torch.no_grad()
+def test_heads_in_turn(batch, hq, hkv, d, fp8):
+    if fp8 and hq // hkv not in (1, 71):
+        pytest.skip("other kernels'")
+    g = torch.Generator().manual_seed(batch)
+    kc, vc = (torch.randn(40, hkv, 16, d, device=DEV).bfloat16()
+              for _ in range(2))
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+    table = torch.randint(0, 40, (batch, 3), generator=g).int().to(DEV)
+    q = torch.randn(batch, hq, d, device=DEV).bfloat16()
+    n = torch.randint(0, 49, (batch,), generator=g).int().to(DEV)
+    out = ops.paged_attn_decode(q, kc, vc, table, n, 0.125)
+    for at in range(0, batch, 512):
+        part = slice(at, at + 512)
+        k, v = (c.float()[table[part].long()].transpose(1, 2).flatten(2, 3)
+                .repeat_interleave(hq // hkv, 1) for c in (kc, vc))
+        s = (k @ q[part].float().unsqueeze(-1)).squeeze(-1) * 0.125
+        none = torch.arange(48, device=DEV) >= n[part, None, None]
+        s = s.masked_fill(none, -torch.inf).softmax(-1).nan_to_num(0.0)
+        want = (v * s.unsqueeze(-1)).sum(2)
+        # results are rounded to bf16, weights have 24 bits
+        assert float((out[part].float() - want).norm()) <= \
+            2.0 ** -8 * float(want.norm()), at
