@@ -361,13 +361,18 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // and 130, 20 x 28672 x 4096, gated, 56.7 and 47.3. More rows lose what there is to
 // gain (96 x 48000 x 6144 146 and 143), or are two blocks, which read the weights
 // twice (130 x 32000 x 4096 65 and 93).
-// A norm that adds up the shares saves a launch, but for short products of few
-// columns. Of 5578 products of those widths, each with the residual's
-// sum and its norm, as they were -> now: 1.07 times as fast on average (2048 to 14336
-// columns' inner sizes and 4096 rows 1.05 to 1.17 where the product was this one's,
-// 1.1 to 1.66 where it was the library's), 20 slower by more than 3 %, by 17 at most.
-// 64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
-// 128 x 5120 x 5120 35.7 -> 25.3, 256 x 4096 x 11008 47.2 -> 43.8.
+// A norm that adds up the shares saves a launch: 3.5 us of a product that would have
+// been this one's (64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
+// 256 x 4096 x 11008 47.2 -> 43.8; of 8070 of those widths none slower by more than
+// 1 %, 1.10 times as fast on average). For its sake products leave the library where
+// these estimates are near enough: not short ones of few columns and up to 128 rows
+// (80 x 2560 x 3584 12.5 -> 15.7, 100 x 2048 x 5632 15.3 -> 17.0; but 100 x 5120
+// x 4096 27.0 -> 21.2), nor of more rows than that where they are wide, narrow, short
+// or little more than 128 (211 x 5760 x 4480 31.7 -> 38.4, 217 x 2112 x 3200 16.2 ->
+// 18.4, 129 x 4544 x 6144 30.1 -> 34.9). Of 5053 products that 3.5 us more would take
+// from the library, 3540 are, 1.23 times as fast, six shapes of them slower by more
+// than 3 %, by 11 at most (of one inner size, 22016, and up to 32 rows, by 7: 83 ->
+// 89 us); of the others 266 would be, by up to 25.
 bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
   if (m <= 16 || m > 256 || k < (paired ? 1024 : 2048) ||
       (m > 96 && n > 12288))
@@ -388,11 +393,18 @@ bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
                        share % 32 == 0;
   const bool saved = normed && plan.splits > 1 &&
                      (m <= 64 || n >= 1536 || k > 4096);
-  const double pass = saved ? 3.5
+  const double theirs = library * (longer ? 1.2 : 1.);
+  const bool near =
+      m <= 64 ? true
+      : m <= 128 ? n <= 10240 && (k > 6144 || n > 4096 ||
+                                  (k > 5120 && n > 2048))
+                 : m > 144 && n > 2048 && n <= 5120 && k >= 3584;
+  const double saves = near ? 3.5 : m > 128 && k > 16384 ? theirs / 100 : 0.;
+  const double pass = saved ? saves
                       : !paired ? 0. : n >= 4096 && k >= 2048 ? 2. : 1.;
   const double ours = plan.us * (in_step ? 1.25 : 1.) -
                       (plan.splits > 1 ? 0. : 2.);
-  return ours < library * (longer ? 1.2 : 1.) + pass;
+  return ours < theirs + pass;
 }
 
 bool mid_norm_takes(long m, long n, long k) {
