@@ -48,7 +48,7 @@ def test_shares_in_step(m):
 
 
 @pytest.mark.parametrize("m,n,k,pays", [
-    (64, 4096, 4096, True), (17, 8192, 28672, True),
+    (64, 4096, 4096, True), (24, 8192, 28672, True),
     (80, 2560, 3584, False), (100, 2048, 5632, False), (100, 5120, 4096, True),
     (128, 5120, 5120, True), (128, 2048, 4096, False),
     (129, 4544, 6144, False), (211, 5760, 4480, False),
