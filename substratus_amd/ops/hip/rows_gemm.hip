@@ -289,16 +289,17 @@ bool rows_gemm_pays(int m, int n, int k, bool paired) {
 // Whether a workgroup has eight weight rows instead of 16. A CU takes in some 45
 // GB/s, so the ones that have most of a matrix are what takes the time: eight rows
 // instead of 16 up to 2048, three times eight instead of two of 16 from 4096 to
-// 6144. (Between and past them it is as many rows either way, and x once more.) us,
-// MI355X, 16 -> eight, of one and eight rows:
+// 6144. (Between and past them it is as many rows either way, and x once more; of
+// those wider ones rows of up to 2048 end before it matters.) us, MI355X, 16 ->
+// eight, of one and eight rows:
 //   768 x 3072   4.6  5.2 ->  3.6  4.2     4608 x 18432  41.6 45.2 -> 34.8 40.7
 //   2048 x 2048  4.7  4.8 ->  4.1  4.2     5120 x 5120   13.7 15.3 -> 12.1 13.7
-//   2048 x 5632  8.6  8.4 ->  6.5  6.8     6144 x 2048    7.4  7.4 ->  7.2  7.4
+//   2048 x 5632  8.6  8.4 ->  6.5  6.8     6144 x 2560    8.1      ->  7.7
 //   2560 x 10240  14 14.9 -> 13.5 16.4     6144 x 16384  44.7 47.2 -> 41.8 43.6
-//   3584 x 18944  26 27.1 -> 26.0 32.3
+//   3584 x 18944  26 27.1 -> 26.0 32.3     5632 x 768     4.1  4.2 ->  4.4  4.5
 bool rows_gemm_thin(int m, int n, int k, bool paired) {
-  return m <= 8 && !paired && (n <= 2048 || (n > 4096 && n <= 6144)) &&
-         k % 128 == 0;
+  return m <= 8 && !paired && k % 128 == 0 &&
+         (n <= 2048 || (n > 4096 && n <= 6144 && k > 2048));
 }
 
 // Whether workgroups begin at different columns: all at the same they meet at few of

@@ -57,3 +57,13 @@ def test_shares_in_step(m):
 def test_products_with_their_norm(m, n, k, pays):
     """Those that lost by it stay with the library and a norm of its own."""
     assert _C.mid_norm_good(m, n, k) == pays
+
+
+@pytest.mark.parametrize("n,k,thin", [
+    (2048, 512, True), (2112, 512, False), (4096, 8192, False),
+    (4160, 2048, False), (4160, 2176, True), (6144, 16384, True),
+    (6208, 4096, False), (5120, 768, False), (5120, 2240, False)])
+def test_eight_rows_of_weights(n, k, thin):
+    """A workgroup has eight of them where that is the faster one."""
+    assert _C.rows_added_parts(8, n, k) == n // (8 if thin else 16)
+    assert _C.rows_added_parts(9, n, k) == n // 16
