@@ -338,9 +338,15 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // matrices are wide and rows many the library has tiles for the chip, and sums of
 // few numbers cannot be shared. Long sums of more than 32 rows take it a fifth
 // longer at least, but for 256, which are whole tiles. Of rows of a multiple of 4 KB
-// it takes a fifth longer in wide paired products, as its CUs all read the same of the
+// it takes a fifth longer in paired products, as its CUs all read the same of the
 // memory's channels (64 x 28672 x 4096 54.4 us, and 45.9 here; 32 x 22016 x 4096 46.1,
-// and 37.0; 64 x 57344 x 8192 182 and 176). Up to 96 rows whose shares begin on whole
+// and 37.0; 64 x 57344 x 8192 182 and 176), but for rows of a multiple of 32 KB (48 x
+// 8192 x 16384 62, and 70 here), and with more than 64 rows short and long ones, and
+// narrow matrices (69 x 6144 x 2048 13.1 and 15.3, 96 x 13824 x 16384 118 and 137,
+// 96 x 2464 x 4096 12.8 and 16.3), and little more than 128 (135 x 4288 x 6144 29.2 and
+// 33.3): of 2206 products that a fifth more takes from it
+// 1413 stay so, 1.15 times as fast, six slower by more than 3 %, of the others 246
+// would be. Up to 96 rows whose shares begin on whole
 // 4 KB of rows of a multiple of 16 KB stay with it: of 8192 x 8192 32 to 40 us either
 // way, of 128 rows 48, and 39 here. What nothing is shared of begins and ends 2 us
 // sooner (55 x 11264 x 2048, gated: 16 us, the library 21).
@@ -360,7 +366,12 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // 32000 x 4096 61.6 and 50.7, 64 x 128256 x 4096 210 and 191, 48 x 29760 x 12288 174
 // and 130, 20 x 28672 x 4096, gated, 56.7 and 47.3. More rows lose what there is to
 // gain (96 x 48000 x 6144 146 and 143), or are two blocks, which read the weights
-// twice (130 x 32000 x 4096 65 and 93).
+// twice (130 x 32000 x 4096 65 and 93). Nor are those of more than 32 rows whose
+// second round of 256 workgroups is all but empty (64 x 33328 x 2048 40.5 us, and 53.4
+// here; 48 x 36864 x 2048, gated, 41.7 and 46.3), and of rows of a multiple of 16 KB
+// others than a whole round (24 x 27648 x 8192 116 and 96, but 20 x 16384 x 8192 55 and
+// 62, 20 x 57344 x 8192 164 and 188). Of 2019 1788 stay, 1.19 times as fast, five
+// slower by more than 3 %, by 5 at most; of the others 67 were.
 // A norm that adds up the shares saves a launch: 3.5 us of a product that would have
 // been this one's (64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
 // 256 x 4096 x 11008 47.2 -> 43.8; of 8070 of those widths none slower by more than
@@ -377,14 +388,20 @@ bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
   if (m <= 16 || m > 256 || k < (paired ? 1024 : 2048) ||
       (m > 96 && n > 12288))
     return false;
-  if (m <= 64 && n >= 16000 && k % 2048 == 0 && k <= (paired ? 6144 : 12288))
+  if (m <= 64 && n >= 16000 && k % 2048 == 0 && k <= (paired ? 6144 : 12288) &&
+      !(m > 32 && n > 32768 && n <= 45056) &&
+      (k % 8192 != 0 || (n >= 24576 && n <= 32768)))
     return true;
   if (!paired && k < 3072) return false;
   const double few = std::min(1., n / 4500.);
   const double inner = m > 128 ? 1.5e-3 + 1.7e-3 * few : .6e-3 + .6e-3 * few;
   const double work = n * k * 2 / 1e7 + k * inner + m * n * k * 2 / 2e9;
-  const double library = (m > 128 ? 1. : 6.6) + work *
-      (k % 256 ? 1.45 : paired && k % 2048 == 0 ? 1.2 : 1.);
+  const bool same = paired && k % 2048 == 0 &&
+                    (m <= 64 ? k % 16384 != 0
+                             : n > 2800 && k < 8192 && (k > 2048 || n > 8300) &&
+                                   (m <= 128 || m > 144));
+  const double library =
+      (m > 128 ? 1. : 6.6) + work * (k % 256 ? 1.45 : same ? 1.2 : 1.);
   const bool longer = m > 32 && m < 256 && n <= 10240 &&
                       k >= (m > 128 ? 12288 : 8192);
   const MidPlan plan = mid_gemm_plan(m, n, k);

@@ -67,3 +67,17 @@ def test_eight_rows_of_weights(n, k, thin):
     """A workgroup has eight of them where that is the faster one."""
     assert _C.rows_added_parts(8, n, k) == n // (8 if thin else 16)
     assert _C.rows_added_parts(9, n, k) == n // 16
+
+
+@pytest.mark.parametrize("m,n,k,paired,pays", [
+    (48, 8192, 4096, True, True), (64, 28672, 4096, True, True),
+    (69, 6144, 2048, True, False), (96, 13824, 16384, True, False),
+    (96, 2464, 4096, True, False), (135, 4288, 6144, True, False),
+    (48, 36864, 2048, True, False), (20, 32000, 2048, False, True),
+    (24, 27648, 8192, False, True), (20, 16384, 8192, False, False),
+    (20, 57344, 8192, False, False), (64, 33328, 2048, False, False),
+    (64, 128256, 4096, False, True)])
+def test_rows_that_meet_in_memory(m, n, k, paired, pays):
+    """Rows of a multiple of 4 KB leave the library where that was measured to
+    be the faster way, and not at its edges."""
+    assert _C.mid_gemm_good(m, n, k, paired) == pays
