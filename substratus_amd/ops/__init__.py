@@ -639,6 +639,7 @@ def linear_added_norm(x: torch.Tensor, weight: torch.Tensor,
     workgroups share the product's sums, which the norm adds up."""
     few = _few_rows(x, weight, bias, False, True)
     if few is None or x.dim() != 2 or x.device != h.device \
+            or bias is not None and bias.data_ptr() % 16 \
             or not may_add(h, norm, x.shape[0], weight.shape[0]):
         return None
     total, rows = torch.empty_like(h), torch.empty_like(h)

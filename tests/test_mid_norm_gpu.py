@@ -54,3 +54,22 @@ def test_refused():
     assert lin.added_norm(x[:64], h[:128:2], w, 1e-5) is None
     with torch.enable_grad():
         assert lin.added_norm(x[:64], h[:64], w.requires_grad_(), 1e-5) is None
+
+
+@torch.no_grad()
+def test_bias_between_boundaries():
+    """Part of a larger tensor: the norm reads four numbers at a time, and the
+    product with a norm of its own takes any."""
+    torch.manual_seed(3)
+    lin, w = made("dense", 4096, 4096, True)
+    x, h = (torch.randn(64, 4096, device=DEV).bfloat16() for _ in range(2))
+    norm = torch.ones(4096, device=DEV).bfloat16()
+    parts = torch.randn(4097, device=DEV).bfloat16()
+    lin.bias = torch.nn.Parameter(parts[1:], requires_grad=False)
+    assert lin.bias.data_ptr() % 16
+    assert lin.added_norm(x, h, norm, 1e-5) is None
+    want = x.double() @ w.T + parts[1:].double()
+    assert float((lin(x).double() - want).norm()) <= \
+        2.0 ** -8 * float(want.norm())
+    lin.bias = torch.nn.Parameter(parts[:-1], requires_grad=False)
+    assert lin.added_norm(x, h, norm, 1e-5) is not None
