@@ -377,9 +377,9 @@ class CausalLM(nn.Module):
         # each block's outputs are added to the residual stream inside the
         # NEXT norm
         deltas = ()
-        norms = [getattr(blk, "norm1", None) for blk in self.blocks[1:]]
+        norms = [getattr(blk, "norm1", None) for blk in self.blocks]
         for blk, after, (kc, vc) in zip(
-                self.blocks, [*norms, self.final_norm], kv_caches):
+                self.blocks, [*norms[1:], self.final_norm], kv_caches):
             h, deltas = yield from blk.decode_ops(h, deltas, positions, kc,
                                                   vc, slots, block_table,
                                                   seq_lens, after)

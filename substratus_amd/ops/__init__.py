@@ -614,10 +614,11 @@ def linear_added(x: torch.Tensor, weight: torch.Tensor,
     """(h + F.linear, RMSNorm of that by the weight norm, undivided) in one
     kernel, or None where it is not made for that. Up to 16 rows: with more of
     them the products that would take such rows are other kernels'."""
-    few = _few_rows(x, weight, bias, False)
-    if few is None or x.dim() != 2 or x.shape[0] > 16 \
-            or x.device != h.device \
+    if x.dim() != 2 or x.shape[0] > 16 or x.device != h.device \
             or not may_add(h, norm, x.shape[0], weight.shape[0]):
+        return None
+    few = _few_rows(x, weight, bias, False)
+    if few is None:
         return None
     total, parts = room_for_added(h, few[1].rows_added_parts(
         x.shape[0], *weight.shape))
@@ -637,10 +638,11 @@ def linear_added_norm(x: torch.Tensor, weight: torch.Tensor,
                       ) -> Optional[tuple[torch.Tensor, Normed]]:
     """(h + F.linear, RMSNorm of that by the weight norm), or None: where
     workgroups share the product's sums, which the norm adds up."""
+    if x.dim() != 2 or x.shape[0] <= 16 or x.device != h.device \
+            or bias is not None and bias.data_ptr() % 16:
+        return None
     few = _few_rows(x, weight, bias, False, True)
-    if few is None or x.dim() != 2 or x.device != h.device \
-            or bias is not None and bias.data_ptr() % 16 \
-            or not may_add(h, norm, x.shape[0], weight.shape[0]):
+    if few is None or not may_add(h, norm, x.shape[0], weight.shape[0]):
         return None
     total, rows = torch.empty_like(h), torch.empty_like(h)
     few[1].mid_normed(rows, total, few[0], weight, bias, h, norm, eps)
