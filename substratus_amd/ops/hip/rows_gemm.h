@@ -288,7 +288,7 @@ DEV_INLINE float silu_times(float g, float u) {
 }
 
 // One of a row's 16 columns that a workgroup adds, the others in the lanes beside
-// it (past the last one h, weight and v are 0).
+// it (past the last one h and v are 0).
 DEV_INLINE void finish_added(const AddTo& add, bf16_t* y, long at, int r,
                              bool there, float h, float weight, float v) {
   const float s = bf2f(f2bf(h + bf2f(f2bf(v))));

@@ -330,10 +330,10 @@ void launch_rows_gemm(bf16_t* y, const bf16_t* x, const bf16_t* w,
       if (heads) kernel = rows_gemm_kernel<Columns::HEADS, N, F, S, T, X>;
       else if (gated) kernel = rows_gemm_kernel<Columns::GATED, N, F, S, T, X>;
     }
-    if constexpr (!N) {
+    if constexpr (!N)
       if (gelu) kernel = rows_gemm_kernel<Columns::GELU, N, F, S, T, X>;
+    if constexpr (!N && F == 1)
       if (add) kernel = rows_gemm_kernel<Columns::ADDED, N, F, S, T, X>;
-    }
     if constexpr (!N && !T && F == 1)
       if (!(heads || gated || gelu) && rows_gemm_spreads(n, k))
         kernel = add ? rows_gemm_kernel<Columns::ADDED, N, F, S, T, X, true>

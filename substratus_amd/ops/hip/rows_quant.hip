@@ -525,7 +525,6 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
 
 }  // namespace
 
-// Blocks whose scales come in pairs (k a multiple of 64), or of 256.
 // Whether a workgroup has eight weight rows instead of 16: where some CUs would have
 // two workgroups and others one, all have two or three half as large. Rows shorter
 // than 4096 are read too soon for that to matter, and x, which is read once more,
@@ -544,6 +543,7 @@ bool rows_quant_thin(int m, int n, int k, Quant q, bool paired) {
          q != Quant::Q6_K && (m > 1 || q != Quant::Q8_0);
 }
 
+// Blocks whose scales come in pairs (k a multiple of 64), or of 256.
 bool rows_quant_takes(int m, int n, int k, Quant q, bool gated) {
   const int step = q == Quant::Q4_K || q == Quant::Q6_K ? 256 : 64;
   return m >= 1 && m <= 64 && n >= 1 && k >= step && k % step == 0 &&
@@ -564,10 +564,12 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
     constexpr int ROWS = THIN ? 8 : 16;
     const dim3 grid((n + ROWS - 1) / ROWS, (m + MR - 1) / MR),
         block(KW * WAVE);
-    auto kernel = add ? rows_quant_kernel<QQ, MR, ME, KW, P, Columns::ADDED,
-                                          false, THIN>
-                      : rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN,
-                                          false, THIN>;
+    auto kernel = rows_quant_kernel<QQ, MR, ME, KW, P, Columns::PLAIN, false,
+                                    THIN>;
+    if constexpr (MR <= 8)
+      if (add)
+        kernel = rows_quant_kernel<QQ, MR, ME, KW, P, Columns::ADDED, false,
+                                   THIN>;
     if constexpr (!THIN) {
       auto pick = [&](auto normed) {
         constexpr bool N = decltype(normed)::value;
