@@ -83,7 +83,7 @@ def passes(name, how, quant, rows):
 @pytest.mark.parametrize("quant", ["", "q4_0"])
 @pytest.mark.parametrize("how", ["hook", "subclass", "instance", "adapter"])
 @pytest.mark.parametrize("name", ["wqkv", "w_gateup", "lm_head", "norm2",
-                                  "final_norm"])
+                                  "final_norm", "wo", "w_down", "norm1"])
 @torch.no_grad()
 def test_called(name, how, quant):
     if how == "adapter" and "norm" in name:

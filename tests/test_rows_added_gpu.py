@@ -2,10 +2,13 @@
 follows, and products of such rows, which end it: against 64 bits and against the
 product, the sum, the norm and the product one after the other."""
 
+from dataclasses import replace
+
 import pytest
 import torch
 
 from substratus_amd import ops
+from substratus_amd.models import CausalLM, get_config
 from tests.test_rows_normed_gpu import DEV, made
 
 pytestmark = pytest.mark.gpu
@@ -104,3 +107,47 @@ def test_refused():
     assert odd.added(x[:2], h[:2, :72].contiguous(), w[:72]) is None
     with torch.enable_grad():
         assert lin.added(x[:2], h[:2], w.requires_grad_()) is None
+
+
+# a head with more columns than it divides rows for, from 9 rows on; tied
+# embeddings, whose product is torch's; rows of either kernel and a norm's own
+@pytest.mark.parametrize("vocab,tied", [(65600, False), (512, True),
+                                        (512, False)])
+@pytest.mark.parametrize("rows", [1, 8, 12, 16, 40])
+@torch.no_grad()
+def test_last_norm(vocab, tied, rows, monkeypatch):
+    """Logits of a step whose last rows come undivided, beside those of a step
+    that adds and norms by itself."""
+    cfg = replace(get_config("llama-tiny"), vocab_size=vocab, num_layers=2,
+                  intermediate_size=8192, tie_word_embeddings=tied)
+    model = CausalLM(cfg, device=DEV, dtype=torch.bfloat16)
+    model.init_random(3)
+    d = cfg.head_dim
+    at = torch.arange(rows, device=DEV, dtype=torch.int32)
+    tokens = torch.randint(0, vocab, (rows,), device=DEV)
+
+    def step():
+        caches = [tuple(torch.zeros(rows, model.n_kv_heads, 16, d,
+                                    device=DEV).bfloat16() for _ in range(2))
+                  for _ in model.blocks]
+        return model.forward_decode(
+            tokens, torch.zeros_like(at), caches, at * 16,
+            at[:, None].contiguous(), torch.ones_like(at)).double()
+
+    kinds = []
+    for name in "linear_added", "linear_added_norm", "linear_scaled":
+        def spy(*a, name=name, run=getattr(ops, name), **kw):
+            got = run(*a, **kw)
+            kinds.append((name, got is not None))
+            return got
+        monkeypatch.setattr(ops, name, spy)
+    got = step()
+    assert (("linear_added", True) in kinds) == (rows <= 16)
+    assert (("linear_added_norm", True) in kinds) == (rows > 16)
+    if vocab > 65536:
+        assert (("linear_scaled", False) in kinds) == (9 <= rows <= 16)
+    for name in "linear_added", "linear_added_norm":
+        monkeypatch.setattr(ops, name, lambda *a: None)
+    want = step()
+    # rows are rounded to bf16 at another place: 2^-9 of each of some ten
+    assert float((got - want).norm()) <= 0.02 * float(want.norm())
