@@ -345,7 +345,7 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // narrow matrices (69 x 6144 x 2048 13.1 and 15.3, 96 x 13824 x 16384 118 and 137,
 // 96 x 2464 x 4096 12.8 and 16.3), and little more than 128 (135 x 4288 x 6144 29.2 and
 // 33.3): of 2206 products that a fifth more takes from it
-// 1413 stay so, 1.15 times as fast, six slower by more than 3 %, of the others 246
+// 1401 stay so, 1.15 times as fast, six slower by more than 3 %, of the others 246
 // would be. Up to 96 rows whose shares begin on whole
 // 4 KB of rows of a multiple of 16 KB stay with it: of 8192 x 8192 32 to 40 us either
 // way, of 128 rows 48, and 39 here. What nothing is shared of begins and ends 2 us

@@ -303,12 +303,16 @@ bool rows_gemm_thin(int m, int n, int k, bool paired) {
 }
 
 // Whether workgroups begin at different columns: all at the same they meet at few of
-// the memory's channels where rows are a multiple of 512 bytes. us: 8 x 4096 x 11008
-// 19.3 -> 17.4, 8 x 4096 x 8192 16.2 -> 13.7, 8 x 8192 x 8192 28.3 -> 25.4, 8 x 32000 x
-// 8192 95.9 -> 92.6; 1 x 9216 x 8448 30.8 -> 31.0. Longer rows are as fast or 1 to 2 %
-// slower (8 x 4096 x 14336 21.9 -> 22.3), and shorter ones gain less than the
-// arithmetic of the loads' addresses costs (a step of 8 rows and 8 layers of llama2-7b:
-// with all products like this 827 -> 837, with these alone 829 -> 816).
+// the memory's channels, of lengths that depend on how addresses are spread over them.
+// us: 8 x 4096 x 11008 19.3 -> 17.4, 8 x 4096 x 8192 16.2 -> 13.7, 8 x 8192 x 8192 28.3
+// -> 25.4, 8 x 32000 x 8192 95.9 -> 92.6; 1 x 9216 x 8448 30.8 -> 31.0. Against that
+// stands the arithmetic of the loads' addresses. Of 1, 4, 8 and 16 rows and 4096 columns
+// and more, at lengths of a multiple of 256, time with it over time without, on average
+// (least, most): up to 4096 1.010 (0.98, 1.05) of 261 products, to 8192 1.003 (0.96,
+// 1.04) of 160, in this range 0.965 (0.85, 1.03) of 88 (8192 0.91, 11008 0.94, of 49
+// others 1.002), to 16384 0.995 (0.94, 1.02) of 43, longer 0.967 (0.75, 1.04) of 70; of
+// other lengths 1.010 (0.88, 1.08) of 156. (A step of 8 rows and 8 layers of llama2-7b:
+// with all products like this 827 -> 837, with this range 829 -> 816.)
 static bool rows_gemm_spreads(int n, int k) {
   return n >= 4096 && k >= 8192 && k < 12288 && k % 256 == 0;
 }
