@@ -246,13 +246,14 @@ class QuantLinear(nn.Module):
         as a norm of its own or longer (two layers of 5120, q4_0: 16 rows 287
         us for 286, 40 rows 578 for 543; of 4096, q8_0: 6 rows 192 for 189)."""
         if self.bias is not None or not bare(self, QuantLinear) or \
+                not ops.inference_only(x) or \
                 x.dim() != 2 or x.dtype != torch.bfloat16 or \
                 x.shape[0] > (4 if self.quant == "q8_0" else 8) or \
                 x.device != h.device or x.shape[1] != self.in_features or \
                 not ops.may_add(h, norm, x.shape[0], self.out_features):
             return None
         ext = self._few_rows(x, False)
-        if ext is None or not ops.inference_only(x):
+        if ext is None:
             return None
         total, parts = ops.room_for_added(h, ext.quant_added_parts(
             x.shape[0], self.out_features, self.in_features, self.quant))

@@ -614,7 +614,9 @@ def linear_added(x: torch.Tensor, weight: torch.Tensor,
     """(h + F.linear, RMSNorm of that by the weight norm, undivided) in one
     kernel, or None where it is not made for that. Up to 16 rows: with more of
     them the products that would take such rows are other kernels'."""
-    if x.dim() != 2 or x.shape[0] > 16 or x.device != h.device \
+    # a compiler would hold the number of rows to a side of 16
+    if _compiling() or x.dim() != 2 or x.shape[0] > 16 \
+            or x.device != h.device \
             or not may_add(h, norm, x.shape[0], weight.shape[0]):
         return None
     few = _few_rows(x, weight, bias, False)
@@ -638,7 +640,8 @@ def linear_added_norm(x: torch.Tensor, weight: torch.Tensor,
                       ) -> Optional[tuple[torch.Tensor, Normed]]:
     """(h + F.linear, RMSNorm of that by the weight norm), or None: where
     workgroups share the product's sums, which the norm adds up."""
-    if x.dim() != 2 or x.shape[0] <= 16 or x.device != h.device \
+    if _compiling() or x.dim() != 2 or x.shape[0] <= 16 \
+            or x.device != h.device \
             or bias is not None and bias.data_ptr() % 16:
         return None
     few = _few_rows(x, weight, bias, False, True)

@@ -9,8 +9,10 @@ from torch.fx.experimental.symbolic_shapes import ShapeEnv
 from torch.overrides import TorchFunctionMode
 
 from substratus_amd import ops
+from substratus_amd.models.model import NormParams, added_product
+from substratus_amd.models.quant import QuantLinear
 from substratus_amd.ops import train
-from substratus_amd.parallel.tp import Linear
+from substratus_amd.parallel.tp import Linear, RowParallelLinear
 
 
 class Seen(TorchFunctionMode):
@@ -75,6 +77,31 @@ def test_compiled():
     want = train.silu_mul(ops.linear(x, w))
     got = torch.compile(fn, backend="eager", fullgraph=True)(x)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("quant", ["", "q8_0"])
+@torch.no_grad()
+def test_added_rows_are_not_counted(quant):
+    """One graph for a step of any number of rows."""
+    dtype = torch.bfloat16 if quant else torch.float32
+    lin = RowParallelLinear(64, 128, dtype=dtype)
+    torch.nn.init.normal_(lin.weight)
+    if quant:
+        lin = QuantLinear.from_linear(lin, quant)
+    norm = NormParams(128, True, dtype=dtype)
+    graphs = []
+
+    def fn(x, h):
+        return added_product(lin, x, h, norm, 1e-5)
+    compiled = torch.compile(
+        fn, backend=lambda graph, _: graphs.append(graph) or graph,
+        dynamic=True)
+    for rows in (3, 8, 12, 40, 300):
+        x, h = (torch.randn(rows, n).to(dtype) for n in (64, 128))
+        assert torch.equal(compiled(x, h)[1][0], fn(x, h)[1][0])
+        if rows == 3:
+            first = len(graphs)
+    assert len(graphs) == first
 
 
 @torch.no_grad()
