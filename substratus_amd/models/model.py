@@ -377,12 +377,11 @@ class CausalLM(nn.Module):
         # each block's outputs are added to the residual stream inside the
         # NEXT norm
         deltas = ()
-        norms = [getattr(blk, "norm1", None) for blk in self.blocks]
-        for blk, after, (kc, vc) in zip(
-                self.blocks, [*norms[1:], self.final_norm], kv_caches):
+        for blk, after, (kc, vc) in zip(self.blocks, self._norms_after(),
+                                        kv_caches):
             h, deltas = yield from blk.decode_ops(h, deltas, positions, kc,
                                                   vc, slots, block_table,
-                                                  seq_lens, after)
+                                                  seq_lens, *after)
             yield
         if self.lm_head is not None:
             got, deltas = scaled_product(self.lm_head, deltas, h,
@@ -393,6 +392,20 @@ class CausalLM(nn.Module):
             deltas = ()
         y, _ = fused_norm_residual(deltas, h, self.final_norm, self.eps)
         return self._logits(y)
+
+    def _norms_after(self) -> list[tuple]:
+        """For every block (the norm after it,), which its last product may
+        begin, or () where that block or the next one has a decode_ops of its
+        own, which knows nothing of it, or an eps of its own."""
+        def knows(blk):
+            return (blk is self or isinstance(blk, Block)
+                    and type(blk).decode_ops is Block.decode_ops
+                    and "decode_ops" not in blk.__dict__
+                    and not blk.parallel_attn)
+        blocks = [*self.blocks, self]
+        return [(nxt.final_norm if nxt is self else nxt.norm1,)
+                if knows(blk) and knows(nxt) and blk.eps == nxt.eps else ()
+                for blk, nxt in zip(blocks, blocks[1:])]
 
     def forward_decode(self, tokens: torch.Tensor, positions: torch.Tensor,
                        kv_caches: list[tuple[torch.Tensor, torch.Tensor]],
