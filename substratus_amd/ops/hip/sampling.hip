@@ -280,9 +280,9 @@ void softmax_sample_kernel(long* __restrict__ out,          // [B]
   const float inv_t = 1.f / temp;
   if (!usual) top = totals.most(wave_max(best));
   const float m = top * inv_t;
-  // NaN, and what went past the largest number beside the largest logit: 0. A
-  // logit below the largest may be equal to it once scaled (of neighbours in 32
-  // bits about a tenth are), and weighs as much then.
+  // NaN, and what went past the largest number beside the largest logit: 0. The
+  // difference to the largest is rounded once (rounded before it, about a tenth of
+  // neighbours in 32 bits would be equal, and thresholds not tell them apart).
   const float past = m == -INFINITY ? m : INFINITY;
   auto weight = [&](float v) {
     const float x = v * inv_t, below = __expf(fmaf(v, inv_t, -m));

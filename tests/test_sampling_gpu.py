@@ -108,6 +108,26 @@ def test_neighbouring_numbers_share_the_draws(temp, k, p):
         assert got.tolist() == [token] * n
 
 
+@pytest.mark.parametrize("temp", [0.6, 0.7, 0.9, 1.3])
+@pytest.mark.parametrize("vocab", [3000, 20000])
+def test_equal_once_scaled(temp, vocab):
+    """One token asked for is the larger of two logits that are a unit of the
+    last place apart, also where they are equal once scaled and rounded."""
+    n = 64
+    g = torch.Generator().manual_seed(1)
+    low = torch.rand(n, generator=g) * 25 + 5
+    top = torch.nextafter(low, torch.tensor(100.0))
+    inv = 1 / torch.tensor(temp)
+    assert int((low * inv == top * inv).sum()) > 0
+    rows = torch.full((n, vocab), -100.0)
+    rows[:, 17], rows[:, 2500] = low, top
+    of = lambda v, **how: torch.full((n,), v, device=DEV, **how)
+    for u in 0.0, 0.25, 0.75:
+        got = ops.softmax_sample(rows.to(DEV), of(temp),
+                                 of(1, dtype=torch.int32), of(1.0), of(u))
+        assert got.tolist() == [2500] * n
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("k,p", [(3, 1.0), (200, 1.0), (0, 0.6), (500, 0.97)])
 @pytest.mark.parametrize("kind", ["close", "equal", "steps", "below zero"])
