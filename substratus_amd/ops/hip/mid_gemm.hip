@@ -375,15 +375,18 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // A norm that adds up the shares saves a launch: 3.5 us of a product that would have
 // been this one's (64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
 // 256 x 4096 x 11008 47.2 -> 43.8; of 8070 of those widths none slower by more than
-// 1 %, 1.10 times as fast on average). For its sake products leave the library where
-// these estimates are near enough: not short ones of few columns and up to 128 rows
-// (80 x 2560 x 3584 12.5 -> 15.7, 100 x 2048 x 5632 15.3 -> 17.0; but 100 x 5120
-// x 4096 27.0 -> 21.2), nor of more rows than that where they are wide, narrow, short
-// or little more than 128 (211 x 5760 x 4480 31.7 -> 38.4, 217 x 2112 x 3200 16.2 ->
-// 18.4, 129 x 4544 x 6144 30.1 -> 34.9). Of 5053 products that 3.5 us more would take
-// from the library, 3540 are, 1.23 times as fast, six shapes of them slower by more
-// than 3 %, by 11 at most (of one inner size, 22016, and up to 32 rows, by 7: 83 ->
-// 89 us); of the others 266 would be, by up to 25.
+// 1 %, 1.10 times as fast on average). For its sake products leave the library, too,
+// from a product and a norm of its own, weights from memory: 96 x 4096 x 4096 25.8 ->
+// 19.2 us, 128 28.3 -> 21.3, 144 25.7 -> 21.5, 96 x 2048 x 5632 19.0 -> 14.2, 192 23.5
+// -> 19.2. But not of more than 64 rows where the estimates are not near enough: short
+// ones whose results are a round of the library's small tiles (69 x 2560 x 3072 13.7
+// -> 15.9, 104 x 1984 x 3840 14.8 -> 18.3), wide ones (68 x 11648 x 3712 37.3 -> 40.8,
+// 144 x 8640 x 6272 50.9 -> 65.0, 162 x 5120 x 8192 42.8 -> 45.3, 231 x 6656 x 12288
+// 86.5 -> 91.3), but for the longest, of which the library has few tiles (256 x 5632 x
+// 24576 292 -> 134). Of 6000 products that 3.5 us more would take from the library
+// 5383 are, 1.19 times as fast, 39 slower by more than 3 % (of 5000 others 4497, 1.19,
+// 30; most 5 to 10 %, a few of some 170 rows and 5500 columns up to 24: 179 x 5440 x
+// 3456 26.0 -> 34.3); of the rest 196 would be.
 bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
   if (m <= 16 || m > 256 || k < (paired ? 1024 : 2048) ||
       (m > 96 && n > 12288))
@@ -408,16 +411,18 @@ bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
   const long share = ((k + STEP - 1) / STEP + plan.splits - 1) / plan.splits;
   const bool in_step = !(paired || normed) && m <= 96 && k % 8192 == 0 &&
                        share % 32 == 0;
-  const bool saved = normed && plan.splits > 1 &&
-                     (m <= 64 || n >= 1536 || k > 4096);
   const double theirs = library * (longer ? 1.2 : 1.);
+  const bool tiles = n <= 2816 && k <= 4096 && m * n > 130000 && m * n <= 262144;
   const bool near =
-      m <= 64 ? true
-      : m <= 128 ? n <= 10240 && (k > 6144 || n > 4096 ||
-                                  (k > 5120 && n > 2048))
-                 : m > 144 && n > 2048 && n <= 5120 && k >= 3584;
-  const double saves = near ? 3.5 : m > 128 && k > 16384 ? theirs / 100 : 0.;
-  const double pass = saved ? saves
+      m <= 64 || k > 16384 ? true
+      : tiles              ? false
+      : m <= 128           ? n <= 10240
+      : k <= 4096          ? n <= 8192
+      : k <= 8448          ? n <= (m > 192 ? 8192 : 4096)
+                           : n <= 5120;
+  const bool saved = normed && near && plan.splits > 1 &&
+                     (m <= 64 || n >= 1536 || k > 4096);
+  const double pass = saved ? 3.5
                       : !paired ? 0. : n >= 4096 && k >= 2048 ? 2. : 1.;
   const double ours = plan.us * (in_step ? 1.25 : 1.) -
                       (plan.splits > 1 ? 0. : 2.);

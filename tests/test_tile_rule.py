@@ -49,11 +49,12 @@ def test_shares_in_step(m):
 
 @pytest.mark.parametrize("m,n,k,pays", [
     (64, 4096, 4096, True), (24, 8192, 28672, True),
-    (80, 2560, 3584, False), (100, 2048, 5632, False), (100, 5120, 4096, True),
-    (128, 5120, 5120, True), (128, 2048, 4096, False),
-    (129, 4544, 6144, False), (211, 5760, 4480, False),
-    (217, 2112, 3200, False), (254, 12288, 7584, False),
-    (256, 4096, 11008, True), (192, 4096, 4096, True)])
+    (69, 2560, 3072, False), (128, 2048, 4096, False), (65, 4096, 4096, True),
+    (128, 4096, 4096, True), (100, 5120, 4096, True), (128, 5120, 5120, True),
+    (100, 2048, 5632, True), (192, 2048, 5632, True), (192, 4096, 4096, True),
+    (129, 4544, 6144, False), (162, 5120, 8192, False),
+    (217, 2112, 3200, True), (254, 12288, 7584, False),
+    (256, 4096, 11008, True), (256, 5632, 24576, True)])
 def test_products_with_their_norm(m, n, k, pays):
     """Those that lost by it stay with the library and a norm of its own."""
     assert _C.mid_norm_good(m, n, k) == pays
