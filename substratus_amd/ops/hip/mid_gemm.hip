@@ -340,13 +340,15 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // longer at least, but for 256, which are whole tiles. Of rows of a multiple of 4 KB
 // it takes a fifth longer in paired products, as its CUs all read the same of the
 // memory's channels (64 x 28672 x 4096 54.4 us, and 45.9 here; 32 x 22016 x 4096 46.1,
-// and 37.0; 64 x 57344 x 8192 182 and 176), but for rows of a multiple of 32 KB (48 x
-// 8192 x 16384 62, and 70 here), and with more than 64 rows short and long ones, and
-// narrow matrices (69 x 6144 x 2048 13.1 and 15.3, 96 x 13824 x 16384 118 and 137,
-// 96 x 2464 x 4096 12.8 and 16.3), and little more than 128 (135 x 4288 x 6144 29.2 and
-// 33.3): of 2206 products that a fifth more takes from it
-// 1401 stay so, 1.15 times as fast, six slower by more than 3 %, of the others 246
-// would be. Up to 96 rows whose shares begin on whole
+// and 37.0; 64 x 57344 x 8192 182 and 176; 120 x 10880 x 8192 62.3 and 49.9; 151 x 6016
+// x 10240 92.8 and 61.4), but for rows of a multiple of 32 KB (48 x 8192 x 16384 62, and
+// 70 here), and with more than 64 rows the shortest and the longest (69 x 6144 x 2048
+// 13.1 and 15.3, 96 x 13824 x 16384 118 and 137), narrow matrices of few rows or
+// of short ones (96 x 2464 x 4096 12.8 and 16.3; but 108 x 2112 x 6144 38.9 and 19.7),
+// and of 129 to 192 rows widths whose second round of tiles is nearly empty (135 x 4288
+// x 6144 29.2 and 33.3, 132 x 4352 x 8192 35.2 and 40.2). Of 3700 products that a fifth more
+// would take from it 1003 stay, 470 slower by more than 3 % here; of the others 65 are,
+// and together they are 1.15 times as fast. Up to 96 rows whose shares begin on whole
 // 4 KB of rows of a multiple of 16 KB stay with it: of 8192 x 8192 32 to 40 us either
 // way, of 128 rows 48, and 39 here. What nothing is shared of begins and ends 2 us
 // sooner (55 x 11264 x 2048, gated: 16 us, the library 21).
@@ -367,11 +369,13 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // and 130, 20 x 28672 x 4096, gated, 56.7 and 47.3. More rows lose what there is to
 // gain (96 x 48000 x 6144 146 and 143), or are two blocks, which read the weights
 // twice (130 x 32000 x 4096 65 and 93). Nor are those of more than 32 rows whose
-// second round of 256 workgroups is all but empty (64 x 33328 x 2048 40.5 us, and 53.4
-// here; 48 x 36864 x 2048, gated, 41.7 and 46.3), and of rows of a multiple of 16 KB
-// others than a whole round (24 x 27648 x 8192 116 and 96, but 20 x 16384 x 8192 55 and
-// 62, 20 x 57344 x 8192 164 and 188). Of 2019 1788 stay, 1.19 times as fast, five
-// slower by more than 3 %, by 5 at most; of the others 67 were.
+// second round of 256 workgroups is all but empty, where rows are of 4 KB (64 x 33328 x
+// 2048 40.5 us, and 53.4 here; 48 x 36864 x 2048, gated, 41.7 and 46.3) or of more than
+// 16 (64 x 38272 x 10240 158 and 175; but 34 x 33216 x 4096 88.8 and 73.5, 57 x 37824 x
+// 8192 169 and 150), and of rows of 16 KB the narrowest and widest (24 x 27648 x 8192
+// 116 and 96, 20 x 22016 x 8192 87.3 and 70.3, but 32 x 16384 x 8192 55.8 and 58.0, 20 x
+// 57344 x 8192 164 and 188). Of 2100 products nine are slower by more than 3 %, by 7 at
+// most, and they are 1.18 times as fast; of the others 246 would be.
 // A norm that adds up the shares saves a launch: 3.5 us of a product that would have
 // been this one's (64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
 // 256 x 4096 x 11008 47.2 -> 43.8; of 8070 of those widths none slower by more than
@@ -392,17 +396,23 @@ bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
       (m > 96 && n > 12288))
     return false;
   if (m <= 64 && n >= 16000 && k % 2048 == 0 && k <= (paired ? 6144 : 12288) &&
-      !(m > 32 && n > 32768 && n <= 45056) &&
-      (k % 8192 != 0 || (n >= 24576 && n <= 32768)))
+      !(m > 32 && n > 32768 && n <= 45056 && (k == 2048 || k > 8192)) &&
+      (k != 8192 || (m <= 32 ? n > 16384 && n <= 32768
+                             : n >= 24576 && n <= 45056)))
     return true;
   if (!paired && k < 3072) return false;
   const double few = std::min(1., n / 4500.);
   const double inner = m > 128 ? 1.5e-3 + 1.7e-3 * few : .6e-3 + .6e-3 * few;
   const double work = n * k * 2 / 1e7 + k * inner + m * n * k * 2 / 2e9;
+  const bool round =
+      k <= 6144 ? m > 144 : n <= 5120 ? m > 192 : n > 6144 || m <= 160;
   const bool same = paired && k % 2048 == 0 &&
-                    (m <= 64 ? k % 16384 != 0
-                             : n > 2800 && k < 8192 && (k > 2048 || n > 8300) &&
-                                   (m <= 128 || m > 144));
+                    (m <= 64     ? k % 16384 != 0
+                     : n <= 2800 ? m > 96 && k > 4096 && k < 16384
+                     : n <= 8300 ? k > 2048 && k < 16384 &&
+                                       (m <= 128 || n <= 4096 || round)
+                     : m <= 128  ? k < 8192 || (n <= 12288 && k < 16384)
+                                 : m > 144 && k < 8192);
   const double library =
       (m > 128 ? 1. : 6.6) + work * (k % 256 ? 1.45 : same ? 1.2 : 1.);
   const bool longer = m > 32 && m < 256 && n <= 10240 &&

@@ -77,7 +77,11 @@ def test_eight_rows_of_weights(n, k, thin):
     (48, 36864, 2048, True, False), (20, 32000, 2048, False, True),
     (24, 27648, 8192, False, True), (20, 16384, 8192, False, False),
     (20, 57344, 8192, False, False), (64, 33328, 2048, False, False),
-    (64, 128256, 4096, False, True)])
+    (64, 128256, 4096, False, True), (20, 22016, 8192, False, True),
+    (34, 33216, 4096, False, True), (48, 36864, 6144, True, True),
+    (64, 40960, 10240, False, False), (120, 10880, 8192, True, True),
+    (108, 2112, 6144, True, True), (151, 6016, 10240, True, True),
+    (132, 4352, 8192, True, False), (230, 6144, 8192, True, False)])
 def test_rows_that_meet_in_memory(m, n, k, paired, pays):
     """Rows of a multiple of 4 KB leave the library where that was measured to
     be the faster way, and not at its edges."""
