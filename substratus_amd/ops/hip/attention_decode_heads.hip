@@ -80,6 +80,11 @@ DEV_INLINE float row_sum(float v) {
   return v;
 }
 
+// In which order workgroups go: every sequence's first head, and so on; a sequence's
+// heads; or its heads from another one on for each sequence.
+enum class Grid { SEQUENCES, HEADS, TURNED };
+
+// ordered: long sequences first where lengths are unlike
 template <int D, bool KV8, int WAVES>
 __global__ __launch_bounds__(WAVES * WAVE, 4)
 void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
@@ -89,19 +94,18 @@ void attn_heads_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit, bool turned, bool ordered,
+                       long q_ld, int nsplit, Grid from, bool ordered,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
-  // turned: workgroups take a sequence's heads in turn, the next sequence's from
-  // the next one on; or every sequence's first head, and so on
-  // ordered: long sequences first where lengths are unlike
   constexpr int LANES = D / 8;                   // of a row
   constexpr int ROWS = WAVE / LANES;             // of a piece of all lanes
   constexpr int KEYS = PIECES * ROWS;            // of a step
   constexpr int SIZE = KV8 ? 1 : 2;
-  const int bsz = turned ? gridDim.y : gridDim.x;
-  int b = turned ? blockIdx.y : blockIdx.x, split = blockIdx.z, at_lane = 0;
-  int head = turned ? (int)(blockIdx.x + blockIdx.y) % hq : blockIdx.y;
+  const bool sequences = from == Grid::SEQUENCES;
+  const int bsz = sequences ? gridDim.x : gridDim.y;
+  int b = sequences ? blockIdx.x : blockIdx.y, split = blockIdx.z, at_lane = 0;
+  int head = sequences ? blockIdx.y : blockIdx.x;
+  if (from == Grid::TURNED) head = (head + b) % hq;
   if (ordered) at_lane = length_at_lane(seq_lens, bsz);
   const int group = hq / hkv;
   int kvh = head / group;
@@ -334,26 +338,34 @@ void launch_attn_heads(bf16_t* out, const bf16_t* q, const void* kc,
                        hipStream_t stream) {
   // Workgroups go to the eighths of the chip in turn. Sequences first, a sequence's
   // heads come to the same eighth where there is a multiple of eight of them: keys
-  // that heads share, and their pages' addresses, come to its caches once. Heads
-  // first, an eighth reads its own eighth of all pages, and meets the others at few
-  // of the memory's channels where lengths are equal; turned by the sequence it does
-  // not, and a long sequence has all of the chip. So turned where heads share no keys
-  // and there are more than the chip holds at a time (four a CU). us, MI355X,
-  // sequences first, heads first, turned; keys from a quarter of the most to all, all
-  // of them, one of them (the others' a twentieth):
+  // that heads share, and their pages' addresses, come to its caches once, but where
+  // lengths are unlike the eighths are, too. Heads first, an eighth reads its own
+  // eighth of all pages, and meets the others at few of the memory's channels where
+  // lengths are equal; turned by the sequence it does not, and a long sequence has all
+  // of the chip. So heads are first where they share no keys, and turned where there
+  // are more than the chip holds at a time (four a CU). us, MI355X, sequences first,
+  // heads first, turned; keys from a quarter of the most to all, all of them, one of
+  // them (the others' a twentieth):
   //   sequences x heads x keys      unlike         all            one (2500)
   //   512 x 32 x 516                             698  764  660
   //   256 x 32 x 516                             387  348  327
   //   64 x 32 x 1500             168  157  158   250  259  239   118   48   48
   //   256 x 12 x 1500 of 64      119  117  117   173  175  174    55   29   29
   //   64 x 16 x 1500 of 64      47.1 44.5 43.8                    51   32   32
-  //   86 x 12 x 1500 of 64      42.6      44.5  67.2      68.2
-  //   16 x 32 x 900 (not turned) 35.6     37.2  31.4      31.3 (516)
-  //   64 x 71 on 1 x 516, fp8 (not turned)      33.7 37.3
+  //   20 x 32 x 900             39.1 35.7 35.7  52.9 51.6 52.5
+  //   8 x 32 x 2000             36.0 35.4 35.5  45.4 45.9 46.0
+  //   8 x 40 x 2000             46.9 44.8 44.8  57.5 57.7 57.7
+  //   64 x 71 on 1 x 516, fp8                   33.7 37.3
+  // Shares come last: behind each sequence's heads, those of a table's unused room are
+  // between those that have keys (4 x 32 x 60 in a table of 4096 6.3 -> 7.9; 4 x 32 x
+  // 2000 unlike 21.1 -> 20.2).
   // Long sequences before short ones, heads first then (attention_order.h): 30 x 40
   // x 1100 unlike 74.7 -> 70.5, 64 x 71 on 1 x 1500, fp8, unlike 71.1 -> 61.5.
-  const bool turned = hq == hkv && (long)bsz * hq >= 1024 && bsz <= MOST;
-  const dim3 grid = turned ? dim3(hq, bsz, nsplit) : dim3(bsz, hq, nsplit);
+  const Grid from = hq != hkv || bsz > MOST ? Grid::SEQUENCES
+                    : (long)bsz * hq < 1024 ? Grid::HEADS
+                                            : Grid::TURNED;
+  const dim3 grid = from == Grid::SEQUENCES ? dim3(bsz, hq, nsplit)
+                                            : dim3(hq, bsz, nsplit);
   const bool ordered = orders_sequences(bsz, max_blocks, nsplit,
                                         (long)bsz * hq * nsplit, 16 / waves);
   auto go = [&](auto dim, auto fp8, auto w) {
@@ -362,7 +374,7 @@ void launch_attn_heads(bf16_t* out, const bf16_t* q, const void* kc,
         <<<grid, dim3(W * WAVE), 0, stream>>>(
             out, q, reinterpret_cast<const char*>(kc),
             reinterpret_cast<const char*>(vc), block_table, seq_lens, hq, hkv,
-            max_blocks, scale, q_ld, nsplit, turned, ordered, part_o, part_ml);
+            max_blocks, scale, q_ld, nsplit, from, ordered, part_o, part_ml);
   };
   auto sized = [&](auto dim, auto fp8) {
     if (waves == 8) go(dim, fp8, std::integral_constant<int, 8>());
