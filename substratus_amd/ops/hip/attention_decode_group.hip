@@ -68,7 +68,7 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
                        const int* __restrict__ block_table,  // [B, max_blocks]
                        const int* __restrict__ seq_lens,
                        int hq, int hkv, int max_blocks, float scale,
-                       long q_ld, int nsplit, bool ordered,
+                       long q_ld, int nsplit, bool turned, bool ordered,
                        float* __restrict__ part_o,   // [B, HQ, NS, D]
                        float* __restrict__ part_ml) {  // [B, HQ, NS, 2]
   constexpr int RC = D / 8;                      // 16-byte pieces of a row
@@ -82,6 +82,10 @@ void attn_group_kernel(bf16_t* __restrict__ out,             // [B, HQ, D]
 
   const int in_group = hq / hkv, parts = (in_group + 15) / 16;
   int b = blockIdx.x, part = blockIdx.y, split = blockIdx.z, n;
+  if (turned) {                   // (no more groups than sequences)
+    b += part;
+    if (b >= (int)gridDim.x) b -= gridDim.x;
+  }
   if (ordered) {
     const int bsz = gridDim.x, at_lane = length_at_lane(seq_lens, bsz);
     if (unlike_lengths(at_lane, max_blocks * PAGE)) {
@@ -315,8 +319,14 @@ void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
   // attention_decode_heads.hip; us, 71 heads on 1, 200 x 516 keys, heads first 31.4,
   // now 23.8; 64 x 32 on 8 x 1500, all of them, 83 and 76.5). Where a part is all of
   // a group, long sequences before short ones, heads first then: 32 on 8, unlike, 64
-  // x 2500 89.6 -> 80.8, 40 x 2000 55.8 -> 49.4.
+  // x 2500 89.6 -> 80.8, 40 x 2000 55.8 -> 49.4. And groups begin at sequences of
+  // their own then, where these are a multiple of eight: an eighth of the chip would
+  // have all groups of the same ones, and eighths with long ones end last. 32 on 8,
+  // unlike, 24 x 2500 46.6 -> 43.9, 40 x 2500 69.0 -> 65.2, 48 x 2500 80.8 -> 73.0, 72 x
+  // 2500 113.9 -> 103.9, 104 x 1500 95.5 -> 91.8; 16 x 2500 30.1 -> 31.3, so not of so
+  // few; all of them 40 x 100 12.7 -> 13.2, longer ones the same.
   const dim3 grid(bsz, hkv * parts, nsplit), block(NW * WAVE);
+  const bool turned = parts == 1 && bsz % 8 == 0 && bsz > 16 && bsz >= hkv;
   const bool ordered =
       parts == 1 && orders_sequences(bsz, max_blocks, nsplit,
                                      (long)bsz * hkv * nsplit,
@@ -324,10 +334,10 @@ void launch_attn_group(bf16_t* out, const bf16_t* q, const bf16_t* kc,
   if (d == 128) {
     attn_group_kernel<128><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, ordered, part_o, part_ml);
+        q_ld, nsplit, turned, ordered, part_o, part_ml);
   } else {
     attn_group_kernel<64><<<grid, block, 0, stream>>>(
         out, q, kc, vc, block_table, seq_lens, hq, hkv, max_blocks, scale,
-        q_ld, nsplit, ordered, part_o, part_ml);
+        q_ld, nsplit, turned, ordered, part_o, part_ml);
   }
 }

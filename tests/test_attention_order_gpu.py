@@ -59,7 +59,10 @@ def check(batch, hq, hkv, d, room, lens, g):
 @pytest.mark.parametrize("batch,hq,hkv,d,room,most", [
     (40, 32, 8, 128, 256, 2000), (33, 128, 8, 64, 256, 4096),
     (64, 32, 8, 128, 157, 961), (64, 32, 8, 128, 256, 960),
-    (40, 71, 71, 64, 300, 1500), (64, 71, 1, 64, 120, 1900)])
+    (40, 71, 71, 64, 300, 1500), (64, 71, 1, 64, 120, 1900),
+    (16, 32, 8, 128, 40, 600), (24, 32, 8, 128, 157, 1500),
+    (24, 192, 24, 64, 20, 300), (24, 200, 25, 64, 20, 300),
+    (32, 128, 32, 128, 20, 300)])
 @torch.no_grad()
 def test_shares_in_order(batch, hq, hkv, d, room, most):
     g = torch.Generator().manual_seed(batch + d)
