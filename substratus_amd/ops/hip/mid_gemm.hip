@@ -374,8 +374,10 @@ MidPlan mid_gemm_plan(long m, long n, long k) {
 // 16 (64 x 38272 x 10240 158 and 175; but 34 x 33216 x 4096 88.8 and 73.5, 57 x 37824 x
 // 8192 169 and 150), and of rows of 16 KB the narrowest and widest (24 x 27648 x 8192
 // 116 and 96, 20 x 22016 x 8192 87.3 and 70.3, but 32 x 16384 x 8192 55.8 and 58.0, 20 x
-// 57344 x 8192 164 and 188). Of 2100 products nine are slower by more than 3 %, by 7 at
-// most, and they are 1.18 times as fast; of the others 246 would be.
+// 57344 x 8192 164 and 188; of 33 to 64 rows the last alone take 175 to 179 either way,
+// and steps of llama2-70b are 2 to 3 % shorter with it: 40 rows 990 -> 955). Of 2100
+// products 22 are slower by more than 3 %, by 7 at most, and they are 1.17 times as
+// fast; of the others 233 would be.
 // A norm that adds up the shares saves a launch: 3.5 us of a product that would have
 // been this one's (64 x 4096 x 4096 16.1 -> 13.8 us, 64 x 4096 x 14336 37.1 -> 33.9,
 // 256 x 4096 x 11008 47.2 -> 43.8; of 8070 of those widths none slower by more than
@@ -398,7 +400,7 @@ bool mid_gemm_pays(long m, long n, long k, bool paired, bool normed) {
   if (m <= 64 && n >= 16000 && k % 2048 == 0 && k <= (paired ? 6144 : 12288) &&
       !(m > 32 && n > 32768 && n <= 45056 && (k == 2048 || k > 8192)) &&
       (k != 8192 || (m <= 32 ? n > 16384 && n <= 32768
-                             : n >= 24576 && n <= 45056)))
+                             : n >= 24576 && n <= 57344)))
     return true;
   if (!paired && k < 3072) return false;
   const double few = std::min(1., n / 4500.);

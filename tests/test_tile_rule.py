@@ -78,6 +78,7 @@ def test_eight_rows_of_weights(n, k, thin):
     (24, 27648, 8192, False, True), (20, 16384, 8192, False, False),
     (20, 57344, 8192, False, False), (64, 33328, 2048, False, False),
     (64, 128256, 4096, False, True), (20, 22016, 8192, False, True),
+    (40, 57344, 8192, False, True), (40, 65024, 8192, False, False),
     (34, 33216, 4096, False, True), (48, 36864, 6144, True, True),
     (64, 40960, 10240, False, False), (120, 10880, 8192, True, True),
     (108, 2112, 6144, True, True), (151, 6016, 10240, True, True),
