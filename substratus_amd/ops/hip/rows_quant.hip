@@ -27,7 +27,16 @@
 // stage is 256 columns; weights, scales and x go straight to LDS with
 // consecutive lanes on consecutive bytes (see rows_gemm.hip), pieces permuted
 // by the row against bank conflicts. Few rows of x: P stages in flight per
-// wave; many: one, and more workgroups per CU instead.
+// wave; many: one, and more workgroups per CU instead. A single row of x comes as
+// such: with three more of no use, stages took half as much LDS again, and two of
+// them in flight left a CU fewer workgroups. us of 15360 x 5120, 5120 x 5120, 27648
+// x 5120, 5120 x 13824, 12288 x 4096, 22016 x 4096, 32000 x 5120, each from memory,
+// four rows (q4_0 and q6_K: four waves, one stage in flight, of wide matrices) ->
+// one (eight waves, of q4_0 two stages):
+//   q4_0  13.8 6.8 22.5 13.8 9.2 15.3 27.8 -> 13.5 6.5 22.4 12.9 8.2 14.8 26.3
+//   q4_K  14.5 7.5 25.5 15.6 9.0 16.4 28.8 -> 14.2 6.8 24.2 15.3 8.8 15.2 27.9
+//   q6_K  20.7 10.7 33.7 26.8 12.6 22.6 37.0 -> 20.0 10.9 33.6 27.1 12.1 21.1 36.6
+// and of a captured step of 8 layers of 5120, q4_0, 523 -> 503.
 // A load takes 8 rows x 128 bytes of weights, where 16 x 64 asked for every
 // line twice. q6_K keeps the halves: a row is half a line more than whole ones,
 // and what a stage asks for is four kinds of pieces, of which two are less than
@@ -181,11 +190,12 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                           Q != Quant::Q6_K));
   constexpr int HALVES = THIN ? 2 : 1, XW = 2 * HALVES;
   constexpr int FM = (MR + 15) / 16;
-  // loads of x, 4 rows x 256 B, XW to a row (normed x does not go through the
-  // ring)
-  constexpr int XL = NORM ? 0 : MR / 4 * XW;
+  // loads of x, 4 rows x 256 B, XW to a row, or all of a single row (normed x
+  // does not go through the ring)
+  constexpr bool ONE = ME == 1 && !NORM;
+  constexpr int XL = NORM ? 0 : ONE ? 1 : MR / 4 * XW;
   constexpr int WS = L::W * TILE + L::S * 16;    // weights and scales
-  constexpr int STAGE = XL * 64 + WS;
+  constexpr int STAGE = (ONE ? HALVES * 32 : XL * 64) + WS;
   constexpr int LOADS = XL + L::LOADS;
   constexpr int BM = FM * 16, PAD = 1;
   constexpr int RED = (KW * BM * (16 + PAD) + 3) / 4, RING = KW * P * STAGE;
@@ -233,10 +243,11 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   const unsigned char* dp = sc + weight_row<C>(n0, lo_w, n, half) * sb;
   const char* xp[XL / XW + 1];
   #pragma unroll
-  for (int d = 0; d < XL / XW; ++d)
+  for (int d = 0; d < (ONE ? 1 : XL / XW); ++d)
     xp[d] = reinterpret_cast<const char*>(
         x + (long)min(d * 4 + (lane >> 4), m - 1) * k);
-  unsigned short dreg[P];                        // q6_K: the stage's d
+  static_assert(P == 1 || Q != Quant::Q6_K);
+  unsigned short dreg;                           // q6_K: the stage's d
   // the 256 columns that a stage's half has, or the last ones again
   auto of_stage = [&](int c, int h) {
     return THIN ? min(c * 2 + h, k / 256 - 1) : c;
@@ -280,9 +291,15 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       load_to_lds<16>(wp + k / 2 + c * 64 + piece * 16, ws + 2 * TILE);
       load_to_lds<4>(wp + k / 4 * 3 + c * 16 + word * 4, ss);
       // two bytes only: words need not be aligned
-      dreg[s] = *reinterpret_cast<const unsigned short*>(dp + c * 2);
+      dreg = *reinterpret_cast<const unsigned short*>(dp + c * 2);
     }
     uint4v* xs = ws + WS;
+    if constexpr (ONE) {
+      const int p = c * HALVES * 32 + (lane ^ (lane >> 5) * 4);
+      if (THIN || lane < 32)
+        load_to_lds<16>(xp[0] + (long)min(p, k / 8 - 1) * 16, xs);
+      return;
+    }
     #pragma unroll
     for (int d = 0; d < XL; ++d) {
       const int p = (c * XW + d % XW) * 16 +
@@ -299,10 +316,16 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
   #pragma unroll
   for (int j = 0; j < FM; ++j) {
     const int r = (j * 16 + lo) & (MR - 1);
-    xr[j] = (r >> 2) * (XW * 64) + lo_up * 128 + (r & 3) * 16;
+    xr[j] = ONE ? lo_up * 32 : (r >> 2) * (XW * 64) + lo_up * 128 + (r & 3) * 16;
   }
-  const int xsw = ((lo & 3) << 2) ^
-                  (((lo & (MR > 16 ? 15 : MR - 1)) >> 2) & 3);
+  const int xsw = ONE ? lo_up * 4
+                      : ((lo & 3) << 2) ^
+                            (((lo & (MR > 16 ? 15 : MR - 1)) >> 2) & 3);
+  // piece i of block b of a row
+  auto x_at = [&](int b, int i) {
+    return ONE ? (b * 4 + i) ^ xsw
+               : (b >> 2) * 64 + (((b * 4 + i) & 15) ^ xsw);
+  };
   const int wsw = Q == Quant::Q6_K ? lo >> 2 : lo >> 1;
   const uint4v* x_row = s_x + min(lo & (MR - 1), m - 1) * (k / 8 + 1);
   float4v acc[FM];
@@ -321,7 +344,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
       d = half_of(dd) / L::TIMES;
       dm = -half_of(dd >> 16);
     }
-    if constexpr (Q == Quant::Q6_K) d = half_of(dreg[s]) / L::TIMES;
+    if constexpr (Q == Quant::Q6_K) d = half_of(dreg) / L::TIMES;
     // the lane's eight weights of a block, k = 8 g on, out of eight bytes
     auto weights = [&](int b) {
       const int at = Q == Quant::Q4_0 ? b & 3
@@ -363,8 +386,7 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
           for (int t = 0; t < 2; ++t) {
             const short8 xv = __builtin_bit_cast(
                 short8, NORM ? x_row[c * 32 + (b + t) * 4 + g]
-                             : xs[xr[j] + (b >> 2) * 64 +
-                                  ((((b + t) * 4 + g) & 15) ^ xsw)]);
+                             : xs[xr[j] + x_at(b + t, g)]);
             p[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, wv[t], zero, 0,
                                                            0, 0);
             if constexpr (Q == Quant::Q4_K)
@@ -399,12 +421,11 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
               (sv[si >> 2] >> (8 * (si & 3))) & 0xff);
           #pragma unroll
           for (int j = 0; j < FM; ++j) {
-            const int p = b * 4 + h * 2 + (g >> 1);
+            const int i = h * 2 + (g >> 1);
             const short4v xv = __builtin_bit_cast(
                 short4v, reinterpret_cast<const uint2v*>(
-                    NORM ? x_row + c * 32 + p
-                         : xs + xr[j] + (p >> 4) * 64 +
-                               ((p & 15) ^ xsw))[g & 1]);
+                    NORM ? x_row + c * 32 + b * 4 + i
+                         : xs + xr[j] + x_at(b, i))[g & 1]);
             add_scaled<ME>(acc[j], scale,
                            __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
                                xv, wv, zero, 0, 0, 0));
@@ -445,27 +466,47 @@ void rows_quant_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
     lds_barrier();
   }
   int i = 0;
-  for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
-    #pragma unroll
-    for (int s = 0; s < P; ++s) {
+  if constexpr (ONE) {
+    // places of the ring by number: unrolled, addresses in LDS take registers, ten
+    // more than there are of two stages of q4_0
+    int slot = 0;
+    auto on = [&]() { slot = slot + 1 == P ? 0 : slot + 1; };
+    #pragma unroll 1
+    for (; i + P < steps; ++i, on()) {      // P stages in flight throughout
       wait_loads<(P - 1) * LOADS>();
-      use(s, c0 + i + s, integral_constant<bool, true>{});
+      use(slot, c0 + i, integral_constant<bool, true>{});
       wait_lds_reads();
-      load(s, c0 + i + s + P);
+      load(slot, c0 + i + P);
     }
-  }
-  for (; i < steps; i += P) {               // the ring runs dry
-    #pragma unroll
-    for (int s = 0; s < P; ++s)
-      if (i + s < steps) {
-        if (i + s + P <= steps) wait_loads<(P - 1) * LOADS>();
-        else wait_loads<0>();
-        use(s, c0 + i + s, integral_constant<bool, K_QUANT && !THIN>{});
-        if (i + s + P < steps) {
-          wait_lds_reads();
-          load(s, c0 + i + s + P);
-        }
+    #pragma unroll 1
+    for (; i < steps; ++i, on()) {          // the ring runs dry
+      if (P > 1 && i + P == steps) wait_loads<(P - 1) * LOADS>();
+      else wait_loads<0>();
+      use(slot, c0 + i, integral_constant<bool, K_QUANT && !THIN>{});
+    }
+  } else {
+    for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
+      #pragma unroll
+      for (int s = 0; s < P; ++s) {
+        wait_loads<(P - 1) * LOADS>();
+        use(s, c0 + i + s, integral_constant<bool, true>{});
+        wait_lds_reads();
+        load(s, c0 + i + s + P);
       }
+    }
+    for (; i < steps; i += P) {               // the ring runs dry
+      #pragma unroll
+      for (int s = 0; s < P; ++s)
+        if (i + s < steps) {
+          if (i + s + P <= steps) wait_loads<(P - 1) * LOADS>();
+          else wait_loads<0>();
+          use(s, c0 + i + s, integral_constant<bool, K_QUANT && !THIN>{});
+          if (i + s + P < steps) {
+            wait_lds_reads();
+            load(s, c0 + i + s + P);
+          }
+        }
+    }
   }
   __syncthreads();
 
@@ -630,10 +671,13 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
         }
       }
     } else if (m == 1) {
-      if constexpr (QQ != Quant::Q8_0) {
-        // q4_0, 4096 x 11008: one stage in flight 11.5 us, two 9.6
-        if (few) go(qc, c4, c1, waves, one_row, no);
-        else go(qc, c4, c1, c4, some, no);
+      // Eight waves of a row, two stages in flight in each: all of rows of 4096
+      // at once, which q4_K's is slower for where workgroups are many.
+      if constexpr (QQ == Quant::Q4_K) {
+        if (few || k > 4096) go(qc, c4, c1, c8, one_row, no);
+        else go(qc, c4, c1, c4, one_row, no);
+      } else if constexpr (QQ != Quant::Q8_0) {
+        go(qc, c4, c1, c8, one_row, no);
       }
     } else if (m <= 4) {
       if (few) go(qc, c4, c4, waves, some, no);

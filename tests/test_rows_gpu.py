@@ -162,6 +162,34 @@ def test_quant_rows(quant, m, n, k):
                      + 2.0 ** -6 * room.mean()).all())
 
 
+# A single row, whose stages hold nothing of other rows: eight waves with none to
+# five stages each, two in flight, a last one in part; workgroups of eight weight
+# rows, whose stages are 512 columns, a last one of half or less (4097 to 6144 rows
+# of 4096 columns and more); four waves (q4_K, more rows of 4096 columns at most)
+@pytest.mark.parametrize("quant", ["q4_0", "q4_K", "q6_K"])
+@pytest.mark.parametrize("n,k", [(41, 64), (40, 1984), (48, 4096), (48, 10240),
+                                 (48, 4416), (4112, 4096), (4112, 4352),
+                                 (4120, 4160), (5000, 12800), (6160, 4096),
+                                 (6160, 4352), (6176, 10304)])
+@torch.no_grad()
+def test_quant_one_row(quant, n, k):
+    if quant.endswith("_K") and k % 256:
+        pytest.skip("blocks of 256")
+    torch.manual_seed(n + k)
+    lin = Linear(k, n, device=DEV, dtype=torch.bfloat16)
+    lin.weight.normal_(0.0, 0.5)
+    ql = QuantLinear.from_linear(lin, quant)
+    w = ql._dequant_cpu().to(DEV).double()
+    x = torch.randn(1, k, device=DEV).bfloat16()
+    want, room = x.double() @ w.T, x.double().abs() @ w.abs().T
+    assert bool(((ql(x).double() - want).abs()
+                 <= 2.0 ** -8 * want.abs() + 2.0 ** -18 * room).all())
+    if n % 16 == 0:
+        y, want = ql.gated(x), gated(want)
+        assert bool(((y.double() - want).abs() <= 2.0 ** -7 * want.abs()
+                     + 2.0 ** -6 * room.mean()).all())
+
+
 def one_column(ql, quant, at, number):
     """Every row's number of column `at`, and its minimum 0."""
     k, qs = ql.in_features, ql.qs
