@@ -16,7 +16,7 @@ template <class T>
 void launch_latent_prepare(T*, long, int, int, int, int, int, const float*, float, const double*, int, const int*, T*, const int*, const float*, int, long, hipStream_t);
 void launch_latent_gather(void*, void*, const void*, int, int, int, const int*, int, const int*, const int*, const int*, int, int, int, int, hipStream_t);
 int moe_max_experts();
-void launch_moe_select(int*, float*, const float*, int, int, int, int, int, int, const float*, bool, bool, const float*, int, hipStream_t);
+void launch_moe_select(int*, float*, const float*, int, int, int, int, int, int, const float*, bool, bool, const float*, int, int*, hipStream_t);
 void launch_moe_sort(int*, int*, int*, int*, const int*, int, int, int, int, hipStream_t);
 template <class T>
 void launch_embed_norm(T*, float*, const T*, const int*, float, const T*, const int*, int, const float*, long, int, int, float, float, hipStream_t);
@@ -532,7 +532,7 @@ Tensor linear32(Tensor x, Tensor w) {
 
 void moe_select(Tensor ids, Tensor weights, Tensor z, int64_t groups,
                 int64_t keep, OptTensor bias, bool over_chosen, bool sigmoid,
-                OptTensor correction, int64_t group_best) {
+                OptTensor correction, int64_t group_best, OptTensor at) {
   TORCH_CHECK(z.dim() == 3, "z must be [splits, rows, experts]");
   const long rows = z.size(1), experts = z.size(2), top = ids.size(1);
   check(ids, torch::kInt32, "ids");
@@ -555,17 +555,22 @@ void moe_select(Tensor ids, Tensor weights, Tensor z, int64_t groups,
   TORCH_CHECK(groups > 0 && experts % groups == 0 && keep > 0 &&
               keep <= groups && top > 0 && top <= experts / groups * keep,
               "moe_select: cannot choose so many");
+  if (at) {
+    check(*at, torch::kInt32, "at");
+    TORCH_CHECK(at->sizes() == ids.sizes(), "one place per choice");
+  }
   if (rows == 0) return;
   launch_moe_select(ptr<int>(ids), ptr<float>(weights), ptr<float>(z),
                     z.size(0), rows, experts, top, groups, keep,
                     ptr<float>(bias), over_chosen, sigmoid,
-                    ptr<float>(correction), group_best, stream());
+                    ptr<float>(correction), group_best, ptr<int>(at), stream());
   post("moe_select");
 }
 
 int64_t moe_tile(int64_t packed, int64_t experts, bool bf16, int64_t k,
                  int64_t n) {
-  return group_gemm_tile(packed, experts, bf16, std::gcd(k, n));
+  const int tile = group_gemm_tile(packed, experts, bf16, std::gcd(k, n));
+  return bf16 ? group_gemm_rows_tile(tile, k, n) : tile;
 }
 
 // tiles: [1 + 2 * bound], of which each expert's last may be short
@@ -620,6 +625,50 @@ void expert_linear(Tensor out, Tensor x, Tensor w, OptTensor src,
   });
 }
 
+// The same of rows that are not packed: row r is of expert ids[r], and of row
+// r / top of x, or of row r (top 0).
+GroupGemm<bf16_t, bf16_t> chosen(const Tensor& out, const Tensor& x,
+                                 const Tensor& w, const Tensor& ids,
+                                 int64_t tile, const std::string& act,
+                                 double limit, int64_t top) {
+  auto a = product<bf16_t>(out, x, w);
+  a.m = out.size(0);
+  a.ids = ptr<int>(ids); a.top = top;
+  a.max_tiles = (a.m + tile - 1) / tile + std::min(a.groups, a.m);
+  if (act == "gelu") a.act = Act::GELU;
+  else if (act != "none") {
+    a.act = Act::GLU; a.glu = glu_of(act); a.limit = limit;
+  }
+  return a;
+}
+
+// Both products of experts without packing: h [rows * top, ff], out [rows * top,
+// width] of x [rows, width] and ids [rows, top]. False where there are no kernels
+// for that: then nothing is written.
+bool experts_chosen(Tensor h, Tensor out, Tensor x, Tensor up, Tensor down,
+                    Tensor ids, int64_t tile, const std::string& act,
+                    double limit, bool ask) {
+  const bool glu = act != "none" && act != "gelu";
+  const long top = ids.size(1), rows = x.size(0), packed = rows * top;
+  TORCH_CHECK(x.dim() == 2 && ids.dim() == 2 && ids.size(0) == rows &&
+              up.dim() == 3 && down.dim() == 3 && up.size(0) == down.size(0) &&
+              up.size(2) == x.size(1) && down.size(1) == x.size(1) &&
+              up.size(1) == (glu ? 2 : 1) * down.size(2) &&
+              h.size(0) == packed && h.size(1) == down.size(2) &&
+              out.size(0) == packed && out.size(1) == x.size(1),
+              "experts: shapes differ");
+  check(ids, torch::kInt32, "ids");
+  if (x.scalar_type() != torch::kBFloat16 || packed == 0) return false;
+  const auto a = chosen(h, x, up, ids, tile, act, limit, top),
+             b = chosen(out, h, down, ids, tile, "none", 0., 0);
+  if (!group_gemm_chosen(a, b, tile)) return false;
+  if (ask) return true;
+  launch_group_gemm(a, tile, stream());
+  launch_group_gemm(b, tile, stream());
+  post("experts_chosen");
+  return true;
+}
+
 void silu_mul(Tensor out, Tensor x) {
   const int f = out.size(-1);
   TORCH_CHECK(x.size(-1) == 2 * f && x.numel() == 2 * out.numel(),
@@ -659,10 +708,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("z"), py::arg("groups"), py::arg("keep"),
         py::arg("bias") = py::none(), py::arg("over_chosen") = false,
         py::arg("sigmoid") = false, py::arg("correction") = py::none(),
-        py::arg("group_best") = 1);
+        py::arg("group_best") = 1, py::arg("at") = py::none());
   m.def("moe_tile", &moe_tile);
   m.def("moe_sort", &moe_sort);
   m.def("expert_linear", &expert_linear);
+  m.def("experts_chosen", &experts_chosen);
   m.def("linear32", &linear32);
   bind_mixers(m);
 }

@@ -3,7 +3,9 @@
 //     group g's part of a row starts at x + g * x_gs and y + g * y_gs;
 //   * tiles given: rows are packed by group (the tokens of every expert) and
 //     cut into tiles on the device; tiles[0] is their number, then come a
-//     group and a first row for each, start[g + 1] ends group g.
+//     group and a first row for each, start[g + 1] ends group g;
+//   * ids given: row r is of group ids[r], and workgroups look for those of
+//     theirs (few rows: group_gemm_rows.hip).
 #pragma once
 
 #include "typed.h"
@@ -33,6 +35,8 @@ struct GroupGemm {
   const int* start;
   const int* tiles;
   int max_tiles;           // bound of tiles[0]
+  const int* ids;          // [m], row r from row r / top of x, or from row r
+  int top;                 //   (top 0)
   const T* gate;           // row r, group g, column n at
   long gate_ld, gate_gs;   //   gate + r * gate_ld + g * gate_gs + n,
   bool gate_each;          //   or not each column: without n
@@ -196,6 +200,11 @@ int group_gemm_tile(long rows, int groups, bool bf16, int ks);
 template <class T, class Y>
 bool group_gemm_takes(const GroupGemm<T, Y>&, int tile);
 
+// Whether the rows of two products, one of the other's, better come with their
+// groups' numbers only.
+bool group_gemm_chosen(const GroupGemm<bf16_t, bf16_t>&,
+                       const GroupGemm<bf16_t, bf16_t>&, int tile);
+
 // Shares of the inner dimension that let one small product fill the chip.
 template <class T, class Y>
 int group_gemm_splits(const GroupGemm<T, Y>&);
@@ -209,6 +218,8 @@ void launch_group_gemm_tile(const GroupGemm<bf16_t, Y>&, int tile,
                             hipStream_t);
 
 // Packed rows, up to 64 of a group (group_gemm_rows.hip).
+int group_gemm_rows_tile(int tile, int k, int n);
+bool group_gemm_ids_pay(int rows, int n, int n2, int groups, int tile);
 template <class Y>
 bool group_gemm_rows_takes(const GroupGemm<bf16_t, Y>&, int tile);
 template <class Y>

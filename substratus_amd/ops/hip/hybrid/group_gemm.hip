@@ -235,6 +235,13 @@ bool group_gemm_takes(const GroupGemm<T, Y>& a, int tile) {
   return tile == AT;
 }
 
+bool group_gemm_chosen(const GroupGemm<bf16_t, bf16_t>& a,
+                       const GroupGemm<bf16_t, bf16_t>& b, int tile) {
+  return tile <= 64 && pieces(a) && pieces(b) &&
+         group_gemm_rows_takes(a, tile) && group_gemm_rows_takes(b, tile) &&
+         group_gemm_ids_pay(a.m, a.n, b.n, a.groups, tile);
+}
+
 // everything a store touches comes in aligned groups of four columns
 template <class T, class Y>
 bool by_quads(const GroupGemm<T, Y>& a) {
@@ -280,7 +287,8 @@ void launch_group_gemm(const GroupGemm<T, Y>& given, int tile,
   GroupGemm<T, Y> a = given;
   a.quads = by_quads(a);
   a.tail_eights = by_eights(a);
-  const bool packed = a.tiles != nullptr, split = a.splits > 1;
+  const bool packed = a.tiles != nullptr || a.ids != nullptr,
+             split = a.splits > 1;
   const int gz = packed ? 1 : split ? a.splits : a.groups;
   if (split) tile = 16;
   if constexpr (std::is_same_v<T, bf16_t>) {

@@ -17,8 +17,16 @@
 //   128 rows  49.3 -> 38.4 (4.8)         50.0 -> 38.8
 //   300 rows  62.9 -> 55.4               65.0 -> 53.9
 //   500 rows  89.0 -> 73.3               86.2 -> 71.8
+//
+// Where rows are not packed, but have their groups' numbers (ids), a workgroup
+// looks through all of these for its group's rows: a step's choices are a few
+// hundred, which each of its waves has in registers after one load, and nothing
+// waits for a kernel that packs them; the first weights are asked for meanwhile.
 #include "../rows_gemm.h"
 #include "group_gemm.h"
+
+#include <algorithm>
+#include <climits>
 
 namespace {
 
@@ -34,55 +42,97 @@ template <int F_, int N_, int P_> struct How {
   static constexpr int PIECES = KW * P * U * (N + F) * TILE;     // of LDS
 };
 
-template <class H, Act ACT, class Y>
-DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
-                              uint4* s_all) {
-  constexpr int F = H::F, N = H::N, P = H::P;
-  constexpr int TILES = N + F, STAGE = U * TILES * TILE, LOADS = U * TILES;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int lane = threadIdx.x % WAVE, lo = lane & 15, g = lane >> 4;
-  // shares begin on whole cache lines
-  const int n0 = blockIdx.x * N * 16, chunks = a.k / KC;
-  const int pairs = (chunks + 1) / 2;
-  const int c0 = pairs * wave / KW * 2;
-  const int c1 = min(pairs * (wave + 1) / KW * 2, chunks);
-  const int steps = (c1 - c0 + U - 1) / U;
-  uint4* ring = s_all + wave * P * STAGE;
+constexpr int IDS = 512;          // that are looked through, at most
 
-  // a load is 8 rows x 128 bytes: of a tile's row lane / 8, or eight later.
-  // Pieces are permuted by the row against bank conflicts.
-  const char *wp[N][2], *xp[F][2];
+// A wave's share of the inner dimension, and its loads of the weights: 8 rows x 128
+// bytes each, of a tile's row lane / 8, or eight later. Pieces are permuted by the
+// row against bank conflicts. Its stages' weights come first in its part of LDS,
+// whatever the rows of x take.
+template <int N> struct Share {
+  static constexpr int STAGE = U * N * TILE, LOADS = U * N;
+  int c0, c1, steps, end;
+  const char* wp[N][2];
   int piece[2];
-  #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int row = h * 8 + (lane >> 3);
-    piece[h] = (lane & 7) ^ (row >> 1);
+
+  template <class Y>
+  DEV_INLINE Share(const GroupGemm<bf16_t, Y>& a) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    // shares begin on whole cache lines
+    const int chunks = a.k / KC, pairs = (chunks + 1) / 2;
+    c0 = pairs * wave / KW * 2;
+    c1 = min(pairs * (wave + 1) / KW * 2, chunks);
+    steps = (c1 - c0 + U - 1) / U;
+    end = (c1 - c0) * 4 - 1;                     // its last piece
     #pragma unroll
-    for (int f = 0; f < N; ++f)
-      wp[f][h] = reinterpret_cast<const char*>(
-          a.w + ((long)t.g * a.n + min(n0 + f * 16 + row, a.n - 1)) * a.k +
-          c0 * KC);
-    #pragma unroll
-    for (int f = 0; f < F; ++f) {
-      const int r = min(t.r0 + f * 16 + row, t.r1 - 1);
-      xp[f][h] = reinterpret_cast<const char*>(
-          a.x + (long)(a.src != nullptr ? a.src[r] : r) * a.x_ld + c0 * KC);
-    }
+    for (int h = 0; h < 2; ++h)
+      piece[h] = (threadIdx.x & 7) ^ ((h * 8 + row()) >> 1);
   }
-  const int end = (c1 - c0) * 4 - 1;             // the share's last piece
-  auto load = [&](int s, int i) {
-    uint4* to = ring + s * STAGE;
+  static DEV_INLINE int row() { return threadIdx.x % WAVE >> 3; }
+  template <class Y>
+  DEV_INLINE void group(const GroupGemm<bf16_t, Y>& a, int g) {
     #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      // a stage may be half of one: then its last piece comes again
-      const unsigned at = (unsigned)min(i * 8 + piece[h], end) * 16;
+    for (int h = 0; h < 2; ++h)
       #pragma unroll
       for (int f = 0; f < N; ++f)
-        load_to_lds<16>(wp[f][h] + at, to + (f * 2 + h) * TILE);
+        wp[f][h] = reinterpret_cast<const char*>(
+            a.w + ((long)g * a.n + min((int)blockIdx.x * N * 16 + f * 16 +
+                                           h * 8 + row(), a.n - 1)) * a.k +
+            c0 * KC);
+  }
+  // a stage may be half of one: then its last piece comes again
+  DEV_INLINE unsigned at(int i, int h) const {
+    return (unsigned)min(i * 8 + piece[h], end) * 16;
+  }
+  DEV_INLINE void load(uint4* ring, int s, int i) const {
+    #pragma unroll
+    for (int h = 0; h < 2; ++h)
+      #pragma unroll
+      for (int f = 0; f < N; ++f)
+        load_to_lds<16>(wp[f][h] + at(i, h),
+                        ring + s * STAGE + (f * 2 + h) * TILE);
+  }
+};
+
+// Of the first E stages the weights are on their way. list: of rows that are not
+// packed, t's numbers are places in it.
+template <class H, Act ACT, bool LISTED, int E, class Y>
+DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
+                              const Share<H::N>& w, uint4* s_all, uint4* ring,
+                              const int* list) {
+  constexpr int F = H::F, N = H::N, P = H::P;
+  constexpr int STAGE = U * F * TILE, LOADS = U * (N + F), XL = U * F;
+  static_assert(E <= P && E <= 2);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, lo = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * N * 16, steps = w.steps;
+  uint4* x_ring = ring + P * Share<N>::STAGE;
+
+  const char* xp[F][2];
+  #pragma unroll
+  for (int h = 0; h < 2; ++h)
+    #pragma unroll
+    for (int f = 0; f < F; ++f) {
+      int r = min(t.r0 + f * 16 + h * 8 + w.row(), t.r1 - 1);
+      if constexpr (LISTED) {
+        r = list[r];
+        if (a.top > 0) r /= a.top;
+      } else if (a.src != nullptr) {
+        r = a.src[r];
+      }
+      xp[f][h] =
+          reinterpret_cast<const char*>(a.x + (long)r * a.x_ld + w.c0 * KC);
+    }
+  auto load_x = [&](int s, int i) {
+    #pragma unroll
+    for (int h = 0; h < 2; ++h)
       #pragma unroll
       for (int f = 0; f < F; ++f)
-        load_to_lds<16>(xp[f][h] + at, to + ((N + f) * 2 + h) * TILE);
-    }
+        load_to_lds<16>(xp[f][h] + w.at(i, h),
+                        x_ring + s * STAGE + (f * 2 + h) * TILE);
+  };
+  auto load = [&](int s, int i) {
+    w.load(ring, s, i);
+    load_x(s, i);
   };
   float4v acc[N][F];
   #pragma unroll
@@ -93,13 +143,15 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
     short8 wf[U][N], xf[U][F];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint4* p = ring + s * STAGE + lo * 8 + ((u * 4 + g) ^ (lo >> 1));
+      const int at = lo * 8 + ((u * 4 + g) ^ (lo >> 1));
       #pragma unroll
       for (int f = 0; f < N; ++f)
-        wf[u][f] = *reinterpret_cast<const short8*>(p + f * 2 * TILE);
+        wf[u][f] = *reinterpret_cast<const short8*>(
+            ring + s * Share<N>::STAGE + at + f * 2 * TILE);
       #pragma unroll
       for (int f = 0; f < F; ++f)
-        xf[u][f] = *reinterpret_cast<const short8*>(p + (N + f) * 2 * TILE);
+        xf[u][f] = *reinterpret_cast<const short8*>(
+            x_ring + s * STAGE + at + f * 2 * TILE);
     }
     if (more) {
       wait_lds_reads();
@@ -107,7 +159,7 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
     }
     #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (c0 + i * U + u < c1) {
+      if (w.c0 + i * U + u < w.c1) {
         #pragma unroll
         for (int j = 0; j < N; ++j)
           #pragma unroll
@@ -117,8 +169,14 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
       }
   };
   #pragma unroll
-  for (int s = 0; s < P; ++s)
+  for (int s = 0; s < E; ++s)
+    if (s < steps) load_x(s, s);
+  #pragma unroll
+  for (int s = E; s < P; ++s)
     if (s < steps) load(s, s);
+  // the first stage's rows came later than the second's weights
+  if (steps >= P) wait_loads<(P - E) * LOADS + (E - 1) * XL>();
+  else wait_loads<0>();
   int i = 0;
   for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
     #pragma unroll
@@ -155,12 +213,43 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
     #pragma unroll
     for (int q = 0; q < KW; ++q)
       v += *reinterpret_cast<const float4v*>(&red[(q * ROWS + r) * LD + c]);
-    store4<ACT>(a, t, t.r0 + r, n0 + c, v);
+    if constexpr (LISTED) {
+      if (r < t.r1) store4<ACT>(a, Tile{t.g, 0, INT_MAX}, list[r], n0 + c, v);
+    } else {
+      store4<ACT>(a, t, t.r0 + r, n0 + c, v);
+    }
   }
 }
 
-// MAX: times 16 rows that a tile may have
-template <class Y, Act ACT, int MAX>
+// A lane's ids, of every wave's rows.
+struct Ids {
+  int id[IDS / WAVE];
+  DEV_INLINE void load(const int* ids, int n) {
+    #pragma unroll
+    for (int i = 0; i < IDS / WAVE; ++i)
+      id[i] = ids[min(i * WAVE + (int)threadIdx.x % WAVE, n - 1)];
+  }
+  // Rows of group g, in order: those from the `from`th on, up to `most`, to a
+  // wave's list. Returns how many there are in all.
+  DEV_INLINE int list(int n, int g, int from, int most, int* to) const {
+    const int lane = threadIdx.x % WAVE;
+    int count = 0;
+    #pragma unroll
+    for (int i = 0; i < IDS / WAVE; ++i) {
+      const bool mine = i * WAVE + lane < n && id[i] == g;
+      const unsigned long long all = __ballot(mine);
+      const int at = count - from + __builtin_amdgcn_mbcnt_hi(
+          (unsigned)(all >> 32),
+          __builtin_amdgcn_mbcnt_lo((unsigned)all, 0));
+      if (mine && at >= 0 && at < most) to[at] = i * WAVE + lane;
+      count += __popcll(all);
+    }
+    return count;
+  }
+};
+
+// MAX: times 16 rows that a tile may have; LISTED: rows by their ids
+template <class Y, Act ACT, int MAX, bool LISTED>
 __global__ __launch_bounds__(KW * WAVE, 2)
 void group_gemm_rows_kernel(GroupGemm<bf16_t, Y> a) {
   constexpr int N = MAX == 1 ? 1 : 2;
@@ -171,24 +260,79 @@ void group_gemm_rows_kernel(GroupGemm<bf16_t, Y> a) {
   using Three = How<3, N, 2>;
   using Four = How<4, N, 1>;
   constexpr int LARGEST = MAX > 2 ? Three::PIECES : One::PIECES;
-  __shared__ alignas(16) uint4 s_all[LARGEST];
+  constexpr int E = MAX > 2 ? 1 : 2;             // the least of them in flight
+  constexpr int LIST = MAX * 4;                  // pieces of a wave's
+  __shared__ alignas(16) uint4 s_all[LARGEST + (LISTED ? KW * LIST : 0)];
   static_assert(MAX == 1 || Two::PIECES <= LARGEST);
-  const Tile t = tile_of(a, blockIdx.y, 0, MAX * 16);
-  if (t.r1 <= t.r0) return;
-  const int tiles = (t.r1 - t.r0 + 15) / 16;     // of the rows there are
-  if (MAX == 1 || tiles == 1) {
-    rows_of_group<One, ACT>(a, t, s_all);
-  } else if constexpr (MAX > 1) {
-    if (MAX == 2 || tiles == 2) {
-      rows_of_group<Two, ACT>(a, t, s_all);
-    } else if constexpr (MAX > 2) {
-      if (tiles == 3) rows_of_group<Three, ACT>(a, t, s_all);
-      else rows_of_group<Four, ACT>(a, t, s_all);
+  int* list = reinterpret_cast<int*>(s_all + LARGEST +
+                                     threadIdx.x / WAVE * LIST);
+  uint4* ring = s_all + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) *
+                            (LARGEST / KW);
+  Share<N> w(a);
+  auto begin = [&](int g) {
+    w.group(a, g);
+    #pragma unroll
+    for (int s = 0; s < E; ++s)
+      if (s < w.steps) w.load(ring, s, s);
+  };
+  auto run = [&](const Tile& t) {
+    const int tiles = (t.r1 - t.r0 + 15) / 16;   // of the rows there are
+    if (MAX == 1 || tiles == 1) {
+      rows_of_group<One, ACT, LISTED, E>(a, t, w, s_all, ring, list);
+    } else if constexpr (MAX > 1) {
+      if (MAX == 2 || tiles == 2) {
+        rows_of_group<Two, ACT, LISTED, E>(a, t, w, s_all, ring, list);
+      } else if constexpr (MAX > 2) {
+        if (tiles == 3)
+          rows_of_group<Three, ACT, LISTED, E>(a, t, w, s_all, ring, list);
+        else
+          rows_of_group<Four, ACT, LISTED, E>(a, t, w, s_all, ring, list);
+      }
     }
+  };
+  if constexpr (LISTED) {
+    // As many workgroups as rows, where that is less than groups: a group's first
+    // row has them. Where a group without rows is unlikely, weights do not wait.
+    const bool by_row = a.m < a.groups, early = a.m >= 2 * a.groups;
+    const int g = by_row ? a.ids[blockIdx.y] : (int)blockIdx.y;
+    Ids ids;
+    ids.load(a.ids, a.m);
+    __builtin_amdgcn_sched_barrier(0);           // ahead of the weights
+    if (early) begin(g);
+    for (int from = 0;; from += MAX * 16) {
+      const int rows = ids.list(a.m, g, from, MAX * 16, list) - from;
+      wait_lds_reads();                          // the list is written
+      if (rows <= 0 || (by_row && from == 0 && list[0] != (int)blockIdx.y)) {
+        wait_loads<0>();          // no load outlives its workgroup's LDS
+        return;
+      }
+      if (!early || from > 0) begin(g);
+      run(Tile{g, 0, min(rows, MAX * 16)});
+      if (rows <= MAX * 16) return;
+      __syncthreads();
+    }
+  } else {
+    const Tile t = tile_of(a, blockIdx.y, 0, MAX * 16);
+    if (t.r1 <= t.r0) return;
+    begin(t.g);
+    run(t);
   }
 }
 
 }  // namespace
+
+// Tiles of 32 where ones of 16 would do: workgroups of 32 columns instead of 16 are
+// half as many, and what it takes to begin one and to add up its waves' shares counts
+// more than rows that are not there. us of both products and of packing, MI355X, 16 ->
+// 32: 32 experts of 2048 x 1408, 6 a row, 1, 4, 16, 40 rows 26.5 50 76.6 80.8 -> 25.3
+// 47.2 71.5 73.5; of 4096 x 2048, 8 a row, 1, 4, 32 rows 58.3 138.5 196 -> 57 131.5
+// 183; 64 of 2048 x 1408, 16 and 48 rows 120 144 -> 109 129; 8 of 4096 x 1408, 2 a
+// row, 4 and 16 rows 34.6 46.5 -> 39.1 45.6. Shorter rows are another kernel's with
+// tiles of 16 (64 of 2048 x 512, 4 a row, 16 rows 43.8 -> 49.6).
+int group_gemm_rows_tile(int tile, int k, int n) {
+  return tile == 16 && k % KC == 0 && n % KC == 0 && std::min(k, n) > 1280
+      ? 32 : tile;
+}
 
 // A workgroup's columns.
 static int columns(int tile) { return tile == 16 ? 16 : 32; }
@@ -205,11 +349,27 @@ static int columns(int tile) { return tile == 16 ? 16 : 32; }
 //                          1.06)      (1.0-1.2)   (0.9-1.7)   1.18    1.38  1.25
 template <class Y>
 bool group_gemm_rows_takes(const GroupGemm<bf16_t, Y>& a, int tile) {
-  if (a.tiles == nullptr || tile > 64 || a.k % KC != 0 || a.k < 4 * KC ||
-      a.tail != 0)
+  if ((a.tiles == nullptr && a.ids == nullptr) || tile > 64 || a.k % KC != 0 ||
+      a.k < 4 * KC || a.tail != 0 ||
+      (a.ids != nullptr && (a.m > IDS || tile > 32)))
     return false;
   const long blocks = (long)(a.n + columns(tile) - 1) / columns(tile) * a.max_tiles;
   return blocks <= 1024 || a.k > (tile == 16 ? 1280 : 128);
+}
+
+// Looking for one's rows takes longer than to be told, in every workgroup, and a kernel
+// that packs 3.5 us. us of two products, MI355X, packed -> not, by tiles of 32, of 1,
+// 4, 16, 32, 64 rows: 32 experts of 2048 x 1408, 6 a row 25.3 47.2 71.5 72.5 75 -> 23
+// 46.2 67.1 68.7 72 (2500 workgroups, 64 rows: 1.3 M); of 4096 x 2048, 8 a row 57
+// 131.5 188.3 183.3 191.4 -> 54.2 129.2 185.1 182.8 195 (6144, 32 rows: 1.6 M); 64 of
+// 2048 x 1408, 6 a row, 48 rows 129.2 -> 127.4 (2 M); 16 of 512 x 256, 2 a row, tiles
+// of 16, 4 and 48 rows 11.6 12.9 -> 8.9 10.1. Tiles of 64 wait for their rows at the
+// start of every stage: 74 -> 97.
+bool group_gemm_ids_pay(int rows, int n, int n2, int groups, int tile) {
+  const int wide = columns(tile);
+  return tile <= 32 &&
+         (long)((n + wide - 1) / wide + (n2 + wide - 1) / wide) * groups *
+                 rows <= 2000000;
 }
 
 template <class Y>
@@ -217,12 +377,23 @@ void launch_group_gemm_rows(const GroupGemm<bf16_t, Y>& a, int tile,
                             hipStream_t stream) {
   by_act(a.act, [&](auto act) {
     constexpr Act ACT = decltype(act)::value;
-    auto kernel = tile == 16 ? group_gemm_rows_kernel<Y, ACT, 1>
-                  : tile == 32 ? group_gemm_rows_kernel<Y, ACT, 2>
-                               : group_gemm_rows_kernel<Y, ACT, 4>;
     const int wide = columns(tile);
-    kernel<<<dim3((a.n + wide - 1) / wide, a.max_tiles), KW * WAVE, 0,
-             stream>>>(a);
+    auto go = [&](auto listed, int tiles) {
+      constexpr bool L = decltype(listed)::value;
+      auto kernel = tile == 16 ? group_gemm_rows_kernel<Y, ACT, 1, L>
+                               : group_gemm_rows_kernel<Y, ACT, 2, L>;
+      if constexpr (!L)
+        if (tile == 64) kernel = group_gemm_rows_kernel<Y, ACT, 4, L>;
+      kernel<<<dim3((a.n + wide - 1) / wide, tiles), KW * WAVE, 0, stream>>>(
+          a);
+    };
+    if constexpr (std::is_same_v<Y, bf16_t> && ACT != Act::GATE &&
+                  ACT != Act::SIDE)
+      if (a.ids != nullptr) {
+        go(std::true_type{}, std::min(a.m, a.groups));
+        return;
+      }
+    go(std::false_type{}, a.max_tiles);
   });
 }
 

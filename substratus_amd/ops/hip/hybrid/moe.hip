@@ -1,6 +1,7 @@
 // Choosing experts and packing tokens by expert.
 //
-//   select   one wave per token: scores (sums of a product's shares of the
+//   select   one wave per token (where rows stay as they are, their places are
+//            written, too): scores (sums of a product's shares of the
 //            inner dimension), softmax over all experts, the best groups
 //            of neighbours, the best experts of those; all in 32 bits.
 //            Or the softmax is over the chosen experts only, or every score
@@ -38,7 +39,7 @@ void moe_select_kernel(int* __restrict__ ids, float* __restrict__ weights,
                        int experts, int top, int groups, int keep,
                        const float* __restrict__ bias, bool over_chosen,
                        bool sigmoid, const float* __restrict__ correction,
-                       int group_best) {
+                       int group_best, int* __restrict__ at) {
   extern __shared__ float4 s_all[];
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int pad = (experts + 3) / 4 * 4;
@@ -49,7 +50,10 @@ void moe_select_kernel(int* __restrict__ ids, float* __restrict__ weights,
   float v[PL], sc[PL];                          // for the choice, as weights
   float mx = -INFINITY;
   // scores that are no numbers: weights are none either, but experts are
-  for (int r = lane; r < top; r += WAVE) ids[row * top + r] = 0;
+  for (int r = lane; r < top; r += WAVE) {
+    ids[row * top + r] = 0;
+    if (at != nullptr) at[row * top + r] = row * top + r;
+  }
   #pragma unroll
   for (int i = 0; i < PL; ++i) {
     const int e = lane + i * WAVE;
@@ -189,14 +193,14 @@ int moe_max_experts() { return SORT; }
 void launch_moe_select(int* ids, float* weights, const float* z, int splits,
                        int rows, int experts, int top, int groups, int keep,
                        const float* bias, bool over_chosen, bool sigmoid,
-                       const float* correction, int group_best,
+                       const float* correction, int group_best, int* at,
                        hipStream_t stream) {
   auto go = [&](auto pl) {
     moe_select_kernel<decltype(pl)::value>
         <<<dim3((rows + SW - 1) / SW), dim3(SW * WAVE),
            SW * 2 * ((experts + 3) / 4 * 4) * sizeof(float), stream>>>(
             ids, weights, z, splits, rows, experts, top, groups, keep, bias,
-            over_chosen, sigmoid, correction, group_best);
+            over_chosen, sigmoid, correction, group_best, at);
   };
   if (experts <= WAVE) go(std::integral_constant<int, 1>{});
   else if (experts <= 4 * WAVE) go(std::integral_constant<int, 4>{});

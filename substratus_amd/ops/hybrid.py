@@ -266,26 +266,30 @@ def experts(y: torch.Tensor, router: torch.Tensor, up: torch.Tensor,
     ext = _ext()
     i32 = dict(dtype=torch.int32, device=y.device)
     z = ext.router_scores(y, router)
-    ids = torch.empty(rows, spec.top, **i32)
+    ids, at = (torch.empty(rows, spec.top, **i32) for _ in range(2))
     weights = torch.empty(rows, spec.top, dtype=torch.float32,
                           device=y.device)
-    ext.moe_select(ids, weights, z, spec.groups, spec.keep, bias,
-                   spec.over_chosen, spec.sigmoid, correction,
-                   spec.group_best)
     packed = rows * spec.top
     tile = ext.moe_tile(packed, spec.experts, y.dtype == torch.bfloat16,
                         y.shape[1], spec.ff)
-    at = torch.empty(rows, spec.top, **i32)
+    h, out = (y.new_empty(packed, n) for n in (spec.ff, y.shape[1]))
+    act, limit = ("gelu", 0.0) if spec.glu is None else \
+        (spec.glu.act, spec.glu.limit)
+    both = h, out, y, up, down, ids, tile, act, limit
+    # a few hundred choices: nothing is packed, rows stay where tokens have them
+    chosen = ext.experts_chosen(*both, True)
+    ext.moe_select(ids, weights, z, spec.groups, spec.keep, bias,
+                   spec.over_chosen, spec.sigmoid, correction,
+                   spec.group_best, at if chosen else None)
+    if chosen:
+        ext.experts_chosen(*both, False)
+        return Picked(out, at, weights)
     src = torch.empty(packed, **i32)
     start = torch.empty(spec.experts + 1, **i32)
     tiles = torch.empty(1 + 2 * ((packed + tile - 1) // tile +
                                  min(spec.experts, packed)), **i32)
     ext.moe_sort(at, src, start, tiles, ids, tile)
-    h = y.new_empty(packed, spec.ff)
-    act, limit = ("gelu", 0.0) if spec.glu is None else \
-        (spec.glu.act, spec.glu.limit)
     ext.expert_linear(h, y, up, src, start, tiles, tile, act, limit)
-    out = y.new_empty(packed, y.shape[1])
     ext.expert_linear(out, h, down, None, start, tiles, tile, "none", 0.0)
     return Picked(out, at, weights)
 

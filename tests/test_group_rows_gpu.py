@@ -47,6 +47,65 @@ def test_experts_of_few_rows(tile, k, n, act):
     close(out[at[:, 0].long()], want.float(), BF16)
 
 
+# Rows that are looked for by their ids: fewer than experts, of one expert more than
+# a tile holds, of a token twice the same (scores that were no numbers), experts
+# without any where weights are asked for first, and the most ids; the packed rows'
+# kernel has the same bits.
+@pytest.mark.parametrize("tile", [16, 32])
+@pytest.mark.parametrize("k,ff,act", [(128, 160, "none"), (1056, 128, "silu"),
+                                      (2080, 1312, "gelu")])
+@pytest.mark.parametrize("rows,top,e", [(1, 2, 5), (3, 1, 5), (3, 2, 6),
+                                        (5, 2, 7), (40, 1, 3), (64, 8, 9),
+                                        (128, 4, 4)])
+def test_experts_by_ids(tile, k, ff, act, rows, top, e):
+    g = torch.Generator().manual_seed(rows + k)
+    ids = torch.stack([torch.randperm(max(e, top), generator=g)[:top] % e
+                       for _ in range(rows)]).int()
+    ids[ids == e - 2] = 0                   # an expert without rows
+    if rows > 2:
+        ids[1] = ids[1, 0]
+    ids = ids.cuda()
+    n, each = rows * top, 2 if act == "silu" else 1
+    x = rand(rows, k + 8, seed=1, dtype=BF16).cuda()[:, :k]
+    up = rand(e, each * ff, k, seed=2, dtype=BF16, scale=k ** -0.5).cuda()
+    down = rand(e, k, ff, seed=3, dtype=BF16, scale=ff ** -0.5).cuda()
+    ext = ops._ext()
+    h, out = (torch.full((n, c), 9.0, dtype=BF16, device="cuda")
+              for c in (ff, k))
+    if not ext.experts_chosen(h, out, x, up, down, ids, tile, act, 0.0, True):
+        assert tile == 16 and n == 512      # many blocks of short rows
+        pytest.skip("another kernel's")
+    assert bool((h == 9).all())
+    assert ext.experts_chosen(h, out, x, up, down, ids, tile, act, 0.0, False)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    at, src = torch.empty(rows, top, **i32), torch.empty(n, **i32)
+    start = torch.empty(e + 1, **i32)
+    tiles = torch.empty(1 + 2 * ((n + tile - 1) // tile + min(e, n)), **i32)
+    ext.moe_sort(at, src, start, tiles, ids, tile)
+    h2, out2 = torch.empty_like(h), torch.empty_like(out)
+    ext.expert_linear(h2, x, up, src, start, tiles, tile, act, 0.0)
+    ext.expert_linear(out2, h2, down, None, start, tiles, tile, "none", 0.0)
+    where = at.view(-1).long()
+    assert torch.equal(h, h2[where]) and torch.equal(out, out2[where])
+
+
+def test_experts_that_are_packed():
+    """Too many ids, tiles of 64 rows, rows that are no whole chunks, float."""
+    ext = ops._ext()
+
+    def asks(rows, k, ff, tile, dtype=BF16):
+        z = dict(dtype=dtype, device="cuda")
+        return ext.experts_chosen(
+            torch.empty(rows * 2, ff, **z), torch.empty(rows * 2, k, **z),
+            torch.empty(rows, k, **z), torch.empty(4, ff, k, **z),
+            torch.empty(4, k, ff, **z),
+            torch.zeros(rows, 2, dtype=torch.int32, device="cuda"), tile,
+            "none", 0.0, True)
+    assert asks(256, 128, 160, 32) and not asks(257, 128, 160, 32)
+    assert not asks(4, 128, 160, 64) and not asks(4, 144, 160, 32)
+    assert not asks(4, 128, 160, 32, torch.float32)
+
+
 @pytest.mark.parametrize("rows", [1, 16, 48, 65, 300])
 @pytest.mark.parametrize("k,n,tail,each", [(512, 128, 0, True),
                                            (512, 72, 0, False),
