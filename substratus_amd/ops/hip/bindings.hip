@@ -680,7 +680,7 @@ torch::Tensor tile_gemm(torch::Tensor a, torch::Tensor b,
                               b_flipped, gated),
               "tile_gemm: unsupported shape ", m, "x", n, "x", k);
   if (bias) check_rows(*bias, n, "bias");
-  const TilePlan plan = tile_gemm_plan(m, n, k);
+  const TilePlan plan = tile_gemm_plan(m, n, k, a_flipped, b_flipped);
   auto out = torch::empty({m, gated ? n / 2 : n}, a.options());
   torch::Tensor shares;
   if (plan.shares())
@@ -1152,6 +1152,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("a_flipped"), py::arg("b_flipped"), py::arg("gated") = false,
         py::arg("gelu") = false);
   m.def("tile_gemm_good", &tile_gemm_good);
+  m.def("tile_gemm_rows", [](long m, long n, long k, bool a_flipped,
+                             bool b_flipped) {
+    return tile_gemm_plan(m, n, k, a_flipped, b_flipped).rows;
+  });
   m.def("rows_heads", &rows_heads);
   m.def("rows_normed", &rows_normed);
   m.def("quant_normed", &quant_normed);

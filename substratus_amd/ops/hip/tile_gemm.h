@@ -6,10 +6,13 @@
 // How a product's tiles are spread: the first `whole` by a workgroup each,
 // each of the others by `split` workgroups that share the inner dimension.
 struct TilePlan {
+  int rows;                       // of a tile: a multiple of 32, 128 to 256
   int tiles_m, tiles_n, whole, split;
   __host__ __device__ int rest() const { return tiles_m * tiles_n - whole; }
   // floats of the shares
-  long shares() const { return split > 1 ? (long)rest() * split * 65536 : 0; }
+  long shares() const {
+    return split > 1 ? (long)rest() * split * rows * 256 : 0;
+  }
   double us;                      // what it is to take
 };
 
@@ -30,7 +33,8 @@ struct TileGemm {
 
 bool tile_gemm_takes(long m, long n, long k, long a_ld, long b_ld,
                      bool a_flipped, bool b_flipped, bool gated);
-TilePlan tile_gemm_plan(long m, long n, long k);
+TilePlan tile_gemm_plan(long m, long n, long k, bool a_flipped,
+                        bool b_flipped);
 bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped,
                     bool gated);
 void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,

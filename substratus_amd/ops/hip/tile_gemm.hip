@@ -26,7 +26,15 @@
 // lane loads, since what is loaded directly lands in the order of lanes.
 //
 // A chip of 256 CUs takes 256 tiles at a time. Tiles left over from that share
-// the CUs along the inner dimension and leave 32-bit sums to a second kernel.
+// the CUs along the inner dimension and leave 32-bit sums to a second kernel. Or
+// tiles have fewer rows, 128 to 224, where those of 256 would leave CUs idle or be
+// partly empty (plan_of): regions of a's halves are not full then, nothing else
+// changes. us, MI355X, from 256 rows: 2331 x 2048 x 2048 35.6 -> 25.8 (128), 11264 x
+// 2048 x 2331, both flipped, 110 -> 104 (192), 2331 x 11264 x 2048 94 -> 88 (224), 908
+// x 11264 x 2048, gated, 45 -> 39 (192), 557 x 18176 x 4544, b flipped, 114 -> 93 (192).
+// Large ones are bound by power: with random numbers the chip holds 1.5 to 1.7 GHz, at
+// 2140 clocks a step of which matrix instructions take 2048 (zeros: 2.4 GHz, 2.1
+// PFLOP/s).
 //
 // TFLOP/s on a MI355X, the library -> this, m x n x k:
 //   neither flipped  4165 x 12288 x 4096  1045 -> 1343   (a prompt's products)
@@ -71,9 +79,9 @@ DEV_INLINE short8 join(uint2v a, uint2v b) {
   return __builtin_bit_cast(short8, (uint4v){a[0], a[1], b[0], b[1]});
 }
 
-// Transposing reads of two, or four, fragments of 16 rows x 64, at `AT` bytes
-// past the fragments' addresses, and the wait for them. (The compiler's own
-// form waits for all direct loads first.)
+// Transposing reads of two fragments of 16 rows x 64, or of two to four with
+// addresses of their own, at `AT` bytes past these, and the wait for them. (The
+// compiler's own form waits for all direct loads first.)
 template <int AT>
 DEV_INLINE void read_flipped2(short8 (&f)[2][2], unsigned p) {
   uint2v r[8];
@@ -100,8 +108,64 @@ DEV_INLINE void read_flipped2(short8 (&f)[2][2], unsigned p) {
 }
 
 template <int AT>
-DEV_INLINE void read_flipped4(short8 (&f)[4][2], unsigned p0, unsigned p1,
-                              unsigned p2, unsigned p3) {
+DEV_INLINE void read_flipped(short8 (&f)[2][2], unsigned p0, unsigned p1) {
+  uint2v r[8];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8 offset:%10\n\t"
+      "ds_read_b64_tr_b16 %1, %8 offset:%11\n\t"
+      "ds_read_b64_tr_b16 %2, %9 offset:%10\n\t"
+      "ds_read_b64_tr_b16 %3, %9 offset:%11\n\t"
+      "ds_read_b64_tr_b16 %4, %8 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %5, %8 offset:%13\n\t"
+      "ds_read_b64_tr_b16 %6, %9 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %7, %9 offset:%13\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]),
+        "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+      : "v"(p0), "v"(p1), "i"(AT), "i"(AT + 1024), "i"(AT + 8192),
+        "i"(AT + 9216)
+      : "memory");
+  #pragma unroll
+  for (int q = 0; q < 2; ++q)
+    #pragma unroll
+    for (int i = 0; i < 2; ++i)
+      f[i][q] = join(r[q * 4 + i * 2], r[q * 4 + i * 2 + 1]);
+}
+
+template <int AT>
+DEV_INLINE void read_flipped(short8 (&f)[3][2], unsigned p0, unsigned p1,
+                             unsigned p2) {
+  uint2v r[12];
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %12 offset:%15\n\t"
+      "ds_read_b64_tr_b16 %1, %12 offset:%16\n\t"
+      "ds_read_b64_tr_b16 %2, %13 offset:%15\n\t"
+      "ds_read_b64_tr_b16 %3, %13 offset:%16\n\t"
+      "ds_read_b64_tr_b16 %4, %14 offset:%15\n\t"
+      "ds_read_b64_tr_b16 %5, %14 offset:%16\n\t"
+      "ds_read_b64_tr_b16 %6, %12 offset:%17\n\t"
+      "ds_read_b64_tr_b16 %7, %12 offset:%18\n\t"
+      "ds_read_b64_tr_b16 %8, %13 offset:%17\n\t"
+      "ds_read_b64_tr_b16 %9, %13 offset:%18\n\t"
+      "ds_read_b64_tr_b16 %10, %14 offset:%17\n\t"
+      "ds_read_b64_tr_b16 %11, %14 offset:%18\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]),
+        "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7]), "=&v"(r[8]), "=&v"(r[9]),
+        "=&v"(r[10]), "=&v"(r[11])
+      : "v"(p0), "v"(p1), "v"(p2), "i"(AT), "i"(AT + 1024), "i"(AT + 8192),
+        "i"(AT + 9216)
+      : "memory");
+  #pragma unroll
+  for (int q = 0; q < 2; ++q)
+    #pragma unroll
+    for (int i = 0; i < 3; ++i)
+      f[i][q] = join(r[q * 6 + i * 2], r[q * 6 + i * 2 + 1]);
+}
+
+template <int AT>
+DEV_INLINE void read_flipped(short8 (&f)[4][2], unsigned p0, unsigned p1,
+                             unsigned p2, unsigned p3) {
   uint2v r[16];
   asm volatile(
       "ds_read_b64_tr_b16 %0, %16 offset:%20\n\t"
@@ -137,12 +201,12 @@ DEV_INLINE void read_flipped4(short8 (&f)[4][2], unsigned p0, unsigned p1,
 
 // Where a tile begins: LINES rows of tiles by columns. The last tiles reach
 // back instead of over the matrix' end; what two of them have is the same.
-template <bool GATED>
+template <bool GATED, int T>
 DEV_INLINE void tile_of(const TileGemm& g, const TilePlan& p, int tile,
                         int& m0, int& n0) {
   const int per = LINES * p.tiles_n, first = tile / per * LINES;
   const int lines = min(p.tiles_m - first, LINES);
-  m0 = min((first + tile % per % lines) * TILE, g.m - TILE);
+  m0 = min((first + tile % per % lines) * (T * 32), g.m - T * 32);
   const int wide = GATED ? TILE / 2 : TILE;
   n0 = min(tile % per / lines * wide, (GATED ? g.n / 2 : g.n) - wide);
 }
@@ -158,7 +222,7 @@ struct Item {
   int share;                      // -1: the whole tile
 };
 
-template <bool GATED>
+template <bool GATED, int T>
 DEV_INLINE Item item_of(const TileGemm& g, const TilePlan& p, int id) {
   const int pairs = pairs_of(g.k);
   Item it;
@@ -178,7 +242,7 @@ DEV_INLINE Item item_of(const TileGemm& g, const TilePlan& p, int id) {
     it.t1 = 2 * (int)((long)pairs * (part + 1) / p.split);
     if (p.split == 1) it.share = -1;
   }
-  tile_of<GATED>(g, p, tile, it.m0, it.n0);
+  tile_of<GATED, T>(g, p, tile, it.m0, it.n0);
   return it;
 }
 
@@ -203,8 +267,9 @@ DEV_INLINE int b_key(int r) { return (r & 3) | (r >> 1 & 4); }
 
 // The row and first column of a thread's eight outputs: accumulators (i, 2j)
 // and (i, 2j + 1), whose fragments' rows are interleaved by fours for that.
+template <int T>
 DEV_INLINE int out_row(int tid, int i) {
-  return (tid >> 8) * 128 + (i >> 2) * 64 + (i & 3) * 16 + (tid & 15);
+  return ((tid >> 8) * T + i) * 16 + (tid & 15);
 }
 DEV_INLINE int out_col(int tid, int j) {
   return (tid >> 6 & 3) * 64 + j * 32 + (tid >> 4 & 3) * 8;
@@ -236,7 +301,9 @@ DEV_INLINE float4v gelu(float4v a) {
   return v;
 }
 
-template <bool FA, bool FB, bool GATED, bool GELU = false>
+// T: fragments of 16 rows that a wave has, the first half of them (one more of
+// odd numbers) in the low regions.
+template <bool FA, bool FB, bool GATED, bool GELU, int T>
 __global__ __launch_bounds__(THREADS, 2)
 void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   // [two steps][a low, a high, b low, b high]
@@ -245,30 +312,51 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   const int lane = threadIdx.x % WAVE, lo = lane & 15, gr = lane >> 4;
   const int wm = wave >> 2, wn = wave & 3;
   static_assert(!GATED || !FB);
-  const Item it = item_of<GATED>(g, plan, blockIdx.x);
+  const Item it = item_of<GATED, T>(g, plan, blockIdx.x);
+  constexpr int LOW = (T + 1) / 2, HIGH = T - LOW;
+  // loads of a thread, of a region: two of 128 rows, or of a flipped operand's
+  constexpr int ROWS[4] = {FA ? 4 : LOW, FA ? 4 : HIGH, 4, 4};  // of either half
+  constexpr int N0 = (ROWS[0] + 1) / 2, N1 = (ROWS[1] + 1) / 2, NB = 2;
+  constexpr int ALL = N0 + N1 + 2 * NB;
 
-  // Loads: a wave has two KB of a region. Of rows: 8 lines of 128 bytes a KB,
-  // of a flipped operand 4 of 256. off: from the low region's first byte on.
-  unsigned off[2][2];
+  // Loads: KBs of a region, 8 lines of 128 bytes each of rows, of a flipped operand
+  // 4 lines of 256. Of regions of fewer rows than 128 the first ones of either half
+  // are there; a wave that has none left takes its own again. off: from the low
+  // region's first byte on.
   const int piece_f = lane & 15, piece_r = lane & 7;
+  // a KB's place in a region of rows, in eights of them
+  auto kb_of = [&](int rows, int p) {
+    const int kb = rows == 4 ? wave * 2 + p : p == 0 || wave >= 4 ? wave
+                                                                  : 8 + wave;
+    return kb / (2 * rows) * 8 + kb % (2 * rows);
+  };
+  unsigned off[4][2];
   #pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const int r = (wave * 2 + p) * 8 + (lane >> 3);
-    const int line = (wave * 2 + p) * 4 + (lane >> 4);
-    const int qa = piece_f ^ ((line & 3) << 1);
-    const int qb = piece_f ^ ((line & 3) << 2);
-    off[0][p] = FA
-        ? (unsigned)(line * g.a_ld + (qa >> 3) * 128 + (qa & 7) * 8) * 2u
-        : (unsigned)(((r >> 6) * 128 + (r & 63)) * g.a_ld) * 2u +
-              (piece_r ^ a_key(r)) * 16;
-    off[1][p] = FB
-        ? (unsigned)(line * g.b_ld + (qb >> 2) * 64 + (qb & 3) * 8) * 2u
-        : (unsigned)((GATED ? r : (r >> 5) * 64 + (r & 31)) * g.b_ld) * 2u +
-              (piece_r ^ b_key(r)) * 16;
-  }
+  for (int e = 0; e < 4; ++e)
+    #pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int r = kb_of(ROWS[e], p) * 8 + (lane >> 3);
+      const int line = (wave * 2 + p) * 4 + (lane >> 4);
+      const int qa = piece_f ^ ((line & 3) << 1);
+      const int qb = piece_f ^ ((line & 3) << 2);
+      if (e < 2) {
+        off[e][p] = FA
+            ? (unsigned)(line * g.a_ld + (qa >> 3) * (T * 16) + (qa & 7) * 8) *
+                  2u
+            : (unsigned)(((r >> 6) * (T * 16) + (r & 63)) * g.a_ld) * 2u +
+                  (piece_r ^ a_key(r)) * 16;
+        if (FA && (qa & 7) >= 2 * (e == 0 ? LOW : HIGH)) off[e][p] = PAST;
+      } else {
+        off[e][p] = FB
+            ? (unsigned)(line * g.b_ld + (qb >> 2) * 64 + (qb & 3) * 8) * 2u
+            : (unsigned)((GATED ? r : (r >> 5) * 64 + (r & 31)) * g.b_ld) *
+                      2u +
+                  (piece_r ^ b_key(r)) * 16;
+      }
+    }
   const long a_step = (FA ? g.a_ld : 1) * STEP * 2;
   const long b_step = (FB ? g.b_ld : 1) * STEP * 2;
-  const int a_high = (FA ? 1 : g.a_ld) * 64 * 2;
+  const int a_high = (FA ? 1 : g.a_ld) * (LOW * 16) * 2;
   const int b_high = (FB ? 1 : g.b_ld) * (GATED ? g.n / 2 : 32) * 2;
   // What is loaded, two steps ahead of what is multiplied: by buffer loads,
   // whose only vector operand is the offset.
@@ -282,19 +370,23 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
     const auto from = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(region < 2 ? la : lb), 0, 0x80000000u, RAW);
     const int high = region & 1 ? (region < 2 ? a_high : b_high) : 0;
-    uint4* to = s + (buf * 4 + region) * REGION + wave * 128;
+    constexpr int LOADS[4] = {N0, N1, NB, NB};
+    uint4* to = s + (buf * 4 + region) * REGION;
+    const bool flipped = region < 2 ? FA : FB;
     #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      unsigned o = off[region >> 1][p];
+    for (int p = 0; p < LOADS[region]; ++p) {
+      unsigned o = off[region][p];
+      const int kb = flipped ? wave * 2 + p : kb_of(ROWS[region], p);
       if constexpr (!decltype(whole)::value) {
-        const int r = (wave * 2 + p) * 8 + (lane >> 3);
-        const int at = (region < 2 ? FA : FB)
-            ? (wave * 2 + p) * 4 + (lane >> 4)
+        const int r = kb * 8 + (lane >> 3);
+        const int at = flipped
+            ? kb * 4 + (lane >> 4)
             : (piece_r ^ (region < 2 ? a_key(r) : b_key(r))) * 8;
         if (at >= g.k - lt * STEP) o = PAST;
       }
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          from, (__attribute__((address_space(3))) unsigned int*)(to + p * 64),
+          from,
+          (__attribute__((address_space(3))) unsigned int*)(to + kb * 64),
           16, o, high, 0, 0);
     }
   };
@@ -304,8 +396,8 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
     lb += b_step;
   };
 
-  float4v acc[8][4];
-  short8 af[4][2], bl[2][2][2], bh[2][2];
+  float4v acc[T][4];
+  short8 al[LOW][2], ah[HIGH][2], bl[2][2][2], bh[2][2];
 
   // flipped: a lane's place in a transposing read of the first fragment
   const int place16 = ((gr * 8 + (lo >> 2)) * 16) * 16;
@@ -314,18 +406,24 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
       (((wm * 8 + ((lo & 3) >> 1)) ^ ((lo >> 2) << 1)) * 16);
   const unsigned at_b = base + place16 +
       (((wn * 4 + (lo & 3)) ^ ((lo >> 2) << 2)) * 16);
-  auto read_a = [&](auto buf, auto half) {
+  auto read_a = [&](auto buf, auto half, auto& f) {
     constexpr int BUF = decltype(buf)::value, H = decltype(half)::value;
+    constexpr int COUNT = sizeof(f) / sizeof(f[0]);
     if constexpr (FA) {
       const unsigned p = at_a + BUF * 4 * REGION * 16;
-      read_flipped4<H * REGION * 16>(af, p, p ^ 32, p ^ 64, p ^ 96);
+      if constexpr (COUNT == 4)
+        read_flipped<H * REGION * 16>(f, p, p ^ 32, p ^ 64, p ^ 96);
+      else if constexpr (COUNT == 3)
+        read_flipped<H * REGION * 16>(f, p, p ^ 32, p ^ 64);
+      else
+        read_flipped<H * REGION * 16>(f, p, p ^ 32);
     } else {
       const uint4* r = s + (BUF * 4 + H) * REGION + (wm * 64 + lo) * 8;
       #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < COUNT; ++i)
         #pragma unroll
         for (int q = 0; q < 2; ++q)
-          af[i][q] = *reinterpret_cast<const short8*>(
+          f[i][q] = *reinterpret_cast<const short8*>(
               r + i * 128 + ((q * 4 + gr) ^ (lo & 7)));
     }
   };
@@ -345,21 +443,22 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
               r + i * 32 + ((q * 4 + gr) ^ (lo & 7)));
     }
   };
-  // the phase's reads are done, and so are the loads of the next one's
-  auto turn = [&]() {
+  // the phase's reads are done, and so are the loads of the next one's, behind
+  // which no more than N were issued
+  auto turn = [&](auto n) {
     wait_lds_reads();
-    wait_loads<12>();
+    wait_loads<decltype(n)::value>();
     barrier();
   };
-  auto take = [&](int i0, int j0, const short8 (&f)[2][2]) {
+  auto take = [&](int i0, int j0, const auto& fa, const short8 (&f)[2][2]) {
     #pragma unroll
     for (int q = 0; q < 2; ++q)
       #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < (int)(sizeof(fa) / sizeof(fa[0])); ++i)
         #pragma unroll
         for (int j = 0; j < 2; ++j)
           acc[i0 + i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              f[j][q], af[i][q], acc[i0 + i][j0 + j], 0, 0, 0);
+              f[j][q], fa[i][q], acc[i0 + i][j0 + j], 0, 0, 0);
     barrier();
   };
   using std::integral_constant;
@@ -368,23 +467,23 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   auto step = [&](auto buf, auto whole) {
     constexpr int B = decltype(buf)::value;
     constexpr integral_constant<int, B ^ 1> other{};
-    read_a(buf, low);
+    read_a(buf, low, al);
     load(whole, B, 2);
-    turn();
-    take(0, 0, bl[B]);
+    turn(integral_constant<int, ALL + N1 + NB>{});
+    take(0, 0, al, bl[B]);
     read_b(buf, high, bh);
     load(whole, B, 0);
-    turn();
-    take(0, 2, bh);
-    read_a(buf, high);
+    turn(integral_constant<int, ALL + NB + N0>{});
+    take(0, 2, al, bh);
+    read_a(buf, high, ah);
     load(whole, B, 3);
-    turn();
-    take(4, 2, bh);
+    turn(integral_constant<int, ALL + N0 + NB>{});
+    take(LOW, 2, ah, bh);
     read_b(other, low, bl[B ^ 1]);
     load(whole, B, 1);
     advance();
-    turn();
-    take(4, 0, bl[B]);
+    turn(integral_constant<int, ALL + NB + N1>{});
+    take(LOW, 0, ah, bl[B]);
   };
   constexpr std::true_type whole{};
   constexpr std::false_type any{};
@@ -398,10 +497,10 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
     advance();
   }
   #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < T; ++i)
     #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
-  wait_loads<12>();
+  wait_loads<ALL + NB + N1>();
   barrier();
   read_b(low, low, bl[0]);
   wait_lds_reads();
@@ -426,9 +525,9 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
 
   const int tid = threadIdx.x;
   if (it.share >= 0) {
-    float4v* to = shares + (long)it.share * (32 * THREADS) + tid;
+    float4v* to = shares + (long)it.share * (4 * T * THREADS) + tid;
     #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < T; ++i)
       #pragma unroll
       for (int j = 0; j < 4; ++j) to[(i * 4 + j) * THREADS] = acc[i][j];
     return;
@@ -439,8 +538,8 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   for (int j = 0; j < 4; ++j)
     add[j] = bias_of(g, col_of<GATED>(g, it.n0, tid, j));
   #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = it.m0 + out_row(tid, i);
+  for (int i = 0; i < T; ++i) {
+    const int row = it.m0 + out_row<T>(tid, i);
     #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] += add[j];
     if constexpr (GELU) {
@@ -459,17 +558,17 @@ void tile_gemm_kernel(TileGemm g, TilePlan plan, float4v* __restrict__ shares) {
   }
 }
 
-// The shares of the tiles left over are added up, an eighth of a tile per
-// workgroup.
-template <bool GATED, bool GELU = false>
+// The shares of the tiles left over are added up, 32 rows of a tile per workgroup.
+template <bool GATED, bool GELU, int T>
 __global__ __launch_bounds__(THREADS)
 void tile_sum_kernel(TileGemm g, TilePlan plan,
                      const float4v* __restrict__ shares) {
   int m0, n0;
-  tile_of<GATED>(g, plan, plan.whole + blockIdx.x, m0, n0);
+  tile_of<GATED, T>(g, plan, plan.whole + blockIdx.x, m0, n0);
   const int tid = threadIdx.x, i = blockIdx.y;
   const float4v* from = shares +
-      (long)blockIdx.x * plan.split * (32 * THREADS) + i * 4 * THREADS + tid;
+      (long)blockIdx.x * plan.split * (4 * T * THREADS) + i * 4 * THREADS +
+      tid;
   float4v v[4];
   #pragma unroll
   for (int j = 0; j < 4; ++j) v[j] = from[j * THREADS];
@@ -477,14 +576,14 @@ void tile_sum_kernel(TileGemm g, TilePlan plan,
   for (int p = 1; p < plan.split; ++p)
     #pragma unroll
     for (int j = 0; j < 4; ++j)
-      v[j] += from[(long)p * 32 * THREADS + j * THREADS];
+      v[j] += from[(long)p * 4 * T * THREADS + j * THREADS];
   #pragma unroll
   for (int j = 0; j < 4; ++j) v[j] += bias_of(g, col_of<GATED>(g, n0, tid, j));
   if constexpr (GELU) {
     #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = gelu(v[j]);
   }
-  const int row = m0 + out_row(tid, i);
+  const int row = m0 + out_row<T>(tid, i);
   if constexpr (GATED) {
     store(g, g.n / 2, row, col_of<true>(g, n0, tid, 0), gate(v[0], v[2]),
           gate(v[1], v[3]));
@@ -514,22 +613,35 @@ bool tile_gemm_takes(long m, long n, long k, long a_ld, long b_ld,
          fits(m, a_ld, a_flipped) && fits(n, b_ld, b_flipped);
 }
 
-TilePlan tile_gemm_plan(long m, long n, long k) {
+// us on a MI355X, by a fit of 2055 products of 260 to 6000 rows with matrices of 2048
+// to 28672 rows and columns, tiles of 128 to 256 rows, a pass over memory before each
+// (rms 8 %): a step of a tile where all CUs have one, and where few do (the chip holds
+// a higher clock then); what a round, all rounds and the sum of shares begin and end
+// with; a tile's share's way through memory. Of the five heights the plan's is 0.6 %
+// slower than the best, 256 rows by themselves 5 %. A step of fewer rows reads LDS, and
+// turns a flipped operand, for longer than it multiplies.
+static TilePlan plan_of(long m, long n, long k, int rows, bool a_flipped,
+                        bool b_flipped) {
   TilePlan p;
-  p.tiles_m = (int)((m + TILE - 1) / TILE);
+  p.rows = rows;
+  p.tiles_m = (int)((m + rows - 1) / rows);
   p.tiles_n = (int)((n + TILE - 1) / TILE);
   const long tiles = (long)p.tiles_m * p.tiles_n;
   const long steps = 2 * pairs_of(k);
   const long rest = tiles % 256, rounds = tiles / 256;
-  // us on a MI355X: a step of a tile 1.5, a round's beginning and end 5, the
-  // sum of shares 5 and their way through memory
-  const double full = rounds * (steps * 1.5 + 5.);
+  constexpr double STEP_US[3][5] = {{0.843, 0.958, 1.083, 1.188, 1.301},
+                                    {1.035, 1.161, 1.265, 1.343, 1.398},
+                                    {1.028, 1.162, 1.314, 1.443, 1.540}};
+  const double step =
+      STEP_US[a_flipped ? 2 : b_flipped ? 1 : 0][rows / 32 - 4];
+  auto busy = [&](long tiles) { return 0.78 + 0.22 * tiles / 256.; };
+  const double full = 2.4 + rounds * (steps * step + 5.5);
   p.whole = (int)tiles;
   p.split = 1;
-  p.us = full + (rest ? steps * 1.5 + 5. : 0.);
+  p.us = full + (rest ? steps * step * busy(rest) + 5.5 : 0.);
   for (int s = 2; rest && rest * s <= 256 && steps / s >= 4; ++s) {
-    const double us = full + (steps + s - 1) / s * 1.5 + 10. +
-                      rest * s * (0.262144 * 2 / 5.);
+    const double us = full + (steps + s - 1) / s * step * busy(rest * s) + 5.5 +
+                      rest * s * rows * (0.0127 / 32);
     if (us < p.us) {
       p.us = us;
       p.whole = (int)(tiles - rest);
@@ -539,55 +651,84 @@ TilePlan tile_gemm_plan(long m, long n, long k) {
   return p;
 }
 
+TilePlan tile_gemm_plan(long m, long n, long k, bool a_flipped,
+                        bool b_flipped) {
+  TilePlan best = plan_of(m, n, k, TILE, a_flipped, b_flipped);
+  for (int rows = 128; rows < TILE; rows += 32) {
+    const TilePlan p = plan_of(m, n, k, rows, a_flipped, b_flipped);
+    if (p.us < (best.rows == TILE ? 0.97 : 1.) * best.us) best = p;
+  }
+  return best;
+}
+
 // Whether the library's product would take longer. What that takes is no smooth
-// function of sizes; by itself it is often a few percent faster, but it writes
-// past the caches, and the pass that reads the results pays for it (2331 x 32000
-// x 2048 0.97, a step's loss after it 90 us instead of 73). So this goes by the
-// product and a pass that reads its results together, less that pass: the
-// library's time over this one's, MI355X, weights that come from memory, 1024 to
-// 8192 rows, matrices of 2048 to 32000 rows and columns, by planned PFLOP/s:
-//   neither flipped   from 0.9 on 158 products of 0.97 to 1.98 (three of 3000
-//                     rows and more x 32000, whose results no cache holds,
-//                     below 0.99; 2331 x 32000 x 2048 1.05, 4096 x 18176 x 4544
-//                     1.25); by themselves 0.92 to 1.9. Whole tiles in whole
-//                     rounds, 1.01 to 1.09, stay with the library: by themselves
-//                     0.94 to 1.0
-//   b flipped         shared ones from 0.7 on, others from 0.9 on where tiles
-//                     take more than three quarters of their rounds' CUs: 155 of
-//                     0.98 to 2.48. Others: 0.86 to 1.69 (2331 x 4096 x 22016,
-//                     160 tiles, 0.86)
-//   both flipped      0.39: 0.90; from 0.7 on 119 of 1.02 to 1.42 by themselves
-//   gated             from 0.9 on 35 of 1.03 and more, whole rounds too: the
-//                     pass that gates them is a tenth of the product
+// function of sizes, so this goes by planned PFLOP/s, and where the lines lie by what
+// all products beyond them gain together. The library's time over this one's, MI355X,
+// 260 to 6000 rows, matrices of 2048 to 28672 rows and columns, a pass over memory
+// before each product as in a model's step:
+//   neither flipped   of 101, all 1.06 (the worst 0.80); from 1.0 on 42 that go, of
+//                     0.96 to 1.9, 1.14 together. From 0.9 on three more, and 3330 x
+//                     2048 x 5632, which lost in a model (0.91). Shares of a single
+//                     round with rows of a multiple of 8 KB, which meet at few of the
+//                     memory's channels, stay (577 x 8192 x 8192 0.77), whole tiles of
+//                     whole rounds stay (by themselves 0.94 to 1.09; the library
+//                     writes past the caches, though, and the pass that reads the
+//                     results pays for that: 2331 x 32000 x 2048 0.97, a step's loss
+//                     after it 90 us instead of 73)
+//   b flipped         of 199, all 1.11; 89 that go, of 0.90 to 2.57, 1.22 together. In
+//                     three and more shares from 0.7 on (36 of 1.03 and more), others
+//                     from 0.85 on (two shares below that 0.82 to 1.01); few rows with
+//                     lines of a multiple of 16 KB stay (483 x 8192 x 3072 0.65)
+//   both flipped      of 111, all 1.22, one slower (0.95); of rows this short that it
+//                     plans less than 0.5 none was slower either, nor much faster
+//   gated             from 0.5 on 22 of 1.08 to 1.70 over the product and the pass
+//                     that gates it; below four of 0.95 to 1.19
+// Of tiles of 256 rows that would take half to three quarters of their rounds' CUs the
+// first two stay with the library, though by tiles of fewer rows they no longer lose:
+// no more than these 5 % of all products.
 bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped,
                     bool gated) {
-  const TilePlan p = tile_gemm_plan(m, n, k);
+  const TilePlan p = tile_gemm_plan(m, n, k, a_flipped, b_flipped);
   const double rate = 2e-9 * m * n * k / p.us;        // PFLOP/s
-  const long tiles = (long)p.tiles_m * p.tiles_n;
-  const long places = (tiles + 255) / 256 * 256;
-  if (a_flipped) return rate >= 0.7;
+  if (a_flipped || gated) return rate >= 0.5;
+  const TilePlan whole = plan_of(m, n, k, TILE, false, b_flipped);
+  const long high = whole.tiles_m * (long)whole.tiles_n;
+  if (whole.split == 1 && 4 * high <= 3 * ((high + 255) / 256 * 256))
+    return false;
   if (b_flipped)
-    return p.split > 1 ? rate >= 0.7 : rate >= 0.9 && 4 * tiles > 3 * places;
-  const bool even = m % TILE == 0 && n % TILE == 0 && tiles == places;
-  return rate >= 0.9 && (gated || !even);
+    return rate >= (p.split > 2 ? 0.7 : 0.85) && (m >= 1024 || n % 8192 != 0);
+  const long tiles = p.tiles_m * (long)p.tiles_n;
+  const bool even = m % p.rows == 0 && n % TILE == 0 && tiles % 256 == 0;
+  const bool meet = p.whole == 0 && k % 4096 == 0;
+  return rate >= 1. && !even && !meet;
 }
 
 void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,
                       hipStream_t stream) {
   float4v* sh = reinterpret_cast<float4v*>(shares);
   const dim3 grid(plan.whole + plan.rest() * plan.split);
-  auto kernel = g.gated ? tile_gemm_kernel<false, false, true>
-      : g.gelu ? tile_gemm_kernel<false, false, false, true>
-      : g.a_flipped
-          ? (g.b_flipped ? tile_gemm_kernel<true, true, false>
-                         : tile_gemm_kernel<true, false, false>)
-          : (g.b_flipped ? tile_gemm_kernel<false, true, false>
-                         : tile_gemm_kernel<false, false, false>);
-  kernel<<<grid, dim3(THREADS), 0, stream>>>(g, plan, sh);
-  if (plan.split > 1) {
-    auto sum = g.gated ? tile_sum_kernel<true>
-               : g.gelu ? tile_sum_kernel<false, true>
-                        : tile_sum_kernel<false>;
-    sum<<<dim3(plan.rest(), 8), dim3(THREADS), 0, stream>>>(g, plan, sh);
+  auto go = [&](auto t) {
+    constexpr int T = decltype(t)::value;
+    auto kernel = g.gated ? tile_gemm_kernel<false, false, true, false, T>
+        : g.gelu ? tile_gemm_kernel<false, false, false, true, T>
+        : g.a_flipped
+            ? (g.b_flipped ? tile_gemm_kernel<true, true, false, false, T>
+                           : tile_gemm_kernel<true, false, false, false, T>)
+            : (g.b_flipped ? tile_gemm_kernel<false, true, false, false, T>
+                           : tile_gemm_kernel<false, false, false, false, T>);
+    kernel<<<grid, dim3(THREADS), 0, stream>>>(g, plan, sh);
+    if (plan.split > 1) {
+      auto sum = g.gated ? tile_sum_kernel<true, false, T>
+                 : g.gelu ? tile_sum_kernel<false, true, T>
+                          : tile_sum_kernel<false, false, T>;
+      sum<<<dim3(plan.rest(), T), dim3(THREADS), 0, stream>>>(g, plan, sh);
+    }
+  };
+  switch (plan.rows / 32) {
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    default: go(std::integral_constant<int, 8>{});
   }
 }

@@ -74,6 +74,43 @@ def test_gated(m, f, k, bias):
                  2.0 ** -8 * want.abs() + room).all())
 
 
+def gated_close(got, a, b):
+    g, u = (a.double() @ b.double().T).chunk(2, 1)
+    want = torch.nn.functional.silu(g) * u
+    room = 2.0 ** -17 * (g.abs() + 1) * (u.abs() + 1)   # as in test_gated
+    assert bool(((got.double() - want).abs() <=
+                 2.0 ** -8 * want.abs() + room).all())
+
+
+# Tiles of fewer rows, the last one of a few rows, or of all but one or eight: the first
+# numbers of rows, of columns, that are cut into such tiles.
+@pytest.mark.parametrize("height", [128, 160, 192, 224])
+@pytest.mark.parametrize("over", [5, -1])
+@pytest.mark.parametrize("k", [2120, 4168])
+@pytest.mark.parametrize("kind", ["plain", "gelu", "gated", "b", "both"])
+def test_heights(height, over, k, kind):
+    torch.manual_seed(height + k)
+    fa, fb = kind == "both", kind in ("b", "both")
+    by = 8 if fa else 1
+    m, n = next(((m, n) for m in range(3 * height + by * over, 8192, height)
+                 for n in (1296, 3600, 4560, 9232)
+                 if _C.tile_gemm_rows(m, n, k, fa, fb) == height), (0, 0))
+    if m == 0:
+        assert (kind, height, over) == ("b", 224, 5)
+        pytest.skip("cut into other tiles")
+    a, b = operand(m, k, fa, 8), operand(n, k, fb, 8)
+    if kind in ("gelu", "gated"):
+        b = (b / k ** 0.5).bfloat16()
+    bias = torch.randn(n, device=DEV).bfloat16() if kind == "plain" else None
+    got = _C.tile_gemm(a, b, bias, fa, fb, kind == "gated", kind == "gelu")
+    if kind == "gated":
+        gated_close(got, a, b)
+    elif kind == "gelu":
+        assert torch.equal(got, ops.gelu(_C.tile_gemm(a, b, None, fa, fb)))
+    else:
+        close(got, a.T if fa else a, b.T if fb else b, bias)
+
+
 def test_rows_of_any_number():
     """Rows that are not flipped need not come in eights."""
     a, b = operand(321, 192, False, 0), operand(264, 192, False, 0)
