@@ -4,7 +4,9 @@
 // weights; the formulas are in attention_ctx.hip. Rows of a portion carry
 // their absolute positions, so a prompt can be cut anywhere.
 //
-// The structure is that of attention_v5.hip: every wave owns 32 query rows
+// A step's chain (products of scores, weights, products of values, the barrier) is what
+// bounds it: 3 us of a wave alone on its SIMD, 4.5 of two; memory and the matrix cores
+// wait. The structure is that of attention_v5.hip: every wave owns 32 query rows
 // kept in registers, 64 keys per step go through LDS, S^T = K Q^T leaves a
 // lane with scores of its own query row only, and softmax stays in registers.
 // Differences:
@@ -16,6 +18,8 @@
 //     with 16 mantissa bits, so softmax weights keep more than bf16 carries;
 //   * keys and values may also lie unpaged, projected for this step from what
 //     the cache holds (FLAT), with a key part that all heads share;
+//   * where tiles of the most rows are too few for the chip, two waves share 32 rows
+//     and take every other 32 keys; their sums meet in LDS at the end;
 //   * V is staged with keys 4..7 and 8..11 of every 16 exchanged, which is
 //     the order in which the score accumulators hold them: weights need no
 //     lane exchange before the second product.
@@ -42,11 +46,14 @@ enum Kind {
   SIGMOID,    // weights are sigmoids: no maximum, no sum
 };
 
-template <int KK, int DC, int WAVES, bool FLAT, Kind KIND>
+// SH: waves that share their 32 query rows, each a part of a step's keys
+template <int KK, int DC, int WAVES, int SH, bool FLAT, Kind KIND>
 __global__ __launch_bounds__(WAVES * WAVE)
 void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
   constexpr int THREADS = WAVES * WAVE;
-  constexpr int QT = WAVES * 32;            // query rows per workgroup
+  constexpr int RW = WAVES / SH;            // waves of unlike rows
+  constexpr int QT = RW * 32;               // query rows per workgroup
+  constexpr int NS = CH / 32 / SH;          // a wave's keys of a step, by 32
   constexpr int KROW = KK * 16 + 8;         // padded LDS row, in elements
   constexpr int BW = QT + CH - 1;           // distances met in one step
   constexpr int LK = (CH * KK * 2 + THREADS - 1) / THREADS;
@@ -73,10 +80,12 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
   const int from = FLAT ? flat_from(a.window, pos0) : 0;
   const long flat0 = FLAT ? (long)a.ctx_start[e] - from : 0;
   const int qa0 = pos0 + q0_tile;                // first position of the tile
-  const int qw0 = qa0 + wave * 32;               // first position of the wave
+  const int part_of = SH > 1 ? wave / RW : 0;    // which of a step's keys
+  const int rw = SH > 1 ? wave % RW : wave;
+  const int qw0 = qa0 + rw * 32;                 // first position of the wave
   const bool wave_live = qw0 < total;
   const int qpos = qw0 + lo5;
-  const int row = min(q0_tile + wave * 32 + lo5, en.n - 1);
+  const int row = min(q0_tile + rw * 32 + lo5, en.n - 1);
   const int lo = first_seen(a, qpos), lo_wave = first_seen(a, qw0);
   const int hi_wave = min(qw0 + 31, total - 1);
   // lo of the wave's last row: keys at or above it are inside every range
@@ -96,7 +105,7 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
     }
   }
   float m = -INFINITY, l = 0.f;
-  if (a.sink != nullptr) { m = a.sink[head] * LOG2E; l = 1.f; }
+  if (a.sink != nullptr && part_of == 0) { m = a.sink[head] * LOG2E; l = 1.f; }
   float16v o_t[DC];
   #pragma unroll
   for (int c = 0; c < DC; ++c) o_t[c] = (float16v){};
@@ -107,6 +116,8 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
   int pgk[LK], pgv[LV];                          // page bases, -1: no key
   uint4 st_k[LK], st_v[LV];
   float st_b = 0.f;
+  const float fall1 = a.r1 != nullptr ? a.r1[head] : 0.f;
+  const float fall2 = a.r1 != nullptr ? a.r2[head] : 0.f;
   const float wb2 = KIND == SIGMOID ? a.wbias[head] * LOG2E : 0.f;
 
   auto pages = [&](int it) {
@@ -158,11 +169,13 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
             a.vc + (((long)pgv[i] * a.kv_heads + kvh) * PAGE +
                     (st * CH + r) % PAGE) * a.v_ld + d);
     }
-    if (a.bias != nullptr || a.r1 != nullptr)
-      st_b = distance_bias2(a, head, qa0 - (st * CH + CH - 1) + tid);
-    if constexpr (KIND == SIGMOID) st_b += wb2;
+    if (!FLAT && a.bias != nullptr)
+      st_b = a.bias[(long)head * a.nbias +
+                    min(max(qa0 - (st * CH + CH - 1) + tid, 0), a.nbias - 1)];
   };
-  auto stage_write = [&](int buf) {
+  // nothing is worked out from what was loaded before this: it would be waited for
+  // ahead of a step's products
+  auto stage_write = [&](int it, int buf) {
     #pragma unroll
     for (int i = 0; i < LK; ++i) {
       const int f = i * THREADS + tid;
@@ -182,13 +195,20 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
                 [col % 16]) = st_v[i];
       }
     }
-    s_b[buf][tid] = st_b;
+    if constexpr (FLAT) return;                  // distances change nothing
+    float b = st_b * LOG2E;
+    if (a.r1 != nullptr) {
+      const int n = qa0 - (part.at(it) * CH + CH - 1) + tid;
+      b -= fall1 * __builtin_amdgcn_logf(1.f + fall2 * (float)max(n, 0));
+    }
+    if constexpr (KIND == SIGMOID) b += wb2;
+    s_b[buf][tid] = b;
   };
 
   pages(0);
   stage_load(0);
   pages(1);
-  stage_write(0);
+  stage_write(0, 0);
   __syncthreads();
 
   for (int it = 0; it < part.n; ++it) {
@@ -197,34 +217,36 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
       stage_load(it + 1);
       pages(it + 2);
     }
-    const int kbase = part.at(it) * CH;
+    const int kbase = part.at(it) * CH + part_of * NS * 32;
     if (wave_live && kbase <= hi_wave &&
-        (kbase + CH > lo_wave || kbase < a.keep)) {
-      float16v sacc[CH / 32];
+        (kbase + NS * 32 > lo_wave || kbase < a.keep)) {
+      const int sc0 = part_of * NS;
+      float16v sacc[NS];
       #pragma unroll
-      for (int sc = 0; sc < CH / 32; ++sc) {
+      for (int sc = 0; sc < NS; ++sc) {
         sacc[sc] = (float16v){};
         #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
           const short8 ka = *reinterpret_cast<const short8*>(
-              &s_k[cur][sc * 32 + lo5][kk * 16 + hi * 8]);
+              &s_k[cur][(sc0 + sc) * 32 + lo5][kk * 16 + hi * 8]);
           sacc[sc] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               ka, qreg[kk], sacc[sc], 0, 0, 0);
         }
       }
-      float sv[CH / 32][16];
-      const float* bw = &s_b[cur][wave * 32 + lo5 + CH - 1 - 4 * hi];
+      float sv[NS][16];
+      const float* bw =
+          &s_b[cur][rw * 32 + lo5 + CH - 1 - 4 * hi - sc0 * 32];
       #pragma unroll
-      for (int sc = 0; sc < CH / 32; ++sc)
+      for (int sc = 0; sc < NS; ++sc)
         #pragma unroll
         for (int r = 0; r < 16; ++r)
           sv[sc][r] = (KIND == CAP ? cap2 * tanh_exp2(sacc[sc][r] * cscale)
                                    : sacc[sc][r] * scale2) +
-                      bw[-(sc * 32 + (r & 3) + 8 * (r >> 2))];
+                      (FLAT ? 0.f : bw[-(sc * 32 + (r & 3) + 8 * (r >> 2))]);
       // steps inside every row's range need no mask
-      if (kbase < lo_last || kbase + CH - 1 > qw0 || qw0 + 31 >= total) {
+      if (kbase < lo_last || kbase + NS * 32 - 1 > qw0 || qw0 + 31 >= total) {
         #pragma unroll
-        for (int sc = 0; sc < CH / 32; ++sc)
+        for (int sc = 0; sc < NS; ++sc)
           #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int kpos =
@@ -237,7 +259,7 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
       if constexpr (KIND != SIGMOID) {
         float mloc = -INFINITY;
         #pragma unroll
-        for (int sc = 0; sc < CH / 32; ++sc)
+        for (int sc = 0; sc < NS; ++sc)
           #pragma unroll
           for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sv[sc][r]);
         mloc = across<32>(mloc, Larger{});
@@ -254,9 +276,11 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
             for (int r = 0; r < 16; ++r) o_t[c][r] *= keep;
         }
       }
+      // -inf less this is -inf: a weight of 0
+      const float mf = m == -INFINITY ? 0.f : m;
       float sum = 0.f;
       #pragma unroll
-      for (int sc = 0; sc < CH / 32; ++sc) {
+      for (int sc = 0; sc < NS; ++sc) {
         #pragma unroll
         for (int g = 0; g < 2; ++g) {
           unsigned wh[4], wl[4];
@@ -269,8 +293,8 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
               p0 = sigmoid_exp2(s0);
               p1 = sigmoid_exp2(s1);
             } else {
-              p0 = s0 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s0 - m);
-              p1 = s1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s1 - m);
+              p0 = __builtin_amdgcn_exp2f(s0 - mf);
+              p1 = __builtin_amdgcn_exp2f(s1 - mf);
               sum += p0 + p1;
             }
             wh[i] = cvt_pk_bf16(p0, p1);
@@ -282,9 +306,9 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
           #pragma unroll
           for (int c = 0; c < DC; ++c) {
             const short4v v0 =
-                tr16_read(&s_v[cur][c][sc][g][0][0][0] + lane * 4);
+                tr16_read(&s_v[cur][c][sc0 + sc][g][0][0][0] + lane * 4);
             const short4v v1 =
-                tr16_read(&s_v[cur][c][sc][g][1][0][0] + lane * 4);
+                tr16_read(&s_v[cur][c][sc0 + sc][g][1][0][0] + lane * 4);
             short8 vt;
             #pragma unroll
             for (int j = 0; j < 4; ++j) { vt[j] = v0[j]; vt[4 + j] = v1[j]; }
@@ -297,11 +321,44 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
       }
       if constexpr (KIND != SIGMOID) l += across<32>(sum, Plus{});
     }
-    if (it + 1 < part.n) stage_write(cur ^ 1);
+    if (it + 1 < part.n) stage_write(it + 1, cur ^ 1);
     __syncthreads();
   }
 
-  if (wave_live && qpos < total) {
+  if constexpr (SH > 1) {
+    // the second wave's sums join the first's, 32 columns at a time
+    static_assert(SH == 2 && sizeof(s_k) >= RW * WAVE * 16 * sizeof(float) &&
+                  sizeof(s_b) >= RW * WAVE * 2 * sizeof(float));
+    float* s_o = reinterpret_cast<float*>(s_k) + rw * 16 * WAVE + lane;
+    float* s_m = &s_b[0][0] + rw * 2 * WAVE + lane;
+    float mine = 1.f, other = 1.f;
+    if constexpr (KIND != SIGMOID) {
+      if (part_of == 1) { s_m[0] = m; s_m[WAVE] = l; }
+      __syncthreads();
+      if (part_of == 0) {
+        const float m1 = s_m[0], mn = fmaxf(m, m1);
+        mine = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+        other = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mn);
+        l = l * mine + s_m[WAVE] * other;
+      }
+    }
+    #pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      if (part_of == 1) {
+        #pragma unroll
+        for (int r = 0; r < 16; ++r) s_o[r * WAVE] = o_t[c][r];
+      }
+      __syncthreads();
+      if (part_of == 0) {
+        #pragma unroll
+        for (int r = 0; r < 16; ++r)
+          o_t[c][r] = o_t[c][r] * mine + s_o[r * WAVE] * other;
+      }
+      __syncthreads();
+    }
+  }
+
+  if (wave_live && qpos < total && part_of == 0) {
     const long r = en.row0 + row;
     float f = KIND == SIGMOID ? a.mult : a.mult / l;
     if (!(FLAT && a.gate_each) && a.gate != nullptr)
@@ -341,25 +398,51 @@ bool attn_ctx_prefill_supported(int dim, int vdim, int block_size) {
          block_size == PAGE;
 }
 
-void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& a, int entries,
+// Whether two waves share their rows. Tiles are half as high then, and as many again;
+// the longest one's steps, one after another, are what a launch takes when the tiles
+// are too few for the chip: with more than three quarters of the CUs at work the
+// halves are no gain. us, MI355X, heads of 128, one wave and two: 900 rows x 16 heads
+// (64 tiles) 67.0 and 49.5, portions of 900, 483 behind 1001, 741, 324 behind 1003
+// (176) 109.1 and 77.9, 2900 rows (192) 172 and 138; 8 x 300 rows (256) 32.2 and 36.7,
+// 6 x 2000 (768) 256 and 299. Heads of 64: 900 rows x 32 58.4 and 42.4, 4 x 500 behind
+// 1500 (256) 125 and 133; of 256: 8 x 300 rows x 8 (192 tiles of 128) 49.7 and 40.2.
+// Keys that are not paged are each head's own, and tiles of half the height read them
+// twice as often: there more than half of the CUs at work are enough (keys of 192,
+// six portions of up to 480 rows x 16, 192 tiles: 57.0 and 63.4).
+static bool attn_ctx_prefill_shared(int entries, long rows, int heads,
+                                    int tile, bool flat) {
+  // a portion's last tile is half full on average
+  return heads * (2 * rows / tile + entries) <= 2 * (flat ? 128 : 192);
+}
+
+void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& a, int entries, long rows,
                              int max_len, hipStream_t stream) {
-  auto go = [&](auto kk, auto dc, auto waves) {
-    constexpr int W = decltype(waves)::value;
-    const dim3 grid(entries, a.heads, (max_len + W * 32 - 1) / (W * 32));
+  auto with = [&](auto kk, auto dc, auto waves, auto sh) {
+    constexpr int W = decltype(waves)::value, SH = decltype(sh)::value;
     constexpr int K = decltype(kk)::value, D = decltype(dc)::value;
+    const dim3 grid(entries, a.heads,
+                    (max_len + W / SH * 32 - 1) / (W / SH * 32));
     const dim3 block(W * WAVE);
     if (a.ctx_start != nullptr)
-      attn_ctx_prefill_kernel<K, D, W, true, PLAIN>
+      attn_ctx_prefill_kernel<K, D, W, SH, true, PLAIN>
           <<<grid, block, 0, stream>>>(a);
     else if (a.wbias != nullptr)
-      attn_ctx_prefill_kernel<K, D, W, false, SIGMOID>
+      attn_ctx_prefill_kernel<K, D, W, SH, false, SIGMOID>
           <<<grid, block, 0, stream>>>(a);
     else if (a.cap > 0.f)
-      attn_ctx_prefill_kernel<K, D, W, false, CAP>
+      attn_ctx_prefill_kernel<K, D, W, SH, false, CAP>
           <<<grid, block, 0, stream>>>(a);
     else
-      attn_ctx_prefill_kernel<K, D, W, false, PLAIN>
+      attn_ctx_prefill_kernel<K, D, W, SH, false, PLAIN>
           <<<grid, block, 0, stream>>>(a);
+  };
+  auto go = [&](auto kk, auto dc, auto waves) {
+    if (attn_ctx_prefill_shared(entries, rows, a.heads,
+                                decltype(waves)::value * 32,
+                                a.ctx_start != nullptr))
+      with(kk, dc, waves, std::integral_constant<int, 2>{});
+    else
+      with(kk, dc, waves, std::integral_constant<int, 1>{});
   };
   using std::integral_constant;
   auto by_dc = [&](auto kk) {

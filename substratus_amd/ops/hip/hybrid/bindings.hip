@@ -255,7 +255,7 @@ void attn_ctx(Tensor out, Tensor q, OptTensor gate, Tensor kc, Tensor vc,
       }
       if (!any && seq_start && aligned && !(wbias && cap > 0) &&
           attn_ctx_prefill_supported(dim, vdim, a.block_size)) {
-        launch_attn_ctx_prefill(a, entries, max_len, stream());
+        launch_attn_ctx_prefill(a, entries, rows, max_len, stream());
         return;
       }
       if (!any && !seq_start &&
@@ -330,7 +330,7 @@ void attn_flat(Tensor out, Tensor q, OptTensor gate, Tensor kv, Tensor kr,
   a.heads = a.kv_heads = heads; a.nbias = 1; a.block_size = 16;
   a.scale = scale; a.mult = 1.f; a.window = window;
   a.out_ld = out.stride(0); a.quads = vdim % 4 == 0;
-  launch_attn_ctx_prefill(a, entries, max_len, stream());
+  launch_attn_ctx_prefill(a, entries, rows, max_len, stream());
   post("attn_flat");
 }
 

@@ -1,0 +1,129 @@
+"""Prompt portions by waves that share their rows (few tiles) and by waves of their
+own (many heads): ends of 32 rows, of tiles and of steps of keys, a wave without keys,
+every kind of weight, against the products in 64 bits."""
+
+import pytest
+import torch
+
+from substratus_amd.ops import hybrid as ops
+from test_hybrid_ops_gpu import BS, make_batch, on_gpu, rand
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+# first position and rows; single ones come first in a batch
+SPANS = [(0, 1), (0, 32), (31, 33), (40, 127), (0, 128), (63, 129), (0, 31)]
+
+
+def wide(q, k, v, first, scale, kind):
+    """One head of one portion in 64 bits."""
+    n, keys = q.shape[0], k.shape[0]
+    i = first + torch.arange(n)[:, None]
+    j = torch.arange(keys)[None]
+    s = scale * q.double() @ k.double().T
+    if kind.get("softcap"):
+        s = kind["softcap"] * torch.tanh(s / kind["softcap"])
+    bias = kind["bias"].double()
+    s = s + bias[(i - j).clamp(0, bias.shape[0] - 1)]
+    seen = j <= i
+    if kind.get("window"):
+        seen &= (i - j < kind["window"]) | (j < kind["keep"])
+    if kind.get("chunk"):
+        seen &= i // kind["chunk"] == j // kind["chunk"]
+    if kind.get("weight_bias") is not None:
+        w = torch.sigmoid(s + kind["weight_bias"].double()) * seen
+    else:
+        s = s.masked_fill(~seen, -torch.inf)
+        if kind.get("sink") is not None:
+            s = torch.cat([s, kind["sink"].double().expand(n, 1)], 1)
+        w = torch.softmax(s, 1)[:, :keys]
+    return w @ v.double()
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (96, 40),
+                                      (192, 72), (256, 256)])
+@pytest.mark.parametrize("kind", ["plain", "sink", "sigmoid", "cap", "window",
+                                  "chunk"])
+@pytest.mark.parametrize("times", [1, 32])
+def test_portions(dim, vdim, kind, times):
+    g, h = 2, 4
+    batch = make_batch(SPANS)
+    n = batch.tokens.shape[0]
+    # one sharp score per row, so that a wrong key shows
+    q = rand(n, h, dim, seed=1, dtype=BF16, scale=2.0)
+    kc = rand(64, g, BS, dim, seed=2, dtype=BF16)
+    vc = rand(64, g, BS, vdim, seed=3, dtype=BF16)
+    bias = rand(h, 77, seed=4)
+    per_head = rand(h, seed=5)
+    kinds = {"sink": dict(sink=per_head), "sigmoid": dict(weight_bias=per_head),
+             "cap": dict(softcap=3.0), "window": dict(window=37, keep=5),
+             "chunk": dict(chunk=48)}.get(kind, {})
+    scale = dim ** -0.5
+    want = torch.empty(n, h, vdim, dtype=torch.float64)
+    row = 0
+    for e, (first, m) in enumerate(SPANS):
+        pages, at = batch.block_table[e].long(), row
+        for x in range(h):
+            k = kc[pages, x // 2].reshape(-1, dim)[:first + m]
+            v = vc[pages, x // 2].reshape(-1, vdim)[:first + m]
+            one = {a: (b[x] if torch.is_tensor(b) else b)
+                   for a, b in kinds.items()}
+            want[at:at + m, x] = wide(q[at:at + m, x], k, v, first, scale,
+                                      dict(one, bias=bias[x]))
+        row += m
+
+    def more(t, at):                    # the same heads again and again
+        return t.repeat_interleave(times, at).cuda()
+    args = {a: (more(b, 0) if torch.is_tensor(b) else b)
+            for a, b in kinds.items()}
+    got = ops.attn_ctx(more(q, 1).flatten(1), None, more(kc, 1), more(vc, 1),
+                       more(bias, 0), on_gpu(batch), scale, **args)
+    got = got.view(n, h, times, vdim).cpu().double()
+    # half a step of the result: 2^-8 of the power of two below it (8 bits of
+    # significand); weights of 16 bits and 32-bit sums before
+    room = 2.0 ** -8 * want.abs() + 2.0 ** -13 * 4 * want.abs().amax()
+    assert bool(((got - want[:, :, None]).abs() <= room[:, :, None]).all())
+
+
+@pytest.mark.parametrize("dim,vdim,shared", [(64, 64, 16), (192, 128, 64),
+                                             (256, 256, 8)])
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("times", [1, 32])
+def test_unpaged(dim, vdim, shared, window, times):
+    h, spans = 4, SPANS[1:]
+    own, i32 = dim - shared, dict(dtype=torch.int32, device="cuda")
+    ends = torch.tensor([0] + [m for _, m in spans]).cumsum(0)
+    froms = [max(f - window + 1, 0) if window else 0 for f, _ in spans]
+    starts = torch.tensor([0] + [f + m - c for (f, m), c in
+                                 zip(spans, froms)]).cumsum(0)
+    n, keys = int(ends[-1]), int(starts[-1])
+    q = rand(n, h, dim, seed=1, dtype=BF16, scale=2.0)
+    k = rand(keys, h, own, seed=2, dtype=BF16)
+    v = rand(keys, h, vdim, seed=3, dtype=BF16)
+    kr = rand(keys, shared, seed=4, dtype=BF16)
+    gate = rand(n, h, seed=5, dtype=BF16)
+    want = torch.empty(n, h, vdim, dtype=torch.float64)
+    for e, (first, m) in enumerate(spans):
+        at, ks = slice(int(ends[e]), int(ends[e + 1])), \
+            slice(int(starts[e]), int(starts[e + 1]))
+        for x in range(h):
+            # keys ahead of the first that lies there are seen by no row
+            pad = (froms[e], 0)
+            kx = torch.cat([k[ks, x], kr[ks]], 1)
+            kx, vx = (torch.nn.functional.pad(t, (0, 0) + pad)
+                      for t in (kx, v[ks, x]))
+            want[at, x] = wide(q[at, x], kx, vx, first, dim ** -0.5, dict(
+                bias=torch.zeros(1), window=window, keep=0))
+    want *= torch.sigmoid(gate.double())[:, :, None]
+
+    def more(t):
+        return t.repeat_interleave(times, 1)
+    out = torch.empty(n, h * times * vdim, dtype=BF16, device="cuda")
+    kv = torch.cat([more(k).flatten(1), more(v).flatten(1)], 1).cuda()
+    pos = torch.cat([f + torch.arange(m) for f, m in spans])
+    ops._ext().attn_flat(
+        out, more(q).flatten(1).cuda(), more(gate).cuda(), kv, kr.cuda(),
+        pos.to(**i32), ends.to(**i32), starts.to(**i32), h * times, vdim,
+        dim ** -0.5, window, max(m for _, m in spans))
+    got = out.view(n, h, times, vdim).cpu().double()
+    room = 2.0 ** -8 * want.abs() + 2.0 ** -13 * 4 * want.abs().amax()
+    assert bool(((got - want[:, :, None]).abs() <= room[:, :, None]).all())
