@@ -178,10 +178,14 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
     }
     split_rows<0>(w, wh, wl);
   };
+  auto load_a2b = [&](int tile) {
+    if constexpr (CONST) return 0.f;
+    return a.a2b[h * a.dim + min(32 * tile + lo5, a.dim - 1)];
+  };
   // Summed logs (base 2) of the decays, b[r] for token crow(r); returns their end.
   // The first 16 inner columns come loaded.
   auto logs = [&](int c0, int tile, const unsigned* a1, short8 wh, short8 wl,
-                  float* b) {
+                  float zb, float* b) {
     const int d = 32 * tile + lo5;
     if constexpr (CONST) {
       const float by = d < a.dim ? ldecay : 0.f;
@@ -199,7 +203,6 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
       z = mma(pack8(more), wh, z);
       z = mma(pack8(more), wl, z);
     }
-    const float zb = a.a2b[h * a.dim + min(d, a.dim - 1)];
     const int lim = d < a.dim ? len - c0 - 4 * hi : 0;
     float gs[4], og[4];
     #pragma unroll
@@ -240,11 +243,11 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
     }
   };
   auto do_task = [&](int c0, int task, const unsigned* a1, short8 wh,
-                     short8 wl, const unsigned* rows) {
+                     short8 wl, float zb, const unsigned* rows) {
     const int tile = OUT ? task >> 1 : task, kind = OUT ? task & 1 : 1;
     const int d = 32 * tile + lo5;
     float b[16], f[16];
-    const float end = logs(c0, tile, a1, wh, wl, b);
+    const float end = logs(c0, tile, a1, wh, wl, zb, b);
     if (kind == 0) {
       const float scale = d < a.dim ? a.qscale : 0.f;
       #pragma unroll
@@ -280,14 +283,17 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
     if (OUT && end < DIRECT_BELOW) s.direct[(c0 / C) & 1] = 1;
   };
 
-  // the wave's first task comes loaded; its part of A2 stays for the segment
+  // The wave's first task comes loaded; its part of A2 and of its bias stay for the
+  // segment: a load within a chunk would be waited for behind the outputs' stores.
+  // Loads for the next chunk are behind no branch, so that their number is known
+  // where one ahead of them is waited for; there may be none of that chunk's rows.
+  const int first = min(wave, TASKS - 1);
   const int vcol = h * a.vdim + min(col, a.vdim - 1);
   unsigned task_rows[16], vraw[16], a1[8] = {};
   short8 wh0 = {}, wl0 = {};
-  if (wave < TASKS) {
-    load_task(0, wave, task_rows);
-    load_a2(OUT ? wave >> 1 : wave, 0, &wh0, &wl0);
-  }
+  load_task(0, first, task_rows);
+  load_a2(OUT ? first >> 1 : first, 0, &wh0, &wl0);
+  const float zb0 = load_a2b(OUT ? first >> 1 : first);
   load_a1(0, 0, a1);
   load16(0, a.v_off + vcol, vraw);
 
@@ -296,11 +302,13 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
     #pragma unroll 1
     for (int task = wave; task < TASKS; task += nw) {
       short8 wh = wh0, wl = wl0;
+      float zb = zb0;
       if (task != wave) {
         load_task(c0, task, task_rows);
         load_a2(OUT ? task >> 1 : task, 0, &wh, &wl);
+        zb = load_a2b(OUT ? task >> 1 : task);
       }
-      do_task(c0, task, a1, wh, wl, task_rows);
+      do_task(c0, task, a1, wh, wl, zb, task_rows);
     }
     // V as the second operand of both products: token order as in the
     // accumulators
@@ -321,7 +329,7 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
         float b[16];
         short8 wh, wl;
         load_a2(tile, 0, &wh, &wl);
-        logs(c0, tile, a1, wh, wl, b);
+        logs(c0, tile, a1, wh, wl, load_a2b(tile), b);
         #pragma unroll
         for (int r = 0; r < 16; ++r) sb[crow(r)][32 * tile + lo5] = b[r];
       }
@@ -343,11 +351,9 @@ void gla_chunk_kernel(Gla<bf16_t> a, int nseg, int seg_len,
 
     unsigned graw[16];
     if (OUT && !CONST) load16(c0, a.g_off + vcol, graw);
-    if (c0 + C < len) {
-      if (wave < TASKS) load_task(c0 + C, wave, task_rows);
-      load_a1(c0 + C, 0, a1);
-      load16(c0 + C, a.v_off + vcol, vraw);
-    }
+    load_task(c0 + C, first, task_rows);
+    load_a1(c0 + C, 0, a1);
+    load16(c0 + C, a.v_off + vcol, vraw);
 
     float16v o = {};
     if (OUT) {
