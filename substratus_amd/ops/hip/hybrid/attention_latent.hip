@@ -18,6 +18,8 @@
 // Long contexts are split over workgroups and merged by attn_ctx_merge.
 #include "attention_ctx.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) short short8;
@@ -299,15 +301,20 @@ bool attn_latent_supported(int dim, int vdim, int block_size) {
          vdim <= 512 && block_size == PAGE;
 }
 
-// Workgroups that share one context: enough for every CU, but at least two
-// steps for each. `span`: most keys a row can see.
+// Workgroups that share one context, of at least two steps each: as many as there
+// are CUs for all contexts, where one has a CU to itself (147 KB of LDS), and its chain
+// of steps is what a launch takes. A power of two, the first that gives every CU one,
+// was up to 1.4 times slower, as some CUs have two then and others none: us, MI355X,
+// keys of 576, 16 heads, contexts of a quarter of the most to the most, with their
+// merge: 1 of 900 20.0 -> 18.7, 20 of 2000 32.3 -> 26.7, 40 of 2000 45.4 -> 38.1, 48 of
+// 900 27.1 -> 25.6; 32 heads, 40 of 900 36.8 -> 27.4, 100 of 300 30.7 -> 21.9; of 72
+// numbers of contexts none more than 2 % slower. 384 or 512 workgroups in all: 0.70 to
+// 1.12 times as fast as the powers.
 int attn_latent_splits(int entries, int max_len, int heads, int span) {
   const int qt = query_tile(entries, max_len, heads, span);
   const long groups = (long)entries * (((long)max_len * heads + qt - 1) / qt);
-  const int steps = (span + CH - 1) / CH;
-  int s = 1;
-  while (s < 32 && groups * s < 256 && steps >= s * 4) s *= 2;
-  return s;
+  const long steps = (span + CH - 1) / CH;
+  return (int)std::max(1L, std::min({256 / groups, steps / 2, 32L}));
 }
 
 void launch_attn_latent(const AttnCtx<bf16_t>& a, int entries, int max_len,

@@ -127,3 +127,25 @@ def test_unpaged(dim, vdim, shared, window, times):
     got = out.view(n, h, times, vdim).cpu().double()
     room = 2.0 ** -8 * want.abs() + 2.0 ** -13 * 4 * want.abs().amax()
     assert bool(((got - want[:, :, None]).abs() <= room[:, :, None]).all())
+
+
+# Contexts in shares whose number is no power of two, some without a step: 256 CUs over
+# the contexts, with two steps of 64 keys each
+@pytest.mark.parametrize("n,most", [(1, 450), (19, 900), (37, 700), (85, 450),
+                                    (129, 300)])
+def test_latent_shares(n, most):
+    h, dim, vdim = 16, 192, 128
+    spans = [(most - 1 - i * (most - 3) // n, 1) for i in range(n)]
+    blocks = sum(f // BS + 1 for f, _ in spans)
+    batch = make_batch(spans, blocks)
+    q = rand(n, h * dim, seed=1, dtype=BF16, scale=2.0)
+    cache = rand(blocks, 1, BS, dim, seed=2, dtype=BF16)
+    on = cache.cuda()
+    got = ops.attn_ctx(q.cuda(), None, on, on[..., :vdim], None,
+                       on_gpu(batch), dim ** -0.5).view(n, h, vdim)
+    for e, (first, _) in enumerate(spans):
+        k = cache[batch.block_table[e].long(), 0].reshape(-1, dim)[:first + 1]
+        s = q[e].view(h, dim).double() @ k.double().T * dim ** -0.5
+        want = torch.softmax(s, 1) @ k[:, :vdim].double()
+        room = 2.0 ** -8 * want.abs() + 2.0 ** -13 * 4 * want.abs().amax()
+        assert bool(((got[e].cpu().double() - want).abs() <= room).all())
