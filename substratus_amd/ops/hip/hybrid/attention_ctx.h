@@ -101,8 +101,12 @@ void launch_attn_ctx_decode(const AttnCtx<bf16_t>&, int entries, int splits,
                             float* part_o, float* part_ml, hipStream_t);
 
 bool attn_ctx_prefill_supported(int dim, int vdim, int block_size);
+int attn_ctx_prefill_splits(int entries, long rows, int heads, int vdim,
+                            int span);
+// splits > 1: of paged keys; shares of sums are left, and attn_ctx_merge follows
 void launch_attn_ctx_prefill(const AttnCtx<bf16_t>&, int entries, long rows,
-                             int max_len, hipStream_t);
+                             int max_len, int splits, float* part_o,
+                             float* part_ml, hipStream_t);
 
 // One head of shared keys whose first columns are the values.
 bool attn_latent_supported(int dim, int vdim, int block_size);

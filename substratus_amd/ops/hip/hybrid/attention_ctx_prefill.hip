@@ -20,10 +20,14 @@
 //     the cache holds (FLAT), with a key part that all heads share;
 //   * where tiles of the most rows are too few for the chip, two waves share 32 rows
 //     and take every other 32 keys; their sums meet in LDS at the end;
+//   * where those are too few, too, workgroups share a tile's keys, merged by
+//     attn_ctx_merge;
 //   * V is staged with keys 4..7 and 8..11 of every 16 exchanged, which is
 //     the order in which the score accumulators hold them: weights need no
 //     lane exchange before the second product.
 #include "attention_ctx.h"
+
+#include <algorithm>
 
 typedef __attribute__((ext_vector_type(8))) short short8;
 typedef __attribute__((ext_vector_type(4))) short short4v;
@@ -49,7 +53,9 @@ enum Kind {
 // SH: waves that share their 32 query rows, each a part of a step's keys
 template <int KK, int DC, int WAVES, int SH, bool FLAT, Kind KIND>
 __global__ __launch_bounds__(WAVES * WAVE)
-void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
+void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a, int splits,
+                             float* __restrict__ part_o,
+                             float* __restrict__ part_ml) {
   constexpr int THREADS = WAVES * WAVE;
   constexpr int RW = WAVES / SH;            // waves of unlike rows
   constexpr int QT = RW * 32;               // query rows per workgroup
@@ -65,7 +71,9 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
   __shared__ float s_b[2][THREADS];
 
   const int e = blockIdx.x, head = blockIdx.y;
-  const int tile = gridDim.z - 1 - blockIdx.z;   // longest rows first
+  // longest rows first
+  const int tile = (gridDim.z - 1 - blockIdx.z) / splits;
+  const int split = blockIdx.z % splits;
   const Entry en = entry_of(a.seq_start, e);
   const int q0_tile = tile * QT;
   if (q0_tile >= en.n) return;
@@ -105,7 +113,7 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
     }
   }
   float m = -INFINITY, l = 0.f;
-  if (a.sink != nullptr && part_of == 0) { m = a.sink[head] * LOG2E; l = 1.f; }
+  if (a.sink != nullptr && part_of == 0 && splits == 1) { m = a.sink[head] * LOG2E; l = 1.f; }
   float16v o_t[DC];
   #pragma unroll
   for (int c = 0; c < DC; ++c) o_t[c] = (float16v){};
@@ -205,15 +213,16 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
     s_b[buf][tid] = b;
   };
 
-  pages(0);
-  stage_load(0);
-  pages(1);
-  stage_write(0, 0);
+  const int it0 = part.n * split / splits, it1 = part.n * (split + 1) / splits;
+  pages(it0);
+  stage_load(it0);
+  pages(it0 + 1);
+  stage_write(it0, 0);
   __syncthreads();
 
-  for (int it = 0; it < part.n; ++it) {
-    const int cur = it & 1;
-    if (it + 1 < part.n) {
+  for (int it = it0; it < it1; ++it) {
+    const int cur = (it - it0) & 1;
+    if (it + 1 < it1) {
       stage_load(it + 1);
       pages(it + 2);
     }
@@ -321,7 +330,7 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
       }
       if constexpr (KIND != SIGMOID) l += across<32>(sum, Plus{});
     }
-    if (it + 1 < part.n) stage_write(it + 1, cur ^ 1);
+    if (it + 1 < it1) stage_write(it + 1, cur ^ 1);
     __syncthreads();
   }
 
@@ -340,6 +349,7 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
         mine = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
         other = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mn);
         l = l * mine + s_m[WAVE] * other;
+        m = mn;
       }
     }
     #pragma unroll
@@ -360,6 +370,25 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a) {
 
   if (wave_live && qpos < total && part_of == 0) {
     const long r = en.row0 + row;
+    if (!FLAT && splits > 1) {
+      const long at = (r * a.heads + head) * splits + split;
+      #pragma unroll
+      for (int c = 0; c < DC; ++c)
+        #pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+          const int d0 = c * 32 + 8 * rr + 4 * hi;
+          if (d0 >= a.vdim) continue;
+          float o[4];
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) o[j] = o_t[c][rr * 4 + j];
+          stv<4>(part_o + at * a.vdim + d0, o);
+        }
+      if (hi == 0 && KIND != SIGMOID) {
+        part_ml[at * 2] = m;
+        part_ml[at * 2 + 1] = l;
+      }
+      return;
+    }
     float f = KIND == SIGMOID ? a.mult : a.mult / l;
     if (!(FLAT && a.gate_each) && a.gate != nullptr)
       f *= sigmoid_f(bf2f(a.gate[r * a.g_ld + head]));
@@ -415,26 +444,50 @@ static bool attn_ctx_prefill_shared(int entries, long rows, int heads,
   return heads * (2 * rows / tile + entries) <= 2 * (flat ? 128 : 192);
 }
 
+// Workgroups that share a tile's keys: those of few tiles, where a step of 64 keys takes
+// 3 us and what follows (a launch, for the host, too; the shares' sums written and read)
+// less than the steps saved; no more workgroups than CUs. us, MI355X, one and by shares, heads of 128,
+// 16 of them: 100 rows behind 2000 96.1 and 29.5, 30 behind 3000 132 and 28.9, 500
+// behind 3500 170 and 65.7, 3 x 100 behind 600 41.3 and 28.0 (900 rows, 49.8 and 41.3,
+// stay whole);
+// heads of 64, 32 of 8: 33.3 and 29.6 of 3 x 100; of 256, 8 of 1: 63.0 and 32.8.
+int attn_ctx_prefill_splits(int entries, long rows, int heads, int vdim,
+                            int span) {
+  const int tile = vdim <= 128 ? 256 : 128;
+  if (!attn_ctx_prefill_shared(entries, rows, heads, tile, false)) return 1;
+  const long blocks = std::max(1L, heads * (4 * rows / tile + entries) / 2);
+  const int steps = (span + CH - 1) / CH;
+  auto cost = [&](long s) {
+    return (steps + s - 1) / s * 3. +
+           (s > 1 ? 14. + (double)rows * heads * s * vdim * (8 / 4e6) : 0.);
+  };
+  int best = 1;
+  for (int s = 2; s <= 16 && blocks * s <= 256; ++s)
+    if (cost(s) < cost(best)) best = s;
+  return best;
+}
+
 void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& a, int entries, long rows,
-                             int max_len, hipStream_t stream) {
+                             int max_len, int splits, float* part_o,
+                             float* part_ml, hipStream_t stream) {
   auto with = [&](auto kk, auto dc, auto waves, auto sh) {
     constexpr int W = decltype(waves)::value, SH = decltype(sh)::value;
     constexpr int K = decltype(kk)::value, D = decltype(dc)::value;
     const dim3 grid(entries, a.heads,
-                    (max_len + W / SH * 32 - 1) / (W / SH * 32));
+                    (max_len + W / SH * 32 - 1) / (W / SH * 32) * splits);
     const dim3 block(W * WAVE);
     if (a.ctx_start != nullptr)
       attn_ctx_prefill_kernel<K, D, W, SH, true, PLAIN>
-          <<<grid, block, 0, stream>>>(a);
+          <<<grid, block, 0, stream>>>(a, splits, part_o, part_ml);
     else if (a.wbias != nullptr)
       attn_ctx_prefill_kernel<K, D, W, SH, false, SIGMOID>
-          <<<grid, block, 0, stream>>>(a);
+          <<<grid, block, 0, stream>>>(a, splits, part_o, part_ml);
     else if (a.cap > 0.f)
       attn_ctx_prefill_kernel<K, D, W, SH, false, CAP>
-          <<<grid, block, 0, stream>>>(a);
+          <<<grid, block, 0, stream>>>(a, splits, part_o, part_ml);
     else
       attn_ctx_prefill_kernel<K, D, W, SH, false, PLAIN>
-          <<<grid, block, 0, stream>>>(a);
+          <<<grid, block, 0, stream>>>(a, splits, part_o, part_ml);
   };
   auto go = [&](auto kk, auto dc, auto waves) {
     if (attn_ctx_prefill_shared(entries, rows, a.heads,

@@ -255,7 +255,21 @@ void attn_ctx(Tensor out, Tensor q, OptTensor gate, Tensor kc, Tensor vc,
       }
       if (!any && seq_start && aligned && !(wbias && cap > 0) &&
           attn_ctx_prefill_supported(dim, vdim, a.block_size)) {
-        launch_attn_ctx_prefill(a, entries, rows, max_len, stream());
+        const int splits =
+            attn_ctx_prefill_splits(entries, rows, heads, vdim, span);
+        Tensor shares;                  // sums, then maxima and weights' sums
+        float *po = nullptr, *pml = nullptr;
+        if (splits > 1) {
+          const long n = rows * heads * splits;
+          shares = torch::empty({n * (vdim + 2)},
+                                out.options().dtype(torch::kFloat32));
+          po = ptr<float>(shares);
+          pml = po + n * vdim;
+        }
+        launch_attn_ctx_prefill(a, entries, rows, max_len, splits, po, pml,
+                                stream());
+        if (splits > 1)
+          launch_attn_ctx_merge(a, rows, splits, po, pml, stream());
         return;
       }
       if (!any && !seq_start &&
@@ -330,7 +344,8 @@ void attn_flat(Tensor out, Tensor q, OptTensor gate, Tensor kv, Tensor kr,
   a.heads = a.kv_heads = heads; a.nbias = 1; a.block_size = 16;
   a.scale = scale; a.mult = 1.f; a.window = window;
   a.out_ld = out.stride(0); a.quads = vdim % 4 == 0;
-  launch_attn_ctx_prefill(a, entries, rows, max_len, stream());
+  launch_attn_ctx_prefill(a, entries, rows, max_len, 1, nullptr, nullptr,
+                          stream());
   post("attn_flat");
 }
 

@@ -12,6 +12,9 @@ pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
 # first position and rows; single ones come first in a batch
 SPANS = [(0, 1), (0, 32), (31, 33), (40, 127), (0, 128), (63, 129), (0, 31)]
+# contexts long enough to be shared, one whose shares have no step each, one behind
+# which a window or a chunk leaves few
+LONG = [(900, 33), (0, 2), (511, 65), (100, 3)]
 
 
 def wide(q, k, v, first, scale, kind):
@@ -43,15 +46,15 @@ def wide(q, k, v, first, scale, kind):
                                       (192, 72), (256, 256)])
 @pytest.mark.parametrize("kind", ["plain", "sink", "sigmoid", "cap", "window",
                                   "chunk"])
-@pytest.mark.parametrize("times", [1, 32])
-def test_portions(dim, vdim, kind, times):
+@pytest.mark.parametrize("times,spans", [(1, SPANS), (32, SPANS), (1, LONG)])
+def test_portions(dim, vdim, kind, times, spans):
     g, h = 2, 4
-    batch = make_batch(SPANS)
+    batch = make_batch(spans, 128)
     n = batch.tokens.shape[0]
     # one sharp score per row, so that a wrong key shows
     q = rand(n, h, dim, seed=1, dtype=BF16, scale=2.0)
-    kc = rand(64, g, BS, dim, seed=2, dtype=BF16)
-    vc = rand(64, g, BS, vdim, seed=3, dtype=BF16)
+    kc = rand(128, g, BS, dim, seed=2, dtype=BF16)
+    vc = rand(128, g, BS, vdim, seed=3, dtype=BF16)
     bias = rand(h, 77, seed=4)
     per_head = rand(h, seed=5)
     kinds = {"sink": dict(sink=per_head), "sigmoid": dict(weight_bias=per_head),
@@ -60,7 +63,7 @@ def test_portions(dim, vdim, kind, times):
     scale = dim ** -0.5
     want = torch.empty(n, h, vdim, dtype=torch.float64)
     row = 0
-    for e, (first, m) in enumerate(SPANS):
+    for e, (first, m) in enumerate(spans):
         pages, at = batch.block_table[e].long(), row
         for x in range(h):
             k = kc[pages, x // 2].reshape(-1, dim)[:first + m]
