@@ -29,8 +29,8 @@
 // the CUs along the inner dimension and leave 32-bit sums to a second kernel. Or
 // tiles have fewer rows, 128 to 224, where those of 256 would leave CUs idle or be
 // partly empty (plan_of): regions of a's halves are not full then, nothing else
-// changes. us, MI355X, from 256 rows: 2331 x 2048 x 2048 35.6 -> 25.8 (128), 11264 x
-// 2048 x 2331, both flipped, 110 -> 104 (192), 2331 x 11264 x 2048 94 -> 88 (224), 908
+// changes. us, MI355X, from 256 rows: 2331 x 2048 x 2048 35.6 -> 25.8 (128), 6144 x
+// 2048 x 2331, both flipped, 60.7 -> 57.4 (192), 2331 x 11264 x 2048 94 -> 88 (224), 908
 // x 11264 x 2048, gated, 45 -> 39 (192), 557 x 18176 x 4544, b flipped, 114 -> 93 (192).
 // Large ones are bound by power: with random numbers the chip holds 1.5 to 1.7 GHz, at
 // 2140 clocks a step of which matrix instructions take 2048 (zeros: 2.4 GHz, 2.1
@@ -651,11 +651,27 @@ static TilePlan plan_of(long m, long n, long k, int rows, bool a_flipped,
   return p;
 }
 
+// Fewer rows turn a flipped operand once more for the same result, and such tiles take
+// longer than planned where no CU was idle before, or where shares keep all busy. By
+// what 256 rows take over what fewer do, MI355X, 2647 products of 256 to 8192 rows:
+//   both flipped   128 rows instead of shares of 256  12 of 0.84 to 1.03 (2048 x 4096 x
+//                  5000 84.6 and 100.6 us), of more shares 0.89 to 1.05; several rounds
+//                  0.93 to 1.12 (5120 x 5120 x 6000 264 and 284); a single round
+//                  instead of one with fewer tiles 1.22 (128), 1.05 (192): only that
+//   b flipped      128 rows instead of shares 0.92, 0.96, 1.09; two shares of 160 rows
+//                  9 of 0.88 to 0.95, of 192 28 of 0.85 to 1.06: neither; three and
+//                  more 1.15 and 1.11, of 224 rows 1.04
+//   neither        1.03 to 1.2 in every group
 TilePlan tile_gemm_plan(long m, long n, long k, bool a_flipped,
                         bool b_flipped) {
-  TilePlan best = plan_of(m, n, k, TILE, a_flipped, b_flipped);
+  const TilePlan high = plan_of(m, n, k, TILE, a_flipped, b_flipped);
+  TilePlan best = high;
   for (int rows = 128; rows < TILE; rows += 32) {
     const TilePlan p = plan_of(m, n, k, rows, a_flipped, b_flipped);
+    if (a_flipped ? high.split > 1 || p.tiles_m * (long)p.tiles_n > 256
+                  : b_flipped && ((rows == 128 && high.split > 1) ||
+                                  (rows < 224 && p.split == 2)))
+      continue;
     if (p.us < (best.rows == TILE ? 0.97 : 1.) * best.us) best = p;
   }
   return best;

@@ -111,6 +111,16 @@ def test_heights(height, over, k, kind):
         close(got, a.T if fa else a, b.T if fb else b, bias)
 
 
+# Tiles of 224 rows of a flipped b whose last one begins early: sizes that are none of
+# test_heights'
+@pytest.mark.parametrize("m,n,k", [(264, 5544, 1096), (264, 9504, 2120)])
+def test_last_tile_of_a_flipped_b(m, n, k):
+    torch.manual_seed(n)
+    assert _C.tile_gemm_rows(m, n, k, False, True) == 224
+    a, b = operand(m, k, False, 8), operand(n, k, True, 8)
+    close(_C.tile_gemm(a, b, None, False, True), a, b.T)
+
+
 def test_rows_of_any_number():
     """Rows that are not flipped need not come in eights."""
     a, b = operand(321, 192, False, 0), operand(264, 192, False, 0)

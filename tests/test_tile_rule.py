@@ -87,3 +87,16 @@ def test_rows_that_meet_in_memory(m, n, k, paired, pays):
     """Rows of a multiple of 4 KB leave the library where that was measured to
     be the faster way, and not at its edges."""
     assert _C.mid_gemm_good(m, n, k, paired) == pays
+
+
+@pytest.mark.parametrize("m,n,k,a,b,rows", [
+    (2048, 4096, 5000, True, True, 256), (4096, 2048, 4096, True, True, 256),
+    (5120, 5120, 6000, True, True, 256), (6144, 4096, 2488, True, True, 256),
+    (2048, 2048, 4165, True, True, 256), (768, 8192, 32768, False, True, 256),
+    (577, 8192, 32768, False, True, 224), (4096, 2048, 4096, False, True, 256),
+    (6144, 2048, 2488, True, True, 192), (320, 4544, 65024, False, True, 160),
+    (384, 57344, 8192, False, False, 192)])
+def test_heights(m, n, k, a, b, rows):
+    """Flipped operands are turned more often by tiles of fewer rows: those that
+    were slower by it have 256, or the most of the others."""
+    assert _C.tile_gemm_rows(m, n, k, a, b) == rows
