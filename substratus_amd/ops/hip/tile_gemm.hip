@@ -678,45 +678,55 @@ TilePlan tile_gemm_plan(long m, long n, long k, bool a_flipped,
 }
 
 // Whether the library's product would take longer. What that takes is no smooth
-// function of sizes, so this goes by planned PFLOP/s, and where the lines lie by what
-// all products beyond them gain together. The library's time over this one's, MI355X,
-// 260 to 6000 rows, matrices of 2048 to 28672 rows and columns, a pass over memory
-// before each product as in a model's step:
-//   neither flipped   of 101, all 1.06 (the worst 0.80); from 1.0 on 42 that go, of
-//                     0.96 to 1.9, 1.14 together. From 0.9 on three more, and 3330 x
-//                     2048 x 5632, which lost in a model (0.91). Shares of a single
-//                     round with rows of a multiple of 8 KB, which meet at few of the
-//                     memory's channels, stay (577 x 8192 x 8192 0.77), whole tiles of
-//                     whole rounds stay (by themselves 0.94 to 1.09; the library
-//                     writes past the caches, though, and the pass that reads the
-//                     results pays for that: 2331 x 32000 x 2048 0.97, a step's loss
-//                     after it 90 us instead of 73)
-//   b flipped         of 199, all 1.11; 89 that go, of 0.90 to 2.57, 1.22 together. In
-//                     three and more shares from 0.7 on (36 of 1.03 and more), others
-//                     from 0.85 on (two shares below that 0.82 to 1.01); few rows with
-//                     lines of a multiple of 16 KB stay (483 x 8192 x 3072 0.65)
-//   both flipped      of 111, all 1.22, one slower (0.95); of rows this short that it
-//                     plans less than 0.5 none was slower either, nor much faster
-//   gated             from 0.5 on 22 of 1.08 to 1.70 over the product and the pass
-//                     that gates it; below four of 0.95 to 1.19
-// Of tiles of 256 rows that would take half to three quarters of their rounds' CUs the
-// first two stay with the library, though by tiles of fewer rows they no longer lose:
-// no more than these 5 % of all products.
+// function of sizes: it has products that it is tuned for, whose neighbours take up to
+// twice as long. So this goes by planned PFLOP/s, and where the lines lie by what all
+// products beyond them gain together. The library's time over this one's, MI355X, 4060
+// products of models of 768 to 8192 columns by 256 to 8192 rows, operands from memory:
+//   neither flipped   in three and more shares from 0.95 on 138 of 0.95 to 2.24, 1.22
+//                     on average; others from 1.0 on 556 of 0.89 to 2.17, 1.07 (from
+//                     0.9 on 43 more, 1.02; 3330 x 2048 x 5632, of those, lost in a
+//                     model, 0.91). Tiles of 256 rows in whole rounds stay, 51 of 0.93
+//                     to 1.05; two shares of 8192 columns whose inner size it is tuned
+//                     for, 15 of 0.81 to 1.06 (10 of other widths and such inner sizes
+//                     1.13); and tiles of fewer rows where 256 would leave a quarter
+//                     of the CUs idle and plan less than 1.0, 52 of 0.92 to 1.23, 1.03
+//                     together (2048 x 4096 x 4096 1.05; 60 that plan more go, 1.04)
+//   b flipped         in three and more shares from 0.7 on 350 of 0.93 to 3.15, 1.50;
+//                     others from 0.85 on 359 of 0.87 to 1.86, 1.14. Two shares of 8192
+//                     columns and up to 1023 rows stay, 24 of 0.78 to 1.05, others of
+//                     a multiple of that below 1.15, 7 of 0.87 to 1.02, and where
+//                     tiles of 256 rows would take up to three quarters of their
+//                     rounds' CUs, 132 of 0.81 to 1.53, 0.98 on average
+//   both flipped      from 0.5 on 502 of 0.84 to 1.57, 1.18; of rows by 32 from 0.55
+//                     on 572 of 0.75 to 1.65, 1.10 (below that 2048 x 2048 x 3072
+//                     0.86); not where a quarter and more of the steps' places is
+//                     empty and the library has no such places (288 tokens: 29 of 0.71
+//                     to 1.30, 0.94)
+//   gated             from 0.5 on 140 of 1.00 to 1.63 over the product and the pass
+//                     that gates it, 1.16
+// Lines 128 bytes longer change the two shares of 8192 columns by up to 5 %, the
+// library's as well: not where the operands lie is what keeps them there.
 bool tile_gemm_pays(long m, long n, long k, bool a_flipped, bool b_flipped,
                     bool gated) {
   const TilePlan p = tile_gemm_plan(m, n, k, a_flipped, b_flipped);
   const double rate = 2e-9 * m * n * k / p.us;        // PFLOP/s
-  if (a_flipped || gated) return rate >= 0.5;
+  if (gated) return rate >= 0.5;
+  if (a_flipped) {
+    const long empty = 2 * pairs_of(k) * STEP - k;
+    return k % 32 == 0 ? rate >= 0.55 && 4 * empty < k : rate >= 0.5;
+  }
   const TilePlan whole = plan_of(m, n, k, TILE, false, b_flipped);
   const long high = whole.tiles_m * (long)whole.tiles_n;
-  if (whole.split == 1 && 4 * high <= 3 * ((high + 255) / 256 * 256))
-    return false;
+  const bool idle = 4 * high <= 3 * ((high + 255) / 256 * 256);
+  const bool halves = p.whole == 0 && p.split == 2 && n % 8192 == 0;
   if (b_flipped)
-    return rate >= (p.split > 2 ? 0.7 : 0.85) && (m >= 1024 || n % 8192 != 0);
-  const long tiles = p.tiles_m * (long)p.tiles_n;
-  const bool even = m % p.rows == 0 && n % TILE == 0 && tiles % 256 == 0;
-  const bool meet = p.whole == 0 && k % 4096 == 0;
-  return rate >= 1. && !even && !meet;
+    return rate >= (p.split > 2 ? 0.7 : n % 8192 == 0 && m < 1024 ? 1.15 : 0.85) &&
+           !(whole.split == 1 && idle) && !(halves && m < 1024);
+  if (p.split > 2) return rate >= 0.95;
+  const bool even = m % TILE == 0 && n % TILE == 0 && high % 256 == 0;
+  const bool fewer = p.split == 1 && (whole.split == 1 || whole.whole == 0);
+  return rate >= 1. && !even && !(halves && k % 4096 == 0) &&
+         !(fewer && idle && 2e-9 * m * n * k / whole.us < 1.);
 }
 
 void launch_tile_gemm(const TileGemm& g, const TilePlan& plan, float* shares,

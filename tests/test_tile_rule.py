@@ -100,3 +100,26 @@ def test_heights(m, n, k, a, b, rows):
     """Flipped operands are turned more often by tiles of fewer rows: those that
     were slower by it have 256, or the most of the others."""
     assert _C.tile_gemm_rows(m, n, k, a, b) == rows
+
+
+@pytest.mark.parametrize("kind,m,n,k,pays", [
+    ("plain", 256, 8192, 28672, True), ("plain", 512, 8192, 28672, True),
+    ("plain", 1333, 8192, 28672, True), ("plain", 1777, 4096, 16384, True),
+    ("plain", 1024, 4096, 16384, True), ("plain", 768, 10240, 8192, True),
+    ("plain", 900, 8192, 8192, False), ("plain", 768, 8192, 32768, False),
+    ("plain", 768, 8192, 27648, True), ("plain", 3000, 4096, 14336, True),
+    ("plain", 1536, 16384, 4096, True), ("plain", 1024, 16384, 4096, False),
+    ("inputs", 256, 8192, 32000, True), ("inputs", 512, 8192, 10240, True),
+    ("inputs", 900, 32768, 8192, True), ("inputs", 640, 8192, 32000, False),
+    ("inputs", 768, 8192, 8192, False),
+    ("weights", 8192, 32768, 288, False), ("weights", 4096, 16384, 288, False),
+    ("weights", 18176, 4544, 256, True), ("weights", 4096, 4096, 257, True),
+    ("inputs", 320, 32768, 8192, False), ("weights", 2048, 2048, 3072, False),
+    ("weights", 27648, 5120, 320, True), ("weights", 5120, 5120, 416, True)])
+def test_products_the_library_is_tuned_for(kind, m, n, k, pays):
+    """They stay with it, and their neighbours, which take twice as long there, do
+    not; wherever the operands' lines lie."""
+    a, b = kind == "weights", kind in ("inputs", "weights")
+    for pad in (0, 64):
+        assert _C.tile_gemm_good(m, n, k, (m if a else k) + pad,
+                                 (n if b else k) + pad, a, b, False) == pays
