@@ -312,7 +312,9 @@ bool attn_latent_supported(int dim, int vdim, int block_size) {
 // 1.12 times as fast as the powers.
 int attn_latent_splits(int entries, int max_len, int heads, int span) {
   const int qt = query_tile(entries, max_len, heads, span);
-  const long groups = (long)entries * (((long)max_len * heads + qt - 1) / qt);
+  // at least one: a call without rows is the launch's to refuse
+  const long groups = std::max(
+      1L, (long)entries * (((long)max_len * heads + qt - 1) / qt));
   const long steps = (span + CH - 1) / CH;
   return (int)std::max(1L, std::min({256 / groups, steps / 2, 32L}));
 }
