@@ -110,7 +110,8 @@ void launch_attn_ctx_prefill(const AttnCtx<bf16_t>&, int entries, long rows,
 
 // One head of shared keys whose first columns are the values.
 bool attn_latent_supported(int dim, int vdim, int block_size);
-int attn_latent_splits(int entries, int max_len, int heads, int span);
+int attn_latent_splits(int entries, int max_len, int heads, int span, int dim,
+                       int vdim);
 void launch_attn_latent(const AttnCtx<bf16_t>&, int entries, int max_len,
                         int span, int splits, float* part_o, float* part_ml,
                         hipStream_t);

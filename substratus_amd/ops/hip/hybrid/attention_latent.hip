@@ -301,22 +301,34 @@ bool attn_latent_supported(int dim, int vdim, int block_size) {
          vdim <= 512 && block_size == PAGE;
 }
 
-// Workgroups that share one context, of at least two steps each: as many as there
-// are CUs for all contexts, where one has a CU to itself (147 KB of LDS), and its chain
-// of steps is what a launch takes. A power of two, the first that gives every CU one,
-// was up to 1.4 times slower, as some CUs have two then and others none: us, MI355X,
-// keys of 576, 16 heads, contexts of a quarter of the most to the most, with their
-// merge: 1 of 900 20.0 -> 18.7, 20 of 2000 32.3 -> 26.7, 40 of 2000 45.4 -> 38.1, 48 of
-// 900 27.1 -> 25.6; 32 heads, 40 of 900 36.8 -> 27.4, 100 of 300 30.7 -> 21.9; of 72
-// numbers of contexts none more than 2 % slower. 384 or 512 workgroups in all: 0.70 to
-// 1.12 times as fast as the powers.
-int attn_latent_splits(int entries, int max_len, int heads, int span) {
+// Workgroups that share one context: as many as there are CUs for all contexts, where
+// one has a CU to itself (87 KB of LDS and more), and its chain of steps, two at least,
+// is what a launch takes. Where that gives contexts one each and the others none, three
+// shares of five steps or more, but no two, whose second round is as long as the first.
+// Keys of up to 192 leave room for two workgroups on a CU, which pays where one would
+// have a long chain (three shares or more are short enough). us, MI355X, with the merge,
+// contexts of a quarter of the most to the most, by a power of two, the first that gives
+// every CU one -> by this:
+//   keys of 576, 16 heads  1 of 900 15.6 -> 14.4, 20 of 2000 27.2 -> 21.5, 40 of 2000
+//                          32.0 -> 27.5, 48 of 900 20.7 -> 19.8, 200 of 900 43.9 ->
+//                          44.4; 130 of 900 33.3 -> 35.8 (one share 39.3; all as long
+//                          as the most 56.7 -> 47.1); 32 heads, 100 of 300 25.8 -> 18.3
+//   of 192, 16 heads       20 of 2000 15.5 -> 13.9, 100 of 900 15.4 -> 14.5, 120 of 1500
+//                          19.4, 130 of 900 16.9; 32 heads, 100 of 300 13.0 -> 9.4
+// More than 16 or 20 shares cost the merge more than the chain gains (one context of
+// 4000: 21.0 by 31).
+int attn_latent_splits(int entries, int max_len, int heads, int span, int dim,
+                       int vdim) {
   const int qt = query_tile(entries, max_len, heads, span);
   // at least one: a call without rows is the launch's to refuse
   const long groups = std::max(
       1L, (long)entries * (((long)max_len * heads + qt - 1) / qt));
   const long steps = (span + CH - 1) / CH;
-  return (int)std::max(1L, std::min({256 / groups, steps / 2, 32L}));
+  const bool two = dim <= 192 && vdim <= 128;
+  long s = std::min({256 / groups, steps / (two ? 3 : 2), two ? 16L : 20L});
+  if (two && groups > 85) s = std::max(s, std::min(512 / groups, steps / 5));
+  if (!two && groups > 128 && groups <= 170 && steps >= 15) s = 3;
+  return (int)std::max(1L, s);
 }
 
 void launch_attn_latent(const AttnCtx<bf16_t>& a, int entries, int max_len,

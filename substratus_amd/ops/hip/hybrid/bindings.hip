@@ -238,7 +238,8 @@ void attn_ctx(Tensor out, Tensor q, OptTensor gate, Tensor kc, Tensor vc,
           cap == 0 && mult == 1 && out.is_contiguous() &&
           attn_latent_supported(dim, vdim, a.block_size)) {
         const int longest = seq_start ? max_len : 1;
-        const int splits = attn_latent_splits(entries, longest, heads, span);
+        const int splits =
+            attn_latent_splits(entries, longest, heads, span, dim, vdim);
         Tensor po, pml;
         if (splits > 1) {
           const auto opt = out.options().dtype(torch::kFloat32);

@@ -8,4 +8,16 @@ _hybrid = pytest.importorskip("substratus_amd._hybrid")
 @pytest.mark.parametrize("entries,rows", [(0, 1), (3, 0), (0, 0)])
 def test_latent_shares_of_nothing(entries, rows):
     """No division by a number of workgroups that is none."""
-    assert _hybrid.attn_latent_splits(entries, rows, 16, 900) >= 1
+    assert _hybrid.attn_latent_splits(entries, rows, 16, 900, 576, 512) >= 1
+
+
+@pytest.mark.parametrize("n,span,dim,vdim,shares", [
+    (1, 900, 576, 512, 7), (20, 2000, 576, 512, 12), (1, 4000, 576, 512, 20),
+    (128, 900, 576, 512, 2), (130, 900, 576, 512, 3), (170, 900, 320, 256, 3),
+    (171, 900, 576, 512, 1), (130, 800, 576, 512, 1), (300, 4000, 576, 512, 1),
+    (64, 1600, 192, 128, 4), (100, 900, 192, 128, 3), (120, 1500, 192, 128, 4),
+    (200, 900, 72, 64, 2), (230, 500, 72, 64, 1), (1, 60000, 192, 128, 16)])
+def test_latent_shares(n, span, dim, vdim, shares):
+    """As many as there is room for on the CUs, which small keys leave more of,
+    and no share without a chain worth its merge."""
+    assert _hybrid.attn_latent_splits(n, 1, 16, span, dim, vdim) == shares

@@ -132,12 +132,8 @@ def test_unpaged(dim, vdim, shared, window, times):
     assert bool(((got - want[:, :, None]).abs() <= room[:, :, None]).all())
 
 
-# Contexts in shares whose number is no power of two, some without a step: 256 CUs over
-# the contexts, with two steps of 64 keys each
-@pytest.mark.parametrize("n,most", [(1, 450), (19, 900), (37, 700), (85, 450),
-                                    (129, 300)])
-def test_latent_shares(n, most):
-    h, dim, vdim = 16, 192, 128
+def latent_shares(n, most, dim, vdim):
+    h = 16
     spans = [(most - 1 - i * (most - 3) // n, 1) for i in range(n)]
     blocks = sum(f // BS + 1 for f, _ in spans)
     batch = make_batch(spans, blocks)
@@ -152,3 +148,19 @@ def test_latent_shares(n, most):
         want = torch.softmax(s, 1) @ k[:, :vdim].double()
         room = 2.0 ** -8 * want.abs() + 2.0 ** -13 * 4 * want.abs().amax()
         assert bool(((got[e].cpu().double() - want).abs() <= room).all())
+
+
+# Contexts in shares whose number is no power of two, some without a step
+@pytest.mark.parametrize("n,most", [(1, 450), (19, 900), (37, 700), (85, 450),
+                                    (129, 300)])
+def test_latent_shares(n, most):
+    latent_shares(n, most, 192, 128)
+
+
+# Keys that leave a CU room for two workgroups, with four shares, and larger ones: three
+# shares of contexts with a round and a half of workgroups, the most shares
+@pytest.mark.parametrize("n,most,dim,vdim", [
+    (120, 1300, 72, 64), (130, 960, 320, 256), (130, 900, 576, 512),
+    (1, 2800, 576, 512)])
+def test_latent_shares_by_size(n, most, dim, vdim):
+    latent_shares(n, most, dim, vdim)
