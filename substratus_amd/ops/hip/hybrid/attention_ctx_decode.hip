@@ -244,15 +244,17 @@ void attn_ctx_merge_kernel(AttnCtx<bf16_t> a, int splits,
   const bool there = threadIdx.x * VEC < a.vdim;
   const int c = there ? threadIdx.x * VEC : 0;
   const bool sig = a.wbias != nullptr;          // sums only, no part_ml
-  // a lane has a share's maximum and sum
-  float m = NEG, l = 0.f, L = sig ? 1.f : 0.f, o[VEC];
+  // A lane has a share's maximum and sum. Scores may be lower than NEG, which is no
+  // floor here: a row that sees no others is their mean.
+  float m = -INFINITY, l = 0.f, L = sig ? 1.f : 0.f, o[VEC];
   if (lane < splits && !sig) {
     m = part_ml[(at + lane) * 2];
     l = part_ml[(at + lane) * 2 + 1];
   }
-  const float sink = a.sink != nullptr ? a.sink[h] * LOG2E : NEG;
+  const float sink = a.sink != nullptr ? a.sink[h] * LOG2E : -INFINITY;
   const float M = sig ? 0.f : fmaxf(wave_max(m), sink);
-  const float w = sig ? 1.f : __builtin_amdgcn_exp2f(m - M);
+  const float w = sig ? 1.f
+                  : m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
   if (!sig) L = wave_sum(l * w);
   if (a.sink != nullptr) L += __builtin_amdgcn_exp2f(sink - M);
   #pragma unroll

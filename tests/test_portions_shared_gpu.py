@@ -12,8 +12,7 @@ pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
 # first position and rows; single ones come first in a batch
 SPANS = [(0, 1), (0, 32), (31, 33), (40, 127), (0, 128), (63, 129), (0, 31)]
-# contexts long enough to be shared, one whose shares have no step each, one behind
-# which a window or a chunk leaves few
+# contexts long enough to be shared, one whose shares have no step each
 LONG = [(900, 33), (0, 2), (511, 65), (100, 3)]
 
 
@@ -48,18 +47,28 @@ def wide(q, k, v, first, scale, kind):
                                   "chunk"])
 @pytest.mark.parametrize("times,spans", [(1, SPANS), (32, SPANS), (1, LONG)])
 def test_portions(dim, vdim, kind, times, spans):
+    portions(dim, vdim, kind, times, spans, dict(window=37, keep=5), 48)
+
+
+def test_shares_of_low_scores():
+    """Lower than any number that stands for no score."""
+    portions(128, 128, "plain", 1, LONG, None, 0, add=-2e30)
+
+
+def portions(dim, vdim, kind, times, spans, window, chunk, add=0.0):
     g, h = 2, 4
-    batch = make_batch(spans, 128)
+    blocks = max(128, sum((f + n) // BS + 1 for f, n in spans))
+    batch = make_batch(spans, blocks)
     n = batch.tokens.shape[0]
     # one sharp score per row, so that a wrong key shows
     q = rand(n, h, dim, seed=1, dtype=BF16, scale=2.0)
-    kc = rand(128, g, BS, dim, seed=2, dtype=BF16)
-    vc = rand(128, g, BS, vdim, seed=3, dtype=BF16)
-    bias = rand(h, 77, seed=4)
+    kc = rand(blocks, g, BS, dim, seed=2, dtype=BF16)
+    vc = rand(blocks, g, BS, vdim, seed=3, dtype=BF16)
+    bias = rand(h, 77, seed=4) + add
     per_head = rand(h, seed=5)
     kinds = {"sink": dict(sink=per_head), "sigmoid": dict(weight_bias=per_head),
-             "cap": dict(softcap=3.0), "window": dict(window=37, keep=5),
-             "chunk": dict(chunk=48)}.get(kind, {})
+             "cap": dict(softcap=3.0), "window": window,
+             "chunk": dict(chunk=chunk)}.get(kind, {})
     scale = dim ** -0.5
     want = torch.empty(n, h, vdim, dtype=torch.float64)
     row = 0
