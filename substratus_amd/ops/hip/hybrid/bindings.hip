@@ -727,6 +727,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("group_best") = 1, py::arg("at") = py::none());
   m.def("moe_tile", &moe_tile);
   m.def("attn_latent_splits", &attn_latent_splits);
+  m.def("attn_ctx_prefill_splits", &attn_ctx_prefill_splits);
   m.def("moe_sort", &moe_sort);
   m.def("expert_linear", &expert_linear);
   m.def("experts_chosen", &experts_chosen);

@@ -21,3 +21,13 @@ def test_latent_shares(n, span, dim, vdim, shares):
     """As many as there is room for on the CUs, which small keys leave more of,
     and no share without a chain worth its merge."""
     assert _hybrid.attn_latent_splits(n, 1, 16, span, dim, vdim) == shares
+
+
+@pytest.mark.parametrize("entries,rows,heads,vdim,span,shares", [
+    (1, 100, 16, 128, 2100, 11), (4, 103, 32, 128, 3093, 3),
+    (4, 103, 32, 64, 1024, 3), (1, 900, 16, 128, 64, 1),
+    (8, 2400, 16, 128, 4000, 1), (0, 0, 16, 128, 0, 1)])
+def test_portion_shares(entries, rows, heads, vdim, span, shares):
+    """As many as there are CUs for, where a chain of steps is worth them."""
+    assert _hybrid.attn_ctx_prefill_splits(entries, rows, heads, vdim,
+                                           span) == shares

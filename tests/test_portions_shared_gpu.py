@@ -14,6 +14,8 @@ BF16 = torch.bfloat16
 SPANS = [(0, 1), (0, 32), (31, 33), (40, 127), (0, 128), (63, 129), (0, 31)]
 # contexts long enough to be shared, one whose shares have no step each
 LONG = [(900, 33), (0, 2), (511, 65), (100, 3)]
+# several steps for each share, a portion on both sides of a chunk's end
+LONGER = [(3060, 33), (0, 2), (1501, 65), (700, 3)]
 
 
 def wide(q, k, v, first, scale, kind):
@@ -48,6 +50,21 @@ def wide(q, k, v, first, scale, kind):
 @pytest.mark.parametrize("times,spans", [(1, SPANS), (32, SPANS), (1, LONG)])
 def test_portions(dim, vdim, kind, times, spans):
     portions(dim, vdim, kind, times, spans, dict(window=37, keep=5), 48)
+
+
+# Shares of three steps and more, which begin within a context, behind a window, kept
+# keys or a chunk's first key too.
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (192, 72), (256, 256)])
+@pytest.mark.parametrize("kind,times", [
+    ("plain", 1), ("sink", 1), ("sigmoid", 1), ("cap", 1), ("sink", 8),
+    ("window", 8), ("chunk", 8)])
+def test_shares_of_several_steps(dim, vdim, kind, times):
+    span = {"window": 970, "chunk": 1024}.get(kind, 3093)
+    rows = sum(n for _, n in LONGER)
+    shares = ops._ext().attn_ctx_prefill_splits(len(LONGER), rows, 4 * times,
+                                                vdim, span)
+    assert 1 < shares <= span // 64 // 3
+    portions(dim, vdim, kind, times, LONGER, dict(window=900, keep=70), 1024)
 
 
 def test_shares_of_low_scores():
