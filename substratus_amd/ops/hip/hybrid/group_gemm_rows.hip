@@ -21,7 +21,11 @@
 // Where rows are not packed, but have their groups' numbers (ids), a workgroup
 // looks through all of these for its group's rows: a step's choices are a few
 // hundred, which each of its waves has in registers after one load, and nothing
-// waits for a kernel that packs them; the first weights are asked for meanwhile.
+// waits for a kernel that packs them. Weights wait for that: asked for ahead of it
+// they are also asked for where a group has no rows (8 experts of 1536 x 1536, 16
+// rows of one 17.4 us, 11.0 now), and x behind two stages' weights is late (packed,
+// 64 experts of 2048 x 512, 128 rows 88.4, 82.1; listed, of unlike groups, no more
+// than 3 % either way).
 #include "../rows_gemm.h"
 #include "group_gemm.h"
 
@@ -44,75 +48,38 @@ template <int F_, int N_, int P_> struct How {
 
 constexpr int IDS = 512;          // that are looked through, at most
 
-// A wave's share of the inner dimension, and its loads of the weights: 8 rows x 128
-// bytes each, of a tile's row lane / 8, or eight later. Pieces are permuted by the
-// row against bank conflicts. Its stages' weights come first in its part of LDS,
-// whatever the rows of x take.
-template <int N> struct Share {
-  static constexpr int STAGE = U * N * TILE, LOADS = U * N;
-  int c0, c1, steps, end;
-  const char* wp[N][2];
-  int piece[2];
-
-  template <class Y>
-  DEV_INLINE Share(const GroupGemm<bf16_t, Y>& a) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    // shares begin on whole cache lines
-    const int chunks = a.k / KC, pairs = (chunks + 1) / 2;
-    c0 = pairs * wave / KW * 2;
-    c1 = min(pairs * (wave + 1) / KW * 2, chunks);
-    steps = (c1 - c0 + U - 1) / U;
-    end = (c1 - c0) * 4 - 1;                     // its last piece
-    #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      piece[h] = (threadIdx.x & 7) ^ ((h * 8 + row()) >> 1);
-  }
-  static DEV_INLINE int row() { return threadIdx.x % WAVE >> 3; }
-  template <class Y>
-  DEV_INLINE void group(const GroupGemm<bf16_t, Y>& a, int g) {
-    #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      #pragma unroll
-      for (int f = 0; f < N; ++f)
-        wp[f][h] = reinterpret_cast<const char*>(
-            a.w + ((long)g * a.n + min((int)blockIdx.x * N * 16 + f * 16 +
-                                           h * 8 + row(), a.n - 1)) * a.k +
-            c0 * KC);
-  }
-  // a stage may be half of one: then its last piece comes again
-  DEV_INLINE unsigned at(int i, int h) const {
-    return (unsigned)min(i * 8 + piece[h], end) * 16;
-  }
-  DEV_INLINE void load(uint4* ring, int s, int i) const {
-    #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      #pragma unroll
-      for (int f = 0; f < N; ++f)
-        load_to_lds<16>(wp[f][h] + at(i, h),
-                        ring + s * STAGE + (f * 2 + h) * TILE);
-  }
-};
-
-// Of the first E stages the weights are on their way. list: of rows that are not
-// packed, t's numbers are places in it.
-template <class H, Act ACT, bool LISTED, int E, class Y>
+// list: of rows that are not packed, t's numbers are places in it.
+template <class H, Act ACT, bool LISTED, class Y>
 DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
-                              const Share<H::N>& w, uint4* s_all, uint4* ring,
-                              const int* list) {
+                              uint4* s_all, const int* list) {
   constexpr int F = H::F, N = H::N, P = H::P;
-  constexpr int STAGE = U * F * TILE, LOADS = U * (N + F), XL = U * F;
-  static_assert(E <= P && E <= 2);
+  constexpr int TILES = N + F, STAGE = U * TILES * TILE, LOADS = U * TILES;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE, lo = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * N * 16, steps = w.steps;
-  uint4* x_ring = ring + P * Share<N>::STAGE;
+  // shares begin on whole cache lines
+  const int n0 = blockIdx.x * N * 16, chunks = a.k / KC;
+  const int pairs = (chunks + 1) / 2;
+  const int c0 = pairs * wave / KW * 2;
+  const int c1 = min(pairs * (wave + 1) / KW * 2, chunks);
+  const int steps = (c1 - c0 + U - 1) / U;
+  uint4* ring = s_all + wave * P * STAGE;
 
-  const char* xp[F][2];
+  // a load is 8 rows x 128 bytes: of a tile's row lane / 8, or eight later.
+  // Pieces are permuted by the row against bank conflicts.
+  const char *wp[N][2], *xp[F][2];
+  int piece[2];
   #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < 2; ++h) {
+    const int row = h * 8 + (lane >> 3);
+    piece[h] = (lane & 7) ^ (row >> 1);
+    #pragma unroll
+    for (int f = 0; f < N; ++f)
+      wp[f][h] = reinterpret_cast<const char*>(
+          a.w + ((long)t.g * a.n + min(n0 + f * 16 + row, a.n - 1)) * a.k +
+          c0 * KC);
     #pragma unroll
     for (int f = 0; f < F; ++f) {
-      int r = min(t.r0 + f * 16 + h * 8 + w.row(), t.r1 - 1);
+      int r = min(t.r0 + f * 16 + row, t.r1 - 1);
       if constexpr (LISTED) {
         r = list[r];
         if (a.top > 0) r /= a.top;
@@ -120,19 +87,23 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
         r = a.src[r];
       }
       xp[f][h] =
-          reinterpret_cast<const char*>(a.x + (long)r * a.x_ld + w.c0 * KC);
+          reinterpret_cast<const char*>(a.x + (long)r * a.x_ld + c0 * KC);
     }
-  auto load_x = [&](int s, int i) {
+  }
+  const int end = (c1 - c0) * 4 - 1;             // the share's last piece
+  auto load = [&](int s, int i) {
+    uint4* to = ring + s * STAGE;
     #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+      // a stage may be half of one: then its last piece comes again
+      const unsigned at = (unsigned)min(i * 8 + piece[h], end) * 16;
+      #pragma unroll
+      for (int f = 0; f < N; ++f)
+        load_to_lds<16>(wp[f][h] + at, to + (f * 2 + h) * TILE);
       #pragma unroll
       for (int f = 0; f < F; ++f)
-        load_to_lds<16>(xp[f][h] + w.at(i, h),
-                        x_ring + s * STAGE + (f * 2 + h) * TILE);
-  };
-  auto load = [&](int s, int i) {
-    w.load(ring, s, i);
-    load_x(s, i);
+        load_to_lds<16>(xp[f][h] + at, to + ((N + f) * 2 + h) * TILE);
+    }
   };
   float4v acc[N][F];
   #pragma unroll
@@ -143,15 +114,13 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
     short8 wf[U][N], xf[U][F];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int at = lo * 8 + ((u * 4 + g) ^ (lo >> 1));
+      const uint4* p = ring + s * STAGE + lo * 8 + ((u * 4 + g) ^ (lo >> 1));
       #pragma unroll
       for (int f = 0; f < N; ++f)
-        wf[u][f] = *reinterpret_cast<const short8*>(
-            ring + s * Share<N>::STAGE + at + f * 2 * TILE);
+        wf[u][f] = *reinterpret_cast<const short8*>(p + f * 2 * TILE);
       #pragma unroll
       for (int f = 0; f < F; ++f)
-        xf[u][f] = *reinterpret_cast<const short8*>(
-            x_ring + s * STAGE + at + f * 2 * TILE);
+        xf[u][f] = *reinterpret_cast<const short8*>(p + (N + f) * 2 * TILE);
     }
     if (more) {
       wait_lds_reads();
@@ -159,7 +128,7 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
     }
     #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (w.c0 + i * U + u < w.c1) {
+      if (c0 + i * U + u < c1) {
         #pragma unroll
         for (int j = 0; j < N; ++j)
           #pragma unroll
@@ -169,14 +138,8 @@ DEV_INLINE void rows_of_group(const GroupGemm<bf16_t, Y>& a, const Tile& t,
       }
   };
   #pragma unroll
-  for (int s = 0; s < E; ++s)
-    if (s < steps) load_x(s, s);
-  #pragma unroll
-  for (int s = E; s < P; ++s)
+  for (int s = 0; s < P; ++s)
     if (s < steps) load(s, s);
-  // the first stage's rows came later than the second's weights
-  if (steps >= P) wait_loads<(P - E) * LOADS + (E - 1) * XL>();
-  else wait_loads<0>();
   int i = 0;
   for (; i + 2 * P <= steps; i += P) {      // P stages in flight throughout
     #pragma unroll
@@ -260,62 +223,44 @@ void group_gemm_rows_kernel(GroupGemm<bf16_t, Y> a) {
   using Three = How<3, N, 2>;
   using Four = How<4, N, 1>;
   constexpr int LARGEST = MAX > 2 ? Three::PIECES : One::PIECES;
-  constexpr int E = MAX > 2 ? 1 : 2;             // the least of them in flight
-  constexpr int LIST = MAX * 4;                  // pieces of a wave's
+  constexpr int T = MAX * 16;
+  constexpr int LIST = T / 4;                    // pieces of a wave's
   __shared__ alignas(16) uint4 s_all[LARGEST + (LISTED ? KW * LIST : 0)];
   static_assert(MAX == 1 || Two::PIECES <= LARGEST);
   int* list = reinterpret_cast<int*>(s_all + LARGEST +
                                      threadIdx.x / WAVE * LIST);
-  uint4* ring = s_all + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) *
-                            (LARGEST / KW);
-  Share<N> w(a);
-  auto begin = [&](int g) {
-    w.group(a, g);
-    #pragma unroll
-    for (int s = 0; s < E; ++s)
-      if (s < w.steps) w.load(ring, s, s);
-  };
   auto run = [&](const Tile& t) {
     const int tiles = (t.r1 - t.r0 + 15) / 16;   // of the rows there are
     if (MAX == 1 || tiles == 1) {
-      rows_of_group<One, ACT, LISTED, E>(a, t, w, s_all, ring, list);
+      rows_of_group<One, ACT, LISTED>(a, t, s_all, list);
     } else if constexpr (MAX > 1) {
       if (MAX == 2 || tiles == 2) {
-        rows_of_group<Two, ACT, LISTED, E>(a, t, w, s_all, ring, list);
+        rows_of_group<Two, ACT, LISTED>(a, t, s_all, list);
       } else if constexpr (MAX > 2) {
-        if (tiles == 3)
-          rows_of_group<Three, ACT, LISTED, E>(a, t, w, s_all, ring, list);
-        else
-          rows_of_group<Four, ACT, LISTED, E>(a, t, w, s_all, ring, list);
+        if (tiles == 3) rows_of_group<Three, ACT, LISTED>(a, t, s_all, list);
+        else rows_of_group<Four, ACT, LISTED>(a, t, s_all, list);
       }
     }
   };
   if constexpr (LISTED) {
     // As many workgroups as rows, where that is less than groups: a group's first
-    // row has them. Where a group without rows is unlikely, weights do not wait.
-    const bool by_row = a.m < a.groups, early = a.m >= 2 * a.groups;
+    // row has them.
+    const bool by_row = a.m < a.groups;
     const int g = by_row ? a.ids[blockIdx.y] : (int)blockIdx.y;
-    Ids ids;
-    ids.load(a.ids, a.m);
-    __builtin_amdgcn_sched_barrier(0);           // ahead of the weights
-    if (early) begin(g);
-    for (int from = 0;; from += MAX * 16) {
-      const int rows = ids.list(a.m, g, from, MAX * 16, list) - from;
+    for (int from = 0;; from += T) {
+      Ids ids;
+      ids.load(a.ids, a.m);
+      const int rows = ids.list(a.m, g, from, T, list) - from;
       wait_lds_reads();                          // the list is written
-      if (rows <= 0 || (by_row && from == 0 && list[0] != (int)blockIdx.y)) {
-        wait_loads<0>();          // no load outlives its workgroup's LDS
+      if (rows <= 0 || (by_row && from == 0 && list[0] != (int)blockIdx.y))
         return;
-      }
-      if (!early || from > 0) begin(g);
-      run(Tile{g, 0, min(rows, MAX * 16)});
-      if (rows <= MAX * 16) return;
+      run(Tile{g, 0, min(rows, T)});
+      if (rows <= T) return;
       __syncthreads();
     }
   } else {
-    const Tile t = tile_of(a, blockIdx.y, 0, MAX * 16);
-    if (t.r1 <= t.r0) return;
-    begin(t.g);
-    run(t);
+    const Tile t = tile_of(a, blockIdx.y, 0, T);
+    if (t.r1 > t.r0) run(t);
   }
 }
 
@@ -323,12 +268,14 @@ void group_gemm_rows_kernel(GroupGemm<bf16_t, Y> a) {
 
 // Tiles of 32 where ones of 16 would do: workgroups of 32 columns instead of 16 are
 // half as many, and what it takes to begin one and to add up its waves' shares counts
-// more than rows that are not there. us of both products and of packing, MI355X, 16 ->
-// 32: 32 experts of 2048 x 1408, 6 a row, 1, 4, 16, 40 rows 26.5 50 76.6 80.8 -> 25.3
-// 47.2 71.5 73.5; of 4096 x 2048, 8 a row, 1, 4, 32 rows 58.3 138.5 196 -> 57 131.5
-// 183; 64 of 2048 x 1408, 16 and 48 rows 120 144 -> 109 129; 8 of 4096 x 1408, 2 a
-// row, 4 and 16 rows 34.6 46.5 -> 39.1 45.6. Shorter rows are another kernel's with
-// tiles of 16 (64 of 2048 x 512, 4 a row, 16 rows 43.8 -> 49.6).
+// more than rows that are not there. us of both products, gated, weights from memory,
+// MI355X, packed 16 -> packed 32 -> 32 by ids: 32 experts of 2048 x 1408, 6 a row, 1, 4,
+// 16, 32 rows 29.7 64.9 100.9 106.9 -> 28.7 62.5 99.3 100.9 -> 26.5 64.1 98.1 100.8; of
+// 4096 x 2048, 8 a row, 1, 4, 24 rows 80.4 193.4 275.1 -> 79.1 181.6 271.6 -> 76.5
+// 182.8 269.6; 64 of 2048 x 1408, 8, 16 and 64 rows 114 149 202 -> 114 145 190 -> 116
+// 143; 8 of 4096 x 1408, 2 a row, 4 and 16 rows 40.5 57 -> 41.4 54.8 -> 39.5 53.4. Shorter
+// rows are another kernel's with tiles of 16 (64 of 2048 x 512, 4 a row, 16 rows 54.2
+// -> 58.8).
 int group_gemm_rows_tile(int tile, int k, int n) {
   return tile == 16 && k % KC == 0 && n % KC == 0 && std::min(k, n) > 1280
       ? 32 : tile;
@@ -358,13 +305,13 @@ bool group_gemm_rows_takes(const GroupGemm<bf16_t, Y>& a, int tile) {
 }
 
 // Looking for one's rows takes longer than to be told, in every workgroup, and a kernel
-// that packs 3.5 us. us of two products, MI355X, packed -> not, by tiles of 32, of 1,
-// 4, 16, 32, 64 rows: 32 experts of 2048 x 1408, 6 a row 25.3 47.2 71.5 72.5 75 -> 23
-// 46.2 67.1 68.7 72 (2500 workgroups, 64 rows: 1.3 M); of 4096 x 2048, 8 a row 57
-// 131.5 188.3 183.3 191.4 -> 54.2 129.2 185.1 182.8 195 (6144, 32 rows: 1.6 M); 64 of
-// 2048 x 1408, 6 a row, 48 rows 129.2 -> 127.4 (2 M); 16 of 512 x 256, 2 a row, tiles
-// of 16, 4 and 48 rows 11.6 12.9 -> 8.9 10.1. Tiles of 64 wait for their rows at the
-// start of every stage: 74 -> 97.
+// that packs 3 us. us of two products, MI355X, packed -> not, by tiles of 32, of 1,
+// 4, 16, 32, 64 rows: 32 experts of 2048 x 1408, 6 a row 28.7 62.5 99.3 100.9 104 ->
+// 26.5 64.1 98.1 100.8 104.3 (4864 workgroups, 64 rows: 1.9 M); of 4096 x 2048, 8 a row,
+// 24 rows 271.6 -> 269.6 (8192: 1.6 M); 8 of 2048 x 1408, 2 a row 17.3 27.1 33.6 34.1
+// 35.4 -> 14.6 24.1 30.9 31.6 33.1; 16 of 512 x 256, 2 a row, tiles of 16, 4 and 48
+// rows 10.5 12.1 -> 8.2 9. Tiles of 64 wait for their rows at the start of every
+// stage: 74 -> 97.
 bool group_gemm_ids_pay(int rows, int n, int n2, int groups, int tile) {
   const int wide = columns(tile);
   return tile <= 32 &&
