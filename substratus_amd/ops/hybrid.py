@@ -276,8 +276,11 @@ def experts(y: torch.Tensor, router: torch.Tensor, up: torch.Tensor,
     act, limit = ("gelu", 0.0) if spec.glu is None else \
         (spec.glu.act, spec.glu.limit)
     both = h, out, y, up, down, ids, tile, act, limit
-    # a few hundred choices: nothing is packed, rows stay where tokens have them
-    chosen = ext.experts_chosen(*both, True)
+    # Few tokens: nothing is packed, rows stay where tokens have them. An expert that
+    # all choose has one tile then; further ones would follow each other in its
+    # workgroups, where packed ones lie side by side: us, MI355X, 16 experts of 1024 x
+    # 2816, one a token, 256 tokens of one 68.6 and 26.3, of 16 61.4 and 62.2.
+    chosen = rows <= 32 and ext.experts_chosen(*both, True)
     ext.moe_select(ids, weights, z, spec.groups, spec.keep, bias,
                    spec.over_chosen, spec.sigmoid, correction,
                    spec.group_best, at if chosen else None)

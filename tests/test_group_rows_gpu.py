@@ -4,6 +4,7 @@ copied by pieces, gates fetched ahead, against the products in 64 bits."""
 import pytest
 import torch
 
+from substratus_amd.models.layers import MoESpec
 from substratus_amd.ops import hybrid as ops
 from test_hybrid_ops_gpu import close, rand
 
@@ -87,6 +88,24 @@ def test_experts_by_ids(tile, k, ff, act, rows, top, e):
     ext.expert_linear(out2, h2, down, None, start, tiles, tile, "none", 0.0)
     where = at.view(-1).long()
     assert torch.equal(h, h2[where]) and torch.equal(out, out2[where])
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33, 100])
+def test_tokens_of_the_same_experts(rows):
+    """All choose alike: an expert's rows are one tile of up to 32, or packed, where
+    its tiles lie side by side."""
+    spec = MoESpec(8, 2, 128)
+    y = rand(1, 256, seed=1, dtype=BF16).repeat(rows, 1)
+    y += rand(rows, 256, seed=2, dtype=BF16, scale=2.0 ** -6)
+    router = rand(8, 256, seed=3, dtype=BF16)
+    up = rand(8, 128, 256, seed=4, dtype=BF16, scale=2.0 ** -4)
+    down = rand(8, 256, 128, seed=5, dtype=BF16, scale=2.0 ** -3.5)
+    want = ops.experts(y, router, up, down, spec)
+    got = ops.experts(y.cuda(), router.cuda(), up.cuda(), down.cuda(), spec)
+    kept = torch.arange(2 * rows, dtype=torch.int32).view(rows, 2)
+    if rows > 1:
+        assert torch.equal(got.at.cpu(), kept) == (rows <= 32)
+    close(got.rows[got.at.long()], want.rows[want.at.long()], BF16)
 
 
 def test_experts_that_are_packed():
