@@ -671,12 +671,20 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
         }
       }
     } else if (m == 1) {
-      // Eight waves of a row, two stages in flight in each: all of rows of 4096
-      // at once, which q4_K's is slower for where workgroups are many.
-      if constexpr (QQ == Quant::Q4_K) {
-        if (few || k > 4096) go(qc, c4, c1, c8, one_row, no);
-        else go(qc, c4, c1, c4, one_row, no);
-      } else if constexpr (QQ != Quant::Q8_0) {
+      // Eight waves of a row, two stages in flight in each, of q6_K one: all of
+      // rows of 4096 at once. Four where rows are short and workgroups many. us,
+      // MI355X, four -> eight, 32000 x 2048, 16384 x 3072, 28672 x 3584, 32000 x
+      // 4096, 28672 x 4608:
+      //   q4_0  10.8 9.2 15.3 18.4 19.1 -> 11.8 9.6 15.6 17.9 18.8
+      //   q4_K  10.5 9.4 18.0 18.6 23.8 -> 14.6 10.5 17.8 20.7 22.7
+      //   q6_K  14.8 13.8 26.1 29.3 33.6 -> 14.4 13.6 23.8 28.7 31.5
+      // of fewer workgroups, 11264 x 2048, q4_0 5.7 -> 5.5.
+      const bool four = QQ == Quant::Q4_K ? !few && k <= 4096
+                                          : n > 12288 && k < 4096;
+      if constexpr (QQ == Quant::Q4_K || QQ == Quant::Q4_0) {
+        if (four) go(qc, c4, c1, c4, one_row, no);
+        else go(qc, c4, c1, c8, one_row, no);
+      } else if constexpr (QQ == Quant::Q6_K) {
         go(qc, c4, c1, c8, one_row, no);
       }
     } else if (m <= 4) {

@@ -165,12 +165,14 @@ def test_quant_rows(quant, m, n, k):
 # A single row, whose stages hold nothing of other rows: eight waves with none to
 # five stages each, two in flight, a last one in part; workgroups of eight weight
 # rows, whose stages are 512 columns, a last one of half or less (4097 to 6144 rows
-# of 4096 columns and more); four waves (q4_K, more rows of 4096 columns at most)
+# of 4096 columns and more); four waves (q4_K, more rows of 4096 columns at most,
+# q4_0, more than 12288 of fewer)
 @pytest.mark.parametrize("quant", ["q4_0", "q4_K", "q6_K"])
 @pytest.mark.parametrize("n,k", [(41, 64), (40, 1984), (48, 4096), (48, 10240),
                                  (48, 4416), (4112, 4096), (4112, 4352),
                                  (4120, 4160), (5000, 12800), (6160, 4096),
-                                 (6160, 4352), (6176, 10304)])
+                                 (6160, 4352), (6176, 10304), (12304, 64),
+                                 (12304, 1984), (12304, 4032), (12304, 4096)])
 @torch.no_grad()
 def test_quant_one_row(quant, n, k):
     if quant.endswith("_K") and k % 256:
