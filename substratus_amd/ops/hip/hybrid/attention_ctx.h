@@ -101,11 +101,14 @@ void launch_attn_ctx_decode(const AttnCtx<bf16_t>&, int entries, int splits,
                             float* part_o, float* part_ml, hipStream_t);
 
 bool attn_ctx_prefill_supported(int dim, int vdim, int block_size);
+bool attn_ctx_prefill_shared(int entries, long rows, int heads, int vdim,
+                             int span, bool window, bool flat);
 int attn_ctx_prefill_splits(int entries, long rows, int heads, int vdim,
                             int span);
-// splits > 1: of paged keys; shares of sums are left, and attn_ctx_merge follows
+// span: most keys that a row sees; splits > 1: of paged keys; shares of sums are left,
+// and attn_ctx_merge follows
 void launch_attn_ctx_prefill(const AttnCtx<bf16_t>&, int entries, long rows,
-                             int max_len, int splits, float* part_o,
+                             int max_len, int span, int splits, float* part_o,
                              float* part_ml, hipStream_t);
 
 // One head of shared keys whose first columns are the values.

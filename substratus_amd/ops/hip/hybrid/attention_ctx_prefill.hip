@@ -70,10 +70,12 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a, int splits,
   __shared__ alignas(16) short s_v[2][DC][CH / 32][2][2][16][16];
   __shared__ float s_b[2][THREADS];
 
-  const int e = blockIdx.x, head = blockIdx.y;
-  // longest rows first
-  const int tile = (gridDim.z - 1 - blockIdx.z) / splits;
-  const int split = blockIdx.z % splits;
+  // longest rows first, of all entries, or, where waves share rows, of each
+  const int e = SH > 1 ? blockIdx.z : blockIdx.x;
+  const int head = SH > 1 ? blockIdx.x : blockIdx.y;
+  const int place = SH > 1 ? gridDim.y - 1 - blockIdx.y
+                           : gridDim.z - 1 - blockIdx.z;
+  const int tile = place / splits, split = place % splits;
   const Entry en = entry_of(a.seq_start, e);
   const int q0_tile = tile * QT;
   if (q0_tile >= en.n) return;
@@ -113,7 +115,10 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a, int splits,
     }
   }
   float m = -INFINITY, l = 0.f;
-  if (a.sink != nullptr && part_of == 0 && splits == 1) { m = a.sink[head] * LOG2E; l = 1.f; }
+  if (a.sink != nullptr && part_of == 0 && splits == 1) {
+    m = a.sink[head] * LOG2E;
+    l = 1.f;
+  }
   float16v o_t[DC];
   #pragma unroll
   for (int c = 0; c < DC; ++c) o_t[c] = (float16v){};
@@ -438,23 +443,31 @@ bool attn_ctx_prefill_supported(int dim, int vdim, int block_size) {
 // Keys that are not paged are each head's own, and tiles of half the height read them
 // twice as often: there more than half of the CUs at work are enough (keys of 192,
 // six portions of up to 480 rows x 16, 192 tiles: 57.0 and 63.4).
-static bool attn_ctx_prefill_shared(int entries, long rows, int heads,
-                                    int tile, bool flat) {
+// A step of 64 keys that is the only one is no chain, but 64 columns are few to add up:
+// 58 rows of 128 x 64 heads 9.4 and 10.2, 14 of 64 x 4 heads 7.8 and 7.4. Behind a window
+// chains are of one length, and a second round takes as long as the first: 2682 rows of
+// 256 x 8 heads, a window of 164, 55.2 and 68.5; 1973 of 64 x 16 of 1216 88 and 61.
+bool attn_ctx_prefill_shared(int entries, long rows, int heads, int vdim,
+                             int span, bool window, bool flat) {
+  const int tile = vdim <= 128 ? 256 : 128;
   // a portion's last tile is half full on average
-  return heads * (2 * rows / tile + entries) <= 2 * (flat ? 128 : 192);
+  return heads * (2 * rows / tile + entries) <=
+             (flat ? 256 : window ? 320 : 384) &&
+         (vdim <= 64 || span > CH);
 }
 
 // Workgroups that share a tile's keys: those of few tiles, where a step of 64 keys takes
 // 3 us and what follows (a launch, for the host, too; the shares' sums written and read)
-// less than the steps saved; no more workgroups than CUs. us, MI355X, one and by shares, heads of 128,
-// 16 of them: 100 rows behind 2000 96.1 and 29.5, 30 behind 3000 132 and 28.9, 500
-// behind 3500 170 and 65.7, 3 x 100 behind 600 41.3 and 28.0 (900 rows, 49.8 and 41.3,
-// stay whole);
+// less than the steps saved; no more workgroups than CUs. us, MI355X, one and by
+// shares, heads of 128, 16 of them: 100 rows behind 2000 96.1 and 29.5, 30 behind 3000
+// 132 and 28.9, 500 behind 3500 170 and 65.7, 3 x 100 behind 600 41.3 and 28.0 (900
+// rows, 49.8 and 41.3 by two shares, stay whole: the cost is a little high there);
 // heads of 64, 32 of 8: 33.3 and 29.6 of 3 x 100; of 256, 8 of 1: 63.0 and 32.8.
 int attn_ctx_prefill_splits(int entries, long rows, int heads, int vdim,
                             int span) {
   const int tile = vdim <= 128 ? 256 : 128;
-  if (!attn_ctx_prefill_shared(entries, rows, heads, tile, false)) return 1;
+  if (!attn_ctx_prefill_shared(entries, rows, heads, vdim, span, false, false))
+    return 1;
   const long blocks = std::max(1L, heads * (4 * rows / tile + entries) / 2);
   const int steps = (span + CH - 1) / CH;
   auto cost = [&](long s) {
@@ -468,13 +481,19 @@ int attn_ctx_prefill_splits(int entries, long rows, int heads, int vdim,
 }
 
 void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& a, int entries, long rows,
-                             int max_len, int splits, float* part_o,
-                             float* part_ml, hipStream_t stream) {
+                             int max_len, int span, int splits,
+                             float* part_o, float* part_ml,
+                             hipStream_t stream) {
   auto with = [&](auto kk, auto dc, auto waves, auto sh) {
     constexpr int W = decltype(waves)::value, SH = decltype(sh)::value;
     constexpr int K = decltype(kk)::value, D = decltype(dc)::value;
-    const dim3 grid(entries, a.heads,
-                    (max_len + W / SH * 32 - 1) / (W / SH * 32) * splits);
+    const int tiles = (max_len + W / SH * 32 - 1) / (W / SH * 32) * splits;
+    // Workgroups go to XCDs, engines and CUs in turn. An entry's tiles at equal
+    // distances, or entries at a multiple of 32, with those between that others do
+    // not have, would meet the same few CUs, which have two then while others have
+    // none: 127, 775, 127 and 127 rows of 256 x 8 heads 152 us, 80 so.
+    const dim3 grid = SH > 1 ? dim3(a.heads, tiles | (entries > 1), entries)
+                             : dim3(entries, a.heads, tiles);
     const dim3 block(W * WAVE);
     if (a.ctx_start != nullptr)
       attn_ctx_prefill_kernel<K, D, W, SH, true, PLAIN>
@@ -490,8 +509,9 @@ void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& a, int entries, long rows,
           <<<grid, block, 0, stream>>>(a, splits, part_o, part_ml);
   };
   auto go = [&](auto kk, auto dc, auto waves) {
-    if (attn_ctx_prefill_shared(entries, rows, a.heads,
-                                decltype(waves)::value * 32,
+    if (splits > 1 ||
+        attn_ctx_prefill_shared(entries, rows, a.heads, a.vdim, span,
+                                a.window > 0 && a.window + a.keep <= span,
                                 a.ctx_start != nullptr))
       with(kk, dc, waves, std::integral_constant<int, 2>{});
     else

@@ -267,8 +267,8 @@ void attn_ctx(Tensor out, Tensor q, OptTensor gate, Tensor kc, Tensor vc,
           po = ptr<float>(shares);
           pml = po + n * vdim;
         }
-        launch_attn_ctx_prefill(a, entries, rows, max_len, splits, po, pml,
-                                stream());
+        launch_attn_ctx_prefill(a, entries, rows, max_len, span, splits, po,
+                                pml, stream());
         if (splits > 1)
           launch_attn_ctx_merge(a, rows, splits, po, pml, stream());
         return;
@@ -345,8 +345,8 @@ void attn_flat(Tensor out, Tensor q, OptTensor gate, Tensor kv, Tensor kr,
   a.heads = a.kv_heads = heads; a.nbias = 1; a.block_size = 16;
   a.scale = scale; a.mult = 1.f; a.window = window;
   a.out_ld = out.stride(0); a.quads = vdim % 4 == 0;
-  launch_attn_ctx_prefill(a, entries, rows, max_len, 1, nullptr, nullptr,
-                          stream());
+  launch_attn_ctx_prefill(a, entries, rows, max_len, kv.size(0), 1, nullptr,
+                          nullptr, stream());
   post("attn_flat");
 }
 
@@ -727,6 +727,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("group_best") = 1, py::arg("at") = py::none());
   m.def("moe_tile", &moe_tile);
   m.def("attn_latent_splits", &attn_latent_splits);
+  m.def("attn_ctx_prefill_shared", &attn_ctx_prefill_shared);
   m.def("attn_ctx_prefill_splits", &attn_ctx_prefill_splits);
   m.def("moe_sort", &moe_sort);
   m.def("expert_linear", &expert_linear);

@@ -31,3 +31,22 @@ def test_portion_shares(entries, rows, heads, vdim, span, shares):
     """As many as there are CUs for, where a chain of steps is worth them."""
     assert _hybrid.attn_ctx_prefill_splits(entries, rows, heads, vdim,
                                            span) == shares
+
+
+@pytest.mark.parametrize("entries,rows,heads,vdim,span,window,flat,shared", [
+    (1, 900, 16, 128, 900, False, False, True),
+    (8, 2400, 16, 128, 300, False, False, False),
+    (1, 58, 64, 128, 64, False, False, False),
+    (1, 59, 64, 128, 65, False, False, True),
+    (1, 14, 4, 64, 14, False, False, True),
+    (1, 2682, 8, 256, 168, True, False, False),
+    (4, 1973, 16, 64, 1220, True, False, True),
+    (2, 2304, 4, 256, 1624, True, False, True),
+    (1, 2682, 8, 256, 2682, False, False, True),
+    (6, 2400, 16, 128, 480, False, True, False),
+    (2, 900, 16, 128, 480, False, True, True)])
+def test_portions_whose_waves_share_rows(entries, rows, heads, vdim, span,
+                                         window, flat, shared):
+    """Where tiles are few, and neither one step nor a round of CUs more."""
+    assert _hybrid.attn_ctx_prefill_shared(entries, rows, heads, vdim, span,
+                                           window, flat) == shared
