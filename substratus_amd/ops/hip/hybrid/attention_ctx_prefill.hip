@@ -445,14 +445,15 @@ bool attn_ctx_prefill_supported(int dim, int vdim, int block_size) {
 // six portions of up to 480 rows x 16, 192 tiles: 57.0 and 63.4).
 // A step of 64 keys that is the only one is no chain, but 64 columns are few to add up:
 // 58 rows of 128 x 64 heads 9.4 and 10.2, 14 of 64 x 4 heads 7.8 and 7.4. Behind a window
-// chains are of one length, and a second round takes as long as the first: 2682 rows of
-// 256 x 8 heads, a window of 164, 55.2 and 68.5; 1973 of 64 x 16 of 1216 88 and 61.
+// chains are of one length, and a second round takes as long as the first; a CU has
+// room for two workgroups of 64 columns, which make none: 2214 and 2682 rows of 256 x 8
+// heads (288 and 336 tiles) 59.2 and 65.8, 55.2 and 68.5, 1973 of 64 x 16 (304) 88 and 61.
 bool attn_ctx_prefill_shared(int entries, long rows, int heads, int vdim,
                              int span, bool window, bool flat) {
   const int tile = vdim <= 128 ? 256 : 128;
   // a portion's last tile is half full on average
   return heads * (2 * rows / tile + entries) <=
-             (flat ? 256 : window ? 320 : 384) &&
+             (flat ? 256 : window && vdim > 64 ? 280 : 384) &&
          (vdim <= 64 || span > CH);
 }
 

@@ -40,6 +40,7 @@ def test_portion_shares(entries, rows, heads, vdim, span, shares):
     (1, 59, 64, 128, 65, False, False, True),
     (1, 14, 4, 64, 14, False, False, True),
     (1, 2682, 8, 256, 168, True, False, False),
+    (2, 2214, 8, 256, 250, True, False, False),
     (4, 1973, 16, 64, 1220, True, False, True),
     (2, 2304, 4, 256, 1624, True, False, True),
     (1, 2682, 8, 256, 2682, False, False, True),
