@@ -39,6 +39,8 @@ struct AttnCtx {
   const int* ctx_start;    // [entries + 1]
   const T* kr;             // [all keys, shared]
   int shared;
+  int entries;             // prompt portions, in which order
+  bool by_entry;
 };
 
 constexpr float LOG2E = 1.44269504088896340736f;

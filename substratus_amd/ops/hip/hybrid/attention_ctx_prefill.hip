@@ -70,12 +70,14 @@ void attn_ctx_prefill_kernel(AttnCtx<bf16_t> a, int splits,
   __shared__ alignas(16) short s_v[2][DC][CH / 32][2][2][16][16];
   __shared__ float s_b[2][THREADS];
 
-  // longest rows first, of all entries, or, where waves share rows, of each
-  const int e = SH > 1 ? blockIdx.z : blockIdx.x;
+  // longest rows first, of all entries or of each
+  const bool each = SH > 1 && a.by_entry;
+  const int e = SH == 1 ? blockIdx.x : each ? blockIdx.z : blockIdx.y;
   const int head = SH > 1 ? blockIdx.x : blockIdx.y;
-  const int place = SH > 1 ? gridDim.y - 1 - blockIdx.y
-                           : gridDim.z - 1 - blockIdx.z;
+  const int place = each ? gridDim.y - 1 - blockIdx.y
+                         : gridDim.z - 1 - blockIdx.z;
   const int tile = place / splits, split = place % splits;
+  if (SH > 1 && e >= a.entries) return;
   const Entry en = entry_of(a.seq_start, e);
   const int q0_tile = tile * QT;
   if (q0_tile >= en.n) return;
@@ -432,6 +434,11 @@ bool attn_ctx_prefill_supported(int dim, int vdim, int block_size) {
          block_size == PAGE;
 }
 
+// Tiles of half the height, whose last of a portion is half full on average.
+static long halves_of(int entries, long rows, int heads, int vdim) {
+  return heads * (rows / (vdim <= 128 ? 128 : 64) + entries);
+}
+
 // Whether two waves share their rows. Tiles are half as high then, and as many again;
 // the longest one's steps, one after another, are what a launch takes when the tiles
 // are too few for the chip: with more than three quarters of the CUs at work the
@@ -450,9 +457,7 @@ bool attn_ctx_prefill_supported(int dim, int vdim, int block_size) {
 // heads (288 and 336 tiles) 59.2 and 65.8, 55.2 and 68.5, 1973 of 64 x 16 (304) 88 and 61.
 bool attn_ctx_prefill_shared(int entries, long rows, int heads, int vdim,
                              int span, bool window, bool flat) {
-  const int tile = vdim <= 128 ? 256 : 128;
-  // a portion's last tile is half full on average
-  return heads * (2 * rows / tile + entries) <=
+  return halves_of(entries, rows, heads, vdim) <=
              (flat ? 256 : window && vdim > 64 ? 280 : 384) &&
          (vdim <= 64 || span > CH);
 }
@@ -481,20 +486,26 @@ int attn_ctx_prefill_splits(int entries, long rows, int heads, int vdim,
   return best;
 }
 
-void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& a, int entries, long rows,
-                             int max_len, int span, int splits,
+// Where waves share rows workgroups are few, and go to XCDs, engines and CUs in turn.
+// Those of an entry that has more rows than others, at equal distances with a power of
+// two in them, would meet the same few CUs, which have two then while others have none:
+// 127, 775, 127 and 127 rows of 256 x 8 heads 152 us. So an entry's come one after
+// another (80 us), or, of more than CUs, whose longest should be the first of all,
+// entries and one that there is not in turn, if they are even in number.
+void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& given, int entries,
+                             long rows, int max_len, int span, int splits,
                              float* part_o, float* part_ml,
                              hipStream_t stream) {
+  AttnCtx<bf16_t> a = given;
+  a.entries = entries;
+  a.by_entry = halves_of(entries, rows, a.heads, a.vdim) <= 256;
   auto with = [&](auto kk, auto dc, auto waves, auto sh) {
     constexpr int W = decltype(waves)::value, SH = decltype(sh)::value;
     constexpr int K = decltype(kk)::value, D = decltype(dc)::value;
     const int tiles = (max_len + W / SH * 32 - 1) / (W / SH * 32) * splits;
-    // Workgroups go to XCDs, engines and CUs in turn. An entry's tiles at equal
-    // distances, or entries at a multiple of 32, with those between that others do
-    // not have, would meet the same few CUs, which have two then while others have
-    // none: 127, 775, 127 and 127 rows of 256 x 8 heads 152 us, 80 so.
-    const dim3 grid = SH > 1 ? dim3(a.heads, tiles | (entries > 1), entries)
-                             : dim3(entries, a.heads, tiles);
+    const dim3 grid = SH == 1      ? dim3(entries, a.heads, tiles)
+                      : a.by_entry ? dim3(a.heads, tiles | (entries > 1), entries)
+                                   : dim3(a.heads, entries | 1, tiles);
     const dim3 block(W * WAVE);
     if (a.ctx_start != nullptr)
       attn_ctx_prefill_kernel<K, D, W, SH, true, PLAIN>
