@@ -503,9 +503,12 @@ void launch_attn_ctx_prefill(const AttnCtx<bf16_t>& given, int entries,
     constexpr int W = decltype(waves)::value, SH = decltype(sh)::value;
     constexpr int K = decltype(kk)::value, D = decltype(dc)::value;
     const int tiles = (max_len + W / SH * 32 - 1) / (W / SH * 32) * splits;
-    const dim3 grid = SH == 1      ? dim3(entries, a.heads, tiles)
-                      : a.by_entry ? dim3(a.heads, tiles | (entries > 1), entries)
-                                   : dim3(a.heads, entries | 1, tiles);
+    // none of no rows or entries: such a launch is refused
+    const int odd = tiles | (tiles > 0 && entries > 1);
+    const dim3 grid =
+        SH == 1      ? dim3(entries, a.heads, tiles)
+        : a.by_entry ? dim3(a.heads, odd, entries)
+                     : dim3(a.heads, entries > 0 ? entries | 1 : 0, tiles);
     const dim3 block(W * WAVE);
     if (a.ctx_start != nullptr)
       attn_ctx_prefill_kernel<K, D, W, SH, true, PLAIN>
