@@ -305,8 +305,8 @@ bool group_gemm_rows_takes(const GroupGemm<bf16_t, Y>& a, int tile) {
 }
 
 // Looking for one's rows takes longer than to be told, in every workgroup, and a kernel
-// that packs 3 us. us of two products, MI355X, packed -> not, by tiles of 32, of 1,
-// 4, 16, 32, 64 rows: 32 experts of 2048 x 1408, 6 a row 28.7 62.5 99.3 100.9 104 ->
+// that packs 3 us (4.5 in a step). us of two products, MI355X, packed -> not, by tiles
+// of 32, of 1, 4, 16, 32, 64 rows: 32 experts of 2048 x 1408, 6 a row 28.7 62.5 99.3 100.9 104 ->
 // 26.5 64.1 98.1 100.8 104.3 (4864 workgroups, 64 rows: 1.9 M); of 4096 x 2048, 8 a row,
 // 24 rows 271.6 -> 269.6 (8192: 1.6 M); 8 of 2048 x 1408, 2 a row 17.3 27.1 33.6 34.1
 // 35.4 -> 14.6 24.1 30.9 31.6 33.1; 16 of 512 x 256, 2 a row, tiles of 16, 4 and 48

@@ -31,8 +31,8 @@
 // such: with three more of no use, stages took half as much LDS again, and two of
 // them in flight left a CU fewer workgroups. us of 15360 x 5120, 5120 x 5120, 27648
 // x 5120, 5120 x 13824, 12288 x 4096, 22016 x 4096, 32000 x 5120, each from memory,
-// four rows (q4_0 and q6_K: four waves, one stage in flight, of wide matrices) ->
-// one (eight waves, of q4_0 two stages):
+// four rows, in four waves of wide matrices (of q4_0 and q6_K with one stage in flight)
+// -> one, in eight waves (of q4_0 with two stages):
 //   q4_0  13.8 6.8 22.5 13.8 9.2 15.3 27.8 -> 13.5 6.5 22.4 12.9 8.2 14.8 26.3
 //   q4_K  14.5 7.5 25.5 15.6 9.0 16.4 28.8 -> 14.2 6.8 24.2 15.3 8.8 15.2 27.9
 //   q6_K  20.7 10.7 33.7 26.8 12.6 22.6 37.0 -> 20.0 10.9 33.6 27.1 12.1 21.1 36.6
@@ -642,11 +642,9 @@ void launch_rows_quant(bf16_t* y, const bf16_t* x, const void* scales,
     // pays for none. Little more than a workgroup per CU: eight waves share k
     // instead of four, since a wave's chain of stages is what takes the time.
     // us on a MI355X, 4096 x 14336, 5120 x 13824, four waves -> eight: q4_0 5
-    // rows 15.5, 18.9 -> 12.1, 16.3; q4_K 1 row 13.1, 17.1 -> 10.6, 16.5, 5
-    // rows 15.1, 20.0 -> 13.3, 19.4; q6_K 1 row 23.0, 28.1 -> 16.7, 25.9.
+    // rows 15.5, 18.9 -> 12.1, 16.3; q4_K 5 rows 15.1, 20.0 -> 13.3, 19.4.
     // 27648 x 5120, q4_0 5 rows: two stages in flight 26.0, one 22.7; eight
-    // waves 24.8. q4_0 1 row, 5120 x 13824 17.4 -> 15.2, 15360 x 5120 12.9 ->
-    // 13.1.
+    // waves 24.8. A single row has rules of its own, below.
     constexpr bool ONE = QQ == Quant::Q6_K || QQ == Quant::Q4_0;
     constexpr integral_constant<int, ONE ? 1 : 2> some{};
     constexpr integral_constant<int, QQ == Quant::Q6_K ? 1 : 2> one_row{};
