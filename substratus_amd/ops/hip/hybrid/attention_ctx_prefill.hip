@@ -450,11 +450,12 @@ static long halves_of(int entries, long rows, int heads, int vdim) {
 // Keys that are not paged are each head's own, and tiles of half the height read them
 // twice as often: there more than half of the CUs at work are enough (keys of 192,
 // six portions of up to 480 rows x 16, 192 tiles: 57.0 and 63.4).
-// A step of 64 keys that is the only one is no chain, but 64 columns are few to add up:
-// 58 rows of 128 x 64 heads 9.4 and 10.2, 14 of 64 x 4 heads 7.8 and 7.4. Behind a window
-// chains are of one length, and a second round takes as long as the first; a CU has
-// room for two workgroups of 64 columns, which make none: 2214 and 2682 rows of 256 x 8
-// heads (288 and 336 tiles) 59.2 and 65.8, 55.2 and 68.5, 1973 of 64 x 16 (304) 88 and 61.
+// A step of 64 keys that is the only one is no chain, but 64 columns are few to add
+// up: 58 rows of 128 x 64 heads 9.4 and 10.2, 14 of 64 x 4 heads 7.8 and 7.4. Behind a
+// window chains are of one length, and a second round takes as long as the first; a CU
+// has room for two workgroups of 64 columns, which make none: 2214 and 2682 rows of 256
+// x 8 heads (288 and 336 tiles) 59.2 and 65.8, 55.2 and 68.5, 1973 of 64 x 16 (304) 88
+// and 61.
 bool attn_ctx_prefill_shared(int entries, long rows, int heads, int vdim,
                              int span, bool window, bool flat) {
   return halves_of(entries, rows, heads, vdim) <=

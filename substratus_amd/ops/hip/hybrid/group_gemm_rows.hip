@@ -273,9 +273,9 @@ void group_gemm_rows_kernel(GroupGemm<bf16_t, Y> a) {
 // 16, 32 rows 29.7 64.9 100.9 106.9 -> 28.7 62.5 99.3 100.9 -> 26.5 64.1 98.1 100.8; of
 // 4096 x 2048, 8 a row, 1, 4, 24 rows 80.4 193.4 275.1 -> 79.1 181.6 271.6 -> 76.5
 // 182.8 269.6; 64 of 2048 x 1408, 8, 16 and 64 rows 114 149 202 -> 114 145 190 -> 116
-// 143; 8 of 4096 x 1408, 2 a row, 4 and 16 rows 40.5 57 -> 41.4 54.8 -> 39.5 53.4. Shorter
-// rows are another kernel's with tiles of 16 (64 of 2048 x 512, 4 a row, 16 rows 54.2
-// -> 58.8).
+// 143; 8 of 4096 x 1408, 2 a row, 4 and 16 rows 40.5 57 -> 41.4 54.8 -> 39.5 53.4.
+// Shorter rows are another kernel's with tiles of 16 (64 of 2048 x 512, 4 a row, 16
+// rows 54.2 -> 58.8).
 int group_gemm_rows_tile(int tile, int k, int n) {
   return tile == 16 && k % KC == 0 && n % KC == 0 && std::min(k, n) > 1280
       ? 32 : tile;
@@ -306,12 +306,12 @@ bool group_gemm_rows_takes(const GroupGemm<bf16_t, Y>& a, int tile) {
 
 // Looking for one's rows takes longer than to be told, in every workgroup, and a kernel
 // that packs 3 us (4.5 in a step). us of two products, MI355X, packed -> not, by tiles
-// of 32, of 1, 4, 16, 32, 64 rows: 32 experts of 2048 x 1408, 6 a row 28.7 62.5 99.3 100.9 104 ->
-// 26.5 64.1 98.1 100.8 104.3 (4864 workgroups, 64 rows: 1.9 M); of 4096 x 2048, 8 a row,
-// 24 rows 271.6 -> 269.6 (8192: 1.6 M); 8 of 2048 x 1408, 2 a row 17.3 27.1 33.6 34.1
-// 35.4 -> 14.6 24.1 30.9 31.6 33.1; 16 of 512 x 256, 2 a row, tiles of 16, 4 and 48
-// rows 10.5 12.1 -> 8.2 9. Tiles of 64 wait for their rows at the start of every
-// stage: 74 -> 97.
+// of 32, of 1, 4, 16, 32, 64 rows: 32 experts of 2048 x 1408, 6 a row 28.7 62.5 99.3
+// 100.9 104 -> 26.5 64.1 98.1 100.8 104.3 (4864 workgroups, 64 rows: 1.9 M); of 4096 x
+// 2048, 8 a row, 24 rows 271.6 -> 269.6 (8192: 1.6 M); 8 of 2048 x 1408, 2 a row 17.3
+// 27.1 33.6 34.1 35.4 -> 14.6 24.1 30.9 31.6 33.1; 16 of 512 x 256, 2 a row, tiles of
+// 16, 4 and 48 rows 10.5 12.1 -> 8.2 9. Tiles of 64 wait for their rows at the start of
+// every stage: 74 -> 97.
 bool group_gemm_ids_pay(int rows, int n, int n2, int groups, int tile) {
   const int wide = columns(tile);
   return tile <= 32 &&

@@ -5,11 +5,11 @@
 //
 // Bound by the matrix cores if they are kept busy. A workgroup of eight waves
 // takes 256 x 256 outputs, a wave 128 x 64 of them, 64 of the inner dimension
-// at a time (or of fewer rows, see below: what follows is of 256). Two waves share a SIMD. One multiplies while the other reads its
-// next operands from LDS and starts loads from memory; a barrier later they
-// change places (without this turn-taking 1.10 instead of 1.33 PFLOP/s at
-// 4096^3). For that a step of 64 is cut into four phases of a 64 x 32
-// quadrant, 16 matrix instructions each:
+// at a time (or of fewer rows, see below: what follows is of 256). Two waves
+// share a SIMD. One multiplies while the other reads its next operands from LDS
+// and starts loads from memory; a barrier later they change places (without this
+// turn-taking 1.10 instead of 1.33 PFLOP/s at 4096^3). For that a step of 64 is
+// cut into four phases of a 64 x 32 quadrant, 16 matrix instructions each:
 //
 //   phase  1         2         3         4
 //   reads  a low     b high    a high    b low of the next step
